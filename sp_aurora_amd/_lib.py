@@ -124,6 +124,25 @@ def load():
     return lib
 
 
+_native = None
+
+
+def native():
+    """The module behind the public calls' fast path (_native.so: torch tensors in, C ABI calls out, no interpreter in between), or
+    None on a thread that records (ops.prepared): there every call goes through load()'s recorder."""
+    global _native
+    if getattr(_tls, "recorder", None) is not None:
+        return None
+    if _native is None:
+        load()  # says what to do when nothing is built
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise ImportError(f"{os.path.join(_HERE, '_native.so')}: {e}; build it with `python -m sp_aurora_amd.build`") from e
+        _native = module
+    return _native
+
+
 _STRIDE_CACHE = {}
 
 

@@ -1,4 +1,5 @@
-"""Builds libsp_aurora_hip.so (the C-ABI library with the gfx950 kernels) in-tree with hipcc.
+"""Builds libsp_aurora_hip.so (the C-ABI library with the gfx950 kernels) in-tree with hipcc, and _native.so (the host path
+from torch tensors to it, csrc/torch_binding.cpp) with the host compiler.
 
 Usage:  python -m sp_aurora_amd.build        (cross-compiles; no GPU needed)
 """
@@ -10,6 +11,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libsp_aurora_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
+NATIVE_PATH = os.path.join(HERE, "_native.so")
 # (source, object, extra flags).  flash_fwd.hip makes three objects: the zigzag variants of the 16-bit forward kernel
 # and the variants for tensors of 2 GiB and more per (batch, head) are translation units of their own, so that the
 # parts of the longest compile run side by side; flash_bwd.hip likewise makes two.
@@ -49,6 +51,24 @@ def _run(cmd, verbose):
         print(out)
 
 
+def _native_command(objdir):
+    """Compiles csrc/torch_binding.cpp against the torch that is installed."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    base = os.path.dirname(torch.__file__)
+    include = [f"-I{d}" for d in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]]
+    compile_ = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+                f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *include,
+                "-c", "-o", os.path.join(objdir, "torch_binding.o"), os.path.join(CSRC, "torch_binding.cpp")]
+    # the kernels' library is found beside the module, torch's libraries are those the interpreter has loaded
+    link = [compile_[0], "-shared", "-o", NATIVE_PATH, os.path.join(objdir, "torch_binding.o"), f"-L{HERE}", f"-l:{LIB_NAME}",
+            f"-L{os.path.join(base, 'lib')}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-lamdhip64",
+            "-Wl,-rpath,$ORIGIN"]
+    return compile_, link
+
+
 def build(verbose: bool = True) -> str:
     """Compile every HIP source into sp_aurora_amd/libsp_aurora_hip.so and return its path."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -62,9 +82,12 @@ def build(verbose: bool = True) -> str:
     with ThreadPoolExecutor(max_workers=min(len(UNITS), os.cpu_count() or 1)) as pool:
         jobs = [pool.submit(_run, [hipcc] + FLAGS + extra + ["-c", "-o", os.path.join(objdir, obj), os.path.join(CSRC, src)], verbose)
                 for src, obj, extra in UNITS]
+        native_compile, native_link = _native_command(objdir)
+        jobs.append(pool.submit(_run, native_compile, verbose))
         for j in jobs:
             j.result()
     _run([hipcc, "--offload-arch=gfx950", "-fPIC", "-shared", "-o", LIB_PATH] + objs, verbose)
+    _run(native_link, verbose)
     return LIB_PATH
 
 

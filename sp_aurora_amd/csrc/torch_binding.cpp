@@ -1,0 +1,514 @@
+// CPython module sp_aurora_amd._native: the host path of the public calls, from torch tensors to the C ABI.
+//
+// A call of the operator on a small block lasts 5 to 15 us on the GPU, and what Python and ctypes spent in front of it
+// was as much again (12 us forward, 150 us for a forward and a backward through torch.autograd.Function).  The
+// functions here take the arguments that a well-formed call has - contiguous head dim, 16-byte aligned rows, one device, one
+// dtype - allocate the results and enqueue the kernels; the differentiable ones are C++ autograd nodes, whose backward runs on
+// the autograd thread without the interpreter.  For anything else (an argument that needs a copy, a check that fails,
+// an entry point that refuses) they return None, and the Python code behind them does the copy or raises the error.
+#include <Python.h>
+#include <hip/hip_runtime_api.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <ATen/ops/zeros.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <cmath>
+
+#include "../../include/sp_aurora_hip.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+constexpr auto kFp8 = at::kFloat8_e4m3fn;
+
+int dtype_code(at::ScalarType t) { return t == at::kFloat ? SPA_F32 : t == at::kBFloat16 ? SPA_BF16 : t == at::kHalf ? SPA_F16 : -1; }
+
+// Rows that the kernels can address: inner stride 1, base and every other stride a multiple of `bytes`.
+bool rows_ok(const Tensor& t, int64_t bytes = 16) {
+  const auto st = t.strides();
+  const int64_t esz = t.element_size(), n = t.dim();
+  if (st[n - 1] != 1 || ((uintptr_t)t.const_data_ptr() % bytes) != 0) return false;
+  for (int64_t i = 0; i + 1 < n; ++i)
+    if ((st[i] * esz) % bytes != 0) return false;
+  return true;
+}
+
+// One operand as the C ABI takes it: pointer, (batch, head, seq) strides in elements, sizes.
+struct View {
+  void* p = nullptr;
+  int64_t st[3] = {0, 0, 0};
+  int B = 0, H = 0, S = 0, D = 0;
+  bool same_shape(const View& o) const { return B == o.B && H == o.H && S == o.S && D == o.D; }
+};
+
+// [B,S,H,D] (bshd) or [B,H,S,D]; `part` of a packed [B,S,n,H,D] tensor when part >= 0; a rank-stacked [P,1,s,H,D] tensor
+// whose ranks' rows follow each other as the one sequence [1,P*s,H,D].
+bool view_of(const Tensor& t, bool bshd, View& v, int part = -1) {
+  const auto sz = t.sizes();
+  const auto st = t.strides();
+  for (const int64_t n : sz)
+    if (n <= 0 || n > 0x7fffffffLL) return false;
+  v.p = t.data_ptr();
+  if (part >= 0) {
+    if (t.dim() != 5) return false;
+    v.B = (int)sz[0]; v.S = (int)sz[1]; v.H = (int)sz[3]; v.D = (int)sz[4];
+    v.st[0] = st[0]; v.st[1] = st[3]; v.st[2] = st[1];
+    v.p = (char*)v.p + part * st[2] * (int64_t)t.element_size();
+    return true;
+  }
+  if (t.dim() == 5) {
+    if (!bshd || sz[1] != 1 || (sz[0] > 1 && st[0] != sz[2] * st[2]) || sz[0] * sz[2] > 0x7fffffffLL) return false;
+    v.B = 1; v.S = (int)(sz[0] * sz[2]); v.H = (int)sz[3]; v.D = (int)sz[4];
+    v.st[0] = v.S * st[2]; v.st[1] = st[3]; v.st[2] = st[2];
+    return true;
+  }
+  if (t.dim() != 4) return false;
+  const int s = bshd ? 1 : 2, h = bshd ? 2 : 1;
+  v.B = (int)sz[0]; v.S = (int)sz[s]; v.H = (int)sz[h]; v.D = (int)sz[3];
+  v.st[0] = st[0]; v.st[1] = st[h]; v.st[2] = st[s];
+  return true;
+}
+
+// A packed [rows,H,D] tensor; strides (head, row).
+bool view_thd(const Tensor& t, View& v) {
+  if (t.dim() != 3) return false;
+  const auto sz = t.sizes();
+  for (const int64_t n : sz)
+    if (n <= 0 || n > 0x7fffffffLL) return false;
+  v.p = t.data_ptr();
+  v.B = 1; v.S = (int)sz[0]; v.H = (int)sz[1]; v.D = (int)sz[2];
+  v.st[0] = t.stride(1); v.st[1] = t.stride(0);
+  return true;
+}
+
+bool on_device(const Tensor& t, const Tensor& q) { return t.is_cuda() && t.device() == q.device(); }
+
+// fp32 [n, H] on q's device.
+bool scale_ok(const Tensor& t, const Tensor& q, int64_t n, int64_t H) {
+  return t.defined() && on_device(t, q) && t.scalar_type() == at::kFloat && t.dim() == 2 && t.size(0) == n && t.size(1) == H && t.is_contiguous();
+}
+
+// The stream that is current on the calling thread (of the current device, as torch.cuda.current_stream()).
+void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+float softmax_scale_or_default(double scale, int D) { return (float)(std::isnan(scale) ? 1.0 / std::sqrt((double)D) : scale); }
+
+Tensor empty_f32(at::IntArrayRef sizes, const Tensor& like) { return at::empty(sizes, like.options().dtype(at::kFloat)); }
+
+// ---------------------------------------------------------------- forward
+// (out, lse) of one block call; false: not a call for this path.
+bool flash_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale_or_nan, bool causal, bool bshd, const Tensor& q_scale,
+               const Tensor& k_scale, const Tensor& v_scale, int out_dtype, Tensor& out, Tensor& lse) {
+  if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || !q.is_cuda() || !on_device(k, q) || !on_device(v, q)) return false;
+  const bool q8 = q.scalar_type() == kFp8, kv8 = k.scalar_type() == kFp8;
+  if (v.scalar_type() != k.scalar_type() || (q8 && !kv8) || (!kv8 && k.scalar_type() != q.scalar_type())) return false;
+  const int dtype = q8 ? out_dtype : dtype_code(q.scalar_type());
+  if (dtype < 0) return false;
+  View a, b, c;
+  if (!rows_ok(q) || !rows_ok(k, kv8 && !q8 ? 8 : 16) || !rows_ok(v, q8 ? 16 : kv8 ? 8 : 16) || !view_of(q, bshd, a) || !view_of(k, bshd, b) ||
+      !view_of(v, bshd, c) || !b.same_shape(c) || a.B != b.B || a.H != b.H || a.D != b.D)
+    return false;
+  if (kv8 && (!scale_ok(k_scale, q, a.B, a.H) || !scale_ok(v_scale, q, a.B, a.H) || (q8 && !scale_ok(q_scale, q, a.B, a.H)))) return false;
+  const float scale = softmax_scale_or_default(scale_or_nan, a.D);
+  void* const stream = current_stream();
+  const c10::DeviceGuard guard(q.device());
+  out = at::empty(q.sizes(), q8 ? q.options().dtype(dtype == SPA_F16 ? at::kHalf : at::kBFloat16) : q.options());
+  lse = empty_f32({a.B, a.H, a.S}, q);
+  View o;
+  view_of(out, bshd, o);
+  float* const lp = (float*)lse.data_ptr();
+  const int mask = causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE;
+  const float* const ks = kv8 ? (const float*)k_scale.const_data_ptr() : nullptr;
+  const float* const vs = kv8 ? (const float*)v_scale.const_data_ptr() : nullptr;
+  if (q8)
+    return spa_flash_fwd_fp8qkv(a.p, b.p, c.p, (const float*)q_scale.const_data_ptr(), ks, vs, o.p, lp, a.B, a.H, a.S, b.S, a.D, a.st, b.st, c.st,
+                                o.st, scale, mask, dtype, stream) == SPA_OK;
+  // few query rows against many keys: the keys split over the grid, the chunks' results in a workspace (not while the
+  // stream is being captured: the workspace would not outlive this call)
+  if (!causal && dtype != SPA_F32 && (a.D == 64 || a.D == 128)) {
+    int n = spa_flash_fwd_splitkv_suggest(a.B, a.H, a.S, b.S, a.D, mask, dtype);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (n > 1 && (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)) n = 1;
+    if (n > 1) {
+      const Tensor ws = at::empty({spa_flash_fwd_splitkv_workspace_bytes(a.B, a.H, a.S, a.D, n, dtype)}, q.options().dtype(at::kByte));
+      return (kv8 ? spa_flash_fwd_splitkv_fp8kv(a.p, b.p, c.p, ks, vs, o.p, lp, ws.data_ptr(), a.B, a.H, a.S, b.S, a.D, n, a.st, b.st, c.st, o.st,
+                                                scale, dtype, stream)
+                  : spa_flash_fwd_splitkv(a.p, b.p, c.p, o.p, lp, ws.data_ptr(), a.B, a.H, a.S, b.S, a.D, n, a.st, b.st, c.st, o.st, scale, dtype,
+                                          stream)) == SPA_OK;
+    }
+  }
+  if (kv8)
+    return spa_flash_fwd_fp8kv(a.p, b.p, c.p, ks, vs, o.p, lp, a.B, a.H, a.S, b.S, a.D, a.st, b.st, c.st, o.st, scale, mask, dtype, stream) == SPA_OK;
+  return spa_flash_fwd(a.p, b.p, c.p, o.p, lp, a.B, a.H, a.S, b.S, a.D, a.st, b.st, c.st, o.st, scale, mask, dtype, stream) == SPA_OK;
+}
+
+bool cu_ok(const Tensor& cu, const Tensor& q) {
+  return on_device(cu, q) && cu.scalar_type() == at::kInt && cu.dim() == 1 && cu.numel() >= 2 && cu.is_contiguous();
+}
+
+bool varlen_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu_q, const Tensor& cu_k, int64_t max_q, int64_t max_k,
+                double scale_or_nan, bool causal, const Tensor& k_scale, const Tensor& v_scale, Tensor& out, Tensor& lse) {
+  if (!q.is_cuda() || !on_device(k, q) || !on_device(v, q) || !cu_ok(cu_q, q) || !cu_ok(cu_k, q) || cu_q.numel() != cu_k.numel()) return false;
+  const bool kv8 = k.scalar_type() == kFp8;
+  const int dtype = dtype_code(q.scalar_type());
+  View a, b, c, o;
+  if (dtype < 0 || v.scalar_type() != k.scalar_type() || (!kv8 && k.scalar_type() != q.scalar_type()) || !view_thd(q, a) || !view_thd(k, b) ||
+      !view_thd(v, c) || !b.same_shape(c) || a.H != b.H || a.D != b.D || !rows_ok(q) || !(kv8 ? k.is_contiguous() && v.is_contiguous() : rows_ok(k) && rows_ok(v)))
+    return false;
+  const int nseq = (int)cu_q.numel() - 1;
+  if (kv8 && (!scale_ok(k_scale, q, nseq, a.H) || !scale_ok(v_scale, q, nseq, a.H))) return false;
+  const float scale = softmax_scale_or_default(scale_or_nan, a.D);
+  void* const stream = current_stream();
+  const c10::DeviceGuard guard(q.device());
+  out = at::empty(q.sizes(), q.options());
+  lse = empty_f32({a.H, a.S}, q);
+  view_thd(out, o);
+  const int mask = causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE;
+  const int* const cq = (const int*)cu_q.const_data_ptr();
+  const int* const ck = (const int*)cu_k.const_data_ptr();
+  float* const lp = (float*)lse.data_ptr();
+  if (kv8)
+    return spa_flash_fwd_varlen_fp8kv(a.p, b.p, c.p, (const float*)k_scale.const_data_ptr(), (const float*)v_scale.const_data_ptr(), o.p, lp, cq, ck,
+                                      nseq, a.H, a.S, b.S, (int)max_q, (int)max_k, a.D, a.st, b.st, c.st, o.st, scale, mask, dtype, stream) == SPA_OK;
+  return spa_flash_fwd_varlen(a.p, b.p, c.p, o.p, lp, cq, ck, nseq, a.H, a.S, b.S, (int)max_q, (int)max_k, a.D, a.st, b.st, c.st, o.st, scale, mask,
+                              dtype, stream) == SPA_OK;
+}
+
+// ---------------------------------------------------------------- differentiable calls
+// The operands of a differentiable call are separate tensors, q and a packed kv, or one packed qkv: `n` tensors, and the
+// gradients come back packed the same way, each written once by the kernels.
+struct Operands {
+  View q, k, v;
+};
+bool operands(const Tensor* t, int n, Operands& o) {
+  if (n == 3) return view_of(t[0], true, o.q) && view_of(t[1], true, o.k) && view_of(t[2], true, o.v);
+  if (n == 2) return view_of(t[0], true, o.q) && view_of(t[1], true, o.k, 0) && view_of(t[1], true, o.v, 1);
+  return view_of(t[0], true, o.q, 0) && view_of(t[0], true, o.k, 1) && view_of(t[0], true, o.v, 2);
+}
+bool differentiable_ok(const Tensor* t, int n) {
+  const int dtype = dtype_code(t[0].scalar_type());
+  if (dtype < 0 || !t[0].is_cuda()) return false;
+  for (int i = 0; i < n; ++i)
+    if (!on_device(t[i], t[0]) || t[i].scalar_type() != t[0].scalar_type() || t[i].dim() < 3 || !rows_ok(t[i])) return false;
+  return true;
+}
+bool attention_ok(const Tensor* t, int n) {
+  Operands o;
+  if (!differentiable_ok(t, n) || !operands(t, n, o)) return false;
+  if (n < 3 && (t[n - 1].dim() != 5 || t[n - 1].size(2) != 4 - n)) return false;
+  if (n == 3 && (t[0].dim() != t[1].dim() || t[0].dim() != t[2].dim() || (t[0].dim() == 5 && t[0].sizes() != t[1].sizes()))) return false;
+  return o.k.same_shape(o.v) && o.q.B == o.k.B && o.q.H == o.k.H && o.q.D == o.k.D && (o.q.D == 32 || o.q.D == 64 || o.q.D == 128);
+}
+
+void check(int rc) { TORCH_CHECK(rc == SPA_OK, "[spa ", rc, "] ", spa_last_error()); }
+
+// Block attention over whole sequences (every ring whose contiguous shards this GPU holds is that: the blocks of the ring
+// tile the score matrix).
+template <int N>
+struct Attention : public torch::autograd::Function<Attention<N>> {
+  static variable_list forward_of(const Tensor* t, double scale_or_nan, bool causal) {
+    Operands x;
+    operands(t, N, x);
+    const Tensor& q = t[0];
+    void* const stream = current_stream();
+    const c10::DeviceGuard guard(q.device());
+    Tensor out = N == 1 ? at::empty({x.q.B, x.q.S, x.q.H, x.q.D}, q.options()) : at::empty(q.sizes(), q.options());
+    Tensor lse = empty_f32({x.q.B, x.q.H, x.q.S}, q);
+    View o;
+    view_of(out, true, o);
+    check(spa_flash_fwd(x.q.p, x.k.p, x.v.p, o.p, (float*)lse.data_ptr(), x.q.B, x.q.H, x.q.S, x.k.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st,
+                        softmax_scale_or_default(scale_or_nan, x.q.D), causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype_code(q.scalar_type()), stream));
+    return {out, lse};
+  }
+  static variable_list save(AutogradContext* ctx, const Tensor* t, double scale, bool causal) {
+    variable_list r = forward_of(t, scale, causal);
+    variable_list saved(t, t + N);
+    saved.insert(saved.end(), r.begin(), r.end());
+    ctx->save_for_backward(std::move(saved));
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["causal"] = causal;
+    ctx->mark_non_differentiable({r[1]});
+    return r;
+  }
+  template <typename... Args>
+  static variable_list forward(AutogradContext* ctx, Args... args) {
+    return unpack(ctx, std::make_index_sequence<N>{}, args...);
+  }
+  template <size_t... I, typename... Args>
+  static variable_list unpack(AutogradContext* ctx, std::index_sequence<I...>, Args&... args) {
+    auto all = std::tie(args...);
+    const Tensor t[N] = {std::get<I>(all)...};
+    return save(ctx, t, std::get<N>(all), std::get<N + 1>(all));
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list saved = ctx->get_saved_variables();
+    const double scale_or_nan = ctx->saved_data["scale"].toDouble();
+    const bool causal = ctx->saved_data["causal"].toBool();
+    Operands x, g;
+    operands(saved.data(), N, x);
+    const Tensor &q = saved[0], &out = saved[N], &lse = saved[N + 1];
+    void* const stream = current_stream();
+    const c10::DeviceGuard guard(q.device());
+    View o, d;
+    const Tensor dout = rows_ok(grads[0]) && view_of(grads[0], true, d) ? grads[0] : grads[0].contiguous();
+    variable_list back;
+    for (int i = 0; i < N; ++i) back.push_back(at::empty(saved[i].sizes(), saved[i].options()));
+    operands(back.data(), N, g);
+    const Tensor delta = empty_f32(lse.sizes(), lse);
+    TORCH_CHECK(view_of(out, true, o) && view_of(dout, true, d) && o.same_shape(d) && dout.scalar_type() == q.scalar_type(), "bad gradient of the output");
+    const int dtype = dtype_code(q.scalar_type());
+    check(spa_bwd_delta(o.p, d.p, (float*)delta.data_ptr(), o.B, o.H, o.S, o.D, o.st, d.st, dtype, stream));
+    check(spa_flash_bwd_out(x.q.p, x.k.p, x.v.p, d.p, (const float*)lse.const_data_ptr(), (const float*)delta.const_data_ptr(), g.q.p, g.k.p, g.v.p,
+                            x.q.B, x.q.H, x.q.S, x.k.S, x.q.D, x.q.st, x.k.st, x.v.st, d.st, g.q.st, g.k.st, g.v.st,
+                            softmax_scale_or_default(scale_or_nan, x.q.D), causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype, stream));
+    back.push_back(Tensor());
+    back.push_back(Tensor());
+    return back;
+  }
+};
+
+bool wants_grad(const Tensor* t, int n) {
+  if (!c10::GradMode::is_enabled()) return false;
+  for (int i = 0; i < n; ++i)
+    if (t[i].requires_grad()) return true;
+  return false;
+}
+
+// Packed batch of sequences of different lengths.
+struct VarlenAttention : public torch::autograd::Function<VarlenAttention> {
+  static variable_list forward(AutogradContext* ctx, Tensor q, Tensor k, Tensor v, Tensor cu_q, Tensor cu_k, int64_t max_q, int64_t max_k, double scale,
+                               bool causal, bool covered) {
+    Tensor out, lse;
+    TORCH_CHECK(varlen_fwd(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, Tensor(), Tensor(), out, lse), spa_last_error());
+    ctx->save_for_backward({q, k, v, out, lse, cu_q, cu_k});
+    ctx->saved_data["max_q"] = max_q;
+    ctx->saved_data["max_k"] = max_k;
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["causal"] = causal;
+    ctx->saved_data["covered"] = covered;
+    ctx->mark_non_differentiable({lse});
+    return {out, lse};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const Tensor &q = s[0], &out = s[3], &lse = s[4];
+    void* const stream = current_stream();
+    const c10::DeviceGuard guard(q.device());
+    const Tensor dout = rows_ok(grads[0]) ? grads[0] : grads[0].contiguous();
+    View a, b, c, d, g[3];
+    TORCH_CHECK(view_thd(q, a) && view_thd(s[1], b) && view_thd(s[2], c) && view_thd(dout, d) && a.same_shape(d), "bad gradient of the output");
+    // the kernels write the rows of the sequences; other rows' gradients are zero
+    const bool covered = ctx->saved_data["covered"].toBool();
+    variable_list back;
+    for (int i = 0; i < 3; ++i) {
+      back.push_back(covered ? at::empty(s[i].sizes(), s[i].options()) : at::zeros(s[i].sizes(), s[i].options()));
+      view_thd(back[i], g[i]);
+    }
+    const Tensor delta = empty_f32(lse.sizes(), lse);
+    const int dtype = dtype_code(q.scalar_type());
+    const int64_t os[3] = {0, out.stride(1), out.stride(0)}, ds[3] = {0, d.st[0], d.st[1]};
+    check(spa_bwd_delta(out.const_data_ptr(), d.p, (float*)delta.data_ptr(), 1, a.H, a.S, a.D, os, ds, dtype, stream));
+    check(spa_flash_bwd_varlen_out(a.p, b.p, c.p, d.p, (const float*)lse.const_data_ptr(), (const float*)delta.const_data_ptr(), g[0].p, g[1].p, g[2].p,
+                                   (const int*)s[5].const_data_ptr(), (const int*)s[6].const_data_ptr(), (int)s[5].numel() - 1, a.H, a.S, b.S,
+                                   (int)ctx->saved_data["max_q"].toInt(), (int)ctx->saved_data["max_k"].toInt(), a.D, a.st, b.st, c.st, d.st, g[0].st,
+                                   g[1].st, g[2].st, softmax_scale_or_default(ctx->saved_data["scale"].toDouble(), a.D),
+                                   ctx->saved_data["causal"].toBool() ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype, stream));
+    back.resize(10);
+    return back;
+  }
+};
+
+// ---------------------------------------------------------------- Python side
+// Arguments come positionally from this package's own functions; a tensor argument that is no tensor (or a number that is no
+// number) is a call for the Python path, which raises what it always raised.
+bool tensor_arg(PyObject* o, Tensor& t) {
+  if (!THPVariable_Check(o)) return false;
+  t = THPVariable_Unpack(o);
+  return true;
+}
+bool optional_tensor(PyObject* o, Tensor& t) { return o == Py_None || tensor_arg(o, t); }
+bool scale_arg(PyObject* o, double& x) {
+  if (o == Py_None) {
+    x = NAN;
+    return true;
+  }
+  if (!PyFloat_Check(o) && !PyLong_Check(o)) return false;
+  x = PyFloat_AsDouble(o);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return std::isfinite(x);
+}
+bool flag_arg(PyObject* o) {
+  const int r = PyObject_IsTrue(o);
+  if (r < 0) throw python_error();
+  return r != 0;
+}
+PyObject* pair(const Tensor& out, const Tensor& lse) {
+  PyObject* const r = PyTuple_New(2);
+  if (!r) throw python_error();
+  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(out));
+  PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(lse));
+  return r;
+}
+
+// flash_fwd(q, k, v, scale, causal, bshd, q_scale, k_scale, v_scale, out_dtype_code)
+PyObject* py_flash_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Tensor q, k, v, qs, ks, vs, out, lse;
+  double scale;
+  if (n != 10 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !scale_arg(a[3], scale) || !optional_tensor(a[6], qs) ||
+      !optional_tensor(a[7], ks) || !optional_tensor(a[8], vs))
+    Py_RETURN_NONE;
+  const bool causal = flag_arg(a[4]), bshd = flag_arg(a[5]);
+  const int out_dtype = (int)PyLong_AsLong(a[9]);
+  bool done;
+  {
+    pybind11::gil_scoped_release no_gil;
+    done = flash_fwd(q, k, v, scale, causal, bshd, qs, ks, vs, out_dtype, out, lse);
+  }
+  if (!done) Py_RETURN_NONE;
+  return pair(out, lse);
+  END_HANDLE_TH_ERRORS
+}
+
+// varlen_fwd(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, k_scale, v_scale)
+PyObject* py_varlen_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Tensor q, k, v, cq, ck, ks, vs, out, lse;
+  double scale;
+  if (n != 11 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], cq) || !tensor_arg(a[4], ck) ||
+      !PyLong_Check(a[5]) || !PyLong_Check(a[6]) || !scale_arg(a[7], scale) || !optional_tensor(a[9], ks) || !optional_tensor(a[10], vs))
+    Py_RETURN_NONE;
+  const int64_t mq = PyLong_AsLongLong(a[5]), mk = PyLong_AsLongLong(a[6]);
+  const bool causal = flag_arg(a[8]);
+  bool done = false;
+  if (mq > 0 && mk > 0 && mq <= 0x7fffffffLL && mk <= 0x7fffffffLL) {
+    pybind11::gil_scoped_release no_gil;
+    done = varlen_fwd(q, k, v, cq, ck, mq, mk, scale, causal, ks, vs, out, lse);
+  }
+  if (!done) Py_RETURN_NONE;
+  return pair(out, lse);
+  END_HANDLE_TH_ERRORS
+}
+
+// attention(tensors..., scale, causal): q, k, v | q, kv | qkv
+template <int N, size_t... I>
+PyObject* attention(PyObject* const* a, std::index_sequence<I...>) {
+  HANDLE_TH_ERRORS
+  Tensor t[N];
+  double scale;
+  for (int i = 0; i < N; ++i)
+    if (!tensor_arg(a[i], t[i])) Py_RETURN_NONE;
+  if (!scale_arg(a[N], scale) || !attention_ok(t, N)) Py_RETURN_NONE;
+  const bool causal = flag_arg(a[N + 1]);
+  variable_list r;
+  {
+    pybind11::gil_scoped_release no_gil;
+    r = wants_grad(t, N) ? Attention<N>::apply(t[I]..., scale, causal) : Attention<N>::forward_of(t, scale, causal);
+  }
+  return pair(r[0], r[1]);
+  END_HANDLE_TH_ERRORS
+}
+PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n == 5) return attention<3>(a, std::make_index_sequence<3>{});
+  if (n == 4) return attention<2>(a, std::make_index_sequence<2>{});
+  if (n == 3) return attention<1>(a, std::make_index_sequence<1>{});
+  Py_RETURN_NONE;
+}
+
+// varlen_attention(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, covered)
+PyObject* py_varlen_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Tensor t[5];
+  double scale;
+  if (n != 10) Py_RETURN_NONE;
+  for (int i = 0; i < 5; ++i)
+    if (!tensor_arg(a[i], t[i])) Py_RETURN_NONE;
+  if (!PyLong_Check(a[5]) || !PyLong_Check(a[6]) || !scale_arg(a[7], scale)) Py_RETURN_NONE;
+  const int64_t mq = PyLong_AsLongLong(a[5]), mk = PyLong_AsLongLong(a[6]);
+  const bool causal = flag_arg(a[8]), covered = flag_arg(a[9]);
+  if (!differentiable_ok(t, 3) || !cu_ok(t[3], t[0]) || !cu_ok(t[4], t[0]) || mq <= 0 || mk <= 0 || mq > 0x7fffffffLL || mk > 0x7fffffffLL)
+    Py_RETURN_NONE;
+  variable_list r(2);
+  {
+    pybind11::gil_scoped_release no_gil;
+    if (wants_grad(t, 3)) {
+      View x, y, z;
+      if (!view_thd(t[0], x) || !view_thd(t[1], y) || !view_thd(t[2], z) || !y.same_shape(z) || x.H != y.H || x.D != y.D || mq > x.S || mk > y.S ||
+          t[3].numel() != t[4].numel() || (x.D != 32 && x.D != 64 && x.D != 128))
+        r.clear();
+      else
+        r = VarlenAttention::apply(t[0], t[1], t[2], t[3], t[4], mq, mk, scale, causal, covered);
+    } else if (!varlen_fwd(t[0], t[1], t[2], t[3], t[4], mq, mk, scale, causal, Tensor(), Tensor(), r[0], r[1])) {
+      r.clear();
+    }
+  }
+  if (r.empty()) Py_RETURN_NONE;
+  return pair(r[0], r[1]);
+  END_HANDLE_TH_ERRORS
+}
+
+// merge(out_acc [B,S,H,D] fp32, lse_acc [B,S,H,1] over a contiguous [B,H,S] buffer, blk_out [B,H,S,D] or [B,S,H,D], blk_lse [B,H,S]):
+// True when the kernel was enqueued.  merge(None, None, blk_out [B,H,S,D], blk_lse): new accumulators (out, lse) holding the block.
+PyObject* py_merge(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Tensor acc, lse, blk, bl;
+  if (n != 4 || !optional_tensor(a[0], acc) || !optional_tensor(a[1], lse) || !tensor_arg(a[2], blk) || !tensor_arg(a[3], bl)) Py_RETURN_NONE;
+  const bool first = !acc.defined();
+  const int dtype = dtype_code(blk.scalar_type());
+  View x, y;
+  if (!blk.is_cuda() || !on_device(bl, blk) || dtype < 0 || blk.dim() != 4 || bl.dim() != 3 || bl.scalar_type() != at::kFloat || !bl.is_contiguous() ||
+      !rows_ok(blk) || first != !lse.defined())
+    Py_RETURN_NONE;
+  if (!first) {
+    // (a block whose dims 1, 2 are those of the accumulator swapped is in operator layout)
+    const bool bhsd = acc.dim() == 4 && blk.size(1) != acc.size(1) && blk.size(2) == acc.size(1);
+    if (acc.dim() != 4 || lse.dim() != 4 || !on_device(acc, blk) || !on_device(lse, blk) || acc.scalar_type() != at::kFloat ||
+        lse.scalar_type() != at::kFloat || !rows_ok(acc) || !view_of(acc, true, x) || !view_of(blk, !bhsd, y) || !x.same_shape(y) || lse.size(0) != x.B ||
+        lse.size(1) != x.S || lse.size(2) != x.H || lse.size(3) != 1 || (x.B > 1 && lse.stride(0) != (int64_t)x.H * x.S) ||
+        (x.S > 1 && lse.stride(1) != 1) || (x.H > 1 && lse.stride(2) != x.S))
+      Py_RETURN_NONE;
+  } else if (!view_of(blk, false, y)) {
+    Py_RETURN_NONE;
+  }
+  if (bl.size(0) != y.B || bl.size(1) != y.H || bl.size(2) != y.S) Py_RETURN_NONE;
+  int rc;
+  {
+    pybind11::gil_scoped_release no_gil;
+    void* const stream = current_stream();
+    const c10::DeviceGuard guard(blk.device());
+    if (first) {
+      acc = empty_f32({y.B, y.S, y.H, y.D}, blk);
+      lse = empty_f32({y.B, y.H, y.S}, blk);
+      view_of(acc, true, x);
+    }
+    rc = spa_merge((float*)x.p, (float*)lse.data_ptr(), y.p, (const float*)bl.const_data_ptr(), x.B, x.H, x.S, x.D, x.st, y.st, dtype, first, stream);
+    if (first) lse = lse.transpose(1, 2).unsqueeze(-1);
+  }
+  if (rc != SPA_OK) Py_RETURN_NONE;
+  if (first) return pair(acc, lse);
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
+#define FAST(name, fn) {name, (PyCFunction)(void (*)(void))fn, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {FAST("flash_fwd", py_flash_fwd), FAST("varlen_fwd", py_varlen_fwd), FAST("attention", py_attention),
+                         FAST("varlen_attention", py_varlen_attention), FAST("merge", py_merge), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module); }

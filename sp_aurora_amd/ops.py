@@ -136,6 +136,12 @@ def flash_fwd(q, k, v, softmax_scale=None, causal=False, layout="bshd", out=None
     of flash_fwd_splitkv_workspace(...) bytes; allocated here when not given, except while the stream is being captured,
     where "auto" then does not split).  With up to three query rows and no mask the library runs a kernel that streams K and V
     past the rows instead of the matrix-instruction kernel, split or not."""
+    if out is None and lse is None and workspace is None and split_kv == "auto" and layout in ("bshd", "bhsd"):
+        nat = _lib.native()
+        if nat is not None:
+            res = nat.flash_fwd(q, k, v, softmax_scale, causal, layout == "bshd", q_scale, k_scale, v_scale, _DT.get(out_dtype, -1))
+            if res is not None:
+                return res
     lib = _lib.load()
     fp8 = k.dtype == FP8 or v.dtype == FP8
     if q.dtype == FP8:
@@ -575,7 +581,7 @@ def check_cu_seqlens_once(cu, total, max_seqlen, what):
     While the current stream is being captured nothing is read (a synchronous copy is illegal
     there): the caller of a captured region vouches for its offsets.  Returns True when the array
     is known to be good, False when the check was skipped."""
-    key = (cu.data_ptr(), cu._version, cu.numel(), str(cu.device), int(total), int(max_seqlen))
+    key = (cu.data_ptr(), cu._version, cu.numel(), cu.device, int(total), int(max_seqlen))
     if key in _CU_CHECKED:
         return True
     if cu.is_cuda and torch.cuda.is_current_stream_capturing():
@@ -647,6 +653,12 @@ def flash_fwd_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seql
     cu_seqlens_* int32 [nseq+1] on the device.  Returns (out like q, lse fp32 [H,total_q]).
     Calls spa_flash_fwd_varlen, or spa_flash_fwd_varlen_fp8kv when k, v are torch.float8_e4m3fn
     (k_scale, v_scale: fp32 [nseq, H])."""
+    if out is None and lse is None:
+        nat = _lib.native()
+        if nat is not None:
+            res = nat.varlen_fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal, k_scale, v_scale)
+            if res is not None:
+                return res
     lib = _lib.load()
     fp8 = k.dtype == FP8 or v.dtype == FP8
     if fp8:

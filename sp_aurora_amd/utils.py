@@ -10,7 +10,7 @@ from functools import cache
 
 import torch
 
-from . import ops
+from . import _lib, ops
 
 __all__ = ["update_out_and_lse", "get_default_args", "flatten_varlen_lse", "unflatten_varlen_lse"]
 
@@ -52,6 +52,13 @@ def update_out_and_lse(out, lse, block_out, block_lse, slice_=None):
     the same).  block_out may come in operator layout [B,H,S,D] or already as [B,S,H,D]; as in
     the reference (:133-137) it is taken as [B,H,S,D] when its dims 1,2 are those of out swapped.
     """
+    if slice_ is None:
+        # (None: a shape or layout that needs a look, or an error to be raised, below)
+        nat = _lib.native()
+        if nat is not None:
+            res = nat.merge(out, lse, block_out, block_lse)
+            if res is not None:
+                return (out, lse) if out is not None else res
     if out is None:
         if slice_ is not None:
             raise RuntimeError("first update_out_and_lse should not pass slice_ args")

@@ -25,7 +25,7 @@ with c > r the second halves of the queries against both halves of the chunk.
 """
 import torch
 
-from . import ops
+from . import _lib, ops
 from .flash_attn import _check_unsupported
 from .ring import _no_multi_gpu
 
@@ -311,6 +311,11 @@ def sp_aurora_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k=None, max_seqlen=N
         raise ValueError("cu_seqlens_q and cu_seqlens_k must describe the same number of sequences")
     # rows of no sequence are not written by the backward kernels: gradients start as zeros unless the look
     # above has shown that the offsets cover every row
+    nat = _lib.native()
+    if nat is not None:
+        res = nat.varlen_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen, max_seqlen_k, softmax_scale, causal, covered)
+        if res is not None:
+            return (res[0], res[1], None) if return_attn_probs else res[0]
     return VarlenFlashAttnFunc.apply(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen, max_seqlen_k, softmax_scale,
                                      causal, return_attn_probs, covered)
 

@@ -1,0 +1,80 @@
+"""The host path of the public calls (_native): every way of packing the operands, rings as one block call, what it hands on to
+the Python path.  Against the oracle's full attention, tolerances of test_gpu_parity."""
+import pytest
+import torch
+
+from conftest import rand_qkv
+from oracle import attn_oracle as O
+import sp_aurora_amd as spa
+from sp_aurora_amd import _lib, ops
+from test_gpu_parity import DEV, check_grad, check_lse, check_out
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ring,S,D,dtype,causal", [(1, 67, 64, torch.float16, True), (3, 99, 128, torch.bfloat16, True),
+                                                   (4, 148, 64, torch.bfloat16, False), (2, 130, 32, torch.float32, True)])
+@pytest.mark.parametrize("packing", ["q,k,v", "q,kv", "qkv"])
+def test_every_packing_of_the_operands(packing, ring, S, D, dtype, causal):
+    B, H = 2, 3
+    q, k, v, dout = rand_qkv((B, S, H, D), 700 + S, dtype, n=4)
+    want, want_lse = O.full_attention(q, k, v, None, causal)
+    want_grads = O.attn_backward_autograd(q, k, v, dout, None, causal)
+    if packing == "q,k,v":
+        leaves = [t.to(DEV).requires_grad_() for t in (q, k, v)]
+        fn, split = spa.sp_aurora_func, lambda g: g
+    elif packing == "q,kv":
+        leaves = [q.to(DEV).requires_grad_(), torch.stack([k, v], 2).to(DEV).requires_grad_()]
+        fn, split = spa.sp_aurora_kvpacked_func, lambda g: (g[0], g[1][:, :, 0], g[1][:, :, 1])
+    else:
+        leaves = [torch.stack([q, k, v], 2).to(DEV).requires_grad_()]
+        fn, split = spa.sp_aurora_qkvpacked_func, lambda g: tuple(g[0][:, :, i] for i in range(3))
+    assert _lib.native().attention(*leaves, None, causal) is not None  # a call this path takes
+    out, lse, _ = fn(*leaves, causal=causal, return_attn_probs=True, ring_size=ring)
+    assert not lse.requires_grad
+    check_out(out, want, dtype)
+    check_lse(lse, want_lse)
+    for g in (dout.to(DEV), dout.to(DEV).transpose(1, 3).contiguous().transpose(1, 3)):  # a dout the kernels cannot read as it is, too
+        grads = split(torch.autograd.grad(out, leaves, g, retain_graph=True))
+        for got, w, name in zip(grads, want_grads, "qkv"):
+            check_grad(got, w, dtype, "d" + name)
+    with torch.no_grad():
+        assert torch.equal(fn(*leaves, causal=causal, ring_size=ring), out)
+
+
+def test_calls_that_need_more_than_the_native_path_still_run():
+    q, k, v = rand_qkv((1, 40, 2, 64), 710, torch.bfloat16)
+    want, _ = O.full_attention(q, k, v, 0.3, True)
+    wide = torch.zeros(1, 40, 2, 67, dtype=torch.bfloat16, device=DEV)
+    wide[..., 3:] = q.to(DEV)
+    odd = wide[..., 3:]  # rows that are not 16-byte aligned: copied by the Python path
+    assert _lib.native().attention(odd, k.to(DEV), v.to(DEV), 0.3, True) is None
+    check_out(spa.sp_aurora_func(odd, k.to(DEV), v.to(DEV), softmax_scale=0.3, causal=True), want, torch.bfloat16)
+    with pytest.raises(ValueError):
+        spa.sp_aurora_func(q, k, v)  # CPU tensors
+    with pytest.raises((TypeError, ValueError)):
+        spa._flash_attn_forward(q.to(DEV), k.to(DEV), v.to(DEV).float())
+    with pytest.raises(ValueError):
+        spa.sp_aurora_func(q.to(DEV), k.to(DEV), v.to(DEV), ring_size=3)  # does not divide the sequence
+    with pytest.raises(ValueError):
+        spa.sp_aurora_func(q.to(DEV), k.to(DEV), v.to(DEV), sharding="striped")
+
+
+@pytest.mark.parametrize("S,H", [(33, 3), (4, 4)])  # (4, 4): a block whose two layouts have one shape is taken as [B,S,H,D]
+def test_merge_of_two_blocks(S, H):
+    B, D, dtype = 2, 64, torch.bfloat16
+    q, = rand_qkv((B, H, S, D), 720, dtype, n=1)
+    k, v = rand_qkv((B, H, 2 * S, D), 721, dtype, n=2)
+    want, want_lse = O.attn_block(q, k, v, None, False)
+    out = lse = None
+    for i in range(2):
+        part = slice(i * S, (i + 1) * S)
+        blk, blk_lse = spa._flash_attn_forward(q.to(DEV), k[:, :, part].to(DEV), v[:, :, part].to(DEV))
+        if i == 0:
+            out, lse = spa.update_out_and_lse(None, None, blk, blk_lse)
+            assert out.shape == (B, S, H, D) and lse.shape == (B, S, H, 1) and out.dtype == lse.dtype == torch.float32
+        else:
+            o2, l2 = spa.update_out_and_lse(out, lse, blk if S != H else blk.transpose(1, 2), blk_lse)
+            assert o2 is out and l2 is lse
+    check_out(out.transpose(1, 2), want, dtype)
+    check_lse(lse.squeeze(-1).transpose(1, 2), want_lse)
