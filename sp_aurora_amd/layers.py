@@ -16,6 +16,7 @@ from enum import Enum
 
 import torch
 
+from . import _lib
 from .flash_attn import _check_unsupported
 from .ring import _no_multi_gpu, ring_flash_attn_func
 from .ulysses import SeqAllToAll4D, ulysses_flash_attn_func
@@ -195,6 +196,16 @@ class LongContextAttention(torch.nn.Module):
             raise ValueError(f"heads {H} must be divisible by the Ulysses degree {U}")
         if softmax_scale is None:
             softmax_scale = D ** (-0.5)
+
+        if B == 1 and query.shape == key.shape == value.shape:
+            # one batch entry: the stacked shards are the whole sequence, and neither the exchange (which head slice is
+            # where) nor the ring (in which order the blocks are visited) changes what is computed from it
+            nat = _lib.native()
+            res = nat.attention(query, key, value, softmax_scale, causal) if nat is not None else None
+            if res is not None:
+                if self.use_sync:
+                    torch.cuda.synchronize()
+                return res[0]
 
         if U == 1:
             # ring only (:198-213): the stacked shards are the ring's chunks
