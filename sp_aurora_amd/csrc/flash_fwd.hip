@@ -620,77 +620,63 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, 1) flash_fwd16_kernel(const 
         }
     }
 
-    // row max of the lane's 32 NT scores: 3-input maxima, two independent chains per 32-key tile.
-    // (Through the instruction itself: fmaxf() makes the compiler quiet possible signalling NaNs
-    // first, one extra instruction per MFMA result; the scores are finite or -inf here.)
-    auto max3 = [](float a, float b, float c3) {
-      float r;
-      asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c3));
-      return r;
+    // P = exp2(s c - m c) against the reference max m of the row as it stands, and the lane's share of the row sum.
+    // m only has to keep P in range, so the maximum of the new scores is not formed unless it is needed (15 three-input
+    // maxima, an exchange with the other half and a comparison saved of ~190 vector instructions a sub-tile): a score that
+    // outgrows m by more than 2^8 shows in the sum, and so does a row that has seen no key yet (m = -inf: infinite or not a
+    // number).  Until then P <= 256, harmless in fp32 sums and 16-bit operands.
+    float lp;
+    auto exponentials = [&](float mc) {
+      float ps[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          float e[8];
+#pragma unroll
+          for (int x = 0; x < 8; ++x) {
+            e[x] = fast_exp2(__builtin_fmaf(s[t][8 * u + x], c, -mc));
+            ps[x & 3] += e[x];
+          }
+          pfr[t][u] = M::pack(e[0], e[1], e[2], e[3], e[4], e[5], e[6], e[7]);
+        }
+      lp = (ps[0] + ps[1]) + (ps[2] + ps[3]);
     };
-    float mxa[NT], mxb[NT];
+    exponentials(m_run * c);
+    if (__builtin_amdgcn_ballot_w64(!(lp <= 256.f)) != 0) {
+      // row max of the lane's 16 NT scores: 3-input maxima, two independent chains per 32-key tile.
+      // (Through the instruction itself: fmaxf() makes the compiler quiet possible signalling NaNs
+      // first, one extra instruction per MFMA result; the scores are finite or -inf here.)
+      auto max3 = [](float a, float b, float c3) {
+        float r;
+        asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c3));
+        return r;
+      };
+      float mx = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      mxa[t] = max3(s[t][0], s[t][1], s[t][2]);
-      mxb[t] = max3(s[t][8], s[t][9], s[t][10]);
-    }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      mxa[t] = max3(mxa[t], s[t][3], s[t][4]);
-      mxb[t] = max3(mxb[t], s[t][11], s[t][12]);
-    }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      mxa[t] = max3(mxa[t], s[t][5], s[t][6]);
-      mxb[t] = max3(mxb[t], s[t][13], s[t][14]);
-    }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) mxa[t] = max3(mxa[t], s[t][7], mxb[t]);
-    float mx;
-    if constexpr (NT == 2) {
-      mx = max3(mxa[0], mxa[1], fmaxf(s[0][15], s[1][15]));
-    } else {
-      static_assert(NT == 4, "sub-tiles of 64 or 128 keys");
-      const float u = max3(mxa[0], mxa[1], s[0][15]), w2 = max3(mxa[2], mxa[3], s[1][15]);
-      mx = max3(u, w2, fmaxf(s[2][15], s[3][15]));
-    }
-    mx = halves_max(mx);
-    // Lazy rescale: the reference max only moves when some row's max grew by more than
-    // 2^8 in the exp2 domain; until then P <= 256, harmless in fp32 sums and bf16 operands.
-    if (__builtin_amdgcn_ballot_w64((mx - m_run) * c > 8.f) != 0) {
-      const float m_new = fmaxf(m_run, mx);
-      // (a lane whose row has seen no key yet, here or before, while another row of the wave asks for the
-      // rescale: -inf - -inf; nothing of that row needs scaling.  Rows of a wave differ in this only when
-      // the tile's first row is not a multiple of the sub-tile size: the second half of a zigzag shard.)
-      const float alpha = ZZ && m_new == -INFINITY ? 1.f : fast_exp2((m_run - m_new) * c);
+      for (int t = 0; t < NT; ++t) {
+        float ma = max3(s[t][0], s[t][1], s[t][2]), mb = max3(s[t][8], s[t][9], s[t][10]);
+        ma = max3(ma, s[t][3], s[t][4]);
+        mb = max3(mb, s[t][11], s[t][12]);
+        ma = max3(ma, s[t][5], s[t][6]);
+        mb = max3(mb, s[t][13], s[t][14]);
+        ma = max3(ma, s[t][7], mb);
+        mx = max3(mx, ma, s[t][15]);
+      }
+      const float m_new = fmaxf(m_run, halves_max(mx));
+      // (a row that has seen no key yet, here or before: -inf - -inf; nothing of it needs scaling)
+      const float alpha = m_new == -INFINITY ? 1.f : fast_exp2((m_run - m_new) * c);
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
       for (int d = 0; d < D / 32; ++d)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
+      exponentials(m_run == -INFINITY ? 0.f : m_run * c);
     }
-    // a row that has seen no key yet (a ragged chunk can leave a whole sub-tile empty) keeps m = -inf
-    const float mc = m_run == -INFINITY ? 0.f : m_run * c;
-
-    float ps[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const float e = fast_exp2(__builtin_fmaf(s[t][v], c, -mc));
-        s[t][v] = e;
-        ps[v & 3] += e;
-      }
-    l_run += (ps[0] + ps[1]) + (ps[2] + ps[3]);
+    l_run += lp;
     asm volatile("" : "+v"(l_run));  // keep the row sum in this phase as well (see below)
 
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-        pfr[t][u] = M::pack(s[t][8 * u + 0], s[t][8 * u + 1], s[t][8 * u + 2], s[t][8 * u + 3],
-                            s[t][8 * u + 4], s[t][8 * u + 5], s[t][8 * u + 6], s[t][8 * u + 7]);
     // P must exist in registers when the phase ends: without this the compiler sinks the
     // exponentials past the barrier into the MFMA phase they are meant to overlap with.
 #pragma unroll
