@@ -210,6 +210,27 @@ __device__ __forceinline__ void select_sequence(BwdParams& p, int& b) {
   b = 0;
 }
 
+// The (batch or sequence, head) and the tile (of `rows` query rows, or keys) of a workgroup: pairs first, in groups
+// (spa_head_groups), or, for a packed batch, heads first and then the tiles of all sequences (sequence_tile).  The tiles that
+// see the most of the other side go first: with a causal mask the last query tiles and the first key tiles.
+__device__ __forceinline__ bool workgroup_tile(const BwdParams& p, bool queries, int rows, int lane, int& b, int& h, int& tile) {
+  int n;
+  if (p.cu_q) {
+    const int number = blockIdx.x / p.H;
+    h = blockIdx.x - number * p.H;
+    if (!sequence_tile(queries ? p.cu_q : p.cu_k, p.B, rows, number, lane, b, tile, n)) return false;
+  } else {
+    const int pair = blockIdx.x + blockIdx.z * gridDim.x;
+    if (pair >= p.B * p.H) return false;
+    h = pair % p.H;
+    b = pair / p.H;
+    tile = blockIdx.y;
+    n = gridDim.y;
+  }
+  if (queries) tile = n - 1 - tile;
+  return true;
+}
+
 // A row of a gradient that is written (BwdParams::grads_in_t) and that no tile contributes to: the
 // lane's share of the row (the columns the epilogues give it) is set to zero.
 template <typename E, int D>
@@ -246,11 +267,8 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_dq_kernel(const BwdParam
   const int lane = tid & 63, ln = lane & 31, hh = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  int bid = blockIdx.x;
-  const int bh = bid % (p.B * p.H);  // (batch, head) pairs first: each keeps to one XCD also when H < 8
-  const int h = bh % p.H;
-  int b = bh / p.H;
-  const int qt = p.nqt - 1 - bid / (p.B * p.H);
+  int b, h, qt;
+  if (!workgroup_tile(p, true, NW * 32, lane, b, h, qt)) return;
   const int q0 = qt * (NW * 32);
   const int qw0 = q0 + w * 32;
   select_sequence<T>(p, b);
@@ -518,11 +536,8 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd_dkdv_kernel(const Bw
   const int lane = tid & 63, ln = lane & 31, hh = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  int bid = blockIdx.x;
-  const int bh = bid % (p.B * p.H);  // (batch, head) pairs first: each keeps to one XCD also when H < 8
-  const int h = bh % p.H;
-  int b = bh / p.H;
-  const int kt = bid / (p.B * p.H);  // causal: low key tiles see the most query tiles, they go first
+  int b, h, kt;
+  if (!workgroup_tile(p, false, 128, lane, b, h, kt)) return;
   const int k0 = kt * 128;
   const int kw0 = k0 + w * 32;
   select_sequence<T>(p, b);
@@ -864,11 +879,8 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dq_kernel(const Bw
   const int tid = threadIdx.x;
   const int lane = tid & 63, w = tid >> 6, ln = lane & 31, hh = lane >> 5;
 
-  int bid = blockIdx.x;
-  const int bh = bid % (p.B * p.H);  // (batch, head) pairs first: each keeps to one XCD also when H < 8
-  const int h = bh % p.H;
-  int b = bh / p.H;
-  const int qt = p.nqt - 1 - bid / (p.B * p.H);
+  int b, h, qt;
+  if (!workgroup_tile(p, true, 128, lane, b, h, qt)) return;
   const int q0 = qt * 128;
   const int qw0 = q0 + w * 32;
   select_sequence<float>(p, b);
@@ -974,11 +986,8 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
   const int tid = threadIdx.x;
   const int lane = tid & 63, w = tid >> 6, ln = lane & 31, hh = lane >> 5;
 
-  int bid = blockIdx.x;
-  const int bh = bid % (p.B * p.H);  // (batch, head) pairs first: each keeps to one XCD also when H < 8
-  const int h = bh % p.H;
-  int b = bh / p.H;
-  const int kt = bid / (p.B * p.H);
+  int b, h, kt;
+  if (!workgroup_tile(p, false, 128, lane, b, h, kt)) return;
   const int k0 = kt * 128;
   const int kw0 = k0 + w * 32;
   select_sequence<float>(p, b);
@@ -1126,44 +1135,48 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
   }
 }
 
+// `rows` query rows, or keys, per workgroup.
 template <auto kernel>
-hipError_t launch(int smem, unsigned blocks, const BwdParams& p, hipStream_t stream, int threads = BWD_THREADS) {
+hipError_t launch(int smem, bool queries, int rows, const BwdParams& p, hipStream_t stream, int threads = BWD_THREADS) {
   const hipError_t e = spa_allow_dynamic_lds<kernel>(smem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), smem, stream, p);
+  dim3 grid;
+  if (p.cu_q) {
+    if (!spa_varlen_grid(p.H, p.B, queries ? p.lse_bh : p.total_k, rows, 1, grid)) return hipErrorInvalidValue;
+  } else {
+    const int tiles = ((queries ? p.Sq : p.Sk) + rows - 1) / rows;
+    if (tiles > 65535) return hipErrorInvalidValue;
+    grid = spa_head_groups((int64_t)p.B * p.H, tiles);
+  }
+  hipLaunchKernelGGL(kernel, grid, dim3(threads), smem, stream, p);
   return hipGetLastError();
 }
 
 template <typename T, int D>
 hipError_t launch_both(const BwdParams& p, hipStream_t stream) {
-  const unsigned kblocks = (unsigned)((int64_t)p.B * p.H * p.nkt);
   // dq kernel: 256-row workgroups (two waves per SIMD, the K/V stream shared by twice the rows) once
   // there are enough of them to occupy every CU; spa_tune() can force 4 or 8 waves (experiments, tests)
-  const int nqt8 = (p.Sq + 255) / 256;
+  const int64_t wgs8 = p.cu_q ? (int64_t)p.H * (p.lse_bh / 256 + (p.B + 1) / 2) : (int64_t)p.B * p.H * ((p.Sq + 255) / 256);
   const int forced = spa_knob(SPA_KNOB_BWD_DQ_WAVES);
   hipError_t e = hipErrorInvalidValue;
   bool wide = false;
   if constexpr (D >= 64) {  // a D = 32 tile has fewer 16-byte slots than 512 threads
-    wide = forced ? forced == 8 : (int64_t)p.B * p.H * nqt8 >= spa_device_cus();
-    if (wide) {
-      BwdParams p8 = p;
-      p8.nqt = nqt8;
-      e = launch<flash_bwd_dq_kernel<T, D, 8>>(DqCfg<D, 8>::SMEM, (unsigned)((int64_t)p.B * p.H * nqt8), p8, stream, 512);
-    }
+    wide = forced ? forced == 8 : wgs8 >= spa_device_cus();
+    if (wide) e = launch<flash_bwd_dq_kernel<T, D, 8>>(DqCfg<D, 8>::SMEM, true, 256, p, stream, 512);
   }
-  if (!wide) e = launch<flash_bwd_dq_kernel<T, D, 4>>(DqCfg<D, 4>::SMEM, (unsigned)((int64_t)p.B * p.H * p.nqt), p, stream);
+  if (!wide) e = launch<flash_bwd_dq_kernel<T, D, 4>>(DqCfg<D, 4>::SMEM, true, 128, p, stream);
   if (e != hipSuccess) return e;
   if constexpr (D == 128)
-    if (spa_knob(SPA_KNOB_BWD_DKDV_FORM) == 1) return launch<flash_bwd_dkdv_kernel<T, D, false>>(DkvCfg<D>::SMEM, kblocks, p, stream);
-  return launch<flash_bwd_dkdv_kernel<T, D>>(DkvCfg<D>::SMEM, kblocks, p, stream);
+    if (spa_knob(SPA_KNOB_BWD_DKDV_FORM) == 1) return launch<flash_bwd_dkdv_kernel<T, D, false>>(DkvCfg<D>::SMEM, false, 128, p, stream);
+  return launch<flash_bwd_dkdv_kernel<T, D>>(DkvCfg<D>::SMEM, false, 128, p, stream);
 }
 
 // A tensor of 2 GiB or more per (batch, head): the re-based variants, 128-row dq workgroups.
 template <typename T, int D>
 hipError_t launch_both_big(const BwdParams& p, hipStream_t stream) {
-  const hipError_t e = launch<flash_bwd_dq_kernel<T, D, 4, true>>(DqCfg<D, 4>::SMEM, (unsigned)((int64_t)p.B * p.H * p.nqt), p, stream);
+  const hipError_t e = launch<flash_bwd_dq_kernel<T, D, 4, true>>(DqCfg<D, 4>::SMEM, true, 128, p, stream);
   if (e != hipSuccess) return e;
-  return launch<flash_bwd_dkdv_kernel<T, D, true, true>>(DkvCfg<D>::SMEM, (unsigned)((int64_t)p.B * p.H * p.nkt), p, stream);
+  return launch<flash_bwd_dkdv_kernel<T, D, true, true>>(DkvCfg<D>::SMEM, false, 128, p, stream);
 }
 
 }  // namespace
@@ -1188,8 +1201,6 @@ hipError_t spa_launch_bwd16_big(const BwdParams& p, int D, int dtype, hipStream_
 
 // Returns hipSuccess, or hipErrorInvalidValue for an unsupported (dtype, D).
 hipError_t spa_launch_flash_bwd(BwdParams p, int D, int dtype, hipStream_t stream) {
-  p.nqt = (p.Sq + 127) / 128;
-  p.nkt = (p.Sk + 127) / 128;
   if (p.big && dtype != 0) return spa_launch_bwd16_big(p, D, dtype, stream);
   if (dtype == 1) {
     if (D == 128) return launch_both<__bf16, 128>(p, stream);
@@ -1200,16 +1211,14 @@ hipError_t spa_launch_flash_bwd(BwdParams p, int D, int dtype, hipStream_t strea
     if (D == 64) return launch_both<_Float16, 64>(p, stream);
     if (D == 32) return launch_both<_Float16, 32>(p, stream);
   } else if (dtype == 0) {
-    const unsigned qblocks = (unsigned)((int64_t)p.B * p.H * p.nqt);
-    const unsigned kblocks = (unsigned)((int64_t)p.B * p.H * p.nkt);
     hipError_t e = hipErrorInvalidValue;
-    if (D == 128) e = launch<flash_bwd32_dq_kernel<128>>(Bwd32Cfg<128>::SMEM_DQ, qblocks, p, stream);
-    if (D == 64) e = launch<flash_bwd32_dq_kernel<64>>(Bwd32Cfg<64>::SMEM_DQ, qblocks, p, stream);
-    if (D == 32) e = launch<flash_bwd32_dq_kernel<32>>(Bwd32Cfg<32>::SMEM_DQ, qblocks, p, stream);
+    if (D == 128) e = launch<flash_bwd32_dq_kernel<128>>(Bwd32Cfg<128>::SMEM_DQ, true, 128, p, stream);
+    if (D == 64) e = launch<flash_bwd32_dq_kernel<64>>(Bwd32Cfg<64>::SMEM_DQ, true, 128, p, stream);
+    if (D == 32) e = launch<flash_bwd32_dq_kernel<32>>(Bwd32Cfg<32>::SMEM_DQ, true, 128, p, stream);
     if (e != hipSuccess) return e;
-    if (D == 128) return launch<flash_bwd32_dkdv_kernel<128>>(Bwd32Cfg<128>::SMEM_DKV, kblocks, p, stream);
-    if (D == 64) return launch<flash_bwd32_dkdv_kernel<64>>(Bwd32Cfg<64>::SMEM_DKV, kblocks, p, stream);
-    if (D == 32) return launch<flash_bwd32_dkdv_kernel<32>>(Bwd32Cfg<32>::SMEM_DKV, kblocks, p, stream);
+    if (D == 128) return launch<flash_bwd32_dkdv_kernel<128>>(Bwd32Cfg<128>::SMEM_DKV, false, 128, p, stream);
+    if (D == 64) return launch<flash_bwd32_dkdv_kernel<64>>(Bwd32Cfg<64>::SMEM_DKV, false, 128, p, stream);
+    if (D == 32) return launch<flash_bwd32_dkdv_kernel<32>>(Bwd32Cfg<32>::SMEM_DKV, false, 128, p, stream);
   }
   return hipErrorInvalidValue;
 }

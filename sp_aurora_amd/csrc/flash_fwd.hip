@@ -62,6 +62,7 @@ struct Fwd16Cfg {
   static constexpr int EPI = (NG * FWD_BM * (D + 4) + NG * FWD_BM * 2 + BMW) * 4;  // epilogue staging
   static constexpr int TILES = SHARE ? GROUP : NG * GROUP;
   static constexpr int SMEM = TILES > EPI ? TILES : EPI;
+  static constexpr int SMEM_PLAIN = NG == 1 ? TILES : SMEM;  // one group writes a plain result from its registers
   static constexpr int CPR = D / 8;                         // 16-byte chunks per row
   static constexpr int DTHREADS = SHARE ? NG * FWD_THREADS : FWD_THREADS;  // threads filling one buffer
   static constexpr int NDMA = TILEB / (DTHREADS * 16);      // direct loads per thread and sub-tile
@@ -107,7 +108,7 @@ __device__ __forceinline__ int v_swizzle(int row) {
 // lie a shard apart, not a sequence length apart.
 template <typename T, int D, int NG, bool SHARE, bool KV8 = false, bool FINALN = false, bool ZZ = false, bool BIG = false,
           bool QK8 = false, bool WAIT = false, bool KS = false, bool VR = false>
-__global__ void __launch_bounds__(FWD_THREADS * NG, 1) flash_fwd16_kernel(const FwdParams pk) {
+__global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) flash_fwd16_kernel(const FwdParams pk) {
   static_assert(!(FINALN && SHARE), "the merging epilogue goes with 128-row workgroups");
   static_assert(!KS || (!SHARE && !FINALN && !ZZ && !BIG && !QK8 && !WAIT), "split keys: 128-row workgroups, plain results");
   static_assert(!QK8 || (KV8 && D == 128 && !ZZ && !BIG), "8-bit scores: e4m3 q, k, v, head dim 128, contiguous chunks");
@@ -132,15 +133,28 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, 1) flash_fwd16_kernel(const 
   // Consecutive workgroup ids walk the (batch, head) pairs first: with round-robin placement of
   // workgroups on the 8 XCDs, all query tiles of a head share one XCD's L2 for K/V.
   // Then query tiles and ranks, heaviest first.
-  // (grid.x = (batch, head) pairs, grid.y = query tiles, grid.z = ranks: workgroups are dispatched
-  // x first, and the decomposition costs no divisions)
-  const int bh = blockIdx.x;  // (batch, head) pairs first: each keeps to one XCD also when H < 8
-  const int h = bh % p.H;
-  int b = bh / p.H;
+  // (grid.x = (batch, head) pairs, grid.y = query tiles, grid.z = ranks, or, for one rank, groups of pairs
+  // (spa_head_groups): workgroups are dispatched x first, and the decomposition costs no divisions)
+  int b, h, qt;
+  if (p.cu_q) {
+    // a packed batch: heads first, then the tiles of all sequences (sequence_tile), each sequence's heaviest first
+    const int number = blockIdx.x / p.H;
+    h = blockIdx.x - number * p.H;
+    int nt = 0;
+    if (!sequence_tile(p.cu_q, p.B, C::BMW, number, lane, b, qt, nt)) return;
+    qt = nt - 1 - qt;
+  } else {
+    const int pair = blockIdx.x + (p.nranks == 1 ? blockIdx.z * gridDim.x : 0u);
+    if (pair >= p.B * p.H) return;  // the last group's remainder
+    h = pair % p.H;
+    b = pair / p.H;
+    qt = p.nqt - 1 - (int)blockIdx.y;
+  }
+  const int zrank = p.nranks == 1 ? 0 : (int)blockIdx.z;
+  const int bh = b * p.H + h;
   // dequantisation scales of this (batch or sequence, head): K = k8 * ksc, V = v8 * vsc
   const float ksc = KV8 ? p.k_scale[bh] * (QK8 ? p.q_scale[bh] : 1.f) : 1.f;  // (with e4m3 q its scale rides along)
   const float vsc = KV8 ? p.v_scale[bh] : 1.f;
-  const int qt = p.nqt - 1 - (int)blockIdx.y;
   // Zigzag shards: the tiles of the two halves of the chunk are laid out one half after the other (a tile
   // never holds rows of both), the second (heavier) half first in dispatch order.
   constexpr bool zz = ZZ;
@@ -150,7 +164,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, 1) flash_fwd16_kernel(const 
   const int q0 = zz ? (zhalf ? zz_hs : 0) + (qt - (zhalf && !p.zz_half ? zz_nqh : 0)) * C::BMW : qt * C::BMW;
   // Ranks heaviest first: the last rank with contiguous chunks.  With zigzag shards the second half of a shard's
   // rows is heavier the lower the rank and the first half the higher, and every grid plane z holds the same work.
-  const int rank = zz && zhalf ? p.rank0 + (int)blockIdx.z : p.rank0 + p.nranks - 1 - (int)blockIdx.z;
+  const int rank = zz && zhalf ? p.rank0 + zrank : p.rank0 + p.nranks - 1 - zrank;
   // WAIT: the flag of the first chunk is requested before anything else (such a load takes microseconds; it is looked
   // at when the first tiles are about to be requested)
   auto flag_of = [&](int ch) { return __hip_atomic_load(p.arrive + ch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
@@ -171,7 +185,6 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, 1) flash_fwd16_kernel(const 
     p.out = (T*)p.out + (int64_t)q_lo * p.os.s;
     p.lse += q_lo;
     b = 0;
-    if (q0 >= p.Sq) return;  // this sequence is shorter than the longest one
     if (p.Sk <= 0) {
       // no keys: the empty sum, out = 0 and lse = -inf
       for (int idx = tid; idx < C::BMW * (D / 8); idx += FWD_THREADS * NG) {
@@ -795,7 +808,8 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, 1) flash_fwd16_kernel(const 
     for (int ks = 0; ks < NKA; ++ks) ka[ks] = kra[ks] + (unsigned)((PAR ^ 1) * C::TILEB);               // k_lds(i + 1)
     // Shared buffers need one barrier per step and group (after the wait for the loads: group 0
     // at the end of its VALU phase, group 1 at the end of its MFMA phase, the same physical
-    // barrier); the other one only holds the two groups in step, and they drift little without it.
+    // barrier); the other one only holds the two groups in step, and they drift little without it.  One group alone needs
+    // one as well: whoever has passed it knows that every wave is done with the MFMA phase before.
     if (!early) {
       loads_landed();
       store_staged((unsigned)((PAR ^ 1) * C::TILEB), (unsigned)(2 * C::TILEB + PAR * C::TILEB));  // K(i + 1), V(i)
@@ -821,7 +835,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, 1) flash_fwd16_kernel(const 
       loads_landed();
       store_staged(kb, vb);  // this group's share of K(i + 2), V(i + 1), loaded at the top of the step
     }
-    if (!SHARE || early) __syncthreads();
+    if ((!SHARE && NG > 1) || early) __syncthreads();
   };
   {
     int i = 0;
@@ -1127,9 +1141,20 @@ __global__ void __launch_bounds__(FWD_THREADS, 1) flash_fwd32_kernel(const FwdPa
   const int ln = lane & 31;
   const int hh = lane >> 5;
 
-  const int h = blockIdx.x % p.H;
-  int b = blockIdx.x / p.H;
-  const int qt = p.nqt - 1 - (int)blockIdx.y;
+  int b, h, qt;
+  if (p.cu_q) {
+    const int number = blockIdx.x / p.H;
+    h = blockIdx.x - number * p.H;
+    int nt = 0;
+    if (!sequence_tile(p.cu_q, p.B, FWD_BM, number, lane, b, qt, nt)) return;
+    qt = nt - 1 - qt;
+  } else {
+    const int pair = blockIdx.x + blockIdx.z * gridDim.x;
+    if (pair >= p.B * p.H) return;
+    h = pair % p.H;
+    b = pair / p.H;
+    qt = p.nqt - 1 - (int)blockIdx.y;
+  }
   const int q0 = qt * FWD_BM;
   const int qw0 = q0 + w * 32;
   if (p.cu_q) {
@@ -1142,7 +1167,6 @@ __global__ void __launch_bounds__(FWD_THREADS, 1) flash_fwd32_kernel(const FwdPa
     p.out = (float*)p.out + (int64_t)q_lo * p.os.s;
     p.lse += q_lo;
     b = 0;
-    if (q0 >= p.Sq) return;
     if (p.Sk <= 0) {
       for (int idx = tid; idx < FWD_BM * (D / 4); idx += FWD_THREADS) {
         const int grow = q0 + idx / (D / 4), ch = idx % (D / 4);
@@ -1339,8 +1363,10 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31;
   const int hh = lane >> 5;
-  const int h = blockIdx.x % p.H;
-  const int b = blockIdx.x / p.H;
+  const int bh = blockIdx.x + blockIdx.z * gridDim.x;
+  if (bh >= p.B * p.H) return;
+  const int h = bh % p.H;
+  const int b = bh / p.H;
   const int qt = p.nqt - 1 - (int)blockIdx.y;
   const int q0 = qt * 32;
   const float* qp = (const float*)p.q + b * p.qs.b + h * p.qs.h;
@@ -1491,12 +1517,19 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
   }
 }
 
+// `rows`: query rows per workgroup.
 template <auto kernel>
-hipError_t launch(int threads, int smem, const FwdParams& p, hipStream_t stream) {
+hipError_t launch(int threads, int smem, int rows, const FwdParams& p, hipStream_t stream) {
   const hipError_t e = spa_allow_dynamic_lds<kernel>(smem);
   if (e != hipSuccess) return e;
   if (p.nqt > 65535 || p.nranks > 65535) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)((int64_t)p.B * p.H), (unsigned)p.nqt, (unsigned)p.nranks);
+  const int64_t pairs = (int64_t)p.B * p.H;
+  dim3 grid;
+  if (p.cu_q) {
+    if (!spa_varlen_grid(p.H, p.B, p.lse_bh / p.P, rows, (unsigned)p.nranks, grid)) return hipErrorInvalidValue;
+  } else {
+    grid = p.nranks == 1 ? spa_head_groups(pairs, p.nqt) : dim3((unsigned)pairs, (unsigned)p.nqt, (unsigned)p.nranks);
+  }
   hipLaunchKernelGGL(kernel, grid, dim3(threads), smem, stream, p);
   return hipGetLastError();
 }
@@ -1509,52 +1542,92 @@ int fwd_tiles(const FwdParams& p, int bm) {
   return p.zz_half ? per_half : 2 * per_half;
 }
 
-// Two wave groups once there are at least two 64-key sub-tiles to split; 256-row workgroups with
-// shared K/V buffers once that still leaves every CU at least two workgroups.  spa_tune() can
-// force either choice (experiments and tests).
-template <typename T, int D, bool ZZ>
-hipError_t launch16(FwdParams p, hipStream_t stream) {
-  const int force = spa_knob(SPA_KNOB_FWD_GROUPS);
-  const int force_share = spa_knob(SPA_KNOB_FWD_SHARE);
-  const bool two = force ? force == 2 : p.Sk > fwd_bn<D>();
-  if (p.epi == SPA_EPI_FINALN) {
-    if (two) return launch<flash_fwd16_kernel<T, D, 2, false, false, true, ZZ>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, p, stream);
-    return launch<flash_fwd16_kernel<T, D, 1, false, false, true, ZZ>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM, p, stream);
+// The three forms of a workgroup: FWD_ONE, 128 rows by one wave group, two or three workgroups to a CU; FWD_SPLIT, 128 rows
+// by two groups that take alternate key tiles; FWD_SHARE, 256 rows by two groups on shared K/V buffers.
+enum FwdForm { FWD_ONE, FWD_SPLIT, FWD_SHARE, FWD_FORMS };
+
+// What a launch of a form takes, in us: the longer of its heaviest workgroup alone (`alone` per 64-key step) and of the whole
+// launch with every CU busy (`busy` per step and workgroup), the workgroup's fixed cost once per round of workgroups, and
+// the launch's own.  Fitted to 72 shapes per row (1 to 64 sequences of 200 to 16384 rows, 8 to 32 heads, with and without the causal
+// mask; residual 4 to 8 %): the form it picks is within 1 % of the best one on average, 8 % at worst.  What
+// decides: FWD_SHARE moves half the K/V bytes per product and is the fastest on long rows at D = 128 (1260 against 1180 TFLOP/s
+// at 8192 keys); FWD_ONE overlaps one workgroup's start and end with another's work and wins on short rows (64 sequences of
+// 512, causal: 506 against 427 TFLOP/s at D = 128), and everywhere at D = 64, where three waves to a SIMD hide the
+// softmax (8192 keys: 980 against 860); FWD_SPLIT halves the heaviest workgroup and wins while the grid does not fill the CUs.
+struct FormCost {
+  float alone, busy, round, fixed;
+};
+enum FwdKind { KIND_16, KIND_KV8, KIND_QK8 };  // 16-bit K/V; e4m3 K/V; e4m3 q, K/V
+float form_us(const FwdParams& p, FwdForm f, int D, FwdKind kind) {
+  static constexpr FormCost cost[4][FWD_FORMS] = {
+      {{0.98f, 0.96f, 5.1f, 2.0f}, {1.36f, 1.81f, 6.2f, 2.2f}, {1.24f, 1.67f, 8.9f, 0.5f}},    // 16 bits, D = 128
+      {{0.79f, 0.56f, 4.9f, 0.4f}, {1.03f, 1.18f, 4.1f, 2.2f}, {1.04f, 1.17f, 5.1f, 1.8f}},    // 16 bits, D <= 64
+      {{1.39f, 0.96f, 5.3f, 0.4f}, {1.68f, 1.91f, 6.0f, 2.7f}, {1.40f, 1.73f, 7.9f, 1.3f}},    // e4m3 K/V
+      {{1.11f, 0.75f, 4.6f, 0.4f}, {1.40f, 1.53f, 5.0f, 2.6f}, {1.16f, 1.38f, 6.6f, 1.4f}}};   // e4m3 q, K/V
+  const FormCost& c = cost[kind == KIND_QK8 ? 3 : kind == KIND_KV8 ? 2 : D > 64 ? 0 : 1][f];
+  const float rows = f == FWD_SHARE ? 2 * FWD_BM : FWD_BM, keys = f == FWD_SPLIT ? 128.f : 64.f;  // of a workgroup, of a step
+  const float slots = (float)spa_device_cus() * (f == FWD_ONE ? (D > 64 ? 2 : 3) : 1), cus = (float)spa_device_cus();
+  // sequences of a packed batch: as many rows as they have on average, the heaviest as many keys as the longest
+  float sq = (float)p.Sq, sk = (float)p.Sk, tiles = ceilf(sq / rows);
+  if (p.cu_q) {
+    sq = (float)p.lse_bh / (float)p.B;
+    sk = fminf(sk, fmaxf(sq, 1.f));
+    tiles = sq / rows + 0.5f;
   }
-  if (two && D >= 64) {
-    const int nqt2 = fwd_tiles(p, 2 * FWD_BM);
-    const int64_t wgs = (int64_t)p.B * p.H * nqt2 * p.nranks;
-    const bool share = force_share ? force_share == 2 : wgs >= 2 * (int64_t)spa_device_cus();
-    if (share) {
-      p.nqt = nqt2;
-      return launch<flash_fwd16_kernel<T, D, 2, (D >= 64), false, false, ZZ>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, (D >= 64)>::SMEM, p, stream);
-    }
+  const float heaviest = p.causal ? fminf((float)p.Sk, (float)p.Sq) : (float)p.Sk;
+  const float longest = ceilf(heaviest / keys), all = ceilf(sk / keys);
+  float mean = all;
+  if (p.causal) {  // tile t walks (t + 1) * rows keys, at most all of them
+    const float m = fminf(tiles, floorf(sk / rows));
+    mean = (rows / keys * m * (m + 1.f) * 0.5f + (tiles - m) * all) / tiles;
   }
-  if (two) return launch<flash_fwd16_kernel<T, D, 2, false, false, false, ZZ>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, p, stream);
-  return launch<flash_fwd16_kernel<T, D, 1, false, false, false, ZZ>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM, p, stream);
+  const float n = (float)p.B * (float)p.H * tiles;
+  // (equal workgroups end together: half of a last round that is not full is lost)
+  const float load = p.causal || p.cu_q ? n / cus : 0.5f * (n / cus + ceilf(n / cus));
+  return fmaxf(longest * c.alone, load * mean * c.busy) + c.round * fmaxf(1.f, n / slots) + c.fixed;
 }
 
-// e4m3 K/V: the register-staged variants, chosen like the 16-bit ones.
-template <typename T, int D, bool ZZ>
-hipError_t launch16_kv8(FwdParams p, hipStream_t stream) {
+FwdForm fwd_form(const FwdParams& p, int D, FwdKind kind) {
   const int force = spa_knob(SPA_KNOB_FWD_GROUPS);
   const int force_share = spa_knob(SPA_KNOB_FWD_SHARE);
-  const bool two = force ? force == 2 : p.Sk > fwd_bn<D>();
-  if (p.epi == SPA_EPI_FINALN) {
-    if (two) return launch<flash_fwd16_kernel<T, D, 2, false, true, true, ZZ>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, p, stream);
-    return launch<flash_fwd16_kernel<T, D, 1, false, true, true, ZZ>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM, p, stream);
+  const bool can_share = D >= 64 && p.epi != SPA_EPI_FINALN;
+  if (force ? force == 1 : p.Sk <= fwd_bn<128>()) return FWD_ONE;  // one sub-tile: nothing to split
+  if (force_share && can_share) return force_share == 2 ? FWD_SHARE : FWD_SPLIT;
+  if (p.P > 1 || p.zigzag || p.epi != SPA_EPI_PLAIN) {
+    // a ring schedule: 256-row workgroups once that still leaves every CU two of them
+    const int64_t wgs = (int64_t)p.B * p.H * fwd_tiles(p, 2 * FWD_BM) * p.nranks;
+    return can_share && wgs >= 2 * (int64_t)spa_device_cus() ? FWD_SHARE : FWD_SPLIT;
   }
-  if (two) {
-    const int nqt2 = fwd_tiles(p, 2 * FWD_BM);
-    const int64_t wgs = (int64_t)p.B * p.H * nqt2 * p.nranks;
-    const bool share = force_share ? force_share == 2 : wgs >= 2 * (int64_t)spa_device_cus();
-    if (share) {
-      p.nqt = nqt2;
-      return launch<flash_fwd16_kernel<T, D, 2, true, true, false, ZZ>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, true>::SMEM, p, stream);
+  FwdForm best = FWD_SPLIT;
+  float us = 0.96f * form_us(p, FWD_SPLIT, D, kind);  // (a margin for the form that suits small grids: near the line it is the safer one)
+  for (const FwdForm f : {FWD_SHARE, FWD_ONE}) {
+    if ((f == FWD_SHARE && !can_share) || (f == FWD_ONE && force == 2)) continue;
+    const float u = form_us(p, f, D, kind);
+    if (u < us) {
+      us = u;
+      best = f;
     }
   }
-  if (two) return launch<flash_fwd16_kernel<T, D, 2, false, true, false, ZZ>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, p, stream);
-  return launch<flash_fwd16_kernel<T, D, 1, false, true, false, ZZ>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM, p, stream);
+  return best;
+}
+
+// The chosen form of a family of variants (KV8, ZZ, QK8 as in the kernel).
+template <typename T, int D, bool KV8, bool ZZ, bool QK8>
+hipError_t launch16(FwdParams p, hipStream_t stream) {
+  const FwdForm form = fwd_form(p, D, QK8 ? KIND_QK8 : KV8 ? KIND_KV8 : KIND_16);
+  if (p.epi == SPA_EPI_FINALN) {
+    if (form != FWD_ONE)
+      return launch<flash_fwd16_kernel<T, D, 2, false, KV8, true, ZZ, false, QK8>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
+    return launch<flash_fwd16_kernel<T, D, 1, false, KV8, true, ZZ, false, QK8>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM, FWD_BM, p, stream);
+  }
+  if constexpr (D >= 64)
+    if (form == FWD_SHARE) {
+      p.nqt = fwd_tiles(p, 2 * FWD_BM);
+      return launch<flash_fwd16_kernel<T, D, 2, true, KV8, false, ZZ, false, QK8>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, true>::SMEM, 2 * FWD_BM, p, stream);
+    }
+  if (form == FWD_SPLIT)
+    return launch<flash_fwd16_kernel<T, D, 2, false, KV8, false, ZZ, false, QK8>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
+  return launch<flash_fwd16_kernel<T, D, 1, false, KV8, false, ZZ, false, QK8>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM_PLAIN, FWD_BM, p, stream);
 }
 
 // K / V spanning 2 GiB or more per (batch, head): the re-based variants, 128-row workgroups with two wave groups
@@ -1562,51 +1635,19 @@ hipError_t launch16_kv8(FwdParams p, hipStream_t stream) {
 template <typename T, int D>
 hipError_t launch16_big(const FwdParams& p, hipStream_t stream) {
   if (p.epi == SPA_EPI_FINALN)
-    return launch<flash_fwd16_kernel<T, D, 2, false, false, true, false, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, p, stream);
-  return launch<flash_fwd16_kernel<T, D, 2, false, false, false, false, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, p, stream);
+    return launch<flash_fwd16_kernel<T, D, 2, false, false, true, false, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
+  return launch<flash_fwd16_kernel<T, D, 2, false, false, false, false, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
 }
 
-// e4m3 q, k, v with the scores on the 8-bit matrix instruction (D = 128, block and ring calls): chosen like the others.
-template <typename T>
-hipError_t launch16_qk8(FwdParams p, hipStream_t stream) {
-  constexpr int D = 128;
-  const int force = spa_knob(SPA_KNOB_FWD_GROUPS);
-  const int force_share = spa_knob(SPA_KNOB_FWD_SHARE);
-  const bool two = force ? force == 2 : p.Sk > fwd_bn<D>();
-  if (p.epi == SPA_EPI_FINALN) {
-    if (two) return launch<flash_fwd16_kernel<T, D, 2, false, true, true, false, false, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, p, stream);
-    return launch<flash_fwd16_kernel<T, D, 1, false, true, true, false, false, true>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM, p, stream);
-  }
-  if (two) {
-    const int nqt2 = fwd_tiles(p, 2 * FWD_BM);
-    const int64_t wgs = (int64_t)p.B * p.H * nqt2 * p.nranks;
-    const bool share = force_share ? force_share == 2 : wgs >= 2 * (int64_t)spa_device_cus();
-    if (share) {
-      p.nqt = nqt2;
-      return launch<flash_fwd16_kernel<T, D, 2, true, true, false, false, false, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, true>::SMEM, p, stream);
-    }
-    return launch<flash_fwd16_kernel<T, D, 2, false, true, false, false, false, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, p, stream);
-  }
-  return launch<flash_fwd16_kernel<T, D, 1, false, true, false, false, false, true>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM, p, stream);
-}
-
-// One launch for a rank whose chunks arrive while it runs: 128-row workgroups, one or two wave groups.
-template <typename T, int D>
+// One launch for a rank whose chunks arrive while it runs: 128-row workgroups, one or two wave groups.  KV8: e4m3 q, k, v with
+// the scores on the 8-bit matrix instruction (D = 128).
+template <typename T, int D, bool KV8>
 hipError_t launch16_wait(const FwdParams& p, hipStream_t stream) {
   const int force = spa_knob(SPA_KNOB_FWD_GROUPS);
   const bool two = force ? force == 2 : p.Sk > fwd_bn<D>();
-  if (two) return launch<flash_fwd16_kernel<T, D, 2, false, false, false, false, false, false, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, p, stream);
-  return launch<flash_fwd16_kernel<T, D, 1, false, false, false, false, false, false, true>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM, p, stream);
-}
-
-// The same for e4m3 q, k, v with the scores on the 8-bit matrix instruction (D = 128).
-template <typename T>
-hipError_t launch16_wait_qk8(const FwdParams& p, hipStream_t stream) {
-  constexpr int D = 128;
-  const int force = spa_knob(SPA_KNOB_FWD_GROUPS);
-  const bool two = force ? force == 2 : p.Sk > fwd_bn<D>();
-  if (two) return launch<flash_fwd16_kernel<T, D, 2, false, true, false, false, false, true, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, p, stream);
-  return launch<flash_fwd16_kernel<T, D, 1, false, true, false, false, false, true, true>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM, p, stream);
+  if (two)
+    return launch<flash_fwd16_kernel<T, D, 2, false, KV8, false, false, false, KV8, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
+  return launch<flash_fwd16_kernel<T, D, 1, false, KV8, false, false, false, KV8, true>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM_PLAIN, FWD_BM, p, stream);
 }
 
 // (dtype, D) -> kernel family; the zigzag variants are instantiated beside the plain ones
@@ -1615,22 +1656,22 @@ hipError_t launch16_any(const FwdParams& p, int D, int dtype, hipStream_t stream
   if (p.k_scale) {  // K / V are e4m3 bytes, q / out of type `dtype`
     if (!p.v_scale) return hipErrorInvalidValue;
     if (dtype == 1) {
-      if (D == 128) return launch16_kv8<__bf16, 128, ZZ>(p, stream);
-      if (D == 64) return launch16_kv8<__bf16, 64, ZZ>(p, stream);
+      if (D == 128) return launch16<__bf16, 128, true, ZZ, false>(p, stream);
+      if (D == 64) return launch16<__bf16, 64, true, ZZ, false>(p, stream);
     } else if (dtype == 2) {
-      if (D == 128) return launch16_kv8<_Float16, 128, ZZ>(p, stream);
-      if (D == 64) return launch16_kv8<_Float16, 64, ZZ>(p, stream);
+      if (D == 128) return launch16<_Float16, 128, true, ZZ, false>(p, stream);
+      if (D == 64) return launch16<_Float16, 64, true, ZZ, false>(p, stream);
     }
     return hipErrorInvalidValue;
   }
   if (dtype == 1) {
-    if (D == 128) return launch16<__bf16, 128, ZZ>(p, stream);
-    if (D == 64) return launch16<__bf16, 64, ZZ>(p, stream);
-    if (D == 32) return launch16<__bf16, 32, ZZ>(p, stream);
+    if (D == 128) return launch16<__bf16, 128, false, ZZ, false>(p, stream);
+    if (D == 64) return launch16<__bf16, 64, false, ZZ, false>(p, stream);
+    if (D == 32) return launch16<__bf16, 32, false, ZZ, false>(p, stream);
   } else if (dtype == 2) {
-    if (D == 128) return launch16<_Float16, 128, ZZ>(p, stream);
-    if (D == 64) return launch16<_Float16, 64, ZZ>(p, stream);
-    if (D == 32) return launch16<_Float16, 32, ZZ>(p, stream);
+    if (D == 128) return launch16<_Float16, 128, false, ZZ, false>(p, stream);
+    if (D == 64) return launch16<_Float16, 64, false, ZZ, false>(p, stream);
+    if (D == 32) return launch16<_Float16, 32, false, ZZ, false>(p, stream);
   }
   return hipErrorInvalidValue;
 }
@@ -1650,7 +1691,7 @@ hipError_t spa_launch_fwd16_splitkv(FwdParams p, int D, int dtype, hipStream_t s
     return hipErrorInvalidValue;
   p.nqt = fwd_tiles(p, FWD_BM);
 #define SPA_KS(T, DD, KV8) \
-  launch<flash_fwd16_kernel<T, DD, 2, false, KV8, false, false, false, false, false, true>>(2 * FWD_THREADS, Fwd16Cfg<DD, 2, false>::SMEM, p, stream)
+  launch<flash_fwd16_kernel<T, DD, 2, false, KV8, false, false, false, false, false, true>>(2 * FWD_THREADS, Fwd16Cfg<DD, 2, false>::SMEM, FWD_BM, p, stream)
   if (p.k_scale) {
     if (dtype == 1) { if (D == 128) return SPA_KS(__bf16, 128, true); if (D == 64) return SPA_KS(__bf16, 64, true); }
     if (dtype == 2) { if (D == 128) return SPA_KS(_Float16, 128, true); if (D == 64) return SPA_KS(_Float16, 64, true); }
@@ -1670,8 +1711,8 @@ hipError_t spa_launch_fwd16_varlen_ring(FwdParams p, int D, int dtype, hipStream
   const int force = spa_knob(SPA_KNOB_FWD_GROUPS);
   const bool two = force ? force == 2 : p.Sk > fwd_bn<128>();
 #define SPA_VR(T, DD)                                                                                                                     \
-  (two ? launch<flash_fwd16_kernel<T, DD, 2, false, false, false, false, false, false, false, false, true>>(2 * FWD_THREADS, Fwd16Cfg<DD, 2, false>::SMEM, p, stream) \
-       : launch<flash_fwd16_kernel<T, DD, 1, false, false, false, false, false, false, false, false, true>>(FWD_THREADS, Fwd16Cfg<DD, 1, false>::SMEM, p, stream))
+  (two ? launch<flash_fwd16_kernel<T, DD, 2, false, false, false, false, false, false, false, false, true>>(2 * FWD_THREADS, Fwd16Cfg<DD, 2, false>::SMEM, FWD_BM, p, stream) \
+       : launch<flash_fwd16_kernel<T, DD, 1, false, false, false, false, false, false, false, false, true>>(FWD_THREADS, Fwd16Cfg<DD, 1, false>::SMEM_PLAIN, FWD_BM, p, stream))
   if (dtype == 1) { if (D == 128) return SPA_VR(__bf16, 128); if (D == 64) return SPA_VR(__bf16, 64); if (D == 32) return SPA_VR(__bf16, 32); }
   if (dtype == 2) { if (D == 128) return SPA_VR(_Float16, 128); if (D == 64) return SPA_VR(_Float16, 64); if (D == 32) return SPA_VR(_Float16, 32); }
 #undef SPA_VR
@@ -1684,24 +1725,24 @@ hipError_t spa_launch_fwd16_zigzag(const FwdParams& p, int D, int dtype, hipStre
 #elif defined(SPA_FWD_BIG_UNIT)
 hipError_t spa_launch_fwd16_qk8(const FwdParams& p, int D, int dtype, hipStream_t stream) {
   if (D != 128 || !p.q_scale || !p.k_scale || !p.v_scale || p.zigzag || p.big || p.cu_q) return hipErrorInvalidValue;
-  if (dtype == 1) return launch16_qk8<__bf16>(p, stream);
-  if (dtype == 2) return launch16_qk8<_Float16>(p, stream);
+  if (dtype == 1) return launch16<__bf16, 128, true, false, true>(p, stream);
+  if (dtype == 2) return launch16<_Float16, 128, true, false, true>(p, stream);
   return hipErrorInvalidValue;
 }
 hipError_t spa_launch_fwd16_wait(const FwdParams& p, int D, int dtype, hipStream_t stream) {
   if (!p.arrive || !p.fault || p.zigzag || p.big || p.epi != SPA_EPI_PLAIN || p.cu_q) return hipErrorInvalidValue;
   if (p.k_scale || p.v_scale || p.q_scale) {  // e4m3 tensors: all three, 8-bit scores
     if (!p.k_scale || !p.v_scale || !p.q_scale || D != 128) return hipErrorInvalidValue;
-    if (dtype == 1) return launch16_wait_qk8<__bf16>(p, stream);
-    if (dtype == 2) return launch16_wait_qk8<_Float16>(p, stream);
+    if (dtype == 1) return launch16_wait<__bf16, 128, true>(p, stream);
+    if (dtype == 2) return launch16_wait<_Float16, 128, true>(p, stream);
     return hipErrorInvalidValue;
   }
   if (dtype == 1) {
-    if (D == 128) return launch16_wait<__bf16, 128>(p, stream);
-    if (D == 64) return launch16_wait<__bf16, 64>(p, stream);
+    if (D == 128) return launch16_wait<__bf16, 128, false>(p, stream);
+    if (D == 64) return launch16_wait<__bf16, 64, false>(p, stream);
   } else if (dtype == 2) {
-    if (D == 128) return launch16_wait<_Float16, 128>(p, stream);
-    if (D == 64) return launch16_wait<_Float16, 64>(p, stream);
+    if (D == 128) return launch16_wait<_Float16, 128, false>(p, stream);
+    if (D == 64) return launch16_wait<_Float16, 64, false>(p, stream);
   }
   return hipErrorInvalidValue;
 }
@@ -1756,12 +1797,12 @@ hipError_t spa_launch_flash_fwd(FwdParams p, int D, int dtype, hipStream_t strea
     if (D <= 64 && !p.cu_q && p.nranks == 1 && p.P == 1 && knob != 1 && (few || knob == 2)) {
       FwdParams ps = p;
       ps.nqt = (p.Sq + 31) / 32;
-      if (D == 64) return launch<flash_fwd32_splitk_kernel<64, 8>>(512, Fwd32SplitCfg<64, 8>::SMEM, ps, stream);
-      return launch<flash_fwd32_splitk_kernel<32, 8>>(512, Fwd32SplitCfg<32, 8>::SMEM, ps, stream);
+      if (D == 64) return launch<flash_fwd32_splitk_kernel<64, 8>>(512, Fwd32SplitCfg<64, 8>::SMEM, 32, ps, stream);
+      return launch<flash_fwd32_splitk_kernel<32, 8>>(512, Fwd32SplitCfg<32, 8>::SMEM, 32, ps, stream);
     }
-    if (D == 128) return launch<flash_fwd32_kernel<128>>(FWD_THREADS, Fwd32Cfg<128>::SMEM, p, stream);
-    if (D == 64) return launch<flash_fwd32_kernel<64>>(FWD_THREADS, Fwd32Cfg<64>::SMEM, p, stream);
-    if (D == 32) return launch<flash_fwd32_kernel<32>>(FWD_THREADS, Fwd32Cfg<32>::SMEM, p, stream);
+    if (D == 128) return launch<flash_fwd32_kernel<128>>(FWD_THREADS, Fwd32Cfg<128>::SMEM, FWD_BM, p, stream);
+    if (D == 64) return launch<flash_fwd32_kernel<64>>(FWD_THREADS, Fwd32Cfg<64>::SMEM, FWD_BM, p, stream);
+    if (D == 32) return launch<flash_fwd32_kernel<32>>(FWD_THREADS, Fwd32Cfg<32>::SMEM, FWD_BM, p, stream);
   }
   return hipErrorInvalidValue;
 }

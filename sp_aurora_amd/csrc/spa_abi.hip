@@ -747,8 +747,6 @@ int flash_bwd(const char* what, const void* q, const void* k, const void* v, con
   p.scale = scale_eff(scale);
   p.scale_log2 = scale_eff(scale) * 1.4426950408889634f;
   p.causal = mask_mode == SPA_MASK_CAUSAL;
-  p.nqt = 0;
-  p.nkt = 0;
   p.lse_bh = Sq;
   p.cu_q = nullptr; p.cu_k = nullptr;
   return launch_result(spa_launch_flash_bwd(p, D, dtype, (hipStream_t)stream), what);
@@ -914,10 +912,9 @@ int flash_bwd_varlen(const char* what, const void* q, const void* k, const void*
   p.scale = scale_eff(scale);
   p.scale_log2 = scale_eff(scale) * 1.4426950408889634f;
   p.causal = mask_mode == SPA_MASK_CAUSAL;
-  p.nqt = 0;
-  p.nkt = 0;
   p.lse_bh = total_q;
   p.cu_q = cu_seqlens_q; p.cu_k = cu_seqlens_k;
+  p.total_k = total_k;
   return launch_result(spa_launch_flash_bwd(p, D, dtype, (hipStream_t)stream), what);
 }
 }  // namespace

@@ -116,13 +116,12 @@ struct BwdParams {
   float scale;
   float scale_log2;
   int causal;
-  int nqt;  // number of query tiles per (batch, head)
-  int nkt;  // number of key tiles per (batch, head)
   int64_t lse_bh;  // elements between consecutive (batch, head) rows of lse and delta
   // variable-length batch, as in FwdParams: rows cu_q[b] .. cu_q[b+1] of q/dout/dq/lse/delta and
   // cu_k[b] .. cu_k[b+1] of k/v/dk/dv belong to sequence b; lse and delta are [H][lse_bh]
   const int* cu_q;
   const int* cu_k;
+  int total_k = 0;  // rows of the packed key-side tensors (total_q is lse_bh)
   // 0: dq/dk/dv are fp32 accumulators, added to; 1: they are tensors of q's element type (strides in
   // those elements) and are WRITTEN: the whole gradient comes from this one launch
   int grads_in_t;
@@ -212,6 +211,38 @@ static __device__ __forceinline__ float halves_sum(float x) {
   float lo, hi;
   both_halves(x, lo, hi);
   return lo + hi;
+}
+
+// ---- variable-length batches ----
+// Which tile of which sequence a workgroup takes.  The tiles (of `rows` rows) of all sequences are numbered back to back,
+// sequence by sequence, so a grid of (total rows / rows + sequences) numbers covers any batch and at most one workgroup
+// per sequence finds nothing to do (a grid of sequences x longest sequence spends a third of its workgroups on rows that
+// do not exist, and each takes a CU from one with work).  Blocks of 64 sequences in the order given, longest first inside a
+// block: the heavy tiles start first, and the tiles of one sequence run side by side and share its K / V in L2.
+// Every wave of the workgroup calls this (a lane holds one sequence of the block); false: no such tile.
+static __device__ __forceinline__ bool sequence_tile(const int* cu, int nseq, int rows, int number, int lane, int& seq, int& tile, int& ntiles) {
+  for (int base = 0; base < nseq; base += 64) {
+    const int n = nseq - base < 64 ? nseq - base : 64;
+    const int i = base + (lane < n ? lane : 0);
+    const int len = lane < n ? cu[i + 1] - cu[i] : 0;
+    const int mine = (len + rows - 1) / rows;
+    int before = 0, total = 0;  // tiles of the sequences that come before this lane's, tiles of the block
+    for (int j = 0; j < n; ++j) {
+      const int lj = __builtin_amdgcn_readlane(len, j), tj = __builtin_amdgcn_readlane(mine, j);
+      before += lj > len || (lj == len && j < lane) ? tj : 0;
+      total += tj;
+    }
+    if (number < total) {
+      const unsigned long long own = __builtin_amdgcn_ballot_w64(number >= before && number < before + mine);
+      const int owner = __builtin_amdgcn_readfirstlane(__builtin_ctzll(own));
+      seq = base + owner;
+      ntiles = __builtin_amdgcn_readlane(mine, owner);
+      tile = number - __builtin_amdgcn_readlane(before, owner);
+      return true;
+    }
+    number -= total;
+  }
+  return false;
 }
 
 // ---- LDS helpers shared by the attention kernels ----

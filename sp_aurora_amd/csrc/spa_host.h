@@ -54,3 +54,26 @@ hipError_t spa_allow_dynamic_lds(int smem) {
   if (e == hipSuccess && dev >= 0 && dev < SPA_MAX_DEVICES) ready.fetch_or(1ull << dev, std::memory_order_release);
   return e;
 }
+
+// Grid of an attention launch with `tiles` workgroups per (batch, head) pair: x = the pairs of one group, y = tiles, z =
+// groups, dispatched in that order, so that a group's tiles run side by side and then the next group's.  A head's tiles
+// share its streamed tensors in the L2 of the XCD they run on (round-robin placement: x % 8 while x has a multiple of 8 pairs), but
+// only while they run at the same time: with more pairs than CUs and no groups, every tile of a head reads them from memory
+// again.  A group holds as many pairs per XCD as fill its CUs with their tiles, at least 4 (fewer were not measured to help
+// long rows, whose tiles walk the keys in step).
+static inline dim3 spa_head_groups(int64_t pairs, int tiles) {
+  const int64_t per_xcd = (spa_device_cus() / 8 + tiles - 1) / tiles;
+  const int64_t group = 8 * (per_xcd > 4 ? per_xcd : 4);
+  if (pairs <= group) return dim3((unsigned)pairs, (unsigned)tiles, 1);
+  const int64_t n = (pairs + group - 1) / group;
+  if (n < 4 || n > 65535) return dim3((unsigned)pairs, (unsigned)tiles, 1);
+  return dim3((unsigned)group, (unsigned)tiles, (unsigned)n);
+}
+
+// Grid of a launch over a packed variable-length batch: one workgroup per head and tile number (sequence_tile), heads first.
+static inline bool spa_varlen_grid(int H, int nseq, int64_t total_rows, int rows, unsigned z, dim3& grid) {
+  const int64_t n = (total_rows / rows + nseq) * H;
+  if (n <= 0 || n > 0x7fffffffLL) return false;
+  grid = dim3((unsigned)n, 1, z);
+  return true;
+}
