@@ -376,6 +376,21 @@ int spa_flash_bwd_out(const void* q, const void* k, const void* v, const void* d
                       float scale, int mask_mode, int dtype, void* stream);
 
 /*
+ * spa_flash_bwd_out from the forward's result: out (q's shape and type) in place of delta, which is scratch here (fp32,
+ * contiguous [B,H,Sq]): delta = rowsum(dout * out) is formed by the kernel that computes dq, for its own rows, and read by the
+ * one that computes dk and dv.  Replaces intel_ring_flash_attn_backward (sp_aurora/intel_ring_flash_attn.py:153-271) for a
+ * ring whose shards are all on this GPU, and the block's own backward.
+ */
+int spa_attention_bwd(const void* q, const void* k, const void* v, const void* out, const void* dout,
+                      const float* lse, float* delta, void* dq, void* dk, void* dv,
+                      int B, int H, int Sq, int Sk, int D,
+                      const int64_t q_strides[3], const int64_t k_strides[3],
+                      const int64_t v_strides[3], const int64_t o_strides[3],
+                      const int64_t do_strides[3], const int64_t dq_strides[3],
+                      const int64_t dk_strides[3], const int64_t dv_strides[3],
+                      float scale, int mask_mode, int dtype, void* stream);
+
+/*
  * Block attention over a batch of sequences of different lengths packed back
  * to back (no padding): q / out are [total_q, H, D], k / v [total_k, H, D];
  * sequence b owns query rows cu_seqlens_q[b] .. cu_seqlens_q[b+1] and key rows
@@ -451,7 +466,7 @@ int spa_flash_bwd_varlen(const void* q, const void* k, const void* v, const void
  * spa_flash_bwd_varlen for the whole gradient in one call, as spa_flash_bwd_out is to spa_flash_bwd:
  * dq [total_q, H, D], dk / dv [total_k, H, D] have the inputs' element type and are WRITTEN (zeros
  * where a sequence has queries but no keys, or keys that no query sees).  Rows that belong to no
- * sequence, or that lie past max_sq / max_sk of a longer sequence, are left untouched.  Same
+ * sequence are left untouched.  Same
  * call site as spa_flash_bwd_varlen (test_intel_ring_flash_attn_varlen.py:85-91).
  */
 int spa_flash_bwd_varlen_out(const void* q, const void* k, const void* v, const void* dout,
@@ -463,6 +478,20 @@ int spa_flash_bwd_varlen_out(const void* q, const void* k, const void* v, const 
                              const int64_t v_strides[2], const int64_t do_strides[2],
                              const int64_t dq_strides[2], const int64_t dk_strides[2],
                              const int64_t dv_strides[2],
+                             float scale, int mask_mode, int dtype, void* stream);
+
+/*
+ * spa_flash_bwd_varlen_out from the forward's result, as spa_attention_bwd is to spa_flash_bwd_out (out [total_q, H, D], delta:
+ * scratch, fp32 [H, total_q]).
+ */
+int spa_attention_bwd_varlen(const void* q, const void* k, const void* v, const void* out, const void* dout,
+                             const float* lse, float* delta, void* dq, void* dk, void* dv,
+                             const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                             int nseq, int H, int total_q, int total_k, int max_sq, int max_sk, int D,
+                             const int64_t q_strides[2], const int64_t k_strides[2],
+                             const int64_t v_strides[2], const int64_t o_strides[2],
+                             const int64_t do_strides[2], const int64_t dq_strides[2],
+                             const int64_t dk_strides[2], const int64_t dv_strides[2],
                              float scale, int mask_mode, int dtype, void* stream);
 
 /*

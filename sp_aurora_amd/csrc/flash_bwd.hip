@@ -117,6 +117,41 @@ struct TileLoader {
   }
 };
 
+// The lane's operands of ROWS = 32 resident rows (row ln; 16 bytes per 16-deep contraction step) out of rows that were
+// loaded like a tile.  Straight from memory they are 16-byte pieces of 32 rows per load instruction: 32 cache lines for 1 KB,
+// and the first 5 us of a workgroup went into them; as a tile every instruction reads whole rows.
+template <typename F, int D>
+__device__ __forceinline__ void read_rows(F (&f)[D / 16], unsigned rows_at, const TileReads<D>& rd) {
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) f[ks] = as_frag<F>(lds_read_b128(rows_at + rd.row[ks]));
+}
+
+// Writes the wave's 32 rows of a gradient (accumulator layout: a lane holds, of row ln, dims 32 db + 8 g + 4 hh .. + 3) in T.
+// Through LDS (32 rows of the wave's own, chunks XOR-permuted), so that a store instruction writes whole rows: the 8-byte
+// pieces a lane holds are 32 cache lines per instruction, and the last 6 us of a workgroup went into them.
+// first_row: number of rows that exist from the wave's first row on; stride in elements.
+template <typename T, int D>
+__device__ __forceinline__ void store_rows(const f32x16 (&acc)[D / 32], float scale, T* rows, int64_t stride, int n_rows, unsigned char* lds, int lane) {
+  constexpr int CPR = D / 8;  // 16-byte chunks per row
+  const int ln = lane & 31, hh = lane >> 5;
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      u32x2 st;
+      st[0] = Mma16<T>::pack2(acc[db][4 * g + 0] * scale, acc[db][4 * g + 1] * scale);
+      st[1] = Mma16<T>::pack2(acc[db][4 * g + 2] * scale, acc[db][4 * g + 3] * scale);
+      *(u32x2*)(lds + ln * (D * 2) + (((db * 4 + g) ^ (ln & (CPR - 1))) * 16) + 8 * hh) = st;
+    }
+  // (the wave's own LDS writes are visible to its later reads)
+#pragma unroll
+  for (int i = 0; i < 32 * CPR / 64; ++i) {
+    const int r = i * (64 / CPR) + lane / CPR, ch = lane % CPR;
+    const u32x4 x = *(const u32x4*)(lds + r * (D * 2) + ((ch ^ (r & (CPR - 1))) * 16));
+    if (r < n_rows) *(u32x4*)(rows + (int64_t)r * stride + ch * 8) = x;
+  }
+}
+
 // One MFMA operand from two transposing reads (rows 0..3 and 8..11 of a lane's group of 16).
 template <typename F>
 __device__ __forceinline__ F frag_tr(unsigned addr_lo, unsigned addr_hi) {
@@ -205,6 +240,7 @@ __device__ __forceinline__ void select_sequence(BwdParams& p, int& b) {
   p.dq = (float*)((char*)p.dq + q_lo * p.dqs.s * gsz);
   p.dk = (float*)((char*)p.dk + k_lo * p.dks.s * gsz);
   p.dv = (float*)((char*)p.dv + k_lo * p.dvs.s * gsz);
+  if (p.out) p.out = (const T*)p.out + (int64_t)q_lo * p.os.s;
   p.lse += q_lo;
   p.delta += q_lo;
   b = 0;
@@ -287,14 +323,8 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_dq_kernel(const BwdParam
   const int qrow_c = qrow < p.Sq ? qrow : p.Sq - 1;
 
   frag qf[D / 16], dof[D / 16];
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
-    qf[ks] = as_frag<frag>(*(const u32x4*)(qp + (int64_t)qrow_c * p.qs.s + ks * 16 + hh * 8));
-    dof[ks] = as_frag<frag>(*(const u32x4*)(dop + (int64_t)qrow_c * p.dos.s + ks * 16 + hh * 8));
-  }
   const int64_t li = ((int64_t)b * p.H + h) * p.lse_bh + qrow_c;
   const float l2 = p.lse[li] * 1.4426950408889634f;
-  const float dl = p.delta[li];
   const float c = p.scale_log2;
   const float hidden = c < 0.f ? INFINITY : -INFINITY;  // a hidden score: exp2(hidden * c - lse) = 0 for either sign of the scale
   const int lim = p.causal ? (qrow < p.Sk - 1 ? qrow : p.Sk - 1) : p.Sk - 1;  // last visible key
@@ -337,8 +367,55 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_dq_kernel(const BwdParam
   constexpr int BWD_LOOK = NA < LOOK_CAP ? NA : LOOK_CAP;
   static_assert(NBODY % BWD_LOOK == 0 && BWD_LOOK <= NA, "the operand window must tile the loop body");
 
+  // The workgroup's rows of q and dout pass through the stages on their way into registers; then those of out, which give
+  // delta = rowsum(dout * out) (written for the dk / dv kernel), while the first two tiles are on their way.
+  {
+    constexpr int RT = NW / 2;  // tiles of 64 rows
+    auto load_rows = [&](const T* base, int64_t stride, unsigned dst) {
+      TileLoader<T, D, NW * 64, BIG> ld;
+      ld.init(base, stride, p.Sq, tid);
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int q = 0; q < C::NDMA; ++q) ld.load(q, q0 + i * BWD_ROWS < p.Sq, q0 + i * BWD_ROWS, dst + i * C::TILEB + w * 1024);
+    };
+    const unsigned own = (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB, other = 2 * G::STAGE;
+    load_rows(qp, p.qs.s, lds0);
+    load_rows(dop, p.dos.s, lds0 + other);
+    wait_loads_but<0>();
+    __syncthreads();
+    read_rows<frag, D>(qf, lds0 + own, rd);
+    read_rows<frag, D>(dof, lds0 + other + own, rd);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): read ...
+    __syncthreads();                     // ... by every wave
+    if (p.out) load_rows((const T*)p.out + b * p.os.b + h * p.os.h, p.os.s, lds0 + other);
+  }
   issue_tile(0);
   issue_tile(1);
+  float dl;
+  if (p.out) {
+    wait_loads_but<2 * G::NL>();
+    __syncthreads();
+    const unsigned own = lds0 + 2 * G::STAGE + (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB;
+    float sum = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      const u32x4 x = lds_read_b128(own + rd.row[ks]), y = __builtin_bit_cast(u32x4, dof[ks]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x0, x1, y0, y1;
+        M::unpack2(x[i], x0, x1);
+        M::unpack2(y[i], y0, y1);
+        sum = __builtin_fmaf(x1, y1, __builtin_fmaf(x0, y0, sum));
+      }
+    }
+    dl = halves_sum(sum);
+    if (hh == 0 && qrow < p.Sq) p.delta[li] = dl;
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __syncthreads();
+  } else {
+    dl = p.delta[li];
+  }
   issue_tile(2);
   wait_loads_but<2 * G::NL>();
   __syncthreads();
@@ -478,18 +555,10 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_dq_kernel(const BwdParam
   // wait, so no read of them can be scheduled above it.
   if constexpr (MIXED) asm volatile("s_nop 15\n s_nop 15" : "+a"(dq[0]), "+a"(dq[1]), "+a"(dq[2]), "+a"(dq[3])::"memory");
 
-  if (qrow < p.Sq && p.grads_in_t) {
+  if (p.grads_in_t) {
     // the whole gradient of the row: written in q's element type, nothing read
-    T* dqp = (T*)p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)qrow * p.dqs.s;
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        u32x2 st;
-        st[0] = Mma16<T>::pack2(dq[db][4 * g + 0] * p.scale, dq[db][4 * g + 1] * p.scale);
-        st[1] = Mma16<T>::pack2(dq[db][4 * g + 2] * p.scale, dq[db][4 * g + 3] * p.scale);
-        *(u32x2*)(dqp + db * 32 + 8 * g + 4 * hh) = st;
-      }
+    __syncthreads();  // every wave is done with the tiles, and with its loads into them
+    store_rows<T, D>(dq, p.scale, (T*)p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)qw0 * p.dqs.s, p.dqs.s, p.Sq - qw0, smem + w * (32 * C::ROWB), lane);
   } else if (qrow < p.Sq) {
     float* dqp = p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)qrow * p.dqs.s;
 #pragma unroll
@@ -557,14 +626,7 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd_dkdv_kernel(const Bw
   const float* delp = p.delta + ((int64_t)b * p.H + h) * p.lse_bh;
 
   const int krow = kw0 + ln;
-  const int krow_c = krow < p.Sk ? krow : p.Sk - 1;
-
   frag kf[D / 16], vf[D / 16];
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
-    kf[ks] = as_frag<frag>(*(const u32x4*)(kp + (int64_t)krow_c * p.ks.s + ks * 16 + hh * 8));
-    vf[ks] = as_frag<frag>(*(const u32x4*)(vp + (int64_t)krow_c * p.vs.s + ks * 16 + hh * 8));
-  }
   const float c = p.scale_log2;
   const float hidden = c < 0.f ? INFINITY : -INFINITY;  // a hidden score: exp2(hidden * c - lse) = 0 for either sign of the scale
 
@@ -619,8 +681,30 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd_dkdv_kernel(const Bw
   static_assert(NBODY % BWD_LOOK == 0 && BWD_LOOK <= NA, "the operand window must tile the loop body");
 
   if (it0 < nt) {  // uniform; a workgroup whose keys no query sees adds nothing
+    // the workgroup's keys first, as two tiles each of K and V in the stages of tiles it0 + 2 and it0 + 3
+    {
+      TileLoader<T, D, BWD_THREADS, BIG> kld, vld;
+      kld.init(kp, p.ks.s, p.Sk, tid);
+      vld.init(vp, p.vs.s, p.Sk, tid);
+      const unsigned kdst = stage_of(it0 + 2) + w * 1024, vdst = stage_of(it0 + 3) + w * 1024;
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int q = 0; q < C::NDMA; ++q) kld.load(q, k0 + half * BWD_ROWS < p.Sk, k0 + half * BWD_ROWS, kdst + half * C::TILEB);
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int q = 0; q < C::NDMA; ++q) vld.load(q, k0 + half * BWD_ROWS < p.Sk, k0 + half * BWD_ROWS, vdst + half * C::TILEB);
+    }
     issue_tile(it0);
     issue_tile(it0 + 1);
+    wait_loads_but<2 * G::NL>();
+    __syncthreads();
+    const unsigned own = (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB;  // the wave's 32 keys in either pair of tiles
+    read_rows<frag, D>(kf, stage_of(it0 + 2) + own, rd);
+    read_rows<frag, D>(vf, stage_of(it0 + 3) + own, rd);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the stage of tile it0 + 2 has been read ...
+    __syncthreads();                     // ... by every wave
     issue_tile(it0 + 2);
     wait_loads_but<2 * G::NL>();
     __syncthreads();
@@ -783,21 +867,12 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd_dkdv_kernel(const Bw
     asm volatile("s_nop 15\n s_nop 15"
                  : "+a"(dk[0]), "+a"(dk[1]), "+a"(dk[2]), "+a"(dk[3]), "+a"(dv[0]), "+a"(dv[1]), "+a"(dv[2]), "+a"(dv[3])::"memory");
 
-  if (krow < p.Sk && p.grads_in_t) {
-    T* dkp = (T*)p.dk + b * p.dks.b + h * p.dks.h + (int64_t)krow * p.dks.s;
-    T* dvp = (T*)p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)krow * p.dvs.s;
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        u32x2 x, y;
-        x[0] = Mma16<T>::pack2(dk[db][4 * g + 0] * p.scale, dk[db][4 * g + 1] * p.scale);
-        x[1] = Mma16<T>::pack2(dk[db][4 * g + 2] * p.scale, dk[db][4 * g + 3] * p.scale);
-        y[0] = Mma16<T>::pack2(dv[db][4 * g + 0], dv[db][4 * g + 1]);
-        y[1] = Mma16<T>::pack2(dv[db][4 * g + 2], dv[db][4 * g + 3]);
-        *(u32x2*)(dkp + db * 32 + 8 * g + 4 * hh) = x;
-        *(u32x2*)(dvp + db * 32 + 8 * g + 4 * hh) = y;
-      }
+  if (p.grads_in_t) {
+    __syncthreads();  // every wave is done with the tiles, and with its loads into them
+    T* const dkp = (T*)p.dk + b * p.dks.b + h * p.dks.h + (int64_t)kw0 * p.dks.s;
+    T* const dvp = (T*)p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)kw0 * p.dvs.s;
+    store_rows<T, D>(dv, 1.f, dvp, p.dvs.s, p.Sk - kw0, smem + w * (64 * C::ROWB), lane);
+    store_rows<T, D>(dk, p.scale, dkp, p.dks.s, p.Sk - kw0, smem + w * (64 * C::ROWB) + 32 * C::ROWB, lane);
   } else if (krow < p.Sk) {
     float* dkp = p.dk + b * p.dks.b + h * p.dks.h + (int64_t)krow * p.dks.s;
     float* dvp = p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)krow * p.dvs.s;
@@ -906,7 +981,21 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dq_kernel(const Bw
   }
   const int64_t li = ((int64_t)b * p.H + h) * p.lse_bh + qrow_c;
   const float l2 = p.lse[li] * 1.4426950408889634f;
-  const float dl = p.delta[li];
+  float dl;
+  if (p.out) {  // delta = rowsum(dout * out), written for the dk / dv kernel
+    const float* op = (const float*)p.out + b * p.os.b + h * p.os.h + (int64_t)qrow_c * p.os.s;
+    float sum = 0.f;
+#pragma unroll
+    for (int g = 0; g < D / 8; ++g) {
+      const f32x4 x = *(const f32x4*)(op + 8 * g + 4 * hh);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(x[e], dof[g][e], sum);
+    }
+    dl = halves_sum(sum);
+    if (hh == 0 && qrow < p.Sq) p.delta[li] = dl;
+  } else {
+    dl = p.delta[li];
+  }
   const float c = p.scale_log2;
   const int lim = p.causal ? (qrow < p.Sk - 1 ? qrow : p.Sk - 1) : p.Sk - 1;  // last visible key
 

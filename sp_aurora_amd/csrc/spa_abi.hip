@@ -710,9 +710,9 @@ int spa_bwd_delta(const void* out, const void* dout, float* delta, int B, int H,
 
 namespace {
 // grads_in_t: dq / dk / dv are tensors of the inputs' element type and are written (spa_flash_bwd_out);
-// else fp32 accumulators that are added to (spa_flash_bwd).
-int flash_bwd(const char* what, const void* q, const void* k, const void* v, const void* dout, const float* lse,
-              const float* delta, void* dq, void* dk, void* dv, bool grads_in_t, int B, int H, int Sq, int Sk,
+// else fp32 accumulators that are added to (spa_flash_bwd).  out (with o_strides): delta is scratch and is computed here.
+int flash_bwd(const char* what, const void* q, const void* k, const void* v, const void* out, const int64_t* o_strides, const void* dout,
+              const float* lse, float* delta, void* dq, void* dk, void* dv, bool grads_in_t, int B, int H, int Sq, int Sk,
               int D, const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
               const int64_t do_strides[3], const int64_t dq_strides[3], const int64_t dk_strides[3],
               const int64_t dv_strides[3], float scale, int mask_mode, int dtype, void* stream) {
@@ -727,18 +727,21 @@ int flash_bwd(const char* what, const void* q, const void* k, const void* v, con
   const int esz = elem_size(dtype), gsz = grads_in_t ? esz : 4;
   if (!aligned16(q, q_strides, esz) || !aligned16(k, k_strides, esz) || !aligned16(v, v_strides, esz) ||
       !aligned16(dout, do_strides, esz) || !aligned16(dq, dq_strides, gsz) || !aligned16(dk, dk_strides, gsz) ||
-      !aligned16(dv, dv_strides, gsz))
+      !aligned16(dv, dv_strides, gsz) || (out && !aligned16(out, o_strides, esz)))
     return fail(SPA_EALIGN, "%s: pointers and row strides must be 16-byte aligned", what);
-  const bool big = !span_ok(Sq, q_strides[2], D, esz) || !span_ok(Sk, k_strides[2], D, esz) || !span_ok(Sk, v_strides[2], D, esz) ||
+  const bool big = (out && !span_ok(Sq, o_strides[2], D, esz)) || !span_ok(Sq, q_strides[2], D, esz) || !span_ok(Sk, k_strides[2], D, esz) || !span_ok(Sk, v_strides[2], D, esz) ||
                    !span_ok(Sq, do_strides[2], D, esz);
   if (big && dtype != SPA_F32 && !(span_rebasable(q_strides[2], esz) && span_rebasable(k_strides[2], esz) &&
-                                   span_rebasable(v_strides[2], esz) && span_rebasable(do_strides[2], esz)))
+                                   span_rebasable(v_strides[2], esz) && span_rebasable(do_strides[2], esz) &&
+                                   (!out || span_rebasable(o_strides[2], esz))))
     return fail(SPA_EUNSUPPORTED, "%s: a tensor of one (batch, head) spans 2 GiB or more and 128 rows of it 1 GiB or more", what);
   if ((int64_t)B * H * ((Sq + 127) / 128) > 0x7fffffffLL || (int64_t)B * H * ((Sk + 127) / 128) > 0x7fffffffLL)
     return fail(SPA_EINVAL, "%s: grid too large", what);
   BwdParams p;
   p.q = q; p.k = k; p.v = v; p.dout = dout; p.lse = lse; p.delta = delta;
   p.dq = (float*)dq; p.dk = (float*)dk; p.dv = (float*)dv;
+  p.out = out;
+  if (out) p.os = S3(o_strides);
   p.grads_in_t = grads_in_t;
   p.big = big && dtype != SPA_F32;
   p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk;
@@ -758,7 +761,7 @@ int spa_flash_bwd(const void* q, const void* k, const void* v, const void* dout,
                   int D, const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
                   const int64_t do_strides[3], const int64_t dq_strides[3], const int64_t dk_strides[3],
                   const int64_t dv_strides[3], float scale, int mask_mode, int dtype, void* stream) {
-  return flash_bwd("spa_flash_bwd", q, k, v, dout, lse, delta, dq_acc, dk_acc, dv_acc, false, B, H, Sq, Sk, D, q_strides, k_strides,
+  return flash_bwd("spa_flash_bwd", q, k, v, nullptr, nullptr, dout, lse, const_cast<float*>(delta), dq_acc, dk_acc, dv_acc, false, B, H, Sq, Sk, D, q_strides, k_strides,
                    v_strides, do_strides, dq_strides, dk_strides, dv_strides, scale, mask_mode, dtype, stream);
 }
 
@@ -767,7 +770,17 @@ int spa_flash_bwd_out(const void* q, const void* k, const void* v, const void* d
                       int D, const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
                       const int64_t do_strides[3], const int64_t dq_strides[3], const int64_t dk_strides[3],
                       const int64_t dv_strides[3], float scale, int mask_mode, int dtype, void* stream) {
-  return flash_bwd("spa_flash_bwd_out", q, k, v, dout, lse, delta, dq, dk, dv, true, B, H, Sq, Sk, D, q_strides, k_strides,
+  return flash_bwd("spa_flash_bwd_out", q, k, v, nullptr, nullptr, dout, lse, const_cast<float*>(delta), dq, dk, dv, true, B, H, Sq, Sk, D,
+                   q_strides, k_strides, v_strides, do_strides, dq_strides, dk_strides, dv_strides, scale, mask_mode, dtype, stream);
+}
+
+int spa_attention_bwd(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse, float* delta,
+                      void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D, const int64_t q_strides[3],
+                      const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3], const int64_t do_strides[3],
+                      const int64_t dq_strides[3], const int64_t dk_strides[3], const int64_t dv_strides[3], float scale,
+                      int mask_mode, int dtype, void* stream) {
+  if (!out || !o_strides) return fail(SPA_EINVAL, "spa_attention_bwd: null pointer");
+  return flash_bwd("spa_attention_bwd", q, k, v, out, o_strides, dout, lse, delta, dq, dk, dv, true, B, H, Sq, Sk, D, q_strides, k_strides,
                    v_strides, do_strides, dq_strides, dk_strides, dv_strides, scale, mask_mode, dtype, stream);
 }
 
@@ -879,8 +892,8 @@ int flash_fwd_varlen(const char* what, const void* q, const void* k, const void*
 }
 
 // grads_in_t: as in flash_bwd above.
-int flash_bwd_varlen(const char* what, const void* q, const void* k, const void* v, const void* dout, const float* lse,
-                     const float* delta, void* dq, void* dk, void* dv, bool grads_in_t, const int32_t* cu_seqlens_q,
+int flash_bwd_varlen(const char* what, const void* q, const void* k, const void* v, const void* out, const int64_t* o_strides,
+                     const void* dout, const float* lse, float* delta, void* dq, void* dk, void* dv, bool grads_in_t, const int32_t* cu_seqlens_q,
                      const int32_t* cu_seqlens_k, int nseq, int H, int total_q, int total_k, int max_sq, int max_sk,
                      int D, const int64_t q_strides[2], const int64_t k_strides[2], const int64_t v_strides[2],
                      const int64_t do_strides[2], const int64_t dq_strides[2], const int64_t dk_strides[2],
@@ -894,17 +907,20 @@ int flash_bwd_varlen(const char* what, const void* q, const void* k, const void*
   const int esz = elem_size(dtype), gsz = grads_in_t ? esz : 4;
   if (!aligned16v(q, q_strides, esz) || !aligned16v(k, k_strides, esz) || !aligned16v(v, v_strides, esz) ||
       !aligned16v(dout, do_strides, esz) || !aligned16v(dq, dq_strides, gsz) || !aligned16v(dk, dk_strides, gsz) ||
-      !aligned16v(dv, dv_strides, gsz) || (((uintptr_t)lse | (uintptr_t)delta) & 3) != 0)
+      !aligned16v(dv, dv_strides, gsz) || (out && !aligned16v(out, o_strides, esz)) || (((uintptr_t)lse | (uintptr_t)delta) & 3) != 0)
     return fail(SPA_EALIGN, "%s: pointers and row strides must be 16-byte aligned", what);
-  const bool big = !span_ok(max_sq, q_strides[1], D, esz) || !span_ok(max_sk, k_strides[1], D, esz) ||
+  const bool big = (out && !span_ok(max_sq, o_strides[1], D, esz)) || !span_ok(max_sq, q_strides[1], D, esz) || !span_ok(max_sk, k_strides[1], D, esz) ||
                    !span_ok(max_sk, v_strides[1], D, esz) || !span_ok(max_sq, do_strides[1], D, esz);
   if (big && dtype != SPA_F32 && !(span_rebasable(q_strides[1], esz) && span_rebasable(k_strides[1], esz) &&
-                                   span_rebasable(v_strides[1], esz) && span_rebasable(do_strides[1], esz)))
+                                   span_rebasable(v_strides[1], esz) && span_rebasable(do_strides[1], esz) &&
+                                   (!out || span_rebasable(o_strides[1], esz))))
     return fail(SPA_EUNSUPPORTED, "%s: a tensor of one (sequence, head) spans 2 GiB or more and 128 rows of it 1 GiB or more", what);
   BwdParams p;
   p.big = big && dtype != SPA_F32;
   p.q = q; p.k = k; p.v = v; p.dout = dout; p.lse = lse; p.delta = delta;
   p.dq = (float*)dq; p.dk = (float*)dk; p.dv = (float*)dv;
+  p.out = out;
+  if (out) p.os = S2(o_strides);
   p.grads_in_t = grads_in_t;
   p.B = nseq; p.H = H; p.Sq = max_sq; p.Sk = max_sk;
   p.qs = S2(q_strides); p.ks = S2(k_strides); p.vs = S2(v_strides); p.dos = S2(do_strides);
@@ -959,8 +975,8 @@ int spa_flash_bwd_varlen(const void* q, const void* k, const void* v, const void
                          const int64_t k_strides[2], const int64_t v_strides[2], const int64_t do_strides[2],
                          const int64_t dq_strides[2], const int64_t dk_strides[2], const int64_t dv_strides[2],
                          float scale, int mask_mode, int dtype, void* stream) {
-  return flash_bwd_varlen("spa_flash_bwd_varlen", q, k, v, dout, lse, delta, dq_acc, dk_acc, dv_acc, false, cu_seqlens_q,
-                          cu_seqlens_k, nseq, H, total_q, total_k, max_sq, max_sk, D, q_strides, k_strides, v_strides,
+  return flash_bwd_varlen("spa_flash_bwd_varlen", q, k, v, nullptr, nullptr, dout, lse, const_cast<float*>(delta), dq_acc, dk_acc, dv_acc,
+                          false, cu_seqlens_q, cu_seqlens_k, nseq, H, total_q, total_k, max_sq, max_sk, D, q_strides, k_strides, v_strides,
                           do_strides, dq_strides, dk_strides, dv_strides, scale, mask_mode, dtype, stream);
 }
 
@@ -971,9 +987,21 @@ int spa_flash_bwd_varlen_out(const void* q, const void* k, const void* v, const 
                              const int64_t v_strides[2], const int64_t do_strides[2], const int64_t dq_strides[2],
                              const int64_t dk_strides[2], const int64_t dv_strides[2], float scale, int mask_mode,
                              int dtype, void* stream) {
-  return flash_bwd_varlen("spa_flash_bwd_varlen_out", q, k, v, dout, lse, delta, dq, dk, dv, true, cu_seqlens_q,
-                          cu_seqlens_k, nseq, H, total_q, total_k, max_sq, max_sk, D, q_strides, k_strides, v_strides,
+  return flash_bwd_varlen("spa_flash_bwd_varlen_out", q, k, v, nullptr, nullptr, dout, lse, const_cast<float*>(delta), dq, dk, dv, true,
+                          cu_seqlens_q, cu_seqlens_k, nseq, H, total_q, total_k, max_sq, max_sk, D, q_strides, k_strides, v_strides,
                           do_strides, dq_strides, dk_strides, dv_strides, scale, mask_mode, dtype, stream);
+}
+
+int spa_attention_bwd_varlen(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse, float* delta,
+                             void* dq, void* dk, void* dv, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int nseq, int H,
+                             int total_q, int total_k, int max_sq, int max_sk, int D, const int64_t q_strides[2],
+                             const int64_t k_strides[2], const int64_t v_strides[2], const int64_t o_strides[2],
+                             const int64_t do_strides[2], const int64_t dq_strides[2], const int64_t dk_strides[2],
+                             const int64_t dv_strides[2], float scale, int mask_mode, int dtype, void* stream) {
+  if (!out || !o_strides) return fail(SPA_EINVAL, "spa_attention_bwd_varlen: null pointer");
+  return flash_bwd_varlen("spa_attention_bwd_varlen", q, k, v, out, o_strides, dout, lse, delta, dq, dk, dv, true, cu_seqlens_q, cu_seqlens_k,
+                          nseq, H, total_q, total_k, max_sq, max_sk, D, q_strides, k_strides, v_strides, do_strides, dq_strides,
+                          dk_strides, dv_strides, scale, mask_mode, dtype, stream);
 }
 
 }  // extern "C"

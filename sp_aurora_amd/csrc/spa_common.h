@@ -107,7 +107,7 @@ struct BwdParams {
   const void* v;
   const void* dout;
   const float* lse;
-  const float* delta;
+  float* delta;
   float* dq;
   float* dk;
   float* dv;
@@ -122,6 +122,10 @@ struct BwdParams {
   const int* cu_q;
   const int* cu_k;
   int total_k = 0;  // rows of the packed key-side tensors (total_q is lse_bh)
+  // the forward's result: the dq kernel forms delta = rowsum(dout * out) from it and writes it for the dk / dv kernel; null:
+  // delta is the caller's and is read
+  const void* out = nullptr;
+  Strides3 os = {0, 0, 0};
   // 0: dq/dk/dv are fp32 accumulators, added to; 1: they are tensors of q's element type (strides in
   // those elements) and are WRITTEN: the whole gradient comes from this one launch
   int grads_in_t;

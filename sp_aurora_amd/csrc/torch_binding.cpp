@@ -268,9 +268,8 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
     const Tensor delta = empty_f32(lse.sizes(), lse);
     TORCH_CHECK(view_of(out, true, o) && view_of(dout, true, d) && o.same_shape(d) && dout.scalar_type() == q.scalar_type(), "bad gradient of the output");
     const int dtype = dtype_code(q.scalar_type());
-    check(spa_bwd_delta(o.p, d.p, (float*)delta.data_ptr(), o.B, o.H, o.S, o.D, o.st, d.st, dtype, stream));
-    check(spa_flash_bwd_out(x.q.p, x.k.p, x.v.p, d.p, (const float*)lse.const_data_ptr(), (const float*)delta.const_data_ptr(), g.q.p, g.k.p, g.v.p,
-                            x.q.B, x.q.H, x.q.S, x.k.S, x.q.D, x.q.st, x.k.st, x.v.st, d.st, g.q.st, g.k.st, g.v.st,
+    check(spa_attention_bwd(x.q.p, x.k.p, x.v.p, o.p, d.p, (const float*)lse.const_data_ptr(), (float*)delta.data_ptr(), g.q.p, g.k.p, g.v.p,
+                            x.q.B, x.q.H, x.q.S, x.k.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, d.st, g.q.st, g.k.st, g.v.st,
                             softmax_scale_or_default(scale_or_nan, x.q.D), causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype, stream));
     back.push_back(Tensor());
     back.push_back(Tensor());
@@ -317,11 +316,11 @@ struct VarlenAttention : public torch::autograd::Function<VarlenAttention> {
     }
     const Tensor delta = empty_f32(lse.sizes(), lse);
     const int dtype = dtype_code(q.scalar_type());
-    const int64_t os[3] = {0, out.stride(1), out.stride(0)}, ds[3] = {0, d.st[0], d.st[1]};
-    check(spa_bwd_delta(out.const_data_ptr(), d.p, (float*)delta.data_ptr(), 1, a.H, a.S, a.D, os, ds, dtype, stream));
-    check(spa_flash_bwd_varlen_out(a.p, b.p, c.p, d.p, (const float*)lse.const_data_ptr(), (const float*)delta.const_data_ptr(), g[0].p, g[1].p, g[2].p,
+    View o;
+    view_thd(out, o);
+    check(spa_attention_bwd_varlen(a.p, b.p, c.p, o.p, d.p, (const float*)lse.const_data_ptr(), (float*)delta.data_ptr(), g[0].p, g[1].p, g[2].p,
                                    (const int*)s[5].const_data_ptr(), (const int*)s[6].const_data_ptr(), (int)s[5].numel() - 1, a.H, a.S, b.S,
-                                   (int)ctx->saved_data["max_q"].toInt(), (int)ctx->saved_data["max_k"].toInt(), a.D, a.st, b.st, c.st, d.st, g[0].st,
+                                   (int)ctx->saved_data["max_q"].toInt(), (int)ctx->saved_data["max_k"].toInt(), a.D, a.st, b.st, c.st, o.st, d.st, g[0].st,
                                    g[1].st, g[2].st, softmax_scale_or_default(ctx->saved_data["scale"].toDouble(), a.D),
                                    ctx->saved_data["causal"].toBool() ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype, stream));
     back.resize(10);
