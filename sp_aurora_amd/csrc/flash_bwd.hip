@@ -19,8 +19,10 @@
 // contractions) and, through the transposing read, columns (A operands K^T, Q^T, dO^T of the
 // gradient contractions).  No transposed copies exist.
 //
-// One wave per SIMD (the 8-wave dq kernel: two, which also halves the K/V traffic per query row),
-// software-pipelined inside the wave at half-tile (32 rows) granularity:
+// D = 128: one wave per SIMD (the 8-wave dq kernel: two, which also halves the K/V traffic per query row).  D <= 64: both
+// kernels fit two 4-wave workgroups to a CU (256 registers a lane); one covers the other's start, end and LDS latency:
+// [2,4096,32,64] causal backward 582 -> 480 us, [64,512,16,64] 312 -> 243 us.
+// Software-pipelined inside the wave at half-tile (32 rows) granularity:
 // the MFMAs that produce S and dP of half-tile g+1 are interleaved, one to one, with the
 // element-wise work (exp, dS) on half-tile g, followed by the gradient MFMAs of half-tile g.
 // MFMA operands come from LDS through a rolling window that runs ahead of the MFMAs and is
@@ -286,7 +288,7 @@ __device__ __forceinline__ void zero_grad_row(E* rowp, int hh) {
 }
 
 template <typename T, int D, int NW, bool BIG = false>
-__global__ void __launch_bounds__(NW * 64, 1) flash_bwd_dq_kernel(const BwdParams pk) {
+__global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd_dq_kernel(const BwdParams pk) {
   BwdParams p = pk;  // a variable-length batch rewrites the sizes and bases for its sequence below
   typedef BwdCfg<D, NW * 64> C;
   typedef DqCfg<D, NW> G;
@@ -363,7 +365,7 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_dq_kernel(const BwdParam
   //   list 2i+1: S^T, dP^T of half 2i+2 (tile i+1, rows 0..31)  | dS^T of half 2i+1 | dQ of half 2i+1
   // NA MFMAs produce, the element-wise work rides between them, NB MFMAs consume.
   constexpr int NA = 2 * (D / 16), NB = 2 * (D / 32), NLIST = NA + NB, NBODY = 2 * NLIST;
-  constexpr int LOOK_CAP = NW == 8 ? 4 : BWD_LOOK_MAX;  // two waves per SIMD: 256 registers each, and the other wave covers LDS latency
+  constexpr int LOOK_CAP = NW == 8 || D <= 64 ? 4 : BWD_LOOK_MAX;  // two waves per SIMD: 256 registers each, and the other wave covers LDS latency
   constexpr int BWD_LOOK = NA < LOOK_CAP ? NA : LOOK_CAP;
   static_assert(NBODY % BWD_LOOK == 0 && BWD_LOOK <= NA, "the operand window must tile the loop body");
 
@@ -591,7 +593,7 @@ struct DkvCfg {
 // ASM = false: the D = 128 kernel with every MFMA left to the compiler (its uniform accumulator
 // form, its own hazard handling): slower, kept as the test twin of the hand-issued form.
 template <typename T, int D, bool ASM = true, bool BIG = false>
-__global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd_dkdv_kernel(const BwdParams pk) {
+__global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_kernel(const BwdParams pk) {
   BwdParams p = pk;  // a variable-length batch rewrites the sizes and bases for its sequence below
   typedef BwdCfg<D> C;
   typedef DkvCfg<D> G;
@@ -677,7 +679,7 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd_dkdv_kernel(const Bw
   //   list 2i  : S, dP of half 2i+1 (tile i rows 32..63)  | P, dS of half 2i   | dV, dK from half 2i
   //   list 2i+1: S, dP of half 2i+2 (tile i+1 rows 0..31) | P, dS of half 2i+1 | dV, dK from half 2i+1
   constexpr int NA = 2 * (D / 16), NB = 4 * (D / 32), NLIST = NA + NB, NBODY = 2 * NLIST;
-  constexpr int BWD_LOOK = NA < BWD_LOOK_MAX ? NA : BWD_LOOK_MAX;
+  constexpr int BWD_LOOK = D <= 64 ? 4 : BWD_LOOK_MAX;  // (two waves per SIMD at D <= 64, as in the dq kernel)
   static_assert(NBODY % BWD_LOOK == 0 && BWD_LOOK <= NA, "the operand window must tile the loop body");
 
   if (it0 < nt) {  // uniform; a workgroup whose keys no query sees adds nothing
@@ -697,13 +699,13 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd_dkdv_kernel(const Bw
         for (int q = 0; q < C::NDMA; ++q) vld.load(q, k0 + half * BWD_ROWS < p.Sk, k0 + half * BWD_ROWS, vdst + half * C::TILEB);
     }
     issue_tile(it0);
-    issue_tile(it0 + 1);
-    wait_loads_but<2 * G::NL>();
+    wait_loads_but<G::NL>();
     __syncthreads();
     const unsigned own = (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB;  // the wave's 32 keys in either pair of tiles
     read_rows<frag, D>(kf, stage_of(it0 + 2) + own, rd);
     read_rows<frag, D>(vf, stage_of(it0 + 3) + own, rd);
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the stage of tile it0 + 2 has been read ...
+    issue_tile(it0 + 1);
     __syncthreads();                     // ... by every wave
     issue_tile(it0 + 2);
     wait_loads_but<2 * G::NL>();
@@ -1243,13 +1245,14 @@ hipError_t launch(int smem, bool queries, int rows, const BwdParams& p, hipStrea
 
 template <typename T, int D>
 hipError_t launch_both(const BwdParams& p, hipStream_t stream) {
-  // dq kernel: 256-row workgroups (two waves per SIMD, the K/V stream shared by twice the rows) once
-  // there are enough of them to occupy every CU; spa_tune() can force 4 or 8 waves (experiments, tests)
+  // dq kernel, D = 128: 256-row workgroups (two waves per SIMD, the K/V stream shared by twice the rows) once
+  // there are enough of them to occupy every CU; spa_tune() can force 4 or 8 waves (experiments, tests).
+  // At D = 64 two 128-row workgroups to a CU are as fast on long rows (+-2 %) and 4 to 7 % faster on short ones.
   const int64_t wgs8 = p.cu_q ? (int64_t)p.H * (p.lse_bh / 256 + (p.B + 1) / 2) : (int64_t)p.B * p.H * ((p.Sq + 255) / 256);
   const int forced = spa_knob(SPA_KNOB_BWD_DQ_WAVES);
   hipError_t e = hipErrorInvalidValue;
   bool wide = false;
-  if constexpr (D >= 64) {  // a D = 32 tile has fewer 16-byte slots than 512 threads
+  if constexpr (D == 128) {
     wide = forced ? forced == 8 : wgs8 >= spa_device_cus();
     if (wide) e = launch<flash_bwd_dq_kernel<T, D, 8>>(DqCfg<D, 8>::SMEM, true, 256, p, stream, 512);
   }
