@@ -55,6 +55,17 @@ enum {
   SPA_ELAUNCH = -4      /* HIP runtime refused the launch */
 };
 
+/*
+ * Rows of a sequence that lie in shards: the sequence is cut into `shards` parts of equal length; part r lies in shard r, and
+ * shard r + 1 starts `pitch` rows after shard r (`lse_pitch` entries in lse).  With zigzag, shard r holds parts r and
+ * 2 * shards - 1 - r of 2 * shards, one after the other.  What a single GPU holds of a ring's or a Ulysses group's ranks: the
+ * rank-stacked tensors of the reference's per-rank calls (sp_aurora/hybrid/long_ctx_attention.py:131-195), zigzag-sharded ring
+ * tensors (test/flash_attention/test_intel_ring_flash_attn_varlen.py:25,205-215).
+ */
+typedef struct {
+  int shards, pitch, lse_pitch, zigzag;
+} spa_shards;
+
 /* Library identity.  Replaces `is_available()` / `get_device_info()` of the
  * reference plugin (sp_aurora/sycl_bindings/bindings.cpp:298-313,357-368). */
 int spa_abi_version(void);
@@ -376,10 +387,27 @@ int spa_flash_bwd_out(const void* q, const void* k, const void* v, const void* d
                       float scale, int mask_mode, int dtype, void* stream);
 
 /*
+ * spa_flash_fwd and spa_flash_fwd_varlen over sequences whose rows lie in shards (16-bit types: k and v with one row stride, less
+ * than 2 GiB per (batch, head)): the sequence is walked in its own order, so the ring over the shards is one block call.
+ * Sq = Sk = S, a multiple of the shards (twice the shards with zigzag).  _varlen: cu_seqlens describes one shard of total_rows
+ * rows (every shard is packed the same way; zigzag: every length even), max_seqlen is the longest sequence's rows in one
+ * shard, lse is fp32 [H, shards * total_rows].  Replaces the step loop of sp_aurora/intel_ring_flash_attn.py:72-148.
+ */
+int spa_attention_fwd(const void* q, const void* k, const void* v, void* out, float* lse, int B, int H, int S, int D,
+                      const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
+                      const int64_t o_strides[3], const spa_shards* rows, float scale, int mask_mode, int dtype, void* stream);
+int spa_attention_fwd_varlen(const void* q, const void* k, const void* v, void* out, float* lse, const int32_t* cu_seqlens,
+                             int nseq, int H, int total_rows, int max_seqlen, int D, const int64_t q_strides[2],
+                             const int64_t k_strides[2], const int64_t v_strides[2], const int64_t o_strides[2],
+                             const spa_shards* rows, float scale, int mask_mode, int dtype, void* stream);
+
+/*
  * spa_flash_bwd_out from the forward's result: out (q's shape and type) in place of delta, which is scratch here (fp32,
  * contiguous [B,H,Sq]): delta = rowsum(dout * out) is formed by the kernel that computes dq, for its own rows, and read by the
  * one that computes dk and dv.  Replaces intel_ring_flash_attn_backward (sp_aurora/intel_ring_flash_attn.py:153-271) for a
  * ring whose shards are all on this GPU, and the block's own backward.
+ * rows: null, or where the rows of every tensor (and of lse and delta) lie; then Sq = Sk = the whole sequence's rows, and K / V, q
+ * and dout of one (batch, head) span less than 2 GiB.
  */
 int spa_attention_bwd(const void* q, const void* k, const void* v, const void* out, const void* dout,
                       const float* lse, float* delta, void* dq, void* dk, void* dv,
@@ -388,7 +416,7 @@ int spa_attention_bwd(const void* q, const void* k, const void* v, const void* o
                       const int64_t v_strides[3], const int64_t o_strides[3],
                       const int64_t do_strides[3], const int64_t dq_strides[3],
                       const int64_t dk_strides[3], const int64_t dv_strides[3],
-                      float scale, int mask_mode, int dtype, void* stream);
+                      const spa_shards* rows, float scale, int mask_mode, int dtype, void* stream);
 
 /*
  * Block attention over a batch of sequences of different lengths packed back
@@ -482,7 +510,7 @@ int spa_flash_bwd_varlen_out(const void* q, const void* k, const void* v, const 
 
 /*
  * spa_flash_bwd_varlen_out from the forward's result, as spa_attention_bwd is to spa_flash_bwd_out (out [total_q, H, D], delta:
- * scratch, fp32 [H, total_q]).
+ * scratch, fp32 [H, total_q]).  rows: as in spa_attention_fwd_varlen (total_q = total_k = rows of one shard).
  */
 int spa_attention_bwd_varlen(const void* q, const void* k, const void* v, const void* out, const void* dout,
                              const float* lse, float* delta, void* dq, void* dk, void* dv,
@@ -492,7 +520,7 @@ int spa_attention_bwd_varlen(const void* q, const void* k, const void* v, const 
                              const int64_t v_strides[2], const int64_t o_strides[2],
                              const int64_t do_strides[2], const int64_t dq_strides[2],
                              const int64_t dk_strides[2], const int64_t dv_strides[2],
-                             float scale, int mask_mode, int dtype, void* stream);
+                             const spa_shards* rows, float scale, int mask_mode, int dtype, void* stream);
 
 /*
  * Kernel-variant override for experiments and tests; no counterpart in the reference and not

@@ -21,6 +21,14 @@ _i = ctypes.c_int
 _f = ctypes.c_float
 _s3 = ctypes.POINTER(ctypes.c_int64)
 
+
+class Shards(ctypes.Structure):
+    """spa_shards of the C ABI: where the rows of a sequence lie."""
+    _fields_ = [("shards", _i), ("pitch", _i), ("lse_pitch", _i), ("zigzag", _i)]
+
+
+_sh = ctypes.POINTER(Shards)
+
 # name -> (restype, argtypes); mirrors include/sp_aurora_hip.h declaration by declaration
 SIGNATURES = {
     "spa_abi_version": (_i, []),
@@ -52,8 +60,10 @@ SIGNATURES = {
     "spa_bwd_delta": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _s3, _s3, _i, _vp]),
     "spa_flash_bwd": (_i, [_vp] * 9 + [_i] * 5 + [_s3] * 7 + [_f, _i, _i, _vp]),
     "spa_flash_bwd_out": (_i, [_vp] * 9 + [_i] * 5 + [_s3] * 7 + [_f, _i, _i, _vp]),
-    "spa_attention_bwd": (_i, [_vp] * 10 + [_i] * 5 + [_s3] * 8 + [_f, _i, _i, _vp]),
-    "spa_attention_bwd_varlen": (_i, [_vp] * 12 + [_i] * 7 + [_s3] * 8 + [_f, _i, _i, _vp]),
+    "spa_attention_fwd": (_i, [_vp] * 5 + [_i] * 4 + [_s3] * 4 + [_sh, _f, _i, _i, _vp]),
+    "spa_attention_fwd_varlen": (_i, [_vp] * 6 + [_i] * 5 + [_s3] * 4 + [_sh, _f, _i, _i, _vp]),
+    "spa_attention_bwd": (_i, [_vp] * 10 + [_i] * 5 + [_s3] * 8 + [_sh, _f, _i, _i, _vp]),
+    "spa_attention_bwd_varlen": (_i, [_vp] * 12 + [_i] * 7 + [_s3] * 8 + [_sh, _f, _i, _i, _vp]),
     "spa_flash_fwd_varlen": (_i, [_vp] * 7 + [_i] * 7 + [_s3] * 4 + [_f, _i, _i, _vp]),
     "spa_ring_fwd_varlen": (_i, [_vp] * 6 + [_i] * 7 + [_s3] * 4 + [_f, _i, _i, _i, _vp]),
     "spa_flash_bwd_varlen": (_i, [_vp] * 11 + [_i] * 7 + [_s3] * 7 + [_f, _i, _i, _vp]),

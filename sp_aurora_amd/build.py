@@ -12,7 +12,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libsp_aurora_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 NATIVE_PATH = os.path.join(HERE, "_native.so")
-# (source, object, extra flags).  flash_fwd.hip makes three objects: the zigzag variants of the 16-bit forward kernel
+# (source, object, extra flags).  flash_fwd.hip makes five objects: the zigzag variants of the 16-bit forward kernel
 # and the variants for tensors of 2 GiB and more per (batch, head) are translation units of their own, so that the
 # parts of the longest compile run side by side; flash_bwd.hip likewise makes two.
 # The forward kernels' softmax phase gains 1-3 % from the scheduler that maximises instruction-level
@@ -23,8 +23,9 @@ UNITS = [
     ("flash_fwd.hip", "flash_fwd_zigzag.o", _FWD + ["-DSPA_FWD_ZIGZAG_UNIT"]),
     ("flash_fwd.hip", "flash_fwd_big.o", _FWD + ["-DSPA_FWD_BIG_UNIT"]),
     ("flash_fwd.hip", "flash_fwd_splitkv.o", _FWD + ["-DSPA_FWD_SPLITKV_UNIT"]),
+    ("flash_fwd.hip", "flash_fwd_map.o", _FWD + ["-DSPA_FWD_MAP_UNIT"]),
     ("flash_bwd.hip", "flash_bwd.o", []),
-    ("flash_bwd.hip", "flash_bwd_big.o", ["-DSPA_BWD_BIG_UNIT"]),
+    ("flash_bwd.hip", "flash_bwd_other.o", ["-DSPA_BWD_OTHER_UNIT"]),
     ("spa_abi.hip", "spa_abi.o", []),
     ("merge.hip", "merge.o", []),
     ("decode_fwd.hip", "decode_fwd.o", []),

@@ -86,36 +86,46 @@ struct TileReads {
 
 // Global side of the direct loads: thread tid owns 16-byte slot tid of every round of 256 slots;
 // round j covers rows j * RPD + tid / CPR.  Slot (row, pos) receives chunk pos ^ swizzle(row).
-// BIG: the tensor's rows of one (batch, head) may span 2 GiB or more; the descriptor is re-based per tile
-// (buffer_window) instead of covering the whole tensor.
-template <typename T, int D, int THREADS = BWD_THREADS, bool BIG = false>
+// ADDR_BIG: the tensor's rows of one (batch, head) may span 2 GiB or more; the descriptor is re-based per tile
+// (buffer_window) instead of covering the whole tensor.  ADDR_MAP: the rows lie in shards (RowMap): every lane looks up
+// its row (about 15 vector instructions per load, in the shadow of the MFMAs between which the loads are issued).
+enum { ADDR_PLAIN = 0, ADDR_BIG = 1, ADDR_MAP = 2 };
+template <typename T, int D, int THREADS = BWD_THREADS, int ADDR = ADDR_PLAIN>
 struct TileLoader {
   u32x4 rsrc;
   unsigned lane_off;  // bytes
   unsigned row_b;     // bytes per tensor row
-  const T* base_;             // BIG only
-  unsigned long long total_;  // BIG only: bytes from base_ to the end of the last row
-  __device__ __forceinline__ void init(const T* base, int64_t row_stride, int rows, int tid) {
+  const T* base_;             // ADDR_BIG only
+  unsigned long long total_;  // ADDR_BIG only: bytes from base_ to the end of the last row
+  int rows_, drow_;           // ADDR_MAP only
+  // rows: rows of the sequence; span: rows of the tensor from base to the sequence's last row
+  __device__ __forceinline__ void init(const T* base, int64_t row_stride, int rows, int span, int tid) {
     typedef BwdCfg<D, THREADS> C;
-    total_ = (unsigned long long)((((int64_t)rows - 1) * row_stride + D) * (int64_t)sizeof(T));
+    total_ = (unsigned long long)((((int64_t)span - 1) * row_stride + D) * (int64_t)sizeof(T));
     base_ = base;
-    rsrc = buffer_descriptor(base, BIG ? 0u : (unsigned)total_);  // (BIG: an empty range, for tiles that are not wanted)
+    rsrc = buffer_descriptor(base, ADDR == ADDR_BIG ? 0u : (unsigned)total_);  // (ADDR_BIG: an empty range, for tiles that are not wanted)
     const int drow = tid / C::CPR, dpos = tid % C::CPR;
-    lane_off = (unsigned)((drow * row_stride + ((dpos ^ tile_swizzle<D>(drow)) * 8)) * (int64_t)sizeof(T));
+    rows_ = rows;
+    drow_ = drow;
+    lane_off = (unsigned)(((ADDR == ADDR_MAP ? 0 : drow * row_stride) + ((dpos ^ tile_swizzle<D>(drow)) * 8)) * (int64_t)sizeof(T));
     row_b = (unsigned)(row_stride * (int64_t)sizeof(T));
   }
-  // round q of the tile whose first tensor row is row0 (on = false: store zeros) into LDS at lds_wave
-  __device__ __forceinline__ void load(int q, bool on, int row0, unsigned lds_wave) const {
+  // round q of the tile whose first row is row0 (on = false: store zeros) into LDS at lds_wave
+  __device__ __forceinline__ void load(int q, bool on, int row0, unsigned lds_wave, const RowMap& map, int pitch) const {
     typedef BwdCfg<D, THREADS> C;
-    if constexpr (BIG) {
+    if constexpr (ADDR == ADDR_MAP) {
+      const int r = row0 + q * C::RPD + drow_;
+      const unsigned off = lane_off + (unsigned)map.at(r, pitch) * row_b;
+      load_to_lds_b128(rsrc, on && r < rows_ ? off : OFF_NONE, lds_wave + q * (THREADS * 16));
+    } else if constexpr (ADDR == ADDR_BIG) {
       unsigned rel = OFF_NONE;
       u32x4 rs = rsrc;
       if (on) rs = buffer_window(base_, total_, (unsigned long long)(unsigned)row0 * row_b, rel);
       load_to_lds_b128(rs, lane_off + rel + (unsigned)(q * C::RPD) * row_b, lds_wave + q * (THREADS * 16));
-      return;
+    } else {
+      const unsigned u = on ? (unsigned)(row0 + q * C::RPD) * row_b : OFF_NONE;
+      load_to_lds_b128(rsrc, lane_off + u, lds_wave + q * (THREADS * 16));
     }
-    const unsigned u = on ? (unsigned)(row0 + q * C::RPD) * row_b : OFF_NONE;
-    load_to_lds_b128(rsrc, lane_off + u, lds_wave + q * (THREADS * 16));
   }
 };
 
@@ -131,9 +141,9 @@ __device__ __forceinline__ void read_rows(F (&f)[D / 16], unsigned rows_at, cons
 // Writes the wave's 32 rows of a gradient (accumulator layout: a lane holds, of row ln, dims 32 db + 8 g + 4 hh .. + 3) in T.
 // Through LDS (32 rows of the wave's own, chunks XOR-permuted), so that a store instruction writes whole rows: the 8-byte
 // pieces a lane holds are 32 cache lines per instruction, and the last 6 us of a workgroup went into them.
-// first_row: number of rows that exist from the wave's first row on; stride in elements.
-template <typename T, int D>
-__device__ __forceinline__ void store_rows(const f32x16 (&acc)[D / 32], float scale, T* rows, int64_t stride, int n_rows, unsigned char* lds, int lane) {
+// n_rows: rows that exist from the wave's first row on; row(r): where row r of the wave's goes.
+template <typename T, int D, typename Row>
+__device__ __forceinline__ void store_rows(const f32x16 (&acc)[D / 32], float scale, Row&& row, int n_rows, unsigned char* lds, int lane) {
   constexpr int CPR = D / 8;  // 16-byte chunks per row
   const int ln = lane & 31, hh = lane >> 5;
 #pragma unroll
@@ -150,7 +160,7 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[D / 32], float sc
   for (int i = 0; i < 32 * CPR / 64; ++i) {
     const int r = i * (64 / CPR) + lane / CPR, ch = lane % CPR;
     const u32x4 x = *(const u32x4*)(lds + r * (D * 2) + ((ch ^ (r & (CPR - 1))) * 16));
-    if (r < n_rows) *(u32x4*)(rows + (int64_t)r * stride + ch * 8) = x;
+    if (r < n_rows) *(u32x4*)((T*)row(r) + ch * 8) = x;
   }
 }
 
@@ -228,9 +238,13 @@ struct DqCfg {
 // Variable-length batch: sequence b owns rows cu_q[b] .. cu_q[b+1] of the query-side tensors and
 // cu_k[b] .. cu_k[b+1] of the key-side ones; the kernel then works on that sequence as on batch 0
 // of a batch whose bases and sizes are the sequence's.
+// map: set up for the sequence's rows where they lie in shards (the sequence is then p.map.P times as long as cu says).
 template <typename T>
-__device__ __forceinline__ void select_sequence(BwdParams& p, int& b) {
-  if (!p.cu_q) return;
+__device__ __forceinline__ void select_sequence(BwdParams& p, int& b, RowMap& map) {
+  if (!p.cu_q) {
+    if (p.map.P) map.init(p.map, p.Sq / p.map.P);
+    return;
+  }
   const int q_lo = p.cu_q[b], k_lo = p.cu_k[b];
   p.Sq = p.cu_q[b + 1] - q_lo;
   p.Sk = p.cu_k[b + 1] - k_lo;
@@ -246,6 +260,11 @@ __device__ __forceinline__ void select_sequence(BwdParams& p, int& b) {
   p.lse += q_lo;
   p.delta += q_lo;
   b = 0;
+  if (p.map.P) {
+    map.init(p.map, p.Sq);
+    p.Sq *= p.map.P;
+    p.Sk = p.Sq;
+  }
 }
 
 // The (batch or sequence, head) and the tile (of `rows` query rows, or keys) of a workgroup: pairs first, in groups
@@ -256,7 +275,7 @@ __device__ __forceinline__ bool workgroup_tile(const BwdParams& p, bool queries,
   if (p.cu_q) {
     const int number = blockIdx.x / p.H;
     h = blockIdx.x - number * p.H;
-    if (!sequence_tile(queries ? p.cu_q : p.cu_k, p.B, rows, number, lane, b, tile, n)) return false;
+    if (!sequence_tile(queries ? p.cu_q : p.cu_k, p.B, p.map.P ? p.map.P : 1, rows, number, lane, b, tile, n)) return false;
   } else {
     const int pair = blockIdx.x + blockIdx.z * gridDim.x;
     if (pair >= p.B * p.H) return false;
@@ -287,7 +306,7 @@ __device__ __forceinline__ void zero_grad_row(E* rowp, int hh) {
     }
 }
 
-template <typename T, int D, int NW, bool BIG = false>
+template <typename T, int D, int NW, int ADDR = ADDR_PLAIN>
 __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd_dq_kernel(const BwdParams pk) {
   BwdParams p = pk;  // a variable-length batch rewrites the sizes and bases for its sequence below
   typedef BwdCfg<D, NW * 64> C;
@@ -309,10 +328,16 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   if (!workgroup_tile(p, true, NW * 32, lane, b, h, qt)) return;
   const int q0 = qt * (NW * 32);
   const int qw0 = q0 + w * 32;
-  select_sequence<T>(p, b);
+  RowMap map = {};
+  select_sequence<T>(p, b, map);
+  constexpr bool MAP = ADDR == ADDR_MAP;
+  auto row_of = [&](int r) { return MAP ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
+  auto stat_of = [&](int r) { return MAP ? map.at(r, p.map.lse_pitch) : r; };   // in lse and delta
+  // rows of the tensors from the sequence's first to its last
+  const int span_q = MAP ? (p.map.P - 1) * p.map.pitch + p.Sq / p.map.P : p.Sq, span_k = MAP ? span_q : p.Sk;
   if (q0 >= p.Sq || p.Sk <= 0) {  // (variable-length batches only) no keys: nothing to add to dq, a written dq is zero
     if (p.grads_in_t && qw0 + ln < p.Sq)
-      zero_grad_row<T, D>((T*)p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)(qw0 + ln) * p.dqs.s, hh);
+      zero_grad_row<T, D>((T*)p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)row_of(qw0 + ln) * p.dqs.s, hh);
     return;
   }
 
@@ -325,7 +350,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   const int qrow_c = qrow < p.Sq ? qrow : p.Sq - 1;
 
   frag qf[D / 16], dof[D / 16];
-  const int64_t li = ((int64_t)b * p.H + h) * p.lse_bh + qrow_c;
+  const int64_t li = ((int64_t)b * p.H + h) * p.lse_bh + stat_of(qrow_c);
   const float l2 = p.lse[li] * 1.4426950408889634f;
   const float c = p.scale_log2;
   const float hidden = c < 0.f ? INFINITY : -INFINITY;  // a hidden score: exp2(hidden * c - lse) = 0 for either sign of the scale
@@ -334,9 +359,9 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   const int kv_end = p.causal ? (q0 + NW * 32 < p.Sk ? q0 + NW * 32 : p.Sk) : p.Sk;
   const int nt = (kv_end + BWD_ROWS - 1) / BWD_ROWS;  // key tiles this workgroup visits
 
-  TileLoader<T, D, NW * 64, BIG> kld, vld;
-  kld.init(kp, p.ks.s, p.Sk, tid);
-  vld.init(vp, p.vs.s, p.Sk, tid);
+  TileLoader<T, D, NW * 64, ADDR> kld, vld;
+  kld.init(kp, p.ks.s, p.Sk, span_k, tid);
+  vld.init(vp, p.vs.s, p.Sk, span_k, tid);
   TileReads<D> rd;
   rd.init(lane);
   const unsigned lds0 = (unsigned)(uintptr_t)(lds_u8*)smem;
@@ -344,16 +369,16 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   auto issue_tile = [&](int i) {  // K and V tile i -> its stage
     const unsigned dst = stage_of(i) + w * 1024;
 #pragma unroll
-    for (int q = 0; q < C::NDMA; ++q) kld.load(q, i < nt, i * BWD_ROWS, dst);
+    for (int q = 0; q < C::NDMA; ++q) kld.load(q, i < nt, i * BWD_ROWS, dst, map, p.map.pitch);
 #pragma unroll
-    for (int q = 0; q < C::NDMA; ++q) vld.load(q, i < nt, i * BWD_ROWS, dst + C::TILEB);
+    for (int q = 0; q < C::NDMA; ++q) vld.load(q, i < nt, i * BWD_ROWS, dst + C::TILEB, map, p.map.pitch);
   };
   auto issue_one = [&](int i, int n) {  // load n of tile i's G::NL, in issue_tile's order
     const unsigned dst = stage_of(i) + w * 1024;
     if (n < C::NDMA)
-      kld.load(n, i < nt, i * BWD_ROWS, dst);
+      kld.load(n, i < nt, i * BWD_ROWS, dst, map, p.map.pitch);
     else
-      vld.load(n - C::NDMA, i < nt, i * BWD_ROWS, dst + C::TILEB);
+      vld.load(n - C::NDMA, i < nt, i * BWD_ROWS, dst + C::TILEB, map, p.map.pitch);
   };
 
   f32x16 dq[D / 32];
@@ -374,12 +399,12 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   {
     constexpr int RT = NW / 2;  // tiles of 64 rows
     auto load_rows = [&](const T* base, int64_t stride, unsigned dst) {
-      TileLoader<T, D, NW * 64, BIG> ld;
-      ld.init(base, stride, p.Sq, tid);
+      TileLoader<T, D, NW * 64, ADDR> ld;
+      ld.init(base, stride, p.Sq, span_q, tid);
 #pragma unroll
       for (int i = 0; i < RT; ++i)
 #pragma unroll
-        for (int q = 0; q < C::NDMA; ++q) ld.load(q, q0 + i * BWD_ROWS < p.Sq, q0 + i * BWD_ROWS, dst + i * C::TILEB + w * 1024);
+        for (int q = 0; q < C::NDMA; ++q) ld.load(q, q0 + i * BWD_ROWS < p.Sq, q0 + i * BWD_ROWS, dst + i * C::TILEB + w * 1024, map, p.map.pitch);
     };
     const unsigned own = (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB, other = 2 * G::STAGE;
     load_rows(qp, p.qs.s, lds0);
@@ -560,7 +585,8 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   if (p.grads_in_t) {
     // the whole gradient of the row: written in q's element type, nothing read
     __syncthreads();  // every wave is done with the tiles, and with its loads into them
-    store_rows<T, D>(dq, p.scale, (T*)p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)qw0 * p.dqs.s, p.dqs.s, p.Sq - qw0, smem + w * (32 * C::ROWB), lane);
+    T* const dqp = (T*)p.dq + b * p.dqs.b + h * p.dqs.h;
+    store_rows<T, D>(dq, p.scale, [&](int r) { return dqp + (int64_t)row_of(qw0 + r) * p.dqs.s; }, p.Sq - qw0, smem + w * (32 * C::ROWB), lane);
   } else if (qrow < p.Sq) {
     float* dqp = p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)qrow * p.dqs.s;
 #pragma unroll
@@ -592,7 +618,7 @@ struct DkvCfg {
 
 // ASM = false: the D = 128 kernel with every MFMA left to the compiler (its uniform accumulator
 // form, its own hazard handling): slower, kept as the test twin of the hand-issued form.
-template <typename T, int D, bool ASM = true, bool BIG = false>
+template <typename T, int D, bool ASM = true, int ADDR = ADDR_PLAIN>
 __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_kernel(const BwdParams pk) {
   BwdParams p = pk;  // a variable-length batch rewrites the sizes and bases for its sequence below
   typedef BwdCfg<D> C;
@@ -611,11 +637,17 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
   if (!workgroup_tile(p, false, 128, lane, b, h, kt)) return;
   const int k0 = kt * 128;
   const int kw0 = k0 + w * 32;
-  select_sequence<T>(p, b);
+  RowMap map = {};
+  select_sequence<T>(p, b, map);
+  constexpr bool MAP = ADDR == ADDR_MAP;
+  auto row_of = [&](int r) { return MAP ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
+  auto stat_of = [&](int r) { return MAP ? map.at(r, p.map.lse_pitch) : r; };   // in lse and delta
+  // rows of the tensors from the sequence's first to its last
+  const int span_q = MAP ? (p.map.P - 1) * p.map.pitch + p.Sq / p.map.P : p.Sq, span_k = MAP ? span_q : p.Sk;
   if (k0 >= p.Sk || p.Sq <= 0 || (p.causal && k0 >= p.Sq)) {  // no query sees these keys: nothing to add to dk, dv
     if (p.grads_in_t && kw0 + ln < p.Sk) {                     // written gradients of such keys are zero
-      zero_grad_row<T, D>((T*)p.dk + b * p.dks.b + h * p.dks.h + (int64_t)(kw0 + ln) * p.dks.s, hh);
-      zero_grad_row<T, D>((T*)p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)(kw0 + ln) * p.dvs.s, hh);
+      zero_grad_row<T, D>((T*)p.dk + b * p.dks.b + h * p.dks.h + (int64_t)row_of(kw0 + ln) * p.dks.s, hh);
+      zero_grad_row<T, D>((T*)p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)row_of(kw0 + ln) * p.dvs.s, hh);
     }
     return;
   }
@@ -636,12 +668,13 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
   const int it0 = p.causal ? k0 / BWD_ROWS : 0;
   const int nt = (p.Sq + BWD_ROWS - 1) / BWD_ROWS;  // query tiles it0 .. nt-1 are visited
 
-  TileLoader<T, D, BWD_THREADS, BIG> qld, dold;
-  qld.init(qp, p.qs.s, p.Sq, tid);
-  dold.init(dop, p.dos.s, p.Sq, tid);
+  TileLoader<T, D, BWD_THREADS, ADDR> qld, dold;
+  qld.init(qp, p.qs.s, p.Sq, span_q, tid);
+  dold.init(dop, p.dos.s, p.Sq, span_q, tid);
   // per-row statistics: waves 0, 2 fetch the tile's 64 lse values, waves 1, 3 its 64 delta values
   // (the pairs store the same bytes to the same place, which keeps every wave's load count equal)
-  const u32x4 stat_rsrc = buffer_descriptor((w & 1) ? delp : lsep, (unsigned)p.Sq * 4u);
+  const u32x4 stat_rsrc = buffer_descriptor((w & 1) ? delp : lsep, (unsigned)(MAP ? (p.map.P - 1) * p.map.lse_pitch + p.Sq / p.map.P : p.Sq) * 4u);
+  auto stat_offset = [&](bool on, int r) { return on && (!MAP || r < p.Sq) ? (unsigned)stat_of(r) * 4u : OFF_NONE; };
   TileReads<D> rd;
   rd.init(lane);
   const unsigned lds0 = (unsigned)(uintptr_t)(lds_u8*)smem;
@@ -650,21 +683,21 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     const unsigned st = stage_of(i);
     const unsigned dst = st + w * 1024;
 #pragma unroll
-    for (int q = 0; q < C::NDMA; ++q) qld.load(q, i < nt, i * BWD_ROWS, dst);
+    for (int q = 0; q < C::NDMA; ++q) qld.load(q, i < nt, i * BWD_ROWS, dst, map, p.map.pitch);
 #pragma unroll
-    for (int q = 0; q < C::NDMA; ++q) dold.load(q, i < nt, i * BWD_ROWS, dst + C::TILEB);
-    load_to_lds_b32(stat_rsrc, i < nt ? (unsigned)(i * BWD_ROWS + lane) * 4u : OFF_NONE,
+    for (int q = 0; q < C::NDMA; ++q) dold.load(q, i < nt, i * BWD_ROWS, dst + C::TILEB, map, p.map.pitch);
+    load_to_lds_b32(stat_rsrc, stat_offset(i < nt, i * BWD_ROWS + lane),
                     st + 2 * C::TILEB + (w & 1) * (BWD_ROWS * 4));
   };
   auto issue_one = [&](int i, int n) {  // load n of tile i's G::NL, in issue_tile's order
     const unsigned st = stage_of(i);
     const unsigned dst = st + w * 1024;
     if (n < C::NDMA)
-      qld.load(n, i < nt, i * BWD_ROWS, dst);
+      qld.load(n, i < nt, i * BWD_ROWS, dst, map, p.map.pitch);
     else if (n < 2 * C::NDMA)
-      dold.load(n - C::NDMA, i < nt, i * BWD_ROWS, dst + C::TILEB);
+      dold.load(n - C::NDMA, i < nt, i * BWD_ROWS, dst + C::TILEB, map, p.map.pitch);
     else
-      load_to_lds_b32(stat_rsrc, i < nt ? (unsigned)(i * BWD_ROWS + lane) * 4u : OFF_NONE,
+      load_to_lds_b32(stat_rsrc, stat_offset(i < nt, i * BWD_ROWS + lane),
                       st + 2 * C::TILEB + (w & 1) * (BWD_ROWS * 4));
   };
 
@@ -685,18 +718,18 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
   if (it0 < nt) {  // uniform; a workgroup whose keys no query sees adds nothing
     // the workgroup's keys first, as two tiles each of K and V in the stages of tiles it0 + 2 and it0 + 3
     {
-      TileLoader<T, D, BWD_THREADS, BIG> kld, vld;
-      kld.init(kp, p.ks.s, p.Sk, tid);
-      vld.init(vp, p.vs.s, p.Sk, tid);
+      TileLoader<T, D, BWD_THREADS, ADDR> kld, vld;
+      kld.init(kp, p.ks.s, p.Sk, span_k, tid);
+      vld.init(vp, p.vs.s, p.Sk, span_k, tid);
       const unsigned kdst = stage_of(it0 + 2) + w * 1024, vdst = stage_of(it0 + 3) + w * 1024;
 #pragma unroll
       for (int half = 0; half < 2; ++half)
 #pragma unroll
-        for (int q = 0; q < C::NDMA; ++q) kld.load(q, k0 + half * BWD_ROWS < p.Sk, k0 + half * BWD_ROWS, kdst + half * C::TILEB);
+        for (int q = 0; q < C::NDMA; ++q) kld.load(q, k0 + half * BWD_ROWS < p.Sk, k0 + half * BWD_ROWS, kdst + half * C::TILEB, map, p.map.pitch);
 #pragma unroll
       for (int half = 0; half < 2; ++half)
 #pragma unroll
-        for (int q = 0; q < C::NDMA; ++q) vld.load(q, k0 + half * BWD_ROWS < p.Sk, k0 + half * BWD_ROWS, vdst + half * C::TILEB);
+        for (int q = 0; q < C::NDMA; ++q) vld.load(q, k0 + half * BWD_ROWS < p.Sk, k0 + half * BWD_ROWS, vdst + half * C::TILEB, map, p.map.pitch);
     }
     issue_tile(it0);
     wait_loads_but<G::NL>();
@@ -871,10 +904,10 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
 
   if (p.grads_in_t) {
     __syncthreads();  // every wave is done with the tiles, and with its loads into them
-    T* const dkp = (T*)p.dk + b * p.dks.b + h * p.dks.h + (int64_t)kw0 * p.dks.s;
-    T* const dvp = (T*)p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)kw0 * p.dvs.s;
-    store_rows<T, D>(dv, 1.f, dvp, p.dvs.s, p.Sk - kw0, smem + w * (64 * C::ROWB), lane);
-    store_rows<T, D>(dk, p.scale, dkp, p.dks.s, p.Sk - kw0, smem + w * (64 * C::ROWB) + 32 * C::ROWB, lane);
+    T* const dkp = (T*)p.dk + b * p.dks.b + h * p.dks.h;
+    T* const dvp = (T*)p.dv + b * p.dvs.b + h * p.dvs.h;
+    store_rows<T, D>(dv, 1.f, [&](int r) { return dvp + (int64_t)row_of(kw0 + r) * p.dvs.s; }, p.Sk - kw0, smem + w * (64 * C::ROWB), lane);
+    store_rows<T, D>(dk, p.scale, [&](int r) { return dkp + (int64_t)row_of(kw0 + r) * p.dks.s; }, p.Sk - kw0, smem + w * (64 * C::ROWB) + 32 * C::ROWB, lane);
   } else if (krow < p.Sk) {
     float* dkp = p.dk + b * p.dks.b + h * p.dks.h + (int64_t)krow * p.dks.s;
     float* dvp = p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)krow * p.dvs.s;
@@ -921,14 +954,15 @@ template <int D>
 struct PairStage {
   typedef Bwd32Cfg<D> C;
   f32x4 ra[C::PASS], rb[C::PASS];
-  __device__ __forceinline__ void gload(const float* a, int64_t as, const float* b, int64_t bs, int row0, int nrows, int tid) {
+  template <typename Row>
+  __device__ __forceinline__ void gload(const float* a, int64_t as, const float* b, int64_t bs, int row0, int nrows, int tid, Row&& row_of) {
     const int cc = tid % C::CPR, cr = tid / C::CPR;
 #pragma unroll
     for (int i = 0; i < C::PASS; ++i) {
       const int lr = cr + i * C::RPP;
       if (lr < B32_ROWS) {
         int r = row0 + lr;
-        r = r < nrows ? r : nrows - 1;
+        r = row_of(r < nrows ? r : nrows - 1);
         ra[i] = *(const f32x4*)(a + (int64_t)r * as + cc * 4);
         rb[i] = *(const f32x4*)(b + (int64_t)r * bs + cc * 4);
       }
@@ -960,10 +994,13 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dq_kernel(const Bw
   if (!workgroup_tile(p, true, 128, lane, b, h, qt)) return;
   const int q0 = qt * 128;
   const int qw0 = q0 + w * 32;
-  select_sequence<float>(p, b);
+  RowMap map = {};
+  select_sequence<float>(p, b, map);
+  auto row_of = [&](int r) { return p.map.P ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
+  auto stat_of = [&](int r) { return p.map.P ? map.at(r, p.map.lse_pitch) : r; };   // in lse and delta
   if (q0 >= p.Sq || p.Sk <= 0) {  // (variable-length batches only) no keys: nothing to add to dq, a written dq is zero
     if (p.grads_in_t && qw0 + ln < p.Sq)
-      zero_grad_row<float, D>(p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)(qw0 + ln) * p.dqs.s, hh);
+      zero_grad_row<float, D>(p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)row_of(qw0 + ln) * p.dqs.s, hh);
     return;
   }
 
@@ -978,14 +1015,14 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dq_kernel(const Bw
   f32x4 qf[D / 8], dof[D / 8];
 #pragma unroll
   for (int g = 0; g < D / 8; ++g) {
-    qf[g] = *(const f32x4*)(qp + (int64_t)qrow_c * p.qs.s + 8 * g + 4 * hh);
-    dof[g] = *(const f32x4*)(dop + (int64_t)qrow_c * p.dos.s + 8 * g + 4 * hh);
+    qf[g] = *(const f32x4*)(qp + (int64_t)row_of(qrow_c) * p.qs.s + 8 * g + 4 * hh);
+    dof[g] = *(const f32x4*)(dop + (int64_t)row_of(qrow_c) * p.dos.s + 8 * g + 4 * hh);
   }
-  const int64_t li = ((int64_t)b * p.H + h) * p.lse_bh + qrow_c;
+  const int64_t li = ((int64_t)b * p.H + h) * p.lse_bh + stat_of(qrow_c);
   const float l2 = p.lse[li] * 1.4426950408889634f;
   float dl;
   if (p.out) {  // delta = rowsum(dout * out), written for the dk / dv kernel
-    const float* op = (const float*)p.out + b * p.os.b + h * p.os.h + (int64_t)qrow_c * p.os.s;
+    const float* op = (const float*)p.out + b * p.os.b + h * p.os.h + (int64_t)row_of(qrow_c) * p.os.s;
     float sum = 0.f;
 #pragma unroll
     for (int g = 0; g < D / 8; ++g) {
@@ -1009,7 +1046,7 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dq_kernel(const Bw
   for (int i = 0; i < D / 32; ++i) zero16(dq[i]);
 
   PairStage<D> st;
-  st.gload(kp, p.ks.s, vp, p.vs.s, 0, p.Sk, tid);
+  st.gload(kp, p.ks.s, vp, p.vs.s, 0, p.Sk, tid, row_of);
   st.lstore(sm, sm + C::TILE, tid);
   __syncthreads();
 
@@ -1017,7 +1054,7 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dq_kernel(const Bw
     const int cur = it & 1;
     const int key0 = it * B32_ROWS;
     const bool more = it + 1 < nt;
-    if (more) st.gload(kp, p.ks.s, vp, p.vs.s, key0 + B32_ROWS, p.Sk, tid);
+    if (more) st.gload(kp, p.ks.s, vp, p.vs.s, key0 + B32_ROWS, p.Sk, tid, row_of);
     if (!(p.causal && key0 > qw0 + 31)) {
       const float* kb = sm + cur * 2 * C::TILE;
       const float* vb = kb + C::TILE;
@@ -1053,7 +1090,7 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dq_kernel(const Bw
   }
 
   if (qrow < p.Sq) {
-    float* dqp = p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)qrow * p.dqs.s;
+    float* dqp = p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)row_of(qrow) * p.dqs.s;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -1081,11 +1118,14 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
   if (!workgroup_tile(p, false, 128, lane, b, h, kt)) return;
   const int k0 = kt * 128;
   const int kw0 = k0 + w * 32;
-  select_sequence<float>(p, b);
+  RowMap map = {};
+  select_sequence<float>(p, b, map);
+  auto row_of = [&](int r) { return p.map.P ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
+  auto stat_of = [&](int r) { return p.map.P ? map.at(r, p.map.lse_pitch) : r; };   // in lse and delta
   if (k0 >= p.Sk || p.Sq <= 0 || (p.causal && k0 >= p.Sq)) {  // no query sees these keys: nothing to add to dk, dv
     if (p.grads_in_t && kw0 + ln < p.Sk) {                     // written gradients of such keys are zero
-      zero_grad_row<float, D>(p.dk + b * p.dks.b + h * p.dks.h + (int64_t)(kw0 + ln) * p.dks.s, hh);
-      zero_grad_row<float, D>(p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)(kw0 + ln) * p.dvs.s, hh);
+      zero_grad_row<float, D>(p.dk + b * p.dks.b + h * p.dks.h + (int64_t)row_of(kw0 + ln) * p.dks.s, hh);
+      zero_grad_row<float, D>(p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)row_of(kw0 + ln) * p.dvs.s, hh);
     }
     return;
   }
@@ -1102,8 +1142,8 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
   f32x4 kf[D / 8], vf[D / 8];
 #pragma unroll
   for (int g = 0; g < D / 8; ++g) {
-    kf[g] = *(const f32x4*)(kp + (int64_t)krow_c * p.ks.s + 8 * g + 4 * hh);
-    vf[g] = *(const f32x4*)(vp + (int64_t)krow_c * p.vs.s + 8 * g + 4 * hh);
+    kf[g] = *(const f32x4*)(kp + (int64_t)row_of(krow_c) * p.ks.s + 8 * g + 4 * hh);
+    vf[g] = *(const f32x4*)(vp + (int64_t)row_of(krow_c) * p.vs.s + 8 * g + 4 * hh);
   }
   const float c = p.scale_log2;
 
@@ -1121,12 +1161,12 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
   PairStage<D> st;
   float st_l = 0.f, st_d = 0.f;
   auto gload = [&](int it) {
-    st.gload(qp, p.qs.s, dop, p.dos.s, it * B32_ROWS, p.Sq, tid);
+    st.gload(qp, p.qs.s, dop, p.dos.s, it * B32_ROWS, p.Sq, tid, row_of);
     if (tid < B32_ROWS) {
       int r = it * B32_ROWS + tid;
       r = r < p.Sq ? r : p.Sq - 1;
-      st_l = lsep[r] * 1.4426950408889634f;
-      st_d = delp[r];
+      st_l = lsep[stat_of(r)] * 1.4426950408889634f;
+      st_d = delp[stat_of(r)];
     }
   };
   auto lstore = [&](int stage) {
@@ -1190,8 +1230,8 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
   }
 
   if (krow < p.Sk && p.grads_in_t) {
-    float* dkp = p.dk + b * p.dks.b + h * p.dks.h + (int64_t)krow * p.dks.s;
-    float* dvp = p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)krow * p.dvs.s;
+    float* dkp = p.dk + b * p.dks.b + h * p.dks.h + (int64_t)row_of(krow) * p.dks.s;
+    float* dvp = p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)row_of(krow) * p.dvs.s;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -1206,8 +1246,8 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
         *(f32x4*)(dvp + db * 32 + 8 * g + 4 * hh) = y;
       }
   } else if (krow < p.Sk) {
-    float* dkp = p.dk + b * p.dks.b + h * p.dks.h + (int64_t)krow * p.dks.s;
-    float* dvp = p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)krow * p.dvs.s;
+    float* dkp = p.dk + b * p.dks.b + h * p.dks.h + (int64_t)row_of(krow) * p.dks.s;
+    float* dvp = p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)row_of(krow) * p.dvs.s;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -1243,57 +1283,57 @@ hipError_t launch(int smem, bool queries, int rows, const BwdParams& p, hipStrea
   return hipGetLastError();
 }
 
-template <typename T, int D>
+template <typename T, int D, int ADDR = ADDR_PLAIN>
 hipError_t launch_both(const BwdParams& p, hipStream_t stream) {
   // dq kernel, D = 128: 256-row workgroups (two waves per SIMD, the K/V stream shared by twice the rows) once
   // there are enough of them to occupy every CU; spa_tune() can force 4 or 8 waves (experiments, tests).
   // At D = 64 two 128-row workgroups to a CU are as fast on long rows (+-2 %) and 4 to 7 % faster on short ones.
+  // (Tensors of 2 GiB or more per (batch, head): 128 rows.)
   const int64_t wgs8 = p.cu_q ? (int64_t)p.H * (p.lse_bh / 256 + (p.B + 1) / 2) : (int64_t)p.B * p.H * ((p.Sq + 255) / 256);
   const int forced = spa_knob(SPA_KNOB_BWD_DQ_WAVES);
   hipError_t e = hipErrorInvalidValue;
   bool wide = false;
-  if constexpr (D == 128) {
+  if constexpr (D == 128 && ADDR != ADDR_BIG) {
     wide = forced ? forced == 8 : wgs8 >= spa_device_cus();
-    if (wide) e = launch<flash_bwd_dq_kernel<T, D, 8>>(DqCfg<D, 8>::SMEM, true, 256, p, stream, 512);
+    if (wide) e = launch<flash_bwd_dq_kernel<T, D, 8, ADDR>>(DqCfg<D, 8>::SMEM, true, 256, p, stream, 512);
   }
-  if (!wide) e = launch<flash_bwd_dq_kernel<T, D, 4>>(DqCfg<D, 4>::SMEM, true, 128, p, stream);
+  if (!wide) e = launch<flash_bwd_dq_kernel<T, D, 4, ADDR>>(DqCfg<D, 4>::SMEM, true, 128, p, stream);
   if (e != hipSuccess) return e;
-  if constexpr (D == 128)
+  if constexpr (D == 128 && ADDR == ADDR_PLAIN)
     if (spa_knob(SPA_KNOB_BWD_DKDV_FORM) == 1) return launch<flash_bwd_dkdv_kernel<T, D, false>>(DkvCfg<D>::SMEM, false, 128, p, stream);
-  return launch<flash_bwd_dkdv_kernel<T, D>>(DkvCfg<D>::SMEM, false, 128, p, stream);
+  return launch<flash_bwd_dkdv_kernel<T, D, true, ADDR>>(DkvCfg<D>::SMEM, false, 128, p, stream);
 }
 
-// A tensor of 2 GiB or more per (batch, head): the re-based variants, 128-row dq workgroups.
 template <typename T, int D>
-hipError_t launch_both_big(const BwdParams& p, hipStream_t stream) {
-  const hipError_t e = launch<flash_bwd_dq_kernel<T, D, 4, true>>(DqCfg<D, 4>::SMEM, true, 128, p, stream);
-  if (e != hipSuccess) return e;
-  return launch<flash_bwd_dkdv_kernel<T, D, true, true>>(DkvCfg<D>::SMEM, false, 128, p, stream);
+hipError_t launch_other(const BwdParams& p, hipStream_t stream) {
+  if (!p.map.P) return launch_both<T, D, ADDR_BIG>(p, stream);
+  if (p.big || !p.grads_in_t) return hipErrorInvalidValue;
+  return launch_both<T, D, ADDR_MAP>(p, stream);
 }
 
 }  // namespace
 
-// This file makes two objects: compiled with SPA_BWD_BIG_UNIT it holds the re-based variants of the 16-bit kernels
-// and nothing else, without it everything else (so that the two parts compile side by side).
-#ifdef SPA_BWD_BIG_UNIT
-hipError_t spa_launch_bwd16_big(const BwdParams& p, int D, int dtype, hipStream_t stream) {
+// This file makes two objects: compiled with SPA_BWD_OTHER_UNIT it holds the re-based variants of the 16-bit kernels and
+// those for rows in shards and nothing else, without it everything else (so that the two parts compile side by side).
+#ifdef SPA_BWD_OTHER_UNIT
+hipError_t spa_launch_bwd16_other(const BwdParams& p, int D, int dtype, hipStream_t stream) {
   if (dtype == 1) {
-    if (D == 128) return launch_both_big<__bf16, 128>(p, stream);
-    if (D == 64) return launch_both_big<__bf16, 64>(p, stream);
-    if (D == 32) return launch_both_big<__bf16, 32>(p, stream);
+    if (D == 128) return launch_other<__bf16, 128>(p, stream);
+    if (D == 64) return launch_other<__bf16, 64>(p, stream);
+    if (D == 32) return launch_other<__bf16, 32>(p, stream);
   } else if (dtype == 2) {
-    if (D == 128) return launch_both_big<_Float16, 128>(p, stream);
-    if (D == 64) return launch_both_big<_Float16, 64>(p, stream);
-    if (D == 32) return launch_both_big<_Float16, 32>(p, stream);
+    if (D == 128) return launch_other<_Float16, 128>(p, stream);
+    if (D == 64) return launch_other<_Float16, 64>(p, stream);
+    if (D == 32) return launch_other<_Float16, 32>(p, stream);
   }
   return hipErrorInvalidValue;
 }
 #else
-hipError_t spa_launch_bwd16_big(const BwdParams& p, int D, int dtype, hipStream_t stream);
+hipError_t spa_launch_bwd16_other(const BwdParams& p, int D, int dtype, hipStream_t stream);
 
 // Returns hipSuccess, or hipErrorInvalidValue for an unsupported (dtype, D).
 hipError_t spa_launch_flash_bwd(BwdParams p, int D, int dtype, hipStream_t stream) {
-  if (p.big && dtype != 0) return spa_launch_bwd16_big(p, D, dtype, stream);
+  if ((p.big || p.map.P) && dtype != 0) return spa_launch_bwd16_other(p, D, dtype, stream);
   if (dtype == 1) {
     if (D == 128) return launch_both<__bf16, 128>(p, stream);
     if (D == 64) return launch_both<__bf16, 64>(p, stream);
@@ -1314,4 +1354,4 @@ hipError_t spa_launch_flash_bwd(BwdParams p, int D, int dtype, hipStream_t strea
   }
   return hipErrorInvalidValue;
 }
-#endif  // SPA_BWD_BIG_UNIT
+#endif  // SPA_BWD_OTHER_UNIT

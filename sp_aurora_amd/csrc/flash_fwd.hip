@@ -106,10 +106,15 @@ __device__ __forceinline__ int v_swizzle(int row) {
 // launcher points at a scratch tensor; a second kernel merges the z results.
 // VR: the variant for a ring over a packed variable-length batch (FwdParams::chunk_rows, rank_rows): chunks and ranks
 // lie a shard apart, not a sequence length apart.
+// MAP: the variant for rows that lie in shards (FwdParams::map), walked in the sequence's own order.  A sub-tile touches at most
+// two segments (shards, or half shards) when a segment has a sub-tile's rows: the two shifts and the row between them are
+// scalars that step with the cursor, and a lane pays a comparison and a selection per load (+2 % of a step's vector work);
+// K and V rows are equally far apart, so V uses what was found for K a step earlier.
 template <typename T, int D, int NG, bool SHARE, bool KV8 = false, bool FINALN = false, bool ZZ = false, bool BIG = false,
-          bool QK8 = false, bool WAIT = false, bool KS = false, bool VR = false>
+          bool QK8 = false, bool WAIT = false, bool KS = false, bool VR = false, bool MAP = false>
 __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) flash_fwd16_kernel(const FwdParams pk) {
   static_assert(!(FINALN && SHARE), "the merging epilogue goes with 128-row workgroups");
+  static_assert(!MAP || (!KV8 && !FINALN && !ZZ && !BIG && !WAIT && !KS && !VR), "rows in shards: 16-bit block calls");
   static_assert(!KS || (!SHARE && !FINALN && !ZZ && !BIG && !QK8 && !WAIT), "split keys: 128-row workgroups, plain results");
   static_assert(!QK8 || (KV8 && D == 128 && !ZZ && !BIG), "8-bit scores: e4m3 q, k, v, head dim 128, contiguous chunks");
   typedef typename std::conditional<KV8, unsigned char, T>::type KVT;  // element type of K / V in memory
@@ -141,7 +146,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     const int number = blockIdx.x / p.H;
     h = blockIdx.x - number * p.H;
     int nt = 0;
-    if (!sequence_tile(p.cu_q, p.B, C::BMW, number, lane, b, qt, nt)) return;
+    if (!sequence_tile(p.cu_q, p.B, MAP ? p.map.P : 1, C::BMW, number, lane, b, qt, nt)) return;
     qt = nt - 1 - qt;
   } else {
     const int pair = blockIdx.x + (p.nranks == 1 ? blockIdx.z * gridDim.x : 0u);
@@ -197,6 +202,13 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
       return;
     }
   }
+  RowMap map = {};
+  int shard_rows = 0;
+  if constexpr (MAP) {
+    shard_rows = p.cu_q ? p.Sq : p.Sq / p.map.P;
+    map.init(p.map, shard_rows);
+    p.Sq = p.Sk = shard_rows * p.map.P;
+  }
   const int q_lim = zz && !zhalf ? zz_hs : p.Sq;  // one past the last row this workgroup may own
   const int qw0 = q0 + (SHARE ? grp * FWD_BM : 0) + w * 32;
   const int64_t qoff = (int64_t)rank * (VR ? p.rank_rows : p.Sq);  // first row of this rank's query chunk
@@ -208,6 +220,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
 
   const int qrow = qw0 + ln;
   const int qrow_c = qrow < q_lim ? qrow : q_lim - 1;
+  const int qrow_t = MAP ? map.at(qrow_c, p.map.pitch) : qrow_c;  // where the row lies in q and out
 
   frag qf[QK8 ? 1 : D / 16];
   i32x8 qf8[QK8 ? D / 64 : 1];  // QK8: 32 bytes per lane and 64-deep contraction step (bytes 32 hh .. 32 hh + 31 of the step)
@@ -226,7 +239,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   } else {
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) {
-      u32x4 x = *(const u32x4*)(qp + (int64_t)qrow_c * p.qs.s + ks * 16 + hh * 8);
+      u32x4 x = *(const u32x4*)(qp + (int64_t)qrow_t * p.qs.s + ks * 16 + hh * 8);
       x[0] ^= qsign; x[1] ^= qsign; x[2] ^= qsign; x[3] ^= qsign;
       qf[ks] = as_frag<frag>(x);
     }
@@ -367,7 +380,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   const unsigned vdoff = (unsigned)((drow * p.vs.s + ((dpos ^ v_swizzle<D>(drow)) * 8)) * (int64_t)sizeof(KVT));
   const unsigned krow_b = (unsigned)(p.ks.s * (int64_t)sizeof(KVT));  // bytes per K row
   const unsigned vrow_b = (unsigned)(p.vs.s * (int64_t)sizeof(KVT));
-  const int64_t rows_all = KS ? (int64_t)(p.P - 1) * p.Sk + p.sk_last : (int64_t)(p.P - 1) * crow + p.Sk;
+  const int64_t rows_all = MAP ? (int64_t)(p.map.P - 1) * p.map.pitch + shard_rows : KS ? (int64_t)(p.P - 1) * p.Sk + p.sk_last : (int64_t)(p.P - 1) * crow + p.Sk;
   const unsigned long long kbytes = (unsigned long long)(((rows_all - 1) * p.ks.s + D) * (int64_t)sizeof(KVT));
   const unsigned long long vbytes = (unsigned long long)(((rows_all - 1) * p.vs.s + D) * (int64_t)sizeof(KVT));
   static_assert(!(BIG && KV8), "the re-based variants are built for 16-bit K / V");
@@ -392,6 +405,29 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   // Split keys, 16-bit K/V, D = 128: a chunk's tiles are read by the one workgroup of their (batch, head) when the rows fit a
   // tile, so they carry the non-temporal hint (3-9 % on five decode shapes; slower for e4m3 K/V and D = 64).
   constexpr bool KS_NT = KS && !KV8 && D == 128;
+  // MAP: what separates a thread's rows of a sub-tile in the tensors from the same rows if they followed each other, in bytes
+  unsigned at_k[MAP ? C::NDMA : 1], at_v[MAP ? C::NDMA : 1];  // of the next K and the next V sub-tile
+  int seg = 0, seg_end = map.L;  // the segment of the sub-tile's first row, and where it ends
+  auto find_rows = [&](int krel, unsigned (&at)[MAP ? C::NDMA : 1]) {
+    if constexpr (MAP) {
+      if (map.L >= BN) {
+        while (krel >= seg_end && seg_end < p.Sk) {
+          ++seg;
+          seg_end += map.L;
+        }
+        const unsigned a = (unsigned)map.shift(seg, p.map.pitch) * krow_b;
+        const unsigned z = seg_end < p.Sk ? (unsigned)map.shift(seg + 1, p.map.pitch) * krow_b : OFF_NONE;  // past the last row: zeros
+#pragma unroll
+        for (int q = 0; q < C::NDMA; ++q) at[q] = krel + q * C::RPD + drow < seg_end ? a : z;
+      } else {
+#pragma unroll
+        for (int q = 0; q < C::NDMA; ++q) {
+          const int r = krel + q * C::RPD + drow;
+          at[q] = r < p.Sk ? (unsigned)map.shift(map.segment(r), p.map.pitch) * krow_b : OFF_NONE;
+        }
+      }
+    }
+  };
   auto load_one = [&](int q, bool kon, int k_row, unsigned kb, bool von, int v_row, unsigned vb, int k_end = 0x7fffffff,
                       int v_end = 0x7fffffff) {
     if constexpr (WAIT) {
@@ -423,6 +459,14 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
           load_to_lds_b128(rs, vdoff + u, lds_wave + vb + r * (C::DTHREADS * 16));
         }
       }
+      return;
+    }
+    if constexpr (MAP) {
+      if (q < NK)
+        load_to_lds_b128(krsrc, kon ? kdoff + (unsigned)(k_row + q * RPD_K) * krow_b + at_k[q] : OFF_NONE, lds_wave + kb + q * (C::DTHREADS * 16));
+      else
+        load_to_lds_b128(vrsrc, von ? vdoff + (unsigned)(v_row + (q - NK) * C::RPD) * krow_b + at_v[q - NK] : OFF_NONE,
+                         lds_wave + vb + (q - NK) * (C::DTHREADS * 16));
       return;
     }
     if (q < NK) {
@@ -749,6 +793,11 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     if (1 < n && cv.sb.ch != cs.sb.ch) wait_chunk(cv.sb.ch);
     if (2 < n && ck.sb.ch != cv.sb.ch) wait_chunk(ck.sb.ch);
   }
+  if constexpr (MAP) {
+    find_rows(cs.sb.krel, at_k);
+#pragma unroll
+    for (int q = 0; q < C::NDMA; ++q) at_v[q] = at_k[q];
+  }
 #pragma unroll
   for (int q = 0; q < NK; ++q) load_one(q, 0 < n, cs.sb.krow, k_lds(0), false, 0, 0, cs.sb.kend, 0);     // K(0)
 #pragma unroll
@@ -760,8 +809,17 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     for (int q = 0; q < NK; ++q)
       *(__attribute__((address_space(3))) u32x4*)(lds_u8*)(uintptr_t)(lds_group + (unsigned)tg * 16 + k_lds(0) + q * (C::DTHREADS * 16)) = widen(stage[q]);
   }
+  if constexpr (MAP) find_rows(cv.sb.krel, at_k);
 #pragma unroll
   for (int q = 0; q < NK; ++q) load_one(q, 1 < n, cv.sb.krow, k_lds(1), false, 0, 0, cv.sb.kend, 0);     // K(1)
+  auto next_rows = [&]() {  // K moves on to sub-tile i + 2 of the next step, V to what K had
+    if constexpr (MAP) {
+#pragma unroll
+      for (int q = 0; q < C::NDMA; ++q) at_v[q] = at_k[q];
+      find_rows(ck.sb.krel, at_k);
+    }
+  };
+  next_rows();
   // S(0) needs Q and K(0) only: loads complete in the order of issue, so at most the loads of V(0)
   // and K(1) may still be in flight here; they are waited for before the barrier that
   // opens the first MFMA phase reading them.
@@ -831,6 +889,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     cursor_next(cs);
     cursor_next(cv);
     cursor_next(ck);
+    next_rows();
     if (early) {
       loads_landed();
       store_staged(kb, vb);  // this group's share of K(i + 2), V(i + 1), loaded at the top of the step
@@ -877,8 +936,8 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   // in the accumulator's own layout (128 rows of D + 4 floats), or null.
   auto store_rows = [&](float a_own, auto with_other, const float* other, float a_other, float lse_val) {
     constexpr bool OTHER = decltype(with_other)::value;
-    if (hh == 0 && qrow < q_lim) lse_bh[qrow] = lse_val;
-    T* const orow = out_bh + qrow_c * out_rs;
+    if (hh == 0 && qrow < q_lim) lse_bh[MAP ? map.at(qrow, p.map.lse_pitch) : qrow] = lse_val;
+    T* const orow = out_bh + qrow_t * out_rs;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -1146,7 +1205,7 @@ __global__ void __launch_bounds__(FWD_THREADS, 1) flash_fwd32_kernel(const FwdPa
     const int number = blockIdx.x / p.H;
     h = blockIdx.x - number * p.H;
     int nt = 0;
-    if (!sequence_tile(p.cu_q, p.B, FWD_BM, number, lane, b, qt, nt)) return;
+    if (!sequence_tile(p.cu_q, p.B, p.map.P ? p.map.P : 1, FWD_BM, number, lane, b, qt, nt)) return;
     qt = nt - 1 - qt;
   } else {
     const int pair = blockIdx.x + blockIdx.z * gridDim.x;
@@ -1179,6 +1238,14 @@ __global__ void __launch_bounds__(FWD_THREADS, 1) flash_fwd32_kernel(const FwdPa
     }
   }
 
+  RowMap map = {};
+  if (p.map.P) {
+    map.init(p.map, p.cu_q ? p.Sq : p.Sq / p.map.P);
+    if (p.cu_q) p.Sq = p.Sk = p.Sq * p.map.P;
+  }
+  auto row_of = [&](int r) { return p.map.P ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
+  auto stat_of = [&](int r) { return p.map.P ? map.at(r, p.map.lse_pitch) : r; };   // in lse
+
   const float* qp = (const float*)p.q + b * p.qs.b + h * p.qs.h;
   const float* kp = (const float*)p.k + b * p.ks.b + h * p.ks.h;
   const float* vp = (const float*)p.v + b * p.vs.b + h * p.vs.h;
@@ -1191,7 +1258,7 @@ __global__ void __launch_bounds__(FWD_THREADS, 1) flash_fwd32_kernel(const FwdPa
   f32x4 qf[D / 8];
 #pragma unroll
   for (int g = 0; g < D / 8; ++g) {
-    qf[g] = *(const f32x4*)(qp + (int64_t)qrow_c * p.qs.s + 8 * g + 4 * hh);
+    qf[g] = *(const f32x4*)(qp + (int64_t)row_of(qrow_c) * p.qs.s + 8 * g + 4 * hh);
     if (p.negq) qf[g] = -qf[g];  // negative softmax scale: -q with |scale|
   }
 
@@ -1209,7 +1276,7 @@ __global__ void __launch_bounds__(FWD_THREADS, 1) flash_fwd32_kernel(const FwdPa
       const int lr = cr + i * C::RPP;
       if (lr < F32_BN) {
         int r = key0 + lr;
-        r = r < p.Sk ? r : p.Sk - 1;
+        r = row_of(r < p.Sk ? r : p.Sk - 1);
         kreg[i] = *(const f32x4*)(kp + (int64_t)r * p.ks.s + cc * 4);
         vreg[i] = *(const f32x4*)(vp + (int64_t)r * p.vs.s + cc * 4);
       }
@@ -1317,7 +1384,7 @@ __global__ void __launch_bounds__(FWD_THREADS, 1) flash_fwd32_kernel(const FwdPa
   const float l_tot = halves_sum(l_run);
   const float inv = 1.f / l_tot;
   if (qrow < p.Sq) {
-    float* op = (float*)p.out + b * p.os.b + h * p.os.h + (int64_t)qrow * p.os.s;
+    float* op = (float*)p.out + b * p.os.b + h * p.os.h + (int64_t)row_of(qrow) * p.os.s;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -1330,7 +1397,7 @@ __global__ void __launch_bounds__(FWD_THREADS, 1) flash_fwd32_kernel(const FwdPa
         *(f32x4*)(op + db * 32 + 8 * g + 4 * hh) = st;
       }
     if (hh == 0)
-      p.lse[((int64_t)b * p.H + h) * p.lse_bh + qrow] = (m_run * c + fast_log2(l_tot)) * 0.6931471805599453f;
+      p.lse[((int64_t)b * p.H + h) * p.lse_bh + stat_of(qrow)] = (m_run * c + fast_log2(l_tot)) * 0.6931471805599453f;
   }
 }
 
@@ -1369,6 +1436,10 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
   const int b = bh / p.H;
   const int qt = p.nqt - 1 - (int)blockIdx.y;
   const int q0 = qt * 32;
+  RowMap map = {};
+  if (p.map.P) map.init(p.map, p.Sq / p.map.P);
+  auto row_of = [&](int r) { return p.map.P ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
+  auto stat_of = [&](int r) { return p.map.P ? map.at(r, p.map.lse_pitch) : r; };   // in lse
   const float* qp = (const float*)p.q + b * p.qs.b + h * p.qs.h;
   const float* kp = (const float*)p.k + b * p.ks.b + h * p.ks.h;
   const float* vp = (const float*)p.v + b * p.vs.b + h * p.vs.h;
@@ -1377,7 +1448,7 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
   f32x4 qf[D / 8];
 #pragma unroll
   for (int g = 0; g < D / 8; ++g) {
-    qf[g] = *(const f32x4*)(qp + (int64_t)qrow_c * p.qs.s + 8 * g + 4 * hh);
+    qf[g] = *(const f32x4*)(qp + (int64_t)row_of(qrow_c) * p.qs.s + 8 * g + 4 * hh);
     if (p.negq) qf[g] = -qf[g];
   }
   const int kv_end = p.causal ? (q0 + 32 < p.Sk ? q0 + 32 : p.Sk) : p.Sk;
@@ -1391,7 +1462,7 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
 #pragma unroll
     for (int i = 0; i < C::PASS; ++i) {
       int r = key0 + cr + i * C::RPP;
-      r = r < p.Sk ? r : p.Sk - 1;
+      r = row_of(r < p.Sk ? r : p.Sk - 1);
       kreg[i] = *(const f32x4*)(kp + (int64_t)r * p.ks.s + cc * 4);
       vreg[i] = *(const f32x4*)(vp + (int64_t)r * p.vs.s + cc * 4);
     }
@@ -1501,7 +1572,7 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
   }
   const float inv = 1.f / l_all;
   if (qrow < p.Sq) {
-    float* const op = (float*)p.out + b * p.os.b + h * p.os.h + (int64_t)qrow * p.os.s;
+    float* const op = (float*)p.out + b * p.os.b + h * p.os.h + (int64_t)row_of(qrow) * p.os.s;
     for (int pc = w; pc < NPC; pc += NW) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1513,7 +1584,7 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
       const int db = pc / 4, g = pc % 4;
       *(f32x4*)(op + db * 32 + 8 * g + 4 * hh) = acc;
     }
-    if (w == 0 && hh == 0) p.lse[((int64_t)b * p.H + h) * p.lse_bh + qrow] = (m_all * c + fast_log2(l_all)) * 0.6931471805599453f;
+    if (w == 0 && hh == 0) p.lse[((int64_t)b * p.H + h) * p.lse_bh + stat_of(qrow)] = (m_all * c + fast_log2(l_all)) * 0.6931471805599453f;
   }
 }
 
@@ -1630,6 +1701,21 @@ hipError_t launch16(FwdParams p, hipStream_t stream) {
   return launch<flash_fwd16_kernel<T, D, 1, false, KV8, false, ZZ, false, QK8>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM_PLAIN, FWD_BM, p, stream);
 }
 
+// Rows in shards: the same three forms.
+template <typename T, int D>
+hipError_t launch16_map(FwdParams p, hipStream_t stream) {
+  const FwdForm form = fwd_form(p, D, KIND_16);
+  constexpr bool N = false;
+  if constexpr (D >= 64)
+    if (form == FWD_SHARE) {
+      p.nqt = fwd_tiles(p, 2 * FWD_BM);
+      return launch<flash_fwd16_kernel<T, D, 2, true, N, N, N, N, N, N, N, N, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, true>::SMEM, 2 * FWD_BM, p, stream);
+    }
+  if (form == FWD_SPLIT)
+    return launch<flash_fwd16_kernel<T, D, 2, false, N, N, N, N, N, N, N, N, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
+  return launch<flash_fwd16_kernel<T, D, 1, false, N, N, N, N, N, N, N, N, true>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM_PLAIN, FWD_BM, p, stream);
+}
+
 // K / V spanning 2 GiB or more per (batch, head): the re-based variants, 128-row workgroups with two wave groups
 // (such a tensor has more than enough rows for them).
 template <typename T, int D>
@@ -1678,9 +1764,9 @@ hipError_t launch16_any(const FwdParams& p, int D, int dtype, hipStream_t stream
 
 }  // namespace
 
-// This file makes four objects: compiled with SPA_FWD_ZIGZAG_UNIT it holds the zigzag variants of the 16-bit
+// This file makes five objects: compiled with SPA_FWD_ZIGZAG_UNIT it holds the zigzag variants of the 16-bit
 // kernel and nothing else, with SPA_FWD_SPLITKV_UNIT those that split the keys over the grid and those for a ring over a
-// packed variable-length batch, with SPA_FWD_BIG_UNIT the
+// packed variable-length batch, with SPA_FWD_MAP_UNIT those for rows in shards, with SPA_FWD_BIG_UNIT the
 // re-based variants, those with 8-bit scores and those that wait for chunk arrival flags, without any of them
 // everything else (so that the parts compile side by side).
 #if defined(SPA_FWD_SPLITKV_UNIT)
@@ -1716,6 +1802,22 @@ hipError_t spa_launch_fwd16_varlen_ring(FwdParams p, int D, int dtype, hipStream
   if (dtype == 1) { if (D == 128) return SPA_VR(__bf16, 128); if (D == 64) return SPA_VR(__bf16, 64); if (D == 32) return SPA_VR(__bf16, 32); }
   if (dtype == 2) { if (D == 128) return SPA_VR(_Float16, 128); if (D == 64) return SPA_VR(_Float16, 64); if (D == 32) return SPA_VR(_Float16, 32); }
 #undef SPA_VR
+  return hipErrorInvalidValue;
+}
+#elif defined(SPA_FWD_MAP_UNIT)
+hipError_t spa_launch_fwd16_map(const FwdParams& p, int D, int dtype, hipStream_t stream) {
+  if (p.map.P < 1 || p.P != 1 || p.nranks != 1 || p.zigzag || p.big || p.arrive || p.k_scale || p.q_scale || p.chunk_rows || p.epi != SPA_EPI_PLAIN ||
+      p.ks.s != p.vs.s)
+    return hipErrorInvalidValue;
+  if (dtype == 1) {
+    if (D == 128) return launch16_map<__bf16, 128>(p, stream);
+    if (D == 64) return launch16_map<__bf16, 64>(p, stream);
+    if (D == 32) return launch16_map<__bf16, 32>(p, stream);
+  } else if (dtype == 2) {
+    if (D == 128) return launch16_map<_Float16, 128>(p, stream);
+    if (D == 64) return launch16_map<_Float16, 64>(p, stream);
+    if (D == 32) return launch16_map<_Float16, 32>(p, stream);
+  }
   return hipErrorInvalidValue;
 }
 #elif defined(SPA_FWD_ZIGZAG_UNIT)
@@ -1765,6 +1867,7 @@ hipError_t spa_launch_fwd16_big(const FwdParams& p, int D, int dtype, hipStream_
 hipError_t spa_launch_fwd16_qk8(const FwdParams& p, int D, int dtype, hipStream_t stream);
 hipError_t spa_launch_fwd16_wait(const FwdParams& p, int D, int dtype, hipStream_t stream);
 hipError_t spa_launch_fwd16_varlen_ring(FwdParams p, int D, int dtype, hipStream_t stream);
+hipError_t spa_launch_fwd16_map(const FwdParams& p, int D, int dtype, hipStream_t stream);
 
 // Returns hipSuccess, or hipErrorInvalidValue for an unsupported (dtype, D).
 hipError_t spa_launch_flash_fwd(FwdParams p, int D, int dtype, hipStream_t stream) {
@@ -1782,6 +1885,7 @@ hipError_t spa_launch_flash_fwd(FwdParams p, int D, int dtype, hipStream_t strea
     p.out = (char*)slots.out<char>(p.part, p.part_slot) - row0 * p.os.s * 2;
     p.lse = slots.lse(p.part, p.P, p.part_slot) - row0;
   }
+  if ((dtype == 1 || dtype == 2) && p.map.P) return spa_launch_fwd16_map(p, D, dtype, stream);
   if ((dtype == 1 || dtype == 2) && p.chunk_rows) return spa_launch_fwd16_varlen_ring(p, D, dtype, stream);
   if ((dtype == 1 || dtype == 2) && p.arrive) return spa_launch_fwd16_wait(p, D, dtype, stream);
   if ((dtype == 1 || dtype == 2) && p.q_scale) return spa_launch_fwd16_qk8(p, D, dtype, stream);
@@ -1806,4 +1910,4 @@ hipError_t spa_launch_flash_fwd(FwdParams p, int D, int dtype, hipStream_t strea
   }
   return hipErrorInvalidValue;
 }
-#endif  // SPA_FWD_SPLITKV_UNIT / SPA_FWD_ZIGZAG_UNIT / SPA_FWD_BIG_UNIT
+#endif  // SPA_FWD_SPLITKV_UNIT / SPA_FWD_MAP_UNIT / SPA_FWD_ZIGZAG_UNIT / SPA_FWD_BIG_UNIT

@@ -709,13 +709,25 @@ int spa_bwd_delta(const void* out, const void* dout, float* delta, int B, int H,
 }
 
 namespace {
+// Rows in shards: checks, and what the kernels get.  `rows` = rows of one sequence in all shards, `per_shard` = the shard's
+// rows that hold them (the pitch may not be less).
+int shard_map(const char* what, const spa_shards* m, int64_t rows, int64_t per_shard, ShardMap& map) {
+  if (m->shards < 1 || m->pitch < 1 || m->lse_pitch < 1) return fail(SPA_EINVAL, "%s: shards and pitches must be positive", what);
+  const int parts = m->zigzag ? 2 * m->shards : m->shards;
+  if (rows % parts != 0) return fail(SPA_EINVAL, "%s: %d parts must divide %lld rows", what, parts, (long long)rows);
+  if (m->shards > 1 && (m->pitch < per_shard || m->lse_pitch < per_shard)) return fail(SPA_EINVAL, "%s: a pitch below a shard's rows", what);
+  if ((int64_t)(m->shards - 1) * m->pitch + per_shard > 0x7fffffffLL) return fail(SPA_EINVAL, "%s: too many rows", what);
+  map.P = m->shards; map.pitch = m->pitch; map.lse_pitch = m->lse_pitch; map.zigzag = m->zigzag != 0;
+  return SPA_OK;
+}
+
 // grads_in_t: dq / dk / dv are tensors of the inputs' element type and are written (spa_flash_bwd_out);
 // else fp32 accumulators that are added to (spa_flash_bwd).  out (with o_strides): delta is scratch and is computed here.
 int flash_bwd(const char* what, const void* q, const void* k, const void* v, const void* out, const int64_t* o_strides, const void* dout,
               const float* lse, float* delta, void* dq, void* dk, void* dv, bool grads_in_t, int B, int H, int Sq, int Sk,
               int D, const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
               const int64_t do_strides[3], const int64_t dq_strides[3], const int64_t dk_strides[3],
-              const int64_t dv_strides[3], float scale, int mask_mode, int dtype, void* stream) {
+              const int64_t dv_strides[3], float scale, int mask_mode, int dtype, void* stream, const spa_shards* rows = nullptr) {
   if (!q || !k || !v || !dout || !lse || !delta || !dq || !dk || !dv) return fail(SPA_EINVAL, "%s: null pointer", what);
   if (!q_strides || !k_strides || !v_strides || !do_strides || !dq_strides || !dk_strides || !dv_strides)
     return fail(SPA_EINVAL, "%s: null strides", what);
@@ -729,8 +741,17 @@ int flash_bwd(const char* what, const void* q, const void* k, const void* v, con
       !aligned16(dout, do_strides, esz) || !aligned16(dq, dq_strides, gsz) || !aligned16(dk, dk_strides, gsz) ||
       !aligned16(dv, dv_strides, gsz) || (out && !aligned16(out, o_strides, esz)))
     return fail(SPA_EALIGN, "%s: pointers and row strides must be 16-byte aligned", what);
-  const bool big = (out && !span_ok(Sq, o_strides[2], D, esz)) || !span_ok(Sq, q_strides[2], D, esz) || !span_ok(Sk, k_strides[2], D, esz) || !span_ok(Sk, v_strides[2], D, esz) ||
-                   !span_ok(Sq, do_strides[2], D, esz);
+  ShardMap map;
+  if (rows) {
+    if (Sq != Sk) return fail(SPA_EINVAL, "%s: rows in shards need as many keys as queries", what);
+    const int rc = shard_map(what, rows, Sq, rows->shards > 0 ? Sq / rows->shards : 0, map);
+    if (rc != SPA_OK) return rc;
+  }
+  const int64_t span = rows ? (int64_t)(map.P - 1) * map.pitch + Sq / map.P : 0;
+  const int64_t span_q = rows ? span : Sq, span_k = rows ? span : Sk;  // rows of the tensors from a sequence's first to its last
+  const bool big = (out && !span_ok(span_q, o_strides[2], D, esz)) || !span_ok(span_q, q_strides[2], D, esz) ||
+                   !span_ok(span_k, k_strides[2], D, esz) || !span_ok(span_k, v_strides[2], D, esz) || !span_ok(span_q, do_strides[2], D, esz);
+  if (big && rows && dtype != SPA_F32) return fail(SPA_EUNSUPPORTED, "%s: rows in shards that span 2 GiB or more", what);
   if (big && dtype != SPA_F32 && !(span_rebasable(q_strides[2], esz) && span_rebasable(k_strides[2], esz) &&
                                    span_rebasable(v_strides[2], esz) && span_rebasable(do_strides[2], esz) &&
                                    (!out || span_rebasable(o_strides[2], esz))))
@@ -742,6 +763,7 @@ int flash_bwd(const char* what, const void* q, const void* k, const void* v, con
   p.dq = (float*)dq; p.dk = (float*)dk; p.dv = (float*)dv;
   p.out = out;
   if (out) p.os = S3(o_strides);
+  p.map = map;
   p.grads_in_t = grads_in_t;
   p.big = big && dtype != SPA_F32;
   p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk;
@@ -777,11 +799,11 @@ int spa_flash_bwd_out(const void* q, const void* k, const void* v, const void* d
 int spa_attention_bwd(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse, float* delta,
                       void* dq, void* dk, void* dv, int B, int H, int Sq, int Sk, int D, const int64_t q_strides[3],
                       const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3], const int64_t do_strides[3],
-                      const int64_t dq_strides[3], const int64_t dk_strides[3], const int64_t dv_strides[3], float scale,
-                      int mask_mode, int dtype, void* stream) {
+                      const int64_t dq_strides[3], const int64_t dk_strides[3], const int64_t dv_strides[3], const spa_shards* rows,
+                      float scale, int mask_mode, int dtype, void* stream) {
   if (!out || !o_strides) return fail(SPA_EINVAL, "spa_attention_bwd: null pointer");
   return flash_bwd("spa_attention_bwd", q, k, v, out, o_strides, dout, lse, delta, dq, dk, dv, true, B, H, Sq, Sk, D, q_strides, k_strides,
-                   v_strides, do_strides, dq_strides, dk_strides, dv_strides, scale, mask_mode, dtype, stream);
+                   v_strides, do_strides, dq_strides, dk_strides, dv_strides, scale, mask_mode, dtype, stream, rows);
 }
 
 namespace {
@@ -891,13 +913,64 @@ int flash_fwd_varlen(const char* what, const void* q, const void* k, const void*
   return launch_result(spa_launch_flash_fwd(p, D, dtype, (hipStream_t)stream), what);
 }
 
+// The forward over rows in shards.  Fixed lengths (cu null): n = batch entries of S rows; packed: n = sequences of at most S rows
+// in one of the shards of `total` rows.
+int attention_fwd(const char* what, const void* q, const void* k, const void* v, void* out, float* lse, const int32_t* cu, int n, int H, int total,
+                  int S, int D, const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os, const spa_shards* rows, float scale,
+                  int mask_mode, int dtype, void* stream) {
+  if (!q || !k || !v || !out || !lse || !qs || !ks || !vs || !os || !rows) return fail(SPA_EINVAL, "%s: null pointer", what);
+  const int r = cu ? 1 : 2;  // position of the row stride
+  const int esz = elem_size(dtype);
+  if (cu) {
+    const int rc = varlen_sizes_ok(what, cu, cu, n, H, total, total, S, S, D, dtype, mask_mode, scale);
+    if (rc != SPA_OK) return rc;
+  } else {
+    if (!dims_ok(n, H, S, D)) return fail(SPA_EINVAL, "%s: sizes must be positive", what);
+    if (!dtype_ok(dtype)) return fail(SPA_EINVAL, "%s: bad dtype %d", what, dtype);
+    if (mask_mode != SPA_MASK_NONE && mask_mode != SPA_MASK_CAUSAL) return fail(SPA_EINVAL, "%s: bad mask_mode %d", what, mask_mode);
+    if (!scale_ok(scale)) return fail(SPA_EINVAL, "%s: softmax scale must be finite", what);
+    if (D != 32 && D != 64 && D != 128) return fail(SPA_EUNSUPPORTED, "%s: head dim %d not in {32,64,128}", what, D);
+    if ((int64_t)n * H > 0x7fffffffLL || (S + 127) / 128 > 65535) return fail(SPA_EINVAL, "%s: grid too large", what);
+  }
+  ShardMap map;
+  const int rc = cu ? shard_map(what, rows, (int64_t)2 * (rows->shards > 0 ? rows->shards : 1), total, map)
+                    : shard_map(what, rows, S, rows->shards > 0 ? S / rows->shards : 0, map);
+  if (rc != SPA_OK) return rc;
+  const auto aligned = [&](const void* p, const int64_t* s) { return cu ? aligned16v(p, s, esz) : aligned16(p, s, esz); };
+  if (!aligned(q, qs) || !aligned(k, ks) || !aligned(v, vs) || !aligned(out, os) || ((uintptr_t)lse & 3) != 0)
+    return fail(SPA_EALIGN, "%s: pointers and row strides must be 16-byte aligned", what);
+  const int64_t span = (int64_t)(map.P - 1) * map.pitch + (cu ? S : S / map.P);
+  if (dtype != SPA_F32 && (ks[r] != vs[r] || !span_ok(span, ks[r], D, esz)))
+    return fail(SPA_EUNSUPPORTED, "%s: k and v need one row stride and less than 2 GiB per (batch, head)", what);
+  if ((int64_t)map.P * (cu ? total : 1) > 0x7fffffffLL || (int64_t)map.P * S > 0x7fffffffLL) return fail(SPA_EINVAL, "%s: too many rows", what);
+  FwdParams p;
+  p.q = q; p.k = k; p.v = v; p.out = out; p.lse = lse;
+  p.B = n; p.H = H;
+  p.Sq = p.Sk = cu ? map.P * S : S;  // (packed: the longest sequence's rows in all shards)
+  p.qs = cu ? S2(qs) : S3(qs); p.ks = cu ? S2(ks) : S3(ks); p.vs = cu ? S2(vs) : S3(vs); p.os = cu ? S2(os) : S3(os);
+  p.scale = scale_eff(scale);
+  p.scale_log2 = fabsf(scale_eff(scale)) * 1.4426950408889634f;
+  p.negq = scale < 0.f;
+  p.causal = mask_mode == SPA_MASK_CAUSAL;
+  p.nqt = 0;
+  p.lse_bh = cu ? (int64_t)map.P * total : S;
+  p.part = nullptr; p.part_slot = 0; p.npart = 0;
+  p.epi = SPA_EPI_PLAIN;
+  p.P = 1; p.rank0 = 0; p.nranks = 1; p.t_begin = 0; p.t_count = -1;
+  p.cu_q = cu; p.cu_k = cu;
+  p.k_scale = nullptr; p.v_scale = nullptr;
+  p.map = map;
+  return launch_result(spa_launch_flash_fwd(p, D, dtype, (hipStream_t)stream), what);
+}
+
 // grads_in_t: as in flash_bwd above.
 int flash_bwd_varlen(const char* what, const void* q, const void* k, const void* v, const void* out, const int64_t* o_strides,
                      const void* dout, const float* lse, float* delta, void* dq, void* dk, void* dv, bool grads_in_t, const int32_t* cu_seqlens_q,
                      const int32_t* cu_seqlens_k, int nseq, int H, int total_q, int total_k, int max_sq, int max_sk,
                      int D, const int64_t q_strides[2], const int64_t k_strides[2], const int64_t v_strides[2],
                      const int64_t do_strides[2], const int64_t dq_strides[2], const int64_t dk_strides[2],
-                     const int64_t dv_strides[2], float scale, int mask_mode, int dtype, void* stream) {
+                     const int64_t dv_strides[2], float scale, int mask_mode, int dtype, void* stream,
+                     const spa_shards* rows = nullptr) {
   if (!q || !k || !v || !dout || !lse || !delta || !dq || !dk || !dv) return fail(SPA_EINVAL, "%s: null pointer", what);
   if (!q_strides || !k_strides || !v_strides || !do_strides || !dq_strides || !dk_strides || !dv_strides)
     return fail(SPA_EINVAL, "%s: null strides", what);
@@ -909,8 +982,17 @@ int flash_bwd_varlen(const char* what, const void* q, const void* k, const void*
       !aligned16v(dout, do_strides, esz) || !aligned16v(dq, dq_strides, gsz) || !aligned16v(dk, dk_strides, gsz) ||
       !aligned16v(dv, dv_strides, gsz) || (out && !aligned16v(out, o_strides, esz)) || (((uintptr_t)lse | (uintptr_t)delta) & 3) != 0)
     return fail(SPA_EALIGN, "%s: pointers and row strides must be 16-byte aligned", what);
-  const bool big = (out && !span_ok(max_sq, o_strides[1], D, esz)) || !span_ok(max_sq, q_strides[1], D, esz) || !span_ok(max_sk, k_strides[1], D, esz) ||
-                   !span_ok(max_sk, v_strides[1], D, esz) || !span_ok(max_sq, do_strides[1], D, esz);
+  ShardMap map;
+  if (rows) {
+    if (cu_seqlens_q != cu_seqlens_k || total_q != total_k || max_sq != max_sk)
+      return fail(SPA_EINVAL, "%s: rows in shards have one cu_seqlens for queries and keys", what);
+    const int rc2 = shard_map(what, rows, (int64_t)2 * (rows->shards > 0 ? rows->shards : 1), total_q, map);
+    if (rc2 != SPA_OK) return rc2;
+  }
+  const int64_t more = rows ? (int64_t)(map.P - 1) * map.pitch : 0, span_q = more + max_sq, span_k = more + max_sk;
+  const bool big = (out && !span_ok(span_q, o_strides[1], D, esz)) || !span_ok(span_q, q_strides[1], D, esz) || !span_ok(span_k, k_strides[1], D, esz) ||
+                   !span_ok(span_k, v_strides[1], D, esz) || !span_ok(span_q, do_strides[1], D, esz);
+  if (big && rows && dtype != SPA_F32) return fail(SPA_EUNSUPPORTED, "%s: rows in shards that span 2 GiB or more", what);
   if (big && dtype != SPA_F32 && !(span_rebasable(q_strides[1], esz) && span_rebasable(k_strides[1], esz) &&
                                    span_rebasable(v_strides[1], esz) && span_rebasable(do_strides[1], esz) &&
                                    (!out || span_rebasable(o_strides[1], esz))))
@@ -921,6 +1003,7 @@ int flash_bwd_varlen(const char* what, const void* q, const void* k, const void*
   p.dq = (float*)dq; p.dk = (float*)dk; p.dv = (float*)dv;
   p.out = out;
   if (out) p.os = S2(o_strides);
+  p.map = map;
   p.grads_in_t = grads_in_t;
   p.B = nseq; p.H = H; p.Sq = max_sq; p.Sk = max_sk;
   p.qs = S2(q_strides); p.ks = S2(k_strides); p.vs = S2(v_strides); p.dos = S2(do_strides);
@@ -928,9 +1011,11 @@ int flash_bwd_varlen(const char* what, const void* q, const void* k, const void*
   p.scale = scale_eff(scale);
   p.scale_log2 = scale_eff(scale) * 1.4426950408889634f;
   p.causal = mask_mode == SPA_MASK_CAUSAL;
-  p.lse_bh = total_q;
+  const int64_t copies = rows ? map.P : 1;
+  if (copies * total_q > 0x7fffffffLL) return fail(SPA_EINVAL, "%s: too many rows", what);
+  p.lse_bh = copies * total_q;
   p.cu_q = cu_seqlens_q; p.cu_k = cu_seqlens_k;
-  p.total_k = total_k;
+  p.total_k = (int)(copies * total_k);
   return launch_result(spa_launch_flash_bwd(p, D, dtype, (hipStream_t)stream), what);
 }
 }  // namespace
@@ -997,11 +1082,27 @@ int spa_attention_bwd_varlen(const void* q, const void* k, const void* v, const 
                              int total_q, int total_k, int max_sq, int max_sk, int D, const int64_t q_strides[2],
                              const int64_t k_strides[2], const int64_t v_strides[2], const int64_t o_strides[2],
                              const int64_t do_strides[2], const int64_t dq_strides[2], const int64_t dk_strides[2],
-                             const int64_t dv_strides[2], float scale, int mask_mode, int dtype, void* stream) {
+                             const int64_t dv_strides[2], const spa_shards* rows, float scale, int mask_mode, int dtype, void* stream) {
   if (!out || !o_strides) return fail(SPA_EINVAL, "spa_attention_bwd_varlen: null pointer");
   return flash_bwd_varlen("spa_attention_bwd_varlen", q, k, v, out, o_strides, dout, lse, delta, dq, dk, dv, true, cu_seqlens_q, cu_seqlens_k,
                           nseq, H, total_q, total_k, max_sq, max_sk, D, q_strides, k_strides, v_strides, do_strides, dq_strides,
-                          dk_strides, dv_strides, scale, mask_mode, dtype, stream);
+                          dk_strides, dv_strides, scale, mask_mode, dtype, stream, rows);
+}
+
+int spa_attention_fwd(const void* q, const void* k, const void* v, void* out, float* lse, int B, int H, int S, int D,
+                      const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3],
+                      const spa_shards* rows, float scale, int mask_mode, int dtype, void* stream) {
+  return attention_fwd("spa_attention_fwd", q, k, v, out, lse, nullptr, B, H, 0, S, D, q_strides, k_strides, v_strides, o_strides, rows, scale,
+                       mask_mode, dtype, stream);
+}
+
+int spa_attention_fwd_varlen(const void* q, const void* k, const void* v, void* out, float* lse, const int32_t* cu_seqlens, int nseq, int H,
+                             int total_rows, int max_seqlen, int D, const int64_t q_strides[2], const int64_t k_strides[2],
+                             const int64_t v_strides[2], const int64_t o_strides[2], const spa_shards* rows, float scale, int mask_mode,
+                             int dtype, void* stream) {
+  if (!cu_seqlens) return fail(SPA_EINVAL, "spa_attention_fwd_varlen: null pointer");
+  return attention_fwd("spa_attention_fwd_varlen", q, k, v, out, lse, cu_seqlens, nseq, H, total_rows, max_seqlen, D, q_strides, k_strides,
+                       v_strides, o_strides, rows, scale, mask_mode, dtype, stream);
 }
 
 }  // extern "C"

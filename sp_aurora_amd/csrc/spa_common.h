@@ -15,6 +15,13 @@ struct Strides3 {
   int64_t b, h, s;  // element strides of (batch, head, seq); head-dim stride is 1
 };
 
+// Rows of a sequence that lie in shards: the sequence is cut into P shards of equal length that are `pitch` rows apart in the
+// tensor (`lse_pitch` entries in lse and delta), each holding the next part of the sequence or, zigzag, parts r and 2P-1-r of
+// 2P.  The kernels walk the sequence in its own order and look up where a row lies.  P = 0: rows follow each other.
+struct ShardMap {
+  int P = 0, pitch = 0, lse_pitch = 0, zigzag = 0;
+};
+
 struct FwdParams {
   const void* q;
   const void* k;
@@ -79,6 +86,8 @@ struct FwdParams {
   // r's queries rank_rows rows after rank r - 1's (0: chunks and ranks follow each other, Sk and Sq rows apart).
   int chunk_rows = 0;
   int rank_rows = 0;
+  // Rows in shards (the MAP variants): Sq = Sk = rows of the whole sequence, or, with cu_q, cu_q describes one shard
+  ShardMap map;
 };
 
 // Layout of the ring-step slots of one rank in the caller's workspace (16-bit inputs, ring of P):
@@ -131,6 +140,7 @@ struct BwdParams {
   int grads_in_t;
   // some tensor's rows of one (batch, head) span 2 GiB or more (see FwdParams::big)
   int big = 0;
+  ShardMap map;  // rows in shards, as in FwdParams
 };
 
 // 16-bit element traits: MFMA 32x32x16 with 8 elements per lane per operand.
@@ -217,6 +227,32 @@ static __device__ __forceinline__ float halves_sum(float x) {
   return lo + hi;
 }
 
+// ---- rows in shards ----
+// Where row r of a sequence lies (ShardMap), as r + a shift that is the same for all rows of a segment (a shard, or half a
+// zigzag shard).
+struct RowMap {
+  int L, P, zigzag;  // rows per segment, shards
+  float per_L;
+  __device__ __forceinline__ void init(const ShardMap& m, int shard_rows) {
+    P = m.P;
+    zigzag = m.zigzag;
+    L = zigzag ? shard_rows >> 1 : shard_rows;
+    per_L = 1.f / (float)L;
+  }
+  __device__ __forceinline__ int shift(int segment, int pitch) const {
+    const bool second = zigzag && segment >= P;
+    return (second ? 2 * P - 1 - segment : segment) * pitch + (second ? L : 0) - segment * L;
+  }
+  // r / L: there are few segments, so the product with 1 / L is off by less than one
+  __device__ __forceinline__ int segment(int r) const {
+    int q = (int)((float)r * per_L);
+    const int rest = r - q * L;
+    q += rest >= L ? 1 : 0;
+    return rest < 0 ? q - 1 : q;
+  }
+  __device__ __forceinline__ int at(int r, int pitch) const { return r + shift(segment(r), pitch); }
+};
+
 // ---- variable-length batches ----
 // Which tile of which sequence a workgroup takes.  The tiles (of `rows` rows) of all sequences are numbered back to back,
 // sequence by sequence, so a grid of (total rows / rows + sequences) numbers covers any batch and at most one workgroup
@@ -224,11 +260,13 @@ static __device__ __forceinline__ float halves_sum(float x) {
 // do not exist, and each takes a CU from one with work).  Blocks of 64 sequences in the order given, longest first inside a
 // block: the heavy tiles start first, and the tiles of one sequence run side by side and share its K / V in L2.
 // Every wave of the workgroup calls this (a lane holds one sequence of the block); false: no such tile.
-static __device__ __forceinline__ bool sequence_tile(const int* cu, int nseq, int rows, int number, int lane, int& seq, int& tile, int& ntiles) {
+// times: the sequences are that many times as long as cu says (shards).
+static __device__ __forceinline__ bool sequence_tile(const int* cu, int nseq, int times, int rows, int number, int lane, int& seq, int& tile,
+                                                     int& ntiles) {
   for (int base = 0; base < nseq; base += 64) {
     const int n = nseq - base < 64 ? nseq - base : 64;
     const int i = base + (lane < n ? lane : 0);
-    const int len = lane < n ? cu[i + 1] - cu[i] : 0;
+    const int len = lane < n ? (cu[i + 1] - cu[i]) * times : 0;
     const int mine = (len + rows - 1) / rows;
     int before = 0, total = 0;  // tiles of the sequences that come before this lane's, tiles of the block
     for (int j = 0; j < n; ++j) {

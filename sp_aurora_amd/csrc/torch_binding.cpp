@@ -44,16 +44,17 @@ bool rows_ok(const Tensor& t, int64_t bytes = 16) {
   return true;
 }
 
-// One operand as the C ABI takes it: pointer, (batch, head, seq) strides in elements, sizes.
+// One operand as the C ABI takes it: pointer, (batch, head, seq) strides in elements, sizes.  pitch: rows from one shard to the
+// next where a sequence's rows lie in shards, 0 where they follow each other.
 struct View {
   void* p = nullptr;
   int64_t st[3] = {0, 0, 0};
-  int B = 0, H = 0, S = 0, D = 0;
+  int B = 0, H = 0, S = 0, D = 0, pitch = 0;
   bool same_shape(const View& o) const { return B == o.B && H == o.H && S == o.S && D == o.D; }
 };
 
-// [B,S,H,D] (bshd) or [B,H,S,D]; `part` of a packed [B,S,n,H,D] tensor when part >= 0; a rank-stacked [P,1,s,H,D] tensor
-// whose ranks' rows follow each other as the one sequence [1,P*s,H,D].
+// [B,S,H,D] (bshd) or [B,H,S,D]; `part` of a packed [B,S,n,H,D] tensor when part >= 0; a rank-stacked [P,B,s,H,D] tensor as the
+// sequences [B,P*s,H,D] in shards.
 bool view_of(const Tensor& t, bool bshd, View& v, int part = -1) {
   const auto sz = t.sizes();
   const auto st = t.strides();
@@ -68,9 +69,13 @@ bool view_of(const Tensor& t, bool bshd, View& v, int part = -1) {
     return true;
   }
   if (t.dim() == 5) {
-    if (!bshd || sz[1] != 1 || (sz[0] > 1 && st[0] != sz[2] * st[2]) || sz[0] * sz[2] > 0x7fffffffLL) return false;
-    v.B = 1; v.S = (int)(sz[0] * sz[2]); v.H = (int)sz[3]; v.D = (int)sz[4];
-    v.st[0] = v.S * st[2]; v.st[1] = st[3]; v.st[2] = st[2];
+    if (!bshd || sz[0] * sz[2] > 0x7fffffffLL || st[2] <= 0) return false;
+    v.B = (int)sz[1]; v.S = (int)(sz[0] * sz[2]); v.H = (int)sz[3]; v.D = (int)sz[4];
+    v.st[0] = st[1]; v.st[1] = st[3]; v.st[2] = st[2];
+    if (sz[0] > 1 && st[0] != sz[2] * st[2]) {
+      if (st[0] % st[2] != 0 || st[0] / st[2] < sz[2] || st[0] / st[2] > 0x7fffffffLL) return false;
+      v.pitch = (int)(st[0] / st[2]);
+    }
     return true;
   }
   if (t.dim() != 4) return false;
@@ -158,7 +163,8 @@ bool cu_ok(const Tensor& cu, const Tensor& q) {
 }
 
 bool varlen_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu_q, const Tensor& cu_k, int64_t max_q, int64_t max_k,
-                double scale_or_nan, bool causal, const Tensor& k_scale, const Tensor& v_scale, Tensor& out, Tensor& lse) {
+                double scale_or_nan, bool causal, const Tensor& k_scale, const Tensor& v_scale, Tensor& out, Tensor& lse, int shards = 1,
+                bool zigzag = false) {
   if (!q.is_cuda() || !on_device(k, q) || !on_device(v, q) || !cu_ok(cu_q, q) || !cu_ok(cu_k, q) || cu_q.numel() != cu_k.numel()) return false;
   const bool kv8 = k.scalar_type() == kFp8;
   const int dtype = dtype_code(q.scalar_type());
@@ -178,6 +184,13 @@ bool varlen_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor&
   const int* const cq = (const int*)cu_q.const_data_ptr();
   const int* const ck = (const int*)cu_k.const_data_ptr();
   float* const lp = (float*)lse.data_ptr();
+  if (shards > 1) {
+    // P stacked shards, cu_q describes one of them
+    if (kv8 || a.S % shards != 0 || b.S != a.S || b.st[1] != c.st[1]) return false;
+    const spa_shards rows = {shards, a.S / shards, a.S / shards, zigzag};
+    return spa_attention_fwd_varlen(a.p, b.p, c.p, o.p, lp, cq, nseq, a.H, a.S / shards, (int)max_q, a.D, a.st, b.st, c.st, o.st, &rows, scale, mask,
+                                    dtype, stream) == SPA_OK;
+  }
   if (kv8)
     return spa_flash_fwd_varlen_fp8kv(a.p, b.p, c.p, (const float*)k_scale.const_data_ptr(), (const float*)v_scale.const_data_ptr(), o.p, lp, cq, ck,
                                       nseq, a.H, a.S, b.S, (int)max_q, (int)max_k, a.D, a.st, b.st, c.st, o.st, scale, mask, dtype, stream) == SPA_OK;
@@ -203,12 +216,39 @@ bool differentiable_ok(const Tensor* t, int n) {
     if (!on_device(t[i], t[0]) || t[i].scalar_type() != t[0].scalar_type() || t[i].dim() < 3 || !rows_ok(t[i])) return false;
   return true;
 }
-bool attention_ok(const Tensor* t, int n) {
+// Where the rows lie: false when the operands do not agree.  zigzag: shards of a zigzag-sharded [B,S,H,D] ring, 0 = none.
+bool rows_of(const Tensor& first, const View& q, const View& k, const View& v, int64_t zigzag, spa_shards& rows, const spa_shards*& arg) {
+  arg = nullptr;
+  if (q.pitch != k.pitch || q.pitch != v.pitch) return false;
+  if (q.pitch) {
+    const int P = (int)first.size(0);
+    if (zigzag || k.S != q.S) return false;
+    if (q.pitch != q.B * (q.S / P)) return false;  // (the results and gradients are compact)
+    rows = {P, q.pitch, q.S / P, 0};
+    arg = &rows;
+  } else if (zigzag) {
+    if (zigzag < 1 || k.S != q.S || q.S % (2 * zigzag) != 0) return false;
+    rows = {(int)zigzag, (int)(q.S / zigzag), (int)(q.S / zigzag), 1};
+    arg = &rows;
+  }
+  return !arg || k.st[2] == v.st[2];
+}
+
+bool attention_ok(const Tensor* t, int n, int64_t zigzag) {
   Operands o;
+  spa_shards rows;
+  const spa_shards* arg;
   if (!differentiable_ok(t, n) || !operands(t, n, o)) return false;
   if (n < 3 && (t[n - 1].dim() != 5 || t[n - 1].size(2) != 4 - n)) return false;
   if (n == 3 && (t[0].dim() != t[1].dim() || t[0].dim() != t[2].dim() || (t[0].dim() == 5 && t[0].sizes() != t[1].sizes()))) return false;
-  return o.k.same_shape(o.v) && o.q.B == o.k.B && o.q.H == o.k.H && o.q.D == o.k.D && (o.q.D == 32 || o.q.D == 64 || o.q.D == 128);
+  if (!o.k.same_shape(o.v) || o.q.B != o.k.B || o.q.H != o.k.H || o.q.D != o.k.D || (o.q.D != 32 && o.q.D != 64 && o.q.D != 128)) return false;
+  if (!rows_of(t[0], o.q, o.k, o.v, zigzag, rows, arg)) return false;
+  if (!arg) return true;
+  // (what the kernels for rows in shards do not take: 2 GiB and more per (batch, head))
+  const int64_t span = (int64_t)(rows.shards - 1) * rows.pitch + o.q.S / rows.shards, esz = t[0].element_size();
+  for (const View* v : {&o.q, &o.k, &o.v})
+    if (((span - 1) * v->st[2] + v->D) * esz >= 0x7fffffffLL) return false;
+  return true;
 }
 
 void check(int rc) { TORCH_CHECK(rc == SPA_OK, "[spa ", rc, "] ", spa_last_error()); }
@@ -217,27 +257,37 @@ void check(int rc) { TORCH_CHECK(rc == SPA_OK, "[spa ", rc, "] ", spa_last_error
 // tile the score matrix).
 template <int N>
 struct Attention : public torch::autograd::Function<Attention<N>> {
-  static variable_list forward_of(const Tensor* t, double scale_or_nan, bool causal) {
+  static variable_list forward_of(const Tensor* t, double scale_or_nan, bool causal, int64_t zigzag) {
     Operands x;
     operands(t, N, x);
     const Tensor& q = t[0];
     void* const stream = current_stream();
     const c10::DeviceGuard guard(q.device());
-    Tensor out = N == 1 ? at::empty({x.q.B, x.q.S, x.q.H, x.q.D}, q.options()) : at::empty(q.sizes(), q.options());
+    Tensor out = N == 1 ? at::empty({x.q.B, x.q.S, x.q.H, x.q.D}, q.options()) : at::empty(q.sizes(), q.options());  // (compact: pitch B * s)
     Tensor lse = empty_f32({x.q.B, x.q.H, x.q.S}, q);
     View o;
     view_of(out, true, o);
-    check(spa_flash_fwd(x.q.p, x.k.p, x.v.p, o.p, (float*)lse.data_ptr(), x.q.B, x.q.H, x.q.S, x.k.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st,
-                        softmax_scale_or_default(scale_or_nan, x.q.D), causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype_code(q.scalar_type()), stream));
+    spa_shards rows;
+    const spa_shards* shards;
+    const float scale = softmax_scale_or_default(scale_or_nan, x.q.D);
+    const int mask = causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype = dtype_code(q.scalar_type());
+    rows_of(q, x.q, x.k, x.v, zigzag, rows, shards);
+    if (shards)
+      check(spa_attention_fwd(x.q.p, x.k.p, x.v.p, o.p, (float*)lse.data_ptr(), x.q.B, x.q.H, x.q.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, shards, scale,
+                              mask, dtype, stream));
+    else
+      check(spa_flash_fwd(x.q.p, x.k.p, x.v.p, o.p, (float*)lse.data_ptr(), x.q.B, x.q.H, x.q.S, x.k.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, scale, mask,
+                          dtype, stream));
     return {out, lse};
   }
-  static variable_list save(AutogradContext* ctx, const Tensor* t, double scale, bool causal) {
-    variable_list r = forward_of(t, scale, causal);
+  static variable_list save(AutogradContext* ctx, const Tensor* t, double scale, bool causal, int64_t zigzag) {
+    variable_list r = forward_of(t, scale, causal, zigzag);
     variable_list saved(t, t + N);
     saved.insert(saved.end(), r.begin(), r.end());
     ctx->save_for_backward(std::move(saved));
     ctx->saved_data["scale"] = scale;
     ctx->saved_data["causal"] = causal;
+    ctx->saved_data["zigzag"] = zigzag;
     ctx->mark_non_differentiable({r[1]});
     return r;
   }
@@ -249,7 +299,7 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
   static variable_list unpack(AutogradContext* ctx, std::index_sequence<I...>, Args&... args) {
     auto all = std::tie(args...);
     const Tensor t[N] = {std::get<I>(all)...};
-    return save(ctx, t, std::get<N>(all), std::get<N + 1>(all));
+    return save(ctx, t, std::get<N>(all), std::get<N + 1>(all), std::get<N + 2>(all));
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list saved = ctx->get_saved_variables();
@@ -261,18 +311,22 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
     void* const stream = current_stream();
     const c10::DeviceGuard guard(q.device());
     View o, d;
-    const Tensor dout = rows_ok(grads[0]) && view_of(grads[0], true, d) ? grads[0] : grads[0].contiguous();
+    view_of(out, true, o);
+    const Tensor dout = rows_ok(grads[0]) && view_of(grads[0], true, d) && d.pitch == o.pitch ? grads[0] : grads[0].contiguous();
     variable_list back;
     for (int i = 0; i < N; ++i) back.push_back(at::empty(saved[i].sizes(), saved[i].options()));
     operands(back.data(), N, g);
     const Tensor delta = empty_f32(lse.sizes(), lse);
-    TORCH_CHECK(view_of(out, true, o) && view_of(dout, true, d) && o.same_shape(d) && dout.scalar_type() == q.scalar_type(), "bad gradient of the output");
+    d = View();
+    TORCH_CHECK(view_of(dout, true, d) && o.same_shape(d) && dout.scalar_type() == q.scalar_type(), "bad gradient of the output");
     const int dtype = dtype_code(q.scalar_type());
+    spa_shards rows;
+    const spa_shards* shards;
+    rows_of(q, x.q, x.k, x.v, ctx->saved_data["zigzag"].toInt(), rows, shards);
     check(spa_attention_bwd(x.q.p, x.k.p, x.v.p, o.p, d.p, (const float*)lse.const_data_ptr(), (float*)delta.data_ptr(), g.q.p, g.k.p, g.v.p,
-                            x.q.B, x.q.H, x.q.S, x.k.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, d.st, g.q.st, g.k.st, g.v.st,
+                            x.q.B, x.q.H, x.q.S, x.k.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, d.st, g.q.st, g.k.st, g.v.st, shards,
                             softmax_scale_or_default(scale_or_nan, x.q.D), causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype, stream));
-    back.push_back(Tensor());
-    back.push_back(Tensor());
+    back.resize(N + 3);
     return back;
   }
 };
@@ -287,15 +341,17 @@ bool wants_grad(const Tensor* t, int n) {
 // Packed batch of sequences of different lengths.
 struct VarlenAttention : public torch::autograd::Function<VarlenAttention> {
   static variable_list forward(AutogradContext* ctx, Tensor q, Tensor k, Tensor v, Tensor cu_q, Tensor cu_k, int64_t max_q, int64_t max_k, double scale,
-                               bool causal, bool covered) {
+                               bool causal, bool covered, int64_t shards, bool zigzag) {
     Tensor out, lse;
-    TORCH_CHECK(varlen_fwd(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, Tensor(), Tensor(), out, lse), spa_last_error());
+    TORCH_CHECK(varlen_fwd(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, Tensor(), Tensor(), out, lse, (int)shards, zigzag), spa_last_error());
     ctx->save_for_backward({q, k, v, out, lse, cu_q, cu_k});
     ctx->saved_data["max_q"] = max_q;
     ctx->saved_data["max_k"] = max_k;
     ctx->saved_data["scale"] = scale;
     ctx->saved_data["causal"] = causal;
     ctx->saved_data["covered"] = covered;
+    ctx->saved_data["shards"] = shards;
+    ctx->saved_data["zigzag"] = zigzag;
     ctx->mark_non_differentiable({lse});
     return {out, lse};
   }
@@ -318,12 +374,14 @@ struct VarlenAttention : public torch::autograd::Function<VarlenAttention> {
     const int dtype = dtype_code(q.scalar_type());
     View o;
     view_thd(out, o);
+    const int P = (int)ctx->saved_data["shards"].toInt();
+    const spa_shards rows = {P, a.S / P, a.S / P, ctx->saved_data["zigzag"].toBool()};
     check(spa_attention_bwd_varlen(a.p, b.p, c.p, o.p, d.p, (const float*)lse.const_data_ptr(), (float*)delta.data_ptr(), g[0].p, g[1].p, g[2].p,
-                                   (const int*)s[5].const_data_ptr(), (const int*)s[6].const_data_ptr(), (int)s[5].numel() - 1, a.H, a.S, b.S,
+                                   (const int*)s[5].const_data_ptr(), (const int*)s[6].const_data_ptr(), (int)s[5].numel() - 1, a.H, a.S / P, b.S / P,
                                    (int)ctx->saved_data["max_q"].toInt(), (int)ctx->saved_data["max_k"].toInt(), a.D, a.st, b.st, c.st, o.st, d.st, g[0].st,
-                                   g[1].st, g[2].st, softmax_scale_or_default(ctx->saved_data["scale"].toDouble(), a.D),
+                                   g[1].st, g[2].st, P > 1 ? &rows : nullptr, softmax_scale_or_default(ctx->saved_data["scale"].toDouble(), a.D),
                                    ctx->saved_data["causal"].toBool() ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype, stream));
-    back.resize(10);
+    back.resize(12);
     return back;
   }
 };
@@ -403,7 +461,7 @@ PyObject* py_varlen_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// attention(tensors..., scale, causal): q, k, v | q, kv | qkv
+// attention(tensors..., scale, causal, zigzag shards or 0): q, k, v | q, kv | qkv
 template <int N, size_t... I>
 PyObject* attention(PyObject* const* a, std::index_sequence<I...>) {
   HANDLE_TH_ERRORS
@@ -411,35 +469,47 @@ PyObject* attention(PyObject* const* a, std::index_sequence<I...>) {
   double scale;
   for (int i = 0; i < N; ++i)
     if (!tensor_arg(a[i], t[i])) Py_RETURN_NONE;
-  if (!scale_arg(a[N], scale) || !attention_ok(t, N)) Py_RETURN_NONE;
+  if (!scale_arg(a[N], scale) || !PyLong_Check(a[N + 2])) Py_RETURN_NONE;
+  const int64_t zigzag = PyLong_AsLongLong(a[N + 2]);
+  if (zigzag < 0 || zigzag > 0x3fffffffLL || !attention_ok(t, N, zigzag)) Py_RETURN_NONE;
   const bool causal = flag_arg(a[N + 1]);
   variable_list r;
   {
     pybind11::gil_scoped_release no_gil;
-    r = wants_grad(t, N) ? Attention<N>::apply(t[I]..., scale, causal) : Attention<N>::forward_of(t, scale, causal);
+    r = wants_grad(t, N) ? Attention<N>::apply(t[I]..., scale, causal, zigzag) : Attention<N>::forward_of(t, scale, causal, zigzag);
   }
   return pair(r[0], r[1]);
   END_HANDLE_TH_ERRORS
 }
 PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n == 5) return attention<3>(a, std::make_index_sequence<3>{});
-  if (n == 4) return attention<2>(a, std::make_index_sequence<2>{});
-  if (n == 3) return attention<1>(a, std::make_index_sequence<1>{});
+  if (n == 6) return attention<3>(a, std::make_index_sequence<3>{});
+  if (n == 5) return attention<2>(a, std::make_index_sequence<2>{});
+  if (n == 4) return attention<1>(a, std::make_index_sequence<1>{});
   Py_RETURN_NONE;
 }
 
-// varlen_attention(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, covered)
+bool varlen_shards_ok(const View& q, const View& k, const View& v, int64_t longest, int64_t shards, int64_t esz) {
+  if (shards == 1) return true;
+  if (q.S % shards != 0 || k.S != q.S || k.st[1] != v.st[1]) return false;
+  for (const View* x : {&q, &k, &v})
+    if ((((shards - 1) * (q.S / shards) + longest - 1) * x->st[1] + x->D) * esz >= 0x7fffffffLL) return false;
+  return true;
+}
+
+// varlen_attention(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, covered, shards, zigzag)
 PyObject* py_varlen_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Tensor t[5];
   double scale;
-  if (n != 10) Py_RETURN_NONE;
+  if (n != 12 || !PyLong_Check(a[10])) Py_RETURN_NONE;
   for (int i = 0; i < 5; ++i)
     if (!tensor_arg(a[i], t[i])) Py_RETURN_NONE;
   if (!PyLong_Check(a[5]) || !PyLong_Check(a[6]) || !scale_arg(a[7], scale)) Py_RETURN_NONE;
   const int64_t mq = PyLong_AsLongLong(a[5]), mk = PyLong_AsLongLong(a[6]);
-  const bool causal = flag_arg(a[8]), covered = flag_arg(a[9]);
-  if (!differentiable_ok(t, 3) || !cu_ok(t[3], t[0]) || !cu_ok(t[4], t[0]) || mq <= 0 || mk <= 0 || mq > 0x7fffffffLL || mk > 0x7fffffffLL)
+  const int64_t shards = PyLong_AsLongLong(a[10]);
+  const bool causal = flag_arg(a[8]), covered = flag_arg(a[9]), zigzag = flag_arg(a[11]);
+  if (!differentiable_ok(t, 3) || !cu_ok(t[3], t[0]) || !cu_ok(t[4], t[0]) || mq <= 0 || mk <= 0 || mq > 0x7fffffffLL || mk > 0x7fffffffLL ||
+      shards < 1 || shards > 0xffffLL)
     Py_RETURN_NONE;
   variable_list r(2);
   {
@@ -447,11 +517,11 @@ PyObject* py_varlen_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (wants_grad(t, 3)) {
       View x, y, z;
       if (!view_thd(t[0], x) || !view_thd(t[1], y) || !view_thd(t[2], z) || !y.same_shape(z) || x.H != y.H || x.D != y.D || mq > x.S || mk > y.S ||
-          t[3].numel() != t[4].numel() || (x.D != 32 && x.D != 64 && x.D != 128))
+          t[3].numel() != t[4].numel() || !varlen_shards_ok(x, y, z, mq, shards, t[0].element_size()) || (x.D != 32 && x.D != 64 && x.D != 128))
         r.clear();
       else
-        r = VarlenAttention::apply(t[0], t[1], t[2], t[3], t[4], mq, mk, scale, causal, covered);
-    } else if (!varlen_fwd(t[0], t[1], t[2], t[3], t[4], mq, mk, scale, causal, Tensor(), Tensor(), r[0], r[1])) {
+        r = VarlenAttention::apply(t[0], t[1], t[2], t[3], t[4], mq, mk, scale, causal, covered, shards, zigzag);
+    } else if (!varlen_fwd(t[0], t[1], t[2], t[3], t[4], mq, mk, scale, causal, Tensor(), Tensor(), r[0], r[1], (int)shards, zigzag)) {
       r.clear();
     }
   }

@@ -197,11 +197,12 @@ class LongContextAttention(torch.nn.Module):
         if softmax_scale is None:
             softmax_scale = D ** (-0.5)
 
-        if B == 1 and query.shape == key.shape == value.shape:
-            # one batch entry: the stacked shards are the whole sequence, and neither the exchange (which head slice is
-            # where) nor the ring (in which order the blocks are visited) changes what is computed from it
+        if query.shape == key.shape == value.shape:
+            # every rank's rows are here, and neither the exchange (which head slice is where) nor the ring (in which order the
+            # blocks are visited) changes what is computed from them: one block call, whose kernels look up where each row
+            # of a sequence lies
             nat = _lib.native()
-            res = nat.attention(query, key, value, softmax_scale, causal) if nat is not None else None
+            res = nat.attention(query, key, value, softmax_scale, causal, 0) if nat is not None else None
             if res is not None:
                 if self.use_sync:
                     torch.cuda.synchronize()

@@ -253,16 +253,16 @@ def _attention(tensors, dropout_p, softmax_scale, causal, window_size, alibi_slo
     The blocks of a ring over contiguous shards tile the score matrix of the whole sequence, and this GPU holds every shard, so
     such a ring is one block call over the sequence (as its backward is): a launch per rank leaves CUs idle at every rank's end
     (ring of 8 over [1,8192,32,128], bf16, causal: 567 -> 490 us), and shards that no tile divides waste the rest of a tile
-    per rank and chunk.  Without a mask the order of the rows does not matter and zigzag shards are the same call.  Packed
-    tensors get packed gradients, written once by the kernels."""
+    per rank and chunk.  Zigzag shards: the same call, whose kernels look up where each row of the sequence lies (without a
+    mask the order of the rows does not matter).  Packed tensors get packed gradients, written once by the kernels."""
     P = int(ring_size)
-    shards = P if sharding == "contiguous" else 2 * P if sharding == "zigzag" and (P == 1 or not causal) else 0
+    shards = P if sharding == "contiguous" else 2 * P if sharding == "zigzag" else 0
     q, kv = tensors[0], tensors[-1]
     if shards > 0 and q.dim() >= 4 and q.shape[1] % shards == 0 and (P == 1 or kv.shape[1] == q.shape[1]):
         _check_unsupported(dropout_p, window_size, alibi_slopes)
         _no_multi_gpu(group)
         nat = _lib.native()
-        res = nat.attention(*tensors, softmax_scale, causal) if nat is not None else None
+        res = nat.attention(*tensors, softmax_scale, causal, P if shards == 2 * P and causal and P > 1 else 0) if nat is not None else None
         if res is not None:
             return (res[0], res[1], None) if return_attn_probs else res[0]
     if len(tensors) == 1:

@@ -209,13 +209,14 @@ class UlyssesFlashAttnFunc(torch.autograd.Function):
 def ulysses_flash_attn_func(q, k, v, dropout_p=0.0, softmax_scale=None, causal=False, window_size=(-1, -1),
                             alibi_slopes=None, deterministic=False, return_attn_probs=False, group=None):
     """sp_aurora/intel_ulysses_attn.py:501-548.  q,k,v rank-stacked [P,B,s,H,D] (or [B,S,H,D])."""
-    if q.dim() == 4 or (q.dim() == 5 and q.shape[1] == 1 and q.shape[3] % q.shape[0] == 0):
-        # one batch entry: the stacked shards are the whole sequence and the head groups lie side by side in it, so
-        # the attention of every rank's head group is one block call on the tensors as they are
+    if q.dim() == 4 or (q.dim() == 5 and q.shape[3] % q.shape[0] == 0 and q.shape == k.shape == v.shape):
+        # the head groups lie side by side in the stacked shards, and the kernels look up where each row of a sequence lies
+        # (with one batch entry the shards are the whole sequence in order), so the attention of every rank's head group
+        # is one block call on the tensors as they are
         _no_multi_gpu(group)
         _check_unsupported(dropout_p, window_size, alibi_slopes)
         nat = _lib.native()
-        res = nat.attention(q, k, v, softmax_scale, causal) if nat is not None else None
+        res = nat.attention(q, k, v, softmax_scale, causal, 0) if nat is not None else None
         if res is not None:
             return (res[0], None) if return_attn_probs else res[0]
     return UlyssesFlashAttnFunc.apply(q, k, v, dropout_p, softmax_scale, causal, window_size, alibi_slopes,

@@ -298,8 +298,17 @@ def sp_aurora_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k=None, max_seqlen=N
         # P stacked shards, cu_seqlens describes one of them (queries and keys alike)
         if cu_seqlens_k is not cu_seqlens_q or max_seqlen_k != max_seqlen or q.shape[0] % int(ring_size):
             raise ValueError("ring_size > 1 needs one cu_seqlens for queries and keys and packed rows divisible by ring_size")
-        if check_offsets:
-            ops.check_cu_seqlens_once(cu_seqlens_q, q.shape[0] // int(ring_size), max_seqlen, "cu_seqlens_q")
+        covered = check_offsets and ops.check_cu_seqlens_once(cu_seqlens_q, q.shape[0] // int(ring_size), max_seqlen, "cu_seqlens_q")
+        zigzag = sharding == "zigzag" and bool(causal)  # (without a mask the order of the rows does not matter)
+        if zigzag:
+            _half_major(cu_seqlens_q, q.shape[0] // int(ring_size))  # every length must be even
+        nat = _lib.native()
+        if nat is not None:
+            # every shard is here: one block call per sequence, whose kernels look up where its rows lie
+            res = nat.varlen_attention(q, k, v, cu_seqlens_q, cu_seqlens_q, max_seqlen, max_seqlen, softmax_scale, causal, covered, int(ring_size),
+                                       zigzag)
+            if res is not None:
+                return (res[0], res[1], None) if return_attn_probs else res[0]
         return VarlenRingFlashAttnFunc.apply(q, k, v, cu_seqlens_q, max_seqlen, softmax_scale, causal, return_attn_probs, int(ring_size),
                                              sharding == "zigzag")
     covered = False
@@ -313,7 +322,7 @@ def sp_aurora_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k=None, max_seqlen=N
     # above has shown that the offsets cover every row
     nat = _lib.native()
     if nat is not None:
-        res = nat.varlen_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen, max_seqlen_k, softmax_scale, causal, covered)
+        res = nat.varlen_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen, max_seqlen_k, softmax_scale, causal, covered, 1, False)
         if res is not None:
             return (res[0], res[1], None) if return_attn_probs else res[0]
     return VarlenFlashAttnFunc.apply(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen, max_seqlen_k, softmax_scale,

@@ -29,7 +29,7 @@ def test_every_packing_of_the_operands(packing, ring, S, D, dtype, causal):
     else:
         leaves = [torch.stack([q, k, v], 2).to(DEV).requires_grad_()]
         fn, split = spa.sp_aurora_qkvpacked_func, lambda g: tuple(g[0][:, :, i] for i in range(3))
-    assert _lib.native().attention(*leaves, None, causal) is not None  # a call this path takes
+    assert _lib.native().attention(*leaves, None, causal, 0) is not None  # a call this path takes
     out, lse, _ = fn(*leaves, causal=causal, return_attn_probs=True, ring_size=ring)
     assert not lse.requires_grad
     check_out(out, want, dtype)
@@ -48,7 +48,7 @@ def test_calls_that_need_more_than_the_native_path_still_run():
     wide = torch.zeros(1, 40, 2, 67, dtype=torch.bfloat16, device=DEV)
     wide[..., 3:] = q.to(DEV)
     odd = wide[..., 3:]  # rows that are not 16-byte aligned: copied by the Python path
-    assert _lib.native().attention(odd, k.to(DEV), v.to(DEV), 0.3, True) is None
+    assert _lib.native().attention(odd, k.to(DEV), v.to(DEV), 0.3, True, 0) is None
     check_out(spa.sp_aurora_func(odd, k.to(DEV), v.to(DEV), softmax_scale=0.3, causal=True), want, torch.bfloat16)
     with pytest.raises(ValueError):
         spa.sp_aurora_func(q, k, v)  # CPU tensors
