@@ -512,7 +512,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   // The loads of tile i + 3 go out one at a time between the MFMAs of the pass: issued in one burst
   // after the barrier, they hold up the wave's instruction stream while the memory pipeline takes them in.
   constexpr int LOAD_GAP = NBODY / G::NL;
-  for (int i = 0; i < nt; ++i) {
+  for (int i = 0; i < nt;) {
     // tile i+1 must have landed before this body reads it; tile i-1 is free for tile i+3
     wait_loads_but<G::NL>();
     __syncthreads();
@@ -576,6 +576,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
       sc = sn;
       dc = dn;
     }
+    if (++i == nt) mfma_settle();
   }
   wait_loads_but<0>();  // nothing may still be writing LDS when the workgroup ends
   // The last MFMAs must have written dq before it is read.  The accumulators are operands of the
@@ -1227,6 +1228,7 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
     }
     if (more) lstore(cur ^ 1);
     __syncthreads();
+    if (!more) mfma_settle();
   }
 
   if (krow < p.Sk && p.grads_in_t) {

@@ -348,5 +348,14 @@ static __device__ __forceinline__ u32x4 lds_read_b128(unsigned lds_addr) {
   return *(const __attribute__((address_space(3))) u32x4*)(lds_u8*)(uintptr_t)lds_addr;
 }
 
+// Wait states between the last matrix instruction of a loop (up to 16 passes) and the first read of its result.  hipcc places them by
+// itself for the builtins, but not behind a matrix instruction that is inline assembly, and it misses the shorter of two ways through
+// empty blocks: loops that a branch can leave right behind a matrix instruction end with this.
+static __device__ __forceinline__ void mfma_settle() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 static __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 static __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
