@@ -24,6 +24,7 @@ UNITS = [
     ("flash_fwd.hip", "flash_fwd_big.o", _FWD + ["-DSPA_FWD_BIG_UNIT"]),
     ("flash_fwd.hip", "flash_fwd_splitkv.o", _FWD + ["-DSPA_FWD_SPLITKV_UNIT"]),
     ("flash_fwd.hip", "flash_fwd_map.o", _FWD + ["-DSPA_FWD_MAP_UNIT"]),
+    ("flash_fwd32.hip", "flash_fwd32.o", _FWD),
     ("flash_bwd.hip", "flash_bwd.o", []),
     ("flash_bwd.hip", "flash_bwd_other.o", ["-DSPA_BWD_OTHER_UNIT"]),
     ("spa_abi.hip", "spa_abi.o", []),

@@ -1,0 +1,606 @@
+// Block attention forward for fp32 tensors: out = softmax(q k^T * scale + mask) v and lse, as in flash_fwd.hip (the same transposed
+// formulation; sp_aurora/intel_flash_attn.py:18-126).
+//
+// Both contractions run on the bf16 matrix instruction.  An fp32 value is the exact sum of three bf16 values, x = h + m + l (8 of
+// its 24 significant bits each, rounded to nearest: |m| <= 2^-8 |x|, |l| <= 2^-16 |x|), and a product of two bf16 values is
+// exact in fp32.  Of the nine products of two split values the six largest are formed, h h', h m', m h', h l', m m', l h'; the
+// three others are less than 2^-23 |x y| together and 2^-26 as a rule, either sign, where the chain of D fused operations that
+// they replace rounds D times at 2^-24 of the running sum (the scheme of Henry, Tang and Heinecke, "Leveraging the bfloat16
+// artificial intelligence datatype for higher-precision computations", 2019).  Against float64 the results are closer than those of
+// v_mfma_f32_32x32x2_f32 were: rms 2.7e-8 and 3.3e-8 at 2048 keys, D = 128, 1.6e-8 and 2.4e-8 at 512, D = 64.
+// That instruction does 64 operations a clock and SIMD; six bf16 products at 1024 do 170.
+// Bound: the matrix pipe, 6 * 2 * (D / 16) * 32 clocks per 32 x 32 scores, beside 136 vector instructions of softmax and splitting P
+// and 22 D / 16 of splitting K and V, once per workgroup and tile.
+#include "spa_common.h"
+#include "spa_host.h"
+
+namespace {
+
+typedef Mma16<__bf16> M;
+typedef M::frag frag;
+
+constexpr int F32_BN = 32;        // keys per tile
+constexpr int F32_THREADS = 256;  // 4 waves x 32 query rows
+
+// Two values as the three bf16 terms of each, packed in pairs.
+__device__ __forceinline__ void split2(float x0, float x1, unsigned& h, unsigned& m, unsigned& l) {
+  h = M::pack2(x0, x1);
+  const float r0 = x0 - __builtin_bit_cast(float, h << 16), r1 = x1 - __builtin_bit_cast(float, h & 0xffff0000u);
+  m = M::pack2(r0, r1);
+  l = M::pack2(r0 - __builtin_bit_cast(float, m << 16), r1 - __builtin_bit_cast(float, m & 0xffff0000u));
+}
+// Eight values as three operands.
+struct Split8 {
+  u32x4 h, m, l;
+  __device__ __forceinline__ void set(const float* x) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      unsigned a, b, c;
+      split2(x[2 * i], x[2 * i + 1], a, b, c);
+      h[i] = a;
+      m[i] = b;
+      l[i] = c;
+    }
+  }
+};
+// acc0 + acc1 += a b: the small terms and the large one in two accumulators (two chains of dependent instructions).
+__device__ __forceinline__ void mma6(const Split8& a, const Split8& b, f32x16& acc0, f32x16& acc1) {
+  const frag ah = as_frag<frag>(a.h), am = as_frag<frag>(a.m), al = as_frag<frag>(a.l);
+  const frag bh = as_frag<frag>(b.h), bm = as_frag<frag>(b.m), bl = as_frag<frag>(b.l);
+  acc1 = M::run(ah, bl, acc1);
+  acc0 = M::run(ah, bm, acc0);
+  acc1 = M::run(am, bm, acc1);
+  acc0 = M::run(am, bh, acc0);
+  acc1 = M::run(al, bh, acc1);
+  acc0 = M::run(ah, bh, acc0);
+}
+template <bool X>
+struct Bool {
+  static constexpr bool value = X;
+};
+__device__ __forceinline__ void zero16(f32x16& x) {
+#pragma unroll
+  for (int v = 0; v < 16; ++v) x[v] = 0.f;
+}
+
+// What a wave keeps of its 32 query rows, and one tile's softmax.
+template <int D>
+struct Rows {
+  Split8 q[D / 16];
+  f32x16 o[D / 32];
+  float m_run, l_run, c;
+  __device__ __forceinline__ void init(const float* row, int hh, bool negate, float scale_log2) {
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      float x[8];
+      const f32x4 a = *(const f32x4*)(row + ks * 16 + hh * 8), b = *(const f32x4*)(row + ks * 16 + hh * 8 + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[e] = negate ? -a[e] : a[e];  // negative softmax scale: -q with |scale|
+        x[4 + e] = negate ? -b[e] : b[e];
+      }
+      q[ks].set(x);
+    }
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) zero16(o[i]);
+    m_run = -INFINITY;
+    l_run = 0.f;
+    c = scale_log2;
+  }
+  // s: raw scores of the tile, keys the row does not see at -inf.  The reference maximum moves only when a row's has grown by
+  // more than 2^8 (flash_fwd.hip).
+  __device__ __forceinline__ void raise(const f32x16& s) {
+    float mx = s[0];
+#pragma unroll
+    for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
+    mx = halves_max(mx);
+    if (__builtin_amdgcn_ballot_w64(!((mx - m_run) * c <= 8.f)) != 0) {
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = m_new == -INFINITY ? 1.f : fast_exp2((m_run - m_new) * c);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[i][v] *= alpha;
+    }
+  }
+  // -> P as the two operands of the second contraction
+  __device__ __forceinline__ void weights(const f32x16& s, Split8 (&pf)[2]) {
+    const float mc = m_run == -INFINITY ? 0.f : m_run * c;
+    float ps[2] = {0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        x[e] = fast_exp2(__builtin_fmaf(s[8 * u + e], c, -mc));
+        ps[e & 1] += x[e];
+      }
+      pf[u].set(x);
+    }
+    l_run += ps[0] + ps[1];
+  }
+};
+
+// Sets the scores of the keys a row does not see to -inf; key0: the tile's first key.
+__device__ __forceinline__ void mask_tile(f32x16& s, int key0, int first_row, int qrow, bool causal, int Sk, int hh) {
+  if ((causal && key0 + F32_BN - 1 > first_row) || key0 + F32_BN > Sk) {
+    const int lim = causal ? (qrow < Sk - 1 ? qrow : Sk - 1) : Sk - 1;
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      if (key0 + 8 * (v >> 2) + 4 * hh + (v & 3) > lim) s[v] = -INFINITY;
+  }
+}
+
+// 16-byte chunk permutations of a tile row in LDS, as in flash_fwd.hip.
+template <int D>
+__device__ __forceinline__ int k_swizzle(int row) {
+  constexpr int CPR = D / 8;
+  return (row / (16 / CPR)) % CPR;
+}
+template <int D>
+__device__ __forceinline__ int v_swizzle(int row) {
+  return D == 128 ? (row & 3) << 2 : D == 64 ? ((row >> 1) & 1) << 2 : 0;
+}
+
+template <int D>
+struct Fwd32Cfg {
+  static constexpr int ROWB = D * 2;               // bytes of a row of one term
+  static constexpr int PLANE = F32_BN * ROWB;      // one term of a tile
+  static constexpr int TENSOR = 3 * PLANE;
+  static constexpr int SMEM = 4 * TENSOR;          // two tiles of K, two of V
+  static constexpr int CPR = D / 8;                // 8-value chunks per row
+  static constexpr int CHUNKS = F32_BN * CPR;      // of a tile
+  static constexpr int NC = (CHUNKS + F32_THREADS - 1) / F32_THREADS;  // per thread
+};
+
+// Many rows: a workgroup of 128 query rows; K and V tiles are split once, on their way into LDS, and read by its four waves.
+// Causal [1, 4096, 32, 128] 1289 -> 778 us (177 TFLOP/s, 1.06 PFLOP/s of bf16 products), [1, 4096, 16, 64] 440 -> 220, full
+// [1, 2048, 16, 32] 118 -> 90.
+template <int D>
+__global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_kernel(const FwdParams pk) {
+  typedef Fwd32Cfg<D> C;
+  FwdParams p = pk;  // a variable-length batch rewrites the sizes and bases for its sequence below
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  int b, h, qt;
+  if (p.cu_q) {
+    const int number = blockIdx.x / p.H;
+    h = blockIdx.x - number * p.H;
+    int nt = 0;
+    if (!sequence_tile(p.cu_q, p.B, p.map.P ? p.map.P : 1, 128, number, lane, b, qt, nt)) return;
+    qt = nt - 1 - qt;
+  } else {
+    const int pair = blockIdx.x + blockIdx.z * gridDim.x;
+    if (pair >= p.B * p.H) return;
+    h = pair % p.H;
+    b = pair / p.H;
+    qt = p.nqt - 1 - (int)blockIdx.y;
+  }
+  const int q0 = qt * 128, qw0 = q0 + w * 32;
+  if (p.cu_q) {
+    const int q_lo = p.cu_q[b], k_lo = p.cu_k[b];
+    p.Sq = p.cu_q[b + 1] - q_lo;
+    p.Sk = p.cu_k[b + 1] - k_lo;
+    p.q = (const float*)p.q + (int64_t)q_lo * p.qs.s;
+    p.k = (const float*)p.k + (int64_t)k_lo * p.ks.s;
+    p.v = (const float*)p.v + (int64_t)k_lo * p.vs.s;
+    p.out = (float*)p.out + (int64_t)q_lo * p.os.s;
+    p.lse += q_lo;
+    b = 0;
+    if (p.Sk <= 0) {
+      for (int idx = tid; idx < 128 * (D / 4); idx += F32_THREADS) {
+        const int grow = q0 + idx / (D / 4), ch = idx % (D / 4);
+        if (grow >= p.Sq) break;
+        f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        *(f32x4*)((float*)p.out + h * p.os.h + (int64_t)grow * p.os.s + ch * 4) = z;
+        if (ch == 0) p.lse[(int64_t)h * p.lse_bh + grow] = -INFINITY;
+      }
+      return;
+    }
+  }
+  RowMap map = {};
+  if (p.map.P) {
+    map.init(p.map, p.cu_q ? p.Sq : p.Sq / p.map.P);
+    if (p.cu_q) p.Sq = p.Sk = p.Sq * p.map.P;
+  }
+  auto row_of = [&](int r) { return p.map.P ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
+  auto stat_of = [&](int r) { return p.map.P ? map.at(r, p.map.lse_pitch) : r; };   // in lse
+
+  const float* qp = (const float*)p.q + b * p.qs.b + h * p.qs.h;
+  const float* kp = (const float*)p.k + b * p.ks.b + h * p.ks.h;
+  const float* vp = (const float*)p.v + b * p.vs.b + h * p.vs.h;
+  const int qrow = qw0 + ln, qrow_c = qrow < p.Sq ? qrow : p.Sq - 1;
+  Rows<D> rows;
+  rows.init(qp + (int64_t)row_of(qrow_c) * p.qs.s, hh, p.negq, p.scale_log2);
+
+  const int kv_end = p.causal ? (q0 + 128 < p.Sk ? q0 + 128 : p.Sk) : p.Sk;
+  const int nt = (kv_end + F32_BN - 1) / F32_BN;
+  const int seen = qw0 / F32_BN + (p.causal ? 1 : nt), ntw = seen < nt ? seen : nt;  // tiles this wave's rows see
+
+  // A thread's 8-value chunks of the tiles after next wait in registers.
+  f32x4 kreg[C::NC][2], vreg[C::NC][2];
+  auto gload = [&](const float* base, int64_t pitch, int it, f32x4 (&reg)[C::NC][2]) {
+#pragma unroll
+    for (int i = 0; i < C::NC; ++i) {
+      const int ch = tid + i * F32_THREADS;
+      if (C::CHUNKS % F32_THREADS == 0 || ch < C::CHUNKS) {
+        int r = it * F32_BN + ch / C::CPR;
+        r = row_of(r < p.Sk ? r : p.Sk - 1);
+        const float* a = base + (int64_t)r * pitch + (ch % C::CPR) * 8;
+        reg[i][0] = *(const f32x4*)a;
+        reg[i][1] = *(const f32x4*)(a + 4);
+      }
+    }
+  };
+  auto lstore = [&](unsigned char* base, bool vt, const f32x4 (&reg)[C::NC][2], int i) {
+    {
+      const int ch = tid + i * F32_THREADS;
+      if (C::CHUNKS % F32_THREADS == 0 || ch < C::CHUNKS) {
+        const int r = ch / C::CPR, pos = ch % C::CPR;
+        Split8 s;
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = reg[i][e >> 2][e & 3];
+        s.set(x);
+        unsigned char* const a = base + r * C::ROWB + ((pos ^ (vt ? v_swizzle<D>(r) : k_swizzle<D>(r))) * 16);
+        *(u32x4*)a = s.h;
+        *(u32x4*)(a + C::PLANE) = s.m;
+        *(u32x4*)(a + 2 * C::PLANE) = s.l;
+      }
+    }
+  };
+  // LDS: two tiles of K and two of V, K one tile ahead of V
+  auto kbuf = [&](int it) { return smem + (it & 1) * C::TENSOR; };
+  auto vbuf = [&](int it) { return smem + (2 + (it & 1)) * C::TENSOR; };
+
+  // operand addresses: K rows (16 bytes of row ln), V columns (the transposing read of flash_fwd.hip)
+  const unsigned lds0 = (unsigned)(uintptr_t)(lds_u8*)smem;
+  unsigned kra[D / 16], vra[D / 32];
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) kra[ks] = lds0 + ln * C::ROWB + (((2 * ks + hh) ^ k_swizzle<D>(ln)) * 16);
+  {
+    const int blk = lane >> 4, e = (lane >> 2) & 3, c4 = lane & 3, krl = 4 * hh + e;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db) {
+      const int chunk = db * 4 + (blk & 1) * 2 + (c4 >> 1);
+      vra[db] = lds0 + 2 * C::TENSOR + krl * C::ROWB + ((chunk ^ v_swizzle<D>(krl)) * 16) + (c4 & 1) * 8;
+    }
+  }
+  auto v_operand = [&](unsigned a) {
+    const u32x2 r0 = lds_read_tr16_b64(a), r1 = lds_read_tr16_b64(a + 8 * C::ROWB);
+    u32x4 x;
+    x[0] = r0[0];
+    x[1] = r0[1];
+    x[2] = r1[0];
+    x[3] = r1[1];
+    return x;
+  };
+  auto scores = [&](int it, f32x16& s) {
+    const unsigned st = (unsigned)((it & 1) * C::TENSOR);
+    f32x16 s1;
+    zero16(s);
+    zero16(s1);
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      Split8 a;
+      a.h = lds_read_b128(kra[ks] + st);
+      a.m = lds_read_b128(kra[ks] + st + C::PLANE);
+      a.l = lds_read_b128(kra[ks] + st + 2 * C::PLANE);
+      mma6(a, rows.q[ks], s, s1);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] += s1[v];
+  };
+
+  gload(kp, p.ks.s, 0, kreg);
+  gload(vp, p.vs.s, 0, vreg);
+  f32x4 k1[C::NC][2];
+  gload(kp, p.ks.s, 1, k1);
+#pragma unroll
+  for (int i = 0; i < C::NC; ++i) {
+    lstore(kbuf(0), false, kreg, i);
+    lstore(vbuf(0), true, vreg, i);
+    lstore(kbuf(1), false, k1, i);
+  }
+  gload(kp, p.ks.s, 2, kreg);
+  gload(vp, p.vs.s, 1, vreg);
+  __syncthreads();
+  f32x16 s;
+  scores(0, s);
+  mfma_settle();
+  __syncthreads();
+  // Step `it`: the weights of tile `it` are formed while the scores of tile it + 1 are, and the tiles after next are split and
+  // written while the products with V run: one wave on a SIMD keeps the matrix pipe and the vector unit busy together.  The
+  // compiler is told the mixture, since it would put the two streams one after the other; LDS writes come
+  // after the reads of the same quarter in program order, past which they could not be moved.
+  constexpr int CH = D > 32 ? 2 : 1;              // head-dim blocks at a time: chains of dependent matrix instructions
+  constexpr int GROUPS = 2 * (D / 32) / CH;       // of products with V
+  auto v_group = [&](unsigned st, int g, Split8 (&a)[CH]) {
+    const int u = g / (GROUPS / 2), db = g % (GROUPS / 2) * CH;
+#pragma unroll
+    for (int x = 0; x < CH; ++x) {
+      const unsigned at = vra[db + x] + st + u * 16 * C::ROWB;
+      a[x].h = v_operand(at);
+      a[x].m = v_operand(at + C::PLANE);
+      a[x].l = v_operand(at + 2 * C::PLANE);
+    }
+  };
+  auto store_next = [&](int it, int i) {  // quarter i of what a thread writes: half of K, or of V (all of each at D <= 64)
+    if (i < C::NC)
+      lstore(kbuf(it), false, kreg, i);
+    else if (i < 2 * C::NC)
+      lstore(vbuf(it + 1), true, vreg, i - C::NC);
+  };
+  auto step = [&](int it, auto last_c) {
+    constexpr bool last = decltype(last_c)::value;
+    const unsigned st = (unsigned)((it & 1) * C::TENSOR);
+    mask_tile(s, it * F32_BN, qw0, qrow, p.causal, p.Sk, hh);
+    rows.raise(s);
+    f32x16 sn;
+    Split8 pf[2];
+    __builtin_amdgcn_sched_barrier(0);
+    if (!last) scores(it + 1, sn);
+    rows.weights(s, pf);
+    Split8 a[2][CH];
+    v_group(st, 0, a[0]);
+    if (!last) {
+#pragma unroll
+      for (int i = 0; i < 6 * (D / 16); ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, (160 + 6 * (D / 16) - 1) / (6 * (D / 16)), 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+      const int u = g / (GROUPS / 2), db = g % (GROUPS / 2) * CH;
+      if (g + 1 < GROUPS) v_group(st, g + 1, a[(g + 1) & 1]);
+#pragma unroll
+      for (int term = 0; term < 6; ++term)
+#pragma unroll
+        for (int x = 0; x < CH; ++x) {
+          const Split8& av = a[g & 1][x];
+          const frag va = as_frag<frag>(term == 2 || term == 3 ? av.m : term == 4 ? av.l : av.h);
+          const frag pb = as_frag<frag>(term == 0 ? pf[u].l : term == 1 || term == 2 ? pf[u].m : pf[u].h);
+          rows.o[db + x] = M::run(va, pb, rows.o[db + x]);
+        }
+      store_next(it, g);
+#pragma unroll
+      for (int i = 0; i < 6 * CH; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, D > 32 ? 4 : 8, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    gload(kp, p.ks.s, it + 3, kreg);
+    gload(vp, p.vs.s, it + 2, vreg);
+    if (!last) s = sn;
+  };
+  int it = 0;
+  for (; it + 1 < ntw; ++it) {
+    step(it, Bool<false>());
+    __syncthreads();
+  }
+  step(it, Bool<true>());
+  while (++it < nt) {  // the workgroup's later rows see more
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2 * C::NC; ++i) store_next(it, i);
+    gload(kp, p.ks.s, it + 3, kreg);
+    gload(vp, p.vs.s, it + 2, vreg);
+  }
+
+  const float l_tot = halves_sum(rows.l_run), inv = 1.f / l_tot;
+  if (qrow < p.Sq) {
+    float* op = (float*)p.out + b * p.os.b + h * p.os.h + (int64_t)row_of(qrow) * p.os.s;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 st;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[e] = rows.o[db][4 * g + e] * inv;
+        *(f32x4*)(op + db * 32 + 8 * g + 4 * hh) = st;
+      }
+    if (hh == 0)
+      p.lse[((int64_t)b * p.H + h) * p.lse_bh + stat_of(qrow)] = (rows.m_run * rows.c + fast_log2(l_tot)) * 0.6931471805599453f;
+  }
+}
+
+// Few rows: a launch of the kernel above with fewer workgroups than CUs lasts as long as one wave's chain over all key tiles.
+// Here a workgroup owns 32 query rows and its NW waves take every NW-th key tile, straight from memory into operands (a lane
+// reads its own key's row of K, and a column of V 32 lanes wide per key) with no LDS and no barrier in the loop; the waves'
+// (O, m, l) are combined through LDS at the end.  Causal [1, 512, 32, 128] 83 -> 38 us, [1, 1697, 8, 64] 41.5 -> 37.
+template <int D, int NW>
+struct Fwd32SplitCfg {
+  static constexpr int REC = 64 * (D / 8) * 4;               // floats of one wave's O
+  static constexpr int SMEM = NW * (REC + 128) * 4;
+};
+
+template <int D, int NW>
+__global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const FwdParams p) {
+  typedef Fwd32SplitCfg<D, NW> C;
+  extern __shared__ __align__(16) unsigned char smem[];
+  float* const sm = (float*)smem;
+  const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int pair = blockIdx.x + blockIdx.z * gridDim.x;
+  if (pair >= p.B * p.H) return;
+  const int h = pair % p.H, b = pair / p.H;
+  const int q0 = (p.nqt - 1 - (int)blockIdx.y) * 32;
+  RowMap map = {};
+  if (p.map.P) map.init(p.map, p.Sq / p.map.P);
+  auto row_of = [&](int r) { return p.map.P ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
+  auto stat_of = [&](int r) { return p.map.P ? map.at(r, p.map.lse_pitch) : r; };   // in lse
+  const float* qp = (const float*)p.q + b * p.qs.b + h * p.qs.h;
+  const float* kp = (const float*)p.k + b * p.ks.b + h * p.ks.h;
+  const float* vp = (const float*)p.v + b * p.vs.b + h * p.vs.h;
+  const int qrow = q0 + ln, qrow_c = qrow < p.Sq ? qrow : p.Sq - 1;
+  const int kv_end = p.causal ? (q0 + 32 < p.Sk ? q0 + 32 : p.Sk) : p.Sk;
+  const int nt = (kv_end + F32_BN - 1) / F32_BN;
+
+  f32x4 kx[D / 16][2];
+  float vx[2][D / 32][8];
+  auto gload = [&](int it) {
+    int r = it * F32_BN + ln;
+    const float* a = kp + (int64_t)row_of(r < p.Sk ? r : p.Sk - 1) * p.ks.s + hh * 8;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      kx[ks][0] = *(const f32x4*)(a + ks * 16);
+      kx[ks][1] = *(const f32x4*)(a + ks * 16 + 4);
+    }
+    // operand element e of half u: key 16 u + 8 (e / 4) + 4 hh + e % 4, as the rows of an accumulator lie
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        r = it * F32_BN + 16 * u + 8 * (e >> 2) + 4 * hh + (e & 3);
+        const float* v = vp + (int64_t)row_of(r < p.Sk ? r : p.Sk - 1) * p.vs.s + ln;
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db) vx[u][db][e] = v[db * 32];
+      }
+  };
+  if (w < nt) gload(w);
+  Rows<D> rows;
+  rows.init(qp + (int64_t)row_of(qrow_c) * p.qs.s, hh, p.negq, p.scale_log2);
+  for (int it = w; it < nt; it += NW) {
+    const int key0 = it * F32_BN;
+    f32x16 s, s1;
+    zero16(s);
+    zero16(s1);
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = kx[ks][e >> 2][e & 3];
+      Split8 a;
+      a.set(x);
+      mma6(a, rows.q[ks], s, s1);
+    }
+    Split8 va[2][D / 32];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db) va[u][db].set(vx[u][db]);
+    if (it + NW < nt) gload(it + NW);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] += s1[v];
+    mask_tile(s, key0, q0, qrow, p.causal, p.Sk, hh);
+    Split8 pf[2];
+    rows.raise(s);
+    rows.weights(s, pf);
+#pragma unroll
+    for (int term = 0; term < 6; ++term)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db) {
+          const frag a = as_frag<frag>(term == 2 || term == 3 ? va[u][db].m : term == 4 ? va[u][db].l : va[u][db].h);
+          const frag pb = as_frag<frag>(term == 0 ? pf[u].l : term == 1 || term == 2 ? pf[u].m : pf[u].h);
+          rows.o[db] = M::run(a, pb, rows.o[db]);
+        }
+  }
+  // ---- combine: every wave leaves its unscaled O (lane-private order) and (m, l); wave j then finishes the
+  // 16-byte pieces j, j + NW, ... of every row ----
+  constexpr int NPC = D / 8;  // 16-byte pieces per lane: (db, g)
+  const float l_own = halves_sum(rows.l_run);
+  float* const orec = sm + w * (C::REC + 128);
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 st;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) st[e] = rows.o[db][4 * g + e];
+      *(f32x4*)(orec + ((db * 4 + g) * 64 + lane) * 4) = st;
+    }
+  if (hh == 0) {
+    orec[C::REC + ln] = rows.m_run;
+    orec[C::REC + 32 + ln] = l_own;
+  }
+  __syncthreads();
+  float mw[NW], m_all = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < NW; ++j) {
+    mw[j] = sm[j * (C::REC + 128) + C::REC + ln];
+    m_all = fmaxf(m_all, mw[j]);
+  }
+  float aw[NW], l_all = 0.f;
+#pragma unroll
+  for (int j = 0; j < NW; ++j) {
+    aw[j] = mw[j] == -INFINITY ? 0.f : fast_exp2((mw[j] - m_all) * rows.c);  // a wave without a visible key
+    l_all += aw[j] * sm[j * (C::REC + 128) + C::REC + 32 + ln];
+  }
+  const float inv = 1.f / l_all;
+  if (qrow < p.Sq) {
+    float* const op = (float*)p.out + b * p.os.b + h * p.os.h + (int64_t)row_of(qrow) * p.os.s;
+    for (int pc = w; pc < NPC; pc += NW) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NW; ++j) {
+        const f32x4 x = *(const f32x4*)(sm + j * (C::REC + 128) + (pc * 64 + lane) * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] += aw[j] * x[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] *= inv;
+      *(f32x4*)(op + (pc / 4) * 32 + 8 * (pc % 4) + 4 * hh) = acc;
+    }
+    if (w == 0 && hh == 0)
+      p.lse[((int64_t)b * p.H + h) * p.lse_bh + stat_of(qrow)] = (m_all * rows.c + fast_log2(l_all)) * 0.6931471805599453f;
+  }
+}
+
+template <auto kernel>
+hipError_t launch(int threads, int smem, int rows, const FwdParams& p, hipStream_t stream) {
+  const hipError_t e = spa_allow_dynamic_lds<kernel>(smem);
+  if (e != hipSuccess) return e;
+  dim3 grid;
+  if (p.cu_q) {
+    if (!spa_varlen_grid(p.H, p.B, p.lse_bh, rows, 1, grid)) return hipErrorInvalidValue;
+  } else {
+    if (p.nqt > 65535) return hipErrorInvalidValue;
+    grid = spa_head_groups((int64_t)p.B * p.H, p.nqt);
+  }
+  hipLaunchKernelGGL(kernel, grid, dim3(threads), smem, stream, p);
+  return hipGetLastError();
+}
+
+// Whether the waves of a workgroup share out the keys of 32 rows rather than taking 32 rows each.  A launch of the kernel for
+// many rows lasts as long as the longest chain of tiles, a launch of the other as long as its work on all SIMDs; microseconds per
+// tile and wave, and per tile and SIMD, fitted to 19 launches of 192 to 4096 rows: of these one is taken the wrong way, for 5 of 45 us.
+bool keys_shared(const FwdParams& p, int D) {
+  const double row_tiles = (p.Sq + 31) / 32, key_tiles = (p.Sk + F32_BN - 1) / F32_BN;
+  const double seen = p.causal && p.Sq <= p.Sk ? (row_tiles + 1) / 2 : key_tiles;  // per row tile (causal with fewer keys than rows: at most)
+  const double chain = p.causal && row_tiles < key_tiles ? row_tiles : key_tiles;
+  const double work = (double)p.B * p.H * row_tiles * seen / (4 * spa_device_cus());
+  const double per_chain = D == 128 ? 2.75 : D == 64 ? 1.43 : 1.3, per_work = D == 128 ? 2.75 : D == 64 ? 1.35 : 0.82;
+  const double many = chain * per_chain > work * per_work ? chain * per_chain : work * per_work;
+  return work * (D == 128 ? 6.0 : D == 64 ? 3.1 : 1.4) < many;
+}
+
+}  // namespace
+
+// One block pair, or whole sequences in shards (p.map).  Returns hipSuccess, or hipErrorInvalidValue for an unsupported D.
+hipError_t spa_launch_fwd32(FwdParams p, int D, hipStream_t stream) {
+  if (p.epi != SPA_EPI_PLAIN || p.P != 1 || p.nranks != 1) return hipErrorInvalidValue;  // ring steps merge with the separate kernel
+  const int knob = spa_knob(SPA_KNOB_FWD32_SPLIT);
+  if (!p.cu_q && knob != 1 && (knob == 2 || keys_shared(p, D))) {
+    p.nqt = (p.Sq + 31) / 32;
+    if (D == 128) return launch<flash_fwd32_splitk_kernel<128, 4>>(256, Fwd32SplitCfg<128, 4>::SMEM, 32, p, stream);
+    if (D == 64) return launch<flash_fwd32_splitk_kernel<64, 8>>(512, Fwd32SplitCfg<64, 8>::SMEM, 32, p, stream);
+    if (D == 32) return launch<flash_fwd32_splitk_kernel<32, 8>>(512, Fwd32SplitCfg<32, 8>::SMEM, 32, p, stream);
+    return hipErrorInvalidValue;
+  }
+  p.nqt = (p.Sq + 127) / 128;
+  if (D == 128) return launch<flash_fwd32_kernel<128>>(F32_THREADS, Fwd32Cfg<128>::SMEM, 128, p, stream);
+  if (D == 64) return launch<flash_fwd32_kernel<64>>(F32_THREADS, Fwd32Cfg<64>::SMEM, 128, p, stream);
+  if (D == 32) return launch<flash_fwd32_kernel<32>>(F32_THREADS, Fwd32Cfg<32>::SMEM, 128, p, stream);
+  return hipErrorInvalidValue;
+}

@@ -1,0 +1,41 @@
+"""The fp32 forward on three bf16 terms per value: both forms, every head dim, at the edges of their tiles (one key tile, two, a last
+one that is whole, workgroups whose later waves have no rows), against float64."""
+import pytest
+import torch
+
+from sp_aurora_amd import _lib, ops
+from test_gpu_parity import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("form", [1, 2])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Sq,Sk,causal", [(1, 1, False), (32, 32, True), (64, 64, False), (96, 128, False), (128, 128, True), (129, 160, False),
+                                          (33, 257, False), (300, 300, True), (200, 40, True)])
+def test_fp32_against_float64(form, D, Sq, Sk, causal):
+    g = torch.Generator().manual_seed(D + Sq + 7 * Sk)
+    H = 3
+    # values over six powers of ten: every term of a split value counts somewhere
+    q, k, v = (torch.randn((1, S, H, D), generator=g) * 10 ** (torch.rand((1, S, H, D), generator=g) * 6 - 5) for S in (Sq, Sk, Sk))
+    qh, kh, vh = (t.double().transpose(1, 2) for t in (q, k, v))
+    s, mass = qh @ kh.transpose(-1, -2) * D ** -0.5, qh.abs() @ kh.abs().transpose(-1, -2) * D ** -0.5
+    if causal:
+        hidden = torch.ones(Sq, Sk, dtype=torch.bool).triu(1)
+        s, mass = s.masked_fill(hidden, -float("inf")), mass.masked_fill(hidden, 0.0)
+    p = torch.softmax(s, -1)
+    want, lse = (p @ vh).transpose(1, 2), torch.logsumexp(s, -1)
+    # A score is off by at most 2^-23 of the sum of its products' sizes for the terms left out, and D / 16 + 6 roundings of 2^-24 for
+    # the sums, the exponent's argument and the exponential itself by 2^-22 more: a weight is off by that much of itself, an output
+    # by twice that and the roundings of its own sum, times what the weights and |v| add up to.
+    ds = mass * (2 + D / 16 + 6) * 2.0 ** -24 + (1 + s.abs().masked_fill(s.isinf(), 0.0)) * 2.0 ** -22
+    worst = ds.amax(-1)
+    bound = (2 * worst + (Sk / 16 + 8) * 2.0 ** -24)[..., None] * (p @ vh.abs())
+    _lib.tune("fwd32_split", form)
+    try:
+        out, got_lse = ops.flash_fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, causal, layout="bshd")
+    finally:
+        _lib.tune("fwd32_split", 0)
+    err = (out.cpu().double() - want).abs().transpose(1, 2)
+    assert (err <= bound + 1e-30).all(), float((err / bound).max())
+    assert ((got_lse.cpu().double() - lse).abs() <= 2 * worst + 2.0 ** -22 * (1 + lse.abs())).all()
