@@ -133,6 +133,53 @@ __device__ __forceinline__ void mask_tile(f32x16& s, int key0, int first_row, in
   }
 }
 
+// An infinity (or a value above the largest bf16 number) has no three exact terms: the rows that it reaches come out as NaN.  Rows
+// with a NaN are computed again here with plain fp32 operations and masked keys left out, so that they are infinite, finite or NaN as
+// the arithmetic of the inputs has it.  bad: the rows q0 + i of this wave, bit i; of the values d the wave stores those with
+// (d / 8) % NW == w, and the lse if w == 0.
+template <int D, int NW, typename RowOf, typename StatOf>
+__device__ __forceinline__ void plain_rows(const FwdParams& p, unsigned bad, int q0, const float* qp, const float* kp, const float* vp, float* out,
+                                           float* lse, float c, int lane, int w, RowOf row_of, StatOf stat_of) {
+  while (bad) {
+    const int qrow = q0 + __builtin_ctz(bad);
+    bad &= bad - 1;
+    const int keys = p.causal && qrow + 1 < p.Sk ? qrow + 1 : p.Sk;
+    const float* const q = qp + (int64_t)row_of(qrow) * p.qs.s;
+    const auto score = [&](int key) {
+      const float* const k = kp + (int64_t)row_of(key) * p.ks.s;
+      float s = 0.f;
+      for (int d = 0; d < D; ++d) s = __builtin_fmaf(q[d], k[d], s);
+      return p.negq ? -s : s;
+    };
+    float m = -INFINITY;
+    for (int key = lane; key < keys; key += 64) m = fmaxf(m, score(key));
+    for (int i = 1; i < 64; i *= 2) m = fmaxf(m, __shfl_xor(m, i));
+    const float mc = m == -INFINITY ? 0.f : m * c;
+    constexpr int ND = (D + 63) / 64;
+    float o[ND] = {}, l = 0.f;
+    for (int key0 = 0; key0 < keys; key0 += 64) {
+      const float x = key0 + lane < keys ? fast_exp2(__builtin_fmaf(score(key0 + lane), c, -mc)) : 0.f;
+      l += x;
+      const int n = keys - key0 < 64 ? keys - key0 : 64;
+      for (int j = 0; j < n; ++j) {
+        const float pj = __shfl(x, j);
+        const float* const v = vp + (int64_t)row_of(key0 + j) * p.vs.s;
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+          if (D % 64 == 0 || lane < D) o[i] = __builtin_fmaf(pj, v[i * 64 + lane], o[i]);
+      }
+    }
+    for (int i = 1; i < 64; i *= 2) l += __shfl_xor(l, i);
+    float* const to = out + (int64_t)row_of(qrow) * p.os.s;
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      const int d = i * 64 + lane;
+      if (d < D && (d / 8) % NW == w) to[d] = o[i] * (1.f / l);
+    }
+    if (lane == 0 && w == 0) lse[stat_of(qrow)] = (m * c + fast_log2(l)) * 0.6931471805599453f;
+  }
+}
+
 // 16-byte chunk permutations of a tile row in LDS, as in flash_fwd.hip.
 template <int D>
 __device__ __forceinline__ int k_swizzle(int row) {
@@ -397,19 +444,29 @@ __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_ker
   }
 
   const float l_tot = halves_sum(rows.l_run), inv = 1.f / l_tot;
+  float* const obase = (float*)p.out + b * p.os.b + h * p.os.h;
+  float* const lbase = p.lse + ((int64_t)b * p.H + h) * p.lse_bh;
+  bool bad = false;
   if (qrow < p.Sq) {
-    float* op = (float*)p.out + b * p.os.b + h * p.os.h + (int64_t)row_of(qrow) * p.os.s;
+    float* op = obase + (int64_t)row_of(qrow) * p.os.s;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         f32x4 st;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) st[e] = rows.o[db][4 * g + e] * inv;
+        for (int e = 0; e < 4; ++e) {
+          st[e] = rows.o[db][4 * g + e] * inv;
+          bad |= st[e] != st[e];
+        }
         *(f32x4*)(op + db * 32 + 8 * g + 4 * hh) = st;
       }
-    if (hh == 0)
-      p.lse[((int64_t)b * p.H + h) * p.lse_bh + stat_of(qrow)] = (rows.m_run * rows.c + fast_log2(l_tot)) * 0.6931471805599453f;
+    if (hh == 0) lbase[stat_of(qrow)] = (rows.m_run * rows.c + fast_log2(l_tot)) * 0.6931471805599453f;
+  }
+  const uint64_t nan = __builtin_amdgcn_ballot_w64(bad);
+  if (nan) {
+    __threadfence();  // (other lanes of this wave write those rows again)
+    plain_rows<D, 1>(p, (unsigned)(nan | nan >> 32), qw0, qp, kp, vp, obase, lbase, rows.c, lane, 0, row_of, stat_of);
   }
 }
 
@@ -538,8 +595,11 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
     l_all += aw[j] * sm[j * (C::REC + 128) + C::REC + 32 + ln];
   }
   const float inv = 1.f / l_all;
+  float* const obase = (float*)p.out + b * p.os.b + h * p.os.h;
+  float* const lbase = p.lse + ((int64_t)b * p.H + h) * p.lse_bh;
+  bool bad = false;
   if (qrow < p.Sq) {
-    float* const op = (float*)p.out + b * p.os.b + h * p.os.h + (int64_t)row_of(qrow) * p.os.s;
+    float* const op = obase + (int64_t)row_of(qrow) * p.os.s;
     for (int pc = w; pc < NPC; pc += NW) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -549,11 +609,18 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
         for (int e = 0; e < 4; ++e) acc[e] += aw[j] * x[e];
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] *= inv;
+      for (int e = 0; e < 4; ++e) {
+        acc[e] *= inv;
+        bad |= acc[e] != acc[e];
+      }
       *(f32x4*)(op + (pc / 4) * 32 + 8 * (pc % 4) + 4 * hh) = acc;
     }
-    if (w == 0 && hh == 0)
-      p.lse[((int64_t)b * p.H + h) * p.lse_bh + stat_of(qrow)] = (m_all * rows.c + fast_log2(l_all)) * 0.6931471805599453f;
+    if (w == 0 && hh == 0) lbase[stat_of(qrow)] = (m_all * rows.c + fast_log2(l_all)) * 0.6931471805599453f;
+  }
+  const uint64_t nan = __builtin_amdgcn_ballot_w64(bad);
+  if (nan) {
+    __threadfence();
+    plain_rows<D, NW>(p, (unsigned)(nan | nan >> 32), q0, qp, kp, vp, obase, lbase, rows.c, lane, w, row_of, stat_of);
   }
 }
 

@@ -39,3 +39,28 @@ def test_fp32_against_float64(form, D, Sq, Sk, causal):
     err = (out.cpu().double() - want).abs().transpose(1, 2)
     assert (err <= bound + 1e-30).all(), float((err / bound).max())
     assert ((got_lse.cpu().double() - lse).abs() <= 2 * worst + 2.0 ** -22 * (1 + lse.abs())).all()
+
+
+@pytest.mark.parametrize("form", [1, 2])
+@pytest.mark.parametrize("D,S,causal", [(32, 70, True), (64, 129, False), (128, 97, True)])
+def test_fp32_values_that_have_no_three_terms(form, D, S, causal):
+    """Infinities, a NaN and values above the largest bf16 number: they reach the results that they reach in plain arithmetic."""
+    g = torch.Generator().manual_seed(S)
+    H = 2
+    q, k, v = (torch.randn((1, S, H, D), generator=g) for _ in range(3))
+    v[0, 5, 0, 3], v[0, 20, 0, 9], v[0, 40, 1, 7] = float("inf"), -float("inf"), 3.4e38
+    k[0, S - 2, 1, 1] = float("nan")
+    s = (q.double().transpose(1, 2) @ k.double().transpose(1, 2).transpose(-1, -2)) * D ** -0.5
+    seen = torch.ones(S, S, dtype=torch.bool).tril() if causal else torch.ones(S, S, dtype=torch.bool)
+    p = torch.softmax(s.masked_fill(~seen, -float("inf")), -1)
+    terms = p[..., None] * v.double().transpose(1, 2)[:, :, None]
+    want = torch.where(seen[None, None, :, :, None], terms, torch.zeros(())).sum(3).transpose(1, 2)
+    _lib.tune("fwd32_split", form)
+    try:
+        out, lse = ops.flash_fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, causal, layout="bshd")
+    finally:
+        _lib.tune("fwd32_split", 0)
+    # plain sums of at most 130 terms: a score is off by D and a weight by 2^-22 |score| roundings, the sum by one rounding a key
+    torch.testing.assert_close(out.cpu().double(), want, rtol=1e-4, atol=1e-5, equal_nan=True)
+    want_lse = torch.logsumexp(s.masked_fill(~seen, -float("inf")), -1)
+    torch.testing.assert_close(lse.cpu().double(), want_lse, rtol=1e-5, atol=1e-5, equal_nan=True)
