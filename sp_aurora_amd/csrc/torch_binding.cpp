@@ -14,10 +14,12 @@
 #include <ATen/ops/zeros.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <cmath>
@@ -251,6 +253,12 @@ bool attention_ok(const Tensor* t, int n, int64_t zigzag) {
   return true;
 }
 
+// Saved tensors as the kernels can read them: what a saved-tensor hook hands back need not lie as what was saved.
+void to_kernel_rows(variable_list& saved, int n) {
+  for (int i = 0; i < n; ++i)
+    if (!rows_ok(saved[i])) saved[i] = saved[i].contiguous();
+}
+
 void check(int rc) { TORCH_CHECK(rc == SPA_OK, "[spa ", rc, "] ", spa_last_error()); }
 
 // Block attention over whole sequences (every ring whose contiguous shards this GPU holds is that: the blocks of the ring
@@ -302,16 +310,20 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
     return save(ctx, t, std::get<N>(all), std::get<N + 1>(all), std::get<N + 2>(all));
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const variable_list saved = ctx->get_saved_variables();
+    variable_list saved = ctx->get_saved_variables();
+    to_kernel_rows(saved, N + 1);
     const double scale_or_nan = ctx->saved_data["scale"].toDouble();
     const bool causal = ctx->saved_data["causal"].toBool();
     Operands x, g;
-    operands(saved.data(), N, x);
     const Tensor &q = saved[0], &out = saved[N], &lse = saved[N + 1];
     void* const stream = current_stream();
     const c10::DeviceGuard guard(q.device());
     View o, d;
-    view_of(out, true, o);
+    spa_shards rows;
+    const spa_shards* shards;
+    TORCH_CHECK(operands(saved.data(), N, x) && rows_of(q, x.q, x.k, x.v, ctx->saved_data["zigzag"].toInt(), rows, shards) &&
+                    view_of(out, true, o) && o.same_shape(x.q) && o.pitch == x.q.pitch && lse.is_contiguous(),
+                "saved tensors came back in another layout");
     const Tensor dout = rows_ok(grads[0]) && view_of(grads[0], true, d) && d.pitch == o.pitch ? grads[0] : grads[0].contiguous();
     variable_list back;
     for (int i = 0; i < N; ++i) back.push_back(at::empty(saved[i].sizes(), saved[i].options()));
@@ -320,9 +332,6 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
     d = View();
     TORCH_CHECK(view_of(dout, true, d) && o.same_shape(d) && dout.scalar_type() == q.scalar_type(), "bad gradient of the output");
     const int dtype = dtype_code(q.scalar_type());
-    spa_shards rows;
-    const spa_shards* shards;
-    rows_of(q, x.q, x.k, x.v, ctx->saved_data["zigzag"].toInt(), rows, shards);
     check(spa_attention_bwd(x.q.p, x.k.p, x.v.p, o.p, d.p, (const float*)lse.const_data_ptr(), (float*)delta.data_ptr(), g.q.p, g.k.p, g.v.p,
                             x.q.B, x.q.H, x.q.S, x.k.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, d.st, g.q.st, g.k.st, g.v.st, shards,
                             softmax_scale_or_default(scale_or_nan, x.q.D), causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype, stream));
@@ -335,6 +344,15 @@ bool wants_grad(const Tensor* t, int n) {
   if (!c10::GradMode::is_enabled()) return false;
   for (int i = 0; i < n; ++i)
     if (t[i].requires_grad()) return true;
+  return false;
+}
+
+// Calls whose derivative or recording is another mechanism's business: forward-mode tangents, torch.func transforms, a trace.  The
+// Python autograd functions refuse or record them.
+bool transformed(const Tensor* t, int n) {
+  if (torch::jit::tracer::isTracing() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) return true;
+  for (int i = 0; i < n; ++i)
+    if (t[i]._fw_grad(0).defined()) return true;
   return false;
 }
 
@@ -356,13 +374,16 @@ struct VarlenAttention : public torch::autograd::Function<VarlenAttention> {
     return {out, lse};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const variable_list s = ctx->get_saved_variables();
+    variable_list s = ctx->get_saved_variables();
+    to_kernel_rows(s, 4);
     const Tensor &q = s[0], &out = s[3], &lse = s[4];
     void* const stream = current_stream();
     const c10::DeviceGuard guard(q.device());
     const Tensor dout = rows_ok(grads[0]) ? grads[0] : grads[0].contiguous();
     View a, b, c, d, g[3];
-    TORCH_CHECK(view_thd(q, a) && view_thd(s[1], b) && view_thd(s[2], c) && view_thd(dout, d) && a.same_shape(d), "bad gradient of the output");
+    TORCH_CHECK(view_thd(q, a) && view_thd(s[1], b) && view_thd(s[2], c) && lse.is_contiguous() && cu_ok(s[5], q) && cu_ok(s[6], q),
+                "saved tensors came back in another layout");
+    TORCH_CHECK(view_thd(dout, d) && a.same_shape(d), "bad gradient of the output");
     // the kernels write the rows of the sequences; other rows' gradients are zero
     const bool covered = ctx->saved_data["covered"].toBool();
     variable_list back;
@@ -390,7 +411,7 @@ struct VarlenAttention : public torch::autograd::Function<VarlenAttention> {
 // Arguments come positionally from this package's own functions; a tensor argument that is no tensor (or a number that is no
 // number) is a call for the Python path, which raises what it always raised.
 bool tensor_arg(PyObject* o, Tensor& t) {
-  if (!THPVariable_Check(o)) return false;
+  if (!THPVariable_CheckExact(o)) return false;  // (a subclass has a say in what is done with it)
   t = THPVariable_Unpack(o);
   return true;
 }
@@ -471,7 +492,7 @@ PyObject* attention(PyObject* const* a, std::index_sequence<I...>) {
     if (!tensor_arg(a[i], t[i])) Py_RETURN_NONE;
   if (!scale_arg(a[N], scale) || !PyLong_Check(a[N + 2])) Py_RETURN_NONE;
   const int64_t zigzag = PyLong_AsLongLong(a[N + 2]);
-  if (zigzag < 0 || zigzag > 0x3fffffffLL || !attention_ok(t, N, zigzag)) Py_RETURN_NONE;
+  if (zigzag < 0 || zigzag > 0x3fffffffLL || transformed(t, N) || !attention_ok(t, N, zigzag)) Py_RETURN_NONE;
   const bool causal = flag_arg(a[N + 1]);
   variable_list r;
   {
@@ -508,7 +529,7 @@ PyObject* py_varlen_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t mq = PyLong_AsLongLong(a[5]), mk = PyLong_AsLongLong(a[6]);
   const int64_t shards = PyLong_AsLongLong(a[10]);
   const bool causal = flag_arg(a[8]), covered = flag_arg(a[9]), zigzag = flag_arg(a[11]);
-  if (!differentiable_ok(t, 3) || !cu_ok(t[3], t[0]) || !cu_ok(t[4], t[0]) || mq <= 0 || mk <= 0 || mq > 0x7fffffffLL || mk > 0x7fffffffLL ||
+  if (transformed(t, 3) || !differentiable_ok(t, 3) || !cu_ok(t[3], t[0]) || !cu_ok(t[4], t[0]) || mq <= 0 || mk <= 0 || mq > 0x7fffffffLL || mk > 0x7fffffffLL ||
       shards < 1 || shards > 0xffffLL)
     Py_RETURN_NONE;
   variable_list r(2);

@@ -258,7 +258,8 @@ def _attention(tensors, dropout_p, softmax_scale, causal, window_size, alibi_slo
     P = int(ring_size)
     shards = P if sharding == "contiguous" else 2 * P if sharding == "zigzag" else 0
     q, kv = tensors[0], tensors[-1]
-    if shards > 0 and q.dim() >= 4 and q.shape[1] % shards == 0 and (P == 1 or kv.shape[1] == q.shape[1]):
+    if (shards > 0 and q.dim() == (5 if len(tensors) == 1 else 4) and q.shape[1] % shards == 0
+            and (P == 1 or kv.shape[1] == q.shape[1])):
         _check_unsupported(dropout_p, window_size, alibi_slopes)
         _no_multi_gpu(group)
         nat = _lib.native()

@@ -78,3 +78,39 @@ def test_merge_of_two_blocks(S, H):
             assert o2 is out and l2 is lse
     check_out(out.transpose(1, 2), want, dtype)
     check_lse(lse.squeeze(-1).transpose(1, 2), want_lse)
+
+
+def test_rank_stacked_tensors_are_no_operands_of_a_ring():
+    q = torch.zeros(2, 2, 16, 2, 64, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(ValueError):
+        spa.sp_aurora_func(q, q, q, ring_size=2)
+    with pytest.raises(ValueError):
+        spa.sp_aurora_kvpacked_func(q, q)
+
+
+def _leaves(seed, dtype=torch.bfloat16):
+    return [t.to(DEV).requires_grad_() for t in rand_qkv((2, 40, 2, 64), seed, dtype)]
+
+
+def test_forward_mode_and_transforms_are_refused():
+    import torch.autograd.forward_ad as fwd_ad
+    q, k, v = (t.detach() for t in _leaves(730))
+    with fwd_ad.dual_level(), pytest.raises(RuntimeError):
+        spa.sp_aurora_func(fwd_ad.make_dual(q, torch.ones_like(q)), k, v)
+    with pytest.raises(RuntimeError):
+        torch.vmap(lambda x: spa.sp_aurora_func(x, k, v))(torch.stack([q, q]))
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda x: spa.sp_aurora_func(x, k, v).float().sum())(q)
+
+
+@pytest.mark.parametrize("unpack", [lambda t: t.to(DEV), lambda t: t.to(DEV).transpose(-1, -2).contiguous().transpose(-1, -2)])
+def test_saved_tensors_that_went_through_a_hook(unpack):
+    """Tensors offloaded to the host between forward and backward, and handed back in a layout that the kernels cannot read."""
+    leaves = _leaves(731)
+    dout = rand_qkv((2, 40, 2, 64), 732, torch.bfloat16, n=1)[0].to(DEV)
+    want = torch.autograd.grad(spa.sp_aurora_func(*leaves, causal=True), leaves, dout)
+    stays = lambda t: t.dim() == 4
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu() if stays(t) else t, lambda t: unpack(t) if stays(t) else t):
+        out = spa.sp_aurora_func(*leaves, causal=True)
+    for g, w in zip(torch.autograd.grad(out, leaves, dout), want):
+        assert torch.equal(g, w)
