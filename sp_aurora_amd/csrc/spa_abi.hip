@@ -741,6 +741,8 @@ int flash_bwd(const char* what, const void* q, const void* k, const void* v, con
       !aligned16(dout, do_strides, esz) || !aligned16(dq, dq_strides, gsz) || !aligned16(dk, dk_strides, gsz) ||
       !aligned16(dv, dv_strides, gsz) || (out && !aligned16(out, o_strides, esz)))
     return fail(SPA_EALIGN, "%s: pointers and row strides must be 16-byte aligned", what);
+  if (dtype != SPA_F32 && Sq > 1 && Sq % 128 != 0 && (q_strides[2] < D || do_strides[2] < D))
+    return fail(SPA_EUNSUPPORTED, "%s: rows of q and dout may not share memory", what);  // (rows past the end are zeros by their address)
   ShardMap map;
   if (rows) {
     if (Sq != Sk) return fail(SPA_EINVAL, "%s: rows in shards need as many keys as queries", what);
@@ -768,6 +770,7 @@ int flash_bwd(const char* what, const void* q, const void* k, const void* v, con
   p.big = big && dtype != SPA_F32;
   p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk;
   p.qs = S3(q_strides); p.ks = S3(k_strides); p.vs = S3(v_strides); p.dos = S3(do_strides);
+  if (Sq == 1) p.qs.s = p.dos.s = D;  // (the stride of a single row says nothing)
   p.dqs = S3(dq_strides); p.dks = S3(dk_strides); p.dvs = S3(dv_strides);
   p.scale = scale_eff(scale);
   p.scale_log2 = scale_eff(scale) * 1.4426950408889634f;
@@ -982,6 +985,8 @@ int flash_bwd_varlen(const char* what, const void* q, const void* k, const void*
       !aligned16v(dout, do_strides, esz) || !aligned16v(dq, dq_strides, gsz) || !aligned16v(dk, dk_strides, gsz) ||
       !aligned16v(dv, dv_strides, gsz) || (out && !aligned16v(out, o_strides, esz)) || (((uintptr_t)lse | (uintptr_t)delta) & 3) != 0)
     return fail(SPA_EALIGN, "%s: pointers and row strides must be 16-byte aligned", what);
+  if (dtype != SPA_F32 && (total_q > 1 || rows) && (q_strides[1] < D || do_strides[1] < D))
+    return fail(SPA_EUNSUPPORTED, "%s: rows of q and dout may not share memory", what);
   ShardMap map;
   if (rows) {
     if (cu_seqlens_q != cu_seqlens_k || total_q != total_k || max_sq != max_sk)
@@ -1007,6 +1012,7 @@ int flash_bwd_varlen(const char* what, const void* q, const void* k, const void*
   p.grads_in_t = grads_in_t;
   p.B = nseq; p.H = H; p.Sq = max_sq; p.Sk = max_sk;
   p.qs = S2(q_strides); p.ks = S2(k_strides); p.vs = S2(v_strides); p.dos = S2(do_strides);
+  if (total_q == 1 && !rows) p.qs.s = p.dos.s = D;
   p.dqs = S2(dq_strides); p.dks = S2(dk_strides); p.dvs = S2(dv_strides);
   p.scale = scale_eff(scale);
   p.scale_log2 = scale_eff(scale) * 1.4426950408889634f;

@@ -99,6 +99,10 @@ bool view_thd(const Tensor& t, View& v) {
   return true;
 }
 
+// Rows that lie over each other (a broadcast): the backward's kernels cannot stream such a q or gradient, whose rows past the end have
+// to be out of the tensor's range.
+bool rows_shared(const View& v, int row) { return v.S > 1 && v.st[row] < v.D; }
+
 bool on_device(const Tensor& t, const Tensor& q) { return t.is_cuda() && t.device() == q.device(); }
 
 // fp32 [n, H] on q's device.
@@ -243,6 +247,7 @@ bool attention_ok(const Tensor* t, int n, int64_t zigzag) {
   if (!differentiable_ok(t, n) || !operands(t, n, o)) return false;
   if (n < 3 && (t[n - 1].dim() != 5 || t[n - 1].size(2) != 4 - n)) return false;
   if (n == 3 && (t[0].dim() != t[1].dim() || t[0].dim() != t[2].dim() || (t[0].dim() == 5 && t[0].sizes() != t[1].sizes()))) return false;
+  if (rows_shared(o.q, 2)) return false;
   if (!o.k.same_shape(o.v) || o.q.B != o.k.B || o.q.H != o.k.H || o.q.D != o.k.D || (o.q.D != 32 && o.q.D != 64 && o.q.D != 128)) return false;
   if (!rows_of(t[0], o.q, o.k, o.v, zigzag, rows, arg)) return false;
   if (!arg) return true;
@@ -324,7 +329,7 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
     TORCH_CHECK(operands(saved.data(), N, x) && rows_of(q, x.q, x.k, x.v, ctx->saved_data["zigzag"].toInt(), rows, shards) &&
                     view_of(out, true, o) && o.same_shape(x.q) && o.pitch == x.q.pitch && lse.is_contiguous(),
                 "saved tensors came back in another layout");
-    const Tensor dout = rows_ok(grads[0]) && view_of(grads[0], true, d) && d.pitch == o.pitch ? grads[0] : grads[0].contiguous();
+    const Tensor dout = rows_ok(grads[0]) && view_of(grads[0], true, d) && d.pitch == o.pitch && !rows_shared(d, 2) ? grads[0] : grads[0].contiguous();
     variable_list back;
     for (int i = 0; i < N; ++i) back.push_back(at::empty(saved[i].sizes(), saved[i].options()));
     operands(back.data(), N, g);
@@ -379,8 +384,8 @@ struct VarlenAttention : public torch::autograd::Function<VarlenAttention> {
     const Tensor &q = s[0], &out = s[3], &lse = s[4];
     void* const stream = current_stream();
     const c10::DeviceGuard guard(q.device());
-    const Tensor dout = rows_ok(grads[0]) ? grads[0] : grads[0].contiguous();
     View a, b, c, d, g[3];
+    const Tensor dout = rows_ok(grads[0]) && view_thd(grads[0], d) && !rows_shared(d, 1) ? grads[0] : grads[0].contiguous();
     TORCH_CHECK(view_thd(q, a) && view_thd(s[1], b) && view_thd(s[2], c) && lse.is_contiguous() && cu_ok(s[5], q) && cu_ok(s[6], q),
                 "saved tensors came back in another layout");
     TORCH_CHECK(view_thd(dout, d) && a.same_shape(d), "bad gradient of the output");
@@ -537,7 +542,7 @@ PyObject* py_varlen_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     pybind11::gil_scoped_release no_gil;
     if (wants_grad(t, 3)) {
       View x, y, z;
-      if (!view_thd(t[0], x) || !view_thd(t[1], y) || !view_thd(t[2], z) || !y.same_shape(z) || x.H != y.H || x.D != y.D || mq > x.S || mk > y.S ||
+      if (!view_thd(t[0], x) || !view_thd(t[1], y) || !view_thd(t[2], z) || !y.same_shape(z) || rows_shared(x, 1) || x.H != y.H || x.D != y.D || mq > x.S || mk > y.S ||
           t[3].numel() != t[4].numel() || !varlen_shards_ok(x, y, z, mq, shards, t[0].element_size()) || (x.D != 32 && x.D != 64 && x.D != 128))
         r.clear();
       else

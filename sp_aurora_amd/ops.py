@@ -44,6 +44,13 @@ def _prep(t):
     return t if _rows_ok(t, t.element_size()) else t.contiguous()
 
 
+def _prep_streamed(t, row_dim):
+    """_prep for what the backward streams past its keys (q, dout): the kernels take rows past the end as zeros from a range check on
+    addresses, so rows must not share memory (a gradient broadcast along the sequence, as of a sum or mean over it)."""
+    t = _prep(t)
+    return t.contiguous() if t.shape[row_dim] > 1 and t.stride(row_dim) < t.shape[-1] else t
+
+
 FP8 = torch.float8_e4m3fn  # OCP e4m3: the 8-bit K/V format of spa_flash_fwd_fp8kv
 
 
@@ -537,7 +544,8 @@ def flash_bwd(q, k, v, dout, lse, delta, dq_acc, dk_acc, dv_acc, softmax_scale=N
     if not (lse.is_contiguous() and delta.is_contiguous()):
         raise ValueError("flash_bwd: lse and delta must be contiguous [B,H,Sq]")
     lib = _lib.load()
-    q, k, v, dout = _prep(q), _prep(k), _prep(v), _prep(dout)
+    row = 1 if layout == "bshd" else 2
+    q, k, v, dout = _prep_streamed(q, row), _prep(k), _prep(v), _prep_streamed(dout, row)
     qs, ks, vs, dos = _bhs(q, layout)[1], _bhs(k, layout)[1], _bhs(v, layout)[1], _bhs(dout, layout)[1]
     if not (_rows_ok(dq_acc, 4) and _rows_ok(dk_acc, 4) and _rows_ok(dv_acc, 4)):
         raise ValueError("flash_bwd: accumulators need an inner stride of 1 and 16-byte aligned rows")
@@ -624,7 +632,8 @@ def flash_bwd_out(q, k, v, dout, lse, delta, softmax_scale=None, causal=False, l
     for t in (lse, delta):
         if t.dtype != torch.float32 or not t.is_contiguous() or t.device != q.device:
             raise ValueError("flash_bwd_out: lse and delta must be contiguous float32 tensors on q's device")
-    q, k, v, dout = _prep(q), _prep(k), _prep(v), _prep(dout)
+    row = 1 if layout == "bshd" else 2
+    q, k, v, dout = _prep_streamed(q, row), _prep(k), _prep(v), _prep_streamed(dout, row)
     dq = torch.empty(q.shape, dtype=q.dtype, device=q.device) if dq is None else dq
     dk = torch.empty(k.shape, dtype=q.dtype, device=q.device) if dk is None else dk
     dv = torch.empty(v.shape, dtype=q.dtype, device=q.device) if dv is None else dv
@@ -762,7 +771,7 @@ def _flash_bwd_varlen(name, q, k, v, dout, lse, delta, dq, dk, dv, grad_dtype, c
     if cu_seqlens_q.numel() != cu_seqlens_k.numel():
         raise ValueError("cu_seqlens_q and cu_seqlens_k must describe the same number of sequences")
     lib = _lib.load()
-    q, k, v, dout = _prep(q), _prep(k), _prep(v), _prep(dout)
+    q, k, v, dout = _prep_streamed(q, 0), _prep(k), _prep(v), _prep_streamed(dout, 0)
     qs, ks, vs, dos = _thd(q, "q")[1], _thd(k, "k")[1], _thd(v, "v")[1], _thd(dout, "dout")[1]
     gsz = dq.element_size()
     if not (_rows_ok(dq, gsz) and _rows_ok(dk, gsz) and _rows_ok(dv, gsz)):

@@ -114,3 +114,38 @@ def test_saved_tensors_that_went_through_a_hook(unpack):
         out = spa.sp_aurora_func(*leaves, causal=True)
     for g, w in zip(torch.autograd.grad(out, leaves, dout), want):
         assert torch.equal(g, w)
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.float16), (32, torch.float32)])
+def test_strides_of_operands_and_gradients(D, dtype):
+    """Broadcast heads, batch entries and rows (stride 0), rows inside a wider tensor, heads before rows: the same as compact copies."""
+    B, S, H = 2, 150, 3
+    tol = {torch.bfloat16: 2e-2, torch.float16: 4e-3, torch.float32: 1e-5}[dtype]
+    base = [t.to(DEV) for t in rand_qkv((B, S, H, D), 733, dtype, n=4)]
+    forms = [lambda t: t[:, :, :1].expand(B, S, H, D), lambda t: t[:1].expand(B, S, H, D), lambda t: torch.cat([t, t], -1)[..., D:],
+             lambda t: t.transpose(1, 2).contiguous().transpose(1, 2), lambda t: torch.cat([t, t], 1)[:, 1:S + 1], lambda t: t[:, :1].expand(B, S, H, D)]
+    for f in forms:
+        for which in range(4):
+            x = [f(t) if i == which else t for i, t in enumerate(base)]
+            got, want = [], []
+            for ops_, res in ((x, got), ([t.contiguous() for t in x], want)):
+                leaves = [t.detach().requires_grad_() for t in ops_[:3]]
+                out = spa.sp_aurora_func(*leaves, causal=True)
+                res += [out, *torch.autograd.grad(out, leaves, ops_[3])]
+            for i, (g, w) in enumerate(zip(got, want)):
+                if f is forms[-1] and which == 0:  # the Python path, whose delta is summed in another order: a rounding of the type here and there
+                    torch.testing.assert_close(g, w, atol=tol, rtol=tol)
+                else:
+                    assert torch.equal(g, w), (forms.index(f), which, i)
+            if which == 3 and f is forms[-1]:  # the Python path's kernels, and a packed batch
+                out, lse = want[0].detach(), spa.sp_aurora_func(*[t.detach() for t in base[:3]], causal=True, return_attn_probs=True)[1]
+                for g, w in zip(spa.ring.ring_flash_attn_backward(x[3], *base[:3], out, lse, None, True), want[1:]):
+                    torch.testing.assert_close(g, w, atol=tol, rtol=tol)
+                cu = torch.tensor([0, S, B * S], dtype=torch.int32, device=DEV)
+                grads = []
+                packed_dout = base[3][:1, :1].expand(B, S, H, D).reshape(B * S, H, D)
+                for d in (base[3][0, :1].expand(B * S, H, D), packed_dout):
+                    leaves = [t.reshape(B * S, H, D).clone().requires_grad_() for t in base[:3]]
+                    grads.append(torch.autograd.grad(spa.sp_aurora_varlen_func(*leaves, cu, max_seqlen=S, causal=True), leaves, d))
+                for g, w in zip(*grads):
+                    assert torch.equal(g, w)
