@@ -446,6 +446,22 @@ int spa_flash_fwd_varlen(const void* q, const void* k, const void* v, void* out,
                          float scale, int mask_mode, int dtype, void* stream);
 
 /*
+ * spa_flash_fwd_varlen / _fp8kv (k_scale, v_scale not null) without a mask, with the keys of every sequence cut into chunks of `chunk` keys
+ * that run side by side where max_sq <= 3 (a decode step of a batch with ragged caches; other calls run as if not cut): a launch of one
+ * workgroup per sequence and head lasts as long as the longest sequence, and few of them leave CUs idle.  The chunks' fp32 sums wait in
+ * the workspace (spa_flash_fwd_varlen_splitkv_workspace_bytes() bytes, 16-byte aligned, the caller's) for a second kernel.
+ * spa_flash_fwd_varlen_splitkv_suggest: the chunk the library would take (0: do not split).  Call sites as spa_flash_fwd_splitkv.
+ */
+int64_t spa_flash_fwd_varlen_splitkv_workspace_bytes(int nseq, int H, int total_k, int max_sq, int max_sk, int D, int chunk);
+int spa_flash_fwd_varlen_splitkv_suggest(int nseq, int H, int total_k, int max_sq, int max_sk, int D, int dtype);
+int spa_flash_fwd_varlen_splitkv(const void* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
+                                 void* out, float* lse, void* workspace, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                 int nseq, int H, int total_q, int total_k, int max_sq, int max_sk, int D, int chunk,
+                                 const int64_t q_strides[2], const int64_t k_strides[2],
+                                 const int64_t v_strides[2], const int64_t o_strides[2],
+                                 float scale, int dtype, void* stream);
+
+/*
  * The ring over a packed variable-length batch in one launch per rank (or one for all ranks): the reference's varlen test
  * runs its function under a process group (test/flash_attention/test_intel_ring_flash_attn_varlen.py:150-215), i.e. every
  * rank holds the r-th of P equal slices of EVERY sequence, packed alike on every rank.  q, k, v, out: the P shards stacked,

@@ -65,6 +65,9 @@ SIGNATURES = {
     "spa_attention_bwd": (_i, [_vp] * 10 + [_i] * 5 + [_s3] * 8 + [_sh, _f, _i, _i, _vp]),
     "spa_attention_bwd_varlen": (_i, [_vp] * 12 + [_i] * 7 + [_s3] * 8 + [_sh, _f, _i, _i, _vp]),
     "spa_flash_fwd_varlen": (_i, [_vp] * 7 + [_i] * 7 + [_s3] * 4 + [_f, _i, _i, _vp]),
+    "spa_flash_fwd_varlen_splitkv_workspace_bytes": (ctypes.c_int64, [_i] * 7),
+    "spa_flash_fwd_varlen_splitkv_suggest": (_i, [_i] * 7),
+    "spa_flash_fwd_varlen_splitkv": (_i, [_vp] * 10 + [_i] * 8 + [_s3] * 4 + [_f, _i, _vp]),
     "spa_ring_fwd_varlen": (_i, [_vp] * 6 + [_i] * 7 + [_s3] * 4 + [_f, _i, _i, _i, _vp]),
     "spa_flash_bwd_varlen": (_i, [_vp] * 11 + [_i] * 7 + [_s3] * 7 + [_f, _i, _i, _vp]),
     "spa_flash_bwd_varlen_out": (_i, [_vp] * 11 + [_i] * 7 + [_s3] * 7 + [_f, _i, _i, _vp]),
@@ -82,7 +85,8 @@ class SpaError(RuntimeError):
 
 
 # entry points that return an int but launch nothing: they run as they are while recording
-_QUERIES = ("spa_abi_version", "spa_tune", "spa_device_info", "spa_static_scratch_init", "spa_flash_fwd_splitkv_suggest")
+_QUERIES = ("spa_abi_version", "spa_tune", "spa_device_info", "spa_static_scratch_init", "spa_flash_fwd_splitkv_suggest",
+            "spa_flash_fwd_varlen_splitkv_suggest")
 
 
 class _Recorder:

@@ -9,8 +9,9 @@
 // (running max, running sum, NQ x E accumulators) lives in the group of lanes and covers the rows that group saw.
 // At the end the groups of a wave merge by shuffles and the waves of the workgroup through LDS.
 //
-// Grid: x = batch * head, y = key chunk (the key split of the caller: chunk y writes rows y * Sq .. of the result
-// tensors it is given).  256 threads.
+// Grid: x = batch * head (or group of HP heads), y = key chunk (the key split of the caller: chunk y writes rows y * Sq .. of the result
+// tensors it is given; of a packed batch, whose sequences have chunks of one length and as many as they need: fp32 partial
+// sums, merged by fewrows_combine_kernel).  256 threads.
 #include "spa_common.h"
 #include "spa_host.h"
 
@@ -57,17 +58,23 @@ struct Piece<T, true> {
   }
 };
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+// What a chunk of a packed batch leaves in the workspace: per (sequence, head, row, chunk) D sums, and behind all of those (max, sum).
+__host__ __device__ inline int64_t part_stats(int64_t pairs, int nq, int n, int D) { return pairs * nq * n * D; }
+
 // kUnroll: loads of K (and of V) a wave keeps in flight.  NT: the loads carry the non-temporal hint (K and V are read
 // once and should not displace anything in the caches).
-template <typename T, int D, bool KV8, int NQ, int kUnroll, bool NT>
+// HP: neighbouring heads a workgroup takes together, whose pieces of a key row lie side by side.
+template <typename T, int D, bool KV8, int NQ, int kUnroll, bool NT, int HP>
 __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParams p) {
   constexpr int AUX = NT ? 2 : 0;
   typedef Piece<T, KV8> Pc;
   constexpr int E = Pc::E;
-  constexpr int LPR = D / E;        // lanes per key row
+  constexpr int LPH = D / E;        // lanes per key row and head
+  constexpr int LPR = LPH * HP;     // lanes per key row
   constexpr int R = 64 / LPR;       // key rows per load of a wave
   constexpr int KESZ = KV8 ? 1 : 2;
-  static_assert(LPR == 4 || LPR == 8 || LPR == 16, "row spread");
+  static_assert((LPH == 4 || LPH == 8 || LPH == 16) && LPR <= 16, "row spread");
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // Workgroups go to the 8 XCDs round robin.  Where a key row of one head is half a cache line (64 e4m3 elements), two
@@ -75,45 +82,48 @@ __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParam
   // time, so that the line comes from HBM once (3.1 -> 4.6-5.1 TB/s; with rows of a whole line or more the same
   // placement is 3-10 % slower than heads round robin).
   int bh = blockIdx.x;
-  if (D * KESZ < 128 && (gridDim.x & 7) == 0) bh = (bh & 7) * (int)(gridDim.x >> 3) + (bh >> 3);
+  if (D * KESZ * HP < 128 && (gridDim.x & 7) == 0) bh = (bh & 7) * (int)(gridDim.x >> 3) + (bh >> 3);
+  bh *= HP;
   const int z = blockIdx.y;
   int b = bh / p.H;
-  const int h = bh - b * p.H;
+  const int h = bh - b * p.H;                    // the first of the heads
   const int c = lane % LPR, g = lane / LPR;
+  const int own = c / LPH;                       // this lane's head is h + own
   int k0 = z * p.Sk;
   int k1 = k0 + (z == p.P - 1 ? p.sk_last : p.Sk);
   int nq = NQ;                                   // rows of this (batch or sequence, head) that exist
   int64_t q_row0 = 0, k_row0 = 0;                // first row of the sequence in the packed tensors
-  int64_t lse_base = (int64_t)bh * p.lse_bh;     // lse is [B, H, rows], or [H, packed rows] for a packed batch
+  int64_t lse_base = (int64_t)bh * p.lse_bh;     // of head h; lse is [B, H, rows], or [H, packed rows] for a packed batch
   if (p.cu_q) {
-    // a packed variable-length batch: sequence b owns rows cu_q[b] .. of q / out / lse and cu_k[b] .. of K / V
-    // (one chunk: the keys of such a batch are not split)
+    // a packed variable-length batch: sequence b owns rows cu_q[b] .. of q / out / lse and cu_k[b] .. of K / V, and
+    // this workgroup chunk z of its keys (the last chunk of the grid takes what is left)
     q_row0 = p.cu_q[b];
     k_row0 = p.cu_k[b];
     nq = p.cu_q[b + 1] - (int)q_row0;
     nq = nq < NQ ? nq : NQ;
-    k0 = 0;
     k1 = p.cu_k[b + 1] - (int)k_row0;
+    if (z > 0 && k0 >= k1) return;
+    if (z != p.P - 1 && k1 > k0 + p.Sk) k1 = k0 + p.Sk;
     lse_base = (int64_t)h * p.lse_bh + q_row0;
     b = 0;
     if (nq <= 0) return;
     if (k1 <= 0) {
       // no keys: the empty sum, out = 0 and lse = -inf
-      for (int t = threadIdx.x; t < nq * D; t += kWaves * 64) {
-        const int i = t / D, d = t - i * D;
-        ((T*)p.out)[h * p.os.h + (q_row0 + i) * p.os.s + d] = (T)0.f;
-        if (d == 0) p.lse[lse_base + i] = -INFINITY;
+      for (int t = threadIdx.x; t < nq * HP * D; t += kWaves * 64) {
+        const int i = t / (HP * D), hd = t / D % HP, d = t % D;
+        ((T*)p.out)[(h + hd) * p.os.h + (q_row0 + i) * p.os.s + d] = (T)0.f;
+        if (d == 0) p.lse[lse_base + hd * p.lse_bh + i] = -INFINITY;
       }
       return;
     }
   }
 
   // the rows' queries, this lane's elements, scaled into the exponent's base-2 domain
-  const float qmul = (p.negq ? -p.scale_log2 : p.scale_log2) * (KV8 ? p.k_scale[bh] : 1.f);
+  const float qmul = (p.negq ? -p.scale_log2 : p.scale_log2) * (KV8 ? p.k_scale[bh + own] : 1.f);
   float qf[NQ][E];
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
-    const T* qp = (const T*)p.q + b * p.qs.b + h * p.qs.h + (q_row0 + (i < nq ? i : nq - 1)) * p.qs.s + c * E;
+    const T* qp = (const T*)p.q + b * p.qs.b + (h + own) * p.qs.h + (q_row0 + (i < nq ? i : nq - 1)) * p.qs.s + c % LPH * E;
 #pragma unroll
     for (int e0 = 0; e0 < E; e0 += 8) {
       float t[8];
@@ -128,9 +138,9 @@ __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParam
   const char* kp = (const char*)p.k + (b * p.ks.b + h * p.ks.h + k_row0 * p.ks.s) * KESZ;
   const char* vp = (const char*)p.v + (b * p.vs.b + h * p.vs.h + k_row0 * p.vs.s) * KESZ;
   const __amdgpu_buffer_rsrc_t krs =
-      __builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, (int)((unsigned)((int64_t)(k1 - 1) * krow_b) + D * KESZ), 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, (int)((unsigned)((int64_t)(k1 - 1) * krow_b) + HP * D * KESZ), 0x00020000);
   const __amdgpu_buffer_rsrc_t vrs =
-      __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, (int)((unsigned)((int64_t)(k1 - 1) * vrow_b) + D * KESZ), 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, (int)((unsigned)((int64_t)(k1 - 1) * vrow_b) + HP * D * KESZ), 0x00020000);
 
   float m[NQ], l[NQ], acc[NQ][E];
 #pragma unroll
@@ -174,7 +184,7 @@ __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParam
         float d = 0.f;
 #pragma unroll
         for (int e = 0; e < E; ++e) d = __builtin_fmaf(qf[i][e], kf[e], d);
-        d = group_sum<LPR>(d);
+        d = group_sum<LPH>(d);
         s[i][u] = live ? d : -INFINITY;
       }
     }
@@ -210,7 +220,7 @@ __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParam
   }
 
   // the R groups of the wave: common max, then sums across the lanes that hold the same elements
-  __shared__ float sm_m[NQ][kWaves], sm_l[NQ][kWaves], sm_acc[NQ][kWaves][D];
+  __shared__ float sm_m[NQ][kWaves][HP], sm_l[NQ][kWaves][HP], sm_acc[NQ][kWaves][HP * D];
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
     float mx = m[i];
@@ -228,62 +238,104 @@ __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParam
       for (int off = LPR; off < 64; off <<= 1) a += __shfl_xor(a, off, 64);
       if (g == 0) sm_acc[i][wave][c * E + e] = a;
     }
-    if (lane == 0) {
-      sm_m[i][wave] = mx;
-      sm_l[i][wave] = ls;
+    if (g == 0 && c % LPH == 0) {
+      sm_m[i][wave][own] = mx;
+      sm_l[i][wave][own] = ls;
     }
   }
   __syncthreads();
 
-  // the waves of the workgroup: thread t takes element t % D of row t / D
-  const float vmul = KV8 ? p.v_scale[bh] : 1.f;
-  for (int t = threadIdx.x; t < NQ * D; t += kWaves * 64) {
-    const int i = t / D, d = t - i * D;
-    float mx = sm_m[i][0];
+  // the waves of the workgroup: thread t takes element t % D of one row and head
+  for (int t = threadIdx.x; t < NQ * HP * D; t += kWaves * 64) {
+    const int i = t / (HP * D), hd = t / D % HP, d = t % D;
+    const float vmul = KV8 ? p.v_scale[bh + hd] : 1.f;
+    float mx = sm_m[i][0][hd];
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) mx = fmaxf(mx, sm_m[i][w]);
+    for (int w = 1; w < kWaves; ++w) mx = fmaxf(mx, sm_m[i][w][hd]);
     float ls = 0.f, a = 0.f;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-      const float f = __builtin_amdgcn_exp2f(sm_m[i][w] - mx);   // (every chunk holds a key: mx is finite)
-      ls += sm_l[i][w] * f;
-      a += sm_acc[i][w][d] * f;
+      const float f = __builtin_amdgcn_exp2f(sm_m[i][w][hd] - mx);   // (every chunk holds a key: mx is finite)
+      ls += sm_l[i][w][hd] * f;
+      a += sm_acc[i][w][hd * D + d] * f;
     }
     if (i >= nq) break;
+    if (p.cu_q && p.P > 1) {
+      const int64_t at = ((int64_t)(bh + hd) * NQ + i) * p.P + z;
+      ((float*)p.part)[at * D + d] = a;
+      if (d == 0) *(f32x2*)((float*)p.part + part_stats((int64_t)p.B * p.H, NQ, p.P, D) + at * 2) = f32x2{mx, ls};
+      continue;
+    }
     const int64_t orow = (int64_t)z * p.Sq + i;
-    T* op = (T*)p.out + b * p.os.b + h * p.os.h + (q_row0 + orow) * p.os.s;
+    T* op = (T*)p.out + b * p.os.b + (h + hd) * p.os.h + (q_row0 + orow) * p.os.s;
     op[d] = (T)(a * vmul / ls);
-    if (d == 0) p.lse[lse_base + orow] = (mx + __builtin_amdgcn_logf(ls)) * 0.6931471805599453f;
+    if (d == 0) p.lse[lse_base + hd * p.lse_bh + orow] = (mx + __builtin_amdgcn_logf(ls)) * 0.6931471805599453f;
   }
 }
 
-// Measured on twelve decode shapes: four loads in flight beat eight (6-10 %) except with three rows and with 64-byte
-// rows; the non-temporal hint gains 5-15 % on 16-bit K/V and on e4m3 rows of a whole line when the keys are not split,
-// and loses where neighbouring workgroups share lines (64-byte rows) and on split e4m3 calls.
-template <typename T, int D, bool KV8, int NQ, int U>
+// Merges the chunks of a packed batch's rows: a workgroup of D threads per (sequence, head), a thread one element of each row.
+template <typename T, int D>
+__global__ void __launch_bounds__(D) fewrows_combine_kernel(const FwdParams p) {
+  const int bh = blockIdx.x, b = bh / p.H, h = bh - b * p.H, d = threadIdx.x;
+  const int q_row0 = p.cu_q[b], keys = p.cu_k[b + 1] - p.cu_k[b];
+  int nq = p.cu_q[b + 1] - q_row0;
+  nq = nq < p.Sq ? nq : p.Sq;
+  if (keys <= 0) return;  // (written by chunk 0)
+  const int have = (keys - 1) / p.Sk + 1, n = have < p.P ? have : p.P;
+  const float vmul = p.k_scale ? p.v_scale[bh] : 1.f;
+  for (int i = 0; i < nq; ++i) {
+    const int64_t at = ((int64_t)bh * p.Sq + i) * p.P;
+    const float* const part = (const float*)p.part + at * D + d;
+    const f32x2* const ml = (const f32x2*)((const float*)p.part + part_stats(gridDim.x, p.Sq, p.P, D)) + at;
+    float mx = ml[0][0];
+    for (int j = 1; j < n; ++j) mx = fmaxf(mx, ml[j][0]);
+    float a = 0.f, l = 0.f;
+    for (int j = 0; j < n; ++j) {
+      const float f = __builtin_amdgcn_exp2f(ml[j][0] - mx);
+      a += part[(int64_t)j * D] * f;
+      l += ml[j][1] * f;
+    }
+    ((T*)p.out)[h * p.os.h + (int64_t)(q_row0 + i) * p.os.s + d] = (T)(a * vmul / l);
+    if (d == 0) p.lse[(int64_t)h * p.lse_bh + q_row0 + i] = (mx + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
+  }
+}
+
+// Loads in flight and the non-temporal hint, measured on twelve decode shapes: four loads beat eight (6-10 %) except with three rows
+// and with single heads of 64-byte rows; the hint gains 5-15 % on 16-bit K/V, on e4m3 rows of a whole line when the keys are not split, and
+// on e4m3 heads taken together (12 % split), and loses where workgroups share lines (64-byte rows) and on split calls of single e4m3 heads.
+template <typename T, int D, bool KV8, int NQ, int U, int HP>
 hipError_t launch_variant(const FwdParams& p, hipStream_t stream) {
-  const dim3 grid((unsigned)(p.B * p.H), (unsigned)p.P), block(kWaves * 64);
-  if constexpr (!KV8) {
-    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, true>), grid, block, 0, stream, p);
-  } else if constexpr (D == 64) {
-    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, false>), grid, block, 0, stream, p);
+  const dim3 grid((unsigned)(p.B * p.H / HP), (unsigned)p.P), block(kWaves * 64);
+  constexpr bool hint = !KV8 || HP > 1;
+  if constexpr (hint || D == 64) {
+    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, hint, HP>), grid, block, 0, stream, p);
   } else if (p.P == 1) {
-    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, true>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, true, HP>), grid, block, 0, stream, p);
   } else {
-    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, false, HP>), grid, block, 0, stream, p);
   }
   return hipGetLastError();
 }
 
+// A head's piece of a key row is 64 to 256 bytes.  Where neighbouring heads lie side by side (the [rows, H, D] layouts) a workgroup takes
+// as many as make 256 bytes: 128-byte requests 4 KiB apart reach 5.1 TB/s, 256-byte ones 6.0 (64 caches of 1 to 4 thousand tokens, H = 32,
+// D = 128, e4m3: 256 -> 221 us; fixed length, B = 16, 4096 keys: e4m3 97 -> 85, bf16 D = 64 95 -> 80).  Not where that leaves CUs without
+// a workgroup: with one per CU and single heads 44 us, 48 together (B = 1, 32768 keys, e4m3, D = 128).
 // A launch that leaves half of the CUs without a workgroup (a caller who did not split the keys) is bound by what its
 // few waves keep in flight: eight loads there too.
 template <typename T, int D, bool KV8, int NQ>
 hipError_t launch_unroll(const FwdParams& p, hipStream_t stream) {
+  constexpr int HP = 256 / (D * (KV8 ? 1 : 2));
+  const int64_t groups = (int64_t)p.B * p.H * p.P;
+  if constexpr (HP > 1) {
+    if (p.H % HP == 0 && p.ks.h == D && p.vs.h == D && groups / HP >= spa_device_cus())
+      return launch_variant<T, D, KV8, NQ, NQ == 3 ? 8 : 4, HP>(p, stream);
+  }
   constexpr int U = NQ == 3 || (KV8 && D == 64) ? 8 : 4;
   if constexpr (U != 8) {
-    if ((int64_t)p.B * p.H * p.P * 2 <= spa_device_cus()) return launch_variant<T, D, KV8, NQ, 8>(p, stream);
+    if (groups * 2 <= spa_device_cus()) return launch_variant<T, D, KV8, NQ, 8, 1>(p, stream);
   }
-  return launch_variant<T, D, KV8, NQ, U>(p, stream);
+  return launch_variant<T, D, KV8, NQ, U, 1>(p, stream);
 }
 
 template <typename T, int D, bool KV8>
@@ -296,11 +348,18 @@ hipError_t launch_nq(const FwdParams& p, hipStream_t stream) {
   }
 }
 
+template <typename T, int D>
+hipError_t launch_d(const FwdParams& p, hipStream_t stream) {
+  const hipError_t e = p.k_scale ? launch_nq<T, D, true>(p, stream) : launch_nq<T, D, false>(p, stream);
+  if (e != hipSuccess || !p.cu_q || p.P == 1) return e;
+  hipLaunchKernelGGL((fewrows_combine_kernel<T, D>), dim3((unsigned)(p.B * p.H)), dim3(D), 0, stream, p);
+  return hipGetLastError();
+}
+
 template <typename T>
 hipError_t launch_t(const FwdParams& p, int D, hipStream_t stream) {
-  const bool kv8 = p.k_scale != nullptr;
-  if (D == 128) return kv8 ? launch_nq<T, 128, true>(p, stream) : launch_nq<T, 128, false>(p, stream);
-  if (D == 64) return kv8 ? launch_nq<T, 64, true>(p, stream) : launch_nq<T, 64, false>(p, stream);
+  if (D == 128) return launch_d<T, 128>(p, stream);
+  if (D == 64) return launch_d<T, 64>(p, stream);
   return hipErrorInvalidValue;
 }
 
@@ -308,11 +367,13 @@ hipError_t launch_t(const FwdParams& p, int D, hipStream_t stream) {
 
 // The caller's FwdParams as for the key-split launch: Sk = keys per chunk, sk_last = keys of the last chunk, P = number of
 // chunks; out / lse take rows z * Sq + i of chunk z.  No mask, 1 <= Sq <= 3, 16-bit q / out, K/V of one
-// (batch, head) below 2 GiB, 16-byte aligned K/V rows.  A packed variable-length batch (cu_q, cu_k; Sq = the longest
-// sequence's rows, B = sequences) runs as one chunk.
+// (batch, head) below 2 GiB, 16-byte aligned K/V rows.  A packed variable-length batch: cu_q, cu_k; Sq = the longest
+// sequence's rows, B = sequences; with P > 1 chunks of Sk keys and their sums in `part`.
 hipError_t spa_launch_fwd_fewrows(FwdParams p, int D, int dtype, hipStream_t stream) {
-  if (p.causal || (p.cu_q && p.P != 1) || p.q_scale || p.big || p.Sq < 1 || p.Sq > 3 || p.P < 1 || p.P > 65535) return hipErrorInvalidValue;
+  if (p.causal || (p.cu_q && p.P != 1 && !p.part) || p.q_scale || p.big || p.Sq < 1 || p.Sq > 3 || p.P < 1 || p.P > 65535) return hipErrorInvalidValue;
   if (dtype == 1) return launch_t<__bf16>(p, D, stream);
   if (dtype == 2) return launch_t<_Float16>(p, D, stream);
   return hipErrorInvalidValue;
 }
+
+int64_t spa_fewrows_part_floats(int64_t pairs, int nq, int n, int D) { return part_stats(pairs, nq, n, D) + pairs * nq * n * 2; }

@@ -19,6 +19,7 @@ static __device__ __align__(256) unsigned char scratch[SPA_STATIC_SCRATCH_BYTES]
 hipError_t spa_launch_flash_fwd(FwdParams p, int D, int dtype, hipStream_t stream);
 hipError_t spa_launch_fwd16_splitkv(FwdParams p, int D, int dtype, hipStream_t stream);
 hipError_t spa_launch_fwd_fewrows(FwdParams p, int D, int dtype, hipStream_t stream);
+int64_t spa_fewrows_part_floats(int64_t pairs, int nq, int n, int D);
 hipError_t spa_launch_splitkv_combine(void* out, float* lse, const void* part, const float* part_lse, int n, int B, int H, int Sq,
                                       int D, Strides3 os, int64_t lse_bh, int dtype, hipStream_t stream);
 hipError_t spa_launch_flash_bwd(BwdParams p, int D, int dtype, hipStream_t stream);
@@ -840,12 +841,19 @@ int varlen_sizes_ok(const char* what, const void* cu_q, const void* cu_k, int ns
 }  // extern "C"
 
 namespace {
+// Chunks per sequence of a packed batch: enough for the longest, but no more than twice the mean sequence's and two (max_sk may be a
+// bound that no sequence is near); the last takes what is left.
+int varlen_chunks(int nseq, int total_k, int max_sk, int chunk) {
+  const int64_t longest = ((int64_t)max_sk - 1) / chunk + 1, mean = (int64_t)total_k / nseq / chunk + 1;
+  return (int)(longest < 2 * mean + 2 ? longest : 2 * mean + 2);
+}
+
 int flash_fwd_varlen(const char* what, const void* q, const void* k, const void* v, const float* k_scale,
                      const float* v_scale, void* out, float* lse, const int32_t* cu_seqlens_q,
                      const int32_t* cu_seqlens_k, int nseq, int H, int total_q, int total_k, int max_sq, int max_sk,
                      int D, const int64_t q_strides[2], const int64_t k_strides[2], const int64_t v_strides[2],
                      const int64_t o_strides[2], float scale, int mask_mode, int dtype, void* stream, int P = 1, int rank = -1,
-                     int fuse = SPA_RING_PER_RANK) {
+                     int fuse = SPA_RING_PER_RANK, int chunk = 0, void* workspace = nullptr) {
   // P > 1: a ring over the packed batch.  The tensors are P stacked shards of total_q = total_k rows, every shard
   // packed as cu_seqlens_q says; rank r (or every rank, -1) walks the shards in ring order, one launch per rank or one for all.
   const bool kv8 = k_scale || v_scale;
@@ -893,10 +901,17 @@ int flash_fwd_varlen(const char* what, const void* q, const void* k, const void*
   p.cu_q = cu_seqlens_q; p.cu_k = cu_seqlens_k;
   p.k_scale = k_scale; p.v_scale = v_scale;
   // Sequences of up to kFewRows query rows without a mask (a decode step of a batch with ragged caches): the kernel that
-  // streams each sequence's K and V past its rows, as in flash_fwd above.
+  // streams each sequence's K and V past its rows, as in flash_fwd above; with chunk > 0 in chunks of that many keys.
   if (P == 1 && !p.causal && dtype != SPA_F32 && D != 32 && !p.big && max_sq <= kFewRows && spa_knob(SPA_KNOB_FEW_ROWS) != 1 &&
       (!kv8 || (aligned16v(k, k_strides, 1) && aligned16v(v, v_strides, 1)))) {
     p.sk_last = max_sk;
+    if (chunk > 0 && chunk < max_sk) {
+      if (!workspace || ((uintptr_t)workspace & 15) != 0) return fail(SPA_EINVAL, "%s: the key split needs a 16-byte aligned workspace", what);
+      p.P = varlen_chunks(nseq, total_k, max_sk, chunk);
+      if (p.P > 65535 || (int64_t)p.P * chunk > 0x7fffffffLL) return fail(SPA_EINVAL, "%s: grid too large", what);
+      p.Sk = chunk;
+      p.part = workspace;
+    }
     return launch_result(spa_launch_fwd_fewrows(p, D, dtype, (hipStream_t)stream), what);
   }
   if (P > 1) {
@@ -1027,6 +1042,36 @@ int flash_bwd_varlen(const char* what, const void* q, const void* k, const void*
 }  // namespace
 
 extern "C" {
+
+int64_t spa_flash_fwd_varlen_splitkv_workspace_bytes(int nseq, int H, int total_k, int max_sq, int max_sk, int D, int chunk) {
+  if (nseq <= 0 || H <= 0 || total_k <= 0 || max_sq <= 0 || max_sq > kFewRows || max_sk <= 0 || D <= 0 || chunk <= 0) return -1;
+  return 4 * spa_fewrows_part_floats((int64_t)nseq * H, max_sq, varlen_chunks(nseq, total_k, max_sk, chunk), D);
+}
+
+// Fewer workgroups than CUs: chunks that give every CU one, of at least 256 keys (8 caches of 2 to 8 thousand tokens, H = 8, bf16, D = 128:
+// 91 -> 36 us; up to 1024 tokens 14.8 -> 10.4).  More: whole sequences until the longest keeps its workgroup busy for 25 us (1.1 MB
+// of K and V, whatever the type: heads are taken together, launch_unroll), since the second kernel costs 3 to 5 us; then chunks of
+// 1024 keys (64 caches of 1 to 4 thousand tokens, H = 32: bf16 437 -> 413 us; 2 to 8 thousand, H = 8, e4m3 145 -> 122; 512 and 2048
+// are 1 to 4 % slower).
+int spa_flash_fwd_varlen_splitkv_suggest(int nseq, int H, int total_k, int max_sq, int max_sk, int D, int dtype) {
+  if (nseq <= 0 || H <= 0 || total_k <= 0 || max_sq <= 0 || max_sq > kFewRows || max_sk <= 0 || (D != 64 && D != 128) ||
+      (dtype != SPA_BF16 && dtype != SPA_F16) || spa_knob(SPA_KNOB_FEW_ROWS) == 1)
+    return 0;
+  const int64_t cus = spa_device_cus();
+  if ((int64_t)nseq * H >= cus) return max_sk > 2200 ? 1024 : 0;
+  const int64_t even = (int64_t)total_k * H / cus, chunk = even <= 256 ? 256 : (even + 255) / 256 * 256;
+  return max_sk >= chunk * 3 / 2 ? (int)chunk : 0;
+}
+
+int spa_flash_fwd_varlen_splitkv(const void* q, const void* k, const void* v, const float* k_scale, const float* v_scale, void* out, float* lse,
+                                 void* workspace, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int nseq, int H, int total_q,
+                                 int total_k, int max_sq, int max_sk, int D, int chunk, const int64_t q_strides[2], const int64_t k_strides[2],
+                                 const int64_t v_strides[2], const int64_t o_strides[2], float scale, int dtype, void* stream) {
+  if (chunk < 1) return fail(SPA_EINVAL, "spa_flash_fwd_varlen_splitkv: chunk must be positive");
+  return flash_fwd_varlen("spa_flash_fwd_varlen_splitkv", q, k, v, k_scale, v_scale, out, lse, cu_seqlens_q, cu_seqlens_k, nseq, H, total_q,
+                          total_k, max_sq, max_sk, D, q_strides, k_strides, v_strides, o_strides, scale, SPA_MASK_NONE, dtype, stream, 1, -1,
+                          SPA_RING_PER_RANK, chunk, workspace);
+}
 
 int spa_flash_fwd_varlen(const void* q, const void* k, const void* v, void* out, float* lse,
                          const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int nseq, int H, int total_q,

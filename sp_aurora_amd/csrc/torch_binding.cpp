@@ -197,6 +197,17 @@ bool varlen_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor&
     return spa_attention_fwd_varlen(a.p, b.p, c.p, o.p, lp, cq, nseq, a.H, a.S / shards, (int)max_q, a.D, a.st, b.st, c.st, o.st, &rows, scale, mask,
                                     dtype, stream) == SPA_OK;
   }
+  // few query rows: the keys in chunks, as in flash_fwd (a call that the split entry does not take runs whole)
+  const int chunk = causal ? 0 : spa_flash_fwd_varlen_splitkv_suggest(nseq, a.H, b.S, (int)max_q, (int)max_k, a.D, dtype);
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (chunk > 0 && hipStreamIsCapturing((hipStream_t)stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+    const Tensor ws = at::empty({spa_flash_fwd_varlen_splitkv_workspace_bytes(nseq, a.H, b.S, (int)max_q, (int)max_k, a.D, chunk)},
+                                q.options().dtype(at::kByte));
+    if (spa_flash_fwd_varlen_splitkv(a.p, b.p, c.p, kv8 ? (const float*)k_scale.const_data_ptr() : nullptr,
+                                     kv8 ? (const float*)v_scale.const_data_ptr() : nullptr, o.p, lp, ws.data_ptr(), cq, ck, nseq, a.H, a.S, b.S,
+                                     (int)max_q, (int)max_k, a.D, chunk, a.st, b.st, c.st, o.st, scale, dtype, stream) == SPA_OK)
+      return true;
+  }
   if (kv8)
     return spa_flash_fwd_varlen_fp8kv(a.p, b.p, c.p, (const float*)k_scale.const_data_ptr(), (const float*)v_scale.const_data_ptr(), o.p, lp, cq, ck,
                                       nseq, a.H, a.S, b.S, (int)max_q, (int)max_k, a.D, a.st, b.st, c.st, o.st, scale, mask, dtype, stream) == SPA_OK;

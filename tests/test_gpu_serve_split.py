@@ -1,0 +1,108 @@
+"""Decode over ragged caches with the keys cut into chunks, and with neighbouring heads taken together: chunk edges, sequences without rows or
+keys, a longest sequence past the last chunk's even share, strides under which heads cannot be taken together; against the kernels that
+do neither (spa_tune few_rows)."""
+import pytest
+import torch
+
+from conftest import rand_qkv
+from sp_aurora_amd import _lib, ops
+from test_gpu_parity import DEV
+
+pytestmark = pytest.mark.gpu
+# both sides round P or the result to the type: as test_gpu_parity's bounds against the oracle, once per side
+TOL = {torch.bfloat16: 2e-2, torch.float16: 4e-3}
+
+
+def caches(lens, H, D, dtype, fp8, seed):
+    q, = rand_qkv((max(1, sum(n for _, n in lens)), H, D), seed, dtype, n=1)
+    k, v = rand_qkv((max(1, sum(n for n, _ in lens)), H, D), seed + 1, dtype, n=2)
+    cu = lambda x: torch.tensor([0] + torch.tensor(x).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    scales = {}
+    if fp8:
+        scales = {n: torch.rand(len(lens), H, device=DEV) * 0.01 + 0.01 for n in ("k_scale", "v_scale")}
+        k, v = ((t.float() * 40).clamp(-448, 448).to(torch.float8_e4m3fn) for t in (k, v))
+    return q.to(DEV), k.to(DEV), v.to(DEV), cu([n for _, n in lens]), cu([n for n, _ in lens]), scales
+
+
+def split(q, k, v, cu_q, cu_k, max_q, max_k, chunk, k_scale=None, v_scale=None):
+    lib, (T, H, D), nseq = _lib.load(), q.shape, cu_q.numel() - 1
+    out, lse = torch.full_like(q, float("nan")), torch.full((H, T), float("nan"), device=DEV)
+    n = lib.spa_flash_fwd_varlen_splitkv_workspace_bytes(nseq, H, k.shape[0], max_q, max_k, D, chunk)
+    ws = torch.full((n,), 255, dtype=torch.uint8, device=DEV)
+    st = lambda t: _lib.strides2((t.stride(1), t.stride(0)))
+    scale = lambda t: 0 if t is None else t.data_ptr()
+    _lib.check(lib.spa_flash_fwd_varlen_splitkv(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), scale(k_scale), scale(v_scale), out.data_ptr(), lse.data_ptr(), ws.data_ptr(), cu_q.data_ptr(),
+        cu_k.data_ptr(), nseq, H, T, k.shape[0], max_q, max_k, D, chunk, st(q), st(k), st(v), st(out), D ** -0.5,
+        _lib.SPA_BF16 if q.dtype == torch.bfloat16 else _lib.SPA_F16, torch.cuda.current_stream().cuda_stream))
+    return out, lse
+
+
+def reference(*args, **kw):
+    _lib.tune("few_rows", 1)
+    try:
+        return ops.flash_fwd_varlen(*args, **kw)
+    finally:
+        _lib.tune("few_rows", 0)
+
+
+def check(got, want, dtype):
+    torch.testing.assert_close(got[0], want[0], atol=TOL[dtype], rtol=TOL[dtype])
+    torch.testing.assert_close(got[1], want[1], atol=1e-3, rtol=1e-5)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("chunk", [1, 64, 257, 512])
+@pytest.mark.parametrize("H,reps", [(3, 1), (4, 1), (4, 30)])
+def test_chunks_of_ragged_caches(H, reps, chunk, D, dtype, fp8):
+    # (keys, rows): around the chunk's length, without keys, without rows, one far longer than the mean
+    lens = [(chunk, 1), (chunk + 1, 2), (0, 1), (7, 0), (max(1, chunk - 1), 3), (5 * chunk + 3, 1), (2 * chunk, 2)] * reps + [(2000, 1)]
+    q, k, v, cu_q, cu_k, scales = caches(lens, H, D, dtype, fp8, 1000 + chunk)
+    max_k = max(n for n, _ in lens)
+    want = reference(q, k, v, cu_q, cu_k, 3, max_k, **scales)
+    check(split(q, k, v, cu_q, cu_k, 3, max_k, chunk, **scales), want, dtype)
+    check(ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 3, max_k, **scales), want, dtype)  # (not split: heads together where there are enough)
+
+
+@pytest.mark.parametrize("nseq,longest", [(3, 900), (70, 2300)])
+def test_suggested_chunks_and_capture(nseq, longest):
+    H, D, dtype = 4, 128, torch.bfloat16
+    lens = [(1 + (i * 997) % 700, 1) for i in range(nseq - 1)] + [(longest, 1)]
+    q, k, v, cu_q, cu_k, _ = caches(lens, H, D, dtype, False, 1100)
+    assert _lib.load().spa_flash_fwd_varlen_splitkv_suggest(nseq, H, k.shape[0], 1, longest, D, _lib.SPA_BF16) > 0
+    want = reference(q, k, v, cu_q, cu_k, 1, longest)
+    check(ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 1, longest), want, dtype)
+    check(ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 1, k.shape[0]), want, dtype)  # a bound that no sequence is near
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        res = ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 1, longest)
+    for _ in range(3):
+        res[0].fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        check(res, want, dtype)
+
+
+@pytest.mark.parametrize("D,fp8", [(64, False), (64, True), (128, True)])
+@pytest.mark.parametrize("rows", [1, 2, 3])
+def test_heads_taken_together_at_a_fixed_length(rows, D, fp8):
+    B, H, S, dtype = 65, 16, 193, torch.bfloat16
+    q, = rand_qkv((B, rows, H, D), 1200, dtype, n=1)
+    k, v = rand_qkv((B, S, H, D), 1201, dtype, n=2)
+    q, k, v = q.to(DEV), k.to(DEV), v.to(DEV)
+    scales = {}
+    if fp8:
+        (k, ks), (v, vs) = (ops.quantize_fp8_per_head(t, layout="bshd") for t in (k, v))
+        scales = {"k_scale": ks, "v_scale": vs}
+    apart = lambda t: t.transpose(1, 2).contiguous().transpose(1, 2)  # heads before rows: not side by side
+    got = ops.flash_fwd(q, k, v, layout="bshd", **scales)
+    single = ops.flash_fwd(q, apart(k), apart(v), layout="bshd", **scales)
+    mixed = ops.flash_fwd(q, k, apart(v), layout="bshd", **scales)
+    _lib.tune("few_rows", 1)
+    try:
+        want = ops.flash_fwd(q, k, v, layout="bshd", **scales)
+    finally:
+        _lib.tune("few_rows", 0)
+    for x in (got, single, mixed):
+        check(x, want, dtype)
