@@ -682,7 +682,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     // maxima, an exchange with the other half and a comparison saved of ~190 vector instructions a sub-tile): a score that
     // outgrows m by more than 2^8 shows in the sum, and so does a row that has seen no key yet (m = -inf: infinite or not a
     // number).  Until then P <= 256, harmless in fp32 sums and 16-bit operands.
-    float lp;
+    float lp = INFINITY;
     auto exponentials = [&](float mc) {
       float ps[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -699,7 +699,10 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
         }
       lp = (ps[0] + ps[1]) + (ps[2] + ps[3]);
     };
-    exponentials(m_run * c);
+    // A first sub-tile's are in vain, which is looked at where that is cheap beside what a short row pays: blocks of 667 rows at D = 64 132 ->
+    // 130 us for eight; at D = 128 the look costs long rows 0.7 %.
+    constexpr bool kLook = D <= 64;
+    if (!kLook || __builtin_amdgcn_ballot_w64(m_run == -INFINITY) == 0) exponentials(m_run * c);
     if (__builtin_amdgcn_ballot_w64(!(lp <= 256.f)) != 0) {
       // row max of the lane's 16 NT scores: 3-input maxima, two independent chains per 32-key tile.
       // (Through the instruction itself: fmaxf() makes the compiler quiet possible signalling NaNs
