@@ -935,8 +935,13 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
 // accumulation, P and dS stay fp32).  Correctness path for fp32 inputs: tiles of 32 rows staged
 // through registers, no software pipeline.  The contraction index of the gradient products is the
 // row an accumulator register holds (8*(v/4) + 4*hh + v%4), so P and dS are used where they are.
+// Bound: the chain of a wave, 192 (dq) or 256 (dk / dv) matrix instructions of 64 clocks per tile at D = 128, while the grid is small.
+// SHARED: a workgroup owns 32 rows (keys) and its four waves take every fourth tile, each through LDS of its own (the next
+// tile waits in registers, no barrier in the loop), and their sums are combined through LDS at the end: a quarter of the chain.
+// Backward, causal: [1, 288, 16, 128] 172 -> 79 us, [1, 1000, 12, 64] 318 -> 108, [1, 2048, 16, 128] 1081 -> 690.
 // ------------------------------------------------------------------------------------------
 constexpr int B32_ROWS = 32;
+constexpr int B32_WAVES = BWD_THREADS / 64;
 
 template <int D>
 struct Bwd32Cfg {
@@ -945,22 +950,23 @@ struct Bwd32Cfg {
   static constexpr int STAT = 2 * B32_ROWS;        // lse * log2 e and delta of a query tile
   static constexpr int SMEM_DQ = 2 * 2 * TILE * 4;
   static constexpr int SMEM_DKV = 2 * (2 * TILE + STAT) * 4;
+  static constexpr int SMEM_SHARED = B32_WAVES * (2 * TILE + STAT) * 4;  // a pair of tiles per wave; later its sums, 64 D floats
   static constexpr int CPR = D / 4;
-  static constexpr int RPP = BWD_THREADS / CPR;
-  static constexpr int PASS = (B32_ROWS + RPP - 1) / RPP;
 };
 
-// two row-major tiles of 32 rows (a, b) of tensors with the same row count, staged together
-template <int D>
+// two row-major tiles of 32 rows (a, b) of tensors with the same row count, staged together by THREADS threads
+template <int D, int THREADS>
 struct PairStage {
   typedef Bwd32Cfg<D> C;
-  f32x4 ra[C::PASS], rb[C::PASS];
+  static constexpr int RPP = THREADS / C::CPR;
+  static constexpr int PASS = (B32_ROWS + RPP - 1) / RPP;
+  f32x4 ra[PASS], rb[PASS];
   template <typename Row>
   __device__ __forceinline__ void gload(const float* a, int64_t as, const float* b, int64_t bs, int row0, int nrows, int tid, Row&& row_of) {
     const int cc = tid % C::CPR, cr = tid / C::CPR;
 #pragma unroll
-    for (int i = 0; i < C::PASS; ++i) {
-      const int lr = cr + i * C::RPP;
+    for (int i = 0; i < PASS; ++i) {
+      const int lr = cr + i * RPP;
       if (lr < B32_ROWS) {
         int r = row0 + lr;
         r = row_of(r < nrows ? r : nrows - 1);
@@ -972,8 +978,8 @@ struct PairStage {
   __device__ __forceinline__ void lstore(float* ta, float* tb, int tid) const {
     const int cc = tid % C::CPR, cr = tid / C::CPR;
 #pragma unroll
-    for (int i = 0; i < C::PASS; ++i) {
-      const int lr = cr + i * C::RPP;
+    for (int i = 0; i < PASS; ++i) {
+      const int lr = cr + i * RPP;
       if (lr < B32_ROWS) {
         *(f32x4*)(ta + lr * C::PITCH + cc * 4) = ra[i];
         *(f32x4*)(tb + lr * C::PITCH + cc * 4) = rb[i];
@@ -982,19 +988,37 @@ struct PairStage {
   }
 };
 
-template <int D>
+// SHARED: a wave's tile goes from registers to the wave's own LDS; its lanes' earlier reads come before, their later ones after.
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+// The sums of block db, over the waves' records of `floats` floats each.
+__device__ __forceinline__ f32x16 sum_records(const float* sm, int floats, int db, int lane) {
+  f32x16 x;
+  zero16(x);
+#pragma unroll
+  for (int j = 0; j < B32_WAVES; ++j)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) x[v] += sm[j * floats + (db * 16 + v) * 64 + lane];
+  return x;
+}
+
+template <int D, bool SHARED>
 __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dq_kernel(const BwdParams pk) {
   BwdParams p = pk;  // a variable-length batch rewrites the sizes and bases for its sequence below
   typedef Bwd32Cfg<D> C;
   extern __shared__ __align__(16) unsigned char smem[];
   float* sm = (float*)smem;
+  constexpr int ROWS = SHARED ? 32 : 128;
   const int tid = threadIdx.x;
-  const int lane = tid & 63, w = tid >> 6, ln = lane & 31, hh = lane >> 5;
+  const int lane = tid & 63, ln = lane & 31, hh = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int b, h, qt;
-  if (!workgroup_tile(p, true, 128, lane, b, h, qt)) return;
-  const int q0 = qt * 128;
-  const int qw0 = q0 + w * 32;
+  if (!workgroup_tile(p, true, ROWS, lane, b, h, qt)) return;
+  const int q0 = qt * ROWS;
+  const int qw0 = SHARED ? q0 : q0 + w * 32;
   RowMap map = {};
   select_sequence<float>(p, b, map);
   auto row_of = [&](int r) { return p.map.P ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
@@ -1032,32 +1056,40 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dq_kernel(const Bw
       for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(x[e], dof[g][e], sum);
     }
     dl = halves_sum(sum);
-    if (hh == 0 && qrow < p.Sq) p.delta[li] = dl;
+    if (hh == 0 && qrow < p.Sq && (!SHARED || w == 0)) p.delta[li] = dl;
   } else {
     dl = p.delta[li];
   }
   const float c = p.scale_log2;
   const int lim = p.causal ? (qrow < p.Sk - 1 ? qrow : p.Sk - 1) : p.Sk - 1;  // last visible key
 
-  const int kv_end = p.causal ? (q0 + 128 < p.Sk ? q0 + 128 : p.Sk) : p.Sk;
+  const int kv_end = p.causal ? (q0 + ROWS < p.Sk ? q0 + ROWS : p.Sk) : p.Sk;
   const int nt = (kv_end + B32_ROWS - 1) / B32_ROWS;
 
   f32x16 dq[D / 32];
 #pragma unroll
   for (int i = 0; i < D / 32; ++i) zero16(dq[i]);
 
-  PairStage<D> st;
-  st.gload(kp, p.ks.s, vp, p.vs.s, 0, p.Sk, tid, row_of);
-  st.lstore(sm, sm + C::TILE, tid);
-  __syncthreads();
+  constexpr int STEP = SHARED ? B32_WAVES : 1, RECORD = 2 * C::TILE + C::STAT;
+  const int st_id = SHARED ? lane : tid, first = SHARED ? w : 0;
+  float* const own = sm + w * RECORD;  // (SHARED)
+  PairStage<D, SHARED ? 64 : BWD_THREADS> st;
+  if (first < nt) {
+    st.gload(kp, p.ks.s, vp, p.vs.s, first * B32_ROWS, p.Sk, st_id, row_of);
+    st.lstore(SHARED ? own : sm, (SHARED ? own : sm) + C::TILE, st_id);
+  }
+  if (SHARED)
+    wave_fence();
+  else
+    __syncthreads();
 
-  for (int it = 0; it < nt; ++it) {
+  for (int it = first; it < nt; it += STEP) {
     const int cur = it & 1;
     const int key0 = it * B32_ROWS;
-    const bool more = it + 1 < nt;
-    if (more) st.gload(kp, p.ks.s, vp, p.vs.s, key0 + B32_ROWS, p.Sk, tid, row_of);
+    const bool more = it + STEP < nt;
+    if (more) st.gload(kp, p.ks.s, vp, p.vs.s, key0 + STEP * B32_ROWS, p.Sk, st_id, row_of);
     if (!(p.causal && key0 > qw0 + 31)) {
-      const float* kb = sm + cur * 2 * C::TILE;
+      const float* kb = SHARED ? own : sm + cur * 2 * C::TILE;
       const float* vb = kb + C::TILE;
       f32x16 s, dp;
       zero16(s);
@@ -1086,39 +1118,61 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dq_kernel(const Bw
           dq[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(kb[kl * C::PITCH + db * 32 + ln], s[v], dq[db], 0, 0, 0);
       }
     }
-    if (more) st.lstore(sm + (cur ^ 1) * 2 * C::TILE, sm + (cur ^ 1) * 2 * C::TILE + C::TILE, tid);
-    __syncthreads();
+    if constexpr (SHARED) {
+      wave_fence();
+      if (more) st.lstore(own, own + C::TILE, st_id);
+      wave_fence();
+    } else {
+      if (more) st.lstore(sm + (cur ^ 1) * 2 * C::TILE, sm + (cur ^ 1) * 2 * C::TILE + C::TILE, tid);
+      __syncthreads();
+    }
+    if (SHARED && !more) mfma_settle();
   }
 
-  if (qrow < p.Sq) {
-    float* dqp = p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)row_of(qrow) * p.dqs.s;
+  float* const dqp = p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)row_of(qrow_c) * p.dqs.s;
+  auto store = [&](int db, const f32x16& sum) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4* dst = (f32x4*)(dqp + db * 32 + 8 * g + 4 * hh);
+      f32x4 x = {0.f, 0.f, 0.f, 0.f};
+      if (!p.grads_in_t) x = *dst;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] += sum[4 * g + e] * p.scale;
+      *dst = x;
+    }
+  };
+  if constexpr (SHARED) {
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        f32x4* dst = (f32x4*)(dqp + db * 32 + 8 * g + 4 * hh);
-        f32x4 x = {0.f, 0.f, 0.f, 0.f};
-        if (!p.grads_in_t) x = *dst;
+      for (int v = 0; v < 16; ++v) own[(db * 16 + v) * 64 + lane] = dq[db][v];
+    __syncthreads();
+    for (int db = w; db < D / 32; db += B32_WAVES) {
+      const f32x16 sum = sum_records(sm, RECORD, db, lane);
+      if (qrow < p.Sq) store(db, sum);
+    }
+  } else if (qrow < p.Sq) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] += dq[db][4 * g + e] * p.scale;
-        *dst = x;
-      }
+    for (int db = 0; db < D / 32; ++db) store(db, dq[db]);
   }
 }
 
-template <int D>
+
+template <int D, bool SHARED>
 __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const BwdParams pk) {
   BwdParams p = pk;  // a variable-length batch rewrites the sizes and bases for its sequence below
   typedef Bwd32Cfg<D> C;
   extern __shared__ __align__(16) unsigned char smem[];
   float* sm = (float*)smem;
+  constexpr int ROWS = SHARED ? 32 : 128;
   const int tid = threadIdx.x;
-  const int lane = tid & 63, w = tid >> 6, ln = lane & 31, hh = lane >> 5;
+  const int lane = tid & 63, ln = lane & 31, hh = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int b, h, kt;
-  if (!workgroup_tile(p, false, 128, lane, b, h, kt)) return;
-  const int k0 = kt * 128;
-  const int kw0 = k0 + w * 32;
+  if (!workgroup_tile(p, false, ROWS, lane, b, h, kt)) return;
+  const int k0 = kt * ROWS;
+  const int kw0 = SHARED ? k0 : k0 + w * 32;
   RowMap map = {};
   select_sequence<float>(p, b, map);
   auto row_of = [&](int r) { return p.map.P ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
@@ -1159,37 +1213,45 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
     zero16(dv[i]);
   }
 
-  PairStage<D> st;
+  constexpr int STEP = SHARED ? B32_WAVES : 1;
+  const int st_id = SHARED ? lane : tid, first = SHARED ? it0 + w : it0;
+  PairStage<D, SHARED ? 64 : BWD_THREADS> st;
   float st_l = 0.f, st_d = 0.f;
+  constexpr bool LATE = SHARED && D == 128;  // no registers left for the next pair of tiles: loaded when its place is free
   auto gload = [&](int it) {
-    st.gload(qp, p.qs.s, dop, p.dos.s, it * B32_ROWS, p.Sq, tid, row_of);
-    if (tid < B32_ROWS) {
-      int r = it * B32_ROWS + tid;
+    if (!LATE) st.gload(qp, p.qs.s, dop, p.dos.s, it * B32_ROWS, p.Sq, st_id, row_of);
+    if (st_id < B32_ROWS) {
+      int r = it * B32_ROWS + st_id;
       r = r < p.Sq ? r : p.Sq - 1;
       st_l = lsep[stat_of(r)] * 1.4426950408889634f;
       st_d = delp[stat_of(r)];
     }
   };
-  auto lstore = [&](int stage) {
+  auto lstore = [&](int stage, int it) {
     float* sb = sm + stage * STAGE;
-    st.lstore(sb, sb + C::TILE, tid);
-    if (tid < B32_ROWS) {
-      sb[2 * C::TILE + tid] = st_l;
-      sb[2 * C::TILE + B32_ROWS + tid] = st_d;
+    if (LATE) st.gload(qp, p.qs.s, dop, p.dos.s, it * B32_ROWS, p.Sq, st_id, row_of);
+    st.lstore(sb, sb + C::TILE, st_id);
+    if (st_id < B32_ROWS) {
+      sb[2 * C::TILE + st_id] = st_l;
+      sb[2 * C::TILE + B32_ROWS + st_id] = st_d;
     }
   };
 
-  if (it0 < nt) {
-    gload(it0);
-    lstore(it0 & 1);
+  // (stage: SHARED, the wave's own; else two in turn)
+  if (first < nt) {
+    gload(first);
+    lstore(SHARED ? w : first & 1, first);
   }
-  __syncthreads();
+  if (SHARED)
+    wave_fence();
+  else
+    __syncthreads();
 
-  for (int it = it0; it < nt; ++it) {
-    const int cur = it & 1;
+  for (int it = first; it < nt; it += STEP) {
+    const int cur = SHARED ? w : it & 1;
     const int r0 = it * B32_ROWS;
-    const bool more = it + 1 < nt;
-    if (more) gload(it + 1);
+    const bool more = it + STEP < nt;
+    if (more) gload(it + STEP);
     if (!(p.causal && r0 + B32_ROWS - 1 < kw0)) {
       const float* qb = sm + cur * STAGE;
       const float* dob = qb + C::TILE;
@@ -1226,45 +1288,51 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
         }
       }
     }
-    if (more) lstore(cur ^ 1);
-    __syncthreads();
+    if constexpr (SHARED) {
+      wave_fence();
+      if (more) lstore(w, it + STEP);
+      wave_fence();
+    } else {
+      if (more) lstore(cur ^ 1, it + 1);
+      __syncthreads();
+    }
     if (!more) mfma_settle();
   }
 
-  if (krow < p.Sk && p.grads_in_t) {
-    float* dkp = p.dk + b * p.dks.b + h * p.dks.h + (int64_t)row_of(krow) * p.dks.s;
-    float* dvp = p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)row_of(krow) * p.dvs.s;
+  float* const dkp = p.dk + b * p.dks.b + h * p.dks.h + (int64_t)row_of(krow_c) * p.dks.s;
+  float* const dvp = p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)row_of(krow_c) * p.dvs.s;
+  auto store = [&](float* to, int db, const f32x16& sum, float scale) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4* dst = (f32x4*)(to + db * 32 + 8 * g + 4 * hh);
+      f32x4 x = {0.f, 0.f, 0.f, 0.f};
+      if (!p.grads_in_t) x = *dst;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] += sum[4 * g + e] * scale;
+      *dst = x;
+    }
+  };
+  if constexpr (SHARED) {
+    float* const own = sm + w * STAGE;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        f32x4 x, y;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[e] = dk[db][4 * g + e] * p.scale;
-          y[e] = dv[db][4 * g + e];
-        }
-        *(f32x4*)(dkp + db * 32 + 8 * g + 4 * hh) = x;
-        *(f32x4*)(dvp + db * 32 + 8 * g + 4 * hh) = y;
+      for (int v = 0; v < 16; ++v) {
+        own[(db * 16 + v) * 64 + lane] = dk[db][v];
+        own[((D / 32 + db) * 16 + v) * 64 + lane] = dv[db][v];
       }
+    __syncthreads();
+    for (int n = w; n < 2 * (D / 32); n += B32_WAVES) {
+      const f32x16 sum = sum_records(sm, STAGE, n, lane);
+      const bool is_v = n >= D / 32;
+      if (krow < p.Sk) store(is_v ? dvp : dkp, is_v ? n - D / 32 : n, sum, is_v ? 1.f : p.scale);
+    }
   } else if (krow < p.Sk) {
-    float* dkp = p.dk + b * p.dks.b + h * p.dks.h + (int64_t)row_of(krow) * p.dks.s;
-    float* dvp = p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)row_of(krow) * p.dvs.s;
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        f32x4* d1 = (f32x4*)(dkp + db * 32 + 8 * g + 4 * hh);
-        f32x4* d2 = (f32x4*)(dvp + db * 32 + 8 * g + 4 * hh);
-        f32x4 x = *d1, y = *d2;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[e] += dk[db][4 * g + e] * p.scale;
-          y[e] += dv[db][4 * g + e];
-        }
-        *d1 = x;
-        *d2 = y;
-      }
+    for (int db = 0; db < D / 32; ++db) {
+      store(dkp, db, dk[db], p.scale);
+      store(dvp, db, dv[db], 1.f);
+    }
   }
 }
 
@@ -1333,6 +1401,30 @@ hipError_t spa_launch_bwd16_other(const BwdParams& p, int D, int dtype, hipStrea
 #else
 hipError_t spa_launch_bwd16_other(const BwdParams& p, int D, int dtype, hipStream_t stream);
 
+// fp32: whether the waves of a workgroup share out the tiles (SHARED).  A launch lasts as long as its longest chain of tiles or as the
+// work of all SIMDs, whichever is more; sharing quarters the chain, and costs the workgroup's sums and, where all SIMDs are busy, 6 to 16 %
+// ([1, 2048, 32, 128] causal 1178 us, shared 1366).  Of 14 launches of 128 to 2048 rows the rule takes the faster form in each.
+bool tiles_shared(const BwdParams& p) {
+  const int knob = spa_knob(SPA_KNOB_FWD32_SPLIT);
+  if (p.Sq > 65535 * B32_ROWS || p.Sk > 65535 * B32_ROWS) return false;
+  if (knob) return knob == 2;
+  const double rows = (p.Sq + 31) / 32, keys = (p.Sk + 31) / 32;
+  const double all = p.cu_q ? (double)p.H * (p.lse_bh / 32 + p.B) : (double)p.B * p.H * rows;  // row tiles of the launch
+  const double chain = p.causal && rows < keys ? rows : keys, work = all * (p.causal ? chain / 2 : chain) / (4 * spa_device_cus());
+  const double shared = chain / B32_WAVES > 1.2 * work ? chain / B32_WAVES : 1.2 * work;
+  return shared + 0.5 < (chain > work ? chain : work);
+}
+template <int D>
+hipError_t launch32(const BwdParams& p, hipStream_t stream) {
+  typedef Bwd32Cfg<D> C;
+  if (tiles_shared(p)) {
+    const hipError_t e = launch<flash_bwd32_dq_kernel<D, true>>(C::SMEM_SHARED, true, 32, p, stream);
+    return e != hipSuccess ? e : launch<flash_bwd32_dkdv_kernel<D, true>>(C::SMEM_SHARED, false, 32, p, stream);
+  }
+  const hipError_t e = launch<flash_bwd32_dq_kernel<D, false>>(C::SMEM_DQ, true, 128, p, stream);
+  return e != hipSuccess ? e : launch<flash_bwd32_dkdv_kernel<D, false>>(C::SMEM_DKV, false, 128, p, stream);
+}
+
 // Returns hipSuccess, or hipErrorInvalidValue for an unsupported (dtype, D).
 hipError_t spa_launch_flash_bwd(BwdParams p, int D, int dtype, hipStream_t stream) {
   if ((p.big || p.map.P) && dtype != 0) return spa_launch_bwd16_other(p, D, dtype, stream);
@@ -1345,14 +1437,9 @@ hipError_t spa_launch_flash_bwd(BwdParams p, int D, int dtype, hipStream_t strea
     if (D == 64) return launch_both<_Float16, 64>(p, stream);
     if (D == 32) return launch_both<_Float16, 32>(p, stream);
   } else if (dtype == 0) {
-    hipError_t e = hipErrorInvalidValue;
-    if (D == 128) e = launch<flash_bwd32_dq_kernel<128>>(Bwd32Cfg<128>::SMEM_DQ, true, 128, p, stream);
-    if (D == 64) e = launch<flash_bwd32_dq_kernel<64>>(Bwd32Cfg<64>::SMEM_DQ, true, 128, p, stream);
-    if (D == 32) e = launch<flash_bwd32_dq_kernel<32>>(Bwd32Cfg<32>::SMEM_DQ, true, 128, p, stream);
-    if (e != hipSuccess) return e;
-    if (D == 128) return launch<flash_bwd32_dkdv_kernel<128>>(Bwd32Cfg<128>::SMEM_DKV, false, 128, p, stream);
-    if (D == 64) return launch<flash_bwd32_dkdv_kernel<64>>(Bwd32Cfg<64>::SMEM_DKV, false, 128, p, stream);
-    if (D == 32) return launch<flash_bwd32_dkdv_kernel<32>>(Bwd32Cfg<32>::SMEM_DKV, false, 128, p, stream);
+    if (D == 128) return launch32<128>(p, stream);
+    if (D == 64) return launch32<64>(p, stream);
+    if (D == 32) return launch32<32>(p, stream);
   }
   return hipErrorInvalidValue;
 }
