@@ -313,6 +313,7 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
     ctx->saved_data["causal"] = causal;
     ctx->saved_data["zigzag"] = zigzag;
     ctx->mark_non_differentiable({r[1]});
+    ctx->set_materialize_grads(false);  // (the lse has none: a fill of 2 to 5 us a pass)
     return r;
   }
   template <typename... Args>
@@ -334,6 +335,7 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
     const Tensor &q = saved[0], &out = saved[N], &lse = saved[N + 1];
     void* const stream = current_stream();
     const c10::DeviceGuard guard(q.device());
+    if (!grads[0].defined()) grads[0] = at::zeros(out.sizes(), out.options());
     View o, d;
     spa_shards rows;
     const spa_shards* shards;
@@ -387,6 +389,7 @@ struct VarlenAttention : public torch::autograd::Function<VarlenAttention> {
     ctx->saved_data["shards"] = shards;
     ctx->saved_data["zigzag"] = zigzag;
     ctx->mark_non_differentiable({lse});
+    ctx->set_materialize_grads(false);
     return {out, lse};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -395,6 +398,7 @@ struct VarlenAttention : public torch::autograd::Function<VarlenAttention> {
     const Tensor &q = s[0], &out = s[3], &lse = s[4];
     void* const stream = current_stream();
     const c10::DeviceGuard guard(q.device());
+    if (!grads[0].defined()) grads[0] = at::zeros(out.sizes(), out.options());
     View a, b, c, d, g[3];
     const Tensor dout = rows_ok(grads[0]) && view_thd(grads[0], d) && !rows_shared(d, 1) ? grads[0] : grads[0].contiguous();
     TORCH_CHECK(view_thd(q, a) && view_thd(s[1], b) && view_thd(s[2], c) && lse.is_contiguous() && cu_ok(s[5], q) && cu_ok(s[6], q),

@@ -149,3 +149,24 @@ def test_strides_of_operands_and_gradients(D, dtype):
                     grads.append(torch.autograd.grad(spa.sp_aurora_varlen_func(*leaves, cu, max_seqlen=S, causal=True), leaves, d))
                 for g, w in zip(*grads):
                     assert torch.equal(g, w)
+
+
+def test_a_gradient_that_never_comes_is_zero():
+    class NoGrad(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    leaves = _leaves(740)
+    out = spa.sp_aurora_func(*leaves, causal=True)
+    for g in torch.autograd.grad(NoGrad.apply(out).float().sum() + sum(t.sum() * 0 for t in leaves), leaves):
+        assert not g.any()
+    cu = torch.tensor([0, 40, 80], dtype=torch.int32, device=DEV)
+    packed = [t.detach().reshape(80, 2, 64).requires_grad_() for t in leaves]
+    out = spa.sp_aurora_varlen_func(*packed, cu, max_seqlen=40, causal=True)
+    for g in torch.autograd.grad(NoGrad.apply(out).float().sum() + sum(t.sum() * 0 for t in packed), packed):
+        assert not g.any()
