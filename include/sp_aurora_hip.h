@@ -547,7 +547,7 @@ int spa_attention_bwd_varlen(const void* q, const void* k, const void* v, const 
  *   SPA_TUNE_BWD_DQ_WAVES  4 | 8   waves per workgroup of the backward's dq kernel
  *   SPA_TUNE_BWD_DKDV_FORM 1       compiler-scheduled MFMAs in the D = 128 dk/dv kernel
  *   SPA_TUNE_FWD32_SPLIT  1 | 2    never / always: the fp32 kernels with 32-row workgroups whose waves share
- *                                  the key tiles (the library takes it when 128-row workgroups would leave half the CUs idle)
+ *                                  the tiles (the library takes them where the longest chain of tiles decides)
  *   SPA_TUNE_FEW_ROWS     1        a key-split forward of up to 4 query rows runs on the MFMA kernels instead of the
  *                                  kernel that streams K and V past those rows
  */
