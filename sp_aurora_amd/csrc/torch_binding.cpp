@@ -46,12 +46,12 @@ bool rows_ok(const Tensor& t, int64_t bytes = 16) {
   return true;
 }
 
-// One operand as the C ABI takes it: pointer, (batch, head, seq) strides in elements, sizes.  pitch: rows from one shard to the
-// next where a sequence's rows lie in shards, 0 where they follow each other.
+// One operand as the C ABI takes it: pointer, (batch, head, seq) strides in elements, sizes.  shards: of a rank-stacked tensor;
+// pitch: rows from one shard to the next where a sequence's rows lie in shards, 0 where they follow each other.
 struct View {
   void* p = nullptr;
   int64_t st[3] = {0, 0, 0};
-  int B = 0, H = 0, S = 0, D = 0, pitch = 0;
+  int B = 0, H = 0, S = 0, D = 0, shards = 1, pitch = 0;
   bool same_shape(const View& o) const { return B == o.B && H == o.H && S == o.S && D == o.D; }
 };
 
@@ -74,6 +74,7 @@ bool view_of(const Tensor& t, bool bshd, View& v, int part = -1) {
     if (!bshd || sz[0] * sz[2] > 0x7fffffffLL || st[2] <= 0) return false;
     v.B = (int)sz[1]; v.S = (int)(sz[0] * sz[2]); v.H = (int)sz[3]; v.D = (int)sz[4];
     v.st[0] = st[1]; v.st[1] = st[3]; v.st[2] = st[2];
+    v.shards = (int)sz[0];
     if (sz[0] > 1 && st[0] != sz[2] * st[2]) {
       if (st[0] % st[2] != 0 || st[0] / st[2] < sz[2] || st[0] / st[2] > 0x7fffffffLL) return false;
       v.pitch = (int)(st[0] / st[2]);
@@ -233,15 +234,18 @@ bool differentiable_ok(const Tensor* t, int n) {
     if (!on_device(t[i], t[0]) || t[i].scalar_type() != t[0].scalar_type() || t[i].dim() < 3 || !rows_ok(t[i])) return false;
   return true;
 }
-// Where the rows lie: false when the operands do not agree.  zigzag: shards of a zigzag-sharded [B,S,H,D] ring, 0 = none.
-bool rows_of(const Tensor& first, const View& q, const View& k, const View& v, int64_t zigzag, spa_shards& rows, const spa_shards*& arg) {
+// Rows from one shard to the next in a compact tensor of the operand's shape (0: they follow each other), as results and gradients are.
+int compact_pitch(const View& v) { return v.shards > 1 && v.B > 1 ? v.B * (v.S / v.shards) : 0; }
+
+// Where the rows lie: false when the operands do not agree among each other or with compact results (rank-stacked tensors that are a
+// view of [B,S,H,D]: their rows follow each other, those of the results do not).  zigzag: shards of a zigzag-sharded [B,S,H,D]
+// ring, 0 = none.
+bool rows_of(const View& q, const View& k, const View& v, int64_t zigzag, spa_shards& rows, const spa_shards*& arg) {
   arg = nullptr;
-  if (q.pitch != k.pitch || q.pitch != v.pitch) return false;
+  if (q.pitch != k.pitch || q.pitch != v.pitch || q.pitch != compact_pitch(q)) return false;
   if (q.pitch) {
-    const int P = (int)first.size(0);
     if (zigzag || k.S != q.S) return false;
-    if (q.pitch != q.B * (q.S / P)) return false;  // (the results and gradients are compact)
-    rows = {P, q.pitch, q.S / P, 0};
+    rows = {q.shards, q.pitch, q.S / q.shards, 0};
     arg = &rows;
   } else if (zigzag) {
     if (zigzag < 1 || k.S != q.S || q.S % (2 * zigzag) != 0) return false;
@@ -260,7 +264,7 @@ bool attention_ok(const Tensor* t, int n, int64_t zigzag) {
   if (n == 3 && (t[0].dim() != t[1].dim() || t[0].dim() != t[2].dim() || (t[0].dim() == 5 && t[0].sizes() != t[1].sizes()))) return false;
   if (rows_shared(o.q, 2)) return false;
   if (!o.k.same_shape(o.v) || o.q.B != o.k.B || o.q.H != o.k.H || o.q.D != o.k.D || (o.q.D != 32 && o.q.D != 64 && o.q.D != 128)) return false;
-  if (!rows_of(t[0], o.q, o.k, o.v, zigzag, rows, arg)) return false;
+  if (!rows_of(o.q, o.k, o.v, zigzag, rows, arg)) return false;
   if (!arg) return true;
   // (what the kernels for rows in shards do not take: 2 GiB and more per (batch, head))
   const int64_t span = (int64_t)(rows.shards - 1) * rows.pitch + o.q.S / rows.shards, esz = t[0].element_size();
@@ -295,7 +299,7 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
     const spa_shards* shards;
     const float scale = softmax_scale_or_default(scale_or_nan, x.q.D);
     const int mask = causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype = dtype_code(q.scalar_type());
-    rows_of(q, x.q, x.k, x.v, zigzag, rows, shards);
+    rows_of(x.q, x.k, x.v, zigzag, rows, shards);
     if (shards)
       check(spa_attention_fwd(x.q.p, x.k.p, x.v.p, o.p, (float*)lse.data_ptr(), x.q.B, x.q.H, x.q.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, shards, scale,
                               mask, dtype, stream));
@@ -339,7 +343,7 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
     View o, d;
     spa_shards rows;
     const spa_shards* shards;
-    TORCH_CHECK(operands(saved.data(), N, x) && rows_of(q, x.q, x.k, x.v, ctx->saved_data["zigzag"].toInt(), rows, shards) &&
+    TORCH_CHECK(operands(saved.data(), N, x) && rows_of(x.q, x.k, x.v, ctx->saved_data["zigzag"].toInt(), rows, shards) &&
                     view_of(out, true, o) && o.same_shape(x.q) && o.pitch == x.q.pitch && lse.is_contiguous(),
                 "saved tensors came back in another layout");
     const Tensor dout = rows_ok(grads[0]) && view_of(grads[0], true, d) && d.pitch == o.pitch && !rows_shared(d, 2) ? grads[0] : grads[0].contiguous();
