@@ -510,7 +510,7 @@ int spa_flash_bwd_varlen(const void* q, const void* k, const void* v, const void
  * spa_flash_bwd_varlen for the whole gradient in one call, as spa_flash_bwd_out is to spa_flash_bwd:
  * dq [total_q, H, D], dk / dv [total_k, H, D] have the inputs' element type and are WRITTEN (zeros
  * where a sequence has queries but no keys, or keys that no query sees).  Rows that belong to no
- * sequence are left untouched.  Same
+ * sequence are left untouched, and rows past max_sq / max_sk of a longer sequence may be.  Same
  * call site as spa_flash_bwd_varlen (test_intel_ring_flash_attn_varlen.py:85-91).
  */
 int spa_flash_bwd_varlen_out(const void* q, const void* k, const void* v, const void* dout,

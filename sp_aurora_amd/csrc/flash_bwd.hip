@@ -268,11 +268,11 @@ __device__ __forceinline__ void select_sequence(BwdParams& p, int& b, RowMap& ma
 }
 
 // The (batch or sequence, head) and the tile (of `rows` query rows, or keys) of a workgroup: pairs first, in groups
-// (spa_head_groups), or, for a packed batch, heads first and then the tiles of all sequences (sequence_tile).  The tiles that
-// see the most of the other side go first: with a causal mask the last query tiles and the first key tiles.
+// (spa_head_groups), or, for a packed batch with a numbered grid, heads first and then the tiles of all sequences (sequence_tile).  The
+// tiles that see the most of the other side go first: with a causal mask the last query tiles and the first key tiles.
 __device__ __forceinline__ bool workgroup_tile(const BwdParams& p, bool queries, int rows, int lane, int& b, int& h, int& tile) {
   int n;
-  if (p.cu_q) {
+  if (p.numbered) {
     const int number = blockIdx.x / p.H;
     h = blockIdx.x - number * p.H;
     if (!sequence_tile(queries ? p.cu_q : p.cu_k, p.B, p.map.P ? p.map.P : 1, rows, number, lane, b, tile, n)) return false;
@@ -1338,12 +1338,13 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
 
 // `rows` query rows, or keys, per workgroup.
 template <auto kernel>
-hipError_t launch(int smem, bool queries, int rows, const BwdParams& p, hipStream_t stream, int threads = BWD_THREADS) {
+hipError_t launch(int smem, bool queries, int rows, BwdParams p, hipStream_t stream, int threads = BWD_THREADS) {
   const hipError_t e = spa_allow_dynamic_lds<kernel>(smem);
   if (e != hipSuccess) return e;
   dim3 grid;
   if (p.cu_q) {
-    if (!spa_varlen_grid(p.H, p.B, queries ? p.lse_bh : p.total_k, rows, 1, grid)) return hipErrorInvalidValue;
+    const int64_t longest = (int64_t)(queries ? p.Sq : p.Sk) * (p.map.P ? p.map.P : 1);
+    if (!spa_varlen_grid(p.H, p.B, queries ? p.lse_bh : p.total_k, longest, rows, 1, grid, p.numbered)) return hipErrorInvalidValue;
   } else {
     const int tiles = ((queries ? p.Sq : p.Sk) + rows - 1) / rows;
     if (tiles > 65535) return hipErrorInvalidValue;

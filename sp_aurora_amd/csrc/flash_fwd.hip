@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   // (grid.x = (batch, head) pairs, grid.y = query tiles, grid.z = ranks, or, for one rank, groups of pairs
   // (spa_head_groups): workgroups are dispatched x first, and the decomposition costs no divisions)
   int b, h, qt;
-  if (p.cu_q) {
+  if (p.numbered) {
     // a packed batch: heads first, then the tiles of all sequences (sequence_tile), each sequence's heaviest first
     const int number = blockIdx.x / p.H;
     h = blockIdx.x - number * p.H;
@@ -209,6 +209,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     map.init(p.map, shard_rows);
     p.Sq = p.Sk = shard_rows * p.map.P;
   }
+  if (p.cu_q && q0 >= p.Sq) return;  // a tile of the longest sequence that this one does not have
   const int q_lim = zz && !zhalf ? zz_hs : p.Sq;  // one past the last row this workgroup may own
   const int qw0 = q0 + (SHARE ? grp * FWD_BM : 0) + w * 32;
   const int64_t qoff = (int64_t)rank * (VR ? p.rank_rows : p.Sq);  // first row of this rank's query chunk
@@ -1175,14 +1176,14 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
 
 // `rows`: query rows per workgroup.
 template <auto kernel>
-hipError_t launch(int threads, int smem, int rows, const FwdParams& p, hipStream_t stream) {
+hipError_t launch(int threads, int smem, int rows, FwdParams p, hipStream_t stream) {
   const hipError_t e = spa_allow_dynamic_lds<kernel>(smem);
   if (e != hipSuccess) return e;
   if (p.nqt > 65535 || p.nranks > 65535) return hipErrorInvalidValue;
   const int64_t pairs = (int64_t)p.B * p.H;
   dim3 grid;
   if (p.cu_q) {
-    if (!spa_varlen_grid(p.H, p.B, p.lse_bh / p.P, rows, (unsigned)p.nranks, grid)) return hipErrorInvalidValue;
+    if (!spa_varlen_grid(p.H, p.B, p.lse_bh / p.P, p.Sq, rows, (unsigned)p.nranks, grid, p.numbered)) return hipErrorInvalidValue;
   } else {
     grid = p.nranks == 1 ? spa_head_groups(pairs, p.nqt) : dim3((unsigned)pairs, (unsigned)p.nqt, (unsigned)p.nranks);
   }

@@ -214,7 +214,7 @@ __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_ker
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int b, h, qt;
-  if (p.cu_q) {
+  if (p.numbered) {
     const int number = blockIdx.x / p.H;
     h = blockIdx.x - number * p.H;
     int nt = 0;
@@ -254,6 +254,7 @@ __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_ker
     map.init(p.map, p.cu_q ? p.Sq : p.Sq / p.map.P);
     if (p.cu_q) p.Sq = p.Sk = p.Sq * p.map.P;
   }
+  if (p.cu_q && q0 >= p.Sq) return;  // a tile of the longest sequence that this one does not have
   auto row_of = [&](int r) { return p.map.P ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
   auto stat_of = [&](int r) { return p.map.P ? map.at(r, p.map.lse_pitch) : r; };   // in lse
 
@@ -625,12 +626,12 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
 }
 
 template <auto kernel>
-hipError_t launch(int threads, int smem, int rows, const FwdParams& p, hipStream_t stream) {
+hipError_t launch(int threads, int smem, int rows, FwdParams p, hipStream_t stream) {
   const hipError_t e = spa_allow_dynamic_lds<kernel>(smem);
   if (e != hipSuccess) return e;
   dim3 grid;
   if (p.cu_q) {
-    if (!spa_varlen_grid(p.H, p.B, p.lse_bh, rows, 1, grid)) return hipErrorInvalidValue;
+    if (!spa_varlen_grid(p.H, p.B, p.lse_bh, p.Sq, rows, 1, grid, p.numbered)) return hipErrorInvalidValue;
   } else {
     if (p.nqt > 65535) return hipErrorInvalidValue;
     grid = spa_head_groups((int64_t)p.B * p.H, p.nqt);

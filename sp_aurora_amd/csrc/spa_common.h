@@ -54,6 +54,7 @@ struct FwdParams {
   // Sq and Sk are the longest sequence's sizes (they shape the grid) and lse is [H][lse_bh]
   const int* cu_q;
   const int* cu_k;
+  int numbered = 0;  // cu_q: the grid counts the tiles of all sequences (sequence_tile); 0: sequences x tiles of the longest
   // e4m3 K/V (16-bit kernels; null: K and V have q's element type): K = k8 * k_scale[b*H + h],
   // V = v8 * v_scale[b*H + h], fp32, one per (batch or sequence, head); strides of k, v in bytes
   const float* k_scale;
@@ -131,6 +132,7 @@ struct BwdParams {
   const int* cu_q;
   const int* cu_k;
   int total_k = 0;  // rows of the packed key-side tensors (total_q is lse_bh)
+  int numbered = 0; // as in FwdParams
   // the forward's result: the dq kernel forms delta = rowsum(dout * out) from it and writes it for the dk / dv kernel; null:
   // delta is the caller's and is read
   const void* out = nullptr;
@@ -254,37 +256,68 @@ struct RowMap {
 };
 
 // ---- variable-length batches ----
-// Which tile of which sequence a workgroup takes.  The tiles (of `rows` rows) of all sequences are numbered back to back,
-// sequence by sequence, so a grid of (total rows / rows + sequences) numbers covers any batch and at most one workgroup
-// per sequence finds nothing to do (a grid of sequences x longest sequence spends a third of its workgroups on rows that
-// do not exist, and each takes a CU from one with work).  Blocks of 64 sequences in the order given, longest first inside a
-// block: the heavy tiles start first, and the tiles of one sequence run side by side and share its K / V in L2.
+// Sum over the 64 lanes of a wave, in every lane.
+static __device__ __forceinline__ int wave_sum(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr 1, 2, 4, 8: lane 15 of a row of 16 has its sum
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast 15 into rows 1 and 3, 31 into rows 2 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
+// Which tile of which sequence a workgroup of a numbered grid (spa_varlen_grid) takes.  The tiles (of `rows` rows) of all sequences
+// are numbered back to back, sequence by sequence, so a grid of (total rows / rows + sequences) numbers covers any batch and at
+// most one workgroup per sequence finds nothing to do.  Blocks of 64 sequences in the order given, longest first inside a block: the
+// heavy tiles start first, and the tiles of one sequence run side by side and share its K / V in L2.  The search adds up the
+// blocks before the number's own, 512 sequences at a time, and orders that one block (a loop over all sequences took tens of microseconds
+// of every workgroup: 2000 sequences of 32 to 256 rows, forward, 15500 us, so 1920).
 // Every wave of the workgroup calls this (a lane holds one sequence of the block); false: no such tile.
 // times: the sequences are that many times as long as cu says (shards).
 static __device__ __forceinline__ bool sequence_tile(const int* cu, int nseq, int times, int rows, int number, int lane, int& seq, int& tile,
                                                      int& ntiles) {
-  for (int base = 0; base < nseq; base += 64) {
-    const int n = nseq - base < 64 ? nseq - base : 64;
-    const int i = base + (lane < n ? lane : 0);
-    const int len = lane < n ? (cu[i + 1] - cu[i]) * times : 0;
-    const int mine = (len + rows - 1) / rows;
-    int before = 0, total = 0;  // tiles of the sequences that come before this lane's, tiles of the block
-    for (int j = 0; j < n; ++j) {
-      const int lj = __builtin_amdgcn_readlane(len, j), tj = __builtin_amdgcn_readlane(mine, j);
-      before += lj > len || (lj == len && j < lane) ? tj : 0;
-      total += tj;
+  constexpr int AHEAD = 8;  // blocks whose offsets are loaded together
+  int base = 0;
+  if (nseq > 64) {
+    bool found = false;
+    for (; base < nseq && !found;) {
+      int tiles[AHEAD];
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) {
+        const int i = base + 64 * u + lane, at = i < nseq ? i : nseq - 1;
+        const int n = ((cu[at + 1] - cu[at]) * times + rows - 1) / rows;
+        tiles[u] = i < nseq ? n : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) {
+        if (found) break;
+        const int total = wave_sum(tiles[u]);
+        found = number < total;
+        if (!found) {
+          number -= total;
+          base += 64;
+        }
+      }
     }
-    if (number < total) {
-      const unsigned long long own = __builtin_amdgcn_ballot_w64(number >= before && number < before + mine);
-      const int owner = __builtin_amdgcn_readfirstlane(__builtin_ctzll(own));
-      seq = base + owner;
-      ntiles = __builtin_amdgcn_readlane(mine, owner);
-      tile = number - __builtin_amdgcn_readlane(before, owner);
-      return true;
-    }
-    number -= total;
+    if (!found) return false;
   }
-  return false;
+  const int n = nseq - base < 64 ? nseq - base : 64;
+  const int i = base + (lane < n ? lane : 0);
+  const int len = lane < n ? (cu[i + 1] - cu[i]) * times : 0;
+  const int mine = (len + rows - 1) / rows;
+  int before = 0;  // tiles of the block's sequences that come before this lane's
+  for (int j = 0; j < n; ++j) {
+    const int lj = __builtin_amdgcn_readlane(len, j), tj = __builtin_amdgcn_readlane(mine, j);
+    before += lj > len || (lj == len && j < lane) ? tj : 0;
+  }
+  const unsigned long long own = __builtin_amdgcn_ballot_w64(number >= before && number < before + mine);
+  if (own == 0) return false;
+  const int owner = __builtin_amdgcn_readfirstlane(__builtin_ctzll(own));
+  seq = base + owner;
+  ntiles = __builtin_amdgcn_readlane(mine, owner);
+  tile = number - __builtin_amdgcn_readlane(before, owner);
+  return true;
 }
 
 // ---- LDS helpers shared by the attention kernels ----

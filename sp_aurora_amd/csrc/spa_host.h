@@ -70,9 +70,23 @@ static inline dim3 spa_head_groups(int64_t pairs, int tiles) {
   return dim3((unsigned)group, (unsigned)tiles, (unsigned)n);
 }
 
-// Grid of a launch over a packed variable-length batch: one workgroup per head and tile number (sequence_tile), heads first.
-static inline bool spa_varlen_grid(int H, int nseq, int64_t total_rows, int rows, unsigned z, dim3& grid) {
-  const int64_t n = (total_rows / rows + nseq) * H;
+// Grid of a launch over a packed variable-length batch: sequences x tiles of the longest sequence, as for fixed lengths
+// (numbered = 0), or one workgroup per head and tile number, heads first (sequence_tile).  A workgroup of the first that finds no
+// rows costs 0.5 us of a CU; one of the second searches for 0.4 us (24 sequences) to 3 us (2000), but the tiles of a long sequence
+// run side by side and the heavy ones first.  So numbers where the mean sequence is long and the other grid has more workgroups (us, forward /
+// backward, H = 16, D = 128, causal: 24 sequences of 500 to 2000 rows 264 / 919, by sequences 278 / 1005; 64 of 200 to 2000 570 / 1977 and
+// 574 / 2129), by sequences for short ones (2000 of 32 to 256 rows 1083 / 4276, numbered 1918 / 7779; 200 of 100 to 1000, H = 8,
+// D = 64, 193 / 616 and 229 / 698) until a bound far above the lengths that are there makes that grid eight times the other (512 of
+// 32 to 256 rows with a bound of 2048 378 / 1463 and 407 / 1705, of 4096 506 / 1880).
+static inline bool spa_varlen_grid(int H, int nseq, int64_t total_rows, int64_t longest, int rows, unsigned z, dim3& grid, int& numbered) {
+  const int64_t tiles = (longest + rows - 1) / rows, numbers = total_rows / rows + nseq, pairs = (int64_t)nseq * H;
+  const bool short_rows = total_rows < (int64_t)nseq * 640;
+  numbered = tiles * nseq > (short_rows ? 8 : 1) * numbers || tiles > 65535 || pairs > 0x7fffffffLL;
+  if (!numbered) {
+    grid = z == 1 ? spa_head_groups(pairs, (int)tiles) : dim3((unsigned)pairs, (unsigned)tiles, z);
+    return true;
+  }
+  const int64_t n = numbers * H;
   if (n <= 0 || n > 0x7fffffffLL) return false;
   grid = dim3((unsigned)n, 1, z);
   return true;
