@@ -119,6 +119,28 @@ float softmax_scale_or_default(double scale, int D) { return (float)(std::isnan(
 Tensor empty_f32(at::IntArrayRef sizes, const Tensor& like) { return at::empty(sizes, like.options().dtype(at::kFloat)); }
 
 // ---------------------------------------------------------------- forward
+// One block call (ks, vs: e4m3 K / V).  Few query rows against many keys: the keys split over the grid, the chunks' results in a
+// workspace (not while the stream is being captured: the workspace would not outlive this call); a call that the split entries do not take
+// runs whole.
+int block_fwd(const View& q, const View& k, const View& v, const View& o, float* lse, const float* ks, const float* vs, float scale, int mask, int dtype,
+              const Tensor& like, void* stream) {
+  if (mask == SPA_MASK_NONE && dtype != SPA_F32 && (q.D == 64 || q.D == 128)) {
+    int n = spa_flash_fwd_splitkv_suggest(q.B, q.H, q.S, k.S, q.D, mask, dtype);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (n > 1 && (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)) n = 1;
+    if (n > 1) {
+      const Tensor ws = at::empty({spa_flash_fwd_splitkv_workspace_bytes(q.B, q.H, q.S, q.D, n, dtype)}, like.options().dtype(at::kByte));
+      const int rc =
+          ks ? spa_flash_fwd_splitkv_fp8kv(q.p, k.p, v.p, ks, vs, o.p, lse, ws.data_ptr(), q.B, q.H, q.S, k.S, q.D, n, q.st, k.st, v.st, o.st, scale,
+                                           dtype, stream)
+             : spa_flash_fwd_splitkv(q.p, k.p, v.p, o.p, lse, ws.data_ptr(), q.B, q.H, q.S, k.S, q.D, n, q.st, k.st, v.st, o.st, scale, dtype, stream);
+      if (rc == SPA_OK) return rc;
+    }
+  }
+  if (ks) return spa_flash_fwd_fp8kv(q.p, k.p, v.p, ks, vs, o.p, lse, q.B, q.H, q.S, k.S, q.D, q.st, k.st, v.st, o.st, scale, mask, dtype, stream);
+  return spa_flash_fwd(q.p, k.p, v.p, o.p, lse, q.B, q.H, q.S, k.S, q.D, q.st, k.st, v.st, o.st, scale, mask, dtype, stream);
+}
+
 // (out, lse) of one block call; false: not a call for this path.
 bool flash_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale_or_nan, bool causal, bool bshd, const Tensor& q_scale,
                const Tensor& k_scale, const Tensor& v_scale, int out_dtype, Tensor& out, Tensor& lse) {
@@ -146,23 +168,7 @@ bool flash_fwd(const Tensor& q, const Tensor& k, const Tensor& v, double scale_o
   if (q8)
     return spa_flash_fwd_fp8qkv(a.p, b.p, c.p, (const float*)q_scale.const_data_ptr(), ks, vs, o.p, lp, a.B, a.H, a.S, b.S, a.D, a.st, b.st, c.st,
                                 o.st, scale, mask, dtype, stream) == SPA_OK;
-  // few query rows against many keys: the keys split over the grid, the chunks' results in a workspace (not while the
-  // stream is being captured: the workspace would not outlive this call)
-  if (!causal && dtype != SPA_F32 && (a.D == 64 || a.D == 128)) {
-    int n = spa_flash_fwd_splitkv_suggest(a.B, a.H, a.S, b.S, a.D, mask, dtype);
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (n > 1 && (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)) n = 1;
-    if (n > 1) {
-      const Tensor ws = at::empty({spa_flash_fwd_splitkv_workspace_bytes(a.B, a.H, a.S, a.D, n, dtype)}, q.options().dtype(at::kByte));
-      return (kv8 ? spa_flash_fwd_splitkv_fp8kv(a.p, b.p, c.p, ks, vs, o.p, lp, ws.data_ptr(), a.B, a.H, a.S, b.S, a.D, n, a.st, b.st, c.st, o.st,
-                                                scale, dtype, stream)
-                  : spa_flash_fwd_splitkv(a.p, b.p, c.p, o.p, lp, ws.data_ptr(), a.B, a.H, a.S, b.S, a.D, n, a.st, b.st, c.st, o.st, scale, dtype,
-                                          stream)) == SPA_OK;
-    }
-  }
-  if (kv8)
-    return spa_flash_fwd_fp8kv(a.p, b.p, c.p, ks, vs, o.p, lp, a.B, a.H, a.S, b.S, a.D, a.st, b.st, c.st, o.st, scale, mask, dtype, stream) == SPA_OK;
-  return spa_flash_fwd(a.p, b.p, c.p, o.p, lp, a.B, a.H, a.S, b.S, a.D, a.st, b.st, c.st, o.st, scale, mask, dtype, stream) == SPA_OK;
+  return block_fwd(a, b, c, o, lp, ks, vs, scale, mask, dtype, q, stream) == SPA_OK;
 }
 
 bool cu_ok(const Tensor& cu, const Tensor& q) {
@@ -304,8 +310,7 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
       check(spa_attention_fwd(x.q.p, x.k.p, x.v.p, o.p, (float*)lse.data_ptr(), x.q.B, x.q.H, x.q.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, shards, scale,
                               mask, dtype, stream));
     else
-      check(spa_flash_fwd(x.q.p, x.k.p, x.v.p, o.p, (float*)lse.data_ptr(), x.q.B, x.q.H, x.q.S, x.k.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, scale, mask,
-                          dtype, stream));
+      check(block_fwd(x.q, x.k, x.v, o, (float*)lse.data_ptr(), nullptr, nullptr, scale, mask, dtype, q, stream));
     return {out, lse};
   }
   static variable_list save(AutogradContext* ctx, const Tensor* t, double scale, bool causal, int64_t zigzag) {

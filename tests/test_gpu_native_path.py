@@ -170,3 +170,28 @@ def test_a_gradient_that_never_comes_is_zero():
     out = spa.sp_aurora_varlen_func(*packed, cu, max_seqlen=40, causal=True)
     for g in torch.autograd.grad(NoGrad.apply(out).float().sum() + sum(t.sum() * 0 for t in packed), packed):
         assert not g.any()
+
+
+@pytest.mark.parametrize("B,Sq,Sk,H,D,dtype", [(1, 1, 4096, 4, 128, torch.bfloat16), (2, 3, 3000, 4, 64, torch.float16), (1, 40, 5000, 4, 128, torch.bfloat16)])
+def test_few_rows_of_a_differentiable_call_split_the_keys(B, Sq, Sk, H, D, dtype):
+    """The differentiable functions take the same route as the operator: the same bits, and with gradients the same result."""
+    q, = rand_qkv((B, Sq, H, D), 640, dtype, n=1)
+    k, v = rand_qkv((B, Sk, H, D), 641, dtype, n=2)
+    dout, = rand_qkv((B, Sq, H, D), 642, dtype, n=1)
+    want, want_lse = O.full_attention(q, k, v, None, False)
+    grads = O.attn_backward_autograd(q, k, v, dout, None, False)
+    x, y, z = (t.to(DEV) for t in (q, k, v))
+    op, op_lse = ops.flash_fwd(x, y, z, layout="bshd")
+    assert _lib.load().spa_flash_fwd_splitkv_suggest(B, H, Sq, Sk, D, _lib.SPA_MASK_NONE, ops._DT[dtype]) > 1
+    for fn in (lambda *t: spa.sp_aurora_func(*t), lambda a, b, c: spa.sp_aurora_kvpacked_func(a, torch.stack([b, c], 2)),
+               lambda *t: spa.ulysses_flash_attn_func(*t), lambda *t: spa.LongContextAttention()(*t)):
+        assert torch.equal(fn(x, y, z), op)
+        leaves = [t.detach().clone().requires_grad_() for t in (x, y, z)]
+        out = fn(*leaves)
+        assert torch.equal(out, op)
+        for name, g, w in zip("qkv", torch.autograd.grad(out, leaves, dout.to(DEV)), grads):
+            check_grad(g, w, dtype, "d" + name)
+    out, lse, _ = spa.sp_aurora_func(x, y, z, return_attn_probs=True)
+    assert torch.equal(lse, op_lse)
+    check_out(out, want, dtype)
+    check_lse(lse, want_lse)
