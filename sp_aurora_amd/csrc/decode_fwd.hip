@@ -252,10 +252,11 @@ __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParam
     float mx = sm_m[i][0][hd];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) mx = fmaxf(mx, sm_m[i][w][hd]);
+    const float ms = mx == -INFINITY ? 0.f : mx;   // (every score of the chunk -inf: nothing of weight, beside chunks that have some)
     float ls = 0.f, a = 0.f;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-      const float f = __builtin_amdgcn_exp2f(sm_m[i][w][hd] - mx);   // (every chunk holds a key: mx is finite)
+      const float f = __builtin_amdgcn_exp2f(sm_m[i][w][hd] - ms);
       ls += sm_l[i][w][hd] * f;
       a += sm_acc[i][w][hd * D + d] * f;
     }
@@ -289,9 +290,10 @@ __global__ void __launch_bounds__(D) fewrows_combine_kernel(const FwdParams p) {
     const f32x2* const ml = (const f32x2*)((const float*)p.part + part_stats(gridDim.x, p.Sq, p.P, D)) + at;
     float mx = ml[0][0];
     for (int j = 1; j < n; ++j) mx = fmaxf(mx, ml[j][0]);
+    const float ms = mx == -INFINITY ? 0.f : mx;
     float a = 0.f, l = 0.f;
     for (int j = 0; j < n; ++j) {
-      const float f = __builtin_amdgcn_exp2f(ml[j][0] - mx);
+      const float f = __builtin_amdgcn_exp2f(ml[j][0] - ms);
       a += part[(int64_t)j * D] * f;
       l += ml[j][1] * f;
     }

@@ -164,7 +164,8 @@ __global__ void __launch_bounds__(256) finalize_kernel(T* __restrict__ out, cons
 
 // Merge of the n block results a key-split forward left behind (rows j * Sq .. of `part`, [B, n * Sq, H, D] in T, and of
 // part_lse, [B, H, n * Sq]): update_out_and_lse (sp_aurora/utils.py:103-104) over all of them at once, as a running
-// (weighted sum, weight sum) relative to the largest lse so far.  All lse are finite (every chunk holds a key).
+// (weighted sum, weight sum) relative to the largest lse so far.  A chunk whose scores are all -inf (lse -inf, no result) has no weight.
+// Bound: the latency of its loads (a few rows, a few workgroups), so eight chunks are requested together.
 template <typename T>
 __global__ void __launch_bounds__(256) splitkv_combine_kernel(T* __restrict__ out, float* __restrict__ lse, const T* __restrict__ part,
                                                               const float* __restrict__ part_lse, int n, int H, int Sq, int D,
@@ -177,17 +178,34 @@ __global__ void __launch_bounds__(256) splitkv_combine_kernel(T* __restrict__ ou
   const int64_t prow = (int64_t)H * D;                                  // elements between rows of `part`
   const T* pp = part + ((int64_t)r.b * n * Sq + r.s) * prow + r.h * D + ch * 8;
   const float* pl = part_lse + ((int64_t)r.b * H + r.h) * ((int64_t)n * Sq) + r.s;
-  float x[8], xb[8], lb = pl[0], wsum = 1.f;
-  Load8<T>::ld(pp, x);
-  for (int j = 1; j < n; ++j) {
-    Load8<T>::ld(pp + (int64_t)j * Sq * prow, xb);
-    const float lj = pl[(int64_t)j * Sq];
-    const float mx = fmaxf(lb, lj);
-    const float wa = __expf(lb - mx), wb = __expf(lj - mx);
-    wsum = wsum * wa + wb;
-    lb = mx;
+  constexpr int NB = 8;
+  float x[8], lb = -INFINITY, wsum = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = x[i] * wa + xb[i] * wb;
+  for (int i = 0; i < 8; ++i) x[i] = 0.f;
+  for (int j0 = 0; j0 < n; j0 += NB) {
+    float xb[NB][8], l[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int j = j0 + u < n ? j0 + u : n - 1;
+      l[u] = pl[(int64_t)j * Sq];
+      Load8<T>::ld(pp + (int64_t)j * Sq * prow, xb[u]);
+    }
+    float mx = lb;
+#pragma unroll
+    for (int u = 0; u < NB; ++u) mx = fmaxf(mx, l[u]);
+    const float ms = mx == -INFINITY ? 0.f : mx, wa = __expf(lb - ms);
+    lb = mx;
+    wsum *= wa;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] *= wa;
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const bool none = j0 + u >= n || l[u] == -INFINITY;
+      const float w = none ? 0.f : __expf(l[u] - ms);
+      wsum += w;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf(none ? 0.f : xb[u][i], w, x[i]);
+    }
   }
   const float inv = 1.f / wsum;
 #pragma unroll

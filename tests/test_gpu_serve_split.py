@@ -106,3 +106,36 @@ def test_heads_taken_together_at_a_fixed_length(rows, D, fp8):
         _lib.tune("few_rows", 0)
     for x in (got, single, mixed):
         check(x, want, dtype)
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+def test_chunks_whose_keys_are_all_hidden(D, dtype):
+    """Keys hidden through the inputs (a head dim that is 1 in q and -inf in those keys): whole chunks without a finite score, first, last
+    and in between, beside chunks with some; against float64."""
+    H = 4
+    hide = [(300, 0, 130), (300, 60, 300), (200, 64, 128), (700, 0, 699)]  # (keys, the hidden ones)
+    lens = [(n, 2) for n, _, _ in hide]
+    q, k, v, cu_q, cu_k, _ = caches(lens, H, D, dtype, False, 1300)
+    q[..., 0], k[..., 0] = 1.0, 0.0
+    at, wants = 0, []
+    for i, (n, lo, hi) in enumerate(hide):
+        k[at + lo:at + hi, :, 0] = -float("inf")
+        s = torch.einsum("qhd,khd->hqk", q[2 * i:2 * i + 2].cpu().double(), k[at:at + n].cpu().double()) * D ** -0.5
+        out = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1), v[at:at + n].cpu().double())
+        wants.append((out, torch.logsumexp(s, -1)))
+        at += n
+    want = torch.cat([o for o, _ in wants]), torch.cat([l for _, l in wants], 1)
+    for got in (split(q, k, v, cu_q, cu_k, 2, 700, 64), ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 2, 700)):
+        check([t.cpu().double() for t in got], want, dtype)
+    # one length: the chunks' results merged by their lse
+    n = 4096
+    q, = rand_qkv((1, 2, H, D), 1301, dtype, n=1)
+    k, v = rand_qkv((1, n, H, D), 1302, dtype, n=2)
+    q[..., 0], k[..., 0] = 1.0, 0.0
+    for lo, hi in ((0, 1500), (1000, n), (600, 3000)):
+        kk = k.clone()
+        kk[:, lo:hi, :, 0] = -float("inf")
+        s = torch.einsum("bqhd,bkhd->bhqk", q.double(), kk.double()) * D ** -0.5
+        want = torch.einsum("bhqk,bkhd->bqhd", torch.softmax(s, -1), v.double()), torch.logsumexp(s, -1)
+        got = ops.flash_fwd(q.to(DEV), kk.to(DEV), v.to(DEV), layout="bshd")
+        check([t.cpu().double() for t in got], want, dtype)
