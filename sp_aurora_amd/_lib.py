@@ -6,6 +6,7 @@ fallback path: a missing library raises, it never degrades to torch ops.
 import ctypes
 import os
 import threading
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsp_aurora_hip.so")
@@ -140,12 +141,13 @@ def load():
     return lib
 
 
-_native = None
+_native = None  # the module, or False where it cannot be loaded
 
 
 def native():
     """The module behind the public calls' fast path (_native.so: torch tensors in, C ABI calls out, no interpreter in between), or
-    None on a thread that records (ops.prepared): there every call goes through load()'s recorder."""
+    None: on a thread that records (ops.prepared), where every call goes through load()'s recorder, and where the module is missing or
+    was built for another torch, which a warning says once; the Python functions behind it need the C library only."""
     global _native
     if getattr(_tls, "recorder", None) is not None:
         return None
@@ -154,9 +156,11 @@ def native():
         try:
             from . import _native as module
         except ImportError as e:
-            raise ImportError(f"{os.path.join(_HERE, '_native.so')}: {e}; build it with `python -m sp_aurora_amd.build`") from e
+            warnings.warn(f"{os.path.join(_HERE, '_native.so')}: {e}; calls go through Python, which costs up to 150 us each: "
+                          "build it with `python -m sp_aurora_amd.build`", RuntimeWarning, stacklevel=3)
+            module = False
         _native = module
-    return _native
+    return _native or None
 
 
 _STRIDE_CACHE = {}

@@ -303,3 +303,24 @@ def test_tensors_of_2_gib_and_more_per_head_pass_the_argument_checks():
     far = _s3(0, D, 8 << 20)
     assert lib.spa_flash_fwd(p, p, p, p, p, 1, 1, 1024, 1024, D, st, far, far, st, 1.0, 0, 1, None) == -2
     assert b"1 GiB" in lib.spa_last_error()
+
+
+def test_a_native_module_that_cannot_be_loaded_is_reported_once(monkeypatch):
+    """Missing, or built for another torch: the Python functions need the C library only."""
+    import sys
+    import warnings
+
+    import torch
+
+    import sp_aurora_amd as spa
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.delattr(spa, "_native", raising=False)
+    monkeypatch.setitem(sys.modules, "sp_aurora_amd._native", None)
+    with pytest.warns(RuntimeWarning, match="_native.so"):
+        assert _lib.native() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.native() is None
+        q = torch.zeros(1, 4, 2, 64)
+        with pytest.raises(ValueError, match="HIP device"):  # (what the Python path says to a CPU tensor)
+            spa.sp_aurora_func(q, q, q)

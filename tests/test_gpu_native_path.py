@@ -195,3 +195,27 @@ def test_few_rows_of_a_differentiable_call_split_the_keys(B, Sq, Sk, H, D, dtype
     assert torch.equal(lse, op_lse)
     check_out(out, want, dtype)
     check_lse(lse, want_lse)
+
+
+def test_every_function_works_without_the_native_module(monkeypatch):
+    q, k, v, dout = (t.to(DEV) for t in rand_qkv((2, 96, 4, 64), 650, torch.bfloat16, n=4))
+    cu = torch.tensor([0, 50, 192], dtype=torch.int32, device=DEV)
+    rows, stacked = lambda t: t.reshape(192, 4, 64), lambda t: t.view(2, 2, 48, 4, 64).transpose(0, 1).contiguous()
+    calls = [(lambda *t: spa.sp_aurora_func(*t, causal=True, ring_size=2), lambda t: t),
+             (lambda *t: spa.sp_aurora_func(*t, causal=True, ring_size=2, sharding="zigzag"), lambda t: t),
+             (lambda *t: spa.sp_aurora_varlen_func(*t, cu, max_seqlen=142, causal=True), rows),
+             (lambda *t: spa.ulysses_flash_attn_func(*t, causal=True), stacked),
+             (lambda *t: spa.LongContextAttention(sp_ulysses_degree=2, sp_ring_degree=1)(*t, causal=True), stacked)]
+    results = []
+    for module in (_lib.native(), False):
+        monkeypatch.setattr(_lib, "_native", module)
+        for fn, shape in calls:
+            leaves = [shape(t).detach().clone().requires_grad_() for t in (q, k, v)]
+            out = fn(*leaves)
+            results.append((out.detach(), *torch.autograd.grad(out, leaves, shape(dout))))
+        out, lse = ops.flash_fwd(q, k, v, None, True, layout="bshd")
+        acc = spa.update_out_and_lse(None, None, out.transpose(1, 2).contiguous(), lse)
+        results.append((out, lse, *spa.update_out_and_lse(*acc, out.transpose(1, 2).contiguous(), lse)))
+    for one, other in zip(results[:len(calls) + 1], results[len(calls) + 1:]):
+        for a, b in zip(one, other):  # (both round to bf16, at most once per ring step)
+            torch.testing.assert_close(a, b, atol=4e-2, rtol=2e-2)
