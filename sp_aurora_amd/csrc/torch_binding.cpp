@@ -5,7 +5,7 @@
 // functions here take the arguments that a well-formed call has - contiguous head dim, 16-byte aligned rows, one device, one
 // dtype - allocate the results and enqueue the kernels; the differentiable ones are C++ autograd nodes, whose backward runs on
 // the autograd thread without the interpreter.  For anything else (an argument that needs a copy, a check that fails,
-// an entry point that refuses) they return None, and the Python code behind them does the copy or raises the error.
+// a forward entry point that refuses) they return None, and the Python code behind them does the copy or raises the error.
 #include <Python.h>
 #include <hip/hip_runtime_api.h>
 
@@ -287,6 +287,12 @@ void to_kernel_rows(variable_list& saved, int n) {
 
 void check(int rc) { TORCH_CHECK(rc == SPA_OK, "[spa ", rc, "] ", spa_last_error()); }
 
+// A forward that an entry point refuses, thrown through the autograd node that is being made: the call is one for the Python path.
+struct Refused {};
+void accepted(bool yes) {
+  if (!yes) throw Refused();
+}
+
 // Block attention over whole sequences (every ring whose contiguous shards this GPU holds is that: the blocks of the ring
 // tile the score matrix).
 template <int N>
@@ -307,10 +313,10 @@ struct Attention : public torch::autograd::Function<Attention<N>> {
     const int mask = causal ? SPA_MASK_CAUSAL : SPA_MASK_NONE, dtype = dtype_code(q.scalar_type());
     rows_of(x.q, x.k, x.v, zigzag, rows, shards);
     if (shards)
-      check(spa_attention_fwd(x.q.p, x.k.p, x.v.p, o.p, (float*)lse.data_ptr(), x.q.B, x.q.H, x.q.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, shards, scale,
-                              mask, dtype, stream));
+      accepted(spa_attention_fwd(x.q.p, x.k.p, x.v.p, o.p, (float*)lse.data_ptr(), x.q.B, x.q.H, x.q.S, x.q.D, x.q.st, x.k.st, x.v.st, o.st, shards,
+                                 scale, mask, dtype, stream) == SPA_OK);
     else
-      check(block_fwd(x.q, x.k, x.v, o, (float*)lse.data_ptr(), nullptr, nullptr, scale, mask, dtype, q, stream));
+      accepted(block_fwd(x.q, x.k, x.v, o, (float*)lse.data_ptr(), nullptr, nullptr, scale, mask, dtype, q, stream) == SPA_OK);
     return {out, lse};
   }
   static variable_list save(AutogradContext* ctx, const Tensor* t, double scale, bool causal, int64_t zigzag) {
@@ -388,7 +394,7 @@ struct VarlenAttention : public torch::autograd::Function<VarlenAttention> {
   static variable_list forward(AutogradContext* ctx, Tensor q, Tensor k, Tensor v, Tensor cu_q, Tensor cu_k, int64_t max_q, int64_t max_k, double scale,
                                bool causal, bool covered, int64_t shards, bool zigzag) {
     Tensor out, lse;
-    TORCH_CHECK(varlen_fwd(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, Tensor(), Tensor(), out, lse, (int)shards, zigzag), spa_last_error());
+    accepted(varlen_fwd(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, Tensor(), Tensor(), out, lse, (int)shards, zigzag));
     ctx->save_for_backward({q, k, v, out, lse, cu_q, cu_k});
     ctx->saved_data["max_q"] = max_q;
     ctx->saved_data["max_k"] = max_k;
@@ -524,9 +530,11 @@ PyObject* attention(PyObject* const* a, std::index_sequence<I...>) {
   if (zigzag < 0 || zigzag > 0x3fffffffLL || transformed(t, N) || !attention_ok(t, N, zigzag)) Py_RETURN_NONE;
   const bool causal = flag_arg(a[N + 1]);
   variable_list r;
-  {
+  try {
     pybind11::gil_scoped_release no_gil;
     r = wants_grad(t, N) ? Attention<N>::apply(t[I]..., scale, causal, zigzag) : Attention<N>::forward_of(t, scale, causal, zigzag);
+  } catch (const Refused&) {
+    Py_RETURN_NONE;
   }
   return pair(r[0], r[1]);
   END_HANDLE_TH_ERRORS
@@ -562,7 +570,7 @@ PyObject* py_varlen_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
       shards < 1 || shards > 0xffffLL)
     Py_RETURN_NONE;
   variable_list r(2);
-  {
+  try {
     pybind11::gil_scoped_release no_gil;
     if (wants_grad(t, 3)) {
       View x, y, z;
@@ -574,6 +582,8 @@ PyObject* py_varlen_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     } else if (!varlen_fwd(t[0], t[1], t[2], t[3], t[4], mq, mk, scale, causal, Tensor(), Tensor(), r[0], r[1], (int)shards, zigzag)) {
       r.clear();
     }
+  } catch (const Refused&) {
+    Py_RETURN_NONE;
   }
   if (r.empty()) Py_RETURN_NONE;
   return pair(r[0], r[1]);

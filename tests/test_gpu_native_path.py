@@ -219,3 +219,18 @@ def test_every_function_works_without_the_native_module(monkeypatch):
     for one, other in zip(results[:len(calls) + 1], results[len(calls) + 1:]):
         for a, b in zip(one, other):  # (both round to bf16, at most once per ring step)
             torch.testing.assert_close(a, b, atol=4e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_a_forward_that_the_entry_point_refuses_is_the_python_paths_error(grad):
+    """Rows 8 MiB apart, more than the kernels can re-base (2 GiB a head, 1 GiB in 128 rows): SpaError from every function, with and
+    without gradients."""
+    S, D, stride = 260, 64, (1 << 22) + 8
+    base = torch.zeros(S * stride, dtype=torch.bfloat16, device=DEV)
+    x = base.as_strided((1, S, 1, D), (S * stride, stride, D, 1)).requires_grad_(grad)
+    cu = torch.tensor([0, S], dtype=torch.int32, device=DEV)
+    for call in (lambda: spa.sp_aurora_func(x, x, x, causal=True), lambda: spa.ulysses_flash_attn_func(x, x, x),
+                 lambda: spa.sp_aurora_varlen_func(x[0], x[0], x[0], cu, max_seqlen=S, causal=True),
+                 lambda: spa._flash_attn_forward(*[x.transpose(1, 2)] * 3)):
+        with pytest.raises(_lib.SpaError, match="1 GiB or more"):
+            call()
