@@ -567,7 +567,9 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     for (int v = 0; v < 16; ++v) o[i][v] = 0.f;
   float m_run = -INFINITY;  // reference row max of the raw scores (may lag the true max, see below)
   float l_run = 0.f;        // this lane's share of the running row sum
-  const float c = p.scale_log2 * ksc;  // scores are q . k8: the scale of K rides on the softmax scale
+  // scores are q . k8: the scale of K rides on the softmax scale.  A scale of 0 (a head of zeros) makes every score 0; as a tiny number
+  // it leaves the hidden ones at -inf.
+  const float c_in = p.scale_log2 * ksc, c = KV8 && c_in == 0.f ? 1e-30f : c_in;
 
   // per-lane LDS addresses of the operands of MFMA phase i: V(i) and K(i+1); computed before the
   // barrier that opens the phase

@@ -264,3 +264,29 @@ def test_ring_forward_with_e4m3_q_k_v(B, H, P, s, causal):
             check_lse(lse, want_lse)
     with pytest.raises(_lib.SpaError):
         ops.ring_fwd(q8.to(DEV), k8.to(DEV), v8.to(DEV), P, None, True, q_scale=qsc, k_scale=ksc, v_scale=vsc, sharding="zigzag")
+
+
+@pytest.mark.parametrize("q8", [False, True])
+@pytest.mark.parametrize("Sq,Sk,causal", [(128, 128, False), (300, 300, True), (260, 515, False), (1, 70, False), (64, 64, True)])
+def test_a_key_scale_of_zero(Sq, Sk, causal, q8):
+    """A head of zeros quantised with a scale of 0: every score is 0, the result the mean of the visible values, in every form."""
+    B, H, D, dtype = 1, 3, 128, torch.bfloat16
+    q, k, v = (rand((B, H, n, D), 590 + i, torch.float32) for i, n in enumerate((Sq, Sk, Sk)))
+    (k8, ksc), (v8, vsc) = (ops.quantize_fp8_per_head(t, layout="bhsd") for t in (k, v))
+    ksc[0, 1] = 0.0
+    scales, x = {"k_scale": ksc.to(DEV), "v_scale": vsc.to(DEV)}, q.to(dtype)
+    deq = q.to(dtype).double()
+    if q8:
+        x, qsc = ops.quantize_fp8_per_head(q, layout="bhsd")
+        scales["q_scale"], deq = qsc.to(DEV), x.double() * qsc[..., None, None].double()
+    want, want_lse = O.attn_block(deq, k8.double() * ksc[..., None, None].double(), v8.double() * vsc[..., None, None].double(), None, causal)
+    for form in ({}, dict(fwd_groups=1), dict(fwd_groups=2, fwd_share=1), dict(fwd_groups=2, fwd_share=2)):
+        try:
+            for knob, value in form.items():
+                _lib.tune(knob, value)
+            out, lse = ops.flash_fwd(x.to(DEV), k8.to(DEV), v8.to(DEV), None, causal, layout="bhsd", **scales)
+        finally:
+            for knob in form:
+                _lib.tune(knob, 0)
+        check_out(out, want, dtype)
+        check_lse(lse, want_lse)
