@@ -810,7 +810,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     // burst after the barrier, they hold up the wave's instruction stream while the memory pipeline
     // takes them in.
     constexpr int LOAD_GAP = NBODY / G::NL;
-    for (int i = it0; i < nt; ++i) {
+    for (int i = it0; i < nt;) {
       wait_loads_but<G::NL>();
       __syncthreads();
       set_addresses(i);
@@ -894,6 +894,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
         sc = sn;
         dc = dn;
       }
+      if (++i == nt) mfma_settle();
     }
     wait_loads_but<0>();
   }
