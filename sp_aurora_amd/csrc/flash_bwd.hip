@@ -394,40 +394,53 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   constexpr int BWD_LOOK = NA < LOOK_CAP ? NA : LOOK_CAP;
   static_assert(NBODY % BWD_LOOK == 0 && BWD_LOOK <= NA, "the operand window must tile the loop body");
 
-  // The workgroup's rows of q and dout pass through the stages on their way into registers; then those of out, which give
-  // delta = rowsum(dout * out) (written for the dk / dv kernel), while the first two tiles are on their way.
-  {
-    constexpr int RT = NW / 2;  // tiles of 64 rows
-    auto load_rows = [&](const T* base, int64_t stride, unsigned dst) {
-      TileLoader<T, D, NW * 64, ADDR> ld;
-      ld.init(base, stride, p.Sq, span_q, tid);
+  // The workgroup's rows of q and dout pass through the stages on their way into registers, and those of out, which give
+  // delta = rowsum(dout * out) (written for the dk / dv kernel).  128 rows are one stage a tensor: all of them and the first tile are
+  // requested together.  256 rows are two: out follows when q and dout have been read, with the first two tiles.
+  constexpr bool TOGETHER = NW == 4;
+  constexpr int RT = NW / 2;  // tiles of 64 rows
+  const unsigned own = (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB;
+  const unsigned q_at = lds0 + (TOGETHER ? 2 * G::STAGE : 0), do_at = lds0 + (TOGETHER ? 3 : 2) * G::STAGE, out_at = lds0 + (TOGETHER ? 1 : 2) * G::STAGE;
+  auto load_rows = [&](const T* base, int64_t stride, unsigned dst) {
+    TileLoader<T, D, NW * 64, ADDR> ld;
+    ld.init(base, stride, p.Sq, span_q, tid);
 #pragma unroll
-      for (int i = 0; i < RT; ++i)
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
-        for (int q = 0; q < C::NDMA; ++q) ld.load(q, q0 + i * BWD_ROWS < p.Sq, q0 + i * BWD_ROWS, dst + i * C::TILEB + w * 1024, map, p.map.pitch);
-    };
-    const unsigned own = (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB, other = 2 * G::STAGE;
-    load_rows(qp, p.qs.s, lds0);
-    load_rows(dop, p.dos.s, lds0 + other);
+      for (int q = 0; q < C::NDMA; ++q) ld.load(q, q0 + i * BWD_ROWS < p.Sq, q0 + i * BWD_ROWS, dst + i * C::TILEB + w * 1024, map, p.map.pitch);
+  };
+  auto load_out = [&]() {
+    if (p.out) load_rows((const T*)p.out + b * p.os.b + h * p.os.h, p.os.s, out_at);
+  };
+  load_rows(qp, p.qs.s, q_at);
+  load_rows(dop, p.dos.s, do_at);
+  if constexpr (TOGETHER) {
+    load_out();
+    issue_tile(0);
+    wait_loads_but<G::NL>();
+  } else {
     wait_loads_but<0>();
-    __syncthreads();
-    read_rows<frag, D>(qf, lds0 + own, rd);
-    read_rows<frag, D>(dof, lds0 + other + own, rd);
+  }
+  __syncthreads();
+  read_rows<frag, D>(qf, q_at + own, rd);
+  read_rows<frag, D>(dof, do_at + own, rd);
+  if constexpr (!TOGETHER) {
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): read ...
     __syncthreads();                     // ... by every wave
-    if (p.out) load_rows((const T*)p.out + b * p.os.b + h * p.os.h, p.os.s, lds0 + other);
+    load_out();
+    issue_tile(0);
+    issue_tile(1);
   }
-  issue_tile(0);
-  issue_tile(1);
   float dl;
   if (p.out) {
-    wait_loads_but<2 * G::NL>();
-    __syncthreads();
-    const unsigned own = lds0 + 2 * G::STAGE + (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB;
+    if constexpr (!TOGETHER) {
+      wait_loads_but<2 * G::NL>();
+      __syncthreads();
+    }
     float sum = 0.f;
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) {
-      const u32x4 x = lds_read_b128(own + rd.row[ks]), y = __builtin_bit_cast(u32x4, dof[ks]);
+      const u32x4 x = lds_read_b128(out_at + own + rd.row[ks]), y = __builtin_bit_cast(u32x4, dof[ks]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float x0, x1, y0, y1;
@@ -438,11 +451,12 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
     }
     dl = halves_sum(sum);
     if (hh == 0 && qrow < p.Sq) p.delta[li] = dl;
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    __syncthreads();
   } else {
     dl = p.delta[li];
   }
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // the rows have been read ...
+  __syncthreads();                     // ... by every wave
+  if constexpr (TOGETHER) issue_tile(1);
   issue_tile(2);
   wait_loads_but<2 * G::NL>();
   __syncthreads();
@@ -1358,7 +1372,8 @@ hipError_t launch(int smem, bool queries, int rows, BwdParams p, hipStream_t str
 template <typename T, int D, int ADDR = ADDR_PLAIN>
 hipError_t launch_both(const BwdParams& p, hipStream_t stream) {
   // dq kernel, D = 128: 256-row workgroups (two waves per SIMD, the K/V stream shared by twice the rows) once
-  // there are enough of them to occupy every CU; spa_tune() can force 4 or 8 waves (experiments, tests).
+  // there are enough of them to occupy every CU and sequences have more than 128 rows (2000 x 16 heads of 16 rows, causal, backward:
+  // 1923 us, 1679 with 128; 500 of 128 rows 800, 764; 400 of 160 rows 921, 1024); spa_tune() can force 4 or 8 waves (experiments, tests).
   // At D = 64 two 128-row workgroups to a CU are as fast on long rows (+-2 %) and 4 to 7 % faster on short ones.
   // (Tensors of 2 GiB or more per (batch, head): 128 rows.)
   const int64_t wgs8 = p.cu_q ? (int64_t)p.H * (p.lse_bh / 256 + (p.B + 1) / 2) : (int64_t)p.B * p.H * ((p.Sq + 255) / 256);
@@ -1366,7 +1381,7 @@ hipError_t launch_both(const BwdParams& p, hipStream_t stream) {
   hipError_t e = hipErrorInvalidValue;
   bool wide = false;
   if constexpr (D == 128 && ADDR != ADDR_BIG) {
-    wide = forced ? forced == 8 : wgs8 >= spa_device_cus();
+    wide = forced ? forced == 8 : wgs8 >= spa_device_cus() && p.Sq > 128;
     if (wide) e = launch<flash_bwd_dq_kernel<T, D, 8, ADDR>>(DqCfg<D, 8>::SMEM, true, 256, p, stream, 512);
   }
   if (!wide) e = launch<flash_bwd_dq_kernel<T, D, 4, ADDR>>(DqCfg<D, 4>::SMEM, true, 128, p, stream);
