@@ -578,8 +578,9 @@ def check_cu_seqlens(cu, total, max_seqlen, what):
         raise ValueError(f"{what}: longest sequence {int(lens.max())} exceeds max_seqlen {int(max_seqlen)}")
 
 
-# (address, version counter, length, device, total rows, max_seqlen) of cu_seqlens arrays that passed
-# check_cu_seqlens: a training loop hands the same array to every layer, and one look is enough
+# (address, version counter, length, device, total rows, max_seqlen) of cu_seqlens arrays that passed check_cu_seqlens, and the array: a
+# training loop hands the same array to every layer, and one look is enough.  The array is held so that no other one can come to lie
+# at its address; at most 256 of them, none of a storage above 1 MiB, all given back when the 257th comes.
 _CU_CHECKED = {}
 
 
@@ -595,9 +596,10 @@ def check_cu_seqlens_once(cu, total, max_seqlen, what):
     if cu.is_cuda and torch.cuda.is_current_stream_capturing():
         return False
     check_cu_seqlens(cu, total, max_seqlen, what)
-    if len(_CU_CHECKED) >= 256:
-        _CU_CHECKED.clear()
-    _CU_CHECKED[key] = True
+    if cu.untyped_storage().nbytes() <= 1 << 20:
+        if len(_CU_CHECKED) >= 256:
+            _CU_CHECKED.clear()
+        _CU_CHECKED[key] = cu.detach()
     return True
 
 

@@ -324,3 +324,22 @@ def test_a_native_module_that_cannot_be_loaded_is_reported_once(monkeypatch):
         q = torch.zeros(1, 4, 2, 64)
         with pytest.raises(ValueError, match="HIP device"):  # (what the Python path says to a CPU tensor)
             spa.sp_aurora_func(q, q, q)
+
+
+def test_offsets_are_looked_at_again_when_another_array_takes_the_address():
+    """An array that was freed and another of the same length, total and longest sequence allocated in its place."""
+    import torch
+
+    from sp_aurora_amd import ops
+    for good in [[0, 4, 10], [0, 3, 10]] * 8:
+        cu = torch.tensor(good, dtype=torch.int32)
+        assert ops.check_cu_seqlens_once(cu, 10, 9, "cu") and ops.check_cu_seqlens_once(cu[:], 10, 9, "cu")
+        del cu
+        bad = torch.tensor([0, 12, 10], dtype=torch.int32)
+        with pytest.raises(ValueError):
+            ops.check_cu_seqlens_once(bad, 10, 9, "cu")
+        del bad
+    big = torch.zeros(1 << 20, dtype=torch.int32)
+    big[1:3] = torch.tensor([5, 10])
+    held = len(ops._CU_CHECKED)
+    assert ops.check_cu_seqlens_once(big[:3], 10, 9, "cu") and len(ops._CU_CHECKED) == held
