@@ -9,8 +9,8 @@
 // artificial intelligence datatype for higher-precision computations", 2019).  Against float64 the results are closer than those of
 // v_mfma_f32_32x32x2_f32 were: rms 2.7e-8 and 3.3e-8 at 2048 keys, D = 128, 1.6e-8 and 2.4e-8 at 512, D = 64.
 // That instruction does 64 operations a clock and SIMD; six bf16 products at 1024 do 170.
-// Bound: the matrix pipe, 6 * 2 * (D / 16) * 32 clocks per 32 x 32 scores, beside 136 vector instructions of softmax and splitting P
-// and 22 D / 16 of splitting K and V, once per workgroup and tile.
+// Bound: the matrix pipe, 6 * 2 * (D / 16) * 32 clocks per 32 x 32 scores, beside 168 vector instructions of softmax and splitting P
+// and 30 D / 16 of splitting K and V, once per workgroup and tile.
 #include "spa_common.h"
 #include "spa_host.h"
 
@@ -29,14 +29,17 @@ __device__ __forceinline__ void split2(float x0, float x1, unsigned& h, unsigned
   m = M::pack2(r0, r1);
   l = M::pack2(r0 - __builtin_bit_cast(float, m << 16), r1 - __builtin_bit_cast(float, m & 0xffff0000u));
 }
-// Eight values as three operands.
+// Eight values as three operands.  They are taken times 2^24: the lowest bit of any fp32 number, denormals included, is then a normal
+// bf16 number, where the low terms of values below 2^-110 would be cut off (relative errors of 3e-6 at 1e-35, 3e-3 at 1e-38; the factors cost 3 % of
+// the times below at D = 128, 7 % at the smaller ones).
+constexpr float F32_UP = 0x1p24f, F32_DOWN = 0x1p-48f;  // F32_DOWN: of a product of two
 struct Split8 {
   u32x4 h, m, l;
-  __device__ __forceinline__ void set(const float* x) {
+  __device__ __forceinline__ void set(const float* x, float up = F32_UP) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       unsigned a, b, c;
-      split2(x[2 * i], x[2 * i + 1], a, b, c);
+      split2(x[2 * i] * up, x[2 * i + 1] * up, a, b, c);
       h[i] = a;
       m[i] = b;
       l[i] = c;
@@ -68,8 +71,13 @@ template <int D>
 struct Rows {
   Split8 q[D / 16];
   f32x16 o[D / 32];
-  float m_run, l_run, c;
+  float m_run, l_run, c, down;
+  // A score above 2^80 is an infinity in the accumulator, and its row a NaN; one below -2^80 has no weight beside a largest score above
+  // -2^70, and rows without one are computed again (lost()).  With a scale that leaves such scores apart the bits that q
+  // needs lie higher: below 2^-93 they cannot move an exponent by 2^-50.
   __device__ __forceinline__ void init(const float* row, int hh, bool negate, float scale_log2) {
+    const bool tiny = scale_log2 < 0x1p-64f;
+    down = tiny ? 0x1p16f : F32_DOWN;
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) {
       float x[8];
@@ -79,7 +87,7 @@ struct Rows {
         x[e] = negate ? -a[e] : a[e];  // negative softmax scale: -q with |scale|
         x[4 + e] = negate ? -b[e] : b[e];
       }
-      q[ks].set(x);
+      q[ks].set(x, tiny ? 0x1p-40f : F32_UP);
     }
 #pragma unroll
     for (int i = 0; i < D / 32; ++i) zero16(o[i]);
@@ -87,6 +95,7 @@ struct Rows {
     l_run = 0.f;
     c = scale_log2;
   }
+  __device__ __forceinline__ bool lost(float m) const { return m < -0x1p70f; }
   // s: raw scores of the tile, keys the row does not see at -inf.  The reference maximum moves only when a row's has grown by
   // more than 2^8 (flash_fwd.hip).
   __device__ __forceinline__ void raise(const f32x16& s) {
@@ -203,8 +212,8 @@ struct Fwd32Cfg {
 };
 
 // Many rows: a workgroup of 128 query rows; K and V tiles are split once, on their way into LDS, and read by its four waves.
-// Causal [1, 4096, 32, 128] 1289 -> 778 us (177 TFLOP/s, 1.06 PFLOP/s of bf16 products), [1, 4096, 16, 64] 440 -> 220, full
-// [1, 2048, 16, 32] 118 -> 90.
+// Causal [1, 4096, 32, 128] 1275 -> 799 us (172 TFLOP/s, 1.03 PFLOP/s of bf16 products), [1, 4096, 16, 64] 446 -> 235, full
+// [1, 2048, 16, 32] 118 -> 93.
 template <int D>
 __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_kernel(const FwdParams pk) {
   typedef Fwd32Cfg<D> C;
@@ -341,7 +350,7 @@ __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_ker
       mma6(a, rows.q[ks], s, s1);
     }
 #pragma unroll
-    for (int v = 0; v < 16; ++v) s[v] += s1[v];
+    for (int v = 0; v < 16; ++v) s[v] = (s[v] + s1[v]) * rows.down;
   };
 
   gload(kp, p.ks.s, 0, kreg);
@@ -400,7 +409,7 @@ __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_ker
       for (int i = 0; i < 6 * (D / 16); ++i) {
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x2, (160 + 6 * (D / 16) - 1) / (6 * (D / 16)), 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, (192 + 6 * (D / 16) - 1) / (6 * (D / 16)), 0);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -444,10 +453,10 @@ __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_ker
     gload(vp, p.vs.s, it + 2, vreg);
   }
 
-  const float l_tot = halves_sum(rows.l_run), inv = 1.f / l_tot;
+  const float l_tot = halves_sum(rows.l_run), inv = 1.f / l_tot * F32_DOWN;
   float* const obase = (float*)p.out + b * p.os.b + h * p.os.h;
   float* const lbase = p.lse + ((int64_t)b * p.H + h) * p.lse_bh;
-  bool bad = false;
+  bool bad = qrow < p.Sq && rows.lost(rows.m_run);
   if (qrow < p.Sq) {
     float* op = obase + (int64_t)row_of(qrow) * p.os.s;
 #pragma unroll
@@ -548,7 +557,7 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
       for (int db = 0; db < D / 32; ++db) va[u][db].set(vx[u][db]);
     if (it + NW < nt) gload(it + NW);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) s[v] += s1[v];
+    for (int v = 0; v < 16; ++v) s[v] = (s[v] + s1[v]) * rows.down;
     mask_tile(s, key0, q0, qrow, p.causal, p.Sk, hh);
     Split8 pf[2];
     rows.raise(s);
@@ -595,10 +604,10 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
     aw[j] = mw[j] == -INFINITY ? 0.f : fast_exp2((mw[j] - m_all) * rows.c);  // a wave without a visible key
     l_all += aw[j] * sm[j * (C::REC + 128) + C::REC + 32 + ln];
   }
-  const float inv = 1.f / l_all;
+  const float inv = 1.f / l_all * F32_DOWN;
   float* const obase = (float*)p.out + b * p.os.b + h * p.os.h;
   float* const lbase = p.lse + ((int64_t)b * p.H + h) * p.lse_bh;
-  bool bad = false;
+  bool bad = qrow < p.Sq && rows.lost(m_all);
   if (qrow < p.Sq) {
     float* const op = obase + (int64_t)row_of(qrow) * p.os.s;
     for (int pc = w; pc < NPC; pc += NW) {

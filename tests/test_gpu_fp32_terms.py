@@ -64,3 +64,28 @@ def test_fp32_values_that_have_no_three_terms(form, D, S, causal):
     torch.testing.assert_close(out.cpu().double(), want, rtol=1e-4, atol=1e-5, equal_nan=True)
     want_lse = torch.logsumexp(s.masked_fill(~seen, -float("inf")), -1)
     torch.testing.assert_close(lse.cpu().double(), want_lse, rtol=1e-5, atol=1e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("form", [1, 2])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("q_size,k_size,v_size,scale", [(1.0, 1.0, 1e-33, 0.1), (1.0, 1.0, 1e-36, 0.1), (1.0, 1.0, 1e-38, 0.1), (1e-36, 1e30, 1.0, 1e5),
+                                                        (1e30, 1e-37, 1.0, 1e6), (1e-38, 1e-5, 1.0, 1e38), (1e15, 1e14, 1.0, 1e-30), (1e14, 1e13, 1e-37, 1e-28)])
+def test_fp32_small_and_large_values(form, D, q_size, k_size, v_size, scale):
+    """Values at which a term of a split value would leave the bf16 range: the results are as exact as those of values around one."""
+    g = torch.Generator().manual_seed(D)
+    S, H = 130, 2
+    q, k, v = (torch.randn((1, S, H, D), generator=g) * x for x in (q_size, k_size, v_size))
+    qh, kh, vh = (t.double().transpose(1, 2) for t in (q, k, v))
+    s, mass = qh @ kh.transpose(-1, -2) * scale, qh.abs() @ kh.abs().transpose(-1, -2) * scale
+    p = torch.softmax(s, -1)
+    _lib.tune("fwd32_split", form)
+    try:
+        out, lse = ops.flash_fwd(q.to(DEV), k.to(DEV), v.to(DEV), scale, False, layout="bshd")
+    finally:
+        _lib.tune("fwd32_split", 0)
+    # the bound of test_fp32_against_float64, and the smallest fp32 number, 2^-149, once for a result and once for its sum
+    ds = mass * (2 + D / 16 + 6) * 2.0 ** -24 + (1 + s.abs()) * 2.0 ** -22
+    bound = (2 * ds.amax(-1) + (S / 16 + 8) * 2.0 ** -24)[..., None] * (p @ vh.abs()) + 2.0 ** -148
+    err = (out.cpu().double() - (p @ vh).transpose(1, 2)).abs().transpose(1, 2)
+    assert (err <= bound).all(), float((err / bound).max())
+    assert ((lse.cpu().double() - torch.logsumexp(s, -1)).abs() <= 2 * ds.amax(-1) + 2.0 ** -22 * (1 + s.abs().amax(-1))).all()
