@@ -142,9 +142,10 @@ __device__ __forceinline__ void mask_tile(f32x16& s, int key0, int first_row, in
   }
 }
 
-// An infinity (or a value above the largest bf16 number) has no three exact terms: the rows that it reaches come out as NaN.  Rows
-// with a NaN are computed again here with plain fp32 operations and masked keys left out, so that they are infinite, finite or NaN as
-// the arithmetic of the inputs has it.  bad: the rows q0 + i of this wave, bit i; of the values d the wave stores those with
+// An infinity (or a value above 2^104) has no three exact terms: the rows that it reaches come out as NaN.  Sums of large values times
+// weights above 1 (raise()) overflow where the weighted mean is finite.  Rows with a result that is not finite are computed again here with plain
+// fp32 operations, weights of at most 1 and masked keys left out, so that they are infinite, finite or NaN as the arithmetic of
+// the inputs has it.  bad: the rows q0 + i of this wave, bit i; of the values d the wave stores those with
 // (d / 8) % NW == w, and the lse if w == 0.
 template <int D, int NW, typename RowOf, typename StatOf>
 __device__ __forceinline__ void plain_rows(const FwdParams& p, unsigned bad, int q0, const float* qp, const float* kp, const float* vp, float* out,
@@ -467,16 +468,16 @@ __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_ker
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           st[e] = rows.o[db][4 * g + e] * inv;
-          bad |= st[e] != st[e];
+          bad |= !(fabsf(st[e]) < INFINITY);
         }
         *(f32x4*)(op + db * 32 + 8 * g + 4 * hh) = st;
       }
     if (hh == 0) lbase[stat_of(qrow)] = (rows.m_run * rows.c + fast_log2(l_tot)) * 0.6931471805599453f;
   }
-  const uint64_t nan = __builtin_amdgcn_ballot_w64(bad);
-  if (nan) {
+  const uint64_t again = __builtin_amdgcn_ballot_w64(bad);
+  if (again) {
     __threadfence();  // (other lanes of this wave write those rows again)
-    plain_rows<D, 1>(p, (unsigned)(nan | nan >> 32), qw0, qp, kp, vp, obase, lbase, rows.c, lane, 0, row_of, stat_of);
+    plain_rows<D, 1>(p, (unsigned)(again | again >> 32), qw0, qp, kp, vp, obase, lbase, rows.c, lane, 0, row_of, stat_of);
   }
 }
 
@@ -621,16 +622,16 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         acc[e] *= inv;
-        bad |= acc[e] != acc[e];
+        bad |= !(fabsf(acc[e]) < INFINITY);
       }
       *(f32x4*)(op + (pc / 4) * 32 + 8 * (pc % 4) + 4 * hh) = acc;
     }
     if (w == 0 && hh == 0) lbase[stat_of(qrow)] = (m_all * rows.c + fast_log2(l_all)) * 0.6931471805599453f;
   }
-  const uint64_t nan = __builtin_amdgcn_ballot_w64(bad);
-  if (nan) {
+  const uint64_t again = __builtin_amdgcn_ballot_w64(bad);
+  if (again) {
     __threadfence();
-    plain_rows<D, NW>(p, (unsigned)(nan | nan >> 32), q0, qp, kp, vp, obase, lbase, rows.c, lane, w, row_of, stat_of);
+    plain_rows<D, NW>(p, (unsigned)(again | again >> 32), q0, qp, kp, vp, obase, lbase, rows.c, lane, w, row_of, stat_of);
   }
 }
 

@@ -89,3 +89,24 @@ def test_fp32_small_and_large_values(form, D, q_size, k_size, v_size, scale):
     err = (out.cpu().double() - (p @ vh).transpose(1, 2)).abs().transpose(1, 2)
     assert (err <= bound).all(), float((err / bound).max())
     assert ((lse.cpu().double() - torch.logsumexp(s, -1)).abs() <= 2 * ds.amax(-1) + 2.0 ** -22 * (1 + s.abs().amax(-1))).all()
+
+
+@pytest.mark.parametrize("form", [1, 2])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("size", [1e16, 1e20, 1e25, 1e31, 3e36])
+def test_fp32_large_values_under_weights_above_one(form, D, size):
+    """Scores that rise along the keys by less than what moves the reference maximum: sums of 2^8 times the values, means that are finite."""
+    g = torch.Generator().manual_seed(D)
+    S, H = 300, 2
+    q, k = torch.zeros(1, S, H, D), torch.zeros(1, S, H, D)
+    q[..., 0], k[..., 0] = 1.0, torch.linspace(0.0, 5.4, S)[None, :, None]  # (times log2 e: 7.8)
+    # (the weights below 1 add up to 300 / 5.4 = 56, times a mean value of 1.5 * 3e36: 2.5e38, less than the largest fp32 number)
+    v = (1 + torch.rand((1, S, H, D), generator=g)) * size
+    p = torch.softmax(q.double().transpose(1, 2) @ k.double().transpose(1, 2).transpose(-1, -2), -1)
+    _lib.tune("fwd32_split", form)
+    try:
+        out, lse = ops.flash_fwd(q.to(DEV), k.to(DEV), v.to(DEV), 1.0, False, layout="bshd")
+    finally:
+        _lib.tune("fwd32_split", 0)
+    # exponents are off by 2^-23 of at most 8, weights by 2^-22 more, sums by a rounding a key at most (all of one sign)
+    torch.testing.assert_close(out.cpu().double(), (p @ v.double().transpose(1, 2)).transpose(1, 2), rtol=(S + 32) * 2.0 ** -24, atol=0.0)
