@@ -46,16 +46,18 @@ struct Split8 {
     }
   }
 };
-// acc0 + acc1 += a b: the small terms and the large one in two accumulators (two chains of dependent instructions).
+// acc0 + acc1 += a b: the large term alone in acc0, the five small ones in acc1.  Where one product dominates a sum, its h h' is exact in
+// acc0 and the sum is rounded once, when the two are added, as a fused operation would round it (with h m' and m h' in acc0 it was
+// rounded twice).
 __device__ __forceinline__ void mma6(const Split8& a, const Split8& b, f32x16& acc0, f32x16& acc1) {
   const frag ah = as_frag<frag>(a.h), am = as_frag<frag>(a.m), al = as_frag<frag>(a.l);
   const frag bh = as_frag<frag>(b.h), bm = as_frag<frag>(b.m), bl = as_frag<frag>(b.l);
   acc1 = M::run(ah, bl, acc1);
-  acc0 = M::run(ah, bm, acc0);
-  acc1 = M::run(am, bm, acc1);
-  acc0 = M::run(am, bh, acc0);
-  acc1 = M::run(al, bh, acc1);
   acc0 = M::run(ah, bh, acc0);
+  acc1 = M::run(am, bm, acc1);
+  acc1 = M::run(al, bh, acc1);
+  acc1 = M::run(ah, bm, acc1);
+  acc1 = M::run(am, bh, acc1);
 }
 template <bool X>
 struct Bool {
