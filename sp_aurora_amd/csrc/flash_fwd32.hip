@@ -7,7 +7,8 @@
 // three others are less than 2^-23 |x y| together and 2^-26 as a rule, either sign, where the chain of D fused operations that
 // they replace rounds D times at 2^-24 of the running sum (the scheme of Henry, Tang and Heinecke, "Leveraging the bfloat16
 // artificial intelligence datatype for higher-precision computations", 2019).  Against float64 the results are closer than those of
-// v_mfma_f32_32x32x2_f32 were: rms 2.7e-8 and 3.3e-8 at 2048 keys, D = 128, 1.6e-8 and 2.4e-8 at 512, D = 64.
+// v_mfma_f32_32x32x2_f32 were: rms 2.7e-8 and 3.4e-8 at 2048 keys, D = 128, 1.3e-8 and 2.4e-8 at 512, D = 64; with one value per row of q 3.7e-8
+// and 4.8e-8, 2.1e-8 and 2.4e-8.
 // That instruction does 64 operations a clock and SIMD; six bf16 products at 1024 do 170.
 // Bound: the matrix pipe, 6 * 2 * (D / 16) * 32 clocks per 32 x 32 scores, beside 168 vector instructions of softmax and splitting P
 // and 30 D / 16 of splitting K and V, once per workgroup and tile.
@@ -145,52 +146,110 @@ __device__ __forceinline__ void mask_tile(f32x16& s, int key0, int first_row, in
 }
 
 // An infinity (or a value above 2^104) has no three exact terms: the rows that it reaches come out as NaN.  Sums of large values times
-// weights above 1 (raise()) overflow where the weighted mean is finite.  Rows with a result that is not finite are computed again here with plain
-// fp32 operations, weights of at most 1 and masked keys left out, so that they are infinite, finite or NaN as the arithmetic of
-// the inputs has it.  bad: the rows q0 + i of this wave, bit i; of the values d the wave stores those with
-// (d / 8) % NW == w, and the lse if w == 0.
-template <int D, int NW, typename RowOf, typename StatOf>
-__device__ __forceinline__ void plain_rows(const FwdParams& p, unsigned bad, int q0, const float* qp, const float* kp, const float* vp, float* out,
-                                           float* lse, float c, int lane, int w, RowOf row_of, StatOf stat_of) {
-  while (bad) {
-    const int qrow = q0 + __builtin_ctz(bad);
-    bad &= bad - 1;
-    const int keys = p.causal && qrow + 1 < p.Sk ? qrow + 1 : p.Sk;
-    const float* const q = qp + (int64_t)row_of(qrow) * p.qs.s;
-    const auto score = [&](int key) {
-      const float* const k = kp + (int64_t)row_of(key) * p.ks.s;
-      float s = 0.f;
-      for (int d = 0; d < D; ++d) s = __builtin_fmaf(q[d], k[d], s);
-      return p.negq ? -s : s;
+// weights above 1 (raise()) overflow where the weighted mean is finite.  Rows with a result that is not finite are computed again here, with the
+// fp32 matrix instruction, weights of at most 1 and masked keys left out, so that they are infinite, finite or NaN as the arithmetic of
+// the inputs has it: a wave's 32 rows together, over the key tiles it0, it0 + step, ..., until every bad row (bit i: row q0 + i) has met a NaN.
+// Bound: that instruction's rate (64 operations a clock and SIMD) and the latency of the loads, which go straight into operands, a tile of V and the next
+// of K ahead.  Every row of causal [1, 4096, 32, 128] again, for an infinity in V: 847 -> 2241 us the call, [1, 1024, 16, 64] 33 -> 90 (row by
+// row with plain operations [1, 1024, 32, 128] took 8500, now 333); a NaN in K ends the pass where it lies (867 and 89).
+template <int D>
+struct PlainRows {
+  f32x16 o[D / 32];
+  float m, l;  // of row ln, over this lane's keys
+  template <typename RowOf>
+  __device__ __forceinline__ void run(const FwdParams& p, unsigned bad, int q0, const float* qp, const float* kp, const float* vp, float c, int lane,
+                                      int it0, int step, RowOf row_of) {
+    const int ln = lane & 31, hh = lane >> 5, qrow = q0 + ln, last = p.Sk - 1;
+    const int lim = p.causal && qrow < last ? qrow : last;
+    const int kv_end = p.causal && q0 + 32 < p.Sk ? q0 + 32 : p.Sk, nt = (kv_end + F32_BN - 1) / F32_BN;
+    // of the products of a score, half hh of the wave takes those of values hh * D / 2 and on
+    const auto half_row = [&](const float* base, int64_t stride, int row) { return (const f32x4*)(base + (int64_t)row_of(row) * stride + hh * (D / 2)); };
+    f32x4 q[D / 8];
+    const f32x4* const qr = half_row(qp, p.qs.s, qrow < p.Sq ? qrow : p.Sq - 1);
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) q[i] = p.negq ? -qr[i] : qr[i];
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) zero16(o[i]);
+    m = -INFINITY;
+    l = 0.f;
+    f32x4 k[D / 8];
+    const auto load_keys = [&](int it) {
+      const f32x4* const kr = half_row(kp, p.ks.s, it * F32_BN + ln < p.Sk ? it * F32_BN + ln : last);
+#pragma unroll
+      for (int i = 0; i < D / 8; ++i) k[i] = kr[i];
     };
-    float m = -INFINITY;
-    for (int key = lane; key < keys; key += 64) m = fmaxf(m, score(key));
-    for (int i = 1; i < 64; i *= 2) m = fmaxf(m, __shfl_xor(m, i));
-    const float mc = m == -INFINITY ? 0.f : m * c;
-    constexpr int ND = (D + 63) / 64;
-    float o[ND] = {}, l = 0.f;
-    for (int key0 = 0; key0 < keys; key0 += 64) {
-      const float x = key0 + lane < keys ? fast_exp2(__builtin_fmaf(score(key0 + lane), c, -mc)) : 0.f;
-      l += x;
-      const int n = keys - key0 < 64 ? keys - key0 : 64;
-      for (int j = 0; j < n; ++j) {
-        const float pj = __shfl(x, j);
-        const float* const v = vp + (int64_t)row_of(key0 + j) * p.vs.s;
+    load_keys(it0);
+#pragma unroll 1
+    for (int it = it0; it < nt; it += step) {
+      const int key0 = it * F32_BN;
+      f32x16 s;
+      zero16(s);
+      const bool whole = !(p.causal && key0 + F32_BN - 1 > q0) && key0 + F32_BN <= p.Sk;  // every row sees every key
+      float vx[16][D / 32];
+      if (whole) {
 #pragma unroll
-        for (int i = 0; i < ND; ++i)
-          if (D % 64 == 0 || lane < D) o[i] = __builtin_fmaf(pj, v[i * 64 + lane], o[i]);
+        for (int v = 0; v < 16; ++v) {
+          const float* const vr = vp + (int64_t)row_of(key0 + 8 * (v >> 2) + 4 * hh + (v & 3)) * p.vs.s + ln;
+#pragma unroll
+          for (int i = 0; i < D / 32; ++i) vx[v][i] = vr[32 * i];
+        }
       }
-    }
-    for (int i = 1; i < 64; i *= 2) l += __shfl_xor(l, i);
-    float* const to = out + (int64_t)row_of(qrow) * p.os.s;
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < ND; ++i) {
-      const int d = i * 64 + lane;
-      if (d < D && (d / 8) % NW == w) to[d] = o[i] * (1.f / l);
+      for (int i = 0; i < D / 8; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i][e], q[i][e], s, 0, 0, 0);
+      if (it + step < nt) load_keys(it + step);
+      mask_tile(s, key0, q0, qrow, p.causal, p.Sk, hh);
+      float mx = s[0];
+#pragma unroll
+      for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
+      const float m_new = fmaxf(m, halves_max(mx)), alpha = m_new == -INFINITY ? 1.f : fast_exp2((m - m_new) * c);
+      const float mc = m_new == -INFINITY ? 0.f : m_new * c;
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        s[v] = fast_exp2(__builtin_fmaf(s[v], c, -mc));
+        l += s[v];
+      }
+#pragma unroll
+      for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[i][v] *= alpha;
+      if (!whole) {
+        // a tile with keys that some rows do not see: what lies there (an infinity times a weight of 0) stays out, key by key
+        const int n = p.Sk - key0 < F32_BN ? p.Sk - key0 : F32_BN;
+#pragma unroll 1
+        for (int j = 0; j < n; ++j) {
+          const int from = 4 * (j >> 3) + (j & 3);
+          float x = s[0];
+#pragma unroll
+          for (int v = 1; v < 16; ++v) x = from == v ? s[v] : x;
+          x = __shfl(x, ln + 32 * ((j >> 2) & 1));
+          const float* const vr = vp + (int64_t)row_of(key0 + j) * p.vs.s + 4 * hh;
+#pragma unroll
+          for (int i = 0; i < D / 8; ++i) {
+            const f32x4 y = *(const f32x4*)(vr + 8 * i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float sum = __builtin_fmaf(x, y[e], o[i / 4][4 * (i % 4) + e]);
+              o[i / 4][4 * (i % 4) + e] = key0 + j <= lim ? sum : o[i / 4][4 * (i % 4) + e];
+            }
+          }
+        }
+      } else {
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+#pragma unroll
+          for (int i = 0; i < D / 32; ++i) o[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(vx[v][i], s[v], o[i], 0, 0, 0);
+      }
+      const uint64_t nan = __builtin_amdgcn_ballot_w64(l != l);
+      if ((bad & ~(unsigned)(nan | nan >> 32)) == 0) break;
     }
-    if (lane == 0 && w == 0) lse[stat_of(qrow)] = (m * c + fast_log2(l)) * 0.6931471805599453f;
+    mfma_settle();
   }
-}
+};
 
 // 16-byte chunk permutations of a tile row in LDS, as in flash_fwd.hip.
 template <int D>
@@ -215,10 +274,10 @@ struct Fwd32Cfg {
 };
 
 // Many rows: a workgroup of 128 query rows; K and V tiles are split once, on their way into LDS, and read by its four waves.
-// Causal [1, 4096, 32, 128] 1275 -> 799 us (172 TFLOP/s, 1.03 PFLOP/s of bf16 products), [1, 4096, 16, 64] 446 -> 235, full
-// [1, 2048, 16, 32] 118 -> 93.
+// Causal [1, 4096, 32, 128] 1285 -> 768 us (179 TFLOP/s, 1.07 PFLOP/s of bf16 products), [1, 4096, 16, 64] 446 -> 234, full
+// [1, 2048, 16, 32] 119 -> 89.
 template <int D>
-__global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_kernel(const FwdParams pk) {
+__global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : D == 64 ? 2 : 3) flash_fwd32_kernel(const FwdParams pk) {
   typedef Fwd32Cfg<D> C;
   FwdParams p = pk;  // a variable-length batch rewrites the sizes and bases for its sequence below
   extern __shared__ __align__(16) unsigned char smem[];
@@ -456,12 +515,12 @@ __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_ker
     gload(vp, p.vs.s, it + 2, vreg);
   }
 
-  const float l_tot = halves_sum(rows.l_run), inv = 1.f / l_tot * F32_DOWN;
   float* const obase = (float*)p.out + b * p.os.b + h * p.os.h;
   float* const lbase = p.lse + ((int64_t)b * p.H + h) * p.lse_bh;
-  bool bad = qrow < p.Sq && rows.lost(rows.m_run);
-  if (qrow < p.Sq) {
+  bool bad = false;
+  auto store = [&](const f32x16 (&o)[D / 32], float m, float l, float down) {
     float* op = obase + (int64_t)row_of(qrow) * p.os.s;
+    const float inv = 1.f / l * down;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -469,28 +528,36 @@ __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : 2) flash_fwd32_ker
         f32x4 st;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          st[e] = rows.o[db][4 * g + e] * inv;
+          st[e] = o[db][4 * g + e] * inv;
           bad |= !(fabsf(st[e]) < INFINITY);
         }
         *(f32x4*)(op + db * 32 + 8 * g + 4 * hh) = st;
       }
-    if (hh == 0) lbase[stat_of(qrow)] = (rows.m_run * rows.c + fast_log2(l_tot)) * 0.6931471805599453f;
+    if (hh == 0) lbase[stat_of(qrow)] = (m * rows.c + fast_log2(l)) * 0.6931471805599453f;
+  };
+  const float l_tot = halves_sum(rows.l_run);
+  if (qrow < p.Sq) {
+    store(rows.o, rows.m_run, l_tot, F32_DOWN);
+    bad |= rows.lost(rows.m_run);
   }
   const uint64_t again = __builtin_amdgcn_ballot_w64(bad);
   if (again) {
-    __threadfence();  // (other lanes of this wave write those rows again)
-    plain_rows<D, 1>(p, (unsigned)(again | again >> 32), qw0, qp, kp, vp, obase, lbase, rows.c, lane, 0, row_of, stat_of);
+    const unsigned which = (unsigned)(again | again >> 32);
+    PlainRows<D> plain;
+    plain.run(p, which, qw0, qp, kp, vp, rows.c, lane, 0, 1, row_of);
+    const float l = halves_sum(plain.l);
+    if (which >> ln & 1) store(plain.o, plain.m, l, 1.f);
   }
 }
 
 // Few rows: a launch of the kernel above with fewer workgroups than CUs lasts as long as one wave's chain over all key tiles.
 // Here a workgroup owns 32 query rows and its NW waves take every NW-th key tile, straight from memory into operands (a lane
 // reads its own key's row of K, and a column of V 32 lanes wide per key) with no LDS and no barrier in the loop; the waves'
-// (O, m, l) are combined through LDS at the end.  Causal [1, 512, 32, 128] 83 -> 38 us, [1, 1697, 8, 64] 41.5 -> 37.
+// (O, m, l) are combined through LDS at the end.  Causal [1, 512, 32, 128] 82 -> 37 us, [1, 1697, 8, 64] 45 -> 39.
 template <int D, int NW>
 struct Fwd32SplitCfg {
   static constexpr int REC = 64 * (D / 8) * 4;               // floats of one wave's O
-  static constexpr int SMEM = NW * (REC + 128) * 4;
+  static constexpr int SMEM = (NW * (REC + 128) + NW) * 4;
 };
 
 template <int D, int NW>
@@ -577,63 +644,73 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
         }
   }
   // ---- combine: every wave leaves its unscaled O (lane-private order) and (m, l); wave j then finishes the
-  // 16-byte pieces j, j + NW, ... of every row ----
+  // 16-byte pieces j, j + NW, ... of every row (of `which`) ----
   constexpr int NPC = D / 8;  // 16-byte pieces per lane: (db, g)
-  const float l_own = halves_sum(rows.l_run);
-  float* const orec = sm + w * (C::REC + 128);
-#pragma unroll
-  for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      f32x4 st;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) st[e] = rows.o[db][4 * g + e];
-      *(f32x4*)(orec + ((db * 4 + g) * 64 + lane) * 4) = st;
-    }
-  if (hh == 0) {
-    orec[C::REC + ln] = rows.m_run;
-    orec[C::REC + 32 + ln] = l_own;
-  }
-  __syncthreads();
-  float mw[NW], m_all = -INFINITY;
-#pragma unroll
-  for (int j = 0; j < NW; ++j) {
-    mw[j] = sm[j * (C::REC + 128) + C::REC + ln];
-    m_all = fmaxf(m_all, mw[j]);
-  }
-  float aw[NW], l_all = 0.f;
-#pragma unroll
-  for (int j = 0; j < NW; ++j) {
-    aw[j] = mw[j] == -INFINITY ? 0.f : fast_exp2((mw[j] - m_all) * rows.c);  // a wave without a visible key
-    l_all += aw[j] * sm[j * (C::REC + 128) + C::REC + 32 + ln];
-  }
-  const float inv = 1.f / l_all * F32_DOWN;
   float* const obase = (float*)p.out + b * p.os.b + h * p.os.h;
   float* const lbase = p.lse + ((int64_t)b * p.H + h) * p.lse_bh;
-  bool bad = qrow < p.Sq && rows.lost(m_all);
-  if (qrow < p.Sq) {
-    float* const op = obase + (int64_t)row_of(qrow) * p.os.s;
-    for (int pc = w; pc < NPC; pc += NW) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  bool bad = false;
+  auto combine = [&](const f32x16 (&o)[D / 32], float m, float l, float down, unsigned which) {
+    float* const orec = sm + w * (C::REC + 128);
 #pragma unroll
-      for (int j = 0; j < NW; ++j) {
-        const f32x4 x = *(const f32x4*)(sm + j * (C::REC + 128) + (pc * 64 + lane) * 4);
+    for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] += aw[j] * x[e];
+      for (int g = 0; g < 4; ++g) {
+        f32x4 st;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[e] = o[db][4 * g + e];
+        *(f32x4*)(orec + ((db * 4 + g) * 64 + lane) * 4) = st;
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[e] *= inv;
-        bad |= !(fabsf(acc[e]) < INFINITY);
-      }
-      *(f32x4*)(op + (pc / 4) * 32 + 8 * (pc % 4) + 4 * hh) = acc;
+    if (hh == 0) {
+      orec[C::REC + ln] = m;
+      orec[C::REC + 32 + ln] = l;
     }
-    if (w == 0 && hh == 0) lbase[stat_of(qrow)] = (m_all * rows.c + fast_log2(l_all)) * 0.6931471805599453f;
-  }
+    __syncthreads();
+    float mw[NW], m_all = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < NW; ++j) {
+      mw[j] = sm[j * (C::REC + 128) + C::REC + ln];
+      m_all = fmaxf(m_all, mw[j]);
+    }
+    float aw[NW], l_all = 0.f;
+#pragma unroll
+    for (int j = 0; j < NW; ++j) {
+      aw[j] = mw[j] == -INFINITY ? 0.f : fast_exp2((mw[j] - m_all) * rows.c);  // a wave without a visible key
+      l_all += aw[j] * sm[j * (C::REC + 128) + C::REC + 32 + ln];
+    }
+    const float inv = 1.f / l_all * down;
+    if (qrow < p.Sq && (which >> ln & 1)) {
+      bad = rows.lost(m_all);
+      float* const op = obase + (int64_t)row_of(qrow) * p.os.s;
+      for (int pc = w; pc < NPC; pc += NW) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NW; ++j) {
+          const f32x4 x = *(const f32x4*)(sm + j * (C::REC + 128) + (pc * 64 + lane) * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[e] += aw[j] * x[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          acc[e] *= inv;
+          bad |= !(fabsf(acc[e]) < INFINITY);
+        }
+        *(f32x4*)(op + (pc / 4) * 32 + 8 * (pc % 4) + 4 * hh) = acc;
+      }
+      if (w == 0 && hh == 0) lbase[stat_of(qrow)] = (m_all * rows.c + fast_log2(l_all)) * 0.6931471805599453f;
+    }
+  };
+  combine(rows.o, rows.m_run, halves_sum(rows.l_run), F32_DOWN, ~0u);
   const uint64_t again = __builtin_amdgcn_ballot_w64(bad);
-  if (again) {
-    __threadfence();
-    plain_rows<D, NW>(p, (unsigned)(again | again >> 32), q0, qp, kp, vp, obase, lbase, rows.c, lane, w, row_of, stat_of);
+  unsigned* const flags = (unsigned*)(sm + NW * (C::REC + 128));
+  if (lane == 0) flags[w] = (unsigned)(again | again >> 32);
+  __syncthreads();
+  unsigned which = 0;
+#pragma unroll
+  for (int j = 0; j < NW; ++j) which |= flags[j];
+  if (__builtin_amdgcn_readfirstlane(which)) {
+    PlainRows<D> plain;
+    plain.run(p, which, q0, qp, kp, vp, rows.c, lane, w, NW, row_of);
+    combine(plain.o, plain.m, halves_sum(plain.l), 1.f, which);
   }
 }
 

@@ -131,3 +131,38 @@ def test_fp32_score_of_one_product_is_rounded_once(form, D):
     # 4 %); a second rounding would move 21 %.
     assert (lse != want).float().mean() < 0.1
     assert ((lse - want).abs() <= 2.0 ** -22 * want.abs()).all()
+
+
+@pytest.mark.parametrize("D,S,H", [(128, 1024, 32), (64, 1024, 16), (64, 512, 8), (32, 1000, 4)])
+@pytest.mark.parametrize("of,value", [("q", float("nan")), ("k", float("nan")), ("v", float("nan")), ("v", float("inf")), ("v", 3.4e38)])
+def test_fp32_rows_that_are_computed_again_cost_a_few_calls(D, S, H, of, value):
+    """A value that reaches every row: as many results again as the call has, at a few times its time (by one row after another: 80 to 250 times)."""
+    g = torch.Generator().manual_seed(D)
+    t = {n: torch.randn((1, S, H, D), generator=g) for n in "qkv"}
+    dev = {n: x.to(DEV) for n, x in t.items()}
+    bad = dev[of].clone()
+    bad[:, 3 if of != "q" else slice(None), :, 5] = value
+    seen = 3 if of != "q" else 0
+
+    def us(args):
+        best = float("inf")
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            out, lse = ops.flash_fwd(*args, None, True, layout="bshd")
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 1e3)
+        return best, out, lse
+    base, want, want_lse = us([dev[n] for n in "qkv"])
+    again, out, lse = us([bad if n == of else dev[n] for n in "qkv"])
+    assert again < 10 * base + 100, (base, again)
+    torch.testing.assert_close(out[:, :seen], want[:, :seen], rtol=1e-5, atol=1e-5)
+    if of == "v":
+        # the other columns are those of the finite value, to two of the bounds of test_fp32_against_float64 (a generous 1e-5 at values around 1)
+        keep = [d for d in range(D) if d != 5]
+        torch.testing.assert_close(out[..., keep], want[..., keep], rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(lse, want_lse, rtol=1e-5, atol=1e-5)
+        assert (out[:, 3:, :, 5].isnan() if value != value else out[:, 3:, :, 5] > 1e30).all()
+    else:
+        assert out[:, seen:].isnan().all() and lse[:, :, seen:].isnan().all()
