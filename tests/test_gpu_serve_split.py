@@ -1,10 +1,11 @@
 """Decode over ragged caches with the keys cut into chunks, and with neighbouring heads taken together: chunk edges, sequences without rows or
 keys, a longest sequence past the last chunk's even share, strides under which heads cannot be taken together; against the kernels that
-do neither (spa_tune few_rows)."""
+do neither (spa_tune few_rows), and these against float64 on the host."""
 import pytest
 import torch
 
 from conftest import rand_qkv
+from oracle import attn_oracle as O
 from sp_aurora_amd import _lib, ops
 from test_gpu_parity import DEV
 
@@ -51,6 +52,26 @@ def check(got, want, dtype):
     torch.testing.assert_close(got[1], want[1], atol=1e-3, rtol=1e-5)
 
 
+def exact(q, k, v, cu_q, cu_k, k_scale=None, v_scale=None):
+    """Every sequence by itself in float64; rows without keys: zeros and -inf."""
+    q, k, v = (t.cpu().double() for t in (q, k, v))
+    out, lse = torch.zeros_like(q), torch.full((q.shape[1], q.shape[0]), -float("inf"), dtype=torch.float64)
+    bounds = lambda cu: list(zip(cu.tolist(), cu.tolist()[1:]))
+    for i, ((a, b), (c, d)) in enumerate(zip(bounds(cu_q), bounds(cu_k))):
+        if a == b or c == d:
+            continue
+        x, y, z = (t.transpose(0, 1) for t in (q[a:b], k[c:d], v[c:d]))
+        y = y if k_scale is None else y * k_scale[i].cpu().double()[:, None, None]
+        z = z if v_scale is None else z * v_scale[i].cpu().double()[:, None, None]
+        s = x @ y.transpose(-1, -2) * q.shape[-1] ** -0.5
+        out[a:b], lse[:, a:b] = (torch.softmax(s, -1) @ z).transpose(0, 1), torch.logsumexp(s, -1)
+    return out, lse
+
+
+def check_exact(got, want, dtype):
+    check([t.cpu().double() for t in got], want, dtype)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
 @pytest.mark.parametrize("chunk", [1, 64, 257, 512])
@@ -61,6 +82,7 @@ def test_chunks_of_ragged_caches(H, reps, chunk, D, dtype, fp8):
     q, k, v, cu_q, cu_k, scales = caches(lens, H, D, dtype, fp8, 1000 + chunk)
     max_k = max(n for n, _ in lens)
     want = reference(q, k, v, cu_q, cu_k, 3, max_k, **scales)
+    check_exact(want, exact(q, k, v, cu_q, cu_k, **scales), dtype)
     check(split(q, k, v, cu_q, cu_k, 3, max_k, chunk, **scales), want, dtype)
     check(ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 3, max_k, **scales), want, dtype)  # (not split: heads together where there are enough)
 
@@ -72,6 +94,7 @@ def test_suggested_chunks_and_capture(nseq, longest):
     q, k, v, cu_q, cu_k, _ = caches(lens, H, D, dtype, False, 1100)
     assert _lib.load().spa_flash_fwd_varlen_splitkv_suggest(nseq, H, k.shape[0], 1, longest, D, _lib.SPA_BF16) > 0
     want = reference(q, k, v, cu_q, cu_k, 1, longest)
+    check_exact(want, exact(q, k, v, cu_q, cu_k), dtype)
     check(ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 1, longest), want, dtype)
     check(ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 1, k.shape[0]), want, dtype)  # a bound that no sequence is near
     graph = torch.cuda.CUDAGraph()
@@ -104,6 +127,9 @@ def test_heads_taken_together_at_a_fixed_length(rows, D, fp8):
         want = ops.flash_fwd(q, k, v, layout="bshd", **scales)
     finally:
         _lib.tune("few_rows", 0)
+    scale = lambda t: 1.0 if t is None else t[:, None, :, None].cpu().double()
+    y, z = k.cpu().double() * scale(scales.get("k_scale")), v.cpu().double() * scale(scales.get("v_scale"))
+    check_exact(want, O.full_attention(q.cpu(), y, z, None, False), dtype)
     for x in (got, single, mixed):
         check(x, want, dtype)
 

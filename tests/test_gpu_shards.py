@@ -1,12 +1,15 @@
 """Attention over sequences whose rows lie in shards (rank-stacked tensors, zigzag rings, packed batches of shards): segments
-shorter and longer than a tile and around its size, every form of the kernels, against the call on the rows in order."""
+shorter and longer than a tile and around its size, every form of the kernels, against the call on the rows in order, which is itself
+compared with float64 on the host."""
 import pytest
 import torch
 
 from conftest import rand_qkv
+from oracle import attn_oracle as O
 import sp_aurora_amd as spa
 from sp_aurora_amd import _lib
-from test_gpu_parity import DEV
+from test_gpu_many_sequences import reference as packed_reference
+from test_gpu_parity import DEV, check_grad, check_out
 
 pytestmark = pytest.mark.gpu
 TOL = {torch.bfloat16: 2e-2, torch.float16: 4e-3, torch.float32: 1e-5}
@@ -22,6 +25,12 @@ def step(fn, leaves, dout):
     return (out.detach(), *torch.autograd.grad(out, leaves, dout))
 
 
+def check_step(got, out, grads, dtype):
+    check_out(got[0], out, dtype)
+    for name, g, w in zip("qkv", got[1:], grads):
+        check_grad(g, w, dtype, "d" + name)
+
+
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 64), (torch.float32, 32)])
 @pytest.mark.parametrize("P,seg", [(2, 1), (8, 17), (3, 63), (4, 64), (5, 65), (2, 200)])
 def test_segments_around_the_tile_size(P, seg, dtype, D):
@@ -30,12 +39,15 @@ def test_segments_around_the_tile_size(P, seg, dtype, D):
     stack = lambda t: torch.stack(t.chunk(P, 1)).contiguous()
     unstack = lambda t: torch.cat(list(t), 1)
     layer = spa.LongContextAttention(sp_ulysses_degree=1, sp_ring_degree=P)
+    host = [t.cpu() for t in (q, k, v, dout)]
+    exact = {c: (O.full_attention(*host[:3], None, c)[0], O.attn_backward_autograd(*host, None, c)) for c in (True, False)}
     for form in FORMS if dtype != torch.float32 else FORMS[:1]:
         try:
             for knob, value in form.items():
                 _lib.tune(knob, value)
             for causal in (True, False):
                 want = step(lambda *x: spa.sp_aurora_func(*x, causal=causal), [t.clone().requires_grad_() for t in (q, k, v)], dout)
+                check_step(want, *exact[causal], dtype)
                 got = step(lambda *x: layer(*x, causal=causal), [stack(t).requires_grad_() for t in (q, k, v)], stack(dout))
                 for g, w in zip(got, want):
                     close(unstack(g), w, 2 * TOL[dtype])
@@ -73,5 +85,6 @@ def test_packed_batches_of_shards(dtype, D, zigzag):
     want = step(lambda *x: spa.sp_aurora_varlen_func(*x, cu_all, max_seqlen=max(lens), causal=True), [t.clone().requires_grad_() for t in (q, k, v)], dout)
     got = step(lambda *x: spa.sp_aurora_varlen_func(*x, cu, max_seqlen=max(local), causal=True, ring_size=P, sharding="zigzag" if zigzag else "contiguous"),
                [t[idx].requires_grad_() for t in (q, k, v)], dout[idx])
+    check_step(want, *packed_reference(*(t.cpu() for t in (q, k, v, dout)), lens), dtype)
     for g, w in zip(got, want):
         close(g, w[idx], 2 * TOL[dtype])
