@@ -1351,6 +1351,9 @@ __global__ void __launch_bounds__(BWD_THREADS, 1) flash_bwd32_dkdv_kernel(const 
   }
 }
 
+// Query rows of the longest sequence (of a packed batch in shards Sq is what lies in one of them).
+int64_t longest_rows(const BwdParams& p) { return (int64_t)p.Sq * (p.cu_q && p.map.P ? p.map.P : 1); }
+
 // `rows` query rows, or keys, per workgroup.
 template <auto kernel>
 hipError_t launch(int smem, bool queries, int rows, BwdParams p, hipStream_t stream, int threads = BWD_THREADS) {
@@ -1358,7 +1361,7 @@ hipError_t launch(int smem, bool queries, int rows, BwdParams p, hipStream_t str
   if (e != hipSuccess) return e;
   dim3 grid;
   if (p.cu_q) {
-    const int64_t longest = (int64_t)(queries ? p.Sq : p.Sk) * (p.map.P ? p.map.P : 1);
+    const int64_t longest = queries ? longest_rows(p) : (int64_t)p.Sk * (p.map.P ? p.map.P : 1);
     if (!spa_varlen_grid(p.H, p.B, queries ? p.lse_bh : p.total_k, longest, rows, 1, grid, p.numbered)) return hipErrorInvalidValue;
   } else {
     const int tiles = ((queries ? p.Sq : p.Sk) + rows - 1) / rows;
@@ -1381,7 +1384,7 @@ hipError_t launch_both(const BwdParams& p, hipStream_t stream) {
   hipError_t e = hipErrorInvalidValue;
   bool wide = false;
   if constexpr (D == 128 && ADDR != ADDR_BIG) {
-    wide = forced ? forced == 8 : wgs8 >= spa_device_cus() && p.Sq > 128;
+    wide = forced ? forced == 8 : wgs8 >= spa_device_cus() && longest_rows(p) > 128;
     if (wide) e = launch<flash_bwd_dq_kernel<T, D, 8, ADDR>>(DqCfg<D, 8>::SMEM, true, 256, p, stream, 512);
   }
   if (!wide) e = launch<flash_bwd_dq_kernel<T, D, 4, ADDR>>(DqCfg<D, 4>::SMEM, true, 128, p, stream);
