@@ -31,8 +31,9 @@ __device__ __forceinline__ void split2(float x0, float x1, unsigned& h, unsigned
   l = M::pack2(r0 - __builtin_bit_cast(float, m << 16), r1 - __builtin_bit_cast(float, m & 0xffff0000u));
 }
 // Eight values as three operands.  They are taken times 2^24: the lowest bit of any fp32 number, denormals included, is then a normal
-// bf16 number, where the low terms of values below 2^-110 would be cut off (relative errors of 3e-6 at 1e-35, 3e-3 at 1e-38; the factors cost 3 % of
-// the times below at D = 128, 7 % at the smaller ones).
+// bf16 number, where the low terms of values below 2^-110 would be cut off (relative errors of 3e-6 at 1e-35, 3e-3 at 1e-38).  The factors and the
+// look at the results cost 5 % at D <= 64 and in the kernel for few rows (causal, us: [1, 4096, 16, 64] 216 -> 228, [1, 512, 32, 128] 38.3 -> 40.5); at
+// D = 128 the two accumulators of a score give it back ([1, 4096, 32, 128] 749 -> 741).
 constexpr float F32_UP = 0x1p24f, F32_DOWN = 0x1p-48f;  // F32_DOWN: of a product of two
 struct Split8 {
   u32x4 h, m, l;
