@@ -464,6 +464,12 @@ bool scale_arg(PyObject* o, double& x) {
   }
   return std::isfinite(x);
 }
+bool int_arg(PyObject* o, int64_t& x) {  // (a number past 64 bits is the Python path's)
+  if (!PyLong_Check(o)) return false;
+  int past = 0;
+  x = PyLong_AsLongLongAndOverflow(o, &past);
+  return past == 0;
+}
 bool flag_arg(PyObject* o) {
   const int r = PyObject_IsTrue(o);
   if (r < 0) throw python_error();
@@ -482,15 +488,15 @@ PyObject* py_flash_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Tensor q, k, v, qs, ks, vs, out, lse;
   double scale;
+  int64_t out_dtype;
   if (n != 10 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !scale_arg(a[3], scale) || !optional_tensor(a[6], qs) ||
-      !optional_tensor(a[7], ks) || !optional_tensor(a[8], vs))
+      !optional_tensor(a[7], ks) || !optional_tensor(a[8], vs) || !int_arg(a[9], out_dtype))
     Py_RETURN_NONE;
   const bool causal = flag_arg(a[4]), bshd = flag_arg(a[5]);
-  const int out_dtype = (int)PyLong_AsLong(a[9]);
   bool done;
   {
     pybind11::gil_scoped_release no_gil;
-    done = flash_fwd(q, k, v, scale, causal, bshd, qs, ks, vs, out_dtype, out, lse);
+    done = flash_fwd(q, k, v, scale, causal, bshd, qs, ks, vs, (int)out_dtype, out, lse);
   }
   if (!done) Py_RETURN_NONE;
   return pair(out, lse);
@@ -502,10 +508,10 @@ PyObject* py_varlen_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Tensor q, k, v, cq, ck, ks, vs, out, lse;
   double scale;
+  int64_t mq, mk;
   if (n != 11 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], cq) || !tensor_arg(a[4], ck) ||
-      !PyLong_Check(a[5]) || !PyLong_Check(a[6]) || !scale_arg(a[7], scale) || !optional_tensor(a[9], ks) || !optional_tensor(a[10], vs))
+      !int_arg(a[5], mq) || !int_arg(a[6], mk) || !scale_arg(a[7], scale) || !optional_tensor(a[9], ks) || !optional_tensor(a[10], vs))
     Py_RETURN_NONE;
-  const int64_t mq = PyLong_AsLongLong(a[5]), mk = PyLong_AsLongLong(a[6]);
   const bool causal = flag_arg(a[8]);
   bool done = false;
   if (mq > 0 && mk > 0 && mq <= 0x7fffffffLL && mk <= 0x7fffffffLL) {
@@ -525,8 +531,8 @@ PyObject* attention(PyObject* const* a, std::index_sequence<I...>) {
   double scale;
   for (int i = 0; i < N; ++i)
     if (!tensor_arg(a[i], t[i])) Py_RETURN_NONE;
-  if (!scale_arg(a[N], scale) || !PyLong_Check(a[N + 2])) Py_RETURN_NONE;
-  const int64_t zigzag = PyLong_AsLongLong(a[N + 2]);
+  int64_t zigzag;
+  if (!scale_arg(a[N], scale) || !int_arg(a[N + 2], zigzag)) Py_RETURN_NONE;
   if (zigzag < 0 || zigzag > 0x3fffffffLL || transformed(t, N) || !attention_ok(t, N, zigzag)) Py_RETURN_NONE;
   const bool causal = flag_arg(a[N + 1]);
   variable_list r;
@@ -559,12 +565,11 @@ PyObject* py_varlen_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Tensor t[5];
   double scale;
-  if (n != 12 || !PyLong_Check(a[10])) Py_RETURN_NONE;
+  int64_t mq, mk, shards;
+  if (n != 12 || !int_arg(a[10], shards)) Py_RETURN_NONE;
   for (int i = 0; i < 5; ++i)
     if (!tensor_arg(a[i], t[i])) Py_RETURN_NONE;
-  if (!PyLong_Check(a[5]) || !PyLong_Check(a[6]) || !scale_arg(a[7], scale)) Py_RETURN_NONE;
-  const int64_t mq = PyLong_AsLongLong(a[5]), mk = PyLong_AsLongLong(a[6]);
-  const int64_t shards = PyLong_AsLongLong(a[10]);
+  if (!int_arg(a[5], mq) || !int_arg(a[6], mk) || !scale_arg(a[7], scale)) Py_RETURN_NONE;
   const bool causal = flag_arg(a[8]), covered = flag_arg(a[9]), zigzag = flag_arg(a[11]);
   if (transformed(t, 3) || !differentiable_ok(t, 3) || !cu_ok(t[3], t[0]) || !cu_ok(t[4], t[0]) || mq <= 0 || mk <= 0 || mq > 0x7fffffffLL || mk > 0x7fffffffLL ||
       shards < 1 || shards > 0xffffLL)

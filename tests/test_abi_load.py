@@ -343,3 +343,16 @@ def test_offsets_are_looked_at_again_when_another_array_takes_the_address():
     big[1:3] = torch.tensor([5, 10])
     held = len(ops._CU_CHECKED)
     assert ops.check_cu_seqlens_once(big[:3], 10, 9, "cu") and len(ops._CU_CHECKED) == held
+
+
+def test_a_number_past_64_bits_is_the_python_paths():
+    """A bound or ring size that no 64-bit number holds: the native calls leave it to the Python functions, without a pending error."""
+    import torch
+    nat, huge = _lib.native(), 2 ** 70
+    x, cu = torch.zeros(4, 2, 64), torch.tensor([0, 4], dtype=torch.int32)
+    for bounds in ((huge, 4), (4, huge), (-huge, 4)):
+        assert nat.varlen_attention(x, x, x, cu, cu, *bounds, None, True, True, 1, False) is None
+        assert nat.varlen_fwd(x, x, x, cu, cu, *bounds, None, True, None, None) is None
+    assert nat.varlen_attention(x, x, x, cu, cu, 4, 4, None, True, True, huge, False) is None
+    assert nat.attention(x[None], x[None], x[None], None, True, huge) is None
+    assert nat.flash_fwd(x[None], x[None], x[None], None, True, True, None, None, None, huge) is None
