@@ -24,7 +24,8 @@
 // [2,4096,32,64] causal backward 582 -> 480 us, [64,512,16,64] 312 -> 243 us.
 // Software-pipelined inside the wave at half-tile (32 rows) granularity:
 // the MFMAs that produce S and dP of half-tile g+1 are interleaved, one to one, with the
-// element-wise work (exp, dS) on half-tile g, followed by the gradient MFMAs of half-tile g.
+// element-wise work (exp, dS) on half-tile g, followed by the gradient MFMAs of half-tile g; in the dk/dv kernel the
+// gradient MFMAs stand between the others as well, so that vector work and matrix work are spread alike over the whole pass.
 // MFMA operands come from LDS through a rolling window that runs ahead of the MFMAs and is
 // carried across loop iterations; one workgroup barrier per 64-row tile.
 // Accumulators are fp32 in HBM and are ADDED to (read-modify-write by the owning lane).
@@ -193,7 +194,7 @@ __device__ __forceinline__ void wait_loads_but() {  // until at most N of this w
 // (touched by MFMAs only) in AGPRs, the S / dP tiles, which the VALU works on, in VGPRs, so that
 // no v_accvgpr_read / v_accvgpr_write copies are needed between the matrix pipe and the VALU.
 // The compiler does not see these as MFMAs: the code keeps the distances the hardware needs
-// (a VALU read of a tile comes at least 16 MFMAs after the tile's last MFMA; srcC is the
+// (a VALU read of a tile comes at least 5 MFMAs after the tile's last MFMA; srcC is the
 // destination itself or the literal 0, never a register a VALU instruction has just written).
 template <typename T>
 struct MmaAsm;
@@ -640,7 +641,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
   typedef DkvCfg<D> G;
   typedef Mma16<T> M;
   typedef MmaAsm<T> MA;
-  constexpr bool MIXED = D == 128 && ASM;  // see the dq kernel; here 16 gradient MFMAs separate a tile's MFMAs from its VALU reads
+  constexpr bool MIXED = D == 128 && ASM;  // see the dq kernel; here 5 gradient MFMAs separate a tile's MFMAs from its VALU reads
   typedef typename M::frag frag;
   extern __shared__ __align__(16) unsigned char smem[];
 
@@ -723,12 +724,19 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     zero16(dv[i]);
   }
 
-  // Half-tile g = 2 i + t is query rows [32 g, 32 g + 32).  Body of tile i:
-  //   list 2i  : S, dP of half 2i+1 (tile i rows 32..63)  | P, dS of half 2i   | dV, dK from half 2i
-  //   list 2i+1: S, dP of half 2i+2 (tile i+1 rows 0..31) | P, dS of half 2i+1 | dV, dK from half 2i+1
-  constexpr int NA = 2 * (D / 16), NB = 4 * (D / 32), NLIST = NA + NB, NBODY = 2 * NLIST;
+  // Half-tile g = 2 i + t is query rows [32 g, 32 g + 32).  Three of them are in work at any time: while the matrix pipe forms S and
+  // dP of half g + 1 and the products of half g - 1 or g with the keys' gradients, the vector unit forms P and dS of half g.  The
+  // matrix instructions come in groups of GROUP, each with the vector work on 8 of the lane's 16 rows between them (one wave a SIMD issues one
+  // instruction every four clocks: with all vector work beside the 16 MFMAs of S and dP, a tile's 64 MFMAs, 2048 clocks, took 3660, 22 % of
+  // them waiting for LDS; spread over all of them, with lse read a group ahead and no drained window at the barrier, 3310.  What is
+  // gained is less, as the board lowers its clock with the matrix pipe's share: causal [1, 16384, 16, 128] dk/dv 2.17 -> 2.07 ms):
+  //   first group of half g : S, dP of half g + 1, contraction steps 0 .. HS - 1  | P, dS of g, rows 0 .. 7  | dV, dK from g - 1, rows 8 .. 15
+  //   second group          : S, dP of half g + 1, steps HS .. 2 HS - 1           | rows 8 .. 15             | dV, dK from g, rows 0 .. 7
+  // One pass of the loop runs the second group of half 2 i, both groups of half 2 i + 1 and the first of half 2 i + 2, so that it
+  // reads tiles i and i + 1 only.
+  constexpr int HS = D / 32, GROUP = 4 * HS, NBODY = 4 * GROUP;
   constexpr int BWD_LOOK = D <= 64 ? 4 : BWD_LOOK_MAX;  // (two waves per SIMD at D <= 64, as in the dq kernel)
-  static_assert(NBODY % BWD_LOOK == 0 && BWD_LOOK <= NA, "the operand window must tile the loop body");
+  static_assert(GROUP % BWD_LOOK == 0, "the operand window must tile a group");
 
   if (it0 < nt) {  // uniform; a workgroup whose keys no query sees adds nothing
     // the workgroup's keys first, as two tiles each of K and V in the stages of tiles it0 + 2 and it0 + 3
@@ -759,138 +767,186 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     wait_loads_but<2 * G::NL>();
     __syncthreads();
 
-    f32x16 sc, dc, sn, dn;
-    {
-      const unsigned qb = stage_of(it0);
+    // V negated: with delta as the accumulator's start the products give delta - dP, and -dS costs one multiplication per element.
 #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) {
-        const frag a0 = as_frag<frag>(lds_read_b128(qb + rd.row[ks]));
-        const frag a1 = as_frag<frag>(lds_read_b128(qb + C::TILEB + rd.row[ks]));
-        if (!MIXED) {
-          if (ks == 0) {
-            zero16(sc);
-            zero16(dc);
-          }
-          sc = M::run(a0, kf[ks], sc);
-          dc = M::run(a1, vf[ks], dc);
-        } else if (ks == 0) {
-          MA::first_v(sc, a0, kf[0]);
-          MA::first_v(dc, a1, vf[0]);
-        } else {
-          MA::acc_v(sc, a0, kf[ks]);
-          MA::acc_v(dc, a1, vf[ks]);
-        }
-      }
+    for (int ks = 0; ks < D / 16; ++ks) {
+      u32x4 x = __builtin_bit_cast(u32x4, vf[ks]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] ^= 0x80008000u;
+      vf[ks] = as_frag<frag>(x);
     }
 
-    unsigned row_cur[D / 16], row_nxt[D / 16], tr_cur[D / 32][2];
-    unsigned stat_cur;
-    auto set_addresses = [&](int i) {
-      const unsigned a = stage_of(i), n = stage_of(i + 1);
+    // Per-lane LDS addresses of the operands; each is moved on to the next tile where that tile is first read through it.
+    unsigned row_at[D / 16], tr_at[D / 32][2], stat_at = stage_of(it0) + 2 * C::TILEB + 16 * hh;
+    unsigned step = 0, last_step = 0;  // from tile i to i + 1, from i - 1 to i
 #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) {
-        row_cur[ks] = a + rd.row[ks];
-        row_nxt[ks] = n + rd.row[ks];
-      }
+    for (int ks = 0; ks < D / 16; ++ks) row_at[ks] = stage_of(it0) + rd.row[ks];
 #pragma unroll
-      for (int db = 0; db < D / 32; ++db)
+    for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-        for (int h8 = 0; h8 < 2; ++h8) tr_cur[db][h8] = a + rd.tr[db][h8];
-      stat_cur = a + 2 * C::TILEB + 16 * hh;
-    };
-    auto fetch = [&](int J) -> frag {
-      const int body = J / NBODY, j2 = J % NBODY;
-      const int list = j2 / NLIST, j = j2 % NLIST;
-      if (j < NA) {  // j = 2 ks + which: Q row (S) or dO row (dP) of the half-tile being produced
-        const int ks = j >> 1, which = j & 1;
-        const unsigned base = (body == 0 && list == 0) ? row_cur[ks] + 32 * C::ROWB
-                              : (body == 0)           ? row_nxt[ks]
-                                                      : row_nxt[ks] + 32 * C::ROWB;
-        return as_frag<frag>(lds_read_b128(base + which * C::TILEB));
-      }
-      // jb = (u * (D/32) + db) * 2 + which: dO^T (for dV) or Q^T (for dK) operand of half-tile `list`
-      const int jb = j - NA;
-      const int which = jb & 1, db = (jb >> 1) % (D / 32), u = (jb >> 1) / (D / 32);
-      const unsigned off = (which ? 0 : C::TILEB) + (list * 32 + u * 16) * C::ROWB;
-      return frag_tr<frag>(tr_cur[db][0] + off, tr_cur[db][1] + off);
+      for (int h8 = 0; h8 < 2; ++h8) tr_at[db][h8] = stage_of(it0) + rd.tr[db][h8];
+    auto advance = [&](unsigned& at, unsigned by) {
+      at += by;
+      asm volatile("" : "+v"(at));  // (kept, not formed again from the tile's number at every use)
     };
 
-    frag win[BWD_LOOK];
+    f32x16 sc, dc, sn, dn;  // S and delta - dP of the current / next half-tile, then P and -dS
     frag pf[2], dsf[2];
-    set_addresses(it0);
+    u32x4 pw, dsw;
+    f32x4 ln_raw[2], ln_cur[2];  // lse of the 8 rows of the next / the current group
+    auto load_lse = [&](f32x4 (&l)[2], unsigned at, int row) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) l[g] = __builtin_bit_cast(f32x4, lds_read_b128(at + (row + 8 * g) * 4));
+    };
+    auto load_delta = [&](f32x16& x, unsigned at, int row) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 d4 = __builtin_bit_cast(f32x4, lds_read_b128(at + (BWD_ROWS + row + 8 * g) * 4));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[4 * g + e] = d4[e];
+      }
+    };
+    // diagonal: a key sees only the queries at or after it
+    auto mask = [&](int half) {
+      const int r0 = half * 32;
+      if (p.causal && kw0 + 31 > r0) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          if (krow > r0 + 8 * (v >> 2) + 4 * hh + (v & 3)) sc[v] = hidden;
+      }
+    };
+    // part n of the vector work of a group on rows 8 u .. 8 u + 7 of the lane's 16: two parts per row
+    // (pinned by the empty asm: left alone, the compiler moves all of it behind the next branch)
+    float pr[8], ds[8];
+    auto element = [&](int u, int n) {
+      const int e = n >> 1, v = 8 * u + e;
+      if ((n & 1) == 0) {
+        pr[e] = fast_exp2(__builtin_fmaf(sc[v], c, ln_cur[e >> 2][e & 3] * -1.4426950408889634f));
+        asm volatile("" : "+v"(pr[e]));
+      } else {
+        ds[e] = dc[v] * pr[e];
+        asm volatile("" : "+v"(ds[e]));
+        if (e & 1) {
+          pw[e >> 1] = M::pack2(pr[e - 1], pr[e]);
+          dsw[e >> 1] = M::pack2(ds[e - 1], ds[e]);
+        }
+        if (e == 7) {
+          pf[u] = as_frag<frag>(pw);
+          dsf[u] = as_frag<frag>(dsw);
+          asm volatile("" : "+v"(pf[u]), "+v"(dsf[u]));
+        }
+      }
+    };
+    auto mma_s = [&](f32x16& x, frag a, int ks) {
+      if (!MIXED) {
+        if (ks == 0) zero16(x);
+        x = M::run(a, kf[ks], x);
+      } else if (ks == 0) {
+        MA::first_v(x, a, kf[0]);
+      } else {
+        MA::acc_v(x, a, kf[ks]);
+      }
+    };
+    auto mma_d = [&](f32x16& x, frag a, int ks) {
+      if (MIXED)
+        MA::acc_v(x, a, vf[ks]);
+      else
+        x = M::run(a, vf[ks], x);
+    };
+
+    // Matrix instruction n of a group: 0 .. KS - 1: S, contraction step; KS .. : dP; 2 KS ..: gradient product number.  The gradient
+    // products, which do not wait for this group's vector work, stand between the others; the last of S and dP is at least
+    // five matrix instructions before the first vector instruction that reads it.
+    constexpr int KS = D / 16;
+    auto instruction = [](bool first, int n) -> int {
+      if (first) {
+        const int k = n >> 1;
+        return (n & 1) ? 2 * KS + k : k < HS ? k : KS + k - HS;
+      }
+      if (n >= 3 * HS) return 2 * KS + n - 2 * HS;
+      const int k = n / 3, what = n % 3;
+      return what == 2 ? 2 * KS + k : what * KS + HS + k;
+    };
+    // operand number J of the pass on tile i (J >= NBODY: the first operands of the next pass)
+    auto fetch = [&](int J) -> frag {
+      const int group = J % NBODY / GROUP;
+      const int n = instruction(group & 1, J % GROUP);
+      if (n < 2 * KS) {  // row of Q (S) or dO (dP) of the half-tile being produced
+        const int ks = n % KS, which = n / KS;
+        if ((group == 1 || group == 2) && which == 0) advance(row_at[ks], step);
+        return as_frag<frag>(lds_read_b128(row_at[ks] + (group == 1 || group == 2 ? 0 : 32 * C::ROWB) + which * C::TILEB));
+      }
+      // jb = db * 2 + which: dO^T (for dV) or Q^T (for dK) of the 16 rows whose P and dS are used
+      const int jb = n - 2 * KS, which = jb & 1, db = jb >> 1;
+      if (group == 0 && which == 0) {
+#pragma unroll
+        for (int h8 = 0; h8 < 2; ++h8) advance(tr_at[db][h8], J >= NBODY ? step : last_step);
+      }
+      const unsigned off = (which ? 0 : C::TILEB) + 16 * group * C::ROWB;
+      return frag_tr<frag>(tr_at[db][0] + off, tr_at[db][1] + off);
+    };
+
+    // Before the loop: S, dP of half 0 and what the first group of half 0 would do, less the gradients of a half before it.
+    load_lse(ln_cur, stat_at, 0);
+    load_lse(ln_raw, stat_at, 16);
+    load_delta(dc, stat_at, 0);
+    load_delta(dn, stat_at, 32);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      mma_s(sc, as_frag<frag>(lds_read_b128(row_at[ks])), ks);
+      mma_d(dc, as_frag<frag>(lds_read_b128(row_at[ks] + C::TILEB)), ks);
+    }
+#pragma unroll
+    for (int ks = 0; ks < HS; ++ks) {
+      mma_s(sn, as_frag<frag>(lds_read_b128(row_at[ks] + 32 * C::ROWB)), ks);
+      mma_d(dn, as_frag<frag>(lds_read_b128(row_at[ks] + 32 * C::ROWB + C::TILEB)), ks);
+    }
+    frag win[BWD_LOOK];
 #pragma unroll
     for (int j = 0; j < BWD_LOOK; ++j) win[j] = fetch(j);
+    if (MIXED) mfma_settle();
+    mask(2 * it0);
+#pragma unroll
+    for (int n = 0; n < 16; ++n) element(0, n);
+
     // The loads of tile i + 3 go out one at a time between the MFMAs of the pass: issued in one
     // burst after the barrier, they hold up the wave's instruction stream while the memory pipeline
     // takes them in.
     constexpr int LOAD_GAP = NBODY / G::NL;
     for (int i = it0; i < nt;) {
+      // tile i + 1 has landed; every wave is done with tile i - 1.  The operands in flight are of tile i, so nothing else is waited for.
       wait_loads_but<G::NL>();
-      __syncthreads();
-      set_addresses(i);
+      if (MIXED)
+        __builtin_amdgcn_s_barrier();
+      else
+        __syncthreads();
+      last_step = step;
+      step = stage_of(i + 1) - stage_of(i);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int list = 0; list < 2; ++list) {
-        const int r0 = (2 * i + list) * 32;  // first query row of the half-tile whose P, dS are formed here
-        if (p.causal && kw0 + 31 > r0) {     // diagonal: a key sees only the queries at or after it
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            if (krow > r0 + 8 * (v >> 2) + 4 * hh + (v & 3)) sc[v] = hidden;
-        }
-        // lse (times -log2 e) and delta of this lane's 16 query rows
-        float nl[16], de[16];
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          // (whole-vector casts: a bit cast of one element of a vector reads element 0)
-          const f32x4 l4 = __builtin_bit_cast(f32x4, lds_read_b128(stat_cur + (list * 32 + 8 * g4) * 4));
-          const f32x4 d4 = __builtin_bit_cast(f32x4, lds_read_b128(stat_cur + (BWD_ROWS + list * 32 + 8 * g4) * 4));
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            nl[4 * g4 + e] = l4[e] * -1.4426950408889634f;
-            de[4 * g4 + e] = d4[e];
-          }
-        }
-        if (!MIXED) {
-          zero16(sn);
-          zero16(dn);
-        }
+      for (int group = 0; group < 4; ++group) {
+        // half-tile of the vector work
+        if (group & 1) mask(2 * i + (group + 1) / 2);
+        ln_cur[0] = ln_raw[0];
+        ln_cur[1] = ln_raw[1];
+        if (group == 2) stat_at += step;
+        // the next group's lse rows; what dP of the half-tile in production starts from
+        if (group & 1) load_delta(dn, group == 1 ? stat_at + step : stat_at, group == 1 ? 0 : 32);
+        load_lse(ln_raw, stat_at, group == 0 ? 32 : group == 1 ? 48 : group == 2 ? 0 : 16);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < NLIST; ++j) {
-          const int J = list * NLIST + j;
+        for (int m = 0; m < GROUP; ++m) {
+          const int J = group * GROUP + m;
           const frag a = win[J % BWD_LOOK];
           win[J % BWD_LOOK] = fetch(J + BWD_LOOK);
           __builtin_amdgcn_sched_barrier(0);
-          if (j < NA) {
-            const int ks = j >> 1;
-            if (!MIXED) {
-              if (j & 1)
-                dn = M::run(a, vf[ks], dn);
-              else
-                sn = M::run(a, kf[ks], sn);
-            } else if (j & 1) {
-              if (ks == 0) MA::first_v(dn, a, vf[0]); else MA::acc_v(dn, a, vf[ks]);
-            } else {
-              if (ks == 0) MA::first_v(sn, a, kf[0]); else MA::acc_v(sn, a, kf[ks]);
-            }
-#pragma unroll
-            for (int v = 0; v < 16; ++v)
-              if (v * NA / 16 == j) {
-                const float pr = fast_exp2(__builtin_fmaf(sc[v], c, nl[v]));
-                sc[v] = pr;
-                dc[v] = pr * (dc[v] - de[v]);
-              }
-            if (j == NA / 2 - 1) {
-              pf[0] = M::pack(sc[0], sc[1], sc[2], sc[3], sc[4], sc[5], sc[6], sc[7]);
-              dsf[0] = M::pack(dc[0], dc[1], dc[2], dc[3], dc[4], dc[5], dc[6], dc[7]);
-            }
-            if (j == NA - 1) {
-              pf[1] = M::pack(sc[8], sc[9], sc[10], sc[11], sc[12], sc[13], sc[14], sc[15]);
-              dsf[1] = M::pack(dc[8], dc[9], dc[10], dc[11], dc[12], dc[13], dc[14], dc[15]);
-            }
+          const int n = instruction(group & 1, m);
+          if (n < KS) {
+            mma_s(sn, a, n);
+          } else if (n < 2 * KS) {
+            mma_d(dn, a, n - KS);
           } else {
-            const int jb = j - NA;
-            const int which = jb & 1, db = (jb >> 1) % (D / 32), u = (jb >> 1) / (D / 32);
+            const int jb = n - 2 * KS, which = jb & 1, db = jb >> 1, u = group & 1;
             if (!MIXED) {
               if (which)
                 dk[db] = M::run(a, dsf[u], dk[db]);
@@ -902,11 +958,16 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
               MA::acc_a(dv[db], a, pf[u]);
             }
           }
+          // rows 8 .. 15 in the second group of a half-tile, 0 .. 7 in the first
+#pragma unroll
+          for (int e = m * 16 / GROUP; e < (m + 1) * 16 / GROUP; ++e) element(group & 1 ? 0 : 1, e);
           if (J % LOAD_GAP == LOAD_GAP / 2 && J / LOAD_GAP < G::NL) issue_one(i + 3, J / LOAD_GAP);
           __builtin_amdgcn_sched_barrier(0);
         }
-        sc = sn;
-        dc = dn;
+        if (!(group & 1)) {
+          sc = sn;
+          dc = dn;
+        }
       }
       if (++i == nt) mfma_settle();
     }
@@ -918,12 +979,13 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     asm volatile("s_nop 15\n s_nop 15"
                  : "+a"(dk[0]), "+a"(dk[1]), "+a"(dk[2]), "+a"(dk[3]), "+a"(dv[0]), "+a"(dv[1]), "+a"(dv[2]), "+a"(dv[3])::"memory");
 
+  const float dk_scale = -p.scale;  // (-dS, see the loop)
   if (p.grads_in_t) {
     __syncthreads();  // every wave is done with the tiles, and with its loads into them
     T* const dkp = (T*)p.dk + b * p.dks.b + h * p.dks.h;
     T* const dvp = (T*)p.dv + b * p.dvs.b + h * p.dvs.h;
     store_rows<T, D>(dv, 1.f, [&](int r) { return dvp + (int64_t)row_of(kw0 + r) * p.dvs.s; }, p.Sk - kw0, smem + w * (64 * C::ROWB), lane);
-    store_rows<T, D>(dk, p.scale, [&](int r) { return dkp + (int64_t)row_of(kw0 + r) * p.dks.s; }, p.Sk - kw0, smem + w * (64 * C::ROWB) + 32 * C::ROWB, lane);
+    store_rows<T, D>(dk, dk_scale, [&](int r) { return dkp + (int64_t)row_of(kw0 + r) * p.dks.s; }, p.Sk - kw0, smem + w * (64 * C::ROWB) + 32 * C::ROWB, lane);
   } else if (krow < p.Sk) {
     float* dkp = p.dk + b * p.dks.b + h * p.dks.h + (int64_t)krow * p.dks.s;
     float* dvp = p.dv + b * p.dvs.b + h * p.dvs.h + (int64_t)krow * p.dvs.s;
@@ -936,7 +998,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
         f32x4 x = *d1, y = *d2;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          x[e] += dk[db][4 * g + e] * p.scale;
+          x[e] += dk[db][4 * g + e] * dk_scale;
           y[e] += dv[db][4 * g + e];
         }
         *d1 = x;
