@@ -89,7 +89,7 @@ struct TileReads {
 // round j covers rows j * RPD + tid / CPR.  Slot (row, pos) receives chunk pos ^ swizzle(row).
 // ADDR_BIG: the tensor's rows of one (batch, head) may span 2 GiB or more; the descriptor is re-based per tile
 // (buffer_window) instead of covering the whole tensor.  ADDR_MAP: the rows lie in shards (RowMap): every lane looks up
-// its row (about 15 vector instructions per load, in the shadow of the MFMAs between which the loads are issued).
+// its row (about 15 vector instructions per load), or, for the tiles that are streamed, ShardTiles finds the rows of a whole tile.
 enum { ADDR_PLAIN = 0, ADDR_BIG = 1, ADDR_MAP = 2 };
 template <typename T, int D, int THREADS = BWD_THREADS, int ADDR = ADDR_PLAIN>
 struct TileLoader {
@@ -99,6 +99,7 @@ struct TileLoader {
   const T* base_;             // ADDR_BIG only
   unsigned long long total_;  // ADDR_BIG only: bytes from base_ to the end of the last row
   int rows_, drow_;           // ADDR_MAP only
+  unsigned row_off_;          // ADDR_MAP only: bytes from the tile's (or round's) first row to this thread's
   // rows: rows of the sequence; span: rows of the tensor from base to the sequence's last row
   __device__ __forceinline__ void init(const T* base, int64_t row_stride, int rows, int span, int tid) {
     typedef BwdCfg<D, THREADS> C;
@@ -108,6 +109,7 @@ struct TileLoader {
     const int drow = tid / C::CPR, dpos = tid % C::CPR;
     rows_ = rows;
     drow_ = drow;
+    row_off_ = (unsigned)(drow * row_stride * (int64_t)sizeof(T));
     lane_off = (unsigned)(((ADDR == ADDR_MAP ? 0 : drow * row_stride) + ((dpos ^ tile_swizzle<D>(drow)) * 8)) * (int64_t)sizeof(T));
     row_b = (unsigned)(row_stride * (int64_t)sizeof(T));
   }
@@ -126,6 +128,51 @@ struct TileLoader {
     } else {
       const unsigned u = on ? (unsigned)(row0 + q * C::RPD) * row_b : OFF_NONE;
       load_to_lds_b128(rsrc, lane_off + u, lds_wave + q * (THREADS * 16));
+    }
+  }
+};
+
+// The tiles of 64 rows of a pair of tensors with rows in shards, one after the other.  Where a segment has 64 rows or more a tile touches
+// two of them at most: which two is the same for all lanes, and a lane's row is in the first or the second.  (Looked up row by row the
+// one-wave dk/dv kernel, which issues an instruction every four clocks, spent 135 of 650 per tile on it.)
+template <typename T, int D, int THREADS>
+struct ShardTiles {
+  typedef BwdCfg<D, THREADS> C;
+  typedef TileLoader<T, D, THREADS, ADDR_MAP> Loader;
+  int seg, seg_end;                      // segment of the tile's first row, and where it ends
+  unsigned at[2][C::NDMA], stat_at;      // byte offsets of this thread's loads, and of the lane's row in lse and delta
+  __device__ __forceinline__ void init(const RowMap& map, int row0) {
+    seg = __builtin_amdgcn_readfirstlane(map.segment(row0));
+    seg_end = (seg + 1) * map.L;
+  }
+  // (called once for every tile, in order)
+  __device__ __forceinline__ void find(const RowMap& map, const ShardMap& m, int row0, int rows, const Loader& a, const Loader& b, int lane, bool on) {
+    if (map.L >= BWD_ROWS) {
+      if (row0 >= seg_end) {
+        ++seg;
+        seg_end += map.L;
+      }
+      const bool two = on && seg_end < rows;
+      const int r1 = row0 + map.shift(seg, m.pitch), r2 = row0 + map.shift(seg + 1, m.pitch);
+#pragma unroll
+      for (int q = 0; q < C::NDMA; ++q) {
+        const bool first = row0 + q * C::RPD + a.drow_ < seg_end;
+        const unsigned a1 = on ? (unsigned)(r1 + q * C::RPD) * a.row_b : OFF_NONE, a2 = two ? (unsigned)(r2 + q * C::RPD) * a.row_b : OFF_NONE;
+        const unsigned b1 = on ? (unsigned)(r1 + q * C::RPD) * b.row_b : OFF_NONE, b2 = two ? (unsigned)(r2 + q * C::RPD) * b.row_b : OFF_NONE;
+        at[0][q] = a.lane_off + a.row_off_ + (first ? a1 : a2);
+        at[1][q] = b.lane_off + b.row_off_ + (first ? b1 : b2);
+      }
+      const unsigned s1 = on ? (unsigned)(row0 + map.shift(seg, m.lse_pitch)) * 4u : OFF_NONE;
+      const unsigned s2 = two ? (unsigned)(row0 + map.shift(seg + 1, m.lse_pitch)) * 4u : OFF_NONE;
+      stat_at = lane * 4 + (row0 + lane < seg_end ? s1 : s2);
+    } else {
+#pragma unroll
+      for (int q = 0; q < C::NDMA; ++q) {
+        const int r = row0 + q * C::RPD + a.drow_, to = map.at(r, m.pitch);
+        at[0][q] = on && r < rows ? a.lane_off + (unsigned)to * a.row_b : OFF_NONE;
+        at[1][q] = on && r < rows ? b.lane_off + (unsigned)to * b.row_b : OFF_NONE;
+      }
+      stat_at = on && row0 + lane < rows ? (unsigned)map.at(row0 + lane, m.lse_pitch) * 4u : OFF_NONE;
     }
   }
 };
@@ -367,19 +414,23 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   rd.init(lane);
   const unsigned lds0 = (unsigned)(uintptr_t)(lds_u8*)smem;
   auto stage_of = [&](int i) { return lds0 + (unsigned)((i & (BWD_STAGES - 1)) * G::STAGE); };
-  auto issue_tile = [&](int i) {  // K and V tile i -> its stage
+  ShardTiles<T, D, NW * 64> tiles;
+  if constexpr (MAP) tiles.init(map, 0);
+  auto issue_one = [&](int i, int n) {  // load n of tile i's G::NL (in order): K, then V -> its stage
     const unsigned dst = stage_of(i) + w * 1024;
-#pragma unroll
-    for (int q = 0; q < C::NDMA; ++q) kld.load(q, i < nt, i * BWD_ROWS, dst, map, p.map.pitch);
-#pragma unroll
-    for (int q = 0; q < C::NDMA; ++q) vld.load(q, i < nt, i * BWD_ROWS, dst + C::TILEB, map, p.map.pitch);
-  };
-  auto issue_one = [&](int i, int n) {  // load n of tile i's G::NL, in issue_tile's order
-    const unsigned dst = stage_of(i) + w * 1024;
-    if (n < C::NDMA)
+    if constexpr (MAP) {
+      if (n == 0) tiles.find(map, p.map, i * BWD_ROWS, p.Sk, kld, vld, lane, i < nt);
+      const int t = n / C::NDMA, q = n % C::NDMA;
+      load_to_lds_b128(t ? vld.rsrc : kld.rsrc, tiles.at[t][q], dst + t * C::TILEB + q * (NW * 64 * 16));
+    } else if (n < C::NDMA) {
       kld.load(n, i < nt, i * BWD_ROWS, dst, map, p.map.pitch);
-    else
+    } else {
       vld.load(n - C::NDMA, i < nt, i * BWD_ROWS, dst + C::TILEB, map, p.map.pitch);
+    }
+  };
+  auto issue_tile = [&](int i) {
+#pragma unroll
+    for (int n = 0; n < G::NL; ++n) issue_one(i, n);
   };
 
   f32x16 dq[D / 32];
@@ -690,31 +741,30 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
   // per-row statistics: waves 0, 2 fetch the tile's 64 lse values, waves 1, 3 its 64 delta values
   // (the pairs store the same bytes to the same place, which keeps every wave's load count equal)
   const u32x4 stat_rsrc = buffer_descriptor((w & 1) ? delp : lsep, (unsigned)(MAP ? (p.map.P - 1) * p.map.lse_pitch + p.Sq / p.map.P : p.Sq) * 4u);
-  auto stat_offset = [&](bool on, int r) { return on && (!MAP || r < p.Sq) ? (unsigned)stat_of(r) * 4u : OFF_NONE; };
   TileReads<D> rd;
   rd.init(lane);
   const unsigned lds0 = (unsigned)(uintptr_t)(lds_u8*)smem;
   auto stage_of = [&](int i) { return lds0 + (unsigned)((i & (BWD_STAGES - 1)) * G::STAGE); };
-  auto issue_tile = [&](int i) {  // Q and dO tile i and their statistics -> stage
+  ShardTiles<T, D, BWD_THREADS> tiles;
+  if constexpr (MAP) tiles.init(map, it0 * BWD_ROWS);
+  auto issue_one = [&](int i, int n) {  // load n of tile i's G::NL (in order): Q, dO and their statistics -> its stage
     const unsigned st = stage_of(i);
     const unsigned dst = st + w * 1024;
-#pragma unroll
-    for (int q = 0; q < C::NDMA; ++q) qld.load(q, i < nt, i * BWD_ROWS, dst, map, p.map.pitch);
-#pragma unroll
-    for (int q = 0; q < C::NDMA; ++q) dold.load(q, i < nt, i * BWD_ROWS, dst + C::TILEB, map, p.map.pitch);
-    load_to_lds_b32(stat_rsrc, stat_offset(i < nt, i * BWD_ROWS + lane),
-                    st + 2 * C::TILEB + (w & 1) * (BWD_ROWS * 4));
-  };
-  auto issue_one = [&](int i, int n) {  // load n of tile i's G::NL, in issue_tile's order
-    const unsigned st = stage_of(i);
-    const unsigned dst = st + w * 1024;
-    if (n < C::NDMA)
+    if (n == 2 * C::NDMA) {
+      load_to_lds_b32(stat_rsrc, MAP ? tiles.stat_at : i < nt ? (unsigned)(i * BWD_ROWS + lane) * 4u : OFF_NONE, st + 2 * C::TILEB + (w & 1) * (BWD_ROWS * 4));
+    } else if constexpr (MAP) {
+      if (n == 0) tiles.find(map, p.map, i * BWD_ROWS, p.Sq, qld, dold, lane, i < nt);
+      const int t = n / C::NDMA, q = n % C::NDMA;
+      load_to_lds_b128(t ? dold.rsrc : qld.rsrc, tiles.at[t][q], dst + t * C::TILEB + q * (BWD_THREADS * 16));
+    } else if (n < C::NDMA) {
       qld.load(n, i < nt, i * BWD_ROWS, dst, map, p.map.pitch);
-    else if (n < 2 * C::NDMA)
+    } else {
       dold.load(n - C::NDMA, i < nt, i * BWD_ROWS, dst + C::TILEB, map, p.map.pitch);
-    else
-      load_to_lds_b32(stat_rsrc, stat_offset(i < nt, i * BWD_ROWS + lane),
-                      st + 2 * C::TILEB + (w & 1) * (BWD_ROWS * 4));
+    }
+  };
+  auto issue_tile = [&](int i) {
+#pragma unroll
+    for (int n = 0; n < G::NL; ++n) issue_one(i, n);
   };
 
   f32x16 dk[D / 32], dv[D / 32];
