@@ -578,7 +578,10 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   // The loads of tile i + 3 go out one at a time between the MFMAs of the pass: issued in one burst
   // after the barrier, they hold up the wave's instruction stream while the memory pipeline takes them in.
   constexpr int LOAD_GAP = NBODY / G::NL;
-  for (int i = 0; i < nt;) {
+  // Causal: the tiles a wave's rows see end with the one that holds its last row.  Behind that a wave only takes its share of the loads, and
+  // leaves the matrix pipe to the wave beside it (of the 4 tiles on the diagonal of 256 rows, 1.5 on average).
+  const int own_nt = p.causal && qw0 / BWD_ROWS + 1 < nt ? qw0 / BWD_ROWS + 1 : nt;
+  for (int i = 0; i < own_nt;) {
     // tile i+1 must have landed before this body reads it; tile i-1 is free for tile i+3
     wait_loads_but<G::NL>();
     __syncthreads();
@@ -642,7 +645,12 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
       sc = sn;
       dc = dn;
     }
-    if (++i == nt) mfma_settle();
+    if (++i == own_nt) mfma_settle();
+  }
+  for (int i = own_nt; i < nt; ++i) {
+    wait_loads_but<G::NL>();
+    __syncthreads();
+    issue_tile(i + 3);
   }
   wait_loads_but<0>();  // nothing may still be writing LDS when the workgroup ends
   // The last MFMAs must have written dq before it is read.  The accumulators are operands of the
