@@ -682,12 +682,17 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
 // ------------------------------------------------------------------------------------------
 // dK / dV kernel
 // ------------------------------------------------------------------------------------------
+template <bool V>
+struct Flag {
+  static constexpr bool value = V;
+};
+
 template <int D>
 struct DkvCfg {
   typedef BwdCfg<D> C;
   static constexpr int STAT = 2 * BWD_ROWS * 4;       // lse and delta of the tile's query rows
   static constexpr int STAGE = 2 * C::TILEB + STAT;   // Q tile, dO tile, stats
-  static constexpr int SMEM = BWD_STAGES * STAGE;
+  static constexpr int SMEM = BWD_STAGES * STAGE + (BWD_THREADS / 64) * 2 * BWD_ROWS * 4;  // (and each wave's copy of two tiles' lse)
   static constexpr int NL = 2 * C::NDMA + 1;          // loads per thread and stage
 };
 
@@ -784,10 +789,10 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
 
   // Half-tile g = 2 i + t is query rows [32 g, 32 g + 32).  Three of them are in work at any time: while the matrix pipe forms S and
   // dP of half g + 1 and the products of half g - 1 or g with the keys' gradients, the vector unit forms P and dS of half g.  The
-  // matrix instructions come in groups of GROUP, each with the vector work on 8 of the lane's 16 rows between them (one wave a SIMD issues one
-  // instruction every four clocks: with all vector work beside the 16 MFMAs of S and dP, a tile's 64 MFMAs, 2048 clocks, took 3660, 22 % of
-  // them waiting for LDS; spread over all of them, with lse read a group ahead and no drained window at the barrier, 3310.  What is
-  // gained is less, as the board lowers its clock with the matrix pipe's share: causal [1, 16384, 16, 128] dk/dv 2.17 -> 2.07 ms):
+  // matrix instructions come in groups of GROUP, each with the vector work on 8 of the lane's 16 rows between them: one wave a SIMD issues one
+  // instruction every four clocks, and with all vector work beside the MFMAs of S and dP those waited for it and the others for LDS.
+  // Bound: matrix pipe and LDS alike (a tile's 64 MFMAs are 2048 clocks; its 112 LDS reads a wave, 4 clocks of the CU's one pipe each whatever
+  // their width, and the loads into LDS, 2050).  Causal [1, 32768, 16, 128]: 7.98 -> 7.35 ms.
   //   first group of half g : S, dP of half g + 1, contraction steps 0 .. HS - 1  | P, dS of g, rows 0 .. 7  | dV, dK from g - 1, rows 8 .. 15
   //   second group          : S, dP of half g + 1, steps HS .. 2 HS - 1           | rows 8 .. 15             | dV, dK from g, rows 0 .. 7
   // One pass of the loop runs the second group of half 2 i, both groups of half 2 i + 1 and the first of half 2 i + 2, so that it
@@ -851,10 +856,17 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     f32x16 sc, dc, sn, dn;  // S and delta - dP of the current / next half-tile, then P and -dS
     frag pf[2], dsf[2];
     u32x4 pw, dsw;
-    f32x4 ln_raw[2], ln_cur[2];  // lse of the 8 rows of the next / the current group
+    f32x4 ln_next[2], ln_cur[2];  // -lse log2 e of the 8 rows of the next / the current group
+    // The wave's own copy of a tile's lse, times -log2 e: a lane prepares one row (a lane works on 16 of each half-tile).
+    typedef __attribute__((address_space(3))) float lds_float;
+    const unsigned own_lse = lds0 + BWD_STAGES * G::STAGE + w * (2 * BWD_ROWS * 4);
+    auto lse_of = [&](int i) { return own_lse + (unsigned)((i & 1) * (BWD_ROWS * 4)); };
+    float lse_row;
+    auto read_lse_row = [&](unsigned stage) { lse_row = *(const lds_float*)(lds_u8*)(uintptr_t)(stage + 2 * C::TILEB + 4 * lane); };
+    auto write_lse_row = [&](unsigned at) { *(lds_float*)(lds_u8*)(uintptr_t)(at + 4 * lane) = lse_row * -1.4426950408889634f; };
     auto load_lse = [&](f32x4 (&l)[2], unsigned at, int row) {
 #pragma unroll
-      for (int g = 0; g < 2; ++g) l[g] = __builtin_bit_cast(f32x4, lds_read_b128(at + (row + 8 * g) * 4));
+      for (int g = 0; g < 2; ++g) l[g] = __builtin_bit_cast(f32x4, lds_read_b128(at + 16 * hh + (row + 8 * g) * 4));
     };
     auto load_delta = [&](f32x16& x, unsigned at, int row) {
 #pragma unroll
@@ -867,11 +879,9 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     // diagonal: a key sees only the queries at or after it
     auto mask = [&](int half) {
       const int r0 = half * 32;
-      if (p.causal && kw0 + 31 > r0) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
-          if (krow > r0 + 8 * (v >> 2) + 4 * hh + (v & 3)) sc[v] = hidden;
-      }
+      for (int v = 0; v < 16; ++v)
+        if (krow > r0 + 8 * (v >> 2) + 4 * hh + (v & 3)) sc[v] = hidden;
     };
     // part n of the vector work of a group on rows 8 u .. 8 u + 7 of the lane's 16: two parts per row
     // (pinned by the empty asm: left alone, the compiler moves all of it behind the next branch)
@@ -879,7 +889,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     auto element = [&](int u, int n) {
       const int e = n >> 1, v = 8 * u + e;
       if ((n & 1) == 0) {
-        pr[e] = fast_exp2(__builtin_fmaf(sc[v], c, ln_cur[e >> 2][e & 3] * -1.4426950408889634f));
+        pr[e] = fast_exp2(__builtin_fmaf(sc[v], c, ln_cur[e >> 2][e & 3]));
         asm volatile("" : "+v"(pr[e]));
       } else {
         ds[e] = dc[v] * pr[e];
@@ -913,17 +923,12 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     };
 
     // Matrix instruction n of a group: 0 .. KS - 1: S, contraction step; KS .. : dP; 2 KS ..: gradient product number.  The gradient
-    // products, which do not wait for this group's vector work, stand between the others; the last of S and dP is at least
-    // five matrix instructions before the first vector instruction that reads it.
+    // products, whose operands take twice as many LDS reads, are every other one; the last of S and dP is two or more matrix
+    // instructions before the first vector instruction that reads it (S nine).
     constexpr int KS = D / 16;
     auto instruction = [](bool first, int n) -> int {
-      if (first) {
-        const int k = n >> 1;
-        return (n & 1) ? 2 * KS + k : k < HS ? k : KS + k - HS;
-      }
-      if (n >= 3 * HS) return 2 * KS + n - 2 * HS;
-      const int k = n / 3, what = n % 3;
-      return what == 2 ? 2 * KS + k : what * KS + HS + k;
+      const int k = n >> 1;
+      return (n & 1) ? 2 * KS + k : (first ? 0 : HS) + (k < HS ? k : KS + k - HS);
     };
     // operand number J of the pass on tile i (J >= NBODY: the first operands of the next pass)
     auto fetch = [&](int J) -> frag {
@@ -945,8 +950,10 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     };
 
     // Before the loop: S, dP of half 0 and what the first group of half 0 would do, less the gradients of a half before it.
-    load_lse(ln_cur, stat_at, 0);
-    load_lse(ln_raw, stat_at, 16);
+    read_lse_row(stage_of(it0));
+    write_lse_row(lse_of(it0));
+    load_lse(ln_cur, lse_of(it0), 0);
+    load_lse(ln_next, lse_of(it0), 16);
     load_delta(dc, stat_at, 0);
     load_delta(dn, stat_at, 32);
 #pragma unroll
@@ -963,7 +970,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
 #pragma unroll
     for (int j = 0; j < BWD_LOOK; ++j) win[j] = fetch(j);
     if (MIXED) mfma_settle();
-    mask(2 * it0);
+    if (p.causal) mask(2 * it0);
 #pragma unroll
     for (int n = 0; n < 16; ++n) element(0, n);
 
@@ -971,7 +978,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     // burst after the barrier, they hold up the wave's instruction stream while the memory pipeline
     // takes them in.
     constexpr int LOAD_GAP = NBODY / G::NL;
-    for (int i = it0; i < nt;) {
+    auto pass = [&](int i, auto diagonal) {
       // tile i + 1 has landed; every wave is done with tile i - 1.  The operands in flight are of tile i, so nothing else is waited for.
       wait_loads_but<G::NL>();
       if (MIXED)
@@ -984,13 +991,15 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
 #pragma unroll
       for (int group = 0; group < 4; ++group) {
         // half-tile of the vector work
-        if (group & 1) mask(2 * i + (group + 1) / 2);
-        ln_cur[0] = ln_raw[0];
-        ln_cur[1] = ln_raw[1];
+        if (diagonal.value && (group & 1)) mask(2 * i + (group + 1) / 2);
+        ln_cur[0] = ln_next[0];
+        ln_cur[1] = ln_next[1];
+        if (group == 0) read_lse_row(stage_of(i + 1));
+        if (group == 1) write_lse_row(lse_of(i + 1));
         if (group == 2) stat_at += step;
         // the next group's lse rows; what dP of the half-tile in production starts from
         if (group & 1) load_delta(dn, group == 1 ? stat_at + step : stat_at, group == 1 ? 0 : 32);
-        load_lse(ln_raw, stat_at, group == 0 ? 32 : group == 1 ? 48 : group == 2 ? 0 : 16);
+        load_lse(ln_next, lse_of(group < 2 ? i : i + 1), group == 0 ? 32 : group == 1 ? 48 : group == 2 ? 0 : 16);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int m = 0; m < GROUP; ++m) {
@@ -1027,8 +1036,12 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
           dc = dn;
         }
       }
-      if (++i == nt) mfma_settle();
-    }
+    };
+    // The halves on the diagonal of 128 keys are of tiles it0 and it0 + 1; a loop of their own, as the others would copy S for the choice.
+    int i = it0;
+    for (const int end = p.causal ? (it0 + 2 < nt ? it0 + 2 : nt) : it0; i < end; ++i) pass(i, Flag<true>());
+    for (; i < nt; ++i) pass(i, Flag<false>());
+    mfma_settle();
     wait_loads_but<0>();
   }
   // The last MFMAs must have written dk / dv before they are read; the accumulators are operands of
