@@ -33,6 +33,7 @@
 // (gradient accumulators in AGPRs, S / dP tiles in VGPRs), see MmaAsm.
 #include "spa_common.h"
 #include "spa_host.h"
+#include <math.h>
 #include <stdlib.h>
 
 namespace {
@@ -275,11 +276,14 @@ struct MmaAsm<_Float16> {
 // ------------------------------------------------------------------------------------------
 // dQ kernel
 // ------------------------------------------------------------------------------------------
-template <int D, int NW = 4>
+// KG = 2: the waves come in two groups that own the same query rows, and each takes 32 of a tile's 64 keys; their sums are added through LDS.
+template <int D, int NW = 4, int KG = 1>
 struct DqCfg {
   typedef BwdCfg<D, NW * 64> C;
+  static constexpr int ROWS = NW / KG * 32;   // query rows of a workgroup
+  static constexpr int STAGES = KG == 2 ? 5 : BWD_STAGES;
   static constexpr int STAGE = 2 * C::TILEB;  // K tile, V tile
-  static constexpr int SMEM = BWD_STAGES * STAGE;
+  static constexpr int SMEM = STAGES * STAGE;
   static constexpr int NL = 2 * C::NDMA;      // loads per thread and stage
 };
 
@@ -354,11 +358,11 @@ __device__ __forceinline__ void zero_grad_row(E* rowp, int hh) {
     }
 }
 
-template <typename T, int D, int NW, int ADDR = ADDR_PLAIN>
+template <typename T, int D, int NW, int ADDR = ADDR_PLAIN, int KG = 1>
 __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd_dq_kernel(const BwdParams pk) {
   BwdParams p = pk;  // a variable-length batch rewrites the sizes and bases for its sequence below
   typedef BwdCfg<D, NW * 64> C;
-  typedef DqCfg<D, NW> G;
+  typedef DqCfg<D, NW, KG> G;
   typedef Mma16<T> M;
   typedef MmaAsm<T> MA;
   // one wave per SIMD: AGPRs are there for the dq accumulators.  D = 128 only: its 8 gradient
@@ -373,9 +377,11 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int b, h, qt;
-  if (!workgroup_tile(p, true, NW * 32, lane, b, h, qt)) return;
-  const int q0 = qt * (NW * 32);
-  const int qw0 = q0 + w * 32;
+  if (!workgroup_tile(p, true, G::ROWS, lane, b, h, qt)) return;
+  const int q0 = qt * G::ROWS;
+  constexpr int RG = NW / KG;            // groups of 32 rows
+  const int rg = w % RG, kg = w / RG;    // the wave's rows, and its half of the keys of a tile
+  const int qw0 = q0 + rg * 32;
   RowMap map = {};
   select_sequence<T>(p, b, map);
   constexpr bool MAP = ADDR == ADDR_MAP;
@@ -404,7 +410,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   const float hidden = c < 0.f ? INFINITY : -INFINITY;  // a hidden score: exp2(hidden * c - lse) = 0 for either sign of the scale
   const int lim = p.causal ? (qrow < p.Sk - 1 ? qrow : p.Sk - 1) : p.Sk - 1;  // last visible key
 
-  const int kv_end = p.causal ? (q0 + NW * 32 < p.Sk ? q0 + NW * 32 : p.Sk) : p.Sk;
+  const int kv_end = p.causal ? (q0 + G::ROWS < p.Sk ? q0 + G::ROWS : p.Sk) : p.Sk;
   const int nt = (kv_end + BWD_ROWS - 1) / BWD_ROWS;  // key tiles this workgroup visits
 
   TileLoader<T, D, NW * 64, ADDR> kld, vld;
@@ -413,7 +419,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   TileReads<D> rd;
   rd.init(lane);
   const unsigned lds0 = (unsigned)(uintptr_t)(lds_u8*)smem;
-  auto stage_of = [&](int i) { return lds0 + (unsigned)((i & (BWD_STAGES - 1)) * G::STAGE); };
+  auto stage_of = [&](int i) { return lds0 + (unsigned)i % G::STAGES * G::STAGE; };
   ShardTiles<T, D, NW * 64> tiles;
   if constexpr (MAP) tiles.init(map, 0);
   auto issue_one = [&](int i, int n) {  // load n of tile i's G::NL (in order): K, then V -> its stage
@@ -440,19 +446,23 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   // Half-tile g = 2 i + t is keys [32 g, 32 g + 32).  One pass of the loop body handles tile i:
   //   list 2i  : S^T, dP^T of half 2i+1 (tile i, rows 32..63)   | dS^T of half 2i   | dQ of half 2i
   //   list 2i+1: S^T, dP^T of half 2i+2 (tile i+1, rows 0..31)  | dS^T of half 2i+1 | dQ of half 2i+1
-  // NA MFMAs produce, the element-wise work rides between them, NB MFMAs consume.
-  constexpr int NA = 2 * (D / 16), NB = 2 * (D / 32), NLIST = NA + NB, NBODY = 2 * NLIST;
+  // NA MFMAs produce, the element-wise work rides between them, NB MFMAs consume.  KG = 2: one list a pass, on the wave's half of tile i, with
+  // S^T, dP^T of its half of tile i + 1 (and the first operands of that of tile i + 2, hence a stage more).
+  constexpr int LISTS = 2 / KG;
+  constexpr int NA = 2 * (D / 16), NB = 2 * (D / 32), NLIST = NA + NB, NBODY = LISTS * NLIST;
   constexpr int LOOK_CAP = NW == 8 || D <= 64 ? 4 : BWD_LOOK_MAX;  // two waves per SIMD: 256 registers each, and the other wave covers LDS latency
   constexpr int BWD_LOOK = NA < LOOK_CAP ? NA : LOOK_CAP;
   static_assert(NBODY % BWD_LOOK == 0 && BWD_LOOK <= NA, "the operand window must tile the loop body");
 
   // The workgroup's rows of q and dout pass through the stages on their way into registers, and those of out, which give
   // delta = rowsum(dout * out) (written for the dk / dv kernel).  128 rows are one stage a tensor: all of them and the first tile are
-  // requested together.  256 rows are two: out follows when q and dout have been read, with the first two tiles.
-  constexpr bool TOGETHER = NW == 4;
-  constexpr int RT = NW / 2;  // tiles of 64 rows
-  const unsigned own = (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB;
-  const unsigned q_at = lds0 + (TOGETHER ? 2 * G::STAGE : 0), do_at = lds0 + (TOGETHER ? 3 : 2) * G::STAGE, out_at = lds0 + (TOGETHER ? 1 : 2) * G::STAGE;
+  // requested together (KG = 2: the first two tiles).  256 rows are two: out follows when q and dout have been read, with the first two tiles.
+  constexpr bool TOGETHER = RG <= 4;
+  constexpr int FIRST = KG;   // (TOGETHER) tiles requested with the rows
+  constexpr int RT = RG / 2;  // tiles of 64 rows
+  const unsigned own = (rg >> 1) * C::TILEB + (rg & 1) * 32 * C::ROWB;
+  const unsigned q_at = lds0 + (TOGETHER ? 2 * G::STAGE : 0), do_at = lds0 + (TOGETHER ? 3 : 2) * G::STAGE;
+  const unsigned out_at = lds0 + (KG == 2 ? 4 : TOGETHER ? 1 : 2) * G::STAGE;
   auto load_rows = [&](const T* base, int64_t stride, unsigned dst) {
     TileLoader<T, D, NW * 64, ADDR> ld;
     ld.init(base, stride, p.Sq, span_q, tid);
@@ -468,8 +478,9 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   load_rows(dop, p.dos.s, do_at);
   if constexpr (TOGETHER) {
     load_out();
-    issue_tile(0);
-    wait_loads_but<G::NL>();
+#pragma unroll
+    for (int i = 0; i < FIRST; ++i) issue_tile(i);
+    wait_loads_but<FIRST * G::NL>();
   } else {
     wait_loads_but<0>();
   }
@@ -502,16 +513,18 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
       }
     }
     dl = halves_sum(sum);
-    if (hh == 0 && qrow < p.Sq) p.delta[li] = dl;
+    if (hh == 0 && qrow < p.Sq && kg == 0) p.delta[li] = dl;
   } else {
     dl = p.delta[li];
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);  // the rows have been read ...
   __syncthreads();                     // ... by every wave
-  if constexpr (TOGETHER) issue_tile(1);
-  issue_tile(2);
+  if constexpr (TOGETHER) issue_tile(FIRST);
+  issue_tile(FIRST + 1 > 2 ? FIRST + 1 : 2);
   wait_loads_but<2 * G::NL>();
   __syncthreads();
+  constexpr int AHEAD = KG == 2 ? 4 : 3;  // tile i + AHEAD is requested in pass i
+  const unsigned half = KG == 2 ? kg * 32 * C::ROWB : 0;  // the wave's half of a tile
 
   f32x16 sc, dc, sn, dn;  // S^T, dP^T of the current / next half-tile
   {
@@ -519,7 +532,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
       zero16(sc);
       zero16(dc);
     }
-    const unsigned kb = stage_of(0);
+    const unsigned kb = stage_of(0) + half;
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) {
       const frag a0 = as_frag<frag>(lds_read_b128(kb + rd.row[ks]));
@@ -541,6 +554,12 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
 
   // operand fetch number J of the body of tile i (J >= NBODY: the first operands of the next body)
   unsigned row_cur[D / 16], row_nxt[D / 16], tr_cur[D / 32][2];
+  // KG = 2: row_cur and tr_cur are moved on to the next tile where that is first read through them; stages of tiles i - 1 .. i + 2
+  unsigned st_before = stage_of(0), st_this = st_before, st_next = stage_of(1), st_after = stage_of(2);
+  auto advance = [&](unsigned& at, unsigned by) {
+    at += by;
+    asm volatile("" : "+v"(at));  // (kept, not formed again from the tile's number at every use)
+  };
   auto set_addresses = [&](int i) {
     const unsigned a = stage_of(i), n = stage_of(i + 1);
 #pragma unroll
@@ -558,6 +577,11 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
     const int list = j2 / NLIST, j = j2 % NLIST;
     if (j < NA) {  // j = 2 ks + which: K row (S^T) or V row (dP^T) of the half-tile being produced
       const int ks = j >> 1, which = j & 1;
+      if constexpr (KG == 2) {
+        // the wave's rows of tile i+1; of the next body, tile i+2
+        if (which == 0) advance(row_cur[ks], body ? st_after - st_next : st_next - st_this);
+        return as_frag<frag>(lds_read_b128(row_cur[ks] + which * C::TILEB));
+      }
       // list 0 of this body: tile i rows 32..; list 1: tile i+1 rows 0..; list 0 of the next body: tile i+1 rows 32..
       const unsigned base = (body == 0 && list == 0) ? row_cur[ks] + 32 * C::ROWB
                             : (body == 0)           ? row_nxt[ks]
@@ -566,6 +590,10 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
     }
     const int jb = j - NA;  // jb = u * (D/32) + db : K^T operand of half-tile `list` of tile i
     const int db = jb % (D / 32), u = jb / (D / 32);
+    if (KG == 2 && u == 0) {
+#pragma unroll
+      for (int h8 = 0; h8 < 2; ++h8) advance(tr_cur[db][h8], st_this - st_before);
+    }
     const unsigned off = (list * 32 + u * 16) * C::ROWB;
     return frag_tr<frag>(tr_cur[db][0] + off, tr_cur[db][1] + off);
   };
@@ -573,95 +601,136 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   frag win[BWD_LOOK];
   frag dsf[2];
   set_addresses(0);
+  if constexpr (KG == 2) {
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) row_cur[ks] += half;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int h8 = 0; h8 < 2; ++h8) tr_cur[db][h8] += half;
+  }
 #pragma unroll
   for (int j = 0; j < BWD_LOOK; ++j) win[j] = fetch(j);
-  // The loads of tile i + 3 go out one at a time between the MFMAs of the pass: issued in one burst
+  // The loads of tile i + AHEAD go out one at a time between the MFMAs of the pass: issued in one burst
   // after the barrier, they hold up the wave's instruction stream while the memory pipeline takes them in.
   constexpr int LOAD_GAP = NBODY / G::NL;
   // Causal: the tiles a wave's rows see end with the one that holds its last row.  Behind that a wave only takes its share of the loads, and
   // leaves the matrix pipe to the wave beside it (of the 4 tiles on the diagonal of 256 rows, 1.5 on average).
-  const int own_nt = p.causal && qw0 / BWD_ROWS + 1 < nt ? qw0 / BWD_ROWS + 1 : nt;
-  for (int i = 0; i < own_nt;) {
-    // tile i+1 must have landed before this body reads it; tile i-1 is free for tile i+3
-    wait_loads_but<G::NL>();
-    __syncthreads();
-    set_addresses(i);
+  // (KG = 2: S and dP change registers from pass to pass, and the passes come in pairs; one behind the last tile has every key hidden.)
+  const int own_nt = (p.causal && qw0 / BWD_ROWS + 1 < nt ? qw0 / BWD_ROWS + 1 : nt) + KG - 1 & ~(KG - 1), all_nt = nt + KG - 1 & ~(KG - 1);
+  auto next_pass = [&]() {
+    // tile i+1 must have landed before this body reads it (KG = 2: i+2); tile i-1 is free for tile i+AHEAD.  (The operands in flight, one read
+    // each, are of tile i+1 or later.)
+    __builtin_amdgcn_s_waitcnt(0x0070 | (G::NL & 15) | ((G::NL >> 4) << 14) | (BWD_LOOK << 8));
+    __builtin_amdgcn_s_barrier();
+  };
+  auto list_of = [&](int i, int list, f32x16& sc, f32x16& dc, f32x16& sn, f32x16& dn) {
+    const int key0 = (2 * i + (KG == 2 ? kg : list)) * 32;  // first key of the half-tile whose dS is formed in this list
+    // diagonal: hide the keys after each lane's query; last tile: hide the keys past the end (their K
+    // and V rows arrive as zeros, but P = exp(0 - lse) overflows for lse < -88 and inf * 0 is NaN)
+    if ((p.causal && key0 + 31 > qw0) || key0 + 31 >= p.Sk) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (key0 + 8 * (v >> 2) + 4 * hh + (v & 3) > lim) sc[v] = hidden;
+    }
+    if (!MIXED) {
+      zero16(sn);
+      zero16(dn);
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int list = 0; list < 2; ++list) {
-      const int key0 = (2 * i + list) * 32;  // first key of the half-tile whose dS is formed in this list
-      // diagonal: hide the keys after each lane's query; last tile: hide the keys past the end (their K
-      // and V rows arrive as zeros, but P = exp(0 - lse) overflows for lse < -88 and inf * 0 is NaN)
-      if ((p.causal && key0 + 31 > qw0) || key0 + 31 >= p.Sk) {
+    for (int j = 0; j < NLIST; ++j) {
+      const int J = list * NLIST + j;
+      const frag a = win[J % BWD_LOOK];
+      win[J % BWD_LOOK] = fetch(J + BWD_LOOK);
+      __builtin_amdgcn_sched_barrier(0);
+      if (j < NA) {
+        const int ks = j >> 1;
+        if (MIXED) {
+          if (j & 1) {
+            if (ks == 0) MA::first_v(dn, a, dof[0]); else MA::acc_v(dn, a, dof[ks]);
+          } else {
+            if (ks == 0) MA::first_v(sn, a, qf[0]); else MA::acc_v(sn, a, qf[ks]);
+          }
+        } else if (j & 1) {
+          dn = M::run(a, dof[ks], dn);
+        } else {
+          sn = M::run(a, qf[ks], sn);
+        }
+        // element-wise work on the current half-tile, spread over the producing MFMAs
 #pragma unroll
         for (int v = 0; v < 16; ++v)
-          if (key0 + 8 * (v >> 2) + 4 * hh + (v & 3) > lim) sc[v] = hidden;
-      }
-      if (!MIXED) {
-        zero16(sn);
-        zero16(dn);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < NLIST; ++j) {
-        const int J = list * NLIST + j;
-        const frag a = win[J % BWD_LOOK];
-        win[J % BWD_LOOK] = fetch(J + BWD_LOOK);
-        __builtin_amdgcn_sched_barrier(0);
-        if (j < NA) {
-          const int ks = j >> 1;
-          if (MIXED) {
-            if (j & 1) {
-              if (ks == 0) MA::first_v(dn, a, dof[0]); else MA::acc_v(dn, a, dof[ks]);
-            } else {
-              if (ks == 0) MA::first_v(sn, a, qf[0]); else MA::acc_v(sn, a, qf[ks]);
-            }
-          } else if (j & 1) {
-            dn = M::run(a, dof[ks], dn);
-          } else {
-            sn = M::run(a, qf[ks], sn);
+          if (v * NA / 16 == j) {
+            const float pr = fast_exp2(__builtin_fmaf(sc[v], c, -l2));
+            sc[v] = pr * (dc[v] - dl);
           }
-          // element-wise work on the current half-tile, spread over the producing MFMAs
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            if (v * NA / 16 == j) {
-              const float pr = fast_exp2(__builtin_fmaf(sc[v], c, -l2));
-              sc[v] = pr * (dc[v] - dl);
-            }
-          if (j == NA / 2 - 1)
-            dsf[0] = M::pack(sc[0], sc[1], sc[2], sc[3], sc[4], sc[5], sc[6], sc[7]);
-          if (j == NA - 1) dsf[1] = M::pack(sc[8], sc[9], sc[10], sc[11], sc[12], sc[13], sc[14], sc[15]);
-        } else {
-          const int jb = j - NA;
-          const int db = jb % (D / 32), u = jb / (D / 32);
-          if (MIXED)
-            MA::acc_a(dq[db], a, dsf[u]);
-          else
-            dq[db] = M::run(a, dsf[u], dq[db]);
-        }
-        if (J % LOAD_GAP == LOAD_GAP / 2 && J / LOAD_GAP < G::NL) issue_one(i + 3, J / LOAD_GAP);
-        __builtin_amdgcn_sched_barrier(0);
+        if (j == NA / 2 - 1)
+          dsf[0] = M::pack(sc[0], sc[1], sc[2], sc[3], sc[4], sc[5], sc[6], sc[7]);
+        if (j == NA - 1) dsf[1] = M::pack(sc[8], sc[9], sc[10], sc[11], sc[12], sc[13], sc[14], sc[15]);
+      } else {
+        const int jb = j - NA;
+        const int db = jb % (D / 32), u = jb / (D / 32);
+        if (MIXED)
+          MA::acc_a(dq[db], a, dsf[u]);
+        else
+          dq[db] = M::run(a, dsf[u], dq[db]);
       }
-      sc = sn;
-      dc = dn;
+      if (J % LOAD_GAP == LOAD_GAP / 2 && J / LOAD_GAP < G::NL) issue_one(i + AHEAD, J / LOAD_GAP);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (++i == own_nt) mfma_settle();
+  };
+  auto pass = [&](int i, f32x16& s0, f32x16& d0, f32x16& s1, f32x16& d1) {
+    next_pass();
+    if constexpr (KG == 1) set_addresses(i);
+    __builtin_amdgcn_sched_barrier(0);
+    list_of(i, 0, s0, d0, s1, d1);
+    if constexpr (KG == 1) {
+      list_of(i, 1, s1, d1, s0, d0);
+    } else {
+      st_before = st_this;
+      st_this = st_next;
+      st_next = st_after;
+      st_after = st_after == stage_of(G::STAGES - 1) ? stage_of(0) : st_after + G::STAGE;
+    }
+  };
+  for (int i = 0; i < own_nt;) {
+    pass(i, sc, dc, sn, dn);
+    if constexpr (KG == 2) pass(i + 1, sn, dn, sc, dc);
+    i += KG;
+    if (i == own_nt) mfma_settle();
   }
-  for (int i = own_nt; i < nt; ++i) {
-    wait_loads_but<G::NL>();
-    __syncthreads();
-    issue_tile(i + 3);
+  for (int i = own_nt; i < all_nt; ++i) {
+    next_pass();
+    issue_tile(i + AHEAD);
   }
   wait_loads_but<0>();  // nothing may still be writing LDS when the workgroup ends
   // The last MFMAs must have written dq before it is read.  The accumulators are operands of the
   // wait, so no read of them can be scheduled above it.
   if constexpr (MIXED) asm volatile("s_nop 15\n s_nop 15" : "+a"(dq[0]), "+a"(dq[1]), "+a"(dq[2]), "+a"(dq[3])::"memory");
 
+  constexpr int SUMS = D / 32 * 16 * 64;  // (KG = 2) floats of a wave's sums
+  if constexpr (KG == 2) {
+    __syncthreads();
+    float* const sums = (float*)smem + rg * SUMS;
+    if (kg == 1) {
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sums[(db * 16 + v) * 64 + lane] = dq[db][v];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) dq[db][v] += sums[(db * 16 + v) * 64 + lane];
+  }
+
   if (p.grads_in_t) {
     // the whole gradient of the row: written in q's element type, nothing read
-    __syncthreads();  // every wave is done with the tiles, and with its loads into them
+    if constexpr (KG == 1) __syncthreads();  // every wave is done with the tiles, and with its loads into them
     T* const dqp = (T*)p.dq + b * p.dqs.b + h * p.dqs.h;
-    store_rows<T, D>(dq, p.scale, [&](int r) { return dqp + (int64_t)row_of(qw0 + r) * p.dqs.s; }, p.Sq - qw0, smem + w * (32 * C::ROWB), lane);
+    store_rows<T, D>(dq, p.scale, [&](int r) { return dqp + (int64_t)row_of(qw0 + r) * p.dqs.s; }, p.Sq - qw0, smem + (KG == 2 ? RG * SUMS * 4 : 0) + w * (32 * C::ROWB), lane);
   } else if (qrow < p.Sq) {
     float* dqp = p.dq + b * p.dqs.b + h * p.dqs.h + (int64_t)qrow * p.dqs.s;
 #pragma unroll
@@ -698,7 +767,9 @@ struct DkvCfg {
 
 // ASM = false: the D = 128 kernel with every MFMA left to the compiler (its uniform accumulator
 // form, its own hazard handling): slower, kept as the test twin of the hand-issued form.
-template <typename T, int D, bool ASM = true, int ADDR = ADDR_PLAIN>
+// QG = 2: 64 keys a workgroup.  Its waves come in two groups that own the same keys, and each takes 32 of a tile's 64 query rows; their sums
+// are added through LDS.
+template <typename T, int D, bool ASM = true, int ADDR = ADDR_PLAIN, int QG = 1>
 __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_kernel(const BwdParams pk) {
   BwdParams p = pk;  // a variable-length batch rewrites the sizes and bases for its sequence below
   typedef BwdCfg<D> C;
@@ -714,9 +785,11 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   int b, h, kt;
-  if (!workgroup_tile(p, false, 128, lane, b, h, kt)) return;
-  const int k0 = kt * 128;
-  const int kw0 = k0 + w * 32;
+  constexpr int KEYS = 128 / QG;
+  if (!workgroup_tile(p, false, KEYS, lane, b, h, kt)) return;
+  const int k0 = kt * KEYS;
+  const int qg = QG == 2 ? w >> 1 : 0;  // the wave's half of the rows of a tile
+  const int kw0 = k0 + (QG == 2 ? w & 1 : w) * 32;
   RowMap map = {};
   select_sequence<T>(p, b, map);
   constexpr bool MAP = ADDR == ADDR_MAP;
@@ -797,38 +870,50 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
   //   second group          : S, dP of half g + 1, steps HS .. 2 HS - 1           | rows 8 .. 15             | dV, dK from g, rows 0 .. 7
   // One pass of the loop runs the second group of half 2 i, both groups of half 2 i + 1 and the first of half 2 i + 2, so that it
   // reads tiles i and i + 1 only.
-  constexpr int HS = D / 32, GROUP = 4 * HS, NBODY = 4 * GROUP;
+  // QG = 2: "half g" is the wave's half of tile g; a pass runs the second group of half i and the first of half i + 1, and reads tiles i to i + 2.
+  constexpr int HS = D / 32, GROUP = 4 * HS, GROUPS = 4 / QG, NBODY = GROUPS * GROUP;
   constexpr int BWD_LOOK = D <= 64 ? 4 : BWD_LOOK_MAX;  // (two waves per SIMD at D <= 64, as in the dq kernel)
   static_assert(GROUP % BWD_LOOK == 0, "the operand window must tile a group");
 
   if (it0 < nt) {  // uniform; a workgroup whose keys no query sees adds nothing
-    // the workgroup's keys first, as two tiles each of K and V in the stages of tiles it0 + 2 and it0 + 3
+    // the workgroup's keys first, as two tiles each of K and V in the stages of tiles it0 + 2 and it0 + 3 (64 keys: both in the last)
     {
       TileLoader<T, D, BWD_THREADS, ADDR> kld, vld;
       kld.init(kp, p.ks.s, p.Sk, span_k, tid);
       vld.init(vp, p.vs.s, p.Sk, span_k, tid);
-      const unsigned kdst = stage_of(it0 + 2) + w * 1024, vdst = stage_of(it0 + 3) + w * 1024;
+      const unsigned kdst = stage_of(it0 + 4 - 2 / QG) + w * 1024, vdst = stage_of(it0 + 3) + (QG - 1) * C::TILEB + w * 1024;
 #pragma unroll
-      for (int half = 0; half < 2; ++half)
+      for (int half = 0; half < 2 / QG; ++half)
 #pragma unroll
         for (int q = 0; q < C::NDMA; ++q) kld.load(q, k0 + half * BWD_ROWS < p.Sk, k0 + half * BWD_ROWS, kdst + half * C::TILEB, map, p.map.pitch);
 #pragma unroll
-      for (int half = 0; half < 2; ++half)
+      for (int half = 0; half < 2 / QG; ++half)
 #pragma unroll
         for (int q = 0; q < C::NDMA; ++q) vld.load(q, k0 + half * BWD_ROWS < p.Sk, k0 + half * BWD_ROWS, vdst + half * C::TILEB, map, p.map.pitch);
     }
     issue_tile(it0);
-    wait_loads_but<G::NL>();
-    __syncthreads();
-    const unsigned own = (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB;  // the wave's 32 keys in either pair of tiles
-    read_rows<frag, D>(kf, stage_of(it0 + 2) + own, rd);
-    read_rows<frag, D>(vf, stage_of(it0 + 3) + own, rd);
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the stage of tile it0 + 2 has been read ...
-    issue_tile(it0 + 1);
-    __syncthreads();                     // ... by every wave
-    issue_tile(it0 + 2);
-    wait_loads_but<2 * G::NL>();
-    __syncthreads();
+    if constexpr (QG == 1) {
+      wait_loads_but<G::NL>();
+      __syncthreads();
+      const unsigned own = (w >> 1) * C::TILEB + (w & 1) * 32 * C::ROWB;  // the wave's 32 keys in either pair of tiles
+      read_rows<frag, D>(kf, stage_of(it0 + 2) + own, rd);
+      read_rows<frag, D>(vf, stage_of(it0 + 3) + own, rd);
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the stage of tile it0 + 2 has been read ...
+      issue_tile(it0 + 1);
+      __syncthreads();                     // ... by every wave
+      issue_tile(it0 + 2);
+      wait_loads_but<2 * G::NL>();
+      __syncthreads();
+    } else {
+      issue_tile(it0 + 1);
+      issue_tile(it0 + 2);
+      wait_loads_but<G::NL>();
+      __syncthreads();
+      const unsigned own = stage_of(it0 + 3) + (w & 1) * 32 * C::ROWB;
+      read_rows<frag, D>(kf, own, rd);
+      read_rows<frag, D>(vf, own + C::TILEB, rd);
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): read, before the barrier of the first pass
+    }
 
     // V negated: with delta as the accumulator's start the products give delta - dP, and -dS costs one multiplication per element.
 #pragma unroll
@@ -841,19 +926,20 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
 
     // Per-lane LDS addresses of the operands; each is moved on to the next tile where that tile is first read through it.
     unsigned row_at[D / 16], tr_at[D / 32][2], stat_at = stage_of(it0) + 2 * C::TILEB + 16 * hh;
-    unsigned step = 0, last_step = 0;  // from tile i to i + 1, from i - 1 to i
+    unsigned step = 0, last_step = 0, next_step = 0;  // from tile i to i + 1, from i - 1 to i, from i + 1 to i + 2
+    const unsigned half = qg * 32 * C::ROWB;          // (QG = 2) the wave's half of a tile
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) row_at[ks] = stage_of(it0) + rd.row[ks];
+    for (int ks = 0; ks < D / 16; ++ks) row_at[ks] = stage_of(it0) + half + rd.row[ks];
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-      for (int h8 = 0; h8 < 2; ++h8) tr_at[db][h8] = stage_of(it0) + rd.tr[db][h8];
+      for (int h8 = 0; h8 < 2; ++h8) tr_at[db][h8] = stage_of(it0) + half + rd.tr[db][h8];
     auto advance = [&](unsigned& at, unsigned by) {
       at += by;
       asm volatile("" : "+v"(at));  // (kept, not formed again from the tile's number at every use)
     };
 
-    f32x16 sc, dc, sn, dn;  // S and delta - dP of the current / next half-tile, then P and -dS
+    f32x16 s0, d0, s1, d1;  // S and delta - dP of the current and the next half-tile, in turn
     frag pf[2], dsf[2];
     u32x4 pw, dsw;
     f32x4 ln_next[2], ln_cur[2];  // -lse log2 e of the 8 rows of the next / the current group
@@ -877,7 +963,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
       }
     };
     // diagonal: a key sees only the queries at or after it
-    auto mask = [&](int half) {
+    auto mask = [&](f32x16& sc, int half) {
       const int r0 = half * 32;
 #pragma unroll
       for (int v = 0; v < 16; ++v)
@@ -886,7 +972,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     // part n of the vector work of a group on rows 8 u .. 8 u + 7 of the lane's 16: two parts per row
     // (pinned by the empty asm: left alone, the compiler moves all of it behind the next branch)
     float pr[8], ds[8];
-    auto element = [&](int u, int n) {
+    auto element = [&](const f32x16& sc, const f32x16& dc, int u, int n) {
       const int e = n >> 1, v = 8 * u + e;
       if ((n & 1) == 0) {
         pr[e] = fast_exp2(__builtin_fmaf(sc[v], c, ln_cur[e >> 2][e & 3]));
@@ -936,6 +1022,10 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
       const int n = instruction(group & 1, J % GROUP);
       if (n < 2 * KS) {  // row of Q (S) or dO (dP) of the half-tile being produced
         const int ks = n % KS, which = n / KS;
+        if constexpr (QG == 2) {
+          if (which == 0) advance(row_at[ks], group == 1 || J >= NBODY ? next_step : step);
+          return as_frag<frag>(lds_read_b128(row_at[ks] + which * C::TILEB));
+        }
         if ((group == 1 || group == 2) && which == 0) advance(row_at[ks], step);
         return as_frag<frag>(lds_read_b128(row_at[ks] + (group == 1 || group == 2 ? 0 : 32 * C::ROWB) + which * C::TILEB));
       }
@@ -952,54 +1042,77 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     // Before the loop: S, dP of half 0 and what the first group of half 0 would do, less the gradients of a half before it.
     read_lse_row(stage_of(it0));
     write_lse_row(lse_of(it0));
-    load_lse(ln_cur, lse_of(it0), 0);
-    load_lse(ln_next, lse_of(it0), 16);
-    load_delta(dc, stat_at, 0);
-    load_delta(dn, stat_at, 32);
+    load_lse(ln_cur, lse_of(it0), 32 * qg);
+    load_lse(ln_next, lse_of(it0), 32 * qg + 16);
+    load_delta(d0, stat_at, 32 * qg);
+    if constexpr (QG == 2) {
+      read_lse_row(stage_of(it0 + 1));
+      write_lse_row(lse_of(it0 + 1));
+      stat_at += stage_of(it0 + 1) - stage_of(it0);
+      load_delta(d1, stat_at, 32 * qg);
+    } else {
+      load_delta(d1, stat_at, 32);
+    }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      mma_s(sc, as_frag<frag>(lds_read_b128(row_at[ks])), ks);
-      mma_d(dc, as_frag<frag>(lds_read_b128(row_at[ks] + C::TILEB)), ks);
+      mma_s(s0, as_frag<frag>(lds_read_b128(row_at[ks])), ks);
+      mma_d(d0, as_frag<frag>(lds_read_b128(row_at[ks] + C::TILEB)), ks);
     }
 #pragma unroll
     for (int ks = 0; ks < HS; ++ks) {
-      mma_s(sn, as_frag<frag>(lds_read_b128(row_at[ks] + 32 * C::ROWB)), ks);
-      mma_d(dn, as_frag<frag>(lds_read_b128(row_at[ks] + 32 * C::ROWB + C::TILEB)), ks);
+      if (QG == 2) row_at[ks] += stage_of(it0 + 1) - stage_of(it0);
+      mma_s(s1, as_frag<frag>(lds_read_b128(row_at[ks] + (QG == 2 ? 0 : 32 * C::ROWB))), ks);
+      mma_d(d1, as_frag<frag>(lds_read_b128(row_at[ks] + (QG == 2 ? 0 : 32 * C::ROWB) + C::TILEB)), ks);
     }
     frag win[BWD_LOOK];
+    if (QG == 2) step = stage_of(it0 + 1) - stage_of(it0);
 #pragma unroll
     for (int j = 0; j < BWD_LOOK; ++j) win[j] = fetch(j);
+    if (QG == 2) step = 0;
     if (MIXED) mfma_settle();
-    if (p.causal) mask(2 * it0);
+    if (p.causal) mask(s0, 2 * it0 + qg);
 #pragma unroll
-    for (int n = 0; n < 16; ++n) element(0, n);
+    for (int n = 0; n < 16; ++n) element(s0, d0, 0, n);
 
     // The loads of tile i + 3 go out one at a time between the MFMAs of the pass: issued in one
     // burst after the barrier, they hold up the wave's instruction stream while the memory pipeline
     // takes them in.
-    constexpr int LOAD_GAP = NBODY / G::NL;
-    auto pass = [&](int i, auto diagonal) {
-      // tile i + 1 has landed; every wave is done with tile i - 1.  The operands in flight are of tile i, so nothing else is waited for.
-      wait_loads_but<G::NL>();
+    constexpr int LOAD_GAP = QG == 2 ? 2 : NBODY / G::NL;
+    static_assert(LOAD_GAP / 2 + (G::NL - 1) * LOAD_GAP < NBODY, "all loads of a tile in one pass");
+    // half-tiles in work at the start: s0, d0 (vector work) and s1, d1 (in production)
+    auto pass = [&](int i, f32x16& s0, f32x16& d0, f32x16& s1, f32x16& d1, auto diagonal) {
+      // tile i + 1 has landed (QG = 2: i + 2, requested in the pass before); every wave is done with tile i - 1.  The operands in flight are of
+      // later tiles, so nothing else is waited for.
+      wait_loads_but<QG == 2 ? 0 : G::NL>();
       if (MIXED)
         __builtin_amdgcn_s_barrier();
       else
         __syncthreads();
       last_step = step;
       step = stage_of(i + 1) - stage_of(i);
+      next_step = stage_of(i + 2) - stage_of(i + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int group = 0; group < 4; ++group) {
-        // half-tile of the vector work
-        if (diagonal.value && (group & 1)) mask(2 * i + (group + 1) / 2);
+      for (int group = 0; group < GROUPS; ++group) {
+        f32x16 &sc = group == 1 || group == 2 ? s1 : s0, &dc = group == 1 || group == 2 ? d1 : d0;  // half-tile of the vector work
+        f32x16 &sn = group == 1 || group == 2 ? s0 : s1, &dn = group == 1 || group == 2 ? d0 : d1;
+        if (diagonal.value && (group & 1)) mask(sc, 2 * i + (group + 1) / 2);
         ln_cur[0] = ln_next[0];
         ln_cur[1] = ln_next[1];
-        if (group == 0) read_lse_row(stage_of(i + 1));
-        if (group == 1) write_lse_row(lse_of(i + 1));
-        if (group == 2) stat_at += step;
-        // the next group's lse rows; what dP of the half-tile in production starts from
-        if (group & 1) load_delta(dn, group == 1 ? stat_at + step : stat_at, group == 1 ? 0 : 32);
-        load_lse(ln_next, lse_of(group < 2 ? i : i + 1), group == 0 ? 32 : group == 1 ? 48 : group == 2 ? 0 : 16);
+        // a row of lse for the wave's copy; the next group's lse rows; what dP of the half-tile in production starts from
+        if (group == 0) read_lse_row(stage_of(i + QG));
+        if (group == 1) write_lse_row(lse_of(i + QG));
+        if constexpr (QG == 2) {
+          if (group == 1) {
+            stat_at += next_step;
+            load_delta(dn, stat_at, 32 * qg);
+          }
+          load_lse(ln_next, lse_of(i + 1), 32 * qg + 16 * group);
+        } else {
+          if (group == 2) stat_at += step;
+          if (group & 1) load_delta(dn, group == 1 ? stat_at + step : stat_at, group == 1 ? 0 : 32);
+          load_lse(ln_next, lse_of(group < 2 ? i : i + 1), group == 0 ? 32 : group == 1 ? 48 : group == 2 ? 0 : 16);
+        }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int m = 0; m < GROUP; ++m) {
@@ -1027,20 +1140,25 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
           }
           // rows 8 .. 15 in the second group of a half-tile, 0 .. 7 in the first
 #pragma unroll
-          for (int e = m * 16 / GROUP; e < (m + 1) * 16 / GROUP; ++e) element(group & 1 ? 0 : 1, e);
+          for (int e = m * 16 / GROUP; e < (m + 1) * 16 / GROUP; ++e) element(sc, dc, group & 1 ? 0 : 1, e);
           if (J % LOAD_GAP == LOAD_GAP / 2 && J / LOAD_GAP < G::NL) issue_one(i + 3, J / LOAD_GAP);
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (!(group & 1)) {
-          sc = sn;
-          dc = dn;
-        }
       }
     };
-    // The halves on the diagonal of 128 keys are of tiles it0 and it0 + 1; a loop of their own, as the others would copy S for the choice.
     int i = it0;
-    for (const int end = p.causal ? (it0 + 2 < nt ? it0 + 2 : nt) : it0; i < end; ++i) pass(i, Flag<true>());
-    for (; i < nt; ++i) pass(i, Flag<false>());
+    if constexpr (QG == 1) {
+      // The halves on the diagonal of 128 keys are of tiles it0 and it0 + 1; a loop of their own, as the others would copy S for the choice.
+      for (const int end = p.causal ? (it0 + 2 < nt ? it0 + 2 : nt) : it0; i < end; ++i) pass(i, s0, d0, s1, d1, Flag<true>());
+      for (; i < nt; ++i) pass(i, s0, d0, s1, d1, Flag<false>());
+    } else {
+      // The diagonal of 64 keys is in tile it0, whose S has been seen to.  Passes in pairs, as S and dP change registers from one to the next
+      // (a pass behind the last tile adds products of zeros).
+      for (; i < nt; i += 2) {
+        pass(i, s0, d0, s1, d1, Flag<false>());
+        pass(i + 1, s1, d1, s0, d0, Flag<false>());
+      }
+    }
     mfma_settle();
     wait_loads_but<0>();
   }
@@ -1051,6 +1169,50 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
                  : "+a"(dk[0]), "+a"(dk[1]), "+a"(dk[2]), "+a"(dk[3]), "+a"(dv[0]), "+a"(dv[1]), "+a"(dv[2]), "+a"(dv[3])::"memory");
 
   const float dk_scale = -p.scale;  // (-dS, see the loop)
+  constexpr int SUMS = D / 32 * 16 * 64;  // (QG = 2) floats of one gradient of a wave
+  if constexpr (QG == 2) {
+    // group 0 writes dv, group 1 dk: each leaves the other's part in LDS
+    __syncthreads();
+    float* const own = (float*)smem + w * SUMS;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) own[(db * 16 + v) * 64 + lane] = qg ? dv[db][v] : dk[db][v];
+    __syncthreads();
+    const float* const other = (const float*)smem + (w ^ 2) * SUMS;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const float x = other[(db * 16 + v) * 64 + lane];
+        if (qg)
+          dk[db][v] += x;
+        else
+          dv[db][v] += x;
+      }
+    T* const dst = qg ? (T*)p.dk + b * p.dks.b + h * p.dks.h : (T*)p.dv + b * p.dvs.b + h * p.dvs.h;
+    float* const dst32 = qg ? p.dk + b * p.dks.b + h * p.dks.h : p.dv + b * p.dvs.b + h * p.dvs.h;
+    const int64_t stride = qg ? p.dks.s : p.dvs.s;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) dv[db][v] = qg ? dk[db][v] * dk_scale : dv[db][v];
+    if (p.grads_in_t) {
+      store_rows<T, D>(dv, 1.f, [&](int r) { return dst + (int64_t)row_of(kw0 + r) * stride; }, p.Sk - kw0, smem + 4 * SUMS * 4 + w * (32 * C::ROWB), lane);
+    } else if (krow < p.Sk) {
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          f32x4* const to = (f32x4*)(dst32 + (int64_t)krow * stride + db * 32 + 8 * g + 4 * hh);
+          f32x4 x = *to;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] += dv[db][4 * g + e];
+          *to = x;
+        }
+    }
+    return;
+  }
   if (p.grads_in_t) {
     __syncthreads();  // every wave is done with the tiles, and with its loads into them
     T* const dkp = (T*)p.dk + b * p.dks.b + h * p.dks.h;
@@ -1505,25 +1667,77 @@ hipError_t launch(int smem, bool queries, int rows, BwdParams p, hipStream_t str
   return hipGetLastError();
 }
 
+// What a launch of one of the forms below takes, in microseconds on a chip that does nothing else: its longest chain of tiles, or the work of all
+// workgroups shared out over the CUs.  rows: what a workgroup owns (query rows of the dq kernel, keys of the dk / dv kernel), start: its
+// start and end, tile: a tile of 64 of the other side (both fitted to launches of 8 heads, 256 to 4096 causal rows).
+double launch_time(const BwdParams& p, bool queries, int rows, double start, double tile) {
+  const int64_t longest = p.cu_q ? longest_rows(p) : queries ? p.Sq : p.Sk;
+  const double pairs = (double)p.B * p.H, total = p.cu_q ? (queries ? (double)p.lse_bh : (double)p.total_k) : (double)p.B * longest;
+  const double mean = total / p.B, wgs = p.cu_q ? pairs * (mean / rows + 0.5) : pairs * ((longest + rows - 1) / rows);
+  // rows of the other side
+  const double top = (double)(p.cu_q ? (longest < total ? longest : total) : !queries ? p.Sq : p.causal && p.Sq < p.Sk ? p.Sq : p.Sk);
+  const double most = ceil(top / BWD_ROWS), other = p.cu_q ? mean : top;
+  const double usual = (p.causal ? (other + rows) / 2 : other) / BWD_ROWS;
+  const double chain = start + tile * most, work = wgs * (start + tile * (usual < most ? usual : most)) / spa_device_cus();
+  return chain > work ? chain : work;
+}
+
+// The forms of the dq kernel, D = 128: 256 rows a workgroup (8 waves, two a SIMD, the K/V stream shared by twice the rows) where there are many;
+// with fewer, 128 rows, or 64 (4 waves), whose waves share out the keys of a tile: more workgroups, each with a shorter chain.  Causal,
+// us, 256 / 128 / 64 rows: 8 heads of 2048 rows 61.4 / 37.8 / 29.5, 4096 119 / 76.8 / 63.8, 8192 263 / 187 / 227; 16 of 4096 138 / 101 / 125; 32 of 512
+// 20.5 / 15.4 / 12.6, 2048 76.4 / 58.5 / 79.2, 4096 181 / 196 / 259; 128 of 512 30.3 / 33.2 / 39.5.  (128 rows on 4 waves that do not share, one a SIMD: 44.9,
+// 86.7, 203; 107; 16.4, 60.7, 209; 33.0.  Taken for tensors of 2 GiB and more per (batch, head), and by a test that wants the bits of 256 rows.)
+// D = 64: 128 rows, two workgroups to a CU, or 64 rows where those are two to a CU at most: 8 heads of 2048 rows 29.4 / 19.9, 4096 56.0 / 39.1, 8192
+// 128 / 119; 16 of 2048 30.0 / 21.6; 32 of 1024 18.7 / 14.3, 2048 36.9 / 36.9; 128 of 512 16.8 / 19.4.
+enum DqForm { DQ_128_PLAIN = 4, DQ_256 = 8, DQ_64 = 20, DQ_128 = 24 };  // the values of SPA_TUNE_BWD_DQ_WAVES
+template <int D, int ADDR>
+int dq_form(const BwdParams& p) {
+  const int forced = spa_knob(SPA_KNOB_BWD_DQ_WAVES);
+  if (D < 64 || ADDR == ADDR_BIG) return DQ_128_PLAIN;
+  if (forced && (D == 128 || forced == DQ_64)) return forced;
+  if (forced) return DQ_128_PLAIN;
+  if (D == 64) {
+    const double wgs = p.cu_q ? (double)p.H * ((double)p.lse_bh / 64 + p.B) : (double)p.B * p.H * ((p.Sq + 63) / 64);
+    return wgs <= 2.0 * spa_device_cus() ? DQ_64 : DQ_128_PLAIN;
+  }
+  const double t256 = launch_time(p, true, 256, 6.0, 1.76), t128 = launch_time(p, true, 128, 8.0, 0.92), t64 = launch_time(p, true, 64, 7.5, 0.69);
+  return t64 < t128 ? (t64 < t256 ? DQ_64 : DQ_256) : t128 < t256 ? DQ_128 : DQ_256;
+}
+
+// Whether the dk / dv kernel takes 64 keys a workgroup.  Causal, us, 128 / 64 keys, D = 128: 8 heads of 512 rows 17.7 / 14.6, 2048 52.1 / 36.8, 4096
+// 103 / 83.6, 8192 259 / 291; 16 of 2048 55.9 / 50.8, 4096 135 / 161; 32 of 512 19.5 / 17.0, 1024 33.9 / 35.5.  D = 64, two workgroups to a
+// CU: 8 of 2048 35.1 / 24.3, 4096 67.9 / 51.2; 16 of 4096 86.5 / 86.1; 32 of 1024 22.2 / 18.5, 2048 47.0 / 48.9; not causal 8 of 2048 36.9 / 27.6, 16 of 2048 41.4 / 41.2.
+template <int D, int ADDR>
+bool keys_64(const BwdParams& p) {
+  const int form = spa_knob(SPA_KNOB_BWD_DKDV_FORM);
+  if (D < 64 || ADDR == ADDR_BIG) return false;
+  if (form > 1) return form == 2;
+  if (D == 64) {
+    const double wgs = p.cu_q ? (double)p.H * ((double)p.total_k / 64 + p.B) : (double)p.B * p.H * ((p.Sk + 63) / 64);
+    return wgs <= (p.causal ? 2.0 : 1.0) * spa_device_cus();
+  }
+  return launch_time(p, false, 64, 6.5, 0.975) < launch_time(p, false, 128, 4.7, 1.48);
+}
+
 template <typename T, int D, int ADDR = ADDR_PLAIN>
 hipError_t launch_both(const BwdParams& p, hipStream_t stream) {
-  // dq kernel, D = 128: 256-row workgroups (two waves per SIMD, the K/V stream shared by twice the rows) once
-  // there are enough of them to occupy every CU and sequences have more than 128 rows (2000 x 16 heads of 16 rows, causal, backward:
-  // 1923 us, 1679 with 128; 500 of 128 rows 800, 764; 400 of 160 rows 921, 1024); spa_tune() can force 4 or 8 waves (experiments, tests).
-  // At D = 64 two 128-row workgroups to a CU are as fast on long rows (+-2 %) and 4 to 7 % faster on short ones.
-  // (Tensors of 2 GiB or more per (batch, head): 128 rows.)
-  const int64_t wgs8 = p.cu_q ? (int64_t)p.H * (p.lse_bh / 256 + (p.B + 1) / 2) : (int64_t)p.B * p.H * ((p.Sq + 255) / 256);
-  const int forced = spa_knob(SPA_KNOB_BWD_DQ_WAVES);
   hipError_t e = hipErrorInvalidValue;
-  bool wide = false;
+  const int form = dq_form<D, ADDR>(p);
   if constexpr (D == 128 && ADDR != ADDR_BIG) {
-    wide = forced ? forced == 8 : wgs8 >= spa_device_cus() && longest_rows(p) > 128;
-    if (wide) e = launch<flash_bwd_dq_kernel<T, D, 8, ADDR>>(DqCfg<D, 8>::SMEM, true, 256, p, stream, 512);
+    if (form == DQ_256) e = launch<flash_bwd_dq_kernel<T, D, 8, ADDR>>(DqCfg<D, 8>::SMEM, true, 256, p, stream, 512);
+    if (form == DQ_128) e = launch<flash_bwd_dq_kernel<T, D, 8, ADDR, 2>>(DqCfg<D, 8, 2>::SMEM, true, 128, p, stream, 512);
   }
-  if (!wide) e = launch<flash_bwd_dq_kernel<T, D, 4, ADDR>>(DqCfg<D, 4>::SMEM, true, 128, p, stream);
+  if constexpr (D >= 64 && ADDR != ADDR_BIG)
+    if (form == DQ_64) e = launch<flash_bwd_dq_kernel<T, D, 4, ADDR, 2>>(DqCfg<D, 4, 2>::SMEM, true, 64, p, stream);
+  if (form == DQ_128_PLAIN) e = launch<flash_bwd_dq_kernel<T, D, 4, ADDR>>(DqCfg<D, 4>::SMEM, true, 128, p, stream);
   if (e != hipSuccess) return e;
+  const bool narrow = keys_64<D, ADDR>(p);
   if constexpr (D == 128 && ADDR == ADDR_PLAIN)
-    if (spa_knob(SPA_KNOB_BWD_DKDV_FORM) == 1) return launch<flash_bwd_dkdv_kernel<T, D, false>>(DkvCfg<D>::SMEM, false, 128, p, stream);
+    if (spa_knob(SPA_KNOB_BWD_DKDV_FORM) == 1)
+      return narrow ? launch<flash_bwd_dkdv_kernel<T, D, false, ADDR, 2>>(DkvCfg<D>::SMEM, false, 64, p, stream)
+                    : launch<flash_bwd_dkdv_kernel<T, D, false>>(DkvCfg<D>::SMEM, false, 128, p, stream);
+  if constexpr (D >= 64 && ADDR != ADDR_BIG)
+    if (narrow) return launch<flash_bwd_dkdv_kernel<T, D, true, ADDR, 2>>(DkvCfg<D>::SMEM, false, 64, p, stream);
   return launch<flash_bwd_dkdv_kernel<T, D, true, ADDR>>(DkvCfg<D>::SMEM, false, 128, p, stream);
 }
 

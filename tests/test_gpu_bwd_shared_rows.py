@@ -1,0 +1,44 @@
+"""Backward forms whose waves share the rows (dq) or keys (dk/dv) of a workgroup and add their sums through LDS: sizes around a
+half-tile, a tile and a workgroup, odd and even numbers of tiles, against float64 autograd on the host."""
+import pytest
+import torch
+
+from conftest import rand_qkv
+from oracle import attn_oracle as O
+import sp_aurora_amd as spa
+from sp_aurora_amd import _lib
+from test_gpu_parity import DEV, check_grad
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,dq,dkdv", [(128, 20, 2), (128, 24, 2), (64, 20, 2)])
+def test_forms_with_shared_rows(D, dq, dkdv, dtype):
+    try:
+        _lib.tune("bwd_dq_waves", dq)
+        _lib.tune("bwd_dkdv_form", dkdv)
+        for S in (2, 31, 33, 64, 65, 96, 127, 129, 192, 257, 320):
+            for causal in (True, False):
+                q, k, v, dout = rand_qkv((1, S, 2, D), 700 + S, dtype, n=4)
+                want = O.attn_backward_autograd(q, k, v, dout, None, causal)
+                xs = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+                spa.ring_flash_attn_func(*xs, causal=causal).backward(dout.to(DEV))
+                for x, w, name in zip(xs, want, "qkv"):
+                    check_grad(x.grad, w, dtype, f"d{name}, {S} rows, causal {causal}")
+        # fp32 accumulators that are added to, more keys than queries and the reverse
+        for Sq, Sk in ((65, 200), (200, 65), (64, 640)):
+            q, _, _, dout = rand_qkv((1, Sq, 2, D), 720, dtype, n=4)
+            k, v, _, _ = rand_qkv((1, Sk, 2, D), 721, dtype, n=4)
+            for causal in (True, False):
+                out, lse = spa.ops.flash_fwd(q.to(DEV), k.to(DEV), v.to(DEV), causal=causal)
+                want = O.attn_backward_autograd(q, k, v, dout, None, causal)
+                base = [torch.randn(t.shape, device=DEV) for t in (q, k, v)]
+                acc = [t.clone() for t in base]
+                delta = spa.ops.bwd_delta(out, dout.to(DEV))
+                spa.ops.flash_bwd(q.to(DEV), k.to(DEV), v.to(DEV), dout.to(DEV), lse, delta, *acc, causal=causal)
+                for a, b, w, name in zip(acc, base, want, "qkv"):
+                    check_grad((a - b).to(dtype), w, dtype, f"d{name} added, {Sq} rows {Sk} keys, causal {causal}")
+    finally:
+        _lib.tune("bwd_dq_waves", 0)
+        _lib.tune("bwd_dkdv_form", 0)
