@@ -11,13 +11,11 @@
 //
 // Grid: x = batch * head (or group of HP heads), y = key chunk (the key split of the caller: chunk y writes rows y * Sq .. of the result
 // tensors it is given; of a packed batch, whose sequences have chunks of one length and as many as they need: fp32 partial
-// sums, merged by fewrows_combine_kernel).  256 threads.
+// sums, merged by fewrows_combine_kernel).  256 or 512 threads.
 #include "spa_common.h"
 #include "spa_host.h"
 
 namespace {
-
-constexpr int kWaves = 4;    // waves per workgroup
 
 template <int CTRL>
 static __device__ __forceinline__ float dpp_add(float x) {
@@ -62,10 +60,10 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 // What a chunk of a packed batch leaves in the workspace: per (sequence, head, row, chunk) D sums, and behind all of those (max, sum).
 __host__ __device__ inline int64_t part_stats(int64_t pairs, int nq, int n, int D) { return pairs * nq * n * D; }
 
-// kUnroll: loads of K (and of V) a wave keeps in flight.  NT: the loads carry the non-temporal hint (K and V are read
+// kWaves: waves of a workgroup.  kUnroll: loads of K (and of V) a wave keeps in flight.  NT: the loads carry the non-temporal hint (K and V are read
 // once and should not displace anything in the caches).
 // HP: neighbouring heads a workgroup takes together, whose pieces of a key row lie side by side.
-template <typename T, int D, bool KV8, int NQ, int kUnroll, bool NT, int HP>
+template <typename T, int D, bool KV8, int NQ, int kUnroll, bool NT, int HP, int kWaves>
 __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParams p) {
   constexpr int AUX = NT ? 2 : 0;
   typedef Piece<T, KV8> Pc;
@@ -305,16 +303,16 @@ __global__ void __launch_bounds__(D) fewrows_combine_kernel(const FwdParams p) {
 // Loads in flight and the non-temporal hint, measured on twelve decode shapes: four loads beat eight (6-10 %) except with three rows
 // and with single heads of 64-byte rows; the hint gains 5-15 % on 16-bit K/V, on e4m3 rows of a whole line when the keys are not split, and
 // on e4m3 heads taken together (12 % split), and loses where workgroups share lines (64-byte rows) and on split calls of single e4m3 heads.
-template <typename T, int D, bool KV8, int NQ, int U, int HP>
+template <typename T, int D, bool KV8, int NQ, int U, int HP, int W = 4>
 hipError_t launch_variant(const FwdParams& p, hipStream_t stream) {
-  const dim3 grid((unsigned)(p.B * p.H / HP), (unsigned)p.P), block(kWaves * 64);
+  const dim3 grid((unsigned)(p.B * p.H / HP), (unsigned)p.P), block(W * 64);
   constexpr bool hint = !KV8 || HP > 1;
   if constexpr (hint || D == 64) {
-    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, hint, HP>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, hint, HP, W>), grid, block, 0, stream, p);
   } else if (p.P == 1) {
-    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, true, HP>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, true, HP, W>), grid, block, 0, stream, p);
   } else {
-    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, false, HP>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, false, HP, W>), grid, block, 0, stream, p);
   }
   return hipGetLastError();
 }
@@ -334,6 +332,12 @@ hipError_t launch_unroll(const FwdParams& p, hipStream_t stream) {
       return launch_variant<T, D, KV8, NQ, NQ == 3 ? 8 : 4, HP>(p, stream);
   }
   constexpr int U = NQ == 3 || (KV8 && D == 64) ? 8 : 4;
+  // At most one workgroup per CU and chunks of 1 MB of K and V at most: bound by the latency of a wave's passes, which eight waves halve (kernel,
+  // us, 4 waves with 8 loads / 8 with 4, bf16, D = 128: 8 heads of 512 keys 8.0 / 7.0, 32 chunks of 2048 23.7 / 20.5, 128 28.5 / 26.0; 256 of 4096 76.8 /
+  // 95.1).  e4m3 rows of 128 elements, with twice the sums of a wave to add up, only for few: 8 of 1024 10.2 / 9.2, 64 9.3 / 10.0.
+  const int64_t chunk_bytes = (int64_t)p.Sk * D * (KV8 ? 1 : 2) * 2, most = KV8 && D == 128 ? spa_device_cus() / 8 : spa_device_cus();
+  if constexpr (NQ < 3)
+    if (groups <= most && chunk_bytes <= 1 << 20) return launch_variant<T, D, KV8, NQ, 4, 1, 8>(p, stream);
   if constexpr (U != 8) {
     if (groups * 2 <= spa_device_cus()) return launch_variant<T, D, KV8, NQ, 8, 1>(p, stream);
   }

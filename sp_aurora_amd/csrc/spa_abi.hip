@@ -251,11 +251,14 @@ int spa_flash_fwd_splitkv_suggest(int B, int H, int Sq, int Sk, int D, int mask_
     return 1;
   const int cus = spa_device_cus();
   // Up to kFewRows query rows run on the kernel that streams K and V: one workgroup per CU measured best on ten decode
-  // shapes (more chunks: 3 to 15 % slower), chunks of at least 512 keys.
+  // shapes (more chunks: 3 to 15 % slower), chunks of at least 64 KB of bf16 keys (512 keys of 128 instead of 256, us a call: [1, 8, 1 against 2048] 9.4
+  // and 8.5, 32 heads 10.9 and 9.1; for head dim 64 256 keys are no faster than 512).
   if (Sq <= kFewRows && spa_knob(SPA_KNOB_FEW_ROWS) != 1) {
     if (Sk < 1024) return 1;
     int64_t n = ((int64_t)cus + (int64_t)B * H / 2) / ((int64_t)B * H);
-    if (n > Sk / 512) n = Sk / 512;
+    // (not more than 16 of them below 512 keys: the second kernel takes 2.3 us for 8 or 16 chunks of 8 heads and 5 for 32)
+    const int64_t shortest = 32768 / D, by_length = Sk / shortest < 16 ? Sk / shortest : Sk / 512 > 16 ? Sk / 512 : 16;
+    if (n > by_length) n = by_length;
     if (n > 64) n = 64;
     return n < 2 ? 1 : KeySplit(Sk, (int)n).n;
   }
