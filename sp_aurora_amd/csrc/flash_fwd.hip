@@ -110,12 +110,17 @@ __device__ __forceinline__ int v_swizzle(int row) {
 // two segments (shards, or half shards) when a segment has a sub-tile's rows: the two shifts and the row between them are
 // scalars that step with the cursor, and a lane pays a comparison and a selection per load (+2 % of a step's vector work);
 // K and V rows are equally far apart, so V uses what was found for K a step earlier.
+// Q_STAGED (two groups on the same 128 rows, 16-bit q, D = 128): the query rows pass through LDS, so that a load instruction reads whole rows.  Straight
+// into the operands it is 16-byte pieces of 32 rows, 32 cache lines for 1 KB, in front of everything else a workgroup loads: causal, 16 heads of 512
+// rows 13.3 -> 12.2 us, 8 of 1024 18.4 -> 17.5.  Not for rows back to back as in [B,H,S,D] (eight blocks of 1024 rows 250.7 -> 252.4 us) and
+// D = 64 (no difference); one group, which has to hold K(1) back for it, and 256 rows: none or 1 % slower.
 template <typename T, int D, int NG, bool SHARE, bool KV8 = false, bool FINALN = false, bool ZZ = false, bool BIG = false,
-          bool QK8 = false, bool WAIT = false, bool KS = false, bool VR = false, bool MAP = false>
+          bool QK8 = false, bool WAIT = false, bool KS = false, bool VR = false, bool MAP = false, bool Q_STAGED = false>
 __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) flash_fwd16_kernel(const FwdParams pk) {
   static_assert(!(FINALN && SHARE), "the merging epilogue goes with 128-row workgroups");
   static_assert(!MAP || (!KV8 && !FINALN && !ZZ && !BIG && !WAIT && !KS && !VR), "rows in shards: 16-bit block calls");
   static_assert(!KS || (!SHARE && !FINALN && !ZZ && !BIG && !QK8 && !WAIT), "split keys: 128-row workgroups, plain results");
+  static_assert(!Q_STAGED || (NG == 2 && !SHARE && !QK8), "staged queries: one copy in the two groups' buffers");
   static_assert(!QK8 || (KV8 && D == 128 && !ZZ && !BIG), "8-bit scores: e4m3 q, k, v, head dim 128, contiguous chunks");
   typedef typename std::conditional<KV8, unsigned char, T>::type KVT;  // element type of K / V in memory
   typedef typename std::conditional<QK8, unsigned char, T>::type QT;   // element type of q in memory
@@ -237,7 +242,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
         qf8[kk][4 + i] = (int)(x1[i] ^ qsign);
       }
     }
-  } else {
+  } else if constexpr (!Q_STAGED) {
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) {
       u32x4 x = *(const u32x4*)(qp + (int64_t)qrow_t * p.qs.s + ks * 16 + hh * 8);
@@ -773,6 +778,17 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   cursor_next(cv);
   ck = cv;
   cursor_next(ck);
+  // (Q_STAGED: into the groups' second V buffers, which nothing else needs before the first MFMA phase; each group loads half of every wave's rows)
+  const unsigned q_block = (unsigned)(uintptr_t)(lds_u8*)smem + (w >> 1) * C::GROUP + 3 * C::TILEB + (w & 1) * 32 * C::ROWB;  // the wave's 32 rows
+  if constexpr (Q_STAGED) {
+#pragma unroll
+    for (int j = 0; j < 16 * C::CPR / 64; ++j) {
+      const int r = grp * 16 + j * (64 / C::CPR) + lane / C::CPR;
+      const int row = qw0 + r < q_lim ? qw0 + r : q_lim - 1;
+      const QT* const src = qp + (int64_t)(MAP ? map.at(row, p.map.pitch) : row) * p.qs.s + ((lane % C::CPR) ^ k_swizzle<D>(r)) * 8;
+      load_to_lds_b128(src, q_block + (grp * 16 + j * (64 / C::CPR)) * C::ROWB);
+    }
+  }
   // WAIT: no tile of a chunk is requested before the chunk's arrival flag has been seen (each wave polls for itself;
   // the acquire at system scope also drops cache lines that could hold the buffer's earlier contents).
   // The flag is read with a relaxed load at system scope (it bypasses the caches; nothing is invalidated: K/V lines can
@@ -831,6 +847,14 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   // opens the first MFMA phase reading them.
   __builtin_amdgcn_s_waitcnt(0x0F70 | ((NK + C::NDMA) & 15) | (((NK + C::NDMA) >> 4) << 14));  // vmcnt(loads of V(0), K(1))
   __syncthreads();
+  if constexpr (Q_STAGED) {  // (read by every wave before the barrier behind S(0))
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      u32x4 x = lds_read_b128(q_block + ln * C::ROWB + (((2 * ks + hh) ^ k_swizzle<D>(ln)) * 16));
+      x[0] ^= qsign; x[1] ^= qsign; x[2] ^= qsign; x[3] ^= qsign;
+      qf[ks] = as_frag<frag>(x);
+    }
+  }
   {
     frag none[NT][2];
     unsigned va[D / 32], ka[NKA];
@@ -1284,6 +1308,10 @@ hipError_t launch16(FwdParams p, hipStream_t stream) {
       p.nqt = fwd_tiles(p, 2 * FWD_BM);
       return launch<flash_fwd16_kernel<T, D, 2, true, KV8, false, ZZ, false, QK8>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, true>::SMEM, 2 * FWD_BM, p, stream);
     }
+  if constexpr (D == 128 && !KV8 && !ZZ)
+    if (form == FWD_SPLIT && p.qs.s != D)
+      return launch<flash_fwd16_kernel<T, D, 2, false, false, false, false, false, false, false, false, false, false, true>>(
+          2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
   if (form == FWD_SPLIT)
     return launch<flash_fwd16_kernel<T, D, 2, false, KV8, false, ZZ, false, QK8>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
   return launch<flash_fwd16_kernel<T, D, 1, false, KV8, false, ZZ, false, QK8>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM_PLAIN, FWD_BM, p, stream);
@@ -1300,7 +1328,7 @@ hipError_t launch16_map(FwdParams p, hipStream_t stream) {
       return launch<flash_fwd16_kernel<T, D, 2, true, N, N, N, N, N, N, N, N, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, true>::SMEM, 2 * FWD_BM, p, stream);
     }
   if (form == FWD_SPLIT)
-    return launch<flash_fwd16_kernel<T, D, 2, false, N, N, N, N, N, N, N, N, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
+    return launch<flash_fwd16_kernel<T, D, 2, false, N, N, N, N, N, N, N, N, true, D == 128>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
   return launch<flash_fwd16_kernel<T, D, 1, false, N, N, N, N, N, N, N, N, true>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM_PLAIN, FWD_BM, p, stream);
 }
 
