@@ -3,10 +3,9 @@
 //              stands in for update_out_and_lse (sp_aurora/utils.py:47-147)
 //   finalize : out = cast(out_acc)   (sp_aurora/intel_ring_flash_attn.py:141-143)
 //   delta    : delta = rowsum(dout * out), first pass of the block-wise backward
-// One thread owns 8 consecutive head dims of two (b, h, s) rows (all loads of both rows are
-// issued before the first store); the D/8 threads of a row sit in one wavefront, so every lane of
-// the row has read lse_acc before the row's first lane overwrites it.  32-bit row arithmetic,
-// the batch index comes from the grid.
+// One thread owns 8 head dims of a (b, h, s) row (all loads are issued before the first store); the D/8 threads of a row
+// sit in one wavefront, so every lane of the row has read lse_acc before the row's first lane overwrites it.  32-bit row
+// arithmetic, the batch index comes from the grid.
 #include "spa_common.h"
 
 namespace {
@@ -80,63 +79,100 @@ struct Load8<_Float16> {
   }
 };
 
-// A thread owns chunk `ch` (8 head dims) of ROWS_PER_THREAD rows, `half` rows apart; the D/8
-// lanes of a row share a wave, so every lane of the row has read lse_acc before lane 0 rewrites it.
+// merge: a thread owns 4 dims of either half of a row, 4 ch .. and D / 2 + 4 ch .., so that the lanes' 16 bytes of the fp32 sums lie back to back (8
+// consecutive dims a thread: two accesses of every other 16 bytes).  A workgroup takes consecutive rows of one head (by_head): its lse is one
+// piece of memory, where rows of 16 heads, heads fastest, read and wrote 4 bytes of 16 cache lines each, lines that 31 other workgroups
+// on all XCDs wrote into as well.  Bound: the memory-side cache and HBM.  32 heads of 1024 rows, D = 128, bf16 (42 MB): 9.1 us, the
+// dims split 8.3, rows by head 8.0 (5.3 TB/s); 2 x 32 of 2048 29.2 -> 26.5 us; D = 64 5.4 -> 4.9.
+template <typename T>
+__device__ __forceinline__ void load44(const T* p, int half, float* x);
+template <>
+__device__ __forceinline__ void load44<float>(const float* p, int half, float* x) {
+  const f32x4 a = *(const f32x4*)p, b = *(const f32x4*)(p + half);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = a[i];
+    x[4 + i] = b[i];
+  }
+}
+template <>
+__device__ __forceinline__ void load44<__bf16>(const __bf16* p, int half, float* x) {
+  const u32x2 a = *(const u32x2*)p, b = *(const u32x2*)(p + half);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    x[2 * i] = __builtin_bit_cast(float, a[i] << 16);
+    x[2 * i + 1] = __builtin_bit_cast(float, a[i] & 0xffff0000u);
+    x[4 + 2 * i] = __builtin_bit_cast(float, b[i] << 16);
+    x[4 + 2 * i + 1] = __builtin_bit_cast(float, b[i] & 0xffff0000u);
+  }
+}
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+template <>
+__device__ __forceinline__ void load44<_Float16>(const _Float16* p, int half, float* x) {
+  const f16x4 a = *(const f16x4*)p, b = *(const f16x4*)(p + half);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = (float)a[i];
+    x[4 + i] = (float)b[i];
+  }
+}
+
 template <typename T, bool INIT>
 __global__ void __launch_bounds__(256) merge_kernel(float* __restrict__ out_acc, float* __restrict__ lse_acc,
                                                     const T* __restrict__ blk_out,
                                                     const float* __restrict__ blk_lse, int H, int Sq,
-                                                    int cpr_shift /* log2(D/8) */, unsigned nrows, unsigned half,
-                                                    Strides3 as, Strides3 bs, int64_t acc_lse_bh) {
-  const unsigned gid = blockIdx.x * 256u + threadIdx.x;
-  const unsigned row0 = gid >> cpr_shift;
-  const int ch = (int)(gid & ((1u << cpr_shift) - 1u));
-  float xb[ROWS_PER_THREAD][8], xa[ROWS_PER_THREAD][8], lb[ROWS_PER_THREAD], la[ROWS_PER_THREAD];
-  float* ap[ROWS_PER_THREAD];
-  int64_t la_i[ROWS_PER_THREAD];
-  bool on[ROWS_PER_THREAD];
-#pragma unroll
-  for (int k = 0; k < ROWS_PER_THREAD; ++k) {
-    const unsigned row = row0 + k * half;
-    on[k] = row0 < half && row < nrows;
-    const RowIdx r = decode_row(on[k] ? row : 0u, H);
-    const int64_t li = ((int64_t)r.b * H + r.h) * Sq + r.s;     // block lse: contiguous [B,H,Sq]
-    la_i[k] = ((int64_t)r.b * H + r.h) * acc_lse_bh + r.s;        // running lse: row pitch acc_lse_bh
-    ap[k] = out_acc + r.b * as.b + r.h * as.h + (int64_t)r.s * as.s + ch * 8;
-    if (on[k]) {
-      Load8<T>::ld(blk_out + r.b * bs.b + r.h * bs.h + (int64_t)r.s * bs.s + ch * 8, xb[k]);
-      lb[k] = blk_lse[li];
-      if (!INIT) {
-        la[k] = lse_acc[la_i[k]];
-        Load8<float>::ld(ap[k], xa[k]);
-      }
-    }
+                                                    int cpr_shift /* log2(D/8) */, bool by_head, Strides3 as, Strides3 bs, int64_t acc_lse_bh) {
+  const int ch = (int)(threadIdx.x & ((1u << cpr_shift) - 1u)), half = 4 << cpr_shift;
+  RowIdx r;
+  if (by_head) {
+    const unsigned block = blockIdx.x / (unsigned)H;
+    r.h = (int)(blockIdx.x - block * (unsigned)H);
+    r.s = (int)((block * 256u + threadIdx.x) >> cpr_shift);
+    r.b = (int)blockIdx.y;
+  } else {
+    r = decode_row((blockIdx.x * 256u + threadIdx.x) >> cpr_shift, H);
   }
+  if (r.s >= Sq) return;
+  const int64_t li = ((int64_t)r.b * H + r.h) * Sq + r.s;           // block lse: contiguous [B,H,Sq]
+  const int64_t la_i = ((int64_t)r.b * H + r.h) * acc_lse_bh + r.s; // running lse: row pitch acc_lse_bh
+  float* const ap = out_acc + r.b * as.b + r.h * as.h + (int64_t)r.s * as.s + ch * 4;
+  float xb[8], xa[8];
+  load44<T>(blk_out + r.b * bs.b + r.h * bs.h + (int64_t)r.s * bs.s + ch * 4, half, xb);
+  const float lb = blk_lse[li];
+  float la = 0.f;
+  if (!INIT) {
+    la = lse_acc[la_i];
+    load44<float>(ap, half, xa);
+  }
+  float ln = lb;
+  if (INIT) {
 #pragma unroll
-  for (int k = 0; k < ROWS_PER_THREAD; ++k) {
-    if (!on[k]) continue;
-    if (INIT) {
-      Load8<float>::st(ap[k], xb[k]);
-      if (ch == 0) lse_acc[la_i[k]] = lb[k];
-      continue;
-    }
+    for (int i = 0; i < 8; ++i) xa[i] = xb[i];
+  } else {
     // w = sigmoid(lb - la); lse' = max + log1p(exp(-|lb - la|))
-    const float d = lb[k] - la[k];
-    float w, ln;
+    const float d = lb - la;
+    float w;
     if (d == d) {  // also covers +-inf on one side
       const float e = __expf(-fabsf(d));
       const float inv = 1.f / (1.f + e);
       w = d >= 0.f ? inv : e * inv;
-      ln = fmaxf(la[k], lb[k]) + log1pf(e);
+      ln = fmaxf(la, lb) + log1pf(e);
     } else {  // both -inf: nothing accumulated on either side
       w = 0.f;
-      ln = la[k];
+      ln = la;
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) xa[k][i] = xa[k][i] - w * (xa[k][i] - xb[k][i]);
-    Load8<float>::st(ap[k], xa[k]);
-    if (ch == 0) lse_acc[la_i[k]] = ln;
+    for (int i = 0; i < 8; ++i) xa[i] = xa[i] - w * (xa[i] - xb[i]);
   }
+  f32x4 a, b;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    a[i] = xa[i];
+    b[i] = xa[4 + i];
+  }
+  *(f32x4*)ap = a;
+  *(f32x4*)(ap + half) = b;
+  if (ch == 0) lse_acc[la_i] = ln;
 }
 
 template <typename T>
@@ -272,9 +308,12 @@ hipError_t spa_launch_merge(float* out_acc, float* lse_acc, const void* blk_out,
                             int64_t acc_lse_bh, hipStream_t stream) {
   const RowGrid g = row_grid(B, H, Sq, D);
   if (!g.ok) return hipErrorInvalidValue;
+  const int64_t blocks = ((int64_t)Sq * (D / 8) + 255) / 256 * H;
+  const bool by_head = (int64_t)Sq * (D / 8) >= 256 && blocks * 256 <= 0x7fffffffLL;  // (fewer rows than a workgroup takes would leave threads idle)
+  const dim3 grid = by_head ? dim3((unsigned)blocks, (unsigned)B) : g.grid;
 #define SPA_MERGE(T, I)                                                                              \
-  hipLaunchKernelGGL((merge_kernel<T, I>), g.grid, dim3(256), 0, stream, out_acc, lse_acc, (const T*)blk_out, \
-                     blk_lse, H, Sq, g.cpr_shift, g.nrows, g.half, as, bs, acc_lse_bh)
+  hipLaunchKernelGGL((merge_kernel<T, I>), grid, dim3(256), 0, stream, out_acc, lse_acc, (const T*)blk_out, \
+                     blk_lse, H, Sq, g.cpr_shift, by_head, as, bs, acc_lse_bh)
   if (dtype == 0) { if (init) SPA_MERGE(float, true); else SPA_MERGE(float, false); }
   else if (dtype == 1) { if (init) SPA_MERGE(__bf16, true); else SPA_MERGE(__bf16, false); }
   else if (dtype == 2) { if (init) SPA_MERGE(_Float16, true); else SPA_MERGE(_Float16, false); }
