@@ -72,7 +72,7 @@ __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParam
   constexpr int LPR = LPH * HP;     // lanes per key row
   constexpr int R = 64 / LPR;       // key rows per load of a wave
   constexpr int KESZ = KV8 ? 1 : 2;
-  static_assert((LPH == 4 || LPH == 8 || LPH == 16) && LPR <= 16, "row spread");
+  static_assert((LPH == 4 || LPH == 8 || LPH == 16) && LPR <= 32, "row spread");
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // Workgroups go to the 8 XCDs round robin.  Where a key row of one head is half a cache line (64 e4m3 elements), two
@@ -321,12 +321,20 @@ hipError_t launch_variant(const FwdParams& p, hipStream_t stream) {
 // as many as make 256 bytes: 128-byte requests 4 KiB apart reach 5.1 TB/s, 256-byte ones 6.0 (64 caches of 1 to 4 thousand tokens, H = 32,
 // D = 128, e4m3: 256 -> 221 us; fixed length, B = 16, 4096 keys: e4m3 97 -> 85, bf16 D = 64 95 -> 80).  Not where that leaves CUs without
 // a workgroup: with one per CU and single heads 44 us, 48 together (B = 1, 32768 keys, e4m3, D = 128).
+// Rows of 128 elements, and eight workgroups per CU left: as many heads as make 512 bytes (64 caches of 2 to 8 thousand tokens, H = 32: e4m3 461 ->
+// 439 us, bf16 875 -> 839; of 1 to 4 thousand 237 -> 234 and 442 -> 435).  With fewer the last workgroups count for more: 32 caches of
+// 512 to 2048, e4m3, two per CU, 65 -> 75; 8 of 2 to 8 thousand, bf16, four, 118 -> 124.
 // A launch that leaves half of the CUs without a workgroup (a caller who did not split the keys) is bound by what its
 // few waves keep in flight: eight loads there too.
 template <typename T, int D, bool KV8, int NQ>
 hipError_t launch_unroll(const FwdParams& p, hipStream_t stream) {
   constexpr int HP = 256 / (D * (KV8 ? 1 : 2));
   const int64_t groups = (int64_t)p.B * p.H * p.P;
+  if constexpr (D == 128) {
+    constexpr int WIDE = 2 * HP;
+    if (p.H % WIDE == 0 && p.ks.h == D && p.vs.h == D && groups / WIDE >= 8 * spa_device_cus())
+      return launch_variant<T, D, KV8, NQ, NQ == 3 ? 8 : 4, WIDE>(p, stream);
+  }
   if constexpr (HP > 1) {
     if (p.H % HP == 0 && p.ks.h == D && p.vs.h == D && groups / HP >= spa_device_cus())
       return launch_variant<T, D, KV8, NQ, NQ == 3 ? 8 : 4, HP>(p, stream);

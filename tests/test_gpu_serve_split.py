@@ -87,6 +87,17 @@ def test_chunks_of_ragged_caches(H, reps, chunk, D, dtype, fp8):
     check(ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 3, max_k, **scales), want, dtype)  # (not split: heads together where there are enough)
 
 
+@pytest.mark.parametrize("dtype,fp8", [(torch.bfloat16, False), (torch.float16, False), (torch.bfloat16, True)])
+@pytest.mark.parametrize("H", [32, 30])  # (30: a count that four does not divide)
+def test_many_small_chunks(H, dtype, fp8):
+    """Eight workgroups and more per CU with 512 bytes of heads each, D = 128."""
+    lens = [(1 + (i * 37) % 130, 1 + i % 3) for i in range(34)] + [(0, 1), (130, 0), (144, 3)]
+    q, k, v, cu_q, cu_k, scales = caches(lens, H, 128, dtype, fp8, 1300 + H)
+    want = reference(q, k, v, cu_q, cu_k, 3, 144, **scales)
+    check_exact(want, exact(q, k, v, cu_q, cu_k, **scales), dtype)
+    check(split(q, k, v, cu_q, cu_k, 3, 144, 16, **scales), want, dtype)
+
+
 @pytest.mark.parametrize("nseq,longest", [(3, 900), (70, 2300)])
 def test_suggested_chunks_and_capture(nseq, longest):
     H, D, dtype = 4, 128, torch.bfloat16
