@@ -1055,13 +1055,15 @@ int64_t spa_flash_fwd_varlen_splitkv_workspace_bytes(int nseq, int H, int total_
 // 91 -> 36 us; up to 1024 tokens 14.8 -> 10.4).  More: whole sequences until the longest keeps its workgroup busy for 25 us (1.1 MB
 // of K and V, whatever the type: heads are taken together, launch_unroll), since the second kernel costs 3 to 5 us; then chunks of
 // 1024 keys (64 caches of 1 to 4 thousand tokens, H = 32: bf16 437 -> 413 us; 2 to 8 thousand, H = 8, e4m3 145 -> 122; 512 and 2048
-// are 1 to 4 % slower).
+// are 1 to 4 % slower), or, at D = 128, of 512 while those are 16 thousand workgroups of one head or fewer and the last of them count (1024 / 512,
+// us, longest of 4096: 64, H = 32, e4m3 234.3 / 228.0, bf16 435.3 / 429.8; of 8192: 8, H = 32, 72.8 / 71.9 and 118.5 / 114.4, 32, H = 8, 75.5 /
+// 72.7 and 125.2 / 123.7, but 64, H = 32, 437 / 446 and 836 / 843; D = 64, 32 of 4096, H = 8, bf16 38.1 / 40.5).
 int spa_flash_fwd_varlen_splitkv_suggest(int nseq, int H, int total_k, int max_sq, int max_sk, int D, int dtype) {
   if (nseq <= 0 || H <= 0 || total_k <= 0 || max_sq <= 0 || max_sq > kFewRows || max_sk <= 0 || (D != 64 && D != 128) ||
       (dtype != SPA_BF16 && dtype != SPA_F16) || spa_knob(SPA_KNOB_FEW_ROWS) == 1)
     return 0;
   const int64_t cus = spa_device_cus();
-  if ((int64_t)nseq * H >= cus) return max_sk > 2200 ? 1024 : 0;
+  if ((int64_t)nseq * H >= cus) return max_sk <= 2200 ? 0 : D == 128 && (int64_t)total_k * H <= 512 * 64 * cus ? 512 : 1024;
   const int64_t even = (int64_t)total_k * H / cus, chunk = even <= 256 ? 256 : (even + 255) / 256 * 256;
   return max_sk >= chunk * 3 / 2 ? (int)chunk : 0;
 }
