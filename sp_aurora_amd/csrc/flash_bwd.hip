@@ -1678,7 +1678,10 @@ double launch_time(const BwdParams& p, bool queries, int rows, double start, dou
   const double top = (double)(p.cu_q ? (longest < total ? longest : total) : !queries ? p.Sq : p.causal && p.Sq < p.Sk ? p.Sq : p.Sk);
   const double most = ceil(top / BWD_ROWS), other = p.cu_q ? mean : top;
   const double usual = (p.causal ? (other + rows) / 2 : other) / BWD_ROWS;
-  const double chain = start + tile * most, work = wgs * (start + tile * (usual < most ? usual : most)) / spa_device_cus();
+  // (Workgroups of one length go in whole rounds of one per CU; causal ones, the long ones first, and those of a ragged batch fill each other's gaps.
+  // Not causal, training step, us, rounds as a fraction / whole: 12 heads of 1536 rows 126 / 93, 16 of 1280 97 / 82, 64 of 640 103 / 97, 32 of 1536 199 / 188.)
+  const double rounds = wgs / spa_device_cus();
+  const double chain = start + tile * most, work = (p.causal || p.cu_q ? rounds : ceil(rounds)) * (start + tile * (usual < most ? usual : most));
   return chain > work ? chain : work;
 }
 
