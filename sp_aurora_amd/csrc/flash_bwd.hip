@@ -176,6 +176,12 @@ struct ShardTiles {
       stat_at = on && row0 + lane < rows ? (unsigned)map.at(row0 + lane, m.lse_pitch) * 4u : OFF_NONE;
     }
   }
+  // behind the last tile: the first tensor's rows once more, zeros for the others
+  __device__ __forceinline__ void repeat_first() {
+#pragma unroll
+    for (int q = 0; q < C::NDMA; ++q) at[1][q] = OFF_NONE;
+    stat_at = OFF_NONE;
+  }
 };
 
 // The lane's operands of ROWS = 32 resident rows (row ln; 16 bytes per 16-deep contraction step) out of rows that were
@@ -839,11 +845,16 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     if (n == 2 * C::NDMA) {
       load_to_lds_b32(stat_rsrc, MAP ? tiles.stat_at : i < nt ? (unsigned)(i * BWD_ROWS + lane) * 4u : OFF_NONE, st + 2 * C::TILEB + (w & 1) * (BWD_ROWS * 4));
     } else if constexpr (MAP) {
-      if (n == 0) tiles.find(map, p.map, i * BWD_ROWS, p.Sq, qld, dold, lane, i < nt);
+      if (n == 0) {
+        if (QG == 1 || i < nt)
+          tiles.find(map, p.map, i * BWD_ROWS, p.Sq, qld, dold, lane, i < nt);
+        else
+          tiles.repeat_first();
+      }
       const int t = n / C::NDMA, q = n % C::NDMA;
       load_to_lds_b128(t ? dold.rsrc : qld.rsrc, tiles.at[t][q], dst + t * C::TILEB + q * (BWD_THREADS * 16));
     } else if (n < C::NDMA) {
-      qld.load(n, i < nt, i * BWD_ROWS, dst, map, p.map.pitch);
+      qld.load(n, QG == 2 || i < nt, (QG == 2 && i >= nt ? nt - 1 : i) * BWD_ROWS, dst, map, p.map.pitch);
     } else {
       dold.load(n - C::NDMA, i < nt, i * BWD_ROWS, dst + C::TILEB, map, p.map.pitch);
     }
@@ -949,7 +960,10 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     auto lse_of = [&](int i) { return own_lse + (unsigned)((i & 1) * (BWD_ROWS * 4)); };
     float lse_row;
     auto read_lse_row = [&](unsigned stage) { lse_row = *(const lds_float*)(lds_u8*)(uintptr_t)(stage + 2 * C::TILEB + 4 * lane); };
-    auto write_lse_row = [&](unsigned at) { *(lds_float*)(lds_u8*)(uintptr_t)(at + 4 * lane) = lse_row * -1.4426950408889634f; };
+    // (QG = 2, behind the last tile: P = 0 for its rows, which are the last tile's of Q; rows of zeros would give NaN where a key holds an infinity)
+    auto write_lse_row = [&](int i) {
+      *(lds_float*)(lds_u8*)(uintptr_t)(lse_of(i) + 4 * lane) = QG == 1 || i < nt ? lse_row * -1.4426950408889634f : -INFINITY;
+    };
     auto load_lse = [&](f32x4 (&l)[2], unsigned at, int row) {
 #pragma unroll
       for (int g = 0; g < 2; ++g) l[g] = __builtin_bit_cast(f32x4, lds_read_b128(at + 16 * hh + (row + 8 * g) * 4));
@@ -1041,13 +1055,13 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
 
     // Before the loop: S, dP of half 0 and what the first group of half 0 would do, less the gradients of a half before it.
     read_lse_row(stage_of(it0));
-    write_lse_row(lse_of(it0));
+    write_lse_row(it0);
     load_lse(ln_cur, lse_of(it0), 32 * qg);
     load_lse(ln_next, lse_of(it0), 32 * qg + 16);
     load_delta(d0, stat_at, 32 * qg);
     if constexpr (QG == 2) {
       read_lse_row(stage_of(it0 + 1));
-      write_lse_row(lse_of(it0 + 1));
+      write_lse_row(it0 + 1);
       stat_at += stage_of(it0 + 1) - stage_of(it0);
       load_delta(d1, stat_at, 32 * qg);
     } else {
@@ -1101,7 +1115,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
         ln_cur[1] = ln_next[1];
         // a row of lse for the wave's copy; the next group's lse rows; what dP of the half-tile in production starts from
         if (group == 0) read_lse_row(stage_of(i + QG));
-        if (group == 1) write_lse_row(lse_of(i + QG));
+        if (group == 1) write_lse_row(i + QG);
         if constexpr (QG == 2) {
           if (group == 1) {
             stat_at += next_step;
@@ -1153,7 +1167,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
       for (; i < nt; ++i) pass(i, s0, d0, s1, d1, Flag<false>());
     } else {
       // The diagonal of 64 keys is in tile it0, whose S has been seen to.  Passes in pairs, as S and dP change registers from one to the next
-      // (a pass behind the last tile adds products of zeros).
+      // (a pass behind the last tile adds zeros: see write_lse_row; left out, the accumulators are copied where the loop has two ends).
       for (; i < nt; i += 2) {
         pass(i, s0, d0, s1, d1, Flag<false>());
         pass(i + 1, s1, d1, s0, d0, Flag<false>());

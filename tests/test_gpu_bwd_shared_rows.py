@@ -42,3 +42,26 @@ def test_forms_with_shared_rows(D, dq, dkdv, dtype):
     finally:
         _lib.tune("bwd_dq_waves", 0)
         _lib.tune("bwd_dkdv_form", 0)
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+@pytest.mark.parametrize("S", [64, 128, 192])  # odd and even numbers of tiles, all of them full
+def test_a_key_that_holds_an_infinity(S, D, dtype):
+    """A key hidden by -inf in one head dim has no weight: its gradients are zero, not NaN, also where passes come in pairs and one lies behind
+    the last tile (dq, 0 * inf, is NaN)."""
+    q, k, v, dout = rand_qkv((1, S, 2, D), 740 + S, dtype, n=4)
+    q[..., 0], k[..., 0] = 1.0, 0.0
+    k[:, S // 2, :, 0] = -float("inf")
+    _, want_dk, want_dv = O.attn_backward_autograd(q, k, v, dout, None, False)
+    assert want_dk.isfinite().all() and want_dv.isfinite().all()
+    stack = lambda t, P: torch.stack(t.to(DEV).chunk(P, 1)).contiguous()
+    try:
+        for form in (2, 3):
+            _lib.tune("bwd_dkdv_form", form)
+            for P in (1, 2):
+                xs = [stack(t, P).requires_grad_(True) for t in (q, k, v)]
+                spa.LongContextAttention(sp_ulysses_degree=1, sp_ring_degree=P)(*xs, causal=False).backward(stack(dout, P))
+                for x, w, name in zip(xs[1:], (want_dk, want_dv), "kv"):
+                    check_grad(torch.cat(list(x.grad), 1), w, dtype, f"d{name}, form {form}, {P} shards")
+    finally:
+        _lib.tune("bwd_dkdv_form", 0)
