@@ -10,8 +10,8 @@
 // At the end the groups of a wave merge by shuffles and the waves of the workgroup through LDS.
 //
 // Grid: x = batch * head (or group of HP heads), y = key chunk (the key split of the caller: chunk y writes rows y * Sq .. of the result
-// tensors it is given; of a packed batch, whose sequences have chunks of one length and as many as they need: fp32 partial
-// sums, merged by fewrows_combine_kernel).  256 or 512 threads.
+// tensors it is given).  A packed batch whose keys are cut (chunks of one length, as many as a sequence needs): x = chunk * head, the
+// chunks of all sequences numbered through (chunk_of); fp32 partial sums, merged by fewrows_combine_kernel.  256 or 512 threads.
 #include "spa_common.h"
 #include "spa_host.h"
 
@@ -57,13 +57,51 @@ struct Piece<T, true> {
 };
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-// What a chunk of a packed batch leaves in the workspace: per (sequence, head, row, chunk) D sums, and behind all of those (max, sum).
-__host__ __device__ inline int64_t part_stats(int64_t pairs, int nq, int n, int D) { return pairs * nq * n * D; }
+// What a chunk of a packed batch leaves in the workspace: per (chunk, head, row) D sums, and behind all of those (max, sum).
+__host__ __device__ inline int64_t part_stats(int64_t pairs, int nq, int D) { return pairs * nq * D; }
+
+// The number of a sequence's first chunk of `chunk` keys: those of the sequences before it take no more than this, whatever their lengths
+// (rounding each up costs less than one number a sequence), so it needs no sum over them, and the longest sequence decides nothing: all
+// numbers are total / chunk + sequences, of which at most one a sequence stays without keys.  (Numbered by sequence, with as many chunks for each as
+// twice the mean and the rest in the last, one workgroup a head read most of a cache far longer than the others: one of 32768 tokens and 63 of 512, H = 32,
+// D = 128, e4m3 986 -> 106 us, bf16 929 -> 178; one of 16384 and 63 of 1024 487 -> 117, 518 -> 212; four of 8192 and 60 of 1024 262 -> 135, 319 -> 243;
+// 64 of 1 to 4 thousand 233 -> 224, 413 -> 415.)
+__device__ __forceinline__ int first_chunk(int k_begin, int seq, int chunk) { return (int)((unsigned)k_begin / (unsigned)chunk) + seq; }
+// The sequence that owns chunk number `slot`, which of its chunks that is (negative: in front of the first), and its rows.  Called by whole waves: each
+// step looks at 64 sequences, evenly spaced; the last reads all offsets at once, so that lists of up to 64 take one memory latency.
+struct ChunkOwner {
+  int seq, z, q_begin, q_end, k_begin, k_end;
+};
+__device__ __forceinline__ ChunkOwner chunk_of(const int* cu_q, const int* cu_k, int nseq, int chunk, int slot, int lane) {
+  int lo = 0, n = nseq;
+  while (n > 64) {
+    const int step = (n + 63) / 64, i = lane * step;
+    const bool before = i < n && first_chunk(cu_k[lo + i], lo + i, chunk) <= slot;
+    const int k = __builtin_popcountll(__builtin_amdgcn_ballot_w64(before));
+    if (k > 1) {
+      lo += (k - 1) * step;
+      n -= (k - 1) * step;
+    }
+    n = n < step ? n : step;
+  }
+  const int i = lo + (lane < n ? lane : n - 1);
+  const int k0 = cu_k[i], k1 = cu_k[i + 1], q0 = cu_q[i], q1 = cu_q[i + 1];
+  const int found = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < n && first_chunk(k0, i, chunk) <= slot)), at = found ? found - 1 : 0;
+  ChunkOwner r;
+  r.seq = lo + at;
+  r.k_begin = __builtin_amdgcn_readlane(k0, at);
+  r.k_end = __builtin_amdgcn_readlane(k1, at);
+  r.q_begin = __builtin_amdgcn_readlane(q0, at);
+  r.q_end = __builtin_amdgcn_readlane(q1, at);
+  r.z = slot - first_chunk(r.k_begin, r.seq, chunk);
+  return r;
+}
 
 // kWaves: waves of a workgroup.  kUnroll: loads of K (and of V) a wave keeps in flight.  NT: the loads carry the non-temporal hint (K and V are read
 // once and should not displace anything in the caches).
-// HP: neighbouring heads a workgroup takes together, whose pieces of a key row lie side by side.
-template <typename T, int D, bool KV8, int NQ, int kUnroll, bool NT, int HP, int kWaves>
+// HP: neighbouring heads a workgroup takes together, whose pieces of a key row lie side by side.  CHUNKS: a packed batch whose keys are cut (a variant
+// of its own: the search costs the others two registers, and with three rows half of the waves).
+template <typename T, int D, bool KV8, int NQ, int kUnroll, bool NT, int HP, int kWaves, bool CHUNKS>
 __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParams p) {
   constexpr int AUX = NT ? 2 : 0;
   typedef Piece<T, KV8> Pc;
@@ -79,29 +117,49 @@ __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParam
   // neighbouring heads share every line: they are given to workgroups 8 apart, which run on one XCD at about the same
   // time, so that the line comes from HBM once (3.1 -> 4.6-5.1 TB/s; with rows of a whole line or more the same
   // placement is 3-10 % slower than heads round robin).
+  // (Chunks of a packed batch, which are not of one size, stay spread over the XCDs: neighbours change places inside 16 workgroups.)
   int bh = blockIdx.x;
-  if (D * KESZ * HP < 128 && (gridDim.x & 7) == 0) bh = (bh & 7) * (int)(gridDim.x >> 3) + (bh >> 3);
+  if (D * KESZ * HP < 128) {
+    if (!CHUNKS) {
+      if ((gridDim.x & 7) == 0) bh = (bh & 7) * (int)(gridDim.x >> 3) + (bh >> 3);
+    } else if ((unsigned)(bh | 15) < gridDim.x) {
+      bh = (bh & ~15) | ((bh & 7) << 1) | ((bh >> 3) & 1);
+    }
+  }
   bh *= HP;
-  const int z = blockIdx.y;
+  int z = blockIdx.y;
   int b = bh / p.H;
   const int h = bh - b * p.H;                    // the first of the heads
+  const int slot = b;                            // (CHUNKS)
+  ChunkOwner seq;                                // (packed batches)
+  if constexpr (CHUNKS) {
+    seq = chunk_of(p.cu_q, p.cu_k, p.B, p.Sk, slot, (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
+    // (the same in all lanes, which the compiler does not see: descriptors built lane by lane cost up to 15 %)
+    for (int* const x : {&seq.q_begin, &seq.q_end, &seq.k_begin, &seq.k_end, &seq.seq, &seq.z}) *x = __builtin_amdgcn_readfirstlane(*x);
+    b = seq.seq;
+    z = seq.z;
+    if (z < 0) return;
+    bh = b * p.H + h;
+  } else if (p.cu_q) {
+    seq = {b, 0, p.cu_q[b], p.cu_q[b + 1], p.cu_k[b], p.cu_k[b + 1]};
+  }
   const int c = lane % LPR, g = lane / LPR;
   const int own = c / LPH;                       // this lane's head is h + own
   int k0 = z * p.Sk;
-  int k1 = k0 + (z == p.P - 1 ? p.sk_last : p.Sk);
+  int k1 = k0 + (z == p.P - 1 && !CHUNKS ? p.sk_last : p.Sk);
   int nq = NQ;                                   // rows of this (batch or sequence, head) that exist
   int64_t q_row0 = 0, k_row0 = 0;                // first row of the sequence in the packed tensors
   int64_t lse_base = (int64_t)bh * p.lse_bh;     // of head h; lse is [B, H, rows], or [H, packed rows] for a packed batch
   if (p.cu_q) {
     // a packed variable-length batch: sequence b owns rows cu_q[b] .. of q / out / lse and cu_k[b] .. of K / V, and
-    // this workgroup chunk z of its keys (the last chunk of the grid takes what is left)
-    q_row0 = p.cu_q[b];
-    k_row0 = p.cu_k[b];
-    nq = p.cu_q[b + 1] - (int)q_row0;
+    // this workgroup all of them or chunk z
+    q_row0 = seq.q_begin;
+    k_row0 = seq.k_begin;
+    nq = seq.q_end - seq.q_begin;
     nq = nq < NQ ? nq : NQ;
-    k1 = p.cu_k[b + 1] - (int)k_row0;
-    if (z > 0 && k0 >= k1) return;
-    if (z != p.P - 1 && k1 > k0 + p.Sk) k1 = k0 + p.Sk;
+    k1 = seq.k_end - seq.k_begin;
+    if (z > 0 && (int64_t)z * p.Sk >= k1) return;
+    if (CHUNKS && k1 - k0 > p.Sk) k1 = k0 + p.Sk;
     lse_base = (int64_t)h * p.lse_bh + q_row0;
     b = 0;
     if (nq <= 0) return;
@@ -259,44 +317,74 @@ __global__ void __launch_bounds__(kWaves * 64) fewrows_fwd_kernel(const FwdParam
       a += sm_acc[i][w][hd * D + d] * f;
     }
     if (i >= nq) break;
-    if (p.cu_q && p.P > 1) {
-      const int64_t at = ((int64_t)(bh + hd) * NQ + i) * p.P + z;
+    if (CHUNKS && seq.k_end - seq.k_begin > p.Sk) {  // not all of the sequence
+      const int64_t at = ((int64_t)slot * p.H + h + hd) * NQ + i;
       ((float*)p.part)[at * D + d] = a;
-      if (d == 0) *(f32x2*)((float*)p.part + part_stats((int64_t)p.B * p.H, NQ, p.P, D) + at * 2) = f32x2{mx, ls};
+      if (d == 0) *(f32x2*)((float*)p.part + part_stats((int64_t)p.P * p.H, NQ, D) + at * 2) = f32x2{mx, ls};
       continue;
     }
-    const int64_t orow = (int64_t)z * p.Sq + i;
+    const int64_t orow = (int64_t)z * p.Sq + i;  // (z = 0 for a sequence of a packed batch)
     T* op = (T*)p.out + b * p.os.b + (h + hd) * p.os.h + (q_row0 + orow) * p.os.s;
     op[d] = (T)(a * vmul / ls);
     if (d == 0) p.lse[lse_base + hd * p.lse_bh + orow] = (mx + __builtin_amdgcn_logf(ls)) * 0.6931471805599453f;
   }
 }
 
-// Merges the chunks of a packed batch's rows: a workgroup of D threads per (sequence, head), a thread one element of each row.
+// Merges the chunks of a packed batch's rows: a workgroup per (sequence, head), a thread one element of every 256 / D-th chunk, eight of them in flight
+// (one after the other they are a chain of memory latencies: 64 caches of 1 to 4 thousand tokens, H = 32, 7.2 -> 6.6 us; 256 chunks of one cache 18 us).
+// A sequence of one chunk has its result from the first kernel (1999 caches of 200 tokens and one of 2500, H = 32, 44 -> 15 us).
 template <typename T, int D>
-__global__ void __launch_bounds__(D) fewrows_combine_kernel(const FwdParams p) {
-  const int bh = blockIdx.x, b = bh / p.H, h = bh - b * p.H, d = threadIdx.x;
-  const int q_row0 = p.cu_q[b], keys = p.cu_k[b + 1] - p.cu_k[b];
+__global__ void __launch_bounds__(256) fewrows_combine_kernel(const FwdParams p) {
+  constexpr int G = 256 / D, AHEAD = 8;
+  const int bh = blockIdx.x, b = bh / p.H, h = bh - b * p.H, tid = threadIdx.x, d = tid % D, g = tid / D;
+  const int q_row0 = p.cu_q[b], k_row0 = p.cu_k[b], keys = p.cu_k[b + 1] - k_row0;
   int nq = p.cu_q[b + 1] - q_row0;
   nq = nq < p.Sq ? nq : p.Sq;
-  if (keys <= 0) return;  // (written by chunk 0)
-  const int have = (keys - 1) / p.Sk + 1, n = have < p.P ? have : p.P;
+  if (keys <= p.Sk) return;  // (written by chunk 0)
+  const int first = first_chunk(k_row0, b, p.Sk), have = (keys - 1) / p.Sk + 1, n = have < p.P - first ? have : p.P - first;
   const float vmul = p.k_scale ? p.v_scale[bh] : 1.f;
+  __shared__ float weight[256], sums[256], ls[4];
   for (int i = 0; i < nq; ++i) {
-    const int64_t at = ((int64_t)bh * p.Sq + i) * p.P;
+    const int64_t at = ((int64_t)first * p.H + h) * p.Sq + i, next = (int64_t)p.H * p.Sq;  // of chunk 0; from chunk to chunk
     const float* const part = (const float*)p.part + at * D + d;
-    const f32x2* const ml = (const f32x2*)((const float*)p.part + part_stats(gridDim.x, p.Sq, p.P, D)) + at;
-    float mx = ml[0][0];
-    for (int j = 1; j < n; ++j) mx = fmaxf(mx, ml[j][0]);
+    const f32x2* const ml = (const f32x2*)((const float*)p.part + part_stats((int64_t)p.P * p.H, p.Sq, D)) + at;
+    float mx = -INFINITY;  // (every wave for itself)
+    for (int j = tid & 63; j < n; j += 64) mx = fmaxf(mx, ml[j * next][0]);
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
     const float ms = mx == -INFINITY ? 0.f : mx;
     float a = 0.f, l = 0.f;
-    for (int j = 0; j < n; ++j) {
-      const float f = __builtin_amdgcn_exp2f(ml[j][0] - ms);
-      a += part[(int64_t)j * D] * f;
-      l += ml[j][1] * f;
+    for (int j0 = 0; j0 < n; j0 += 256) {
+      const int m = n - j0 < 256 ? n - j0 : 256;
+      if (tid < m) {
+        const f32x2 x = ml[(j0 + tid) * next];
+        weight[tid] = __builtin_amdgcn_exp2f(x[0] - ms);
+        l += x[1] * weight[tid];
+      }
+      __syncthreads();
+      for (int j = g; j < m; j += AHEAD * G) {
+        float x[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) x[u] = part[(j0 + (j + u * G < m ? j + u * G : j)) * next * D];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+          if (j + u * G < m) a += x[u] * weight[j + u * G];
+      }
+      __syncthreads();
     }
-    ((T*)p.out)[h * p.os.h + (int64_t)(q_row0 + i) * p.os.s + d] = (T)(a * vmul / l);
-    if (d == 0) p.lse[(int64_t)h * p.lse_bh + q_row0 + i] = (mx + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) l += __shfl_xor(l, off, 64);
+    sums[tid] = a;
+    if ((tid & 63) == 0) ls[tid >> 6] = l;
+    __syncthreads();
+    if (g == 0) {
+      l = (ls[0] + ls[1]) + (ls[2] + ls[3]);
+#pragma unroll
+      for (int k = 1; k < G; ++k) a += sums[k * D + d];
+      ((T*)p.out)[h * p.os.h + (int64_t)(q_row0 + i) * p.os.s + d] = (T)(a * vmul / l);
+      if (d == 0) p.lse[(int64_t)h * p.lse_bh + q_row0 + i] = (mx + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
+    }
+    __syncthreads();
   }
 }
 
@@ -305,14 +393,15 @@ __global__ void __launch_bounds__(D) fewrows_combine_kernel(const FwdParams p) {
 // on e4m3 heads taken together (12 % split), and loses where workgroups share lines (64-byte rows) and on split calls of single e4m3 heads.
 template <typename T, int D, bool KV8, int NQ, int U, int HP, int W = 4>
 hipError_t launch_variant(const FwdParams& p, hipStream_t stream) {
-  const dim3 grid((unsigned)(p.B * p.H / HP), (unsigned)p.P), block(W * 64);
+  const bool chunks = p.cu_q && p.part;
+  const dim3 grid((unsigned)((int64_t)(chunks ? p.P : p.B) * p.H / HP), chunks ? 1u : (unsigned)p.P), block(W * 64);
   constexpr bool hint = !KV8 || HP > 1;
-  if constexpr (hint || D == 64) {
-    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, hint, HP, W>), grid, block, 0, stream, p);
-  } else if (p.P == 1) {
-    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, true, HP, W>), grid, block, 0, stream, p);
-  } else {
-    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, false, HP, W>), grid, block, 0, stream, p);
+  if (chunks) {
+    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, hint, HP, W, true>), grid, block, 0, stream, p);
+  } else if (hint || D == 64 || p.P > 1) {
+    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, hint, HP, W, false>), grid, block, 0, stream, p);
+  } else if constexpr (!hint && D != 64) {  // (keys not split)
+    hipLaunchKernelGGL((fewrows_fwd_kernel<T, D, KV8, NQ, U, true, HP, W, false>), grid, block, 0, stream, p);
   }
   return hipGetLastError();
 }
@@ -323,16 +412,19 @@ hipError_t launch_variant(const FwdParams& p, hipStream_t stream) {
 // a workgroup: with one per CU and single heads 44 us, 48 together (B = 1, 32768 keys, e4m3, D = 128).
 // Rows of 128 elements, and eight workgroups per CU left: as many heads as make 512 bytes (64 caches of 2 to 8 thousand tokens, H = 32: e4m3 461 ->
 // 439 us, bf16 875 -> 839; of 1 to 4 thousand 237 -> 234 and 442 -> 435).  With fewer the last workgroups count for more: 32 caches of
-// 512 to 2048, e4m3, two per CU, 65 -> 75; 8 of 2 to 8 thousand, bf16, four, 118 -> 124.
+// 512 to 2048, e4m3, two per CU, 65 -> 75; 8 of 2 to 8 thousand, bf16, four, 118 -> 124.  Nor where one sequence, which is twice as long in such a
+// workgroup, is a good part of the whole launch: 255 caches of 256 tokens and one of 2200, e4m3 116 -> 155, bf16 194 -> 216.
 // A launch that leaves half of the CUs without a workgroup (a caller who did not split the keys) is bound by what its
 // few waves keep in flight: eight loads there too.
 template <typename T, int D, bool KV8, int NQ>
 hipError_t launch_unroll(const FwdParams& p, hipStream_t stream) {
   constexpr int HP = 256 / (D * (KV8 ? 1 : 2));
-  const int64_t groups = (int64_t)p.B * p.H * p.P;
+  const int64_t groups = (int64_t)(p.cu_q && p.part ? 1 : p.B) * p.H * p.P;
   if constexpr (D == 128) {
     constexpr int WIDE = 2 * HP;
-    if (p.H % WIDE == 0 && p.ks.h == D && p.vs.h == D && groups / WIDE >= 8 * spa_device_cus())
+    // (a packed batch: what one workgroup has to read, the longest sequence or a chunk, at 44 GB/s; all that is read, at 6 TB/s)
+    const double longest = p.Sk * 1024.0 / 44e9, all = (double)p.chunk_rows * p.H * D * (KV8 ? 2 : 4) / 6e12;
+    if (p.H % WIDE == 0 && p.ks.h == D && p.vs.h == D && groups / WIDE >= 8 * spa_device_cus() && (!p.cu_q || 4 * longest <= all))
       return launch_variant<T, D, KV8, NQ, NQ == 3 ? 8 : 4, WIDE>(p, stream);
   }
   if constexpr (HP > 1) {
@@ -365,8 +457,8 @@ hipError_t launch_nq(const FwdParams& p, hipStream_t stream) {
 template <typename T, int D>
 hipError_t launch_d(const FwdParams& p, hipStream_t stream) {
   const hipError_t e = p.k_scale ? launch_nq<T, D, true>(p, stream) : launch_nq<T, D, false>(p, stream);
-  if (e != hipSuccess || !p.cu_q || p.P == 1) return e;
-  hipLaunchKernelGGL((fewrows_combine_kernel<T, D>), dim3((unsigned)(p.B * p.H)), dim3(D), 0, stream, p);
+  if (e != hipSuccess || !p.cu_q || !p.part) return e;
+  hipLaunchKernelGGL((fewrows_combine_kernel<T, D>), dim3((unsigned)(p.B * p.H)), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -381,13 +473,17 @@ hipError_t launch_t(const FwdParams& p, int D, hipStream_t stream) {
 
 // The caller's FwdParams as for the key-split launch: Sk = keys per chunk, sk_last = keys of the last chunk, P = number of
 // chunks; out / lse take rows z * Sq + i of chunk z.  No mask, 1 <= Sq <= 3, 16-bit q / out, K/V of one
-// (batch, head) below 2 GiB, 16-byte aligned K/V rows.  A packed variable-length batch: cu_q, cu_k; Sq = the longest
-// sequence's rows, B = sequences; with P > 1 chunks of Sk keys and their sums in `part`.
+// (batch, head) below 2 GiB, 16-byte aligned K/V rows.  A packed variable-length batch: cu_q, cu_k; Sq, Sk = the longest sequence's rows
+// and keys, B = sequences, chunk_rows = rows of K and V; with `part` Sk = keys of a chunk and P = spa_fewrows_chunks(), whose sums go there.
 hipError_t spa_launch_fwd_fewrows(FwdParams p, int D, int dtype, hipStream_t stream) {
-  if (p.causal || (p.cu_q && p.P != 1 && !p.part) || p.q_scale || p.big || p.Sq < 1 || p.Sq > 3 || p.P < 1 || p.P > 65535) return hipErrorInvalidValue;
+  const bool chunks = p.cu_q && p.part;
+  if (p.causal || (p.cu_q && p.P != 1 && !p.part) || p.q_scale || p.big || p.Sq < 1 || p.Sq > 3 || p.P < 1 || p.Sk < 1 ||
+      (chunks ? (int64_t)p.P * p.H > 0x7fffffffLL : p.P > 65535))
+    return hipErrorInvalidValue;
   if (dtype == 1) return launch_t<__bf16>(p, D, stream);
   if (dtype == 2) return launch_t<_Float16>(p, D, stream);
   return hipErrorInvalidValue;
 }
 
-int64_t spa_fewrows_part_floats(int64_t pairs, int nq, int n, int D) { return part_stats(pairs, nq, n, D) + pairs * nq * n * 2; }
+int64_t spa_fewrows_chunks(int nseq, int total_k, int chunk) { return (int64_t)total_k / chunk + nseq; }
+int64_t spa_fewrows_part_floats(int64_t pairs, int nq, int D) { return part_stats(pairs, nq, D) + pairs * nq * 2; }

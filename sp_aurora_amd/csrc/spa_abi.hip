@@ -19,7 +19,8 @@ static __device__ __align__(256) unsigned char scratch[SPA_STATIC_SCRATCH_BYTES]
 hipError_t spa_launch_flash_fwd(FwdParams p, int D, int dtype, hipStream_t stream);
 hipError_t spa_launch_fwd16_splitkv(FwdParams p, int D, int dtype, hipStream_t stream);
 hipError_t spa_launch_fwd_fewrows(FwdParams p, int D, int dtype, hipStream_t stream);
-int64_t spa_fewrows_part_floats(int64_t pairs, int nq, int n, int D);
+int64_t spa_fewrows_chunks(int nseq, int total_k, int chunk);
+int64_t spa_fewrows_part_floats(int64_t pairs, int nq, int D);
 hipError_t spa_launch_splitkv_combine(void* out, float* lse, const void* part, const float* part_lse, int n, int B, int H, int Sq,
                                       int D, Strides3 os, int64_t lse_bh, int dtype, hipStream_t stream);
 hipError_t spa_launch_flash_bwd(BwdParams p, int D, int dtype, hipStream_t stream);
@@ -844,13 +845,6 @@ int varlen_sizes_ok(const char* what, const void* cu_q, const void* cu_k, int ns
 }  // extern "C"
 
 namespace {
-// Chunks per sequence of a packed batch: enough for the longest, but no more than twice the mean sequence's and two (max_sk may be a
-// bound that no sequence is near); the last takes what is left.
-int varlen_chunks(int nseq, int total_k, int max_sk, int chunk) {
-  const int64_t longest = ((int64_t)max_sk - 1) / chunk + 1, mean = (int64_t)total_k / nseq / chunk + 1;
-  return (int)(longest < 2 * mean + 2 ? longest : 2 * mean + 2);
-}
-
 int flash_fwd_varlen(const char* what, const void* q, const void* k, const void* v, const float* k_scale,
                      const float* v_scale, void* out, float* lse, const int32_t* cu_seqlens_q,
                      const int32_t* cu_seqlens_k, int nseq, int H, int total_q, int total_k, int max_sq, int max_sk,
@@ -908,10 +902,13 @@ int flash_fwd_varlen(const char* what, const void* q, const void* k, const void*
   if (P == 1 && !p.causal && dtype != SPA_F32 && D != 32 && !p.big && max_sq <= kFewRows && spa_knob(SPA_KNOB_FEW_ROWS) != 1 &&
       (!kv8 || (aligned16v(k, k_strides, 1) && aligned16v(v, v_strides, 1)))) {
     p.sk_last = max_sk;
+    p.chunk_rows = total_k;
     if (chunk > 0 && chunk < max_sk) {
       if (!workspace || ((uintptr_t)workspace & 15) != 0) return fail(SPA_EINVAL, "%s: the key split needs a 16-byte aligned workspace", what);
-      p.P = varlen_chunks(nseq, total_k, max_sk, chunk);
-      if (p.P > 65535 || (int64_t)p.P * chunk > 0x7fffffffLL) return fail(SPA_EINVAL, "%s: grid too large", what);
+      const int64_t n = spa_fewrows_chunks(nseq, total_k, chunk);
+      // (nor more than 65535 chunks of a sequence, the mean's as well)
+      if (n * H > 0x7fffffffLL || ((max_sk - 1) / chunk >= 65535 && total_k / nseq / chunk >= 32766)) return fail(SPA_EINVAL, "%s: grid too large", what);
+      p.P = (int)n;
       p.Sk = chunk;
       p.part = workspace;
     }
@@ -1048,7 +1045,7 @@ extern "C" {
 
 int64_t spa_flash_fwd_varlen_splitkv_workspace_bytes(int nseq, int H, int total_k, int max_sq, int max_sk, int D, int chunk) {
   if (nseq <= 0 || H <= 0 || total_k <= 0 || max_sq <= 0 || max_sq > kFewRows || max_sk <= 0 || D <= 0 || chunk <= 0) return -1;
-  return 4 * spa_fewrows_part_floats((int64_t)nseq * H, max_sq, varlen_chunks(nseq, total_k, max_sk, chunk), D);
+  return 4 * spa_fewrows_part_floats(spa_fewrows_chunks(nseq, total_k, chunk) * H, max_sq, D);
 }
 
 // Fewer workgroups than CUs: chunks that give every CU one, of at least 256 keys (8 caches of 2 to 8 thousand tokens, H = 8, bf16, D = 128:
@@ -1056,8 +1053,8 @@ int64_t spa_flash_fwd_varlen_splitkv_workspace_bytes(int nseq, int H, int total_
 // of K and V, whatever the type: heads are taken together, launch_unroll), since the second kernel costs 3 to 5 us; then chunks of
 // 1024 keys (64 caches of 1 to 4 thousand tokens, H = 32: bf16 437 -> 413 us; 2 to 8 thousand, H = 8, e4m3 145 -> 122; 512 and 2048
 // are 1 to 4 % slower), or, at D = 128, of 512 while those are 16 thousand workgroups of one head or fewer and the last of them count (1024 / 512,
-// us, longest of 4096: 64, H = 32, e4m3 234.3 / 228.0, bf16 435.3 / 429.8; of 8192: 8, H = 32, 72.8 / 71.9 and 118.5 / 114.4, 32, H = 8, 75.5 /
-// 72.7 and 125.2 / 123.7, but 64, H = 32, 437 / 446 and 836 / 843; D = 64, 32 of 4096, H = 8, bf16 38.1 / 40.5).
+// us, longest of 4096: 64, H = 32, e4m3 232 / 224, bf16 438 / 438; of 8192: 8, H = 32, 63.5 / 59.5 and 130 / 125, 32, H = 8, 74.7 /
+// 65.4 and 125 / 122, but 64, H = 32, 483 / 487 and 808 / 812).
 int spa_flash_fwd_varlen_splitkv_suggest(int nseq, int H, int total_k, int max_sq, int max_sk, int D, int dtype) {
   if (nseq <= 0 || H <= 0 || total_k <= 0 || max_sq <= 0 || max_sq > kFewRows || max_sk <= 0 || (D != 64 && D != 128) ||
       (dtype != SPA_BF16 && dtype != SPA_F16) || spa_knob(SPA_KNOB_FEW_ROWS) == 1)

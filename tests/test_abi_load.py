@@ -356,3 +356,15 @@ def test_a_number_past_64_bits_is_the_python_paths():
     assert nat.varlen_attention(x, x, x, cu, cu, 4, 4, None, True, True, huge, False) is None
     assert nat.attention(x[None], x[None], x[None], None, True, huge) is None
     assert nat.flash_fwd(x[None], x[None], x[None], None, True, True, None, None, None, huge) is None
+
+
+def test_workspace_of_a_ragged_key_split_follows_the_keys():
+    """As many chunks as the keys make, and one a sequence: none is left with what others did not take, whatever the longest sequence's
+    length (or a bound on it)."""
+    lib = _lib.load()
+    size = lambda nseq, total, longest, chunk: lib.spa_flash_fwd_varlen_splitkv_workspace_bytes(nseq, 32, total, 1, longest, 128, chunk)
+    per_chunk = 4 * 32 * (128 + 2)
+    for nseq, total in ((64, 32768 + 63 * 512), (4, 4096), (1, 131072), (2000, 2001)):
+        for chunk in (1, 512, 1000):
+            for longest in (total // nseq + 1, total):
+                assert size(nseq, total, longest, chunk) == per_chunk * (total // chunk + nseq)

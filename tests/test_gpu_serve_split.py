@@ -176,3 +176,29 @@ def test_chunks_whose_keys_are_all_hidden(D, dtype):
         want = torch.einsum("bhqk,bkhd->bqhd", torch.softmax(s, -1), v.double()), torch.logsumexp(s, -1)
         got = ops.flash_fwd(q.to(DEV), kk.to(DEV), v.to(DEV), layout="bshd")
         check([t.cpu().double() for t in got], want, dtype)
+
+
+@pytest.mark.parametrize("nseq", [1, 2, 63, 64, 65, 129, 4095, 4097, 4200])
+@pytest.mark.parametrize("chunk", [1, 16, 100])
+def test_chunks_are_found_in_long_lists(nseq, chunk):
+    """The chunks of all sequences are numbered through: one far longer than the others (up to 1500 chunks), sequences without keys, lists
+    around the 64 sequences and the 64 * 64 that a step of the search takes, and offsets that do not begin at the first row."""
+    H, D, dtype, at = 2, 64, torch.float16, 150
+    lens = [((i * 37) % 41 if i % 5 else 0, 1) for i in range(nseq)]
+    lens[nseq // 3] = (1500, 2)
+    q, k, v, cu_q, cu_k, _ = caches(lens, H, D, dtype, False, 1400 + nseq)
+    want = reference(q, k, v, cu_q, cu_k, 2, 1500)
+    check_exact(want, exact(q, k, v, cu_q, cu_k), dtype)
+    check(split(q, k, v, cu_q, cu_k, 2, 1500, chunk), want, dtype)
+    behind = lambda t: torch.cat([torch.full_like(t[:1], float("nan")).expand(at, -1, -1), t])
+    check(split(q, behind(k), behind(v), cu_q, cu_k + at, 2, 1500, chunk), want, dtype)
+
+
+@pytest.mark.parametrize("H,fp8", [(8, False), (32, True)])
+def test_one_long_cache_beside_short_ones(H, fp8):
+    """The library's own choice of chunks, at D = 128: chunks of the one cache go to workgroups of their own, also with 512 bytes of heads each."""
+    lens = [(300, 1)] * 70 + [(20000, 1)] + [(257, 1)] * 20
+    q, k, v, cu_q, cu_k, scales = caches(lens, H, 128, torch.bfloat16, fp8, 1500)
+    want = reference(q, k, v, cu_q, cu_k, 1, 20000, **scales)
+    check_exact(want, exact(q, k, v, cu_q, cu_k, **scales), torch.bfloat16)
+    check(ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 1, 20000, **scales), want, torch.bfloat16)
