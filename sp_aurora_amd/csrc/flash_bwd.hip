@@ -623,7 +623,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   // Causal: the tiles a wave's rows see end with the one that holds its last row.  Behind that a wave only takes its share of the loads, and
   // leaves the matrix pipe to the wave beside it (of the 4 tiles on the diagonal of 256 rows, 1.5 on average).
   // (KG = 2: S and dP change registers from pass to pass, and the passes come in pairs; one behind the last tile has every key hidden.)
-  const int own_nt = (p.causal && qw0 / BWD_ROWS + 1 < nt ? qw0 / BWD_ROWS + 1 : nt) + KG - 1 & ~(KG - 1), all_nt = nt + KG - 1 & ~(KG - 1);
+  const int own_nt = qw0 >= p.Sq ? 0 : (p.causal && qw0 / BWD_ROWS + 1 < nt ? qw0 / BWD_ROWS + 1 : nt) + KG - 1 & ~(KG - 1), all_nt = nt + KG - 1 & ~(KG - 1);
   auto next_pass = [&]() {
     // tile i+1 must have landed before this body reads it (KG = 2: i+2); tile i-1 is free for tile i+AHEAD.  (The operands in flight, one read
     // each, are of tile i+1 or later.)
@@ -705,6 +705,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
     i += KG;
     if (i == own_nt) mfma_settle();
   }
+  if (own_nt == 0) mfma_settle();  // (a wave without rows)
   for (int i = own_nt; i < all_nt; ++i) {
     next_pass();
     issue_tile(i + AHEAD);
@@ -886,6 +887,10 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
   constexpr int BWD_LOOK = D <= 64 ? 4 : BWD_LOOK_MAX;  // (two waves per SIMD at D <= 64, as in the dq kernel)
   static_assert(GROUP % BWD_LOOK == 0, "the operand window must tile a group");
 
+  // A wave without keys, or with keys that no query sees, only takes its share of the loads: of a sequence of 16 rows three of four, which held up the
+  // fourth at LDS.  Causal, with the masks of halves that need none left out, 16 heads: 2000 sequences of 16 rows 942 -> 881 us, 1000 of 64 546 -> 522,
+  // 500 of 128 404 -> 395.
+  const bool idle = kw0 >= p.Sk || (p.causal && kw0 >= p.Sq);
   if (it0 < nt) {  // uniform; a workgroup whose keys no query sees adds nothing
     // the workgroup's keys first, as two tiles each of K and V in the stages of tiles it0 + 2 and it0 + 3 (64 keys: both in the last)
     {
@@ -926,6 +931,17 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): read, before the barrier of the first pass
     }
 
+  }
+  if (it0 < nt && idle) {
+    // its share of the loads, and the barriers of the passes (of which there is an even number with QG = 2)
+    for (int i = it0, end = QG == 1 ? nt : it0 + (nt - it0 + 1 & ~1); i < end; ++i) {
+      wait_loads_but<QG == 2 ? 0 : G::NL>();
+      __builtin_amdgcn_s_barrier();
+      issue_tile(i + 3);
+    }
+    wait_loads_but<0>();
+  }
+  if (it0 < nt && !idle) {
     // V negated: with delta as the accumulator's start the products give delta - dP, and -dS costs one multiplication per element.
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) {
@@ -979,6 +995,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     // diagonal: a key sees only the queries at or after it
     auto mask = [&](f32x16& sc, int half) {
       const int r0 = half * 32;
+      if (kw0 + 31 <= r0) return;
 #pragma unroll
       for (int v = 0; v < 16; ++v)
         if (krow > r0 + 8 * (v >> 2) + 4 * hh + (v & 3)) sc[v] = hidden;

@@ -7,6 +7,7 @@ from conftest import rand_qkv
 from oracle import attn_oracle as O
 import sp_aurora_amd as spa
 from sp_aurora_amd import _lib
+from test_gpu_many_sequences import reference as packed_reference
 from test_gpu_parity import DEV, check_grad
 
 pytestmark = pytest.mark.gpu
@@ -64,4 +65,28 @@ def test_a_key_that_holds_an_infinity(S, D, dtype):
                 for x, w, name in zip(xs[1:], (want_dk, want_dv), "kv"):
                     check_grad(torch.cat(list(x.grad), 1), w, dtype, f"d{name}, form {form}, {P} shards")
     finally:
+        _lib.tune("bwd_dkdv_form", 0)
+
+
+def packed_step(lens, q, k, v, dout, causal, longest=None):
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    xs = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+    out = spa.sp_aurora_varlen_func(*xs, cu, max_seqlen=longest or max(lens), causal=causal)
+    return torch.autograd.grad(out, xs, dout.to(DEV))
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (128, torch.float16), (64, torch.bfloat16)])
+@pytest.mark.parametrize("lens", [[1, 16, 0, 31, 33, 2], [64, 65, 96, 127, 128], [129, 3, 161, 200, 257]])
+def test_short_sequences_in_every_form(lens, D, dtype):
+    """Sequences that leave waves of a workgroup without rows or keys: those take part in loads and barriers only."""
+    q, k, v, dout = rand_qkv((sum(lens), 2, D), 760, dtype, n=4)
+    want = packed_reference(q, k, v, dout, lens)[1]
+    try:
+        for dq, dkdv in ((0, 0), (4, 3), (8, 1), (20, 2), (24, 3)):
+            _lib.tune("bwd_dq_waves", dq)
+            _lib.tune("bwd_dkdv_form", dkdv)
+            for g, w, name in zip(packed_step(lens, q, k, v, dout, True), want, "qkv"):
+                check_grad(g, w, dtype, f"d{name}, forms {dq} and {dkdv}")
+    finally:
+        _lib.tune("bwd_dq_waves", 0)
         _lib.tune("bwd_dkdv_form", 0)
