@@ -1700,27 +1700,48 @@ hipError_t launch(int smem, bool queries, int rows, BwdParams p, hipStream_t str
 
 // What a launch of one of the forms below takes, in microseconds on a chip that does nothing else: its longest chain of tiles, or the work of all
 // workgroups shared out over the CUs.  rows: what a workgroup owns (query rows of the dq kernel, keys of the dk / dv kernel), start: its
-// start and end, tile: a tile of 64 of the other side (both fitted to launches of 8 heads, 256 to 4096 causal rows).
-double launch_time(const BwdParams& p, bool queries, int rows, double start, double tile) {
-  const int64_t longest = p.cu_q ? longest_rows(p) : queries ? p.Sq : p.Sk;
-  const double pairs = (double)p.B * p.H, total = p.cu_q ? (queries ? (double)p.lse_bh : (double)p.total_k) : (double)p.B * longest;
-  const double mean = total / p.B, wgs = p.cu_q ? pairs * (mean / rows + 0.5) : pairs * ((longest + rows - 1) / rows);
-  // rows of the other side
-  const double top = (double)(p.cu_q ? (longest < total ? longest : total) : !queries ? p.Sq : p.causal && p.Sq < p.Sk ? p.Sq : p.Sk);
-  const double most = ceil(top / BWD_ROWS), other = p.cu_q ? mean : top;
-  const double usual = (p.causal ? (other + rows) / 2 : other) / BWD_ROWS;
-  // (Workgroups of one length go in whole rounds of one per CU; causal ones, the long ones first, and those of a ragged batch fill each other's gaps.
-  // Not causal, training step, us, rounds as a fraction / whole: 12 heads of 1536 rows 126 / 93, 16 of 1280 97 / 82, 64 of 640 103 / 97, 32 of 1536 199 / 188.)
-  const double rounds = wgs / spa_device_cus();
-  const double chain = start + tile * most, work = (p.causal || p.cu_q ? rounds : ceil(rounds)) * (start + tile * (usual < most ? usual : most));
+// start and end behind another's, alone: in a launch of few, tile: a tile of 64 of the other side (fitted to launches of 8 heads, 64 to 4096 causal rows,
+// and of thousands of workgroups of 16 to 512 rows).
+double launch_time(const BwdParams& p, bool queries, int rows, double start, double alone, double tile) {
+  const int cus = spa_device_cus(), shards = p.cu_q && p.map.P ? p.map.P : 1;
+  const double own = (double)(queries ? p.Sq : p.Sk) * shards;
+  double other = (double)(queries ? p.Sk : p.Sq) * shards;  // rows of the other side
+  if (p.causal && queries && own < other) other = own;
+  const double chain = alone + tile * ceil(other / BWD_ROWS);
+  // of a workgroup whose sequence has `o` rows on the other side
+  const auto tiles = [&](double o) {
+    const double n = (p.causal && (o + rows) / 2 < o ? (o + rows) / 2 : o) / BWD_ROWS;
+    return n < 1 ? 1 : n;
+  };
+  double work;
+  if (p.cu_q) {
+    // The host knows the longest sequence and the mean of the others, and counts a batch of those: a workgroup for every sequence however short it is, and
+    // one sequence that is longer than all others together as what it is (by the mean of all: one of 16384 rows and 100 of 128, 16 heads, 64 rows
+    // and 64 keys instead of 256 and 128, dq 1450 -> 1560 us, dk / dv 1980 -> 2440).
+    const double total = queries ? (double)p.lse_bh : (double)p.total_k, per_row = (queries ? (double)p.total_k : (double)p.lse_bh) / total;
+    const double rest = p.B > 1 && total > own ? (total - own) / (p.B - 1) : 0;
+    const bool alike = rest == own;
+    const auto cost = [&](double s) {
+      const double wgs = s <= rows ? 1 : alike ? ceil(s / rows) : s / rows + 0.5;
+      return wgs * (start + tile * tiles(s * per_row));
+    };
+    work = p.H * (cost(own) + (p.B - 1) * cost(rest)) / cus;
+  } else {
+    // (Workgroups of one length go in whole rounds of one per CU; causal ones, the long ones first, and those of a ragged batch fill each other's gaps.
+    // Not causal, training step, us, rounds as a fraction / whole: 12 heads of 1536 rows 126 / 93, 16 of 1280 97 / 82, 64 of 640 103 / 97, 32 of 1536 199 / 188.)
+    const double rounds = (double)p.B * p.H * ceil(own / rows) / cus;
+    work = (p.causal ? rounds : ceil(rounds)) * (start + tile * tiles(other));
+  }
   return chain > work ? chain : work;
 }
 
 // The forms of the dq kernel, D = 128: 256 rows a workgroup (8 waves, two a SIMD, the K/V stream shared by twice the rows) where there are many;
 // with fewer, 128 rows, or 64 (4 waves), whose waves share out the keys of a tile: more workgroups, each with a shorter chain.  Causal,
 // us, 256 / 128 / 64 rows: 8 heads of 2048 rows 61.4 / 37.8 / 29.5, 4096 119 / 76.8 / 63.8, 8192 263 / 187 / 227; 16 of 4096 138 / 101 / 125; 32 of 512
-// 20.5 / 15.4 / 12.6, 2048 76.4 / 58.5 / 79.2, 4096 181 / 196 / 259; 128 of 512 30.3 / 33.2 / 39.5.  (128 rows on 4 waves that do not share, one a SIMD: 44.9,
-// 86.7, 203; 107; 16.4, 60.7, 209; 33.0.  Taken for tensors of 2 GiB and more per (batch, head), and by a test that wants the bits of 256 rows.)
+// 20.5 / 15.4 / 12.6, 2048 76.4 / 58.5 / 79.2, 4096 181 / 196 / 259; 128 of 512 30.3 / 33.2 / 39.5.
+// 128 rows on 4 waves that do not share, one a SIMD, where sequences are short (and for tensors of 2 GiB and more per (batch, head)): it starts the
+// soonest.  Causal, us, 256 / 128 / 64 / 128 rows on 4 waves, 16 heads: 2000 sequences of 16 rows 988 / 1042 / 841 / 829, 1000 of 64 552 / 580 / 505 / 465, 500 of
+// 128 376 / 381 / 514 / 367, 400 of 160 377 / 558 / 611 / 504, 200 of 320 424 / 491 / 587 / 460; 8 of 192 13.7 / 13.2 / 16.7 / 12.2, 8 of 128 10.8 / 10.4 / 9.2 / 10.4.
 // D = 64: 128 rows, two workgroups to a CU, or 64 rows where those are two to a CU at most: 8 heads of 2048 rows 29.4 / 19.9, 4096 56.0 / 39.1, 8192
 // 128 / 119; 16 of 2048 30.0 / 21.6; 32 of 1024 18.7 / 14.3, 2048 36.9 / 36.9; 128 of 512 16.8 / 19.4.
 enum DqForm { DQ_128_PLAIN = 4, DQ_256 = 8, DQ_64 = 20, DQ_128 = 24 };  // the values of SPA_TUNE_BWD_DQ_WAVES
@@ -1734,8 +1755,10 @@ int dq_form(const BwdParams& p) {
     const double wgs = p.cu_q ? (double)p.H * ((double)p.lse_bh / 64 + p.B) : (double)p.B * p.H * ((p.Sq + 63) / 64);
     return wgs <= 2.0 * spa_device_cus() ? DQ_64 : DQ_128_PLAIN;
   }
-  const double t256 = launch_time(p, true, 256, 6.0, 1.76), t128 = launch_time(p, true, 128, 8.0, 0.92), t64 = launch_time(p, true, 64, 7.5, 0.69);
-  return t64 < t128 ? (t64 < t256 ? DQ_64 : DQ_256) : t128 < t256 ? DQ_128 : DQ_256;
+  const double t256 = launch_time(p, true, 256, 6.0, 7.0, 1.76), t128 = launch_time(p, true, 128, 8.0, 8.4, 0.92);
+  const double t64 = launch_time(p, true, 64, 7.5, 7.5, 0.69), plain = launch_time(p, true, 128, 5.5, 6.6, 1.2);
+  const DqForm form = t64 < t128 ? (t64 < t256 ? DQ_64 : DQ_256) : t128 < t256 ? DQ_128 : DQ_256;
+  return plain < (form == DQ_64 ? t64 : form == DQ_128 ? t128 : t256) ? DQ_128_PLAIN : form;
 }
 
 // Whether the dk / dv kernel takes 64 keys a workgroup.  Causal, us, 128 / 64 keys, D = 128: 8 heads of 512 rows 17.7 / 14.6, 2048 52.1 / 36.8, 4096
@@ -1750,7 +1773,7 @@ bool keys_64(const BwdParams& p) {
     const double wgs = p.cu_q ? (double)p.H * ((double)p.total_k / 64 + p.B) : (double)p.B * p.H * ((p.Sk + 63) / 64);
     return wgs <= (p.causal ? 2.0 : 1.0) * spa_device_cus();
   }
-  return launch_time(p, false, 64, 6.5, 0.975) < launch_time(p, false, 128, 4.7, 1.48);
+  return launch_time(p, false, 64, 6.5, 6.5, 0.975) < launch_time(p, false, 128, 4.7, 4.7, 1.48);
 }
 
 template <typename T, int D, int ADDR = ADDR_PLAIN>

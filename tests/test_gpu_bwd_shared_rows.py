@@ -90,3 +90,22 @@ def test_short_sequences_in_every_form(lens, D, dtype):
     finally:
         _lib.tune("bwd_dq_waves", 0)
         _lib.tune("bwd_dkdv_form", 0)
+
+
+def test_a_long_sequence_among_short_ones_decides_the_forms():
+    """Most of the work of such a batch is the one sequence's: 256 rows and 128 keys a workgroup, whose sums differ in their last bits from
+    those of 64."""
+    lens = [64] * 50 + [6000] + [128] * 50
+    q, k, v, dout = rand_qkv((sum(lens), 16, 128), 770, torch.bfloat16, n=4)
+    got = packed_step(lens, q, k, v, dout, True)
+    try:
+        grads = {}
+        for dq, dkdv in ((8, 3), (20, 2)):
+            _lib.tune("bwd_dq_waves", dq)
+            _lib.tune("bwd_dkdv_form", dkdv)
+            grads[dq] = packed_step(lens, q, k, v, dout, True)
+    finally:
+        _lib.tune("bwd_dq_waves", 0)
+        _lib.tune("bwd_dkdv_form", 0)
+    for g, a, b in zip(got, grads[8], grads[20]):
+        assert torch.equal(g, a) and not torch.equal(g, b)
