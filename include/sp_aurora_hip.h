@@ -548,6 +548,7 @@ int spa_attention_bwd_varlen(const void* q, const void* k, const void* v, const 
  *                          20 | 24 4 | 8 waves of which two share 32 query rows (head dims 64 and 128; 24: 128 only)
  *   SPA_TUNE_BWD_DKDV_FORM 1       compiler-scheduled MFMAs in the D = 128 dk/dv kernel
  *                          2 | 3   64 | 128 keys per workgroup of the dk/dv kernel (2: head dims 64 and 128)
+ *                          4 | 5   2 | 3 with compiler-scheduled MFMAs (at D = 128; otherwise as 2 | 3)
  *   SPA_TUNE_FWD32_SPLIT  1 | 2    never / always: the fp32 kernels with 32-row workgroups whose waves share
  *                                  the tiles (the library takes them where the longest chain of tiles decides)
  *   SPA_TUNE_FEW_ROWS     1        a key-split forward of up to 4 query rows runs on the MFMA kernels instead of the

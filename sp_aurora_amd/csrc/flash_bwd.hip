@@ -1766,7 +1766,7 @@ int dq_form(const BwdParams& p) {
 // CU: 8 of 2048 35.1 / 24.3, 4096 67.9 / 51.2; 16 of 4096 86.5 / 86.1; 32 of 1024 22.2 / 18.5, 2048 47.0 / 48.9; not causal 8 of 2048 36.9 / 27.6, 16 of 2048 41.4 / 41.2.
 template <int D, int ADDR>
 bool keys_64(const BwdParams& p) {
-  const int form = spa_knob(SPA_KNOB_BWD_DKDV_FORM);
+  const int knob = spa_knob(SPA_KNOB_BWD_DKDV_FORM), form = knob > 3 ? knob - 2 : knob;  // (4, 5: the twins of 2, 3)
   if (D < 64 || ADDR == ADDR_BIG) return false;
   if (form > 1) return form == 2;
   if (D == 64) {
@@ -1790,7 +1790,7 @@ hipError_t launch_both(const BwdParams& p, hipStream_t stream) {
   if (e != hipSuccess) return e;
   const bool narrow = keys_64<D, ADDR>(p);
   if constexpr (D == 128 && ADDR == ADDR_PLAIN)
-    if (spa_knob(SPA_KNOB_BWD_DKDV_FORM) == 1)
+    if (const int form = spa_knob(SPA_KNOB_BWD_DKDV_FORM); form == 1 || form > 3)
       return narrow ? launch<flash_bwd_dkdv_kernel<T, D, false, ADDR, 2>>(DkvCfg<D>::SMEM, false, 64, p, stream)
                     : launch<flash_bwd_dkdv_kernel<T, D, false>>(DkvCfg<D>::SMEM, false, 128, p, stream);
   if constexpr (D >= 64 && ADDR != ADDR_BIG)

@@ -1,5 +1,5 @@
-"""Backward forms whose waves share the rows (dq) or keys (dk/dv) of a workgroup and add their sums through LDS: sizes around a
-half-tile, a tile and a workgroup, odd and even numbers of tiles, against float64 autograd on the host."""
+"""The forms of the backward's workgroups, among them those whose waves share rows (dq) or keys (dk/dv) and add their sums through LDS: sizes
+around a half-tile, a tile and a workgroup, odd and even numbers of tiles, against float64 autograd on the host."""
 import pytest
 import torch
 
@@ -14,12 +14,12 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("D,dq,dkdv", [(128, 20, 2), (128, 24, 2), (64, 20, 2)])
+@pytest.mark.parametrize("D,dq,dkdv", [(128, 20, 2), (128, 24, 2), (64, 20, 2), (128, 4, 3), (128, 8, 3), (64, 4, 3)])
 def test_forms_with_shared_rows(D, dq, dkdv, dtype):
     try:
         _lib.tune("bwd_dq_waves", dq)
         _lib.tune("bwd_dkdv_form", dkdv)
-        for S in (2, 31, 33, 64, 65, 96, 127, 129, 192, 257, 320):
+        for S in (2, 31, 33, 64, 65, 96, 127, 129, 192, 257, 320, 449, 575):
             for causal in (True, False):
                 q, k, v, dout = rand_qkv((1, S, 2, D), 700 + S, dtype, n=4)
                 want = O.attn_backward_autograd(q, k, v, dout, None, causal)
@@ -28,7 +28,7 @@ def test_forms_with_shared_rows(D, dq, dkdv, dtype):
                 for x, w, name in zip(xs, want, "qkv"):
                     check_grad(x.grad, w, dtype, f"d{name}, {S} rows, causal {causal}")
         # fp32 accumulators that are added to, more keys than queries and the reverse
-        for Sq, Sk in ((65, 200), (200, 65), (64, 640)):
+        for Sq, Sk in ((65, 200), (200, 65), (64, 640), (575, 300), (300, 575)):
             q, _, _, dout = rand_qkv((1, Sq, 2, D), 720, dtype, n=4)
             k, v, _, _ = rand_qkv((1, Sk, 2, D), 721, dtype, n=4)
             for causal in (True, False):

@@ -17,6 +17,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 N_CASES = 3000
 SEED = 20240611
+_backward_forms = random.Random(SEED + 1)  # (a generator of their own: the cases stay those of SEED)
 
 OUT_TOL = {torch.float32: (1e-5, 1e-3), torch.bfloat16: (2e-2, 1.6e-2), torch.float16: (2e-3, 2e-3)}
 LSE_ATOL = 1e-3
@@ -55,6 +56,8 @@ def _case(rng):
     _lib.tune("fwd_share", share)
     _lib.tune("fwd_groups", groups)
     _lib.tune("fwd32_split", rng.choice([0, 0, 1, 2]))
+    _lib.tune("bwd_dq_waves", _backward_forms.choice([0, 0, 4, 8, 20, 24]))
+    _lib.tune("bwd_dkdv_form", _backward_forms.choice([0, 0, 1, 2, 3, 4, 5]))
     _lib.tune("few_rows", rng.choice([0, 0, 1]))   # up to three unmasked query rows: the streaming kernel, or the MFMA kernels
     g = torch.Generator().manual_seed(rng.randrange(1 << 30))
     mk = lambda *shape, dt=None: torch.randn(shape, generator=g).to(dt or dtype)
@@ -221,4 +224,6 @@ def test_fixed_seed_sweep_of_random_shapes_against_the_oracle():
         _lib.tune("fwd_share", 0)
         _lib.tune("fwd_groups", 0)
         _lib.tune("fwd32_split", 0)
+        _lib.tune("bwd_dq_waves", 0)
+        _lib.tune("bwd_dkdv_form", 0)
         _lib.tune("few_rows", 0)

@@ -521,12 +521,12 @@ def test_dkdv_kernel_hand_issued_and_compiler_scheduled_forms_agree(B, S, H, D, 
     """The D = 128 dk/dv kernel issues its MFMAs from inline assembly with the MFMA -> VALU hazard
     distances kept by the order of the loop; its twin leaves every MFMA (and every hazard) to the
     compiler.  Same operations in the same order on the same values: the gradients must be
-    bit-identical, and right."""
+    bit-identical, and right, whether a workgroup has 64 keys (forms 2 and 4) or 128 (3 and 5)."""
     q, k, v, dout = rand_qkv((B, S, H, D), 141, dtype, n=4)
     want = O.attn_backward_autograd(q, k, v, dout, None, causal)
     got = {}
     try:
-        for form in (0, 1):
+        for form in (0, 1, 2, 3, 4, 5):
             _lib.tune("bwd_dkdv_form", form)
             xs = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
             spa.ring_flash_attn_func(*xs, causal=causal).backward(dout.to(DEV))
@@ -535,8 +535,27 @@ def test_dkdv_kernel_hand_issued_and_compiler_scheduled_forms_agree(B, S, H, D, 
                 check_grad(g, w, dtype, f"d{name}, form {form}")
     finally:
         _lib.tune("bwd_dkdv_form", 0)
-    for a, b in zip(got[0], got[1]):
-        assert torch.equal(a, b)
+    for hand, twin in ((0, 1), (2, 4), (3, 5)):
+        for a, b in zip(got[hand], got[twin]):
+            assert torch.equal(a, b), (hand, twin)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,S,H,causal", [(1, 300, 2, True), (2, 515, 2, False), (1, 1000, 2, True), (1, 77, 1, True), (1, 64, 1, False)])
+def test_dq_kernel_hand_issued_and_compiler_scheduled_shared_forms_agree(B, S, H, causal, dtype):
+    """Of the dq kernel whose waves share rows, the 4-wave form (64 rows a workgroup) issues its MFMAs from inline assembly at D = 128 and the
+    8-wave form (128 rows) leaves them to the compiler; a row's sums are the same."""
+    q, k, v, dout = rand_qkv((B, S, H, 128), 142, dtype, n=4)
+    got = {}
+    try:
+        for form in (20, 24):
+            _lib.tune("bwd_dq_waves", form)
+            x = q.to(DEV).requires_grad_(True)
+            got[form], = torch.autograd.grad(spa.ring_flash_attn_func(x, k.to(DEV), v.to(DEV), causal=causal), (x,), dout.to(DEV))
+    finally:
+        _lib.tune("bwd_dq_waves", 0)
+    check_grad(got[20], O.attn_backward_autograd(q, k, v, dout, None, causal)[0], dtype, "dq")
+    assert torch.equal(got[20], got[24])
 
 
 def test_backward_packed_and_operator_entry():

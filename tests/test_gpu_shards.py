@@ -13,7 +13,8 @@ from test_gpu_parity import DEV, check_grad, check_out
 
 pytestmark = pytest.mark.gpu
 TOL = {torch.bfloat16: 2e-2, torch.float16: 4e-3, torch.float32: 1e-5}
-FORMS = [dict(fwd_groups=1, bwd_dq_waves=4), dict(fwd_groups=2, fwd_share=1, bwd_dq_waves=4), dict(fwd_groups=2, fwd_share=2, bwd_dq_waves=8)]
+FORMS = [dict(fwd_groups=1, bwd_dq_waves=4, bwd_dkdv_form=3), dict(fwd_groups=2, fwd_share=1, bwd_dq_waves=20, bwd_dkdv_form=2),
+         dict(fwd_groups=2, fwd_share=2, bwd_dq_waves=8, bwd_dkdv_form=3), dict(bwd_dq_waves=24, bwd_dkdv_form=3)]
 
 
 def close(got, want, tol):
@@ -69,8 +70,18 @@ def test_segments_around_the_tile_size(P, seg, dtype, D):
 
 
 @pytest.mark.parametrize("zigzag", [False, True])
-@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.float32, 64)])
-def test_packed_batches_of_shards(dtype, D, zigzag):
+@pytest.mark.parametrize("dtype,D,form", [(torch.bfloat16, 64, {}), (torch.float32, 64, {})] + [(torch.bfloat16, 128, form) for form in FORMS])
+def test_packed_batches_of_shards(dtype, D, form, zigzag):
+    try:
+        for knob, value in form.items():
+            _lib.tune(knob, value)
+        packed_batch_of_shards(dtype, D, zigzag)
+    finally:
+        for knob in form:
+            _lib.tune(knob, 0)
+
+
+def packed_batch_of_shards(dtype, D, zigzag):
     P, local, H = 3, [2, 0, 64, 130, 36], 2
     T = sum(local)
     cu = torch.tensor([0] + torch.tensor(local).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
