@@ -5,11 +5,12 @@
 // (sp_aurora/intel_ring_flash_attn.py:192-258), which re-runs autograd on each block.
 //
 // Two kernels, no atomics, every output row has one owner (deterministic):
-//   dq kernel   : workgroup = 128 or 256 query rows (4 or 8 waves x 32), walks key tiles of 64.
+//   dq kernel   : workgroup = 64, 128 or 256 query rows, walks key tiles of 64: 4 or 8 waves of 32 rows, or half as many rows and
+//                 pairs of waves that share 32 rows and each take half of a tile's keys (dq_form, KG).
 //                 S^T = K Q^T and dP^T = V dO^T land with a lane owning one query row,
 //                 so lse/delta are per-lane scalars and dS^T is, register for register,
 //                 the B operand of dQ^T = K^T dS^T.
-//   dkdv kernel : workgroup = 128 keys (4 waves x 32), walks query tiles of 64.
+//   dkdv kernel : workgroup = 128 keys (4 waves x 32), walks query tiles of 64; or 64 keys, pairs of waves sharing 32 (keys_64, QG).
 //                 S = Q K^T and dP = dO V^T land with a lane owning one key, so P and dS
 //                 are the B operands of dV^T = dO^T P and dK^T = Q^T dS.
 //
@@ -243,13 +244,24 @@ __device__ __forceinline__ void wait_loads_but() {  // until at most N of this w
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
+// The barrier without the waits of __syncthreads(), which would drain the operands in flight: the caller has waited for what it needs.  The compiler
+// knows no memory access of s_barrier; the empty assembly keeps loads and stores on their side of it, and a sched_barrier(0) follows in the loops.
+__device__ __forceinline__ void barrier_alone() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // MFMAs with the accumulator's register file spelled out.  The compiler gives every MFMA of a
 // function the same form; the one-wave-per-SIMD kernels want both: the gradient accumulators
 // (touched by MFMAs only) in AGPRs, the S / dP tiles, which the VALU works on, in VGPRs, so that
 // no v_accvgpr_read / v_accvgpr_write copies are needed between the matrix pipe and the VALU.
-// The compiler does not see these as MFMAs: the code keeps the distances the hardware needs
-// (a VALU read of a tile comes at least 5 MFMAs after the tile's last MFMA; srcC is the
-// destination itself or the literal 0, never a register a VALU instruction has just written).
+// The compiler does not see these as MFMAs: the code keeps the distances the hardware needs (srcC is the
+// destination itself or the literal 0, never a register a VALU instruction has just written).  A VALU read of a tile needs 11 wait states after
+// the tile's last MFMA, which takes the matrix pipe for 8 passes: with MFMA_APART others issued in between, each of which had to wait for the one
+// before it, at least 16 have gone by.  The loops' orders are held to that by static_asserts: 8 gradient MFMAs in the dq kernel, 3 MFMAs in the
+// dk/dv kernel.  Where no others follow, mfma_settle() waits.
+constexpr int MFMA_APART = 2;
 template <typename T>
 struct MmaAsm;
 template <>
@@ -371,9 +383,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   typedef DqCfg<D, NW, KG> G;
   typedef Mma16<T> M;
   typedef MmaAsm<T> MA;
-  // one wave per SIMD: AGPRs are there for the dq accumulators.  D = 128 only: its 8 gradient
-  // MFMAs (with their operand reads) between a tile's last MFMA and the first VALU read of the
-  // tile give the matrix pipe the time it needs; the shorter lists of smaller D would not.
+  // one wave per SIMD: AGPRs are there for the dq accumulators (D = 128; two workgroups to a CU at smaller D)
   constexpr bool MIXED = NW == 4 && D == 128;
   typedef typename M::frag frag;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -459,6 +469,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
   constexpr int LOOK_CAP = NW == 8 || D <= 64 ? 4 : BWD_LOOK_MAX;  // two waves per SIMD: 256 registers each, and the other wave covers LDS latency
   constexpr int BWD_LOOK = NA < LOOK_CAP ? NA : LOOK_CAP;
   static_assert(NBODY % BWD_LOOK == 0 && BWD_LOOK <= NA, "the operand window must tile the loop body");
+  static_assert(!MIXED || NB >= MFMA_APART, "the gradient MFMAs stand between a tile's last MFMA and its element-wise work");
 
   // The workgroup's rows of q and dout pass through the stages on their way into registers, and those of out, which give
   // delta = rowsum(dout * out) (written for the dk / dv kernel).  128 rows are one stage a tensor: all of them and the first tile are
@@ -628,7 +639,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D <= 64 ? 2 : 1) flash_bwd
     // tile i+1 must have landed before this body reads it (KG = 2: i+2); tile i-1 is free for tile i+AHEAD.  (The operands in flight, one read
     // each, are of tile i+1 or later.)
     __builtin_amdgcn_s_waitcnt(0x0070 | (G::NL & 15) | ((G::NL >> 4) << 14) | (BWD_LOOK << 8));
-    __builtin_amdgcn_s_barrier();
+    barrier_alone();
   };
   auto list_of = [&](int i, int list, f32x16& sc, f32x16& dc, f32x16& sn, f32x16& dn) {
     const int key0 = (2 * i + (KG == 2 ? kg : list)) * 32;  // first key of the half-tile whose dS is formed in this list
@@ -783,7 +794,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
   typedef DkvCfg<D> G;
   typedef Mma16<T> M;
   typedef MmaAsm<T> MA;
-  constexpr bool MIXED = D == 128 && ASM;  // see the dq kernel; here 5 gradient MFMAs separate a tile's MFMAs from its VALU reads
+  constexpr bool MIXED = D == 128 && ASM;  // see the dq kernel, and MmaAsm
   typedef typename M::frag frag;
   extern __shared__ __align__(16) unsigned char smem[];
 
@@ -936,7 +947,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     // its share of the loads, and the barriers of the passes (of which there is an even number with QG = 2)
     for (int i = it0, end = QG == 1 ? nt : it0 + (nt - it0 + 1 & ~1); i < end; ++i) {
       wait_loads_but<QG == 2 ? 0 : G::NL>();
-      __builtin_amdgcn_s_barrier();
+      barrier_alone();
       issue_tile(i + 3);
     }
     wait_loads_but<0>();
@@ -1040,13 +1051,17 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
     };
 
     // Matrix instruction n of a group: 0 .. KS - 1: S, contraction step; KS .. : dP; 2 KS ..: gradient product number.  The gradient
-    // products, whose operands take twice as many LDS reads, are every other one; the last of S and dP is two or more matrix
-    // instructions before the first vector instruction that reads it (S nine).
+    // products, whose operands take twice as many LDS reads, are every other one.
     constexpr int KS = D / 16;
     auto instruction = [](bool first, int n) -> int {
       const int k = n >> 1;
       return (n & 1) ? 2 * KS + k : (first ? 0 : HS) + (k < HS ? k : KS + k - HS);
     };
+    // The first vector instruction that reads S is the mask in front of the next group, the first that reads dP part 1 of element(), behind the
+    // second matrix instruction of that group: nine of them come after the last of S and three after the last of dP.
+    constexpr int LAST_S = 2 * HS - 2, LAST_DP = 4 * HS - 2;
+    static_assert(instruction(false, LAST_S) == KS - 1 && instruction(false, LAST_DP) == 2 * KS - 1, "the last of S and of dP");
+    static_assert(!MIXED || (GROUP == 16 && GROUP - 1 - LAST_S >= MFMA_APART && GROUP - 1 - LAST_DP + 2 >= MFMA_APART), "distance to the element-wise work");
     // operand number J of the pass on tile i (J >= NBODY: the first operands of the next pass)
     auto fetch = [&](int J) -> frag {
       const int group = J % NBODY / GROUP;
@@ -1116,7 +1131,7 @@ __global__ void __launch_bounds__(BWD_THREADS, D <= 64 ? 2 : 1) flash_bwd_dkdv_k
       // later tiles, so nothing else is waited for.
       wait_loads_but<QG == 2 ? 0 : G::NL>();
       if (MIXED)
-        __builtin_amdgcn_s_barrier();
+        barrier_alone();
       else
         __syncthreads();
       last_step = step;
