@@ -56,8 +56,9 @@ def _case(rng):
     _lib.tune("fwd_share", share)
     _lib.tune("fwd_groups", groups)
     _lib.tune("fwd32_split", rng.choice([0, 0, 1, 2]))
-    _lib.tune("bwd_dq_waves", _backward_forms.choice([0, 0, 4, 8, 20, 24]))
-    _lib.tune("bwd_dkdv_form", _backward_forms.choice([0, 0, 1, 2, 3, 4, 5]))
+    dq_form, dkdv_form = _backward_forms.choice([0, 0, 4, 8, 20, 24]), _backward_forms.choice([0, 0, 1, 2, 3, 4, 5])
+    _lib.tune("bwd_dq_waves", dq_form)
+    _lib.tune("bwd_dkdv_form", dkdv_form)
     _lib.tune("few_rows", rng.choice([0, 0, 1]))   # up to three unmasked query rows: the streaming kernel, or the MFMA kernels
     g = torch.Generator().manual_seed(rng.randrange(1 << 30))
     mk = lambda *shape, dt=None: torch.randn(shape, generator=g).to(dt or dtype)
@@ -121,7 +122,7 @@ def _case(rng):
     elif kind == "ring_bwd":
         S = rng.choice([2, 33, 64, 100, 128, 200, 257, 384])
         P = rng.choice([1, 1, 2, 4]) if S % 4 == 0 else 1
-        info = (kind, dtype, B, H, S, D, causal, P)
+        info = (kind, dtype, B, H, S, D, causal, P, dq_form, dkdv_form)
         q, k, v, do = (mk(B, S, H, D) for _ in range(4))
         want = O.attn_backward_autograd(q, k, v, do, None, causal)
         xs = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
@@ -130,7 +131,7 @@ def _case(rng):
     elif kind == "block_bwd":
         Sq = rng.choice([2, 33, 64, 100, 128, 130, 257, 300])
         Sk = rng.choice([2, 40, 64, 128, 129, 200, 260, 384, 520])
-        info = (kind, dtype, B, H, Sq, Sk, D, causal)
+        info = (kind, dtype, B, H, Sq, Sk, D, causal, dq_form, dkdv_form)
         q, do, k, v = mk(B, Sq, H, D), mk(B, Sq, H, D), mk(B, Sk, H, D), mk(B, Sk, H, D)
         want = O.attn_backward_autograd(q, k, v, do, None, causal)
         qd, kd, vd, dd = (t.to(DEV) for t in (q, k, v, do))
@@ -145,7 +146,7 @@ def _case(rng):
         lk = [rng.choice([0, 2, 40, 64, 130, 260]) for _ in range(ns)]
         if sum(lq) == 0 or sum(lk) == 0:
             return
-        info = (kind, dtype, lq, lk, H, D, causal)
+        info = (kind, dtype, lq, lk, H, D, causal, dq_form, dkdv_form)
         q, do, k, v = mk(sum(lq), H, D), mk(sum(lq), H, D), mk(sum(lk), H, D), mk(sum(lk), H, D)
         xs = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
         spa.sp_aurora_varlen_func(*xs, _cu(lq).to(DEV), _cu(lk).to(DEV), causal=causal).backward(do.to(DEV))
