@@ -14,9 +14,9 @@ LIB_PATH = os.path.join(HERE, LIB_NAME)
 NATIVE_PATH = os.path.join(HERE, "_native.so")
 # (source, object, extra flags).  flash_fwd.hip makes five objects: the zigzag variants of the 16-bit forward kernel
 # and the variants for tensors of 2 GiB and more per (batch, head) are translation units of their own, so that the
-# parts of the longest compile run side by side; flash_bwd.hip likewise makes two.
+# parts of the longest compile run side by side; flash_bwd.hip and flash_fwd32.hip likewise make two.
 # The forward kernels' softmax phase gains 1-3 % from the scheduler that maximises instruction-level
-# parallelism; the backward kernels lose 2 % with it.
+# parallelism; the backward kernels lose 2 % with it, and the fp32 forward for few rows at D = 128, whose two waves a SIMD fill all registers, 5 %.
 _FWD = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
 UNITS = [
     ("flash_fwd.hip", "flash_fwd.o", _FWD),
@@ -25,6 +25,7 @@ UNITS = [
     ("flash_fwd.hip", "flash_fwd_splitkv.o", _FWD + ["-DSPA_FWD_SPLITKV_UNIT"]),
     ("flash_fwd.hip", "flash_fwd_map.o", _FWD + ["-DSPA_FWD_MAP_UNIT"]),
     ("flash_fwd32.hip", "flash_fwd32.o", _FWD),
+    ("flash_fwd32.hip", "flash_fwd32_wide.o", ["-DSPA_FWD32_WIDE_UNIT"]),
     ("flash_bwd.hip", "flash_bwd.o", []),
     ("flash_bwd.hip", "flash_bwd_other.o", ["-DSPA_BWD_OTHER_UNIT"]),
     ("spa_abi.hip", "spa_abi.o", []),

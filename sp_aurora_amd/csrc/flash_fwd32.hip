@@ -14,6 +14,7 @@
 // and 30 D / 16 of splitting K and V, once per workgroup and tile.
 #include "spa_common.h"
 #include "spa_host.h"
+#include <math.h>
 
 namespace {
 
@@ -70,31 +71,36 @@ __device__ __forceinline__ void zero16(f32x16& x) {
   for (int v = 0; v < 16; ++v) x[v] = 0.f;
 }
 
-// What a wave keeps of its 32 query rows, and one tile's softmax.
-template <int D>
+// What a wave keeps of its 32 query rows (DV: head dims of its results), and one tile's softmax.
+template <int D, int DV = D>
 struct Rows {
   Split8 q[D / 16];
-  f32x16 o[D / 32];
+  f32x16 o[DV / 32];
   float m_run, l_run, c, down;
   // A score above 2^80 is an infinity in the accumulator, and its row a NaN; one below -2^80 has no weight beside a largest score above
   // -2^70, and rows without one are computed again (lost()).  With a scale that leaves such scores apart the bits that q
   // needs lie higher: below 2^-93 they cannot move an exponent by 2^-50.
   __device__ __forceinline__ void init(const float* row, int hh, bool negate, float scale_log2) {
-    const bool tiny = scale_log2 < 0x1p-64f;
-    down = tiny ? 0x1p16f : F32_DOWN;
+    start(scale_log2);
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) {
-      float x[8];
-      const f32x4 a = *(const f32x4*)(row + ks * 16 + hh * 8), b = *(const f32x4*)(row + ks * 16 + hh * 8 + 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        x[e] = negate ? -a[e] : a[e];  // negative softmax scale: -q with |scale|
-        x[4 + e] = negate ? -b[e] : b[e];
-      }
-      q[ks].set(x, tiny ? 0x1p-40f : F32_UP);
+      const f32x4* const at = (const f32x4*)(row + ks * 16 + hh * 8);
+      split_queries(at[0], at[1], negate, q[ks]);
     }
+  }
+  __device__ __forceinline__ void split_queries(f32x4 a, f32x4 b, bool negate, Split8& to) const {
+    float x[8];
 #pragma unroll
-    for (int i = 0; i < D / 32; ++i) zero16(o[i]);
+    for (int e = 0; e < 4; ++e) {
+      x[e] = negate ? -a[e] : a[e];  // negative softmax scale: -q with |scale|
+      x[4 + e] = negate ? -b[e] : b[e];
+    }
+    to.set(x, c < 0x1p-64f ? 0x1p-40f : F32_UP);
+  }
+  __device__ __forceinline__ void start(float scale_log2) {
+    down = scale_log2 < 0x1p-64f ? 0x1p16f : F32_DOWN;
+#pragma unroll
+    for (int i = 0; i < DV / 32; ++i) zero16(o[i]);
     m_run = -INFINITY;
     l_run = 0.f;
     c = scale_log2;
@@ -113,7 +119,7 @@ struct Rows {
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
-      for (int i = 0; i < D / 32; ++i)
+      for (int i = 0; i < DV / 32; ++i)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[i][v] *= alpha;
     }
@@ -153,9 +159,11 @@ __device__ __forceinline__ void mask_tile(f32x16& s, int key0, int first_row, in
 // Bound: that instruction's rate (64 operations a clock and SIMD) and the latency of the loads, which go straight into operands, a tile of V and the next
 // of K ahead.  Every row of causal [1, 4096, 32, 128] again, for an infinity in V: 847 -> 2241 us the call, [1, 1024, 16, 64] 33 -> 90 (row by
 // row with plain operations [1, 1024, 32, 128] took 8500, now 333); a NaN in K ends the pass where it lies (867 and 89).
-template <int D>
+// VA: keys of V asked for at a time (16: a tile's, and the next tile's of K, ahead of their use; 4, and of K in parts: where two waves share a SIMD
+// and the registers do not hold them).
+template <int D, int DV = D, int VA = 16>
 struct PlainRows {
-  f32x16 o[D / 32];
+  f32x16 o[DV / 32];
   float m, l;  // of row ln, over this lane's keys
   template <typename RowOf>
   __device__ __forceinline__ void run(const FwdParams& p, unsigned bad, int q0, const float* qp, const float* kp, const float* vp, float c, int lane,
@@ -170,37 +178,44 @@ struct PlainRows {
 #pragma unroll
     for (int i = 0; i < D / 8; ++i) q[i] = p.negq ? -qr[i] : qr[i];
 #pragma unroll
-    for (int i = 0; i < D / 32; ++i) zero16(o[i]);
+    for (int i = 0; i < DV / 32; ++i) zero16(o[i]);
     m = -INFINITY;
     l = 0.f;
-    f32x4 k[D / 8];
-    const auto load_keys = [&](int it) {
+    constexpr int KA = VA == 16 ? D / 8 : 4;
+    f32x4 k[KA];
+    const auto load_keys = [&](int it, int i0) {
       const f32x4* const kr = half_row(kp, p.ks.s, it * F32_BN + ln < p.Sk ? it * F32_BN + ln : last);
 #pragma unroll
-      for (int i = 0; i < D / 8; ++i) k[i] = kr[i];
+      for (int i = 0; i < KA; ++i) k[i] = kr[i0 + i];
     };
-    load_keys(it0);
+    if (VA == 16) load_keys(it0, 0);
 #pragma unroll 1
     for (int it = it0; it < nt; it += step) {
       const int key0 = it * F32_BN;
       f32x16 s;
       zero16(s);
       const bool whole = !(p.causal && key0 + F32_BN - 1 > q0) && key0 + F32_BN <= p.Sk;  // every row sees every key
-      float vx[16][D / 32];
-      if (whole) {
+      float vx[VA][DV / 32];
+      const auto load_values = [&](int v0) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const float* const vr = vp + (int64_t)row_of(key0 + 8 * (v >> 2) + 4 * hh + (v & 3)) * p.vs.s + ln;
+        for (int v = 0; v < VA; ++v) {
+          const float* const vr = vp + (int64_t)row_of(key0 + 8 * ((v0 + v) >> 2) + 4 * hh + ((v0 + v) & 3)) * p.vs.s + ln;
 #pragma unroll
-          for (int i = 0; i < D / 32; ++i) vx[v][i] = vr[32 * i];
+          for (int i = 0; i < DV / 32; ++i) vx[v][i] = vr[32 * i];
         }
-      }
+      };
+      if (whole && VA == 16) load_values(0);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < D / 8; ++i)
+      for (int i = 0; i < D / 8; ++i) {
+        if (VA < 16 && i % KA == 0) {
+          __builtin_amdgcn_sched_barrier(0);
+          load_keys(it, i);
+        }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i][e], q[i][e], s, 0, 0, 0);
-      if (it + step < nt) load_keys(it + step);
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i % KA][e], q[i][e], s, 0, 0, 0);
+      }
+      if (VA == 16 && it + step < nt) load_keys(it + step, 0);
       mask_tile(s, key0, q0, qrow, p.causal, p.Sk, hh);
       float mx = s[0];
 #pragma unroll
@@ -215,7 +230,7 @@ struct PlainRows {
         l += s[v];
       }
 #pragma unroll
-      for (int i = 0; i < D / 32; ++i)
+      for (int i = 0; i < DV / 32; ++i)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[i][v] *= alpha;
       if (!whole) {
@@ -230,7 +245,7 @@ struct PlainRows {
           x = __shfl(x, ln + 32 * ((j >> 2) & 1));
           const float* const vr = vp + (int64_t)row_of(key0 + j) * p.vs.s + 4 * hh;
 #pragma unroll
-          for (int i = 0; i < D / 8; ++i) {
+          for (int i = 0; i < DV / 8; ++i) {
             const f32x4 y = *(const f32x4*)(vr + 8 * i);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -241,9 +256,14 @@ struct PlainRows {
         }
       } else {
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
+        for (int v0 = 0; v0 < 16; v0 += VA) {
+          if (VA < 16) load_values(v0);
 #pragma unroll
-          for (int i = 0; i < D / 32; ++i) o[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(vx[v][i], s[v], o[i], 0, 0, 0);
+          for (int v = 0; v < VA; ++v)
+#pragma unroll
+            for (int i = 0; i < DV / 32; ++i) o[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(vx[v][i], s[v0 + v], o[i], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
       const uint64_t nan = __builtin_amdgcn_ballot_w64(l != l);
       if ((bad & ~(unsigned)(nan | nan >> 32)) == 0) break;
@@ -552,18 +572,31 @@ __global__ void __launch_bounds__(F32_THREADS, D == 128 ? 1 : D == 64 ? 2 : 3) f
 }
 
 // Few rows: a launch of the kernel above with fewer workgroups than CUs lasts as long as one wave's chain over all key tiles.
-// Here a workgroup owns 32 query rows and its NW waves take every NW-th key tile, straight from memory into operands (a lane
-// reads its own key's row of K, and a column of V 32 lanes wide per key) with no LDS and no barrier in the loop; the waves'
-// (O, m, l) are combined through LDS at the end.  Causal [1, 512, 32, 128] 82 -> 37 us, [1, 1697, 8, 64] 45 -> 39.
-template <int D, int NW>
+// Here a workgroup owns 32 query rows and its NW waves take every NW-th key tile, without a barrier in the loop: a tile of K goes
+// straight to LDS that is the wave's own (whole rows at a time; read by the lanes that need them, 16 bytes of 32 rows are 32 cache lines
+// an instruction), V straight into operands (a column of V 32 lanes wide per key).  The rows' own three terms are formed once and lie in LDS.
+// The waves' (O, m, l) are combined through LDS at the end.  Where that leaves CUs without a workgroup, D / DV of them take the same rows and keys, each
+// for its DV head dims of the result: the scores are formed again, the splitting of V, its products and the combination are shared out.
+// Bound: the vector instructions that split K and V (D = 128: 830 of 1000 a tile and wave, 4000 clocks beside 3072 of the matrix pipe), with two
+// waves a SIMD to run beside each other.  Before, K came as operands row by row, a branch for rows in shards stood around every load, D = 128 had one wave a SIMD,
+// and half of the CUs were idle under small grids: [1, 8, 512, 64] 14.6 -> 10.9 us, [1, 8, 512, 128] 28.5 -> 17.5 (with whole rows 21), [1, 8, 256, 128]
+// 17.1 -> 9.8, [1, 12, 2048, 128] causal 177 -> 115.
+template <int D, int DV, int NW>
 struct Fwd32SplitCfg {
-  static constexpr int REC = 64 * (D / 8) * 4;               // floats of one wave's O
-  static constexpr int SMEM = (NW * (REC + 128) + NW) * 4;
+  static constexpr int REC = 64 * (DV / 8) * 4;              // floats of one wave's O
+  static constexpr int QPLANE = 32 * D * 2;                  // one term of the rows
+  static constexpr int KTILE = F32_BN * D * 4;
+  static constexpr int CPR = D / 4;                          // 16-byte chunks of a row of K
+  static constexpr int LOOP = 3 * QPLANE + NW * KTILE, COMBINE = (NW * (REC + 128) + NW) * 4;
+  static constexpr int SMEM = LOOP > COMBINE ? LOOP : COMBINE;
+  // chunk permutation of a row: 16 rows at one chunk lie in 16 different 16-byte bank groups
+  static __device__ __forceinline__ int swizzle(int row) { return D == 32 ? row >> 1 & 7 : row & 15; }
 };
 
-template <int D, int NW>
+template <int D, int DV, int NW, bool MAP>
 __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const FwdParams p) {
-  typedef Fwd32SplitCfg<D, NW> C;
+  typedef Fwd32SplitCfg<D, DV, NW> C;
+  constexpr int PARTS = D / DV;
   extern __shared__ __align__(16) unsigned char smem[];
   float* const sm = (float*)smem;
   const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
@@ -571,44 +604,71 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
   const int pair = blockIdx.x + blockIdx.z * gridDim.x;
   if (pair >= p.B * p.H) return;
   const int h = pair % p.H, b = pair / p.H;
-  const int q0 = (p.nqt - 1 - (int)blockIdx.y) * 32;
+  const int q0 = (p.nqt - 1 - (int)blockIdx.y / PARTS) * 32, d0 = (int)blockIdx.y % PARTS * DV;
   RowMap map = {};
-  if (p.map.P) map.init(p.map, p.Sq / p.map.P);
-  auto row_of = [&](int r) { return p.map.P ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
-  auto stat_of = [&](int r) { return p.map.P ? map.at(r, p.map.lse_pitch) : r; };   // in lse
+  if (MAP) map.init(p.map, p.Sq / p.map.P);
+  auto row_of = [&](int r) { return MAP ? map.at(r, p.map.pitch) : r; };        // where row r of the sequence lies
+  auto stat_of = [&](int r) { return MAP ? map.at(r, p.map.lse_pitch) : r; };   // in lse
   const float* qp = (const float*)p.q + b * p.qs.b + h * p.qs.h;
   const float* kp = (const float*)p.k + b * p.ks.b + h * p.ks.h;
-  const float* vp = (const float*)p.v + b * p.vs.b + h * p.vs.h;
-  const int qrow = q0 + ln, qrow_c = qrow < p.Sq ? qrow : p.Sq - 1;
+  const float* vp = (const float*)p.v + b * p.vs.b + h * p.vs.h + d0;
+  const int qrow = q0 + ln;
   const int kv_end = p.causal ? (q0 + 32 < p.Sk ? q0 + 32 : p.Sk) : p.Sk;
   const int nt = (kv_end + F32_BN - 1) / F32_BN;
 
-  f32x4 kx[D / 16][2];
-  float vx[2][D / 32][8];
-  auto gload = [&](int it) {
-    int r = it * F32_BN + ln;
-    const float* a = kp + (int64_t)row_of(r < p.Sk ? r : p.Sk - 1) * p.ks.s + hh * 8;
+  const unsigned lds0 = (unsigned)(uintptr_t)(lds_u8*)smem, ktile = lds0 + 3 * C::QPLANE + w * C::KTILE;
+  auto load_keys = [&](int it) {  // (rows past the end: the last one, masked below)
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-      kx[ks][0] = *(const f32x4*)(a + ks * 16);
-      kx[ks][1] = *(const f32x4*)(a + ks * 16 + 4);
+    for (int j = 0; j < C::KTILE / 1024; ++j) {
+      const int slot = j * 64 + lane, row = slot / C::CPR, r = it * F32_BN + row;
+      const float* a = kp + (int64_t)row_of(r < p.Sk ? r : p.Sk - 1) * p.ks.s + ((slot % C::CPR) ^ C::swizzle(row)) * 4;
+      load_to_lds_b128(a, ktile + j * 1024);
     }
+  };
+  float vx[2][DV / 32][8];
+  auto load_values = [&](int it) {
     // operand element e of half u: key 16 u + 8 (e / 4) + 4 hh + e % 4, as the rows of an accumulator lie
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        r = it * F32_BN + 16 * u + 8 * (e >> 2) + 4 * hh + (e & 3);
+        const int r = it * F32_BN + 16 * u + 8 * (e >> 2) + 4 * hh + (e & 3);
         const float* v = vp + (int64_t)row_of(r < p.Sk ? r : p.Sk - 1) * p.vs.s + ln;
 #pragma unroll
-        for (int db = 0; db < D / 32; ++db) vx[u][db][e] = v[db * 32];
+        for (int db = 0; db < DV / 32; ++db) vx[u][db][e] = v[db * 32];
       }
   };
-  if (w < nt) gload(w);
-  Rows<D> rows;
-  rows.init(qp + (int64_t)row_of(qrow_c) * p.qs.s, hh, p.negq, p.scale_log2);
+  constexpr int CH = DV > 32 ? 2 : 1, UH = DV > 64 ? 1 : 2;  // head-dim blocks and halves of a tile's keys at a time
+  Rows<D, DV> rows;
+  rows.start(p.scale_log2);
+  // (a whole chunk of eight values a thread, or none)
+  const int qr = tid / (D / 8), qc = tid % (D / 8);
+  static_assert(32 * D / 8 <= 64 * NW, "the rows' chunks are split in one go");
+  f32x4 qa, qb;
+  if (qr < 32) {
+    const int r = q0 + qr < p.Sq ? q0 + qr : p.Sq - 1;
+    const f32x4* const at = (const f32x4*)(qp + (int64_t)row_of(r) * p.qs.s + qc * 8);
+    qa = at[0];
+    qb = at[1];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (w < nt) {
+    load_keys(w);
+    load_values(w);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (qr < 32) {
+    Split8 x;
+    rows.split_queries(qa, qb, p.negq, x);
+    unsigned char* const to = smem + qr * (D * 2) + (qc ^ k_swizzle<D>(qr)) * 16;
+    *(u32x4*)to = x.h;
+    *(u32x4*)(to + C::QPLANE) = x.m;
+    *(u32x4*)(to + 2 * C::QPLANE) = x.l;
+  }
+  __syncthreads();
   for (int it = w; it < nt; it += NW) {
     const int key0 = it * F32_BN;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tile of K (and of V, which was asked for with it)
     f32x16 s, s1;
     zero16(s);
     zero16(s1);
@@ -616,44 +676,64 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
     for (int ks = 0; ks < D / 16; ++ks) {
       float x[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = kx[ks][e >> 2][e & 3];
-      Split8 a;
+      for (int j = 0; j < 2; ++j) {
+        const f32x4 y = __builtin_bit_cast(f32x4, lds_read_b128(ktile + ln * (D * 4) + ((4 * ks + 2 * hh + j) ^ C::swizzle(ln)) * 16));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[4 * j + e] = y[e];
+      }
+      Split8 a, q;
       a.set(x);
-      mma6(a, rows.q[ks], s, s1);
+      const unsigned at = lds0 + ln * (D * 2) + ((2 * ks + hh) ^ k_swizzle<D>(ln)) * 16;
+      q.h = lds_read_b128(at);
+      q.m = lds_read_b128(at + C::QPLANE);
+      q.l = lds_read_b128(at + 2 * C::QPLANE);
+      mma6(a, q, s, s1);
     }
-    Split8 va[2][D / 32];
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int db = 0; db < D / 32; ++db) va[u][db].set(vx[u][db]);
-    if (it + NW < nt) gload(it + NW);
+    if (it + NW < nt) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this tile of K has been read
+      load_keys(it + NW);
+    }
 #pragma unroll
     for (int v = 0; v < 16; ++v) s[v] = (s[v] + s1[v]) * rows.down;
     mask_tile(s, key0, q0, qrow, p.causal, p.Sk, hh);
     Split8 pf[2];
     rows.raise(s);
     rows.weights(s, pf);
+    // (the small terms of all of the tile's keys first, where the registers hold them: 5 to 8 % less rounding error)
 #pragma unroll
-    for (int term = 0; term < 6; ++term)
+    for (int u0 = 0; u0 < 2; u0 += UH)
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int db = 0; db < DV / 32; db += CH) {
+        Split8 va[UH][CH];
 #pragma unroll
-        for (int db = 0; db < D / 32; ++db) {
-          const frag a = as_frag<frag>(term == 2 || term == 3 ? va[u][db].m : term == 4 ? va[u][db].l : va[u][db].h);
-          const frag pb = as_frag<frag>(term == 0 ? pf[u].l : term == 1 || term == 2 ? pf[u].m : pf[u].h);
-          rows.o[db] = M::run(a, pb, rows.o[db]);
-        }
+        for (int u = 0; u < UH; ++u)
+#pragma unroll
+          for (int x = 0; x < CH; ++x) va[u][x].set(vx[u0 + u][db + x]);
+#pragma unroll
+        for (int term = 0; term < 6; ++term)
+#pragma unroll
+          for (int u = 0; u < UH; ++u)
+#pragma unroll
+            for (int x = 0; x < CH; ++x) {
+              const Split8 &vs = va[u][x], &ps = pf[u0 + u];
+              const frag a = as_frag<frag>(term == 2 || term == 3 ? vs.m : term == 4 ? vs.l : vs.h);
+              const frag pb = as_frag<frag>(term == 0 ? ps.l : term == 1 || term == 2 ? ps.m : ps.h);
+              rows.o[db + x] = M::run(a, pb, rows.o[db + x]);
+            }
+      }
+    if (it + NW < nt) load_values(it + NW);
   }
+  __syncthreads();  // (the same LDS again)
   // ---- combine: every wave leaves its unscaled O (lane-private order) and (m, l); wave j then finishes the
   // 16-byte pieces j, j + NW, ... of every row (of `which`) ----
-  constexpr int NPC = D / 8;  // 16-byte pieces per lane: (db, g)
-  float* const obase = (float*)p.out + b * p.os.b + h * p.os.h;
+  constexpr int NPC = DV / 8;  // 16-byte pieces per lane: (db, g)
+  float* const obase = (float*)p.out + b * p.os.b + h * p.os.h + d0;
   float* const lbase = p.lse + ((int64_t)b * p.H + h) * p.lse_bh;
   bool bad = false;
-  auto combine = [&](const f32x16 (&o)[D / 32], float m, float l, float down, unsigned which) {
+  auto combine = [&](const f32x16 (&o)[DV / 32], float m, float l, float down, unsigned which) {
     float* const orec = sm + w * (C::REC + 128);
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db)
+    for (int db = 0; db < DV / 32; ++db)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         f32x4 st;
@@ -697,7 +777,7 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
         }
         *(f32x4*)(op + (pc / 4) * 32 + 8 * (pc % 4) + 4 * hh) = acc;
       }
-      if (w == 0 && hh == 0) lbase[stat_of(qrow)] = (m_all * rows.c + fast_log2(l_all)) * 0.6931471805599453f;
+      if (w == 0 && hh == 0 && d0 == 0) lbase[stat_of(qrow)] = (m_all * rows.c + fast_log2(l_all)) * 0.6931471805599453f;
     }
   };
   combine(rows.o, rows.m_run, halves_sum(rows.l_run), F32_DOWN, ~0u);
@@ -709,41 +789,81 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
 #pragma unroll
   for (int j = 0; j < NW; ++j) which |= flags[j];
   if (__builtin_amdgcn_readfirstlane(which)) {
-    PlainRows<D> plain;
+    constexpr int VA = D == 128 && DV >= 64 ? 4 : 16;
+    PlainRows<D, DV, VA> plain;
     plain.run(p, which, q0, qp, kp, vp, rows.c, lane, w, NW, row_of);
     combine(plain.o, plain.m, halves_sum(plain.l), 1.f, which);
   }
 }
 
+// parts: workgroups that share the rows of a tile
 template <auto kernel>
-hipError_t launch(int threads, int smem, int rows, FwdParams p, hipStream_t stream) {
+hipError_t launch(int threads, int smem, int rows, int parts, FwdParams p, hipStream_t stream) {
   const hipError_t e = spa_allow_dynamic_lds<kernel>(smem);
   if (e != hipSuccess) return e;
   dim3 grid;
   if (p.cu_q) {
     if (!spa_varlen_grid(p.H, p.B, p.lse_bh, p.Sq, rows, 1, grid, p.numbered)) return hipErrorInvalidValue;
   } else {
-    if (p.nqt > 65535) return hipErrorInvalidValue;
-    grid = spa_head_groups((int64_t)p.B * p.H, p.nqt);
+    if (p.nqt * parts > 65535) return hipErrorInvalidValue;
+    grid = spa_head_groups((int64_t)p.B * p.H, p.nqt * parts);
   }
   hipLaunchKernelGGL(kernel, grid, dim3(threads), smem, stream, p);
   return hipGetLastError();
 }
 
-// Whether the waves of a workgroup share out the keys of 32 rows rather than taking 32 rows each.  A launch of the kernel for
-// many rows lasts as long as the longest chain of tiles, a launch of the other as long as its work on all SIMDs; microseconds per
-// tile and wave, and per tile and SIMD, fitted to 19 launches of 192 to 4096 rows: of these one is taken the wrong way, for 5 of 45 us.
+// (rows in shards are looked up row by row: a variant of its own, since the branch would stand around every load)
+template <int D, int DV>
+hipError_t launch_part(const FwdParams& p, hipStream_t stream) {
+  constexpr int NW = 8, smem = Fwd32SplitCfg<D, DV, NW>::SMEM, parts = D / DV;
+  return p.map.P ? launch<flash_fwd32_splitk_kernel<D, DV, NW, true>>(64 * NW, smem, 32, parts, p, stream)
+                 : launch<flash_fwd32_splitk_kernel<D, DV, NW, false>>(64 * NW, smem, 32, parts, p, stream);
+}
+template <int D>
+hipError_t launch_splitk(const FwdParams& p, hipStream_t stream) {
+  const int64_t tiles = (int64_t)p.B * p.H * p.nqt;
+  // as many as there are CUs for: 128 tiles of 512 keys at D = 64 in one, two parts 12.4, 10.9 us, D = 128 21.2, 17.4; 64 of 256 keys at D = 128 in
+  // one, two, four 12.8, 10.2, 9.5; with more workgroups than CUs a second round costs more: 200 tiles of 777 keys 31 and 37
+  int parts = 1;
+  while (parts * 2 * tiles <= spa_device_cus()) parts *= 2;
+  if constexpr (D == 128)
+    if (parts >= 4) return launch_part<D, D / 4>(p, stream);
+  if constexpr (D >= 64)
+    if (parts >= 2) return launch_part<D, D / 2>(p, stream);
+  return launch_part<D, D>(p, stream);
+}
+
+#ifdef SPA_FWD32_WIDE_UNIT
+}  // namespace
+hipError_t spa_launch_fwd32_shared_keys_128(const FwdParams& p, hipStream_t stream) { return launch_splitk<128>(p, stream); }
+#else
+// Whether the waves of a workgroup share out the keys of 32 rows rather than taking 32 rows each.  Microseconds of a launch, from 90 launches of
+// 128 to 4096 rows and 8 to 32 heads (of which the faster kernel is taken but for three, 5 % at most): workgroups of the kernel for many rows take
+// the tiles of the longest chain at `first` each alone on their CU and at `full` each and workgroup where several share it; those for few rows, one to a
+// CU, `start` and `step` for every eighth tile.  Not causal, whole rounds of workgroups; causal, heaviest first, the longest or all of them over the CUs.
 bool keys_shared(const FwdParams& p, int D) {
-  const double row_tiles = (p.Sq + 31) / 32, key_tiles = (p.Sk + F32_BN - 1) / F32_BN;
-  const double seen = p.causal && p.Sq <= p.Sk ? (row_tiles + 1) / 2 : key_tiles;  // per row tile (causal with fewer keys than rows: at most)
-  const double chain = p.causal && row_tiles < key_tiles ? row_tiles : key_tiles;
-  const double work = (double)p.B * p.H * row_tiles * seen / (4 * spa_device_cus());
-  const double per_chain = D == 128 ? 2.75 : D == 64 ? 1.43 : 1.3, per_work = D == 128 ? 2.75 : D == 64 ? 1.35 : 0.82;
-  const double many = chain * per_chain > work * per_work ? chain * per_chain : work * per_work;
-  return work * (D == 128 ? 6.0 : D == 64 ? 3.1 : 1.4) < many;
+  const double first = D == 128 ? 2.7 : D == 64 ? 1.65 : 1.4, full = D == 128 ? 2.8 : D == 64 ? 1.33 : 1.02;
+  const double start = D == 128 ? 2.5 : D == 64 ? 3.5 : 3.3, step = D == 128 ? 8.0 : D == 64 ? 4.1 : 2.7;
+  const double r = (p.Sq + 31) / 32, k = (p.Sk + F32_BN - 1) / F32_BN, cus = spa_device_cus(), pairs = (double)p.B * p.H;
+  const double chain = p.causal && r < k ? r : k;
+  // tiles that 32 rows see, and 128
+  const double seen = !p.causal ? k : r <= k ? (r + 1) / 2 : k - k * (k - 1) / (2 * r), seen4 = seen + 1.5 < k ? seen + 1.5 : k;
+  const double few = pairs * r / cus, many = pairs * ((p.Sq + 127) / 128) / cus;
+  double t_few, t_many;
+  if (p.causal) {
+    const double longest = start + chain / 8 * step, all = few * (start + seen / 8 * step);
+    t_few = longest > all ? longest : all;
+    t_many = chain * first > many * seen4 * full ? chain * first : many * seen4 * full;
+  } else {
+    t_few = ceil(few) * (start + k / 8 * step);
+    t_many = many <= 1 ? k * first : ceil(many) * k * full;
+  }
+  return t_few < t_many;
 }
 
 }  // namespace
+
+hipError_t spa_launch_fwd32_shared_keys_128(const FwdParams& p, hipStream_t stream);
 
 // One block pair, or whole sequences in shards (p.map).  Returns hipSuccess, or hipErrorInvalidValue for an unsupported D.
 hipError_t spa_launch_fwd32(FwdParams p, int D, hipStream_t stream) {
@@ -751,14 +871,15 @@ hipError_t spa_launch_fwd32(FwdParams p, int D, hipStream_t stream) {
   const int knob = spa_knob(SPA_KNOB_FWD32_SPLIT);
   if (!p.cu_q && knob != 1 && (knob == 2 || keys_shared(p, D))) {
     p.nqt = (p.Sq + 31) / 32;
-    if (D == 128) return launch<flash_fwd32_splitk_kernel<128, 4>>(256, Fwd32SplitCfg<128, 4>::SMEM, 32, p, stream);
-    if (D == 64) return launch<flash_fwd32_splitk_kernel<64, 8>>(512, Fwd32SplitCfg<64, 8>::SMEM, 32, p, stream);
-    if (D == 32) return launch<flash_fwd32_splitk_kernel<32, 8>>(512, Fwd32SplitCfg<32, 8>::SMEM, 32, p, stream);
+    if (D == 128) return spa_launch_fwd32_shared_keys_128(p, stream);
+    if (D == 64) return launch_splitk<64>(p, stream);
+    if (D == 32) return launch_splitk<32>(p, stream);
     return hipErrorInvalidValue;
   }
   p.nqt = (p.Sq + 127) / 128;
-  if (D == 128) return launch<flash_fwd32_kernel<128>>(F32_THREADS, Fwd32Cfg<128>::SMEM, 128, p, stream);
-  if (D == 64) return launch<flash_fwd32_kernel<64>>(F32_THREADS, Fwd32Cfg<64>::SMEM, 128, p, stream);
-  if (D == 32) return launch<flash_fwd32_kernel<32>>(F32_THREADS, Fwd32Cfg<32>::SMEM, 128, p, stream);
+  if (D == 128) return launch<flash_fwd32_kernel<128>>(F32_THREADS, Fwd32Cfg<128>::SMEM, 128, 1, p, stream);
+  if (D == 64) return launch<flash_fwd32_kernel<64>>(F32_THREADS, Fwd32Cfg<64>::SMEM, 128, 1, p, stream);
+  if (D == 32) return launch<flash_fwd32_kernel<32>>(F32_THREADS, Fwd32Cfg<32>::SMEM, 128, 1, p, stream);
   return hipErrorInvalidValue;
 }
+#endif

@@ -65,3 +65,54 @@ def test_strided_views_and_the_librarys_choice():
         check_lse(res[form][1].cpu(), want_l)
     assert torch.equal(res[0][0], res[2][0]), "32 workgroups of 128 rows on this device: the library takes the 32-row form"
     assert (res[1][0] - res[2][0]).abs().max().item() < 1e-5
+
+
+# One, two and four workgroups to 32 rows, by how many tiles of 32 rows there are for the CUs (256): 10 to 13, 96, 120 and 200.
+@pytest.mark.parametrize("B,H,Sq,Sk,D,causal", [(1, 3, 100, 333, 128, False), (1, 2, 161, 161, 128, True), (1, 24, 100, 333, 128, False),
+                                                (1, 24, 129, 200, 128, True), (1, 40, 129, 333, 128, False), (2, 20, 129, 100, 128, True),
+                                                (1, 24, 129, 333, 64, True), (1, 40, 130, 97, 64, False), (1, 2, 33, 31, 128, False)])
+def test_workgroups_that_share_rows(B, H, Sq, Sk, D, causal):
+    """Results of the forms whose workgroups take a part of the head dims each against the oracle, and, with an infinity in one value,
+    infinite and NaN where those of 128-row workgroups are (rows in shards as well)."""
+    g = torch.Generator().manual_seed(Sq * D + H)
+    q, k, v = (torch.randn((B, s, H, D), generator=g) for s in (Sq, Sk, Sk))
+    want_o, want_l = O.full_attention(q, k, v, None, causal)
+    bad = v.clone()
+    bad[0, Sk // 2, 1, D - 3] = float("inf")
+    bad[0, 0, 0, 5] = float("nan")
+    dev = [t.to(DEV) for t in (q, k, v, bad)]
+    res = {}
+    for form in (1, 2):
+        _lib.tune("fwd32_split", form)
+        try:
+            out, lse = ops.flash_fwd(*dev[:3], None, causal, layout="bshd")
+            res[form] = ops.flash_fwd(dev[0], dev[1], dev[3], None, causal, layout="bshd")[0]
+        finally:
+            _lib.tune("fwd32_split", 0)
+        check_out(out.cpu(), want_o, torch.float32, f"form {form}")
+        check_lse(lse.cpu(), want_l)
+    assert torch.equal(res[1].isnan(), res[2].isnan()) and torch.equal(res[1].isinf(), res[2].isinf())
+    finite = res[1].isfinite()
+    assert finite.any() and not finite.all()
+    # (fp32 sums of Sk weighted values of size 1 in another order)
+    assert (res[1] - res[2])[finite].abs().max().item() < 1e-5
+
+
+@pytest.mark.parametrize("B,H,D", [(1, 2, 128), (1, 12, 128), (1, 12, 64), (2, 12, 128)])
+def test_workgroups_that_share_rows_of_shards(B, H, D):
+    import sp_aurora_amd as sp
+    S, P = 4 * 66, 4
+    q, k, v = rand_qkv((B, S, H, D), 5 + H, torch.float32)
+    want_o, _ = O.full_attention(q, k, v, None, True)
+    order = torch.as_tensor(sp.ring.zigzag_order(S, P)) if hasattr(sp, "ring") else None
+    for sharding in ("contiguous", "zigzag"):
+        if sharding == "zigzag":
+            x, want = [t[:, order].to(DEV) for t in (q, k, v)], want_o[:, order]
+        else:
+            x, want = [t.to(DEV) for t in (q, k, v)], want_o
+        _lib.tune("fwd32_split", 2)
+        try:
+            out = sp.sp_aurora_func(*x, causal=True, ring_size=P, sharding=sharding)
+        finally:
+            _lib.tune("fwd32_split", 0)
+        check_out(out.cpu(), want, torch.float32, sharding)
