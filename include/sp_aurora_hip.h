@@ -122,9 +122,10 @@ int spa_flash_fwd_fp8kv(const void* q, const void* k8, const void* v8,
  * nsplit = 1 is spa_flash_fwd.  Chunks hold a multiple of 128 keys, so fewer than nsplit may run.  bf16 / fp16, D in
  * {64, 128}, mask none, K/V below 2 GiB per (batch, head).  workspace: spa_flash_fwd_splitkv_workspace_bytes() bytes, 16-byte
  * aligned, the caller's.  _fp8kv: K / V as e4m3 bytes with scales, as for spa_flash_fwd_fp8kv.
- * With up to three query rows (and no mask, the same types and sizes; e4m3 K/V rows 16-byte aligned) these entry points and
- * spa_flash_fwd / spa_flash_fwd_fp8kv run a kernel without matrix instructions that streams K and V past the rows at the
- * rate of HBM (a 128-row tile would hold one to three live rows); spa_tune(SPA_TUNE_FEW_ROWS, 1) keeps the other kernels.
+ * With up to sixteen query rows (and no mask, the same types and sizes; e4m3 K/V rows 16-byte aligned) these entry points and
+ * spa_flash_fwd / spa_flash_fwd_fp8kv run kernels that stream K and V past the rows at the rate of HBM (a 128-row tile would
+ * hold a few live rows): up to three rows whatever lies between the rows of K and V, more except from large 16-bit caches with
+ * other heads in between.  spa_tune(SPA_TUNE_FEW_ROWS, 1) keeps the other kernels.
  */
 int64_t spa_flash_fwd_splitkv_workspace_bytes(int B, int H, int Sq, int D, int nsplit, int dtype);
 int spa_flash_fwd_splitkv_suggest(int B, int H, int Sq, int Sk, int D, int mask_mode, int dtype);
@@ -551,8 +552,8 @@ int spa_attention_bwd_varlen(const void* q, const void* k, const void* v, const 
  *                          4 | 5   2 | 3 with compiler-scheduled MFMAs (at D = 128; otherwise as 2 | 3)
  *   SPA_TUNE_FWD32_SPLIT  1 | 2    never / always: the fp32 kernels with 32-row workgroups whose waves share
  *                                  the tiles (the library takes them where the longest chain of tiles decides)
- *   SPA_TUNE_FEW_ROWS     1        a key-split forward of up to 4 query rows runs on the MFMA kernels instead of the
- *                                  kernel that streams K and V past those rows
+ *   SPA_TUNE_FEW_ROWS     1        an unmasked forward of up to 16 query rows runs on the kernels for long rows instead of
+ *                                  those that stream K and V past a few
  */
 enum { SPA_TUNE_FWD_GROUPS = 0, SPA_TUNE_FWD_SHARE = 1, SPA_TUNE_BWD_DQ_WAVES = 2, SPA_TUNE_BWD_DKDV_FORM = 3, SPA_TUNE_FWD32_SPLIT = 4, SPA_TUNE_FEW_ROWS = 5 };
 int spa_tune(int knob, int value);

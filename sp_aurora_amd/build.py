@@ -31,6 +31,7 @@ UNITS = [
     ("spa_abi.hip", "spa_abi.o", []),
     ("merge.hip", "merge.o", []),
     ("decode_fwd.hip", "decode_fwd.o", []),
+    ("decode_rows_fwd.hip", "decode_rows_fwd.o", []),
     ("relayout.hip", "relayout.o", []),
 ]
 FLAGS = [

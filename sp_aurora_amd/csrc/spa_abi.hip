@@ -19,6 +19,8 @@ static __device__ __align__(256) unsigned char scratch[SPA_STATIC_SCRATCH_BYTES]
 hipError_t spa_launch_flash_fwd(FwdParams p, int D, int dtype, hipStream_t stream);
 hipError_t spa_launch_fwd16_splitkv(FwdParams p, int D, int dtype, hipStream_t stream);
 hipError_t spa_launch_fwd_fewrows(FwdParams p, int D, int dtype, hipStream_t stream);
+hipError_t spa_launch_fwd_rows16(const FwdParams& p, int D, int dtype, hipStream_t stream);
+bool spa_rows16_takes(const FwdParams& p, int D);
 int64_t spa_fewrows_chunks(int nseq, int total_k, int chunk);
 int64_t spa_fewrows_part_floats(int64_t pairs, int nq, int D);
 hipError_t spa_launch_splitkv_combine(void* out, float* lse, const void* part, const float* part_lse, int n, int B, int H, int Sq,
@@ -131,7 +133,8 @@ bool aligned8(const void* p, const int64_t* s, int n) {
 
 // The key-split forward: how the keys are cut for a wanted number of chunks (chunks of a multiple of 128 keys, the
 // last one what is left), and the scratch the chunks' results need.
-constexpr int kFewRows = 3;   // query rows the K/V-streaming kernel takes (spa_launch_fwd_fewrows)
+constexpr int kFewRows = 3;    // query rows of the kernel that streams K and V past them whatever lies between their rows (spa_launch_fwd_fewrows)
+constexpr int kRows16 = 16;    // and of the one that does on matrix instructions (spa_launch_fwd_rows16)
 struct KeySplit {
   int n, chunk, last;
   KeySplit(int Sk, int nsplit) {
@@ -196,12 +199,13 @@ int flash_fwd(const char* what, const void* q, const void* k, const void* v, con
       if (!can) return fail(SPA_EUNSUPPORTED, "%s: built for bf16 / fp16, head dim 64 or 128, K/V below 2 GiB per (batch, head)", what);
       if (!workspace || ((uintptr_t)workspace & 15) != 0) return fail(SPA_EINVAL, "%s: the key split needs a 16-byte aligned workspace", what);
     }
-    // Up to kFewRows query rows without a mask, split or not: the kernel that streams K and V past them (16 bytes a lane,
+    // Up to kRows16 query rows without a mask, split or not: the kernels that stream K and V past them (16 bytes a lane,
     // so e4m3 rows must be 16-byte aligned as well); more rows, or spa_tune(SPA_TUNE_FEW_ROWS, 1): the MFMA kernels (for a
     // split with the chunks as grid planes).
-    const bool few = can && Sq <= kFewRows && spa_knob(SPA_KNOB_FEW_ROWS) != 1 &&
+    const bool few = can && Sq <= kRows16 && spa_knob(SPA_KNOB_FEW_ROWS) != 1 &&
                      (!kv8 || (aligned16(k, k_strides, 1) && aligned16(v, v_strides, 1)));
     if (ks.n > 1 || few) {
+      const FwdParams whole = p;
       p.Sk = ks.chunk; p.sk_last = ks.last;
       p.P = ks.n; p.rank0 = 0; p.nranks = ks.n; p.t_begin = 0; p.t_count = 1;
       char* part_out = (char*)workspace;
@@ -212,7 +216,15 @@ int flash_fwd(const char* what, const void* q, const void* k, const void* v, con
         p.os.b = (int64_t)ks.n * Sq * H * D; p.os.s = (int64_t)H * D; p.os.h = D;
         p.lse_bh = (int64_t)ks.n * Sq;
       }
-      hipError_t e = few ? spa_launch_fwd_fewrows(p, D, dtype, (hipStream_t)stream) : spa_launch_fwd16_splitkv(p, D, dtype, (hipStream_t)stream);
+      hipError_t e;
+      if (few && spa_rows16_takes(p, D))
+        e = spa_launch_fwd_rows16(p, D, dtype, (hipStream_t)stream);
+      else if (few && Sq <= kFewRows)
+        e = spa_launch_fwd_fewrows(p, D, dtype, (hipStream_t)stream);
+      else if (ks.n > 1)
+        e = spa_launch_fwd16_splitkv(p, D, dtype, (hipStream_t)stream);
+      else
+        return launch_result(spa_launch_flash_fwd(whole, D, dtype, (hipStream_t)stream), what);
       if (e == hipSuccess && ks.n > 1)
         e = spa_launch_splitkv_combine(out, lse, part_out, part_lse, ks.n, B, H, Sq, D, S3(o_strides), Sq, dtype, (hipStream_t)stream);
       return launch_result(e, what);
@@ -251,11 +263,11 @@ int spa_flash_fwd_splitkv_suggest(int B, int H, int Sq, int Sk, int D, int mask_
   if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || mask_mode != SPA_MASK_NONE || (dtype != SPA_BF16 && dtype != SPA_F16) || (D != 64 && D != 128))
     return 1;
   const int cus = spa_device_cus();
-  // Up to kFewRows query rows run on the kernel that streams K and V: one workgroup per CU measured best on ten decode
+  // Up to kRows16 query rows run on the kernels that stream K and V: one workgroup per CU measured best on ten decode
   // shapes (more chunks: 3 to 15 % slower), chunks of at least 64 KB of bf16 keys (512 keys of 128 instead of 256, us a call: [1, 8, 1 against 2048] 9.4
   // and 8.5, 32 heads 10.9 and 9.1; for head dim 64 256 keys are no faster than 512).
-  if (Sq <= kFewRows && spa_knob(SPA_KNOB_FEW_ROWS) != 1) {
-    if (Sk < 1024) return 1;
+  if (Sq <= kRows16 && spa_knob(SPA_KNOB_FEW_ROWS) != 1) {
+    if (Sk < (Sq <= kFewRows ? 1024 : 2048)) return 1;
     int64_t n = ((int64_t)cus + (int64_t)B * H / 2) / ((int64_t)B * H);
     // (not more than 16 of them below 512 keys: the second kernel takes 2.3 us for 8 or 16 chunks of 8 heads and 5 for 32)
     const int64_t shortest = 32768 / D, by_length = Sk / shortest < 16 ? Sk / shortest : Sk / 512 > 16 ? Sk / 512 : 16;

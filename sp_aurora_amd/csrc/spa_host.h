@@ -16,7 +16,7 @@ enum {
   SPA_KNOB_BWD_DQ_WAVES = 2,  // the backward's dq kernel: 4 | 8 waves, 32 rows each; 20 | 24: 4 | 8 waves, pairs share 32 rows
   SPA_KNOB_BWD_DKDV_FORM = 3, // dk/dv kernel: 1 compiler-scheduled MFMAs at D = 128 (test twin), 2 | 3: 64 | 128 keys a workgroup, 4 | 5: their twins
   SPA_KNOB_FWD32_SPLIT = 4,   // 1: never the fp32 kernels of 32 rows whose waves share the tiles, 2: always
-  SPA_KNOB_FEW_ROWS = 5,     // 1: a key-split forward of up to 4 query rows stays on the MFMA kernels
+  SPA_KNOB_FEW_ROWS = 5,     // 1: a forward of up to 16 unmasked query rows stays on the kernels for long rows
   SPA_KNOB_COUNT = 6
 };
 extern std::atomic<int> g_spa_knob[SPA_KNOB_COUNT];

@@ -141,8 +141,8 @@ def flash_fwd(q, k, v, softmax_scale=None, causal=False, layout="bshd", out=None
     cache) the keys are cut into chunks that run side by side (spa_flash_fwd_splitkv[_fp8kv]): "auto" = as many as
     the library suggests, an int = that many, None or 1 = never.  The chunks' results wait in `workspace` (a uint8 tensor
     of flash_fwd_splitkv_workspace(...) bytes; allocated here when not given, except while the stream is being captured,
-    where "auto" then does not split).  With up to three query rows and no mask the library runs a kernel that streams K and V
-    past the rows instead of the matrix-instruction kernel, split or not."""
+    where "auto" then does not split).  With up to sixteen query rows and no mask the library runs kernels that stream K and V
+    past the rows instead of the kernels for long rows, split or not."""
     if out is None and lse is None and workspace is None and split_kv == "auto" and layout in ("bshd", "bhsd"):
         nat = _lib.native()
         if nat is not None:

@@ -1,0 +1,119 @@
+"""Calls of up to 16 query rows without a mask on the kernel that streams K and V through matrix instructions (rows of a head back to back, layout
+[B, H, S, D]; more than three rows also with other heads in between): edges of its tiles of 32 keys and of a workgroup's pass, chunks, both
+element types and e4m3, the values a weight of several terms has to get right."""
+import pytest
+import torch
+
+from conftest import rand
+from oracle import attn_oracle as O
+from sp_aurora_amd import _lib, ops
+from test_gpu_fp8kv import quantised
+from test_gpu_parity import DEV, check_lse, check_out
+
+pytestmark = pytest.mark.gpu
+
+
+def both(q, k, v, scale=None, layout="bhsd", **kw):
+    """The call on this kernel and on the others (spa_tune few_rows = 1)."""
+    res = []
+    for knob in (0, 1):
+        _lib.tune("few_rows", knob)
+        try:
+            res.append(ops.flash_fwd(q, k, v, scale, False, layout=layout, **kw))
+        finally:
+            _lib.tune("few_rows", 0)
+    return res
+
+
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("Sq,Sk,nsplit", [(1, 1, 1), (3, 31, 1), (4, 32, 1), (16, 33, 1), (2, 255, 2), (9, 256, 1), (1, 257, 1), (16, 257, 2), (5, 1300, 4), (15, 777, 6),
+                                          (3, 2049, 5)])
+def test_edges_against_the_oracle(layout, D, dtype, Sq, Sk, nsplit):
+    B, H = 2, 3
+    q, k, v = (rand((B, s, H, D), 40 + Sk + i, dtype) for i, s in enumerate((Sq, Sk, Sk)))
+    place = (lambda t: t.transpose(1, 2).contiguous().to(DEV)) if layout == "bhsd" else (lambda t: t.to(DEV))
+    for scale in (None, -0.4):
+        want_o, want_l = O.full_attention(q, k, v, scale, False)
+        out, lse = ops.flash_fwd(place(q), place(k), place(v), scale, False, layout=layout, split_kv=nsplit)
+        check_out(out.transpose(1, 2) if layout == "bhsd" else out, want_o, dtype, f"scale {scale}")
+        check_lse(lse, want_l)
+    k8, ks, k_deq = quantised((B, Sk, H, D), 50 + Sk, "bshd", spread=1.3)
+    v8, vs, v_deq = quantised((B, Sk, H, D), 51 + Sk, "bshd")
+    ks, vs = ks.to(DEV).clone(), vs.to(DEV)
+    ks[0, 1] = 0.0  # every key counts alike
+    k_deq = k_deq.clone()
+    k_deq[0, :, 1] = 0.0
+    want_o, want_l = O.full_attention(q, k_deq, v_deq, None, False)
+    out, lse = ops.flash_fwd(place(q), place(k8), place(v8), None, False, layout=layout, k_scale=ks, v_scale=vs, split_kv=nsplit)
+    check_out(out.transpose(1, 2) if layout == "bhsd" else out, want_o, dtype, "e4m3")
+    check_lse(lse, want_l)
+
+
+@pytest.mark.parametrize("e4m3", [False, True])
+@pytest.mark.parametrize("Sq", [1, 2, 8])
+def test_more_keys_than_the_memory_side_cache_holds(e4m3, Sq):
+    """Above 96 MiB of K and V the loads carry the non-temporal hint (16-bit: four waves): the same results as for the heads' halves, which are below."""
+    B, H, Sk, D = 2, 32, 6200 if e4m3 else 3100, 128
+    q, k, v = (rand((B, H, s, D), 60 + i, torch.bfloat16).to(DEV) for i, s in enumerate((Sq, Sk, Sk)))
+    kw = [{}, {}, {}]
+    if e4m3:
+        (k, ks), (v, vs) = (ops.quantize_fp8_per_head(t, layout="bhsd") for t in (k, v))
+        kw = [dict(k_scale=a, v_scale=b) for a, b in ((ks, vs), (ks[:1], vs[:1]), (ks[1:], vs[1:]))]
+    assert k.numel() * k.element_size() * 2 > 96 << 20 >= k.numel() * k.element_size()
+    out, lse = ops.flash_fwd(q, k, v, None, False, layout="bhsd", split_kv=2, **kw[0])
+    for i in range(2):
+        o, l = ops.flash_fwd(q[i:i + 1], k[i:i + 1], v[i:i + 1], None, False, layout="bhsd", split_kv=2, **kw[1 + i])
+        # sums over another number of waves, results (of chunks as well) rounded to bf16
+        assert (o.float() - out[i:i + 1].float()).abs().max().item() <= 2.0 ** -6 * out.float().abs().max().item()
+        assert (l - lse[i:i + 1]).abs().max().item() < 1e-5
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("Sq", [1, 3, 8])
+def test_infinities_and_nan(Sq, D, dtype):
+    """An infinity or a NaN in V reaches the dims that hold it and no others; a NaN in K reaches every row."""
+    B, H, Sk = 1, 2, 300
+    q, k, v = (rand((B, H, s, D), 70 + i, dtype) for i, s in enumerate((Sq, Sk, Sk)))
+    v[0, 0, 7, 3] = float("inf")
+    v[0, 0, 200, 5] = -float("inf")
+    v[0, 1, 33, D - 1] = float("nan")
+    out = ops.flash_fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, False, layout="bhsd")[0].float().cpu()
+    assert (out[0, 0, :, 3] == float("inf")).all() and (out[0, 0, :, 5] == -float("inf")).all() and out[0, 1, :, D - 1].isnan().all()
+    clean = torch.ones_like(out, dtype=torch.bool)
+    clean[0, 0, :, 3] = clean[0, 0, :, 5] = clean[0, 1, :, D - 1] = False
+    assert out[clean].isfinite().all()
+    k[0, 0, 10, 0] = float("nan")
+    out = ops.flash_fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, False, layout="bhsd")[0]
+    assert out[0, 0].isnan().all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Sq", [1, 3])
+def test_many_small_weights_beside_a_large_one(Sq, dtype):
+    """One key of weight 1 and value 0, thousands of weight 2^-23.1 and value 2^12: the result, about 3.8, is the sum of what the element type alone
+    would round away in fp16 (2^-24 is its smallest step)."""
+    D, Sk = 64, 8192
+    q = torch.zeros((1, 1, Sq, D), dtype=dtype)
+    k = torch.zeros((1, 1, Sk, D), dtype=dtype)
+    v = torch.full((1, 1, Sk, D), 4096.0, dtype=dtype)
+    q[..., 0] = 4.0
+    k[:, :, 1:, 0] = -4.0
+    v[:, :, 0] = 0.0
+    want, want_l = O.full_attention(*(t.transpose(1, 2) for t in (q, k, v)), 1.0, False)
+    out, lse = ops.flash_fwd(q.to(DEV), k.to(DEV), v.to(DEV), 1.0, False, layout="bhsd", split_kv=None)
+    # rounded once to the element type, weights off by 2^-22 at most
+    assert (out.cpu().double() / want.transpose(1, 2) - 1).abs().max().item() < (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -10)
+    check_lse(lse, want_l)
+
+
+@pytest.mark.parametrize("Sq", [1, 3, 4, 16])
+def test_large_values_do_not_overflow(Sq):
+    """bf16 values near the largest number under weights that grow along the keys: finite, as on the other kernels."""
+    B, H, Sk, D = 1, 2, 400, 128
+    q = torch.ones((B, H, Sq, D), dtype=torch.bfloat16)
+    k = (torch.arange(Sk).float()[None, None, :, None] * (0.05 if Sq <= 3 else 1.0) / D).expand(B, H, Sk, D).to(torch.bfloat16).contiguous()
+    v = torch.full((B, H, Sk, D), 1e36, dtype=torch.bfloat16)
+    (out, lse), (out2, lse2) = both(q.to(DEV), k.to(DEV), v.to(DEV), 1.0)
+    assert out.isfinite().all() and (out / 1e36 - 1).abs().max().item() < 2.0 ** -6
+    assert (lse - lse2).abs().max().item() < 1e-4
