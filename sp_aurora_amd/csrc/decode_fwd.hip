@@ -388,8 +388,8 @@ __global__ void __launch_bounds__(256) fewrows_combine_kernel(const FwdParams p)
   }
 }
 
-// Loads in flight and the non-temporal hint, measured on twelve decode shapes: four loads beat eight (6-10 %) except with three rows
-// and with single heads of 64-byte rows; the hint gains 5-15 % on 16-bit K/V, on e4m3 rows of a whole line when the keys are not split, and
+// Loads in flight and the non-temporal hint, measured on twelve decode shapes: four loads beat eight (6-10 %) except with three rows,
+// with single heads of 64-byte rows and with 512 bytes of a row; the hint gains 5-15 % on 16-bit K/V, on e4m3 rows of a whole line when the keys are not split, and
 // on e4m3 heads taken together (12 % split), and loses where workgroups share lines (64-byte rows) and on split calls of single e4m3 heads.
 template <typename T, int D, bool KV8, int NQ, int U, int HP, int W = 4>
 hipError_t launch_variant(const FwdParams& p, hipStream_t stream) {
@@ -410,10 +410,13 @@ hipError_t launch_variant(const FwdParams& p, hipStream_t stream) {
 // as many as make 256 bytes: 128-byte requests 4 KiB apart reach 5.1 TB/s, 256-byte ones 6.0 (64 caches of 1 to 4 thousand tokens, H = 32,
 // D = 128, e4m3: 256 -> 221 us; fixed length, B = 16, 4096 keys: e4m3 97 -> 85, bf16 D = 64 95 -> 80).  Not where that leaves CUs without
 // a workgroup: with one per CU and single heads 44 us, 48 together (B = 1, 32768 keys, e4m3, D = 128).
-// Rows of 128 elements, and eight workgroups per CU left: as many heads as make 512 bytes (64 caches of 2 to 8 thousand tokens, H = 32: e4m3 461 ->
-// 439 us, bf16 875 -> 839; of 1 to 4 thousand 237 -> 234 and 442 -> 435).  With fewer the last workgroups count for more: 32 caches of
-// 512 to 2048, e4m3, two per CU, 65 -> 75; 8 of 2 to 8 thousand, bf16, four, 118 -> 124.  Nor where one sequence, which is twice as long in such a
-// workgroup, is a good part of the whole launch: 255 caches of 256 tokens and one of 2200, e4m3 116 -> 155, bf16 194 -> 216.
+// Rows of 128 elements, and six workgroups per CU left: as many heads as make 512 bytes, eight loads of them in flight (caches of a quarter to all of
+// the length, H = 32, us, 256 bytes with four loads / 512 with four / 512 with eight: 64 of 4096, e4m3 233 / 224 / 217, bf16 416 / 400 / 391; 64 of 8192, e4m3
+// - / 411 / 399, bf16 - / 785 / 767; 32 of 4096, e4m3, six workgroups per CU, 112 / 117 / 107; 1 KB with four or eight 234 / 227 for the first).  With
+// fewer the last workgroups count for more: 32 caches of 480 to 1915, e4m3, 59.4 / 70.7 / 59.1, 8 of 2 to 8 thousand 65.3 / 61.7 / 66.4.  Two rows, which hold
+// half as many waves, gain with 32 heads and lose with 8 (64 of 8192, bf16, 512 with four / eight 204 / 207): four loads, and from eight workgroups per CU on.
+// Nor where one sequence, which is twice as long in such a workgroup, is a good part of the whole launch: 255 caches of 256 tokens and one of 2200, e4m3
+// 116 -> 155, bf16 194 -> 216.
 // A launch that leaves half of the CUs without a workgroup (a caller who did not split the keys) is bound by what its
 // few waves keep in flight: eight loads there too.
 template <typename T, int D, bool KV8, int NQ>
@@ -421,11 +424,11 @@ hipError_t launch_unroll(const FwdParams& p, hipStream_t stream) {
   constexpr int HP = 256 / (D * (KV8 ? 1 : 2));
   const int64_t groups = (int64_t)(p.cu_q && p.part ? 1 : p.B) * p.H * p.P;
   if constexpr (D == 128) {
-    constexpr int WIDE = 2 * HP;
+    constexpr int WIDE = 2 * HP, LOADS = NQ == 2 ? 4 : 8, LEAST = NQ == 1 ? 6 : 8;
     // (a packed batch: what one workgroup has to read, the longest sequence or a chunk, at 44 GB/s; all that is read, at 6 TB/s)
     const double longest = p.Sk * 1024.0 / 44e9, all = (double)p.chunk_rows * p.H * D * (KV8 ? 2 : 4) / 6e12;
-    if (p.H % WIDE == 0 && p.ks.h == D && p.vs.h == D && groups / WIDE >= 8 * spa_device_cus() && (!p.cu_q || 4 * longest <= all))
-      return launch_variant<T, D, KV8, NQ, NQ == 3 ? 8 : 4, WIDE>(p, stream);
+    if (p.H % WIDE == 0 && p.ks.h == D && p.vs.h == D && groups / WIDE >= LEAST * spa_device_cus() && (!p.cu_q || 4 * longest <= all))
+      return launch_variant<T, D, KV8, NQ, LOADS, WIDE>(p, stream);
   }
   if constexpr (HP > 1) {
     if (p.H % HP == 0 && p.ks.h == D && p.vs.h == D && groups / HP >= spa_device_cus())
