@@ -542,7 +542,7 @@ int spa_attention_bwd_varlen(const void* q, const void* k, const void* v, const 
 /*
  * Kernel-variant override for experiments and tests; no counterpart in the reference and not
  * needed in production (value 0 restores the library's own choice).  Process-wide.
- *   SPA_TUNE_FWD_GROUPS    1 | 2   wave groups per forward workgroup
+ *   SPA_TUNE_FWD_GROUPS    1 | 2 | 4   wave groups per forward workgroup (4: block calls)
  *   SPA_TUNE_FWD_SHARE     1 | 2   1 = 128-row workgroups, private K/V buffers per wave group;
  *                                  2 = 256-row workgroups sharing one set of buffers
  *   SPA_TUNE_BWD_DQ_WAVES  4 | 8   waves per workgroup of the backward's dq kernel, 32 query rows each

@@ -42,8 +42,9 @@ constexpr int FWD_BM = 128;  // query rows per workgroup
 // 128.  128-key sub-tiles for D = 64 (whose phases hold half the MFMA work against the same softmax
 // work) were measured 5-8 % slower than 64-key ones on every shape tried, long rows included:
 // fewer barriers do not pay for the coarser ping-pong and the 247-register VALU phase.
-template <int D>
-constexpr int fwd_bn() { return 64; }
+// (Four wave groups at D = 128: 32, so that their eight K and V buffers fit the LDS.)
+template <int D, int NG = 2>
+constexpr int fwd_bn() { return NG == 4 && D == 128 ? 32 : 64; }
 constexpr int FWD_THREADS = 256;  // threads of one wave group (4 waves x 32 query rows)
 constexpr int FWD_LOOK = 8;       // MFMA operands are fetched from LDS this many MFMAs ahead
 
@@ -51,20 +52,23 @@ constexpr int FWD_LOOK = 8;       // MFMA operands are fetched from LDS this man
 // each through LDS buffers of its own.  SHARE = true (NG = 2): the groups work on different query
 // rows (256 per workgroup), every group takes every sub-tile, and all 8 waves fill one set of
 // buffers together: half the global -> LDS traffic per FLOP and half as many workgroups.
+// NG = 4: 64 query rows by four groups of two waves; groups 0 and 1, then 2 and 3 are a phase apart.
 template <int D, int NG, bool SHARE>
 struct Fwd16Cfg {
-  static constexpr int BN = fwd_bn<D>();       // keys per sub-tile
+  static constexpr int BN = fwd_bn<D, NG>();   // keys per sub-tile
+  static constexpr int GROUP_ROWS = NG == 4 ? 64 : FWD_BM;  // query rows of a wave group
+  static constexpr int GROUP_THREADS = GROUP_ROWS * 2;      // a wave has 32 rows
   static constexpr int NT = BN / 32;           // 32-key score tiles per sub-tile
   static constexpr int ROWB = D * 2;           // bytes per K / V row in LDS: no padding, the tiles are swizzled
   static constexpr int TILEB = BN * ROWB;      // one K or V sub-tile
   static constexpr int GROUP = 4 * TILEB;      // one set of K[2] and V[2] buffers
-  static constexpr int BMW = SHARE ? NG * FWD_BM : FWD_BM;  // query rows per workgroup
-  static constexpr int EPI = (NG * FWD_BM * (D + 4) + NG * FWD_BM * 2 + BMW) * 4;  // epilogue staging
+  static constexpr int BMW = SHARE ? NG * FWD_BM : GROUP_ROWS;  // query rows per workgroup
+  static constexpr int EPI = NG == 4 ? 3 * GROUP_ROWS * (D + 6) * 4 : (NG * FWD_BM * (D + 4) + NG * FWD_BM * 2 + BMW) * 4;  // epilogue staging
   static constexpr int TILES = SHARE ? GROUP : NG * GROUP;
   static constexpr int SMEM = TILES > EPI ? TILES : EPI;
   static constexpr int SMEM_PLAIN = NG == 1 ? TILES : SMEM;  // one group writes a plain result from its registers
   static constexpr int CPR = D / 8;                         // 16-byte chunks per row
-  static constexpr int DTHREADS = SHARE ? NG * FWD_THREADS : FWD_THREADS;  // threads filling one buffer
+  static constexpr int DTHREADS = SHARE ? NG * FWD_THREADS : GROUP_THREADS;  // threads filling one buffer
   static constexpr int NDMA = TILEB / (DTHREADS * 16);      // direct loads per thread and sub-tile
   static constexpr int RPD = DTHREADS / CPR;                // rows one round of loads covers
   static_assert(!SHARE || (NG == 2 && NDMA >= 1), "shared buffers: two groups, at least one load per thread");
@@ -75,7 +79,7 @@ struct Fwd16Cfg {
 // K is read 16 bytes per lane by 16 consecutive rows at one chunk index; V is read by the
 // transposing 8-byte read, a half wave covering 4 rows x 64 bytes.
 template <int D>
-__device__ __forceinline__ int k_swizzle(int row) {
+__device__ __forceinline__ constexpr int k_swizzle(int row) {
   constexpr int CPR = D / 8;
   return (row / (16 / CPR)) % CPR;
 }
@@ -116,11 +120,12 @@ __device__ __forceinline__ int v_swizzle(int row) {
 // D = 64 (no difference); one group, which has to hold K(1) back for it, and 256 rows: none or 1 % slower.
 template <typename T, int D, int NG, bool SHARE, bool KV8 = false, bool FINALN = false, bool ZZ = false, bool BIG = false,
           bool QK8 = false, bool WAIT = false, bool KS = false, bool VR = false, bool MAP = false, bool Q_STAGED = false>
-__global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) flash_fwd16_kernel(const FwdParams pk) {
+__global__ void __launch_bounds__((Fwd16Cfg<D, NG, SHARE>::GROUP_THREADS * NG), NG == 1 && !FINALN ? 2 : 1) flash_fwd16_kernel(const FwdParams pk) {
   static_assert(!(FINALN && SHARE), "the merging epilogue goes with 128-row workgroups");
   static_assert(!MAP || (!KV8 && !FINALN && !ZZ && !BIG && !WAIT && !KS && !VR), "rows in shards: 16-bit block calls");
   static_assert(!KS || (!SHARE && !FINALN && !ZZ && !BIG && !QK8 && !WAIT), "split keys: 128-row workgroups, plain results");
-  static_assert(!Q_STAGED || (NG == 2 && !SHARE && !QK8), "staged queries: one copy in the two groups' buffers");
+  static_assert(!Q_STAGED || (NG >= 2 && !SHARE && !QK8), "staged queries: one copy in the groups' buffers");
+  static_assert(NG != 4 || (!SHARE && !FINALN && !ZZ && !BIG && !WAIT && !KS && !VR), "four groups: block calls");
   static_assert(!QK8 || (KV8 && D == 128 && !ZZ && !BIG), "8-bit scores: e4m3 q, k, v, head dim 128, contiguous chunks");
   typedef typename std::conditional<KV8, unsigned char, T>::type KVT;  // element type of K / V in memory
   typedef typename std::conditional<QK8, unsigned char, T>::type QT;   // element type of q in memory
@@ -134,9 +139,11 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int w = wave & 3;     // which 32 query rows
-  const int grp = wave >> 2;  // wave group: which key sub-tiles (or, with shared buffers, which 128 query rows)
-  const int tg = SHARE ? tid : tid & (FWD_THREADS - 1);  // thread index among those filling one buffer
+  constexpr int GT = C::GROUP_THREADS;
+  const int w = wave & (GT / 64 - 1);  // which 32 query rows
+  const int grp = wave / (GT / 64);    // wave group: which key sub-tiles (or, with shared buffers, which 128 query rows)
+  const int late = NG == 4 ? grp >> 1 : grp;     // 1: one phase behind (of the two waves of a SIMD, four apart, one each)
+  const int tg = SHARE ? tid : tid & (GT - 1);   // thread index among those filling one buffer
   const int ln = lane & 31;
   const int hh = lane >> 5;
 
@@ -197,7 +204,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     b = 0;
     if (p.Sk <= 0) {
       // no keys: the empty sum, out = 0 and lse = -inf
-      for (int idx = tid; idx < C::BMW * (D / 8); idx += FWD_THREADS * NG) {
+      for (int idx = tid; idx < C::BMW * (D / 8); idx += GT * NG) {
         const int grow = q0 + idx / (D / 8), ch = idx % (D / 8);
         if (grow >= p.Sq) break;
         u32x4 z = {0u, 0u, 0u, 0u};
@@ -292,7 +299,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
       const int64_t qoff0 = (int64_t)rank * p.Sq;
       T* const out0 = (T*)p.out + b * p.os.b + h * p.os.h + qoff0 * p.os.s;
       float* const lse0 = p.lse + ((int64_t)b * p.H + h) * p.lse_bh + qoff0;
-      for (int idx = tid; idx < C::BMW * (D / 8); idx += FWD_THREADS * NG) {
+      for (int idx = tid; idx < C::BMW * (D / 8); idx += GT * NG) {
         const int grow = q0 + idx / (D / 8), ch = idx % (D / 8);
         if (grow >= q_lim) break;
         float x[8], lb = -INFINITY, wsum = 0.f;
@@ -383,6 +390,10 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   auto k8_swizzle = [](int row) { return (row >> 1) & (CPR8 - 1); };
   const unsigned kdoff = QK8 ? (unsigned)((tg / CPR8) * p.ks.s + (((tg % CPR8) ^ k8_swizzle(tg / CPR8)) * 16))
                              : (unsigned)((drow * p.ks.s + ((dpos ^ k_swizzle<D>(drow)) * 8)) * (int64_t)sizeof(KVT));
+  // (fewer rows a round than K's permutation repeats after: the odd rounds have offsets of their own)
+  constexpr bool ODD_K = !QK8 && k_swizzle<D>(C::RPD) != 0;
+  const unsigned kdoff_odd = ODD_K ? (unsigned)((drow * p.ks.s + ((dpos ^ k_swizzle<D>(drow + C::RPD)) * 8)) * (int64_t)sizeof(KVT)) : kdoff;
+  static_assert(QK8 || k_swizzle<D>(2 * C::RPD) == 0, "K's permutation repeats after two rounds");
   const unsigned vdoff = (unsigned)((drow * p.vs.s + ((dpos ^ v_swizzle<D>(drow)) * 8)) * (int64_t)sizeof(KVT));
   const unsigned krow_b = (unsigned)(p.ks.s * (int64_t)sizeof(KVT));  // bytes per K row
   const unsigned vrow_b = (unsigned)(p.vs.s * (int64_t)sizeof(KVT));
@@ -399,6 +410,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   auto v_lds = [&](int i) { return (unsigned)(2 * C::TILEB + (i & 1) * C::TILEB); };
   // load number q of the pair (K sub-tile with first row k_row into buffer kb, V sub-tile v_row into vb)
   constexpr int NLOADS = NK + C::NDMA;
+  auto k_off = [&](int q) { return ODD_K && (q & 1) ? kdoff_odd : kdoff; };
   // the same two descriptors as compiler-visible resources, for loads into registers
   const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, (int)krsrc[2], 0x00020000);
   const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void*)vp, 0, (int)vrsrc[2], 0x00020000);
@@ -445,11 +457,11 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
         const unsigned lim = end < krsrc[2] ? end : krsrc[2];
         if constexpr (KSTAGE) {
           stage[q] = __builtin_bit_cast(
-              u32x2, __builtin_amdgcn_raw_buffer_load_b64(__builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, (int)lim, 0x00020000), kdoff + u, 0, 0));
+              u32x2, __builtin_amdgcn_raw_buffer_load_b64(__builtin_amdgcn_make_buffer_rsrc((void*)kp, 0, (int)lim, 0x00020000), k_off(q) + u, 0, 0));
         } else {
           u32x4 rs = krsrc;
           rs[2] = lim;
-          load_to_lds_b128(rs, kdoff + u, lds_wave + kb + q * (C::DTHREADS * 16));
+          load_to_lds_b128(rs, k_off(q) + u, lds_wave + kb + q * (C::DTHREADS * 16));
         }
       } else {
         const int r = q - NK;
@@ -469,7 +481,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     }
     if constexpr (MAP) {
       if (q < NK)
-        load_to_lds_b128(krsrc, kon ? kdoff + (unsigned)(k_row + q * RPD_K) * krow_b + at_k[q] : OFF_NONE, lds_wave + kb + q * (C::DTHREADS * 16));
+        load_to_lds_b128(krsrc, kon ? k_off(q) + (unsigned)(k_row + q * RPD_K) * krow_b + at_k[q] : OFF_NONE, lds_wave + kb + q * (C::DTHREADS * 16));
       else
         load_to_lds_b128(vrsrc, von ? vdoff + (unsigned)(v_row + (q - NK) * C::RPD) * krow_b + at_v[q - NK] : OFF_NONE,
                          lds_wave + vb + (q - NK) * (C::DTHREADS * 16));
@@ -481,16 +493,16 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
         unsigned rel = OFF_NONE;
         u32x4 rs = krsrc;
         if (kon) rs = buffer_window(kp, kbytes, (unsigned long long)(unsigned)k_row * krow_b, rel);
-        load_to_lds_b128(rs, kdoff + rel + (unsigned)(q * C::RPD) * krow_b, lds_wave + kb + q * (C::DTHREADS * 16));
+        load_to_lds_b128(rs, k_off(q) + rel + (unsigned)(q * C::RPD) * krow_b, lds_wave + kb + q * (C::DTHREADS * 16));
         return;
       }
       const unsigned u = kon ? (unsigned)(k_row + q * RPD_K) * krow_b : OFF_NONE;
       if constexpr (KSTAGE)
-        stage[q] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(krs, kdoff + u, 0, 0));
+        stage[q] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(krs, k_off(q) + u, 0, 0));
       else if constexpr (KS_NT)
-        load_to_lds_b128_nt(krsrc, kdoff + u, lds_wave + kb + q * (C::DTHREADS * 16));
+        load_to_lds_b128_nt(krsrc, k_off(q) + u, lds_wave + kb + q * (C::DTHREADS * 16));
       else
-        load_to_lds_b128(krsrc, kdoff + u, lds_wave + kb + q * (C::DTHREADS * 16));
+        load_to_lds_b128(krsrc, k_off(q) + u, lds_wave + kb + q * (C::DTHREADS * 16));
     } else {
       const int r = q - NK;
       if constexpr (BIG) {
@@ -774,19 +786,23 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     cs.sb.krow = ch * crow + cs.sb.krel;
     cs.sb.kend = ch * crow + p.Sk;
   }
+  // Four groups on 64 rows: of the keys of a step on the diagonal some groups' whole sub-tiles lie behind the last row.  They count for nothing (P = 0), as
+  // zeros, so that an infinity in V reaches no row further away than with the other forms.
+  auto seen = [&](const Sub& sb) { return NG != 4 || !sb.masked || sb.krel < kv_end; };
   cv = cs;
   cursor_next(cv);
   ck = cv;
   cursor_next(ck);
-  // (Q_STAGED: into the groups' second V buffers, which nothing else needs before the first MFMA phase; each group loads half of every wave's rows)
-  const unsigned q_block = (unsigned)(uintptr_t)(lds_u8*)smem + (w >> 1) * C::GROUP + 3 * C::TILEB + (w & 1) * 32 * C::ROWB;  // the wave's 32 rows
+  // (Q_STAGED: into the groups' second V buffers, which nothing else needs before the first MFMA phase; each group loads its share of every wave's rows)
+  const unsigned q_block = (unsigned)(uintptr_t)(lds_u8*)smem + (NG == 4 ? w * C::GROUP + 3 * C::TILEB : (w >> 1) * C::GROUP + 3 * C::TILEB + (w & 1) * 32 * C::ROWB);  // the wave's 32 rows
   if constexpr (Q_STAGED) {
+    constexpr int SHARE_ROWS = 32 / NG;
 #pragma unroll
-    for (int j = 0; j < 16 * C::CPR / 64; ++j) {
-      const int r = grp * 16 + j * (64 / C::CPR) + lane / C::CPR;
+    for (int j = 0; j < SHARE_ROWS * C::CPR / 64; ++j) {
+      const int r = grp * SHARE_ROWS + j * (64 / C::CPR) + lane / C::CPR;
       const int row = qw0 + r < q_lim ? qw0 + r : q_lim - 1;
       const QT* const src = qp + (int64_t)(MAP ? map.at(row, p.map.pitch) : row) * p.qs.s + ((lane % C::CPR) ^ k_swizzle<D>(r)) * 8;
-      load_to_lds_b128(src, q_block + (grp * 16 + j * (64 / C::CPR)) * C::ROWB);
+      load_to_lds_b128(src, q_block + (grp * SHARE_ROWS + j * (64 / C::CPR)) * C::ROWB);
     }
   }
   // WAIT: no tile of a chunk is requested before the chunk's arrival flag has been seen (each wave polls for itself;
@@ -821,9 +837,9 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     for (int q = 0; q < C::NDMA; ++q) at_v[q] = at_k[q];
   }
 #pragma unroll
-  for (int q = 0; q < NK; ++q) load_one(q, 0 < n, cs.sb.krow, k_lds(0), false, 0, 0, cs.sb.kend, 0);     // K(0)
+  for (int q = 0; q < NK; ++q) load_one(q, 0 < n && seen(cs.sb), cs.sb.krow, k_lds(0), false, 0, 0, cs.sb.kend, 0);     // K(0)
 #pragma unroll
-  for (int q = 0; q < C::NDMA; ++q) load_one(NK + q, false, 0, 0, 0 < n, cs.sb.krow, v_lds(0), 0, cs.sb.kend);  // V(0)
+  for (int q = 0; q < C::NDMA; ++q) load_one(NK + q, false, 0, 0, 0 < n && seen(cs.sb), cs.sb.krow, v_lds(0), 0, cs.sb.kend);  // V(0)
   if constexpr (KSTAGE) {
     // K(0) goes to LDS now; V(0) stays staged together with K(1), loaded next, and both are written
     // by the first VALU phase like every later pair
@@ -833,7 +849,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   }
   if constexpr (MAP) find_rows(cv.sb.krel, at_k);
 #pragma unroll
-  for (int q = 0; q < NK; ++q) load_one(q, 1 < n, cv.sb.krow, k_lds(1), false, 0, 0, cv.sb.kend, 0);     // K(1)
+  for (int q = 0; q < NK; ++q) load_one(q, 1 < n && seen(cv.sb), cv.sb.krow, k_lds(1), false, 0, 0, cv.sb.kend, 0);     // K(1)
   auto next_rows = [&]() {  // K moves on to sub-tile i + 2 of the next step, V to what K had
     if constexpr (MAP) {
 #pragma unroll
@@ -862,7 +878,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     mfma_phase(std::false_type{}, std::true_type{}, va, ka, none, [](int) {});  // S(0)
   }
   __syncthreads();
-  if (NG > 1 && grp == 1) {  // group 1 runs one phase behind group 0
+  if (NG > 1 && late == 1) {  // group 1 runs one phase behind group 0
     loads_landed();          // (with shared buffers group 0 reads this group's share of V(0), K(1) after this barrier)
     if constexpr (SHARE) store_staged(k_lds(1), v_lds(0));
     __syncthreads();
@@ -882,7 +898,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   auto body = [&](auto parity, int i) __attribute__((always_inline)) {
     constexpr int PAR = decltype(parity)::value;  // == i & 1
     frag pf[NT][2];
-    const bool kon = ck.i < n, von = cv.i < n;
+    const bool kon = ck.i < n && seen(ck.sb), von = cv.i < n && seen(cv.sb);
     constexpr unsigned kb = (unsigned)(PAR * C::TILEB), vb = (unsigned)(2 * C::TILEB + (PAR ^ 1) * C::TILEB);  // k_lds(i), v_lds(i + 1)
     if (early) {
 #pragma unroll
@@ -945,7 +961,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
     mfma_phase(std::true_type{}, std::false_type{}, va, ka, pf, [](int) {});
     if (!SHARE || early) __syncthreads();
   }
-  if (NG > 1 && grp == 0) __syncthreads();  // matches group 1's leading barrier
+  if (NG > 1 && late == 0) __syncthreads();  // matches group 1's leading barrier
 
   // ---- epilogue ----
   // The groups exchange only (m, l) per row; each scales its own partial O by
@@ -964,7 +980,7 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   // next 4; one v_permlane32_swap per dword pairs them up so that every lane stores 16-byte pieces, the two
   // lanes of a row side by side.  `other`: the same rows' partial sums of the other wave group, staged in LDS
   // in the accumulator's own layout (128 rows of D + 4 floats), or null.
-  auto store_rows = [&](float a_own, auto with_other, const float* other, float a_other, float lse_val) {
+  auto store_rows = [&](float a_own, auto with_other, const float* other, const float* a_other, float lse_val) {
     constexpr bool OTHER = decltype(with_other)::value;
     if (hh == 0 && qrow < q_lim) lse_bh[MAP ? map.at(qrow, p.map.lse_pitch) : qrow] = lse_val;
     T* const orow = out_bh + qrow_t * out_rs;
@@ -976,12 +992,16 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
 #pragma unroll
         for (int i = 0; i < 8; ++i) e[i] = o[db][8 * gp + i] * a_own;
         if constexpr (OTHER) {
-          const f32x4 p0 = *(const f32x4*)(other + db * 32 + 8 * (2 * gp) + 4 * hh);
-          const f32x4 p1 = *(const f32x4*)(other + db * 32 + 8 * (2 * gp + 1) + 4 * hh);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            e[i] = __builtin_fmaf(p0[i], a_other, e[i]);
-            e[4 + i] = __builtin_fmaf(p1[i], a_other, e[4 + i]);
+          for (int g = 0; g < NG - 1; ++g) {
+            const float* const rows = other + g * (C::GROUP_ROWS * (D + 4)) + db * 32 + 4 * hh;
+            const f32x4 p0 = *(const f32x4*)(rows + 8 * (2 * gp));
+            const f32x4 p1 = *(const f32x4*)(rows + 8 * (2 * gp + 1));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              e[i] = __builtin_fmaf(p0[i], a_other[g], e[i]);
+              e[4 + i] = __builtin_fmaf(p1[i], a_other[g], e[4 + i]);
+            }
           }
         }
         unsigned x[2], y[2];  // as two packed pairs each
@@ -1003,18 +1023,20 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
   if constexpr (SHARE || (NG == 1 && !FINALN)) {
     // a wave's rows are complete: no LDS round trip, no barrier
     const float l_tot = halves_sum(l_run);
-    store_rows(vsc / l_tot, std::false_type{}, nullptr, 0.f, (m_run * c + fast_log2(l_tot)) * 0.6931471805599453f);
+    store_rows(vsc / l_tot, std::false_type{}, nullptr, nullptr, (m_run * c + fast_log2(l_tot)) * 0.6931471805599453f);
     return;
   } else if constexpr (!FINALN) {
-    // Two groups hold partial sums of the same rows.  Group 1 stages its unscaled partial O (fp32, its own
-    // register layout) and (m, l) in LDS, free now, and leaves; group 0 weighs both by exp2((m - m_all) c) / l_all
-    // and stores the rows from its registers.  One barrier, one staged tile.
+    // The groups hold partial sums of the same rows.  All but the first stage their unscaled partial O (fp32, its own
+    // register layout) and (m, l) in LDS, free now, and leave; group 0 weighs all by exp2((m - m_all) c) / l_all
+    // and stores the rows from its registers.  One barrier.
     constexpr int TP = D + 4;  // floats per staged row
+    constexpr int GR = C::GROUP_ROWS;
     float* const tile = (float*)smem;
-    float* const ml = tile + FWD_BM * TP;  // [128](m, l) of group 1
+    float* const ml = tile + (NG - 1) * (GR * TP);  // (m, l) of the rows of groups 1 ..
     const int rloc = w * 32 + ln;
     const float l_own = halves_sum(l_run);
-    if (grp == 1) {
+    if (grp > 0) {
+      const int at = (grp - 1) * GR + rloc;
 #pragma unroll
       for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -1024,22 +1046,29 @@ __global__ void __launch_bounds__(FWD_THREADS * NG, NG == 1 && !FINALN ? 2 : 1) 
           st[1] = o[db][4 * g + 1];
           st[2] = o[db][4 * g + 2];
           st[3] = o[db][4 * g + 3];
-          *(f32x4*)(tile + rloc * TP + db * 32 + 8 * g + 4 * hh) = st;
+          *(f32x4*)(tile + at * TP + db * 32 + 8 * g + 4 * hh) = st;
         }
       if (hh == 0) {
-        ml[rloc * 2] = m_run;
-        ml[rloc * 2 + 1] = l_own;
+        ml[at * 2] = m_run;
+        ml[at * 2 + 1] = l_own;
       }
     }
     __syncthreads();
-    if (grp == 1) return;
-    const float m2 = ml[rloc * 2], l2 = ml[rloc * 2 + 1];
-    const float m_all = fmaxf(m_run, m2);  // finite: some group has seen key 0 of the first chunk
-    const float a1 = fast_exp2((m_run - m_all) * c);
-    const float a2 = fast_exp2((m2 - m_all) * c);
-    const float l_all = l_own * a1 + l2 * a2;
+    if (grp > 0) return;
+    float a[NG], m_all = m_run;  // finite in the end: some group has seen key 0 of the first chunk
+#pragma unroll
+    for (int g = 1; g < NG; ++g) m_all = fmaxf(m_all, ml[((g - 1) * GR + rloc) * 2]);
+    a[0] = fast_exp2((m_run - m_all) * c);
+    float l_all = l_own * a[0];
+#pragma unroll
+    for (int g = 1; g < NG; ++g) {
+      a[g] = fast_exp2((ml[((g - 1) * GR + rloc) * 2] - m_all) * c);
+      l_all += ml[((g - 1) * GR + rloc) * 2 + 1] * a[g];
+    }
     const float sc = vsc / l_all;
-    store_rows(a1 * sc, std::true_type{}, tile + rloc * TP, a2 * sc, (m_all * c + fast_log2(l_all)) * 0.6931471805599453f);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) a[g] *= sc;
+    store_rows(a[0], std::true_type{}, tile + rloc * TP, a + 1, (m_all * c + fast_log2(l_all)) * 0.6931471805599453f);
     return;
   } else {
     constexpr int TP = D + 4;  // floats per staged row
@@ -1225,9 +1254,10 @@ int fwd_tiles(const FwdParams& p, int bm) {
   return p.zz_half ? per_half : 2 * per_half;
 }
 
-// The three forms of a workgroup: FWD_ONE, 128 rows by one wave group, two or three workgroups to a CU; FWD_SPLIT, 128 rows
-// by two groups that take alternate key tiles; FWD_SHARE, 256 rows by two groups on shared K/V buffers.
-enum FwdForm { FWD_ONE, FWD_SPLIT, FWD_SHARE, FWD_FORMS };
+// The four forms of a workgroup: FWD_ONE, 128 rows by one wave group, two or three workgroups to a CU; FWD_SPLIT, 128 rows
+// by two groups that take alternate key tiles; FWD_SHARE, 256 rows by two groups on shared K/V buffers; FWD_FOUR, 64 rows by four groups of
+// two waves that take every fourth key tile.
+enum FwdForm { FWD_ONE, FWD_SPLIT, FWD_SHARE, FWD_FOUR, FWD_FORMS };
 
 // What a launch of a form takes, in us: the longer of its heaviest workgroup alone (`alone` per 64-key step) and of the whole
 // launch with every CU busy (`busy` per step and workgroup), the workgroup's fixed cost once per round of workgroups, and
@@ -1236,19 +1266,23 @@ enum FwdForm { FWD_ONE, FWD_SPLIT, FWD_SHARE, FWD_FORMS };
 // decides: FWD_SHARE moves half the K/V bytes per product and is the fastest on long rows at D = 128 (1260 against 1180 TFLOP/s
 // at 8192 keys); FWD_ONE overlaps one workgroup's start and end with another's work and wins on short rows (64 sequences of
 // 512, causal: 506 against 427 TFLOP/s at D = 128), and everywhere at D = 64, where three waves to a SIMD hide the
-// softmax (8192 keys: 980 against 860); FWD_SPLIT halves the heaviest workgroup and wins while the grid does not fill the CUs.
+// softmax (8192 keys: 980 against 860); FWD_SPLIT halves the heaviest workgroup and wins while the grid does not fill the CUs; FWD_FOUR,
+// with twice the workgroups and half as long a chain, while its own does not (bf16, causal, us, ONE / SPLIT / FOUR: [1,512,8,128] 13.7 / 11.7 / 9.8,
+// [1,2048,8,128] 39.5 / 27.6 / 21.2, [1,926,16,128] 20.6 / 17.1 / 13.7, [1,512,32,64] 10.7 / 10.0 / 8.3, [1,2048,8,64] 29.5 / 21.8 / 15.4; 300 workgroups and
+// more: [1,768,32,128] 19.1 / 15.5 / 16.8, [2,512,32,64] 11.1 / 10.5 / 14.1).
 struct FormCost {
   float alone, busy, round, fixed;
 };
 enum FwdKind { KIND_16, KIND_KV8, KIND_QK8 };  // 16-bit K/V; e4m3 K/V; e4m3 q, K/V
 float form_us(const FwdParams& p, FwdForm f, int D, FwdKind kind) {
   static constexpr FormCost cost[4][FWD_FORMS] = {
-      {{0.98f, 0.96f, 5.1f, 2.0f}, {1.36f, 1.81f, 6.2f, 2.2f}, {1.24f, 1.67f, 8.9f, 0.5f}},    // 16 bits, D = 128
-      {{0.79f, 0.56f, 4.9f, 0.4f}, {1.03f, 1.18f, 4.1f, 2.2f}, {1.04f, 1.17f, 5.1f, 1.8f}},    // 16 bits, D <= 64
-      {{1.39f, 0.96f, 5.3f, 0.4f}, {1.68f, 1.91f, 6.0f, 2.7f}, {1.40f, 1.73f, 7.9f, 1.3f}},    // e4m3 K/V
-      {{1.11f, 0.75f, 4.6f, 0.4f}, {1.40f, 1.53f, 5.0f, 2.6f}, {1.16f, 1.38f, 6.6f, 1.4f}}};   // e4m3 q, K/V
+      {{0.98f, 0.96f, 5.1f, 2.0f}, {1.36f, 1.81f, 6.2f, 2.2f}, {1.24f, 1.67f, 8.9f, 0.5f}, {0.98f, 1.00f, 5.5f, 2.6f}},    // 16 bits, D = 128
+      {{0.79f, 0.56f, 4.9f, 0.4f}, {1.03f, 1.18f, 4.1f, 2.2f}, {1.04f, 1.17f, 5.1f, 1.8f}, {1.25f, 1.25f, 5.0f, 1.45f}},    // 16 bits, D <= 64
+      {{1.39f, 0.96f, 5.3f, 0.4f}, {1.68f, 1.91f, 6.0f, 2.7f}, {1.40f, 1.73f, 7.9f, 1.3f}, {1.31f, 1.32f, 5.6f, 3.0f}},    // e4m3 K/V
+      {{1.11f, 0.75f, 4.6f, 0.4f}, {1.40f, 1.53f, 5.0f, 2.6f}, {1.16f, 1.38f, 6.6f, 1.4f}, {1.09f, 1.05f, 5.0f, 2.4f}}};   // e4m3 q, K/V
   const FormCost& c = cost[kind == KIND_QK8 ? 3 : kind == KIND_KV8 ? 2 : D > 64 ? 0 : 1][f];
-  const float rows = f == FWD_SHARE ? 2 * FWD_BM : FWD_BM, keys = f == FWD_SPLIT ? 128.f : 64.f;  // of a workgroup, of a step
+  const float rows = f == FWD_SHARE ? 2 * FWD_BM : f == FWD_FOUR ? 64 : FWD_BM;                                  // of a workgroup
+  const float keys = f == FWD_SPLIT ? 128.f : f == FWD_FOUR ? (D > 64 ? 4.f * fwd_bn<128, 4>() : 4.f * fwd_bn<64, 4>()) : 64.f;  // of a step
   const float slots = (float)spa_device_cus() * (f == FWD_ONE ? (D > 64 ? 2 : 3) : 1), cus = (float)spa_device_cus();
   // sequences of a packed batch: as many rows as they have on average, the heaviest as many keys as the longest
   float sq = (float)p.Sq, sk = (float)p.Sk, tiles = ceilf(sq / rows);
@@ -1275,6 +1309,10 @@ FwdForm fwd_form(const FwdParams& p, int D, FwdKind kind) {
   const int force_share = spa_knob(SPA_KNOB_FWD_SHARE);
   const bool can_share = D >= 64 && p.epi != SPA_EPI_FINALN;
   if (force ? force == 1 : p.Sk <= fwd_bn<128>()) return FWD_ONE;  // one sub-tile: nothing to split
+  // (e4m3 K/V of 64 elements have the constants of 128: only where those say the same as the clock, in one round of workgroups)
+  const bool can_four = D >= 64 && !p.cu_q && p.P == 1 && !p.zigzag && p.epi == SPA_EPI_PLAIN &&
+                        (kind != KIND_KV8 || D > 64 || (int64_t)p.B * p.H * fwd_tiles(p, 64) <= spa_device_cus());
+  if (force == 4 && can_four) return FWD_FOUR;
   if (force_share && can_share) return force_share == 2 ? FWD_SHARE : FWD_SPLIT;
   if (p.P > 1 || p.zigzag || p.epi != SPA_EPI_PLAIN) {
     // a ring schedule: 256-row workgroups once that still leaves every CU two of them
@@ -1283,8 +1321,8 @@ FwdForm fwd_form(const FwdParams& p, int D, FwdKind kind) {
   }
   FwdForm best = FWD_SPLIT;
   float us = 0.96f * form_us(p, FWD_SPLIT, D, kind);  // (a margin for the form that suits small grids: near the line it is the safer one)
-  for (const FwdForm f : {FWD_SHARE, FWD_ONE}) {
-    if ((f == FWD_SHARE && !can_share) || (f == FWD_ONE && force == 2)) continue;
+  for (const FwdForm f : {FWD_SHARE, FWD_ONE, FWD_FOUR}) {
+    if ((f == FWD_SHARE && !can_share) || (f == FWD_ONE && force == 2) || (f == FWD_FOUR && (force || !can_four))) continue;
     const float u = form_us(p, f, D, kind);
     if (u < us) {
       us = u;
@@ -1308,6 +1346,16 @@ hipError_t launch16(FwdParams p, hipStream_t stream) {
       p.nqt = fwd_tiles(p, 2 * FWD_BM);
       return launch<flash_fwd16_kernel<T, D, 2, true, KV8, false, ZZ, false, QK8>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, true>::SMEM, 2 * FWD_BM, p, stream);
     }
+  if constexpr (D >= 64 && !ZZ)
+    if (form == FWD_FOUR) {
+      constexpr int rows = Fwd16Cfg<D, 4, false>::GROUP_ROWS;
+      p.nqt = fwd_tiles(p, rows);
+      if constexpr (D == 128 && !KV8)
+        if (p.qs.s != D)
+          return launch<flash_fwd16_kernel<T, D, 4, false, false, false, false, false, false, false, false, false, false, true>>(
+              2 * FWD_THREADS, Fwd16Cfg<D, 4, false>::SMEM, rows, p, stream);
+      return launch<flash_fwd16_kernel<T, D, 4, false, KV8, false, ZZ, false, QK8>>(2 * FWD_THREADS, Fwd16Cfg<D, 4, false>::SMEM, rows, p, stream);
+    }
   if constexpr (D == 128 && !KV8 && !ZZ)
     if (form == FWD_SPLIT && p.qs.s != D)
       return launch<flash_fwd16_kernel<T, D, 2, false, false, false, false, false, false, false, false, false, false, true>>(
@@ -1317,7 +1365,7 @@ hipError_t launch16(FwdParams p, hipStream_t stream) {
   return launch<flash_fwd16_kernel<T, D, 1, false, KV8, false, ZZ, false, QK8>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM_PLAIN, FWD_BM, p, stream);
 }
 
-// Rows in shards: the same three forms.
+// Rows in shards: the same forms.
 template <typename T, int D>
 hipError_t launch16_map(FwdParams p, hipStream_t stream) {
   const FwdForm form = fwd_form(p, D, KIND_16);
@@ -1326,6 +1374,12 @@ hipError_t launch16_map(FwdParams p, hipStream_t stream) {
     if (form == FWD_SHARE) {
       p.nqt = fwd_tiles(p, 2 * FWD_BM);
       return launch<flash_fwd16_kernel<T, D, 2, true, N, N, N, N, N, N, N, N, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, true>::SMEM, 2 * FWD_BM, p, stream);
+    }
+  if constexpr (D >= 64)
+    if (form == FWD_FOUR) {
+      constexpr int rows = Fwd16Cfg<D, 4, false>::GROUP_ROWS;
+      p.nqt = fwd_tiles(p, rows);
+      return launch<flash_fwd16_kernel<T, D, 4, false, N, N, N, N, N, N, N, N, true, D == 128>>(2 * FWD_THREADS, Fwd16Cfg<D, 4, false>::SMEM, rows, p, stream);
     }
   if (form == FWD_SPLIT)
     return launch<flash_fwd16_kernel<T, D, 2, false, N, N, N, N, N, N, N, N, true, D == 128>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);

@@ -275,15 +275,17 @@ int spa_flash_fwd_splitkv_suggest(int B, int H, int Sq, int Sk, int D, int mask_
     if (n > 64) n = 64;
     return n < 2 ? 1 : KeySplit(Sk, (int)n).n;
   }
-  // Otherwise worth it when the 128-row workgroups of the plain launch leave at least half of the CUs idle and every
-  // chunk keeps at least 512 keys: as many chunks as give every CU one workgroup (measured on six decode shapes: more
-  // chunks only add the workgroups' fixed cost and rows for the merge).
+  // Otherwise worth it when 128-row workgroups would leave two thirds of the CUs idle and every
+  // chunk keeps at least 512 keys: as many chunks as give no CU more than one workgroup (measured on six decode shapes: more
+  // chunks only add the workgroups' fixed cost and rows for the merge).  Not fewer than four, or three of long rows: beside the form of the plain
+  // launch that shares 64 rows out over four wave groups (us, D = 128, split / plain: 8 heads of 2048 rows and 4096 keys, two, 44.4 / 40.9; 16 of 600
+  // and 2048, three, 24.6 / 20.9, of 640 and 4096 33.9 / 35.1; 8 of 1024 and 2048, four, 22.0 / 21.1, of 400 17.8 / 20.6).
   const int64_t wgs = (int64_t)B * H * ((Sq + 127) / 128);
-  if (wgs * 2 > cus || Sk < 2048) return 1;
-  int64_t n = ((int64_t)cus + wgs / 2) / wgs;
+  if (wgs * 3 > cus || Sk < 2048) return 1;
+  int64_t n = cus / wgs;
   if (n > Sk / 512) n = Sk / 512;
   if (n > 64) n = 64;
-  return n < 2 ? 1 : KeySplit(Sk, (int)n).n;
+  return n < 3 || (n == 3 && Sk < 4096) ? 1 : KeySplit(Sk, (int)n).n;
 }
 
 int spa_flash_fwd_splitkv(const void* q, const void* k, const void* v, void* out, float* lse, void* workspace, int B, int H, int Sq,

@@ -11,7 +11,7 @@ constexpr int SPA_MAX_DEVICES = 64;
 // Variant overrides for experiments and tests (set through spa_tune, never read from the
 // environment); 0 = the library's own choice.
 enum {
-  SPA_KNOB_FWD_GROUPS = 0,    // 1 | 2 wave groups per forward workgroup
+  SPA_KNOB_FWD_GROUPS = 0,    // 1 | 2 | 4 wave groups per forward workgroup (4: block calls)
   SPA_KNOB_FWD_SHARE = 1,     // 1: private K/V buffers per group, 2: 256-row workgroups sharing them
   SPA_KNOB_BWD_DQ_WAVES = 2,  // the backward's dq kernel: 4 | 8 waves, 32 rows each; 20 | 24: 4 | 8 waves, pairs share 32 rows
   SPA_KNOB_BWD_DKDV_FORM = 3, // dk/dv kernel: 1 compiler-scheduled MFMAs at D = 128 (test twin), 2 | 3: 64 | 128 keys a workgroup, 4 | 5: their twins

@@ -1,0 +1,103 @@
+"""The 16-bit forward's form of 64 query rows by four wave groups (taken where a launch leaves CUs idle; forced here by spa_tune fwd_groups = 4): edges of
+its row tiles, of a step's 128 (D = 128) or 256 keys and of a group's share of them, rows staged through LDS and not, rows in shards, e4m3."""
+import pytest
+import torch
+
+from conftest import rand
+from oracle import attn_oracle as O
+import sp_aurora_amd as spa
+from sp_aurora_amd import _lib, ops
+from test_gpu_fp8kv import quantised
+from test_gpu_parity import DEV, check_lse, check_out
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 1), (63, 64), (64, 65), (65, 33), (100, 257), (128, 128), (129, 129), (200, 511), (257, 300), (320, 513)]
+
+
+@pytest.fixture
+def four():
+    _lib.tune("fwd_groups", 4)
+    yield
+    _lib.tune("fwd_groups", 0)
+
+
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])  # (whole rows of q in a line: straight into the operands; the others through LDS)
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float16), (128, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("Sq,Sk", SIZES)
+def test_edges_against_the_oracle(four, layout, D, dtype, Sq, Sk):
+    B, H = 2, 3
+    q, k, v = (rand((B, s, H, D), 70 + Sk + i, dtype) for i, s in enumerate((Sq, Sk, Sk)))
+    place = (lambda t: t.transpose(1, 2).contiguous().to(DEV)) if layout == "bhsd" else (lambda t: t.to(DEV))
+    back = (lambda t: t.transpose(1, 2)) if layout == "bhsd" else (lambda t: t)
+    for causal in (False, True):
+        for scale in (None, -0.3):
+            want_o, want_l = O.full_attention(q, k, v, scale, causal)
+            out, lse = ops.flash_fwd(place(q), place(k), place(v), scale, causal, layout=layout, split_kv=1)
+            check_out(back(out), want_o, dtype, f"causal {causal} scale {scale}")
+            check_lse(lse, want_l)
+
+
+@pytest.mark.parametrize("q8", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Sq,Sk", SIZES[1:])
+def test_e4m3(four, D, q8, Sq, Sk):
+    if q8 and D == 64:
+        pytest.skip("8-bit scores: head dim 128")
+    B, H, dtype = 1, 3, torch.bfloat16
+    k8, ks, k = quantised((B, Sk, H, D), 90 + Sk, "bshd")
+    v8, vs, v = quantised((B, Sk, H, D), 91 + Sk, "bshd")
+    kw = {"k_scale": ks.to(DEV), "v_scale": vs.to(DEV)}
+    if q8:
+        q, qs, q_deq = quantised((B, Sq, H, D), 92 + Sk, "bshd")
+        kw["q_scale"] = qs.to(DEV)
+    else:
+        q = q_deq = rand((B, Sq, H, D), 92 + Sk, dtype)
+    for causal in (False, True):
+        want_o, want_l = O.full_attention(q_deq, k, v, None, causal)
+        out, lse = ops.flash_fwd(q.to(DEV), k8.to(DEV), v8.to(DEV), None, causal, split_kv=1, **kw)
+        check_out(out, want_o, dtype, f"causal {causal}")
+        check_lse(lse, want_l)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("P,half", [(2, 64), (4, 20), (3, 50)])  # (shards' halves of a sub-tile's rows and more, and of fewer)
+def test_rows_in_shards(four, D, P, half):
+    dtype, shape = torch.bfloat16, (1, 2 * P * half, 3, D)
+    q, k, v = (rand(shape, 110 + i, dtype) for i in range(3))
+    idx = O.zigzag_order(shape[1], P)
+    want_o, want_l = O.full_attention(q, k, v, None, True)
+    out, lse, _ = spa.sp_aurora_func(*(t[:, idx].contiguous().to(DEV) for t in (q, k, v)), causal=True, ring_size=P, sharding="zigzag", return_attn_probs=True)
+    got_o, got_l = torch.empty_like(out.cpu()), torch.empty_like(lse.cpu())
+    got_o[:, idx], got_l[:, :, idx] = out.cpu(), lse.cpu()
+    check_out(got_o, want_o, dtype)
+    check_lse(got_l, want_l)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bad", [65, 130, 200])
+def test_an_infinite_value_stays_behind_its_tile(four, D, bad):
+    """Causal: the rows of earlier tiles of 64 do not meet it, also where a step on the diagonal reaches further."""
+    q, k, v = (rand((1, 256, 2, D), 130 + i, torch.bfloat16) for i in range(3))
+    want_o, want_l = O.full_attention(q, k, v, None, True)
+    v[0, bad] = float("inf")
+    out, lse = ops.flash_fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, True)
+    before = bad // 64 * 64
+    check_out(out[:, :before], want_o[:, :before], torch.bfloat16)
+    check_lse(lse, want_l)
+    assert not torch.isfinite(out[:, bad]).any()
+
+
+@pytest.mark.parametrize("H,S", [(8, 700), (5, 1300)])
+def test_the_form_is_taken_for_small_launches(H, S):
+    """Bits tell the forms apart: the library's choice is this one."""
+    q, k, v = (rand((1, S, H, 128), 140 + i, torch.bfloat16).to(DEV) for i in range(3))
+    own = ops.flash_fwd(q, k, v, None, True)
+    got = {}
+    for groups in (2, 4):
+        _lib.tune("fwd_groups", groups)
+        try:
+            got[groups] = ops.flash_fwd(q, k, v, None, True)
+        finally:
+            _lib.tune("fwd_groups", 0)
+    assert torch.equal(own[0], got[4][0]) and not torch.equal(own[0], got[2][0])
