@@ -1279,7 +1279,7 @@ float form_us(const FwdParams& p, FwdForm f, int D, FwdKind kind) {
       {{0.98f, 0.96f, 5.1f, 2.0f}, {1.36f, 1.81f, 6.2f, 2.2f}, {1.24f, 1.67f, 8.9f, 0.5f}, {0.98f, 1.00f, 5.5f, 2.6f}},    // 16 bits, D = 128
       {{0.79f, 0.56f, 4.9f, 0.4f}, {1.03f, 1.18f, 4.1f, 2.2f}, {1.04f, 1.17f, 5.1f, 1.8f}, {1.25f, 1.25f, 5.0f, 1.45f}},    // 16 bits, D <= 64
       {{1.39f, 0.96f, 5.3f, 0.4f}, {1.68f, 1.91f, 6.0f, 2.7f}, {1.40f, 1.73f, 7.9f, 1.3f}, {1.31f, 1.32f, 5.6f, 3.0f}},    // e4m3 K/V
-      {{1.11f, 0.75f, 4.6f, 0.4f}, {1.40f, 1.53f, 5.0f, 2.6f}, {1.16f, 1.38f, 6.6f, 1.4f}, {1.09f, 1.05f, 5.0f, 2.4f}}};   // e4m3 q, K/V
+      {{1.11f, 0.75f, 4.6f, 0.4f}, {1.40f, 1.53f, 5.0f, 2.6f}, {1.16f, 1.38f, 6.6f, 1.4f}, {1.09f, 1.05f, 5.9f, 1.5f}}};   // e4m3 q, K/V
   const FormCost& c = cost[kind == KIND_QK8 ? 3 : kind == KIND_KV8 ? 2 : D > 64 ? 0 : 1][f];
   const float rows = f == FWD_SHARE ? 2 * FWD_BM : f == FWD_FOUR ? 64 : FWD_BM;                                  // of a workgroup
   const float keys = f == FWD_SPLIT ? 128.f : f == FWD_FOUR ? (D > 64 ? 4.f * fwd_bn<128, 4>() : 4.f * fwd_bn<64, 4>()) : 64.f;  // of a step
@@ -1301,6 +1301,20 @@ float form_us(const FwdParams& p, FwdForm f, int D, FwdKind kind) {
   const float n = (float)p.B * (float)p.H * tiles;
   // (equal workgroups end together: half of a last round that is not full is lost)
   const float load = p.causal || p.cu_q ? n / cus : 0.5f * (n / cus + ceilf(n / cus));
+  if (f == FWD_FOUR && n > cus) {
+    // One workgroup to a CU, whose start and end nothing covers.  Not causal: whole rounds of them.  Causal, the long ones first: the second round begins where
+    // the shortest of the first ends, and what is left over behind whole rounds, which end together, adds one of its own.
+    const float pairs = (float)p.B * (float)p.H, own = rows / keys;  // steps from one tile to the next
+    if (!p.causal) return ceilf(n / cus) * (mean * c.busy + c.round) + c.fixed;
+    auto steps = [&](float i) { return fminf(longest, (tiles - floorf(i / pairs)) * own); };  // of workgroup i of the launch
+    const float rounds = floorf(n / cus), work = n / cus * (mean * c.busy + c.round);
+    float last = work;
+    if (rounds == 1.f)
+      last = 2.f * c.round + (steps(cus - 1.f) + steps(cus)) * c.busy;
+    else if (rounds * cus < n)
+      last = rounds * (c.round + (longest - (rounds * cus / pairs - 1.f) * 0.5f * own) * c.busy) + c.round + steps(rounds * cus) * c.busy;
+    return fmaxf(longest * c.alone + c.round, fmaxf(work, last)) + c.fixed;
+  }
   return fmaxf(longest * c.alone, load * mean * c.busy) + c.round * fmaxf(1.f, n / slots) + c.fixed;
 }
 
