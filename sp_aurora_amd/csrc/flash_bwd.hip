@@ -1750,6 +1750,15 @@ double launch_time(const BwdParams& p, bool queries, int rows, double start, dou
   return chain > work ? chain : work;
 }
 
+// D = 64: workgroups of 64 rows, or keys, up to which they are the faster ones.  Two run on a CU: all at once up to two a CU, and beyond that, causal, while
+// the chains are long beside a workgroup's start and end (`rounds` - `start` / tiles, of workgroups of 128): the longest of the others decides, whose CU another
+// one shares.  Backward, causal, us, 128 / 64 rows (dq), and 128 / 64 keys: 12 heads of 2811 rows 91.9 / 78.7, / 79.1; 8 of 4763 147.4 / 127.7, / 128.0; 16 of 2501
+// 87.7 / 76.1, / 75.4; 4 x 16 of 674 33.6 / 35.1, / 38.2.  Of 1900 launches of 250 to 8000 rows, a quarter of them not causal, none got slower by it.
+double most_64(const BwdParams& p, double rounds, double start) {
+  const double of_128 = p.causal && !p.cu_q ? rounds - start / ((p.Sq + BWD_ROWS - 1) / BWD_ROWS) : 1.0;
+  return 2.0 * spa_device_cus() * (of_128 > 1.0 ? of_128 : 1.0);
+}
+
 // The forms of the dq kernel, D = 128: 256 rows a workgroup (8 waves, two a SIMD, the K/V stream shared by twice the rows) where there are many;
 // with fewer, 128 rows, or 64 (4 waves), whose waves share out the keys of a tile: more workgroups, each with a shorter chain.  Causal,
 // us, 256 / 128 / 64 rows: 8 heads of 2048 rows 61.4 / 37.8 / 29.5, 4096 119 / 76.8 / 63.8, 8192 263 / 187 / 227; 16 of 4096 138 / 101 / 125; 32 of 512
@@ -1757,7 +1766,7 @@ double launch_time(const BwdParams& p, bool queries, int rows, double start, dou
 // 128 rows on 4 waves that do not share, one a SIMD, where sequences are short (and for tensors of 2 GiB and more per (batch, head)): it starts the
 // soonest.  Causal, us, 256 / 128 / 64 / 128 rows on 4 waves, 16 heads: 2000 sequences of 16 rows 988 / 1042 / 841 / 829, 1000 of 64 552 / 580 / 505 / 465, 500 of
 // 128 376 / 381 / 514 / 367, 400 of 160 377 / 558 / 611 / 504, 200 of 320 424 / 491 / 587 / 460; 8 of 192 13.7 / 13.2 / 16.7 / 12.2, 8 of 128 10.8 / 10.4 / 9.2 / 10.4.
-// D = 64: 128 rows, two workgroups to a CU, or 64 rows where those are two to a CU at most: 8 heads of 2048 rows 29.4 / 19.9, 4096 56.0 / 39.1, 8192
+// D = 64: 128 rows, two workgroups to a CU, or 64 rows (most_64): 8 heads of 2048 rows 29.4 / 19.9, 4096 56.0 / 39.1, 8192
 // 128 / 119; 16 of 2048 30.0 / 21.6; 32 of 1024 18.7 / 14.3, 2048 36.9 / 36.9; 128 of 512 16.8 / 19.4.
 enum DqForm { DQ_128_PLAIN = 4, DQ_256 = 8, DQ_64 = 20, DQ_128 = 24 };  // the values of SPA_TUNE_BWD_DQ_WAVES
 template <int D, int ADDR>
@@ -1768,7 +1777,7 @@ int dq_form(const BwdParams& p) {
   if (forced) return DQ_128_PLAIN;
   if (D == 64) {
     const double wgs = p.cu_q ? (double)p.H * ((double)p.lse_bh / 64 + p.B) : (double)p.B * p.H * ((p.Sq + 63) / 64);
-    return wgs <= 2.0 * spa_device_cus() ? DQ_64 : DQ_128_PLAIN;
+    return wgs <= most_64(p, 2.25, 14.0) ? DQ_64 : DQ_128_PLAIN;
   }
   const double t256 = launch_time(p, true, 256, 6.0, 7.0, 1.76), t128 = launch_time(p, true, 128, 8.0, 8.4, 0.92);
   const double t64 = launch_time(p, true, 64, 7.5, 7.5, 0.69), plain = launch_time(p, true, 128, 5.5, 6.6, 1.2);
@@ -1786,7 +1795,7 @@ bool keys_64(const BwdParams& p) {
   if (form > 1) return form == 2;
   if (D == 64) {
     const double wgs = p.cu_q ? (double)p.H * ((double)p.total_k / 64 + p.B) : (double)p.B * p.H * ((p.Sk + 63) / 64);
-    return wgs <= (p.causal ? 2.0 : 1.0) * spa_device_cus();
+    return wgs <= (p.causal ? most_64(p, 2.1, 15.0) : 1.0 * spa_device_cus());
   }
   return launch_time(p, false, 64, 6.5, 6.5, 0.975) < launch_time(p, false, 128, 4.7, 4.7, 1.48);
 }
