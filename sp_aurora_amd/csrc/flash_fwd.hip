@@ -1324,7 +1324,7 @@ FwdForm fwd_form(const FwdParams& p, int D, FwdKind kind) {
   const bool can_share = D >= 64 && p.epi != SPA_EPI_FINALN;
   if (force ? force == 1 : p.Sk <= fwd_bn<128>()) return FWD_ONE;  // one sub-tile: nothing to split
   // (e4m3 K/V of 64 elements have the constants of 128: only where those say the same as the clock, in one round of workgroups)
-  const bool can_four = D >= 64 && !p.cu_q && p.P == 1 && !p.zigzag && p.epi == SPA_EPI_PLAIN &&
+  const bool can_four = !p.cu_q && p.P == 1 && !p.zigzag && p.epi == SPA_EPI_PLAIN &&
                         (kind != KIND_KV8 || D > 64 || (int64_t)p.B * p.H * fwd_tiles(p, 64) <= spa_device_cus());
   if (force == 4 && can_four) return FWD_FOUR;
   if (force_share && can_share) return force_share == 2 ? FWD_SHARE : FWD_SPLIT;
@@ -1360,7 +1360,7 @@ hipError_t launch16(FwdParams p, hipStream_t stream) {
       p.nqt = fwd_tiles(p, 2 * FWD_BM);
       return launch<flash_fwd16_kernel<T, D, 2, true, KV8, false, ZZ, false, QK8>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, true>::SMEM, 2 * FWD_BM, p, stream);
     }
-  if constexpr (D >= 64 && !ZZ)
+  if constexpr (!ZZ)
     if (form == FWD_FOUR) {
       constexpr int rows = Fwd16Cfg<D, 4, false>::GROUP_ROWS;
       p.nqt = fwd_tiles(p, rows);
@@ -1389,12 +1389,11 @@ hipError_t launch16_map(FwdParams p, hipStream_t stream) {
       p.nqt = fwd_tiles(p, 2 * FWD_BM);
       return launch<flash_fwd16_kernel<T, D, 2, true, N, N, N, N, N, N, N, N, true>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, true>::SMEM, 2 * FWD_BM, p, stream);
     }
-  if constexpr (D >= 64)
-    if (form == FWD_FOUR) {
-      constexpr int rows = Fwd16Cfg<D, 4, false>::GROUP_ROWS;
-      p.nqt = fwd_tiles(p, rows);
-      return launch<flash_fwd16_kernel<T, D, 4, false, N, N, N, N, N, N, N, N, true, D == 128>>(2 * FWD_THREADS, Fwd16Cfg<D, 4, false>::SMEM, rows, p, stream);
-    }
+  if (form == FWD_FOUR) {
+    constexpr int rows = Fwd16Cfg<D, 4, false>::GROUP_ROWS;
+    p.nqt = fwd_tiles(p, rows);
+    return launch<flash_fwd16_kernel<T, D, 4, false, N, N, N, N, N, N, N, N, true, D == 128>>(2 * FWD_THREADS, Fwd16Cfg<D, 4, false>::SMEM, rows, p, stream);
+  }
   if (form == FWD_SPLIT)
     return launch<flash_fwd16_kernel<T, D, 2, false, N, N, N, N, N, N, N, N, true, D == 128>>(2 * FWD_THREADS, Fwd16Cfg<D, 2, false>::SMEM, FWD_BM, p, stream);
   return launch<flash_fwd16_kernel<T, D, 1, false, N, N, N, N, N, N, N, N, true>>(FWD_THREADS, Fwd16Cfg<D, 1, false>::SMEM_PLAIN, FWD_BM, p, stream);

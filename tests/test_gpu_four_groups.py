@@ -23,7 +23,7 @@ def four():
 
 
 @pytest.mark.parametrize("layout", ["bhsd", "bshd"])  # (whole rows of q in a line: straight into the operands; the others through LDS)
-@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float16), (128, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("D,dtype", [(32, torch.bfloat16), (64, torch.bfloat16), (64, torch.float16), (128, torch.float16), (128, torch.bfloat16)])
 @pytest.mark.parametrize("Sq,Sk", SIZES)
 def test_edges_against_the_oracle(four, layout, D, dtype, Sq, Sk):
     B, H = 2, 3
@@ -60,7 +60,7 @@ def test_e4m3(four, D, q8, Sq, Sk):
         check_lse(lse, want_l)
 
 
-@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("P,half", [(2, 64), (4, 20), (3, 50)])  # (shards' halves of a sub-tile's rows and more, and of fewer)
 def test_rows_in_shards(four, D, P, half):
     dtype, shape = torch.bfloat16, (1, 2 * P * half, 3, D)
