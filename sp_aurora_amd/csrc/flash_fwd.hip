@@ -63,7 +63,7 @@ struct Fwd16Cfg {
   static constexpr int TILEB = BN * ROWB;      // one K or V sub-tile
   static constexpr int GROUP = 4 * TILEB;      // one set of K[2] and V[2] buffers
   static constexpr int BMW = SHARE ? NG * FWD_BM : GROUP_ROWS;  // query rows per workgroup
-  static constexpr int EPI = NG == 4 ? 3 * GROUP_ROWS * (D + 6) * 4 : (NG * FWD_BM * (D + 4) + NG * FWD_BM * 2 + BMW) * 4;  // epilogue staging
+  static constexpr int EPI = NG == 4 ? 4 * GROUP_ROWS * (D + 6) * 4 : (NG * FWD_BM * (D + 4) + NG * FWD_BM * 2 + BMW) * 4;  // epilogue staging
   static constexpr int TILES = SHARE ? GROUP : NG * GROUP;
   static constexpr int SMEM = TILES > EPI ? TILES : EPI;
   static constexpr int SMEM_PLAIN = NG == 1 ? TILES : SMEM;  // one group writes a plain result from its registers
@@ -980,7 +980,7 @@ __global__ void __launch_bounds__((Fwd16Cfg<D, NG, SHARE>::GROUP_THREADS * NG), 
   // next 4; one v_permlane32_swap per dword pairs them up so that every lane stores 16-byte pieces, the two
   // lanes of a row side by side.  `other`: the same rows' partial sums of the other wave group, staged in LDS
   // in the accumulator's own layout (128 rows of D + 4 floats), or null.
-  auto store_rows = [&](float a_own, auto with_other, const float* other, const float* a_other, float lse_val) {
+  auto store_rows = [&](float a_own, auto with_other, const float* other, float a_other, float lse_val) {
     constexpr bool OTHER = decltype(with_other)::value;
     if (hh == 0 && qrow < q_lim) lse_bh[MAP ? map.at(qrow, p.map.lse_pitch) : qrow] = lse_val;
     T* const orow = out_bh + qrow_t * out_rs;
@@ -992,16 +992,12 @@ __global__ void __launch_bounds__((Fwd16Cfg<D, NG, SHARE>::GROUP_THREADS * NG), 
 #pragma unroll
         for (int i = 0; i < 8; ++i) e[i] = o[db][8 * gp + i] * a_own;
         if constexpr (OTHER) {
+          const f32x4 p0 = *(const f32x4*)(other + db * 32 + 8 * (2 * gp) + 4 * hh);
+          const f32x4 p1 = *(const f32x4*)(other + db * 32 + 8 * (2 * gp + 1) + 4 * hh);
 #pragma unroll
-          for (int g = 0; g < NG - 1; ++g) {
-            const float* const rows = other + g * (C::GROUP_ROWS * (D + 4)) + db * 32 + 4 * hh;
-            const f32x4 p0 = *(const f32x4*)(rows + 8 * (2 * gp));
-            const f32x4 p1 = *(const f32x4*)(rows + 8 * (2 * gp + 1));
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              e[i] = __builtin_fmaf(p0[i], a_other[g], e[i]);
-              e[4 + i] = __builtin_fmaf(p1[i], a_other[g], e[4 + i]);
-            }
+          for (int i = 0; i < 4; ++i) {
+            e[i] = __builtin_fmaf(p0[i], a_other, e[i]);
+            e[4 + i] = __builtin_fmaf(p1[i], a_other, e[4 + i]);
           }
         }
         unsigned x[2], y[2];  // as two packed pairs each
@@ -1023,20 +1019,67 @@ __global__ void __launch_bounds__((Fwd16Cfg<D, NG, SHARE>::GROUP_THREADS * NG), 
   if constexpr (SHARE || (NG == 1 && !FINALN)) {
     // a wave's rows are complete: no LDS round trip, no barrier
     const float l_tot = halves_sum(l_run);
-    store_rows(vsc / l_tot, std::false_type{}, nullptr, nullptr, (m_run * c + fast_log2(l_tot)) * 0.6931471805599453f);
+    store_rows(vsc / l_tot, std::false_type{}, nullptr, 0.f, (m_run * c + fast_log2(l_tot)) * 0.6931471805599453f);
+    return;
+  } else if constexpr (NG == 4) {
+    // All groups stage their unscaled partial O (fp32) and (m, l) in LDS, free now; then the threads walk the rows, eight head dims of a row each, weigh the four
+    // by exp2((m - m_all) c) / l_all and store whole rows.  (Against the first group's two waves adding up and storing what the others stage, us: causal
+    // [1,926,16,128] 14.0 -> 13.4, [1,512,8,128] 9.6 -> 9.3, [1,256,8,64] 6.8 -> 6.5.  Two groups, whose stores four waves share as it is, lose 1 to 3 % with it.)
+    constexpr int TP = D + 4, CH = D / 8, GR = C::GROUP_ROWS;  // floats per staged row; pieces of a row
+    float* const tile = (float*)smem;
+    float* const ml = tile + NG * (GR * TP);
+    const int at = grp * GR + w * 32 + ln;
+    const float l_own = halves_sum(l_run);
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *(f32x4*)(tile + at * TP + db * 32 + 8 * g + 4 * hh) = f32x4{o[db][4 * g + 0], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
+    if (hh == 0) {
+      ml[at * 2] = m_run;
+      ml[at * 2 + 1] = l_own;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < (GR * CH + GT * NG - 1) / (GT * NG); ++i) {
+      const int idx = i * (GT * NG) + tid, r = idx / CH, ch = idx % CH, row = q0 + r;
+      if (r >= GR || row >= q_lim) break;
+      float m[NG], m_all = -INFINITY, l_all = 0.f;  // (finite in the end: some group has seen key 0)
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        m[g] = ml[(g * GR + r) * 2];
+        m_all = fmaxf(m_all, m[g]);
+      }
+      float e[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const float a = fast_exp2((m[g] - m_all) * c);
+        l_all = __builtin_fmaf(ml[(g * GR + r) * 2 + 1], a, l_all);
+        const f32x4 p0 = *(const f32x4*)(tile + (g * GR + r) * TP + ch * 8), p1 = *(const f32x4*)(tile + (g * GR + r) * TP + ch * 8 + 4);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          e[k] = __builtin_fmaf(p0[k], a, e[k]);
+          e[4 + k] = __builtin_fmaf(p1[k], a, e[4 + k]);
+        }
+      }
+      const float sc = vsc / l_all;
+      u32x4 st;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) st[k] = M::pack2(e[2 * k] * sc, e[2 * k + 1] * sc);
+      *(u32x4*)(out_bh + (int64_t)(MAP ? map.at(row, p.map.pitch) : row) * out_rs + ch * 8) = st;
+      if (ch == 0) lse_bh[MAP ? map.at(row, p.map.lse_pitch) : row] = (m_all * c + fast_log2(l_all)) * 0.6931471805599453f;
+    }
     return;
   } else if constexpr (!FINALN) {
-    // The groups hold partial sums of the same rows.  All but the first stage their unscaled partial O (fp32, its own
-    // register layout) and (m, l) in LDS, free now, and leave; group 0 weighs all by exp2((m - m_all) c) / l_all
-    // and stores the rows from its registers.  One barrier.
+    // Two groups hold partial sums of the same rows.  Group 1 stages its unscaled partial O (fp32, its own
+    // register layout) and (m, l) in LDS, free now, and leaves; group 0 weighs both by exp2((m - m_all) c) / l_all
+    // and stores the rows from its registers.  One barrier, one staged tile.
     constexpr int TP = D + 4;  // floats per staged row
-    constexpr int GR = C::GROUP_ROWS;
     float* const tile = (float*)smem;
-    float* const ml = tile + (NG - 1) * (GR * TP);  // (m, l) of the rows of groups 1 ..
+    float* const ml = tile + FWD_BM * TP;  // [128](m, l) of group 1
     const int rloc = w * 32 + ln;
     const float l_own = halves_sum(l_run);
-    if (grp > 0) {
-      const int at = (grp - 1) * GR + rloc;
+    if (grp == 1) {
 #pragma unroll
       for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -1046,29 +1089,22 @@ __global__ void __launch_bounds__((Fwd16Cfg<D, NG, SHARE>::GROUP_THREADS * NG), 
           st[1] = o[db][4 * g + 1];
           st[2] = o[db][4 * g + 2];
           st[3] = o[db][4 * g + 3];
-          *(f32x4*)(tile + at * TP + db * 32 + 8 * g + 4 * hh) = st;
+          *(f32x4*)(tile + rloc * TP + db * 32 + 8 * g + 4 * hh) = st;
         }
       if (hh == 0) {
-        ml[at * 2] = m_run;
-        ml[at * 2 + 1] = l_own;
+        ml[rloc * 2] = m_run;
+        ml[rloc * 2 + 1] = l_own;
       }
     }
     __syncthreads();
-    if (grp > 0) return;
-    float a[NG], m_all = m_run;  // finite in the end: some group has seen key 0 of the first chunk
-#pragma unroll
-    for (int g = 1; g < NG; ++g) m_all = fmaxf(m_all, ml[((g - 1) * GR + rloc) * 2]);
-    a[0] = fast_exp2((m_run - m_all) * c);
-    float l_all = l_own * a[0];
-#pragma unroll
-    for (int g = 1; g < NG; ++g) {
-      a[g] = fast_exp2((ml[((g - 1) * GR + rloc) * 2] - m_all) * c);
-      l_all += ml[((g - 1) * GR + rloc) * 2 + 1] * a[g];
-    }
+    if (grp == 1) return;
+    const float m2 = ml[rloc * 2], l2 = ml[rloc * 2 + 1];
+    const float m_all = fmaxf(m_run, m2);  // finite: some group has seen key 0 of the first chunk
+    const float a1 = fast_exp2((m_run - m_all) * c);
+    const float a2 = fast_exp2((m2 - m_all) * c);
+    const float l_all = l_own * a1 + l2 * a2;
     const float sc = vsc / l_all;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) a[g] *= sc;
-    store_rows(a[0], std::true_type{}, tile + rloc * TP, a + 1, (m_all * c + fast_log2(l_all)) * 0.6931471805599453f);
+    store_rows(a1 * sc, std::true_type{}, tile + rloc * TP, a2 * sc, (m_all * c + fast_log2(l_all)) * 0.6931471805599453f);
     return;
   } else {
     constexpr int TP = D + 4;  // floats per staged row
