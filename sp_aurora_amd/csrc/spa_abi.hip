@@ -1069,13 +1069,26 @@ int64_t spa_flash_fwd_varlen_splitkv_workspace_bytes(int nseq, int H, int total_
 // are 1 to 4 % slower), or, at D = 128, of 512 while those are 16 thousand workgroups of one head or fewer and the last of them count (1024 / 512,
 // us, longest of 4096: 64, H = 32, e4m3 232 / 224, bf16 438 / 438; of 8192: 8, H = 32, 63.5 / 59.5 and 130 / 125, 32, H = 8, 74.7 /
 // 65.4 and 125 / 122, but 64, H = 32, 483 / 487 and 808 / 812).
+// One row: 256 keys while those are 4 (D = 64: 8) thousand chunks of one head or fewer, and where single caches would have more than 1024 for each CU: a workgroup
+// more or less on a CU, and the last ones, cost less.  Of 950 random batches (8 to 64 caches of 512 to 8192 tokens) the choice is 2.7 % faster than
+// the one before, 1.42x at most (8 caches of up to 7966, H = 8, D = 64, bf16), none more than 2.5 % slower.  Two or three rows, with as many
+// sums to merge: up to 5 and 16 % slower with it.
 int spa_flash_fwd_varlen_splitkv_suggest(int nseq, int H, int total_k, int max_sq, int max_sk, int D, int dtype) {
   if (nseq <= 0 || H <= 0 || total_k <= 0 || max_sq <= 0 || max_sq > kFewRows || max_sk <= 0 || (D != 64 && D != 128) ||
       (dtype != SPA_BF16 && dtype != SPA_F16) || spa_knob(SPA_KNOB_FEW_ROWS) == 1)
     return 0;
   const int64_t cus = spa_device_cus();
-  if ((int64_t)nseq * H >= cus) return max_sk <= 2200 ? 0 : D == 128 && (int64_t)total_k * H <= 512 * 64 * cus ? 512 : 1024;
-  const int64_t even = (int64_t)total_k * H / cus, chunk = even <= 256 ? 256 : (even + 255) / 256 * 256;
+  const int64_t even = (int64_t)total_k * H / cus;  // keys of all heads for each CU
+  const bool one = max_sq == 1;
+  if ((int64_t)nseq * H >= cus) {
+    if (max_sk <= 2200) return 0;
+    if (one) {
+      if (D == 64) return even <= 32 * 512 ? 256 : 512;
+      if (even <= 16 * 512 && max_sk > 2400) return 256;
+    }
+    return D == 128 && even <= 64 * 512 ? 512 : 1024;
+  }
+  const int64_t chunk = even <= 256 || (one && even > 1024) ? 256 : (even + 255) / 256 * 256;
   return max_sk >= chunk * 3 / 2 ? (int)chunk : 0;
 }
 

@@ -202,3 +202,24 @@ def test_one_long_cache_beside_short_ones(H, fp8):
     want = reference(q, k, v, cu_q, cu_k, 1, 20000, **scales)
     check_exact(want, exact(q, k, v, cu_q, cu_k, **scales), torch.bfloat16)
     check(ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 1, 20000, **scales), want, torch.bfloat16)
+
+
+@pytest.mark.parametrize("D,dtype,fp8", [(64, torch.float16, False), (64, torch.bfloat16, True), (128, torch.bfloat16, False), (128, torch.bfloat16, True)])
+@pytest.mark.parametrize("H,count,longest", [(8, 9, 9000), (32, 12, 2500)])  # (fewer workgroups than CUs, and more)
+def test_one_row_in_chunks_of_the_librarys_choice(H, count, longest, D, dtype, fp8):
+    lens = [(1 + (i * 1997) % longest, 1) for i in range(count - 1)] + [(longest, 1)]
+    q, k, v, cu_q, cu_k, scales = caches(lens, H, D, dtype, fp8, 1500 + H + count)
+    assert _lib.load().spa_flash_fwd_varlen_splitkv_suggest(count, H, k.shape[0], 1, longest, D, _lib.SPA_BF16 if dtype == torch.bfloat16 else _lib.SPA_F16) == 256
+    want = reference(q, k, v, cu_q, cu_k, 1, longest, **scales)
+    check_exact(want, exact(q, k, v, cu_q, cu_k, **scales), dtype)
+    check(ops.flash_fwd_varlen(q, k, v, cu_q, cu_k, 1, longest, **scales), want, dtype)
+
+
+@pytest.mark.parametrize("dtype,fp8", [(torch.float16, False), (torch.bfloat16, True)])
+def test_one_row_of_many_heads_together(dtype, fp8):
+    """Six workgroups and more per CU with 512 bytes of heads each and eight loads in flight."""
+    lens = [(1 + (i * 37) % 330, 1) for i in range(60)] + [(0, 1), (344, 1)]
+    q, k, v, cu_q, cu_k, scales = caches(lens, 32, 128, dtype, fp8, 1600)
+    want = reference(q, k, v, cu_q, cu_k, 1, 344, **scales)
+    check_exact(want, exact(q, k, v, cu_q, cu_k, **scales), dtype)
+    check(split(q, k, v, cu_q, cu_k, 1, 344, 16, **scales), want, dtype)
