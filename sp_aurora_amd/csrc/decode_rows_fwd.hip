@@ -308,8 +308,8 @@ hipError_t launch_variant(const FwdParams& p, hipStream_t stream) {
 
 // K and V up to this many bytes stay in the memory-side cache (256 MiB) from one call to the next where a program's other data leave them there; larger ones are
 // read past it.  Us a call, three sets of inputs in turn, plain / non-temporal: 16 x 8 heads of 698 keys, D = 128, e4m3 (23 MB) 8.1 / 10.1, bf16 (46) 10.8 /
-// 14.5; 32 of 4096, bf16 (67) 15.4 / 16.2; 16 x 32 of 512, bf16 (134) 26.5 / 24.0; 16 x 32 of 4000, e4m3 (524) 91.8 / 83.8.
-constexpr int64_t kCachedBytes = (int64_t)96 << 20;
+// 14.5; 32 of 4096, bf16 (67) 15.4 / 16.2; six sets, 32 of 5000, bf16 (82) 20.2 / 18.7; 16 x 32 of 512, bf16 (134) 26.5 / 24.0; 16 x 32 of 4000, e4m3 (524) 91.8 / 83.8.
+constexpr int64_t kCachedBytes = (int64_t)64 << 20;
 int64_t kv_bytes(const FwdParams& p, int D) {
   const int64_t keys = (int64_t)(p.P - 1) * p.Sk + p.sk_last;
   return (int64_t)p.B * p.H * keys * D * (p.k_scale ? 2 : 4);
@@ -335,11 +335,12 @@ hipError_t launch(const FwdParams& p, hipStream_t stream) {
 // Whether this kernel is the faster one for a call of up to 16 rows (p as for the launch).  Us a call, before / here, 32 heads of 32768 keys and 16 x 32 heads of
 // 4000: rows back to back, one row, e4m3, D = 64 30.5 / 28.2, 50.8 / 45.5, D = 128 51.4 / 46.4, 81.5 / 84.8, bf16, D = 128 81.9 / 80.6, 155.9 / 155.2, three rows
 // 92.2 / 80.8; eight rows (before on flash_fwd.hip's kernels), e4m3, D = 64 52.8 / 26.2, 85.8 / 44.2, D = 128 79.5 / 45.8, 136 / 83.7, bf16 99.5 / 80.4, 183 / 155.
-// Not for one row, from memory, of 64 16-bit elements (45.1 / 45.8, 79.7 / 81.0) or of 128 e4m3 elements whose keys are not split.  Rows of other heads in between:
+// Not for one row, of 64 16-bit elements from memory (45.1 / 45.8, 79.7 / 81.0) or of few heads whose keys are not split (8 of 600 keys 6.1 / 7.0), or of 128 e4m3 elements whose keys are not split.  Rows of other heads in between:
 // up to three rows stay on decode_fwd.hip, which takes neighbouring heads together (its 225 us for 64 caches of 1 to 4 thousand e4m3 tokens were 303 here);
 // eight rows, e4m3, D = 128 72.7 / 61.9, 131 / 111, bf16 181 / 177, but 32 heads of 32768 91.4 / 93.3, and of 64 16-bit elements 57.8 / 60.0, 97.9 / 108.6.
 bool spa_rows16_takes(const FwdParams& p, int D) {
   const bool kv8 = p.k_scale != nullptr, memory = kv_bytes(p, D) > kCachedBytes;
+  if (p.Sq == 1 && !kv8 && D == 64 && p.P == 1 && (int64_t)p.B * p.H <= 16) return false;
   if (p.ks.s == D && p.vs.s == D) return !memory || p.Sq > 1 || (kv8 ? D == 64 || p.P > 1 : D == 128);
   return p.Sq > kRowsInFp32 && !(memory && !kv8 && (D == 64 || p.P > 1));
 }

@@ -264,13 +264,15 @@ int spa_flash_fwd_splitkv_suggest(int B, int H, int Sq, int Sk, int D, int mask_
     return 1;
   const int cus = spa_device_cus();
   // Up to kRows16 query rows run on the kernels that stream K and V: one workgroup per CU measured best on ten decode
-  // shapes (more chunks: 3 to 15 % slower), chunks of at least 64 KB of bf16 keys (512 keys of 128 instead of 256, us a call: [1, 8, 1 against 2048] 9.4
-  // and 8.5, 32 heads 10.9 and 9.1; for head dim 64 256 keys are no faster than 512).
+  // shapes (more chunks: 3 to 15 % slower), chunks of at least 256 keys (instead of 512, us, device: [1, 8, 1 against 2048], D = 128 9.4
+  // and 8.5, 32 heads 10.9 and 9.1, D = 64 against 1024 9.1 and 8.0, 32 heads 10.3 and 8.5).  From 1024 keys on, with four rows and more, whose kernel is faster
+  // by itself than two launches are sent off, from 2048, or, at D = 128 and few heads, 1280 (us, whole / split: 8 rows, 8 heads against 1926, bf16 21.2 / 10.7, e4m3
+  // 12.9 / 9.0; D = 64, e4m3 8.4 / 7.1).
   if (Sq <= kRows16 && spa_knob(SPA_KNOB_FEW_ROWS) != 1) {
-    if (Sk < (Sq <= kFewRows ? 1024 : 2048)) return 1;
+    if (Sk < (Sq <= kFewRows ? 1024 : D == 128 && (int64_t)B * H * 4 <= cus ? 1280 : 2048)) return 1;
     int64_t n = ((int64_t)cus + (int64_t)B * H / 2) / ((int64_t)B * H);
     // (not more than 16 of them below 512 keys: the second kernel takes 2.3 us for 8 or 16 chunks of 8 heads and 5 for 32)
-    const int64_t shortest = 32768 / D, by_length = Sk / shortest < 16 ? Sk / shortest : Sk / 512 > 16 ? Sk / 512 : 16;
+    const int64_t by_length = Sk / 256 < 16 ? Sk / 256 : Sk / 512 > 16 ? Sk / 512 : 16;
     if (n > by_length) n = by_length;
     if (n > 64) n = 64;
     return n < 2 ? 1 : KeySplit(Sk, (int)n).n;
