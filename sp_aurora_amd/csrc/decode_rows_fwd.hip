@@ -290,8 +290,13 @@ __global__ void __launch_bounds__(kWaves * 64) rows16_fwd_kernel(const FwdParams
     }
     const int64_t orow = (int64_t)z * p.Sq + i;
     const float inv = vmul / ls;
-    const u32x2 st = {M::pack2(a[0] * inv, a[1] * inv), M::pack2(a[2] * inv, a[3] * inv)};
-    *(u32x2*)((T*)p.out + b * p.os.b + h * p.os.h + orow * p.os.s + d) = st;
+    const int64_t at = b * p.os.b + h * p.os.h + orow * p.os.s + d;
+    if (p.out32) {
+      *(f32x4*)((float*)p.out + at) = a * inv;
+    } else {
+      const u32x2 st = {M::pack2(a[0] * inv, a[1] * inv), M::pack2(a[2] * inv, a[3] * inv)};
+      *(u32x2*)((T*)p.out + at) = st;
+    }
     if (d == 0) p.lse[(int64_t)bh * p.lse_bh + orow] = (mx + __builtin_amdgcn_logf(ls)) * 0.6931471805599453f;
   }
 }

@@ -1000,6 +1000,15 @@ __global__ void __launch_bounds__((Fwd16Cfg<D, NG, SHARE>::GROUP_THREADS * NG), 
             e[4 + i] = __builtin_fmaf(p1[i], a_other, e[4 + i]);
           }
         }
+        if constexpr (KS)
+          if (p.out32) {  // (few rows, against keys that lie as no kernel for few rows takes them)
+            if (qrow < q_lim) {
+              float* const row32 = (float*)p.out + b * p.os.b + h * p.os.h + qoff * p.os.s + qrow_t * out_rs + db * 32 + 16 * gp + 4 * hh;
+              *(f32x4*)row32 = f32x4{e[0], e[1], e[2], e[3]};
+              *(f32x4*)(row32 + 8) = f32x4{e[4], e[5], e[6], e[7]};
+            }
+            continue;
+          }
         unsigned x[2], y[2];  // as two packed pairs each
 #pragma unroll
         for (int k = 0; k < 2; ++k) {

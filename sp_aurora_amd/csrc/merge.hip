@@ -198,12 +198,12 @@ __global__ void __launch_bounds__(256) finalize_kernel(T* __restrict__ out, cons
     if (on[k]) Load8<T>::st(op[k], x[k]);
 }
 
-// Merge of the n block results a key-split forward left behind (rows j * Sq .. of `part`, [B, n * Sq, H, D] in T, and of
+// Merge of the n block results a key-split forward left behind (rows j * Sq .. of `part`, [B, n * Sq, H, D] in P, and of
 // part_lse, [B, H, n * Sq]): update_out_and_lse (sp_aurora/utils.py:103-104) over all of them at once, as a running
 // (weighted sum, weight sum) relative to the largest lse so far.  A chunk whose scores are all -inf (lse -inf, no result) has no weight.
 // Bound: the latency of its loads (a few rows, a few workgroups), so eight chunks are requested together.
-template <typename T>
-__global__ void __launch_bounds__(256) splitkv_combine_kernel(T* __restrict__ out, float* __restrict__ lse, const T* __restrict__ part,
+template <typename T, typename P>
+__global__ void __launch_bounds__(256) splitkv_combine_kernel(T* __restrict__ out, float* __restrict__ lse, const P* __restrict__ part,
                                                               const float* __restrict__ part_lse, int n, int H, int Sq, int D,
                                                               int cpr_shift, unsigned nrows, Strides3 os, int64_t lse_bh) {
   const unsigned gid = blockIdx.x * 256u + threadIdx.x;
@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(256) splitkv_combine_kernel(T* __restrict__ ou
   if (row >= nrows) return;
   const RowIdx r = decode_row(row, H);
   const int64_t prow = (int64_t)H * D;                                  // elements between rows of `part`
-  const T* pp = part + ((int64_t)r.b * n * Sq + r.s) * prow + r.h * D + ch * 8;
+  const P* pp = part + ((int64_t)r.b * n * Sq + r.s) * prow + r.h * D + ch * 8;
   const float* pl = part_lse + ((int64_t)r.b * H + r.h) * ((int64_t)n * Sq) + r.s;
   constexpr int NB = 8;
   float x[8], lb = -INFINITY, wsum = 0.f;
@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(256) splitkv_combine_kernel(T* __restrict__ ou
     for (int u = 0; u < NB; ++u) {
       const int j = j0 + u < n ? j0 + u : n - 1;
       l[u] = pl[(int64_t)j * Sq];
-      Load8<T>::ld(pp + (int64_t)j * Sq * prow, xb[u]);
+      Load8<P>::ld(pp + (int64_t)j * Sq * prow, xb[u]);
     }
     float mx = lb;
 #pragma unroll
@@ -352,17 +352,19 @@ hipError_t spa_launch_delta(const void* out, const void* dout, float* delta, int
   return hipGetLastError();
 }
 
+// part32: `part` is fp32, not of the element type.
 hipError_t spa_launch_splitkv_combine(void* out, float* lse, const void* part, const float* part_lse, int n, int B, int H, int Sq,
-                                      int D, Strides3 os, int64_t lse_bh, int dtype, hipStream_t stream) {
+                                      int D, Strides3 os, int64_t lse_bh, int dtype, bool part32, hipStream_t stream) {
   const RowGrid g = row_grid(B, H, Sq, D);
-  if (!g.ok || n < 1) return hipErrorInvalidValue;
-  if (dtype == 1)
-    hipLaunchKernelGGL((splitkv_combine_kernel<__bf16>), g.grid, dim3(256), 0, stream, (__bf16*)out, lse, (const __bf16*)part, part_lse, n, H,
-                       Sq, D, g.cpr_shift, g.nrows, os, lse_bh);
-  else if (dtype == 2)
-    hipLaunchKernelGGL((splitkv_combine_kernel<_Float16>), g.grid, dim3(256), 0, stream, (_Float16*)out, lse, (const _Float16*)part,
-                       part_lse, n, H, Sq, D, g.cpr_shift, g.nrows, os, lse_bh);
-  else
-    return hipErrorInvalidValue;
+  if (!g.ok || n < 1 || (dtype != 1 && dtype != 2)) return hipErrorInvalidValue;
+#define SPA_COMBINE(T, P)                                                                                                                              \
+  hipLaunchKernelGGL((splitkv_combine_kernel<T, P>), g.grid, dim3(256), 0, stream, (T*)out, lse, (const P*)part, part_lse, n, H, Sq, D, g.cpr_shift, \
+                     g.nrows, os, lse_bh)
+  if (dtype == 1) {
+    if (part32) SPA_COMBINE(__bf16, float); else SPA_COMBINE(__bf16, __bf16);
+  } else {
+    if (part32) SPA_COMBINE(_Float16, float); else SPA_COMBINE(_Float16, _Float16);
+  }
+#undef SPA_COMBINE
   return hipGetLastError();
 }

@@ -49,6 +49,7 @@ struct FwdParams {
   int part_slot;     // SPA_EPI_PART: the slot this step fills (the launcher points out / lse at it)
   int npart;         // SPA_EPI_FINALN: slots 0 .. npart-1 are merged, in that order, then this step's block
   int epi;
+  bool out32 = false;  // keys cut into chunks: out takes the chunks' results in fp32 instead of q's element type
   // variable-length batch (null: every sequence has Sq queries and Sk keys): sequence b owns rows
   // cu_q[b] .. cu_q[b+1] of q/out/lse and cu_k[b] .. cu_k[b+1] of k/v, batch strides are unused,
   // Sq and Sk are the longest sequence's sizes (they shape the grid) and lse is [H][lse_bh]

@@ -53,6 +53,35 @@ def test_key_split_matches_the_oracle_and_the_plain_call(B, H, Sq, Sk, D, dtype,
     assert torch.equal(o2.transpose(1, 2), out) and torch.equal(l2, lse)
 
 
+def _relative_error(out, want):
+    return ((out.cpu().double() - want).norm() / want.norm()).item()
+
+
+@pytest.mark.parametrize("e4m3", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+@pytest.mark.parametrize("H,Sq,Sk,D", [(8, 8, 1926, 128), (64, 4, 1300, 128), (34, 16, 3000, 64), (8, 5, 2500, 128)])
+def test_chunks_of_few_rows_add_no_error(H, Sq, Sk, D, layout, dtype, e4m3):
+    """The chunks' results of 4 to 16 rows wait in fp32: the library's own split is as near to float64 as the call in one piece.  (The mean over 1 / n
+    of the keys is sqrt(n) times as large and counts 1 / n, so n of them rounded to 16 bits add as much squared error as the result's own
+    rounding, 15 to 40 % of the error by what the weights' rounding adds; in fp32 2^-16 of that.  3 %: the norm over 1000 elements scatters by 1.)"""
+    from test_gpu_fp8kv import quantised
+    assert _lib.load().spa_flash_fwd_splitkv_suggest(1, H, Sq, Sk, D, 0, ops._DT[dtype]) > 1
+    q = rand((1, Sq, H, D), 1040, dtype)
+    if e4m3:
+        k, ks, k_deq = quantised((1, Sk, H, D), 1041, "bshd")
+        v, vs, v_deq = quantised((1, Sk, H, D), 1042, "bshd")
+        kw = dict(k_scale=ks, v_scale=vs)
+    else:
+        k, v = k_deq, v_deq = rand((1, Sk, H, D), 1041, dtype), rand((1, Sk, H, D), 1042, dtype)
+        kw = {}
+    want, _ = O.full_attention(q, k_deq, v_deq, None, False)
+    place = (lambda t: t.to(DEV)) if layout == "bshd" else (lambda t: t.transpose(1, 2).contiguous().to(DEV))
+    back = (lambda t: t) if layout == "bshd" else (lambda t: t.transpose(1, 2))
+    whole, cut = (_relative_error(back(ops.flash_fwd(place(q), place(k), place(v), layout=layout, split_kv=n, **kw)[0]), want) for n in (1, "auto"))
+    assert cut <= 1.03 * whole, f"split {cut:.3e}, whole {whole:.3e}"
+
+
 def test_key_split_with_e4m3_cache():
     B, H, Sq, Sk, D = 1, 8, 4, 6000, 128
     from test_gpu_fp8kv import quantised
