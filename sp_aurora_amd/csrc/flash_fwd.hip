@@ -1369,7 +1369,11 @@ FwdForm fwd_form(const FwdParams& p, int D, FwdKind kind) {
   const bool can_share = D >= 64 && p.epi != SPA_EPI_FINALN;
   if (force ? force == 1 : p.Sk <= fwd_bn<128>()) return FWD_ONE;  // one sub-tile: nothing to split
   // (e4m3 K/V of 64 elements have the constants of 128: only where those say the same as the clock, in one round of workgroups)
+  // (Nor where the 32-bit offsets of a last step's rows behind the last key come round to the tensor again, rows of 17 MB and more: what lies there would count for
+  // nothing, but an infinity in V times that is no number.  The other forms' steps are half as long, and end before.)
+  const int64_t step_keys = 4 * (D > 64 ? fwd_bn<128, 4>() : fwd_bn<64, 4>()), pitch = (p.ks.s > p.vs.s ? p.ks.s : p.vs.s) * (kind == KIND_16 ? 2 : 1);
   const bool can_four = !p.cu_q && p.P == 1 && !p.zigzag && p.epi == SPA_EPI_PLAIN &&
+                        (p.Sk + step_keys - 1) / step_keys * step_keys * pitch < ((int64_t)1 << 32) &&
                         (kind != KIND_KV8 || D > 64 || (int64_t)p.B * p.H * fwd_tiles(p, 64) <= spa_device_cus());
   if (force == 4 && can_four) return FWD_FOUR;
   if (force_share && can_share) return force_share == 2 ? FWD_SHARE : FWD_SPLIT;

@@ -88,6 +88,32 @@ def test_an_infinite_value_stays_behind_its_tile(four, D, bad):
     assert not torch.isfinite(out[:, bad]).any()
 
 
+@pytest.mark.parametrize("D,e4m3", [(32, False), (64, False), (64, True), (128, False)])
+@pytest.mark.parametrize("Sk", [65, 100, 127])
+def test_rows_far_apart(four, Sk, D, e4m3):
+    """Rows 17 MB apart, all that lies between them infinite: a step of 256 keys would reach rows whose 32-bit offsets come round to the tensor again."""
+    Sq, pitch = 70, 17 << 20
+    if (Sk - 1) * pitch >= 2 ** 31:
+        pitch = (2 ** 31 // (Sk - 1) - 1) // 256 * 256
+    q, k, v = (rand((1, s, 1, D), 150 + i, torch.bfloat16) for i, s in enumerate((Sq, Sk, Sk)))
+    kw, dtype, gap = {}, torch.bfloat16, float("inf")
+    k_in, v_in, k_deq, v_deq = k, v, k, v
+    if e4m3:
+        (k_in, ks, k_deq), (v_in, vs, v_deq) = quantised((1, Sk, 1, D), 151, "bshd"), quantised((1, Sk, 1, D), 152, "bshd")
+        kw, dtype, gap = dict(k_scale=ks.to(DEV), v_scale=vs.to(DEV)), torch.float8_e4m3fn, float("nan")
+
+    def far(t):
+        step = pitch // t.element_size()
+        wide = torch.full(((Sk - 1) * step + D,), gap, device=DEV, dtype=torch.bfloat16).to(dtype)
+        wide = wide.as_strided((1, Sk, 1, D), (0, step, D, 1))
+        wide.copy_(t)
+        return wide
+    want_o, want_l = O.full_attention(q, k_deq, v_deq, None, False)
+    out, lse = ops.flash_fwd(q.to(DEV), far(k_in), far(v_in), None, False, split_kv=1, **kw)
+    check_out(out, want_o, torch.bfloat16)
+    check_lse(lse, want_l)
+
+
 @pytest.mark.parametrize("H,S", [(8, 700), (5, 1300)])
 def test_the_form_is_taken_for_small_launches(H, S):
     """Bits tell the forms apart: the library's choice is this one."""
