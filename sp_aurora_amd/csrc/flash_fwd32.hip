@@ -638,7 +638,7 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
         for (int db = 0; db < DV / 32; ++db) vx[u][db][e] = v[db * 32];
       }
   };
-  constexpr int CH = DV > 32 ? 2 : 1, UH = DV > 64 ? 1 : 2;  // head-dim blocks and halves of a tile's keys at a time
+  constexpr int CH = DV == 64 ? 2 : 1;  // head-dim blocks at a time (of four only one, so that the registers hold both halves of a tile's keys)
   Rows<D, DV> rows;
   rows.start(p.scale_log2);
   // (a whole chunk of eight values a thread, or none)
@@ -699,28 +699,26 @@ __global__ void __launch_bounds__(64 * NW, 1) flash_fwd32_splitk_kernel(const Fw
     Split8 pf[2];
     rows.raise(s);
     rows.weights(s, pf);
-    // (the small terms of all of the tile's keys first, where the registers hold them: 5 to 8 % less rounding error)
+    // (the small terms of all of the tile's keys first: 5 to 8 % less rounding error)
 #pragma unroll
-    for (int u0 = 0; u0 < 2; u0 += UH)
+    for (int db = 0; db < DV / 32; db += CH) {
+      Split8 va[2][CH];
 #pragma unroll
-      for (int db = 0; db < DV / 32; db += CH) {
-        Split8 va[UH][CH];
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int u = 0; u < UH; ++u)
+        for (int x = 0; x < CH; ++x) va[u][x].set(vx[u][db + x]);
 #pragma unroll
-          for (int x = 0; x < CH; ++x) va[u][x].set(vx[u0 + u][db + x]);
+      for (int term = 0; term < 6; ++term)
 #pragma unroll
-        for (int term = 0; term < 6; ++term)
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
-          for (int u = 0; u < UH; ++u)
-#pragma unroll
-            for (int x = 0; x < CH; ++x) {
-              const Split8 &vs = va[u][x], &ps = pf[u0 + u];
-              const frag a = as_frag<frag>(term == 2 || term == 3 ? vs.m : term == 4 ? vs.l : vs.h);
-              const frag pb = as_frag<frag>(term == 0 ? ps.l : term == 1 || term == 2 ? ps.m : ps.h);
-              rows.o[db + x] = M::run(a, pb, rows.o[db + x]);
-            }
-      }
+          for (int x = 0; x < CH; ++x) {
+            const Split8 &vs = va[u][x], &ps = pf[u];
+            const frag a = as_frag<frag>(term == 2 || term == 3 ? vs.m : term == 4 ? vs.l : vs.h);
+            const frag pb = as_frag<frag>(term == 0 ? ps.l : term == 1 || term == 2 ? ps.m : ps.h);
+            rows.o[db + x] = M::run(a, pb, rows.o[db + x]);
+          }
+    }
     if (it + NW < nt) load_values(it + NW);
   }
   __syncthreads();  // (the same LDS again)

@@ -116,3 +116,19 @@ def test_workgroups_that_share_rows_of_shards(B, H, D):
         finally:
             _lib.tune("fwd32_split", 0)
         check_out(out.cpu(), want, torch.float32, sharding)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D,Sk", [(128, 256), (128, 300), (64, 300)])
+def test_workgroups_that_share_head_dims_sum_in_the_same_order(D, Sk, causal):
+    """8, 16 and 32 heads of 256 rows leave four, two and one workgroup for the head dims of a row (at D = 64 two at most): the small terms of a tile's
+    products come first in each, so the bits are the same however many there are."""
+    q, k, v = (torch.randn((1, 32, s, D), generator=torch.Generator().manual_seed(160 + i)).to(DEV) for i, s in enumerate((256, Sk, Sk)))
+    _lib.tune("fwd32_split", 2)
+    try:
+        whole, lse = ops.flash_fwd(q, k, v, None, causal, layout="bhsd")
+        for heads in (8, 16):
+            out, l = ops.flash_fwd(q[:, :heads], k[:, :heads], v[:, :heads], None, causal, layout="bhsd")
+            assert torch.equal(out, whole[:, :heads]) and torch.equal(l, lse[:, :heads]), f"{heads} heads"
+    finally:
+        _lib.tune("fwd32_split", 0)
