@@ -61,9 +61,11 @@ __device__ __forceinline__ Words<DW> load_words(__amdgpu_buffer_rsrc_t rs, unsig
   return r;
 }
 
-// The weights of up to three rows are as exact as in fp32: the sum of three terms of the element type, none above that of the largest score (so that
-// large values do not overflow under it).  bf16 terms have fp32's range; fp16's end at 2^-24, so there the largest weight is 2^15 and the finest
-// step 2^-39 of it.  More rows round their weights once, as the kernels for long rows do, and the reference may be 2^8 too low.
+// The weights of up to three rows are the sum of three terms of the element type, none above that of the largest score (so that large values do not overflow
+// under it).  bf16 terms have fp32's range and hold all 24 bits.  fp16's end at 2^-24, so there the largest weight is 2^15 and the terms beside the first, which
+// hold 2^-10 of it at most, are 2^11 times as large as what they stand for: 24 bits down to 2^-27 of the largest weight, steps of 2^-50 of it below.  A weight whose
+// first term would round to 0 has the smallest one there and the difference in the others, so that an infinity in V under it is one in the result.
+// More rows round their weights once, as the kernels for long rows do, and the reference may be 2^8 too low.
 constexpr int kRowsInFp32 = 3;
 constexpr int weight_terms(int rows) { return rows <= kRowsInFp32 ? 3 : 1; }
 template <typename T, int TERMS>
@@ -71,6 +73,10 @@ struct WeightRange {
   static constexpr bool half = std::is_same<T, _Float16>::value;
   static constexpr float slack = TERMS > 1 ? 0.f : 8.f;            // log2 of what a score may exceed the reference by
   static constexpr float up = !half ? 0.f : TERMS > 1 ? 15.f : 7.f;        // log2 of the weight of a score at the reference
+  static constexpr bool scaled = half && TERMS > 1;
+  static constexpr float later = scaled ? 0x1p11f : 1.f;                   // of the terms beside the first
+  // what the first term is rounded from: x, or the smallest fp16 number where 0 < x < that
+  static __device__ __forceinline__ float first(float x) { return scaled ? __builtin_amdgcn_fmed3f(x, x * 0x1p102f, 0x1p-24f) : x; }
 };
 
 template <int D, int kWaves>
@@ -84,16 +90,22 @@ struct DecodeCfg {
 template <typename T, int D, bool KV8, int TERMS, int kWaves, bool NT>
 __global__ void __launch_bounds__(kWaves * 64) rows16_fwd_kernel(const FwdParams p) {
   constexpr int AUX = NT ? 2 : 0;
+  // (e4m3 values are as exact in bf16: weights of several terms have fp32's range there, whatever the type of the queries)
+  typedef typename std::conditional<KV8 && (TERMS > 1), __bf16, T>::type PT;
+  typedef Mma16<PT> MP;
+  typedef Mma16x16<PT> MMP;
+  typedef typename MP::frag pfrag;
   typedef Mma16<T> M;
   typedef Mma16x16<T> MM;
   typedef typename M::frag frag;
   typedef DecodeCfg<D, kWaves> C;
-  typedef WeightRange<T, TERMS> W;
+  typedef WeightRange<PT, TERMS> W;
   constexpr int KESZ = KV8 ? 1 : 2;
   constexpr int NK = D * KESZ / 64;        // 16-byte loads of a key's row by the four lanes that share it
   constexpr int DL = D / 16;               // dims of V per lane
   constexpr int VW = DL * KESZ / 4;        // their 4-byte words
-  // Terms beside the first have sums of their own (e4m3 has no infinities): where V holds one they are NaN, and the first term's sum is the result.
+  // Terms beside the first have sums of their own, for their scale and for V's infinities (e4m3 has neither): where V holds one these sums are no numbers, and
+  // the first term's sum is the result.
   constexpr bool REST = TERMS > 1 && !KV8;
   extern __shared__ __align__(16) unsigned char smem[];
   float* const sm = (float*)smem;
@@ -219,12 +231,12 @@ __global__ void __launch_bounds__(kWaves * 64) rows16_fwd_kernel(const FwdParams
       l += p0 + p1;
 #pragma unroll
       for (int j = 0; j < TERMS; ++j) {
-        pw[j][i] = M::pack2(p0, p1);
+        pw[j][i] = j == 0 ? MP::pack2(W::first(p0), W::first(p1)) : MP::pack2(p0, p1);
         if (j + 1 < TERMS) {
           float y0, y1;
-          M::unpack2(pw[j][i], y0, y1);
-          p0 -= y0;
-          p1 -= y1;
+          MP::unpack2(pw[j][i], y0, y1);
+          p0 = (p0 - y0) * (j == 0 ? W::later : 1.f);
+          p1 = (p1 - y1) * (j == 0 ? W::later : 1.f);
         }
       }
     }
@@ -232,7 +244,7 @@ __global__ void __launch_bounds__(kWaves * 64) rows16_fwd_kernel(const FwdParams
 #pragma unroll
     for (int e = 0; e < 8; ++e)
 #pragma unroll
-      for (int i = 0; i < DL / 2; ++i) y[e][i] = KV8 ? MM::widen(vx[e].w[i / 2], i & 1) : vx[e].w[KV8 ? 0 : i];
+      for (int i = 0; i < DL / 2; ++i) y[e][i] = KV8 ? MMP::widen(vx[e].w[i / 2], i & 1) : vx[e].w[KV8 ? 0 : i];
 #pragma unroll
     for (int d = 0; d < DL; ++d) {
       u32x4 v;
@@ -241,7 +253,7 @@ __global__ void __launch_bounds__(kWaves * 64) rows16_fwd_kernel(const FwdParams
 #pragma unroll
       for (int j = TERMS - 1; j >= 0; --j) {
         f32x4& to = REST && j > 0 ? rest[REST ? d : 0] : o[d];
-        to = MM::run(as_frag<frag>(v), as_frag<frag>(pw[j]), to);
+        to = MMP::run(as_frag<pfrag>(v), as_frag<pfrag>(pw[j]), to);
       }
     }
     if (key0 + PASS < k1) load_v(key0 + PASS);
@@ -260,7 +272,7 @@ __global__ void __launch_bounds__(kWaves * 64) rows16_fwd_kernel(const FwdParams
       for (int d = 0; d < 4; ++d) {
         y[d] = o[d0 + d][i];
         if (REST) {
-          const float r = rest[REST ? d0 + d : 0][i];
+          const float r = rest[REST ? d0 + d : 0][i] * (1.f / W::later);
           y[d] += fabsf(r) < INFINITY ? r : 0.f;
         }
       }

@@ -1,6 +1,8 @@
 """Calls of up to 16 query rows without a mask on the kernel that streams K and V through matrix instructions (rows of a head back to back, layout
 [B, H, S, D]; more than three rows also with other heads in between): edges of its tiles of 32 keys and of a workgroup's pass, chunks, both
 element types and e4m3, the values a weight of several terms has to get right."""
+import math
+
 import pytest
 import torch
 
@@ -105,6 +107,47 @@ def test_many_small_weights_beside_a_large_one(Sq, dtype):
     # rounded once to the element type, weights off by 2^-22 at most
     assert (out.cpu().double() / want.transpose(1, 2) - 1).abs().max().item() < (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -10)
     check_lse(lse, want_l)
+
+
+@pytest.mark.parametrize("e4m3", [False, True])
+@pytest.mark.parametrize("Sq", [1, 2, 3])
+def test_weights_far_below_the_largest(Sq, e4m3):
+    """fp16: one key of weight 1 and value 0, 1023 of weight e^-30 = 2^-43.3 and value 57344: 5.5e-6 of a result whose steps are 2^-24 = 6e-8, half a step
+    of error, and of weights in steps of 2^-50 half of 1023 * 57344 * 2^-50 at most."""
+    D, Sk = 64, 1024
+    q, k = torch.zeros((1, 1, Sq, D)), torch.zeros((1, 1, Sk, D))
+    q[..., 0], k[:, :, 1:, 0] = 7.5, -4.0
+    v = torch.full((1, 1, Sk, D), 448.0 if e4m3 else 57344.0)
+    v[:, :, 0] = 0.0
+    kw = {}
+    if e4m3:
+        kw = dict(k_scale=torch.ones((1, 1), device=DEV), v_scale=torch.full((1, 1), 128.0, device=DEV))
+    place = lambda t: (t.to(torch.float8_e4m3fn) if e4m3 else t.half()).to(DEV)
+    out, _ = ops.flash_fwd(q.half().to(DEV), place(k), place(v), 1.0, False, layout="bhsd", split_kv=None, **kw)
+    want = 1023 * math.exp(-30.0) * 57344
+    assert (out.double() - want).abs().max().item() <= 2.0 ** -25 + 0.5 * 1023 * 57344 * 2.0 ** -50
+
+
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Sq", [1, 2, 3])
+@pytest.mark.parametrize("nats", [10, 20, 40, 80])
+def test_an_infinity_under_a_small_weight(nats, Sq, dtype, layout):
+    """Up to three rows: a weight that fp32 holds (e^-80 = 2^-115) makes an infinity of V one in the result, however small it is; one of a score of
+    -infinity is 0, and 0 times infinity no number."""
+    D, Sk, H = 64, 700, 2
+    q, k, v = torch.zeros((1, Sq, H, D)), torch.zeros((1, Sk, H, D)), rand((1, Sk, H, D), 75, torch.float32)
+    q[..., 0], k[:, 333, :, 0] = 8.0, -nats / 8.0
+    v[:, 333, 0, 3], v[:, 333, 1, 5] = float("inf"), -float("inf")
+    place = (lambda t: t.to(dtype).transpose(1, 2).contiguous().to(DEV)) if layout == "bhsd" else (lambda t: t.to(dtype).to(DEV))
+    run = lambda: ops.flash_fwd(place(q), place(k), place(v), 1.0, False, layout=layout, split_kv=None)[0].float().cpu()
+    out = run() if layout == "bshd" else run().transpose(1, 2)
+    assert (out[:, :, 0, 3] == float("inf")).all() and (out[:, :, 1, 5] == -float("inf")).all()
+    out[:, :, 0, 3] = out[:, :, 1, 5] = 0.0
+    assert out.isfinite().all()
+    k[:, 333, :, 0] = -float("inf")
+    out = run() if layout == "bshd" else run().transpose(1, 2)
+    assert out[:, :, 0, 3].isnan().all() and out[:, :, 1, 5].isnan().all() and out[:, :, 0, 4].isfinite().all()
 
 
 @pytest.mark.parametrize("Sq", [1, 3, 4, 16])
