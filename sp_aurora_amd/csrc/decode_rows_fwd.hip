@@ -349,17 +349,42 @@ hipError_t launch(const FwdParams& p, hipStream_t stream) {
 
 }  // namespace
 
-// Whether this kernel is the faster one for a call of up to 16 rows (p as for the launch).  Us a call, before / here, 32 heads of 32768 keys and 16 x 32 heads of
-// 4000: rows back to back, one row, e4m3, D = 64 30.5 / 28.2, 50.8 / 45.5, D = 128 51.4 / 46.4, 81.5 / 84.8, bf16, D = 128 81.9 / 80.6, 155.9 / 155.2, three rows
-// 92.2 / 80.8; eight rows (before on flash_fwd.hip's kernels), e4m3, D = 64 52.8 / 26.2, 85.8 / 44.2, D = 128 79.5 / 45.8, 136 / 83.7, bf16 99.5 / 80.4, 183 / 155.
-// Not for one row, of 64 16-bit elements from memory (45.1 / 45.8, 79.7 / 81.0) or of few heads whose keys are not split (8 of 600 keys 6.1 / 7.0), or of 128 e4m3 elements whose keys are not split.  Rows of other heads in between:
-// up to three rows stay on decode_fwd.hip, which takes neighbouring heads together (its 225 us for 64 caches of 1 to 4 thousand e4m3 tokens were 303 here);
-// eight rows, e4m3, D = 128 72.7 / 61.9, 131 / 111, bf16 181 / 177, but 32 heads of 32768 91.4 / 93.3, and of 64 16-bit elements 57.8 / 60.0, 97.9 / 108.6.
+// Whether this kernel is the faster one for a call of up to 16 rows (p as for the launch), from 9000 calls of 3 to 4096 heads and 16 to 32768 keys; us a call,
+// decode_fwd.hip's kernel (up to three rows) or flash_fwd.hip's / this one.  What it has against it: a workgroup, of eight waves mostly, fills a CU and is long, so
+// that a second round of them which is not full, or CUs without one, cost more (`uneven`: long chunks in such a launch), and its start and end count in
+// launches of thousands of short ones.
+// Rows back to back.  One row: not of 16-bit elements (D = 128: 64 x 32 heads of 48 keys 12.2 / 28.5, 8 of 2048 8.5 / 9.6, 32 of 32768 86.8 / 86.1; D = 64, 8 of
+// 700 6.9 / 8.4); of e4m3 ones (D = 64: 64 x 32 heads of 100 keys 22.8 / 14.4, 32 of 4096 12.1 / 10.4, but 5 x 40 of 4096 24.7 / 27.7), at D = 128 in one round
+// (32 of 16384 31.9 / 27.9, 2 x 32 of 100 6.8 / 5.5, 64 x 32 of 256 26.3 / 40.2), but for the few workgroups of a call that is not split (8 of 512 7.7 / 7.9, 4 x
+// 32 of 16384 106 / 134).
+// Two rows of 16 bits: 32 of 4096 keys, D = 128 18.3 / 17.2, 8 x 32 of 512, D = 64 11.1 / 9.4; 3 x 32 of 8192 42.5 / 51.3, 16 x 20 of 1024, D = 128
+// 32.3 / 38.3, 64 x 32 of 48 14.8 / 28.9; of e4m3 elements 8 x 32 of 2048, D = 128 31.1 / 26.1, but 64 x 32 of 256 35.9 / 40.4.
+// Three: 16 x 32 of 1300, D = 128 63.1 / 58.5, e4m3 42.5 / 33.8; 4 x 34 of 8192, in two chunks 130 / 140.
+// More: e4m3 elements everywhere (0.41 to 0.9 of flash_fwd.hip's time); 16-bit ones, D = 128, 8 x 32 of 2048 51.3 / 44.0, 20 of 16384, split, 38.3 / 34.2; where
+// uneven, up to three quarters of the CUs, 4 x 34 of 2048 33.3 / 37.8.  More than eight rows against a few keys, of which most of the eight waves have none, in
+// several rounds: 16 x 32 of 256, D = 128 16.0 / 17.2, 512 x 8 of 48 e4m3 44.9 / 47.4, in between other heads 47.0 / 53.8.
+// Rows of other heads in between.  Up to three stay on decode_fwd.hip, which takes neighbouring heads together.  More: e4m3 as back to back, but from memory and not
+// split at D = 128 (8 x 32 of 4096 59.4 / 62.4); 16-bit ones as back to back up to what stays in the cache (2 x 32 of 512 keys 11.0 / 10.2; 16 x 20 of 512 20.1 / 26.3).
 bool spa_rows16_takes(const FwdParams& p, int D) {
   const bool kv8 = p.k_scale != nullptr, memory = kv_bytes(p, D) > kCachedBytes;
-  if (p.Sq == 1 && !kv8 && D == 64 && p.P == 1 && (int64_t)p.B * p.H <= 16) return false;
-  if (p.ks.s == D && p.vs.s == D) return !memory || p.Sq > 1 || (kv8 ? D == 64 || p.P > 1 : D == 128);
-  return p.Sq > kRowsInFp32 && !(memory && !kv8 && (D == 64 || p.P > 1));
+  const int64_t cus = spa_device_cus(), wgs = (int64_t)p.B * p.H * p.P;
+  const bool whole = p.P == 1, longer = (int64_t)p.Sk * D >= 2048 * 64, second = wgs > cus && wgs < 2 * cus;
+  const bool uneven = longer && (second || (whole && wgs < cus));
+  const bool back = p.ks.s == D && p.vs.s == D;
+  if (p.Sq > 8 && D == 128 && p.Sk <= 256 && (kv8 ? wgs >= 8 * cus && (!back || p.Sk <= 64) : wgs > cus && wgs < 4 * cus)) return false;
+  if (!back) {
+    if (p.Sq <= kRowsInFp32) return false;
+    if (kv8) return !(D == 128 && memory && whole && p.Sk >= 2048);
+    return !memory && !(longer && whole && 4 * wgs < 3 * cus);
+  }
+  switch (p.Sq) {
+    case 1: return kv8 && (D == 64 ? !uneven : wgs <= cus && (!whole || p.Sk <= 256 || 2 * wgs > cus));
+    case 2:
+      if (kv8) return D == 64 ? !uneven : !(longer && second) && wgs < 4 * cus;
+      return wgs <= cus ? !uneven : wgs >= 2 * cus && p.Sk > 256;
+    case 3: return kv8 || !uneven;
+    default: return kv8 || !(longer && whole && 4 * wgs < 3 * cus);
+  }
 }
 
 // As spa_launch_fwd_fewrows, for 1 <= Sq <= 16 rows of calls that are not packed batches.

@@ -274,10 +274,11 @@ int spa_flash_fwd_splitkv_suggest(int B, int H, int Sq, int Sk, int D, int mask_
   // shapes (more chunks: 3 to 15 % slower), chunks of at least 256 keys (instead of 512, us, device: [1, 8, 1 against 2048], D = 128 9.4
   // and 8.5, 32 heads 10.9 and 9.1, D = 64 against 1024 9.1 and 8.0, 32 heads 10.3 and 8.5).  From 1024 keys on, with four rows and more, whose kernel is faster
   // by itself than two launches are sent off, from 2048, or, at D = 128 and few heads, 1280 (us, whole / split: 8 rows, 8 heads against 1926, bf16 21.2 / 10.7, e4m3
-  // 12.9 / 9.0; D = 64, e4m3 8.4 / 7.1).
+  // 12.9 / 9.0; D = 64, e4m3 8.4 / 7.1).  Those have workgroups that fill a CU: not one more than there are CUs (D = 128, 20 heads of 16384 keys in 12 / 13 chunks 34.2 /
+  // 46.2, 4 x 34 of 4096 in one / two 58.6 / 75.9).
   if (Sq <= kRows16 && spa_knob(SPA_KNOB_FEW_ROWS) != 1) {
     if (Sk < (Sq <= kFewRows ? 1024 : D == 128 && (int64_t)B * H * 4 <= cus ? 1280 : 2048)) return 1;
-    int64_t n = ((int64_t)cus + (int64_t)B * H / 2) / ((int64_t)B * H);
+    int64_t n = ((int64_t)cus + (Sq <= kFewRows ? (int64_t)B * H / 2 : 0)) / ((int64_t)B * H);
     // (not more than 16 of them below 512 keys: the second kernel takes 2.3 us for 8 or 16 chunks of 8 heads and 5 for 32)
     const int64_t by_length = Sk / 256 < 16 ? Sk / 256 : Sk / 512 > 16 ? Sk / 512 : 16;
     if (n > by_length) n = by_length;

@@ -368,3 +368,17 @@ def test_workspace_of_a_ragged_key_split_follows_the_keys():
         for chunk in (1, 512, 1000):
             for longest in (total // nseq + 1, total):
                 assert size(nseq, total, longest, chunk) == per_chunk * (total // chunk + nseq)
+
+
+def test_a_key_split_of_few_rows_fills_the_compute_units_once():
+    """Four to sixteen rows, whose workgroups fill a CU: not one more of them than there are CUs (without a device the library reckons with 256)."""
+    lib = _lib.load()
+    for D in (64, 128):
+        for Sq in (4, 8, 16):
+            for pairs in list(range(1, 40)) + [48, 64, 85, 86, 96, 103, 128, 129, 136, 160, 171, 200, 256]:
+                for Sk in (1280, 1926, 2048, 3000, 8192, 32768, 262144):
+                    n = lib.spa_flash_fwd_splitkv_suggest(1, pairs, Sq, Sk, D, _lib.SPA_MASK_NONE, _lib.SPA_BF16)
+                    assert 1 <= n <= 64 and (n == 1 or n * pairs <= 256), (D, Sq, pairs, Sk, n)
+    for pairs in (20, 96, 136):  # up to three rows: as near to the number of CUs as whole chunks come
+        n = lib.spa_flash_fwd_splitkv_suggest(1, pairs, 3, 32768, 128, _lib.SPA_MASK_NONE, _lib.SPA_BF16)
+        assert n == round(256 / pairs)
