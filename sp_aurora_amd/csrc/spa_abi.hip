@@ -1079,10 +1079,17 @@ int64_t spa_flash_fwd_varlen_splitkv_workspace_bytes(int nseq, int H, int total_
 // are 1 to 4 % slower), or, at D = 128, of 512 while those are 16 thousand workgroups of one head or fewer and the last of them count (1024 / 512,
 // us, longest of 4096: 64, H = 32, e4m3 232 / 224, bf16 438 / 438; of 8192: 8, H = 32, 63.5 / 59.5 and 130 / 125, 32, H = 8, 74.7 /
 // 65.4 and 125 / 122, but 64, H = 32, 483 / 487 and 808 / 812).
-// One row: 256 keys while those are 4 (D = 64: 8) thousand chunks of one head or fewer, and where single caches would have more than 1024 for each CU: a workgroup
+// One row: 256 keys while those are 8 (D = 64: 16) thousand chunks of one head or fewer, and where single caches would have more than 1024 for each CU: a workgroup
 // more or less on a CU, and the last ones, cost less.  Of 950 random batches (8 to 64 caches of 512 to 8192 tokens) the choice is 2.7 % faster than
-// the one before, 1.42x at most (8 caches of up to 7966, H = 8, D = 64, bf16), none more than 2.5 % slower.  Two or three rows, with as many
+// the one before, 1.42x at most (8 caches of up to 7966, H = 8, D = 64, bf16), none more than 2.5 % slower; of 950 of 100 to 2000 short caches and a few of 2210 to
+// 13260 tokens 8.6 %, one in fourteen 5 to 15 % slower (those of 16 workgroups a CU and more, which keep longer chunks).  Two or three rows, with as many
 // sums to merge: up to 5 and 16 % slower with it.
+// The merge of a long cache's chunks is one workgroup's work (D = 128, one of 32768 / 65536 / 131072 tokens, H = 8, e4m3, chunks of 256: 27 / 44 / 81 us, of
+// 1024 22 / 32 / 57): not more than 128 of them.  And an even share for each CU is the best chunk where next to nothing is left over, a second round of workgroups
+// otherwise (2 caches of 32768 and 30000, H = 32, D = 128, bf16 219 / 172 with 256): one cache that is nearly all of the batch (65536, H = 8, D = 128, bf16 65 / 48 us,
+// 131072, H = 32 360 / 309; D = 64 up to 4096 keys a chunk, beyond which neighbouring heads, whose rows share lines, drift apart: 65536, H = 32, e4m3 67 / 81, 52 in chunks
+// of 1024), or up to 32 caches' heads and 2048 keys (4 caches of up to 29742, H = 8, D = 128, e4m3 28.7 / 21.1).  Of 1140 random batches of up to 64 caches of 4096 to
+// 262144 tokens, one or a few long ones among them, H = 4 to 40: 3.0 % slower than the best of ten lengths on average (with chunks of 256 alone 8.1, even shares alone 16.6).
 int spa_flash_fwd_varlen_splitkv_suggest(int nseq, int H, int total_k, int max_sq, int max_sk, int D, int dtype) {
   if (nseq <= 0 || H <= 0 || total_k <= 0 || max_sq <= 0 || max_sq > kFewRows || max_sk <= 0 || (D != 64 && D != 128) ||
       (dtype != SPA_BF16 && dtype != SPA_F16) || spa_knob(SPA_KNOB_FEW_ROWS) == 1)
@@ -1090,15 +1097,24 @@ int spa_flash_fwd_varlen_splitkv_suggest(int nseq, int H, int total_k, int max_s
   const int64_t cus = spa_device_cus();
   const int64_t even = (int64_t)total_k * H / cus;  // keys of all heads for each CU
   const bool one = max_sq == 1;
+  const int64_t least = ((int64_t)max_sk + 128 * 256 - 1) / (128 * 256) * 256;  // (one row) at most 128 chunks of a cache
   if ((int64_t)nseq * H >= cus) {
     if (max_sk <= 2200) return 0;
-    if (one) {
-      if (D == 64) return even <= 32 * 512 ? 256 : 512;
-      if (even <= 16 * 512 && max_sk > 2400) return 256;
-    }
-    return D == 128 && even <= 64 * 512 ? 512 : 1024;
+    const int64_t several = D == 128 && even <= 64 * 512 ? 512 : 1024;
+    if (!one) return (int)several;
+    // (16 workgroups of one head per CU and more are enough of them; at D = 64 where most of them are short, that is.  Up to 2400 tokens 512 keys are 2 % faster
+    // for e4m3 caches and 5 to 10 % slower for bf16, 32 and 64 of them, H = 8)
+    const bool many = (int64_t)nseq * H >= 16 * cus;
+    const int64_t chunk = D == 64 ? (even > 32 * 512 ? 512 : many && total_k >= (int64_t)256 * nseq ? 1024 : 256)
+                                  : even <= 16 * 512 && max_sk > 2400 && !many ? 256 : several;
+    return (int)(chunk > least ? chunk : least);
   }
-  const int64_t chunk = even <= 256 || (one && even > 1024) ? 256 : (even + 255) / 256 * 256;
+  int64_t shares = INT64_MAX;  // even shares up to this many keys
+  if (one) {
+    shares = (int64_t)nseq * H <= 32 ? 2048 : 1024;
+    if ((int64_t)total_k * 20 <= (int64_t)max_sk * 21) shares = D == 128 ? INT64_MAX : 4096;
+  }
+  const int64_t share = even <= 256 ? 256 : (even + 255) / 256 * 256, chunk = even <= shares || share < least ? share : least;
   return max_sk >= chunk * 3 / 2 ? (int)chunk : 0;
 }
 

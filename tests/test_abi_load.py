@@ -370,6 +370,26 @@ def test_workspace_of_a_ragged_key_split_follows_the_keys():
                 assert size(nseq, total, longest, chunk) == per_chunk * (total // chunk + nseq)
 
 
+def test_the_chunks_a_ragged_key_split_suggests_stay_few():
+    """One row: at most 128 chunks of the longest cache, whose merge is one workgroup's work; one cache (nearly) alone, and a few caches with little to
+    do, are shared out evenly over 256 CUs (without a device the library reckons with 256)."""
+    lib = _lib.load()
+    suggest = lambda lens, H, D, rows=1: lib.spa_flash_fwd_varlen_splitkv_suggest(len(lens), H, sum(lens), rows, max(lens), D, _lib.SPA_BF16)
+    for D in (64, 128):
+        for H in (2, 4, 8, 32, 40):
+            for lens in ([1 << 20], [131072], [65536, 60000], [100000] * 4, [131072] + [256] * 31, [32768] + [256] * 300, [500000] + [100] * 2000, [262144, 9, 9]):
+                chunk = suggest(lens, H, D)
+                assert chunk % 256 == 0 and 0 < max(lens) <= 128 * chunk, (D, H, len(lens), max(lens), chunk)
+    share = lambda lens, H: (sum(lens) * H // 256 + 255) // 256 * 256
+    for lens, H in (([65536], 8), ([131072], 32), ([300000], 8), ([131072, 500], 8)):
+        assert suggest(lens, H, 128) == share(lens, H)
+    assert suggest([65536], 8, 64) == share([65536], 8) and suggest([65536], 32, 64) == 512
+    assert suggest([29742, 1000, 1000, 1724], 8, 128) == share([29742, 1000, 1000, 1724], 8)
+    assert suggest([4000] * 8, 32, 128) == 256  # (what most ragged batches get)
+    for rows in (2, 3):  # as many sums to merge: even shares
+        assert suggest([65536, 50000], 8, 128, rows) == share([65536, 50000], 8)
+
+
 def test_a_key_split_of_few_rows_fills_the_compute_units_once():
     """Four to sixteen rows, whose workgroups fill a CU: not one more of them than there are CUs (without a device the library reckons with 256)."""
     lib = _lib.load()
