@@ -1346,11 +1346,15 @@ float form_us(const FwdParams& p, FwdForm f, int D, FwdKind kind) {
   const float n = (float)p.B * (float)p.H * tiles;
   // (equal workgroups end together: half of a last round that is not full is lost)
   const float load = p.causal || p.cu_q ? n / cus : 0.5f * (n / cus + ceilf(n / cus));
-  if (f == FWD_FOUR && n > cus) {
-    // One workgroup to a CU, whose start and end nothing covers.  Not causal: whole rounds of them.  Causal, the long ones first: the second round begins where
-    // the shortest of the first ends, and what is left over behind whole rounds, which end together, adds one of its own.
-    const float pairs = (float)p.B * (float)p.H, own = rows / keys;  // steps from one tile to the next
-    if (!p.causal) return ceilf(n / cus) * (mean * c.busy + c.round) + c.fixed;
+  float us = fmaxf(longest * c.alone, load * mean * c.busy) + c.round * fmaxf(1.f, n / slots) + c.fixed;
+  if (f != FWD_FOUR) return us;
+  const float pairs = (float)p.B * (float)p.H, own = rows / keys;  // steps from one tile to the next
+  if (n > cus && !p.causal) {
+    // One workgroup to a CU, whose start and end nothing covers: whole rounds of them.
+    us = ceilf(n / cus) * (mean * c.busy + c.round) + c.fixed;
+  } else if (n > cus) {
+    // Causal, the long ones first: the second round begins where the shortest of the first ends, and what is left over behind whole rounds, which end together,
+    // adds one of its own.
     auto steps = [&](float i) { return fminf(longest, (tiles - floorf(i / pairs)) * own); };  // of workgroup i of the launch
     const float rounds = floorf(n / cus), work = n / cus * (mean * c.busy + c.round);
     float last = work;
@@ -1358,9 +1362,22 @@ float form_us(const FwdParams& p, FwdForm f, int D, FwdKind kind) {
       last = 2.f * c.round + (steps(cus - 1.f) + steps(cus)) * c.busy;
     else if (rounds * cus < n)
       last = rounds * (c.round + (longest - (rounds * cus / pairs - 1.f) * 0.5f * own) * c.busy) + c.round + steps(rounds * cus) * c.busy;
-    return fmaxf(longest * c.alone + c.round, fmaxf(work, last)) + c.fixed;
+    us = fmaxf(longest * c.alone + c.round, fmaxf(work, last)) + c.fixed;
   }
-  return fmaxf(longest * c.alone, load * mean * c.busy) + c.round * fmaxf(1.f, n / slots) + c.fixed;
+  // Its few rows read K and V often: a (batch, head)'s tiles share what they read while they run side by side on one XCD, which they do where there are a multiple of 8
+  // pairs, in one round, or later ones with little to read (2 MB, half of an L2).  Rows of other heads in between come as whole lines.  At 6.7 TB/s, of the memory-side
+  // cache mostly.  (us, faster form of the others / FOUR: [1, 128 rows, 100 heads, 128] against 2048 keys, bf16 32 / 39; [2, 164, 128, 32] against 8645 132 / 263;
+  // [16, 379, 8, 64] against 22380 423 / 576.)
+  const int pair = p.B * p.H;
+  const float esz = kind == KIND_16 ? 2.f : 1.f, row = p.ks.s == D ? D * esz : fmaxf(128.f, D * esz);
+  float reads = fminf(tiles, (pair % 8 == 0 ? 1.f : pair % 4 == 0 ? 2.f : pair % 2 == 0 ? 4.f : 8.f) * ceilf(n / cus));
+  if (n > cus && 2.f * sk * D * esz > 2e6f) reads = tiles;
+  us = fmaxf(us, reads * pairs * sk * row * (p.causal ? 1.f : 2.f) / 6.7e6f + c.round + c.fixed);
+  // Margins, for what the constants (e4m3 K/V of 64 elements have those of 128, 16-bit of 32 those of 64) do not know.  Of 7800 launches that this form was then taken
+  // for (1 to 1500 heads, 17 to 1000 rows, 65 to 32000 keys, not those of the fit) 13 lose more than 2 % by it, 12 % at most, and 0.79 of the others' time is the
+  // mean; without the reads and the margins 227 of 8700 lost that, up to 1.93 x.
+  if (kind == KIND_KV8) us *= D > 64 ? 1.04f : 1.14f;
+  return n > cus && !p.causal ? 1.05f * us : us;
 }
 
 FwdForm fwd_form(const FwdParams& p, int D, FwdKind kind) {

@@ -127,3 +127,19 @@ def test_the_form_is_taken_for_small_launches(H, S):
         finally:
             _lib.tune("fwd_groups", 0)
     assert torch.equal(own[0], got[4][0]) and not torch.equal(own[0], got[2][0])
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk,D", [(1, 100, 128, 2048, 128), (2, 128, 164, 8645, 32), (16, 8, 379, 22380, 64)])
+def test_the_form_is_left_out_where_its_reads_decide(B, H, Sq, Sk, D):
+    """Launches that fit its work but read K and V once a tile: the bits are another form's."""
+    g = torch.Generator(device=DEV).manual_seed(170)
+    q, k, v = (torch.randn((B, s, H, D), generator=g, device=DEV).bfloat16() for s in (Sq, Sk, Sk))
+    own = ops.flash_fwd(q, k, v, None, False, split_kv=1)[0]
+    _lib.tune("fwd_groups", 4)
+    try:
+        four = ops.flash_fwd(q, k, v, None, False, split_kv=1)[0]
+    finally:
+        _lib.tune("fwd_groups", 0)
+    assert not torch.equal(own, four)
+    # (weights rounded beside another reference maximum, sums in another order, rounded to bf16)
+    assert (own.float() - four.float()).norm().item() <= 2.0 ** -7 * own.float().norm().item()
