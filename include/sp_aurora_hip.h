@@ -116,7 +116,7 @@ int spa_flash_fwd_fp8kv(const void* q, const void* k8, const void* v8,
  * The block forward for calls with few query rows and many keys (a decode step against a KV cache: the call sites that hand
  * the operator a cache, adapters/hf_adapter.py:141-155): without a mask the keys can be cut into nsplit chunks that run
  * side by side on the same query rows (grid planes of one launch), each leaving its block result (out in q's type, in fp32
- * for four to sixteen rows, and lse) in the workspace; a second kernel applies update_out_and_lse (sp_aurora/utils.py:103-104) to all of them.  The plain
+ * for four to sixteen rows or two chunks of more, and lse) in the workspace; a second kernel applies update_out_and_lse (sp_aurora/utils.py:103-104) to all of them.  The plain
  * launch has B * H * ceil(Sq / 128) workgroups however long the keys are, which leaves most of the 256 CUs idle for such a call.
  * spa_flash_fwd_splitkv_suggest returns the number of chunks the library would take for a shape (1: do not split);
  * nsplit = 1 is spa_flash_fwd.  Chunks hold a multiple of 128 keys, so fewer than nsplit may run.  bf16 / fp16, D in

@@ -145,10 +145,10 @@ struct KeySplit {
 };
 // Chunks of more than kFewRows and up to kRows16 rows leave their results in fp32: rounded to 16 bits they add 15 to 22 % to the error of the rows (four to
 // seven chunks; bf16 against float64, 8 heads of 1926 keys, D = 128, 2.3e-3 -> 2.7e-3), and calls of 1280 keys on are cut that sum in fp32 to the end
-// in one piece.  The cost is 0.6 % of a call on average, 0.2 us of the shortest (8 rows, 8 heads of 2048 e4m3 keys, D = 128 7.6 -> 7.9 us, device).
-bool splitkv_part32(int Sq) { return Sq > kFewRows && Sq <= kRows16; }
+// in one piece.  So do two chunks of more rows, for the same reason (three and more have always been 16-bit).  The cost is 0.6 % of a call on average, 0.2 us of the shortest (8 rows, 8 heads of 2048 e4m3 keys, D = 128 7.6 -> 7.9 us, device).
+bool splitkv_part32(int Sq, int nsplit) { return Sq > kFewRows && (Sq <= kRows16 || nsplit == 2); }
 int64_t splitkv_out_bytes(int B, int H, int Sq, int D, int n) {
-  return ((int64_t)B * n * Sq * H * D * (splitkv_part32(Sq) ? 4 : 2) + 255) / 256 * 256;
+  return ((int64_t)B * n * Sq * H * D * (splitkv_part32(Sq, n) ? 4 : 2) + 255) / 256 * 256;
 }
 
 // k_scale / v_scale non-null: K and V are e4m3 bytes (strides in bytes), q / out of type `dtype`.
@@ -219,7 +219,7 @@ int flash_fwd(const char* what, const void* q, const void* k, const void* v, con
       if (ks.n > 1) {
         // plane z writes rows z * Sq .. of the scratch tensors [B, n * Sq, H, D] and [B, H, n * Sq]
         p.out = part_out; p.lse = part_lse;
-        p.out32 = splitkv_part32(Sq);
+        p.out32 = splitkv_part32(Sq, nsplit);
         p.os.b = (int64_t)ks.n * Sq * H * D; p.os.s = (int64_t)H * D; p.os.h = D;
         p.lse_bh = (int64_t)ks.n * Sq;
       }
@@ -285,17 +285,20 @@ int spa_flash_fwd_splitkv_suggest(int B, int H, int Sq, int Sk, int D, int mask_
     if (n > 64) n = 64;
     return n < 2 ? 1 : KeySplit(Sk, (int)n).n;
   }
-  // Otherwise worth it when 128-row workgroups would leave two thirds of the CUs idle and every
+  // Otherwise worth it when 128-row workgroups would leave half of the CUs idle and every
   // chunk keeps at least 512 keys: as many chunks as give no CU more than one workgroup (measured on six decode shapes: more
-  // chunks only add the workgroups' fixed cost and rows for the merge).  Not fewer than four, or three of long rows: beside the form of the plain
-  // launch that shares 64 rows out over four wave groups (us, D = 128, split / plain: 8 heads of 2048 rows and 4096 keys, two, 44.4 / 40.9; 16 of 600
-  // and 2048, three, 24.6 / 20.9, of 640 and 4096 33.9 / 35.1; 8 of 1024 and 2048, four, 22.0 / 21.1, of 400 17.8 / 20.6).
+  // chunks only add the workgroups' fixed cost and rows for the merge).  Fewer than four only of long rows, beside the form of the plain
+  // launch that shares 64 rows out over four wave groups and needs less of a merge's fixed cost: three from 4096 keys on (us, D = 128, split / plain: 16
+  // heads of 600 rows and 2048 24.6 / 20.9, of 640 and 4096 33.9 / 35.1; four, 8 of 1024 and 2048 22.0 / 21.1, of 400 17.8 / 20.6), two from 8192, at D = 64
+  // 16384 (split / plain, 12 heads of 1024 rows, 8 of 2048, 100 of 100, D = 128 against 4096 1.06, 1.19, 0.94, 8192 0.94, 1.01, 0.69, 65536 (32768) 0.66, 0.83, 0.62; D =
+  // 64, 8192 1.04, 1.07, 0.72, 16384 0.99, 1.01, 0.69; e4m3, which gains more, D = 128, 4096 0.88, 1.04, 0.85, 8192 0.77, 0.86, 0.78).
   const int64_t wgs = (int64_t)B * H * ((Sq + 127) / 128);
-  if (wgs * 3 > cus || Sk < 2048) return 1;
+  if (wgs * 2 > cus || Sk < 2048) return 1;
   int64_t n = cus / wgs;
   if (n > Sk / 512) n = Sk / 512;
   if (n > 64) n = 64;
-  return n < 3 || (n == 3 && Sk < 4096) ? 1 : KeySplit(Sk, (int)n).n;
+  if (Sk < (n > 3 ? 2048 : n == 3 ? 4096 : D == 128 ? 8192 : 16384)) return 1;
+  return KeySplit(Sk, (int)n).n;
 }
 
 int spa_flash_fwd_splitkv(const void* q, const void* k, const void* v, void* out, float* lse, void* workspace, int B, int H, int Sq,

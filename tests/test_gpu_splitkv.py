@@ -82,6 +82,23 @@ def test_chunks_of_few_rows_add_no_error(H, Sq, Sk, D, layout, dtype, e4m3):
     assert cut <= 1.03 * whole, f"split {cut:.3e}, whole {whole:.3e}"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,Sq,Sk,D", [(90, 17, 8192, 128), (100, 33, 16384, 64), (43, 130, 9000, 128)])
+def test_two_chunks_of_long_rows(H, Sq, Sk, D, dtype):
+    """Launches of 86 to 128 workgroups of 128 rows are cut in two where the keys are long, and the halves wait in fp32 (bounds as above)."""
+    assert _lib.load().spa_flash_fwd_splitkv_suggest(1, H, Sq, Sk, D, 0, ops._DT[dtype]) == 2
+    q, k, v = (rand((1, s, H, D), 1050 + i, dtype).to(DEV) for i, s in enumerate((Sq, Sk, Sk)))
+    want, want_l = [], []
+    for h in range(H):
+        s = q[0, :, h].double() @ k[0, :, h].double().t().contiguous() * D ** -0.5
+        want.append(torch.softmax(s, -1) @ v[0, :, h].double())
+        want_l.append(torch.logsumexp(s, -1))
+    want = torch.stack(want, 1)[None].cpu()
+    whole, cut = (ops.flash_fwd(q, k, v, split_kv=n) for n in (1, "auto"))
+    assert _relative_error(cut[0], want) <= 1.03 * _relative_error(whole[0], want)
+    check_lse(cut[1], torch.stack(want_l)[None].cpu())
+
+
 def test_key_split_with_e4m3_cache():
     B, H, Sq, Sk, D = 1, 8, 4, 6000, 128
     from test_gpu_fp8kv import quantised
