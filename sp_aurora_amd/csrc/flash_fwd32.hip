@@ -835,13 +835,16 @@ hipError_t launch_splitk(const FwdParams& p, hipStream_t stream) {
 }  // namespace
 hipError_t spa_launch_fwd32_shared_keys_128(const FwdParams& p, hipStream_t stream) { return launch_splitk<128>(p, stream); }
 #else
-// Whether the waves of a workgroup share out the keys of 32 rows rather than taking 32 rows each.  Microseconds of a launch, from 90 launches of
-// 128 to 4096 rows and 8 to 32 heads (of which the faster kernel is taken but for three, 5 % at most): workgroups of the kernel for many rows take
-// the tiles of the longest chain at `first` each alone on their CU and at `full` each and workgroup where several share it; those for few rows, one to a
-// CU, `start` and `step` for every eighth tile.  Not causal, whole rounds of workgroups; causal, heaviest first, the longest or all of them over the CUs.
+// Whether the waves of a workgroup share out the keys of 32 rows rather than taking 32 rows each.  Microseconds of a launch, less what both have in common, from
+// 5700 launches of 1 to 4000 rows and keys and 1 to 512 heads (of which the kernel that is taken is more than 5 % the slower one for 54, 2 us at most): workgroups of the
+// kernel for many rows begin `begin` later, take the tiles of the longest chain at `first` each alone on their CU and at `full` each and workgroup where
+// several share it, and each round of them `round`; those for few rows, one to a CU, `start` and `step` for every eighth tile.  Not causal, whole rounds of
+// workgroups; causal, heaviest first, the longest or all of them over the CUs.  (Short calls, many / few rows: 16 heads of 14 causal rows, D = 32 9.9 / 6.8 us; 4 x 16 of
+// 20, D = 128 17.8 / 8.9; 4 x 8 of 409 against 3565, D = 128 307 / 228, of 2964 against 1299 413 / 550.)
 bool keys_shared(const FwdParams& p, int D) {
-  const double first = D == 128 ? 2.7 : D == 64 ? 1.65 : 1.4, full = D == 128 ? 2.8 : D == 64 ? 1.33 : 1.02;
-  const double start = D == 128 ? 2.5 : D == 64 ? 3.5 : 3.3, step = D == 128 ? 8.0 : D == 64 ? 4.1 : 2.7;
+  const double first = D == 128 ? 2.1 : D == 64 ? 1.53 : 1.49, full = D == 128 ? 2.11 : 1.04;
+  const double begin = D == 128 ? 3.2 : D == 64 ? 2.7 : 2.0, round = D == 128 ? 1.9 : D == 64 ? 0.55 : 0.7;
+  const double start = D == 128 ? 4.45 : D == 64 ? 3.55 : 2.85, step = D == 128 ? 5.52 : D == 64 ? 3.9 : 2.94;
   const double r = (p.Sq + 31) / 32, k = (p.Sk + F32_BN - 1) / F32_BN, cus = spa_device_cus(), pairs = (double)p.B * p.H;
   const double chain = p.causal && r < k ? r : k;
   // tiles that 32 rows see, and 128
@@ -851,10 +854,11 @@ bool keys_shared(const FwdParams& p, int D) {
   if (p.causal) {
     const double longest = start + chain / 8 * step, all = few * (start + seen / 8 * step);
     t_few = longest > all ? longest : all;
-    t_many = chain * first > many * seen4 * full ? chain * first : many * seen4 * full;
+    const double work = many * (seen4 * full + round);
+    t_many = begin + (chain * first > work ? chain * first : work);
   } else {
     t_few = ceil(few) * (start + k / 8 * step);
-    t_many = many <= 1 ? k * first : ceil(many) * k * full;
+    t_many = begin + (many <= 1 ? k * first : ceil(many) * (k * full + round));
   }
   return t_few < t_many;
 }

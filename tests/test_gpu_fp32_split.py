@@ -132,3 +132,18 @@ def test_workgroups_that_share_head_dims_sum_in_the_same_order(D, Sk, causal):
             assert torch.equal(out, whole[:, :heads]) and torch.equal(l, lse[:, :heads]), f"{heads} heads"
     finally:
         _lib.tune("fwd32_split", 0)
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk,D,causal,form", [(1, 5, 79, 386, 64, True, 2), (4, 16, 70, 390, 128, True, 2), (1, 16, 114, 69, 32, False, 2), (4, 8, 409, 3565, 128, False, 2),
+                                                     (4, 8, 2964, 1299, 128, False, 1)])
+def test_the_librarys_choice_by_size(B, H, Sq, Sk, D, causal, form):
+    """Short calls, and those whose longest chain of tiles decides, run on the kernel of few rows, large ones on the other: the bits tell."""
+    q, k, v = (torch.randn((B, s, H, D), generator=torch.Generator().manual_seed(180 + i)).to(DEV) for i, s in enumerate((Sq, Sk, Sk)))
+    own, got = ops.flash_fwd(q, k, v, None, causal)[0], {}
+    for knob in (1, 2):
+        _lib.tune("fwd32_split", knob)
+        try:
+            got[knob] = ops.flash_fwd(q, k, v, None, causal)[0]
+        finally:
+            _lib.tune("fwd32_split", 0)
+    assert torch.equal(own, got[form]) and not torch.equal(own, got[3 - form])
