@@ -6,6 +6,7 @@ import torch
 
 from conftest import rand_qkv
 from oracle import attn_oracle as O
+import sp_aurora_amd as sp
 from sp_aurora_amd import _lib, ops
 from test_gpu_parity import DEV, check_lse, check_out
 
@@ -100,11 +101,10 @@ def test_workgroups_that_share_rows(B, H, Sq, Sk, D, causal):
 
 @pytest.mark.parametrize("B,H,D", [(1, 2, 128), (1, 12, 128), (1, 12, 64), (2, 12, 128)])
 def test_workgroups_that_share_rows_of_shards(B, H, D):
-    import sp_aurora_amd as sp
     S, P = 4 * 66, 4
     q, k, v = rand_qkv((B, S, H, D), 5 + H, torch.float32)
     want_o, _ = O.full_attention(q, k, v, None, True)
-    order = torch.as_tensor(sp.ring.zigzag_order(S, P)) if hasattr(sp, "ring") else None
+    order = torch.as_tensor(sp.ring.zigzag_order(S, P))
     for sharding in ("contiguous", "zigzag"):
         if sharding == "zigzag":
             x, want = [t[:, order].to(DEV) for t in (q, k, v)], want_o[:, order]

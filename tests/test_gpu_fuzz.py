@@ -18,6 +18,7 @@ DEV = "cuda:0"
 N_CASES = 3000
 SEED = 20240611
 _backward_forms = random.Random(SEED + 1)  # (a generator of their own: the cases stay those of SEED)
+_more = random.Random(SEED + 2)  # (likewise: the form of four wave groups, two to seventeen rows)
 
 OUT_TOL = {torch.float32: (1e-5, 1e-3), torch.bfloat16: (2e-2, 1.6e-2), torch.float16: (2e-3, 2e-3)}
 LSE_ATOL = 1e-3
@@ -53,13 +54,15 @@ def _case(rng):
     kind = rng.choice(["block", "block", "ring", "ring_bwd", "fp8", "fp8", "fp8_ring", "varlen", "block_bwd", "block_bwd",
                        "varlen_bwd", "varlen_bwd", "zigzag", "zigzag", "fp8_qkv", "flags", "varlen_decode"])
     share, groups = rng.choice([0, 0, 1, 2, 2]), rng.choice([0, 0, 1, 2])
+    groups = _more.choice([4, groups, groups])
+    few = _more.choice([2, 4, 8, 15, 16, 17, None, None, None])
     _lib.tune("fwd_share", share)
     _lib.tune("fwd_groups", groups)
     _lib.tune("fwd32_split", rng.choice([0, 0, 1, 2]))
     dq_form, dkdv_form = _backward_forms.choice([0, 0, 4, 8, 20, 24]), _backward_forms.choice([0, 0, 1, 2, 3, 4, 5])
     _lib.tune("bwd_dq_waves", dq_form)
     _lib.tune("bwd_dkdv_form", dkdv_form)
-    _lib.tune("few_rows", rng.choice([0, 0, 1]))   # up to three unmasked query rows: the streaming kernel, or the MFMA kernels
+    _lib.tune("few_rows", rng.choice([0, 0, 1]))   # up to sixteen unmasked query rows: the kernels that stream K and V, or those for long rows
     g = torch.Generator().manual_seed(rng.randrange(1 << 30))
     mk = lambda *shape, dt=None: torch.randn(shape, generator=g).to(dt or dtype)
     atol, rtol = OUT_TOL[dtype]
@@ -94,6 +97,7 @@ def _case(rng):
     if kind == "block":
         Sq = rng.choice([1, 2, 3, 7, 64, 65, 127, 128, 129, 200, 256, 300, 513, 700])
         Sk = rng.choice([1, 3, 64, 65, 128, 130, 255, 256, 400, 769])
+        Sq = few or Sq
         split = rng.choice(["auto", "auto", 2, 3, 5])   # keys cut into chunks that run side by side (calls without a mask, 16-bit, D >= 64)
         info = (kind, dtype, B, H, Sq, Sk, D, causal, share, groups, split)
         q, k, v = mk(B, H, Sq, D), mk(B, H, Sk, D), mk(B, H, Sk, D)
@@ -162,6 +166,7 @@ def _case(rng):
             k0 += b
     elif kind == "fp8":
         Sq, Sk = rng.choice([1, 64, 100, 128, 256, 300]), rng.choice([1, 64, 65, 128, 200, 513])
+        Sq = few or Sq
         info = (kind, dtype, B, H, Sq, Sk, D, causal, share, groups)
         q, kf, vf = mk(B, H, Sq, D), mk(B, H, Sk, D, dt=torch.float32), mk(B, H, Sk, D, dt=torch.float32)
         k8, ks = ops.quantize_fp8_per_head(kf, "bhsd")

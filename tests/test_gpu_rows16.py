@@ -1,6 +1,6 @@
-"""Calls of up to 16 query rows without a mask on the kernel that streams K and V through matrix instructions (rows of a head back to back, layout
-[B, H, S, D]; more than three rows also with other heads in between): edges of its tiles of 32 keys and of a workgroup's pass, chunks, both
-element types and e4m3, the values a weight of several terms has to get right."""
+"""Calls of up to 16 query rows without a mask, for the kernel that streams K and V through matrix instructions (rows of a head back to back, layout
+[B, H, S, D], two rows and more or e4m3 K and V; more than three rows also with other heads in between) and those beside it: edges of its tiles of
+32 keys and of a workgroup's pass, chunks, both element types and e4m3, the values a weight of several terms has to get right."""
 import math
 
 import pytest
@@ -69,6 +69,52 @@ def test_more_keys_than_the_memory_side_cache_holds(e4m3, Sq):
         # sums over another number of waves, results (of chunks as well) rounded to bf16
         assert (o.float() - out[i:i + 1].float()).abs().max().item() <= 2.0 ** -6 * out.float().abs().max().item()
         assert (l - lse[i:i + 1]).abs().max().item() < 1e-5
+
+
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float16), (128, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("e4m3,Sq", [(False, 2), (False, 8), (True, 1), (True, 3), (True, 16)])
+def test_large_caches_of_each_type(e4m3, Sq, D, dtype, layout):
+    """Above 64 MiB of K and V, in one piece and in two: every variant of the loads, and the kernels that take what this one leaves (16-bit rows of other heads in
+    between), against one another and, for two heads, against float64."""
+    B, H, Sk = 2, 32, (7000 if e4m3 else 3500) * 128 // D
+    q, k, v = (rand((B, H, s, D), 62 + i, dtype).to(DEV) for i, s in enumerate((Sq, Sk, Sk)))
+    kw, scales = {}, (None, None)
+    if e4m3:
+        (k, ks), (v, vs) = (ops.quantize_fp8_per_head(t, layout="bhsd") for t in (k, v))
+        kw, scales = dict(k_scale=ks, v_scale=vs), (ks, vs)
+    assert k.numel() * k.element_size() * 2 > 64 << 20
+    place = (lambda t: t) if layout == "bhsd" else (lambda t: t.transpose(1, 2).contiguous())
+    whole, cut = (ops.flash_fwd(place(q), place(k), place(v), None, False, layout=layout, split_kv=n, **kw) for n in (1, 2))
+    if layout == "bshd":
+        whole, cut = ((o.transpose(1, 2), l) for o, l in (whole, cut))
+    for b, h in ((0, 0), (1, 31)):
+        one = [q[b, h].double().cpu()] + [t[b, h].double().cpu() * (sc[b, h].double().cpu() if e4m3 else 1) for t, sc in zip((k, v), scales)]
+        want_o, want_l = O.full_attention(*(t[None, :, None] for t in one), None, False)
+        for o, l in (whole, cut):
+            check_out(o[b, h][None, :, None], want_o, dtype)
+            check_lse(l[b, h][None, None], want_l)
+    # (results of chunks and of the call rounded to the type)
+    assert (whole[0].float() - cut[0].float()).abs().max().item() <= 2.0 ** -6 * whole[0].float().abs().max().item()
+    assert (whole[1] - cut[1]).abs().max().item() < 1e-5
+
+
+@pytest.mark.parametrize("B,H", [(1, 8), (2, 8), (1, 16)])
+@pytest.mark.parametrize("Sq,Sk,nsplit", [(1, 300, 1), (3, 700, 3), (8, 1300, 1), (16, 1300, 4)])
+def test_neighbouring_e4m3_heads_that_share_lines(B, H, Sq, Sk, nsplit):
+    """64 e4m3 elements are half a line: with a multiple of 8 heads, workgroups are renumbered so that neighbours run on one XCD.  Every head has its own scales."""
+    D = 64
+    q = rand((B, Sq, H, D), 64, torch.bfloat16)
+    k8, ks, k = quantised((B, Sk, H, D), 65, "bshd")
+    v8, vs, v = quantised((B, Sk, H, D), 66, "bshd")
+    grow = torch.linspace(0.25, 2.0, B * H).reshape(B, H)
+    ks, vs = ks.cpu() * grow, vs.cpu() * grow.flip(1)
+    k, v = (t.cpu() * g[:, None, :, None] for t, g in ((k, grow.double()), (v, grow.flip(1).double())))
+    want_o, want_l = O.full_attention(q, k, v, None, False)
+    place = lambda t: t.transpose(1, 2).contiguous().to(DEV)
+    out, lse = ops.flash_fwd(place(q), place(k8), place(v8), None, False, layout="bhsd", k_scale=ks.to(DEV), v_scale=vs.to(DEV), split_kv=nsplit)
+    check_out(out.transpose(1, 2), want_o, torch.bfloat16)
+    check_lse(lse, want_l)
 
 
 @pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
