@@ -124,8 +124,8 @@ int spa_flash_fwd_fp8kv(const void* q, const void* k8, const void* v8,
  * aligned, the caller's.  _fp8kv: K / V as e4m3 bytes with scales, as for spa_flash_fwd_fp8kv.
  * With up to sixteen query rows (and no mask, the same types and sizes; e4m3 K/V rows 16-byte aligned) these entry points and
  * spa_flash_fwd / spa_flash_fwd_fp8kv run kernels that stream K and V past the rows at the rate of HBM (a 128-row tile would
- * hold a few live rows): up to three rows whatever lies between the rows of K and V, more except from large 16-bit caches with
- * other heads in between.  spa_tune(SPA_TUNE_FEW_ROWS, 1) keeps the other kernels.
+ * hold a few live rows): up to three rows always, more where those are the faster ones (not from large 16-bit caches with other
+ * heads in between, nor where their workgroups would leave CUs idle for long).  spa_tune(SPA_TUNE_FEW_ROWS, 1) keeps the other kernels.
  */
 int64_t spa_flash_fwd_splitkv_workspace_bytes(int B, int H, int Sq, int D, int nsplit, int dtype);
 int spa_flash_fwd_splitkv_suggest(int B, int H, int Sq, int Sk, int D, int mask_mode, int dtype);

@@ -8,7 +8,7 @@
 //                  long as P has the same: those whose scores the first product left in it.
 // A lane owns one query row (lane % 16) in S^T, P^T and O^T alike: the running maximum and sum are per-lane values.  The waves of a
 // workgroup take every kWaves-th tile of 32 keys, each with a state of its own, and add up through LDS at the end.
-// Up to three rows keep their weights in fp32, as three terms of the element type (weight_terms).
+// Up to three rows keep their weights in fp32, as three terms of the element type, of bf16 beside e4m3 values (weight_terms).
 //
 // Grid: x = batch * head, y = key chunk (the key split of the caller: chunk y writes rows y * Sq .. of the result tensors it is given).
 // Bound: HBM.  A key's row is requested in pieces of 64 bytes and 16 keys at a time, which is as good as whole rows only where rows lie back to
@@ -356,7 +356,7 @@ hipError_t launch(const FwdParams& p, hipStream_t stream) {
 // Rows back to back.  One row: not of 16-bit elements (D = 128: 64 x 32 heads of 48 keys 12.2 / 28.5, 8 of 2048 8.5 / 9.6, 32 of 32768 86.8 / 86.1; D = 64, 8 of
 // 700 6.9 / 8.4); of e4m3 ones (D = 64: 64 x 32 heads of 100 keys 22.8 / 14.4, 32 of 4096 12.1 / 10.4, but 5 x 40 of 4096 24.7 / 27.7), at D = 128 in one round
 // (32 of 16384 31.9 / 27.9, 2 x 32 of 100 6.8 / 5.5, 64 x 32 of 256 26.3 / 40.2), but for the few workgroups of a call that is not split (8 of 512 7.7 / 7.9, 4 x
-// 32 of 16384 106 / 134).
+// 32 of 16384 106 / 134; of 700 0.95).
 // Two rows of 16 bits: 32 of 4096 keys, D = 128 18.3 / 17.2, 8 x 32 of 512, D = 64 11.1 / 9.4; 3 x 32 of 8192 42.5 / 51.3, 16 x 20 of 1024, D = 128
 // 32.3 / 38.3, 64 x 32 of 48 14.8 / 28.9; of e4m3 elements 8 x 32 of 2048, D = 128 31.1 / 26.1, but 64 x 32 of 256 35.9 / 40.4.
 // Three: 16 x 32 of 1300, D = 128 63.1 / 58.5, e4m3 42.5 / 33.8; 4 x 34 of 8192, in two chunks 130 / 140.
@@ -378,7 +378,7 @@ bool spa_rows16_takes(const FwdParams& p, int D) {
     return !memory && !(longer && whole && 4 * wgs < 3 * cus);
   }
   switch (p.Sq) {
-    case 1: return kv8 && (D == 64 ? !uneven : wgs <= cus && (!whole || p.Sk <= 256 || 2 * wgs > cus));
+    case 1: return kv8 && (D == 64 ? !uneven : wgs <= cus && (!whole || p.Sk <= 256 || 2 * wgs > cus || (2 * wgs == cus && p.Sk < 1024)));
     case 2:
       if (kv8) return D == 64 ? !uneven : !(longer && second) && wgs < 4 * cus;
       return wgs <= cus ? !uneven : wgs >= 2 * cus && p.Sk > 256;

@@ -1752,8 +1752,8 @@ double launch_time(const BwdParams& p, bool queries, int rows, double start, dou
 
 // D = 64: workgroups of 64 rows, or keys, up to which they are the faster ones.  Two run on a CU: all at once up to two a CU, and beyond that, causal, while
 // the chains are long beside a workgroup's start and end (`rounds` - `start` / tiles, of workgroups of 128): the longest of the others decides, whose CU another
-// one shares.  Backward, causal, us, 128 / 64 rows (dq), and 128 / 64 keys: 12 heads of 2811 rows 91.9 / 78.7, / 79.1; 8 of 4763 147.4 / 127.7, / 128.0; 16 of 2501
-// 87.7 / 76.1, / 75.4; 4 x 16 of 674 33.6 / 35.1, / 38.2.  Of 1900 launches of 250 to 8000 rows, a quarter of them not causal, none got slower by it.
+// one shares.  Both kernels, causal, us, with 128 rows and keys / 64 rows and 128 keys / 128 rows and 64 keys: 12 heads of 2811 rows 91.9 / 78.7 / 79.1; 8 of 4763 147.4 /
+// 127.7 / 128.0; 16 of 2501 87.7 / 76.1 / 75.4; 4 x 16 of 674 33.6 / 35.1 / 38.2 (and with 64 of both 12 heads of 2811 72, 8 of 4763 116).  Of 1900 launches of 250 to 8000 rows, a quarter of them not causal, none got slower by it.
 double most_64(const BwdParams& p, double rounds, double start) {
   const double of_128 = p.causal && !p.cu_q ? rounds - start / ((p.Sq + BWD_ROWS - 1) / BWD_ROWS) : 1.0;
   return 2.0 * spa_device_cus() * (of_128 > 1.0 ? of_128 : 1.0);
